@@ -1,151 +1,200 @@
 // Tiled MFMA GEMM for the batched (prefill) projections: y = epi(x W^T) with many rows.
 //
-// A workgroup (4 waves) owns a tile of 128 activation rows x 128 packed weight rows.  Each wave
-// owns two 16-row weight strips for all 128 activation rows: 16 accumulators of
-// v_mfma_f32_16x16x32_bf16 (weights = A operand, activations = B operand, exactly as in the
-// skinny kernel, so the epilogues are shared).  Per 64-deep k-step
-//   * the weights of a wave's strips come straight from the packed layout into registers
-//     (one contiguous 1 KiB per wave-load, no duplication between waves, prefetched one
-//     step ahead),
-//   * the 128 x 64 activation tile is loaded once per workgroup with 128-byte row segments,
-//     staged in LDS (rows padded to 144 B: conflict-free 16-byte reads) and double-buffered,
-//     so one barrier per step suffices.
-// Workgroup ids are remapped so that all weight tiles of one activation tile run on the same
-// XCD (ids round-robin over the 8 XCDs): the activation tile is then fetched into one L2 only,
-// while the weights (a few MB) live in every L2.
+// A workgroup owns a tile of TM activation rows x TS packed 16-row weight strips; its WM x WN waves own FM x FN
+// fragments of v_mfma_f32_16x16x32_bf16 each (weights = A operand, activations = B operand, exactly as in the skinny
+// kernel, so the epilogues are shared).  K is walked in order, KH MFMA steps of 32 at a time, so the sums do not depend
+// on the tile.  Both operands of a step travel straight from global memory into LDS (global_load_lds, 16 bytes a lane: no
+// registers held in flight, NST - 1 steps ahead) and every wave reads its fragments from there:
+//   * a packed weight tile (strip, k-step) is 1 KiB in lane order: one load, and a conflict-free 16-byte read;
+//   * a load of activations is 1 KiB of whole row segments of 64 KH bytes; the 16-byte pieces of a row are permuted by the
+//     row's number on their way in (each lane chooses its global address, the LDS side is always in lane order), which
+//     is what makes the fragment reads of sixteen rows conflict-free without padding.
+// One barrier per step: it says that the step's loads have arrived (every wave waits for its own first) and that the slot
+// of the step before is free for the next loads.
+//
+// What bounds it: in large tiles the LDS side and the matrix pipe together (a step of 128 x 192 x 64 takes 0.72 us where its
+// products alone take 0.41 us at the 2.0 GHz the chip holds under them); in small ones the chain barrier - read - multiply
+// of a step (0.135 to 0.34 us).  The kernel before this one (128 x 128, weights straight to registers) against this one,
+// us a call: 8192 rows 6144 x 768 with SwiGLU 114 / 93, 2304 x 768 44.4 / 36.8, 768 x 768 22.7 / 18.2, 768 x 3072 61 / 45;
+// 4001 rows 11264 x 2048 250 / 202, 2048 x 5632 115 / 94; 128 rows 6144 x 768 19.1 / 6.0, 768 x 3072 41.6 / 9.1.
+// Measured and dropped: fragments of the next half step read ahead into registers of their own (no gain at four
+// waves, spills at 256 x 256), the loads spread among the products (they then arrive late: 971 -> 1192 us at 8192^3), deeper
+// rings (no gain, fewer workgroups a CU), four waves a tile of 128 x 192 (99 / 52 us against 93 / 45).
+//
+// Workgroup ids go round-robin over the eight XCDs: an XCD gets a contiguous run of tiles, eight activation tiles side
+// by side, so that a run shares its operands in that XCD's L2.
 //
 // Replaces the F.linear calls of ohara/models/llama.py:84-86,142,322 and
 // ohara/modules/mlp.py:152 when the call carries more than 64 rows.
 #include "gemm_epilogue.h"
 
+#include <type_traits>
+
 namespace {
 
-constexpr int TM = 128;        // activation rows per tile
-constexpr int TS = 8;          // weight strips per tile (128 packed rows)
-constexpr int KB = 64;         // k per step
-constexpr int LDX = KB + 8;    // LDS row stride in elements (144 B)
+// 16 bytes per lane from sbase + voff to LDS byte lds + 16 * lane.  (Assembly: behind the builtin the compiler waits for
+// every such load in flight before any LDS read, which would undo the ring.  No vector register is written; the waits
+// are wait_loads below; M0 holds nothing of the compiler's here, the kernel has no other instruction that reads it.)
+__device__ __forceinline__ void load_lds16(uint32_t lds, const void* sbase, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(sbase) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() {  // until at most N of this wave's loads are in flight
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 
-template <int EPI>
-__global__ __launch_bounds__(256, 2) void gemm_tile_kernel(GemmArgs a, int MT, int NT, int nstrips) {
-  __shared__ __align__(16) bf16_t xs[2][TM][LDX];
-  const int id = blockIdx.x;
-  const int xcd = id & 7, q = id >> 3;
-  const int tn = q % NT;
-  const int tm = (q / NT) * 8 + xcd;
-  if (tm >= MT) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+template <int WM_, int WN_, int FM_, int FN_, int KH_, int NST_>
+struct Tile {
+  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, KH = KH_, NST = NST_;
+  static constexpr int NW = WM * WN;                       // waves
+  static constexpr int TM = WM * FM * 16, TS = WN * FN;    // rows, strips
+  static constexpr int RPL = 16 / KH;                      // activation rows of a 1 KiB load
+  static constexpr int XL = TM / RPL, WL = TS * KH;        // 1 KiB loads of a step
+  static constexpr int LPW = (XL + WL) / NW;               // of one wave
+  static constexpr int STAGE = (XL + WL) * 1024, LDS = NST * STAGE;
+  static_assert(XL % NW == 0 && WL % NW == 0, "loads split evenly over the waves");
+  static_assert((KH == 2 || KH == 4) && LDS <= 160 * 1024, "");
+};
+
+// ALIGNED: activation rows start on 16 bytes and a tile of them spans less than 4 GiB (false: through registers, any)
+template <int EPI, class C, bool ALIGNED>
+__global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, int MT, int NT, int nstrips) {
+  constexpr int FM = C::FM, FN = C::FN, KH = C::KH, NST = C::NST, NW = C::NW, XL = C::XL, WL = C::WL, LPW = C::LPW;
+  constexpr int STAGE = C::STAGE, KB = 32 * KH, GM = 8;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int T = MT * NT;
+  const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+  const int base = T >> 3, rem = T & 7;
+  if (q >= base + (xcd < rem ? 1 : 0)) return;
+  const int pid = xcd * base + min(xcd, rem) + q;
+  const int grp = pid / (GM * NT), first = grp * GM, gsz = min(GM, MT - first), r = pid - grp * GM * NT;
+  const int row0 = (first + r % gsz) * C::TM, strip0 = (r / gsz) * C::TS;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / C::WN, wn = wave % C::WN;
   const int m = lane & 15, g = lane >> 4;
-  const int row0 = tm * TM;
-  const int strip0 = tn * TS + wave * 2;
-  const int KS = (a.K + 31) >> 5;
-  const int nsteps = (KS + 1) >> 1;
+  const int KS = (a.K + 31) >> 5, nsteps = (KS + KH - 1) / KH;
+  const bool tail = a.K % KB != 0;                         // the last step is not full
 
-  // activation tile loader: 8 threads x 16 B per row, 32 rows per pass, 4 passes
-  const int lr = tid >> 3, lc = (tid & 7) * 8;
-  auto load_x = [&](int step, uint4* xr) {
-    const int k = step * KB + lc;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
+  const char* xb = reinterpret_cast<const char*>(a.x + (size_t)row0 * a.ldx);
+  const char* wb = reinterpret_cast<const char*>(a.wp);
+  const uint32_t lane16 = lane * 16;
+  const int lrow = lane / (4 * KH);                        // this lane's row of a load
+  typedef typename std::conditional<ALIGNED, uint32_t, uint64_t>::type offset_t;
+  offset_t xoff[XL / NW];                                  // rows past the end read the last row
+  int piece[XL / NW];                                      // the 16-byte piece of its row that this lane fetches
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int r = row0 + p * 32 + lr;
-      xr[p] = (r < a.B && k < a.K) ? ldg16(a.x + (size_t)r * a.ldx + k) : make_uint4(0, 0, 0, 0);
+  for (int i = 0; i < XL / NW; ++i) {
+    const int rr = (wave + i * NW) * C::RPL + lrow;
+    piece[i] = (lane & (4 * KH - 1)) ^ (rr & 7);
+    xoff[i] = ((offset_t)(min(row0 + rr, a.B - 1) - row0) * a.ldx + piece[i] * 8) * 2;
+  }
+  auto issue = [&](int s, uint32_t slot) {
+    const char* xs = xb + (size_t)s * (2 * KB);
+    const bool last = tail && s == nsteps - 1;
+#pragma unroll
+    for (int i = 0; i < XL / NW; ++i) {
+      const uint32_t dst = slot + (wave + i * NW) * 1024;
+      // pieces past K read the row's last piece and are multiplied by zero
+      const uint32_t back = last ? (uint32_t)max(0, s * KB + piece[i] * 8 - (a.K - 8)) * 2 : 0u;
+      if (ALIGNED) {
+        load_lds16(dst, xs, xoff[i] - back);
+      } else {
+        const uint4 v = ldg16(xs + xoff[i] - back);
+        *(OHARA_LDS u32x4*)(uintptr_t)(dst + lane16) = (u32x4){v.x, v.y, v.z, v.w};
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < WL / NW; ++i) {
+      const int t = wave + i * NW;  // strip t / KH, k-step t % KH; past the end: the last one, never used
+      const int strip = min(strip0 + t / KH, nstrips - 1), j = min(KH * s + t % KH, KS - 1);
+      load_lds16(slot + (XL + t) * 1024, wb + ((size_t)strip * KS + j) * 1024, lane16);
     }
   };
-  auto store_x = [&](int buf, const uint4* xr) {
-#pragma unroll
-    for (int p = 0; p < 4; ++p) *reinterpret_cast<uint4*>(&xs[buf][p * 32 + lr][lc]) = xr[p];
-  };
-  const uint4* w0 = a.wp + (size_t)strip0 * KS * 64 + lane;
-  const uint4* w1 = w0 + (size_t)KS * 64;
-  const bool live0 = strip0 < nstrips, live1 = strip0 + 1 < nstrips;
-  auto load_w = [&](int step, uint4* wv) {
-    const int j = step * 2;
-    wv[0] = (live0 && j < KS) ? ldg16(w0 + (size_t)j * 64) : make_uint4(0, 0, 0, 0);
-    wv[1] = (live0 && j + 1 < KS) ? ldg16(w0 + (size_t)(j + 1) * 64) : make_uint4(0, 0, 0, 0);
-    wv[2] = (live1 && j < KS) ? ldg16(w1 + (size_t)j * 64) : make_uint4(0, 0, 0, 0);
-    wv[3] = (live1 && j + 1 < KS) ? ldg16(w1 + (size_t)(j + 1) * 64) : make_uint4(0, 0, 0, 0);
-  };
 
-  f32x4 acc[2][8];
+  f32x4 acc[FN][FM];
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int u = 0; u < FN; ++u)
 #pragma unroll
-    for (int t = 0; t < 8; ++t) acc[u][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  uint4 xr[4], wv[4], wn[4];
-  load_x(0, xr);
-  load_w(0, wv);
-  store_x(0, xr);
-  __syncthreads();
+    for (int t = 0; t < FM; ++t) acc[u][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < nsteps) issue(s, lds0 + s * STAGE);
+  const uint32_t xrd = lds0 + (wm * FM * 16 + m) * (64 * KH);
+  const uint32_t wrd = lds0 + (XL + wn * FN * KH) * 1024 + lane16;
+  uint32_t so = 0, si = (NST - 1) * STAGE;
   for (int s = 0; s < nsteps; ++s) {
-    const int buf = s & 1;
-    const bool more = s + 1 < nsteps;
-    if (more) {
-      load_x(s + 1, xr);
-      load_w(s + 1, wn);
-    }
-    // The eight B operands of a half step are read from LDS into registers of their own before its
-    // products.  (Left to itself the compiler reuses one register quad: read, wait, two products,
-    // sixteen times per step, every LDS latency exposed.  All sixteen up front would take the
-    // kernel from three workgroups per CU to two, which costs more than it gains.)
+    if (!ALIGNED) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    else if (NST == 2 || s + NST - 2 >= nsteps) wait_loads<0>();
+    else wait_loads<(NST - 2) * LPW>();
+    __builtin_amdgcn_s_barrier();
+    if (s + NST - 1 < nsteps) issue(s + NST - 1, lds0 + si);
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      uint4 bv[8];
+    for (int jj = 0; jj < KH; ++jj) {
+      // all fragments of a k-step into registers of their own before its products
+      uint4 xf[FM], wf[FN];
+      const uint32_t sw = (uint32_t)((4 * jj + g) ^ (m & 7)) * 16;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) bv[t] = *reinterpret_cast<const uint4*>(&xs[buf][t * 16 + m][jj * 32 + 8 * g]);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int u = 0; u < FN; ++u) wf[u] = lds16_at(wrd + so + (u * KH + jj) * 1024);
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[jj]),
-                                                            __builtin_bit_cast(bf16x8, bv[t]), acc[0][t], 0, 0, 0);
-        acc[1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[2 + jj]),
-                                                            __builtin_bit_cast(bf16x8, bv[t]), acc[1][t], 0, 0, 0);
+      for (int t = 0; t < FM; ++t) xf[t] = lds16_at(xrd + so + t * (1024 * KH) + sw);
+      if (tail && s == nsteps - 1) {
+        const bool in = KB * s + 32 * jj + 8 * g < a.K;
+#pragma unroll
+        for (int t = 0; t < FM; ++t) xf[t] = in ? xf[t] : make_uint4(0, 0, 0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
-    }
-    if (more) {
-      store_x(buf ^ 1, xr);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) wv[i] = wn[i];
+      for (int t = 0; t < FM; ++t)
+#pragma unroll
+        for (int u = 0; u < FN; ++u)
+          acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[u]),
+                                                              __builtin_bit_cast(bf16x8, xf[t]), acc[u][t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
+    so = so + STAGE == NST * STAGE ? 0 : so + STAGE;
+    si = si + STAGE == NST * STAGE ? 0 : si + STAGE;
   }
+  const int rbase = row0 + wm * FM * 16, sbase = strip0 + wn * FN;
 
-  // A thread finishes sixteen fragments.  What their epilogues read (residual rows, biases, rotary
-  // values) is fetched for eight of them before the first is used, instead of one dependent round trip
+  // A thread finishes FM * FN fragments.  What their epilogues read (residual rows, biases, rotary
+  // values) is fetched for a strip's before the first is used, instead of one dependent round trip
   // per fragment.
-  // Rotary epilogue: position, sequence and cache row depend on the activation row alone (eight per
+  // Rotary epilogue: position, sequence and cache row depend on the activation row alone (FM per
   // thread, and rows of a tile are consecutive: no division per row when a sequence is at least a tile
   // long), the region (q / k / v) and the feature index inside the head on the strip alone (uniform
   // over the wave).  Worked out per fragment they were 40 % of this kernel's instructions.
-  if (EPI == EPI_ROPE && a.S >= TM && ((a.ldo | a.Dh) & 15) == 0 && ((a.H * a.Dh) & 15) == 0 && !a.stage) {
+  if (rbase >= a.B) return;
+  if (EPI == EPI_ROPE && a.S >= FM * 16 && ((a.ldo | a.Dh) & 15) == 0 && ((a.H * a.Dh) & 15) == 0 && !a.stage) {
     const int nq = a.H * a.Dh, nk = a.Hkv * a.Dh;
-    const int base = a.row0 + row0;                            // global row of the tile's first row
-    const int seq0 = base / a.S, rem0 = base - seq0 * a.S;     // uniform over the workgroup
-    int pos_t[8];
-    size_t qoff_t[8], coff_t[8];
+    const int gbase = a.row0 + rbase;                          // global row of the wave's first row
+    const int seq0 = gbase / a.S, rem0 = gbase - seq0 * a.S;   // uniform over the wave
+    int pos_t[FM];
+    size_t qoff_t[FM], coff_t[FM];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int x = rem0 + t * 16 + m;
+    for (int t = 0; t < FM; ++t) {
+      const int x = rem0 + min(t * 16 + m, a.B - 1 - rbase);  // rows past the end: the last row, never stored
       const bool wrap = x >= a.S;
       const int seq = seq0 + (wrap ? 1 : 0), sidx = x - (wrap ? a.S : 0);
-      const int grow = base + t * 16 + m;
+      const int grow = gbase + t * 16 + m;
       pos_t[t] = (a.pos_dev ? a.pos_dev[(size_t)seq * a.pos_stride] : a.pos) + sidx;
       qoff_t[t] = (size_t)grow * a.ldo;
       coff_t[t] = (((size_t)seq * a.Tmax + pos_t[t]) * a.Hkv) * a.Dh;
     }
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int strip = strip0 + u;
+    for (int u = 0; u < FN; ++u) {
+      const int strip = sbase + u;
       if (strip >= nstrips) continue;
       const int rr = strip * 16;  // uniform: the whole strip lies in one region and one head
       if (rr >= nq + 2 * nk) continue;
       const int region = rr < nq ? 0 : (rr < nq + nk ? 1 : 2);
       const int rloc = rr - (region == 0 ? 0 : (region == 1 ? nq : nq + nk)) + 4 * g;  // column inside q, k or v
       const int d = (rr - (region == 0 ? 0 : nq)) % a.Dh + 4 * g;
-      uint32_t cv[8], sv[8];
+      uint32_t cv[FM], sv[FM];
       if (region < 2) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
+        for (int t = 0; t < FM; ++t) {
           const int pc = min(max(pos_t[t], 0), a.Tmax - 1);
           cv[t] = *reinterpret_cast<const uint32_t*>(a.cos + (size_t)pc * (a.Dh >> 1) + (d >> 1));
           sv[t] = *reinterpret_cast<const uint32_t*>(a.sin + (size_t)pc * (a.Dh >> 1) + (d >> 1));
@@ -153,8 +202,8 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(GemmArgs a, int MT, i
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int b = row0 + t * 16 + m;
+      for (int t = 0; t < FM; ++t) {
+        const int b = rbase + t * 16 + m;
         if (b >= a.B || pos_t[t] < 0 || pos_t[t] >= a.Tmax) continue;
         float v[4] = {rbf(acc[u][t][0]), rbf(acc[u][t][1]), rbf(acc[u][t][2]), rbf(acc[u][t][3])};
         if (region < 2) {
@@ -177,28 +226,97 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(GemmArgs a, int MT, i
                          EPI == EPI_BIAS_ADD2 || EPI == EPI_PHI_IN || EPI == EPI_BIAS_XIELU;
   if (READS && a.N >= 4 && ((a.N | a.ldo | a.ldr | (EPI == EPI_BIAS_ADD2 ? a.ldr2 : 0)) & 3) == 0) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {  // eight fragments at a time: sixteen sets of operands cost a resident workgroup
-      EpiPre pre[8];
+    for (int u = 0; u < FN; ++u) {  // a strip at a time: more sets of operands would cost a resident workgroup
+      EpiPre pre[FM];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) gemm_epilogue_fetch<EPI>(a, row0 + t * 16 + m, min(strip0 + u, nstrips - 1), g, pre[t]);
+      for (int t = 0; t < FM; ++t) gemm_epilogue_fetch<EPI>(a, rbase + t * 16 + m, min(sbase + u, nstrips - 1), g, pre[t]);
       __builtin_amdgcn_sched_barrier(0);
-      if (strip0 + u >= nstrips) continue;
+      if (sbase + u >= nstrips) continue;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int b = row0 + t * 16 + m;
-        if (b < a.B) gemm_epilogue<EPI, true>(a, b, strip0 + u, g, acc[u][t], pre[t]);
+      for (int t = 0; t < FM; ++t) {
+        const int b = rbase + t * 16 + m;
+        if (b < a.B) gemm_epilogue<EPI, true>(a, b, sbase + u, g, acc[u][t], pre[t]);
       }
     }
     return;
   }
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    if (strip0 + u >= nstrips) continue;
+  for (int u = 0; u < FN; ++u) {
+    if (sbase + u >= nstrips) continue;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int b = row0 + t * 16 + m;
-      if (b < a.B) gemm_epilogue<EPI>(a, b, strip0 + u, g, acc[u][t]);
+    for (int t = 0; t < FM; ++t) {
+      const int b = rbase + t * 16 + m;
+      if (b < a.B) gemm_epilogue<EPI>(a, b, sbase + u, g, acc[u][t]);
     }
+  }
+}
+
+template <int EPI, class C, bool ALIGNED = true>
+int launch_tile(const GemmArgs& a, int nstrips, hipStream_t st) {
+  const int64_t MT = (a.B + C::TM - 1) / C::TM, NT = (nstrips + C::TS - 1) / C::TS;
+  if (MT * NT > INT32_MAX - 8) return OHARA_ESIZE;
+  if (C::LDS > 64 * 1024)
+    (void)hipFuncSetAttribute((const void*)gemm_tile_kernel<EPI, C, ALIGNED>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+  hipLaunchKernelGGL((gemm_tile_kernel<EPI, C, ALIGNED>), dim3((unsigned)(MT * NT + 7) / 8 * 8), dim3(C::NW * 64), C::LDS, st, a,
+                     (int)MT, (int)NT, nstrips);
+  return ohara_launch_status();
+}
+
+//           waves fragments k-steps slots
+typedef Tile<2, 2, 1, 1, 4, 3> T32;       //  32 x  32
+typedef Tile<2, 2, 2, 2, 4, 2> T64;       //  64 x  64
+typedef Tile<2, 4, 2, 2, 2, 3> T64x128;
+typedef Tile<2, 4, 4, 2, 2, 2> T128;
+typedef Tile<2, 4, 4, 3, 2, 2> T128x192;
+typedef Tile<2, 4, 8, 4, 2, 2> T256;
+
+// Which tile: the one that should take least time.  A large tile needs less LDS traffic a product, a small one keeps more
+// CUs busy and its chain of steps is shorter.  The times are measured (33 shapes: 96 to 8192 rows, 768 to 17920 packed
+// rows, K 768 to 10240); the choice they give is within 1 % of the best of the six on average, 20 % at worst.
+struct TileTime {
+  int rows, strips;
+  int slots;    // workgroups that share a CU
+  float alone;  // us a step of 64 takes one workgroup on a CU
+  float more;   // what another one beside it adds, as a share of that
+  float full;   // us a step takes each of the workgroups of a full chip
+  float ends;   // us the start and the epilogue add
+};
+constexpr TileTime TIMES[6] = {
+    {T32::TM, T32::TS, 3, 0.135f, 0.25f, 0.10f, 0.9f},        {T64::TM, T64::TS, 2, 0.25f, 0.3f, 0.215f, 1.3f},
+    {T64x128::TM, T64x128::TS, 2, 0.335f, 0.4f, 0.37f, 1.6f}, {T128::TM, T128::TS, 2, 0.50f, 0.8f, 0.54f, 2.5f},
+    {T128x192::TM, T128x192::TS, 2, 0.74f, 0.75f, 0.72f, 3.0f}, {T256::TM, T256::TS, 1, 1.70f, 1.0f, 1.75f, 8.0f},
+};
+float tile_time(const TileTime& t, int rows, int strips, int K) {
+  constexpr int CUS = 256;
+  const int64_t tiles = ((int64_t)rows + t.rows - 1) / t.rows * ((strips + t.strips - 1) / t.strips);
+  const int64_t waves = tiles / (CUS * t.slots), rest = tiles % (CUS * t.slots);
+  float step = waves * t.slots * t.full;
+  if (rest) {
+    const float chain = t.alone * (1.f + t.more * ((rest + CUS - 1) / CUS - 1)), chip = rest * (1.f / CUS) * t.full;
+    step += rest <= CUS || chain > chip ? chain : chip;
+  }
+  return step * K * (1.f / 64.f) + t.ends * (tiles > CUS ? tiles * (1.f / CUS) : 1.f);
+}
+
+template <int EPI>
+int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
+  if (((uintptr_t)a.x & 15) != 0 || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return launch_tile<EPI, T64, false>(a, nstrips, st);
+  int best = 0;
+  float low = tile_time(TIMES[0], a.B, nstrips, a.K);
+  for (int i = 1; i < 6; ++i) {
+    const float t = tile_time(TIMES[i], a.B, nstrips, a.K);
+    if (t < low) {
+      low = t;
+      best = i;
+    }
+  }
+  switch (best) {
+    case 0: return launch_tile<EPI, T32>(a, nstrips, st);
+    case 1: return launch_tile<EPI, T64>(a, nstrips, st);
+    case 2: return launch_tile<EPI, T64x128>(a, nstrips, st);
+    case 3: return launch_tile<EPI, T128>(a, nstrips, st);
+    case 4: return launch_tile<EPI, T128x192>(a, nstrips, st);
+    default: return launch_tile<EPI, T256>(a, nstrips, st);
   }
 }
 
@@ -207,27 +325,21 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(GemmArgs a, int MT, i
 // Launcher shared with the skinny entry points (declared there).
 int ohara_launch_gemm_tile(const GemmArgs& a, int epi, int packed_rows, hipStream_t st) {
   const int nstrips = packed_rows / 16;
-  const int NT = (nstrips + TS - 1) / TS;
-  const int MT = (a.B + TM - 1) / TM;
-  const int64_t blocks = (int64_t)((MT + 7) / 8) * 8 * NT;
-  if (blocks > INT32_MAX) return OHARA_ESIZE;
-  dim3 grid((unsigned)blocks), block(256);
   switch (epi) {
-    case EPI_STORE: hipLaunchKernelGGL((gemm_tile_kernel<EPI_STORE>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_RESIDUAL: hipLaunchKernelGGL((gemm_tile_kernel<EPI_RESIDUAL>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_SWIGLU: hipLaunchKernelGGL((gemm_tile_kernel<EPI_SWIGLU>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_ROPE: hipLaunchKernelGGL((gemm_tile_kernel<EPI_ROPE>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_BIAS: hipLaunchKernelGGL((gemm_tile_kernel<EPI_BIAS>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_BIAS_GELU: hipLaunchKernelGGL((gemm_tile_kernel<EPI_BIAS_GELU>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_BIAS_ADD2: hipLaunchKernelGGL((gemm_tile_kernel<EPI_BIAS_ADD2>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_PHI_IN: hipLaunchKernelGGL((gemm_tile_kernel<EPI_PHI_IN>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_SOFTCAP: hipLaunchKernelGGL((gemm_tile_kernel<EPI_SOFTCAP>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_GELU_LOOKUP: hipLaunchKernelGGL((gemm_tile_kernel<EPI_GELU_LOOKUP>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_BIAS_XIELU: hipLaunchKernelGGL((gemm_tile_kernel<EPI_BIAS_XIELU>), grid, block, 0, st, a, MT, NT, nstrips); break;
-    case EPI_GLU: hipLaunchKernelGGL((gemm_tile_kernel<EPI_GLU>), grid, block, 0, st, a, MT, NT, nstrips); break;
+    case EPI_STORE: return launch_epi<EPI_STORE>(a, nstrips, st);
+    case EPI_RESIDUAL: return launch_epi<EPI_RESIDUAL>(a, nstrips, st);
+    case EPI_SWIGLU: return launch_epi<EPI_SWIGLU>(a, nstrips, st);
+    case EPI_ROPE: return launch_epi<EPI_ROPE>(a, nstrips, st);
+    case EPI_BIAS: return launch_epi<EPI_BIAS>(a, nstrips, st);
+    case EPI_BIAS_GELU: return launch_epi<EPI_BIAS_GELU>(a, nstrips, st);
+    case EPI_BIAS_ADD2: return launch_epi<EPI_BIAS_ADD2>(a, nstrips, st);
+    case EPI_PHI_IN: return launch_epi<EPI_PHI_IN>(a, nstrips, st);
+    case EPI_SOFTCAP: return launch_epi<EPI_SOFTCAP>(a, nstrips, st);
+    case EPI_GELU_LOOKUP: return launch_epi<EPI_GELU_LOOKUP>(a, nstrips, st);
+    case EPI_BIAS_XIELU: return launch_epi<EPI_BIAS_XIELU>(a, nstrips, st);
+    case EPI_GLU: return launch_epi<EPI_GLU>(a, nstrips, st);
     default: return OHARA_EINVAL;
   }
-  return ohara_launch_status();
 }
 
 extern "C" int ohara_gemm_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, int rows, int epilogue,
