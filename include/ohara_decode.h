@@ -284,6 +284,19 @@ int ohara_act_quant_int8(const uint16_t* x, int ldx, const uint16_t* norm_w, flo
 int ohara_gemv_ternary_i8(const int8_t* q, int ldq, const float* s, const int32_t* sumq, const uint32_t* wp, int n,
                           int k, float gamma, int rows, const uint16_t* resid, int ldr, uint16_t* out, int ldo,
                           int32_t* acc_out, int ldacc, void* stream);
+/* Many rows: each row quantised once for each of `sets` (at most three) BitLinears that read it and differ in their norm
+ * weight; q: (sets, rows, ldq), s and sumq: (sets, rows).  ohara_gemv_ternary_i8 (more than 64 rows, q on 16 bytes),
+ * ohara_gemm_ternary_sets_i8 (`sets` weights of n columns, one output each) and ohara_gemm_ternary_qkv_rope_append (query, key,
+ * value: rotary + append as in ohara_bitlinear_qkv_rope_append_bf16, any number of rows) multiply the codes in tiles; the
+ * accumulators are those of ohara_bitlinear_bf16.  ldq a multiple of 16, q on 16 bytes, k a multiple of 8. */
+int ohara_act_quant_sets_int8(const uint16_t* x, int ldx, const uint16_t* pre_norm_w, const uint16_t* const* norm_w, int sets,
+                              float eps, int rows, int k, int8_t* q, int ldq, float* s, int32_t* sumq, void* stream);
+int ohara_gemm_ternary_sets_i8(const int8_t* q, int ldq, const float* s, const int32_t* sumq, const uint32_t* const* wp,
+                               const float* gamma, int sets, int n, int k, int rows, uint16_t* const* out, int ldo, void* stream);
+int ohara_gemm_ternary_qkv_rope_append(const int8_t* q, int ldq, const float* s, const int32_t* sumq, const uint32_t* const* wp,
+                                       const float* gamma, int k, int batch, int seq_len, int h, int h_kv, int dh,
+                                       const uint16_t* cos, const uint16_t* sin, int pos, const int32_t* pos_dev, uint16_t* q_out,
+                                       uint16_t* kcache, uint16_t* vcache, int t_max, void* stream);
 int ohara_bitlinear_bf16(const uint16_t* x, int ldx, const uint16_t* pre_norm_w, const uint16_t* norm_w, float eps,
                          const uint32_t* wp, int n, int k, float gamma, int rows, const uint16_t* resid, int ldr,
                          uint16_t* out, int ldo, int32_t* acc_out, int ldacc, void* stream);

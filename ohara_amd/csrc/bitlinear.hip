@@ -212,6 +212,26 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const bf16_t* x, int ldx
   }
 }
 
+// Many rows (more than a workgroup's LDS holds): every row is quantised once for each of up to three BitLinears that read it
+// (blockIdx.y: they differ in their norm weight), and ternary_tile_kernel multiplies the codes.
+struct QuantSets {
+  const bf16_t* nw[3];
+};
+__global__ __launch_bounds__(256) void act_quant_sets_kernel(const bf16_t* x, int ldx, const bf16_t* pre_w, QuantSets sets, int rows,
+                                                             int K, float eps, int8_t* q, int ldq, float* s_out, int* sumq_out) {
+  extern __shared__ __align__(16) unsigned char qsm[];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int r = blockIdx.x * 4 + wave;
+  if (r >= rows) return;
+  const bf16_t* nw = blockIdx.y == 0 ? sets.nw[0] : (blockIdx.y == 1 ? sets.nw[1] : sets.nw[2]);
+  const size_t o = (size_t)blockIdx.y * rows + r;
+  const QuantOut v = wave_quant_row(x + (size_t)r * ldx, pre_w, nw, K, eps, q + o * ldq, reinterpret_cast<bf16_t*>(qsm) + (size_t)wave * K);
+  if (lane == 0) {
+    s_out[o] = v.s;
+    sumq_out[o] = v.sumq;
+  }
+}
+
 struct BitArgs {
   const uint4* wp;       // packed ternary
   float gamma;
@@ -561,6 +581,234 @@ __global__ __launch_bounds__(256) void rope_append_kernel(bf16_t* q, const bf16_
   for (int i = threadIdx.x; i < Hkv * D; i += 256) vd[i] = v[(size_t)row * Hkv * D + i];
 }
 
+// ---- many rows ---------------------------------------------------------------------------------
+// Up to three BitLinears (their own codes, weights and outputs) as one launch of the tiled product of gemm_tile.hip on
+// v_mfma_i32_16x16x64_i8: a workgroup owns TM rows of codes x TS strips, steps of 256 columns travel straight into LDS
+// (codes: 256-byte row segments with their 16-byte pieces permuted by the row, weights: one 1 KiB tile a strip), a
+// wave unpacks a strip's tile into operands once for its FM row blocks.  The sums are whole numbers, so neither the tile nor the
+// order shows in them.
+// What bounds it: the chain of a step (barrier, reads, unpacking, products).  A layer of the 2048 x 5632 ternary model over
+// 300 rows took nine to twelve launches a projection group of the kernel above, each of which quantised its rows
+// again in every one of its 128 to 352 workgroups (3.0 ms a layer); quantised once and multiplied here it takes 0.13 ms.
+struct TernarySet {
+  const uint4* wp;
+  const int8_t* q;
+  const float* s;
+  const int* sumq;
+  float gamma;
+  int N, tiles;          // columns, tiles of columns
+  bf16_t* out;           // ROPE: q rows, key cache, value cache
+  int ldo;
+  const bf16_t* resid;
+  int ldr;
+  int32_t* acc_out;
+  int ldacc;
+};
+struct TernaryArgs {
+  TernarySet set[3];
+  int rows, K, ldq, MT, NT;
+  int wide;              // columns and leading dimensions in fours: 8-byte stores
+  // ROPE
+  int S, Dh, Tmax, pos;
+  const int32_t* pos_dev;
+  const bf16_t* cos;
+  const bf16_t* sin;
+};
+
+template <int WM, int WN, int FM, int FN, int NST, bool ROPE>
+__global__ __launch_bounds__(WM * WN * 64, 2) void ternary_tile_kernel(TernaryArgs a) {
+  constexpr int NW = WM * WN, TM = WM * FM * 16, TS = WN * FN, XL = TM / 4, WL = TS, LPW = (XL + WL) / NW;
+  constexpr int STAGE = (XL + WL) * 1024, GM = 8;
+  static_assert(XL % NW == 0 && WL % NW == 0, "loads split evenly over the waves");
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int T = a.MT * a.NT;
+  const int xcd = blockIdx.x & 7, qd = blockIdx.x >> 3;
+  const int base = T >> 3, rem = T & 7;
+  if (qd >= base + (xcd < rem ? 1 : 0)) return;
+  const int pid = xcd * base + min(xcd, rem) + qd;
+  const int grp = pid / (GM * a.NT), first = grp * GM, gsz = min(GM, a.MT - first), r = pid - grp * GM * a.NT;
+  const int row0 = (first + r % gsz) * TM;
+  int tn = r / gsz, which = 0;
+  TernarySet w = a.set[0];  // (no dynamic indexing of the argument block: that would copy it to scratch memory)
+  if (tn >= w.tiles) { tn -= w.tiles; which = 1; w = a.set[1]; }
+  if (which == 1 && tn >= w.tiles) { tn -= w.tiles; which = 2; w = a.set[2]; }
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int m = lane & 15, g = lane >> 4;
+  const int KC = (a.K + 255) >> 8, strip0 = tn * TS, nstrips = (w.N + 15) >> 4;
+  const bool tail = (a.K & 255) != 0;
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
+  const uint32_t lane16 = lane * 16;
+  const char* xb = reinterpret_cast<const char*>(w.q) + (size_t)row0 * a.ldq;
+  const char* wb = reinterpret_cast<const char*>(w.wp);
+  uint32_t xoff[XL / NW];
+  int piece[XL / NW];
+#pragma unroll
+  for (int i = 0; i < XL / NW; ++i) {
+    const int rr = (wave + i * NW) * 4 + (lane >> 4);
+    piece[i] = (lane & 15) ^ (rr & 7);
+    xoff[i] = (uint32_t)((min(row0 + rr, a.rows - 1) - row0) * a.ldq + piece[i] * 16);  // rows past the end: the last row
+  }
+  auto issue = [&](int s, uint32_t slot) {
+    const bool last = tail && s == KC - 1;  // pieces past the row's end read its last one and are multiplied as zeros
+#pragma unroll
+    for (int i = 0; i < XL / NW; ++i)
+      load_lds16(slot + (wave + i * NW) * 1024, xb + (size_t)s * 256,
+                 xoff[i] - (last ? (uint32_t)max(0, s * 256 + piece[i] * 16 - (a.ldq - 16)) : 0u));
+#pragma unroll
+    for (int i = 0; i < WL / NW; ++i) {
+      const int t = wave + i * NW;
+      load_lds16(slot + (XL + t) * 1024, wb + ((size_t)min(strip0 + t, nstrips - 1) * KC + s) * 1024, lane16);
+    }
+  };
+  i32x4 acc[FN][FM];
+#pragma unroll
+  for (int u = 0; u < FN; ++u)
+#pragma unroll
+    for (int t = 0; t < FM; ++t) acc[u][t] = (i32x4){0, 0, 0, 0};
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < KC) issue(s, lds0 + s * STAGE);
+  const uint32_t xrd = lds0 + (wm * FM * 16 + m) * 256;
+  const uint32_t wrd = lds0 + (XL + wn * FN) * 1024 + lane16;
+  uint32_t so = 0, si = (NST - 1) * STAGE;
+  for (int s = 0; s < KC; ++s) {
+    if (NST == 2 || s + NST - 2 >= KC) wait_loads<0>();
+    else wait_loads<(NST - 2) * LPW>();
+    __builtin_amdgcn_s_barrier();
+    if (s + NST - 1 < KC) issue(s + NST - 1, lds0 + si);
+    uint32_t wv[FN][4];
+#pragma unroll
+    for (int u = 0; u < FN; ++u) {
+      const uint4 v = lds16_at(wrd + so + u * 1024);
+      wv[u][0] = v.x; wv[u][1] = v.y; wv[u][2] = v.z; wv[u][3] = v.w;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint4 xf[FM];
+#pragma unroll
+      for (int t = 0; t < FM; ++t) xf[t] = lds16_at(xrd + so + t * 4096 + (uint32_t)((4 * j + g) ^ (m & 7)) * 16);
+      if (tail && s == KC - 1) {
+        const int left = a.K - (256 * s + 64 * j + 16 * g);  // codes of this piece inside the row (K: a multiple of 8)
+#pragma unroll
+        for (int t = 0; t < FM; ++t) {
+          if (left < 16) xf[t].z = xf[t].w = 0;
+          if (left < 8) xf[t].x = xf[t].y = 0;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < FN; ++u) {
+        i32x4 av;
+        av[0] = (int)(wv[u][j] & 0x03030303u);
+        av[1] = (int)((wv[u][j] >> 2) & 0x03030303u);
+        av[2] = (int)((wv[u][j] >> 4) & 0x03030303u);
+        av[3] = (int)((wv[u][j] >> 6) & 0x03030303u);
+#pragma unroll
+        for (int t = 0; t < FM; ++t) {
+          i32x4 bv;
+          bv[0] = (int)xf[t].x; bv[1] = (int)xf[t].y; bv[2] = (int)xf[t].z; bv[3] = (int)xf[t].w;
+          acc[u][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, acc[u][t], 0, 0, 0);
+        }
+      }
+    }
+    so = so + STAGE == NST * STAGE ? 0 : so + STAGE;
+    si = si + STAGE == NST * STAGE ? 0 : si + STAGE;
+  }
+
+  const int sbase = strip0 + wn * FN;
+#pragma unroll
+  for (int t = 0; t < FM; ++t) {
+    const int b = row0 + wm * FM * 16 + t * 16 + m;
+    if (b >= a.rows) continue;
+    const float s = w.s[b];
+    const int sq = w.sumq[b];
+    int pos = 0;
+    size_t row = (size_t)b;
+    if (ROPE) {
+      const int seq = b / a.S;
+      pos = (a.pos_dev ? *a.pos_dev : a.pos) + (b - seq * a.S);
+      if (pos < 0 || pos >= a.Tmax) continue;
+      if (which > 0) row = (size_t)seq * a.Tmax + pos;
+    }
+#pragma unroll
+    for (int u = 0; u < FN; ++u) {
+      const int r0 = (sbase + u) * 16 + 4 * g;
+      if (r0 >= w.N) continue;
+      int ai[4];
+      float v[4];
+      bit_scale4(acc[u][t], sq, s, w.gamma, ai, v);
+      if (ROPE) {
+        if (which < 2) {
+          const int d = r0 % a.Dh;
+          const uint32_t c2 = *reinterpret_cast<const uint32_t*>(a.cos + (size_t)pos * (a.Dh >> 1) + (d >> 1));
+          const uint32_t s2 = *reinterpret_cast<const uint32_t*>(a.sin + (size_t)pos * (a.Dh >> 1) + (d >> 1));
+#pragma unroll
+          for (int pr = 0; pr < 2; ++pr) {
+            const float c = pr ? hi_bf(c2) : lo_bf(c2), sn = pr ? hi_bf(s2) : lo_bf(s2);
+            const float e = v[2 * pr], od = v[2 * pr + 1];
+            v[2 * pr] = __fsub_rn(__fmul_rn(e, c), __fmul_rn(od, sn));
+            v[2 * pr + 1] = __fadd_rn(__fmul_rn(e, sn), __fmul_rn(od, c));
+          }
+        }
+        *reinterpret_cast<uint2*>(w.out + row * w.ldo + r0) = make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
+        continue;
+      }
+      if (a.wide) {
+        if (w.resid) {
+          const uint2 rv = *reinterpret_cast<const uint2*>(w.resid + (size_t)b * w.ldr + r0);
+          v[0] = lo_bf(rv.x) + v[0]; v[1] = hi_bf(rv.x) + v[1]; v[2] = lo_bf(rv.y) + v[2]; v[3] = hi_bf(rv.y) + v[3];
+        }
+        *reinterpret_cast<uint2*>(w.out + (size_t)b * w.ldo + r0) = make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
+        if (w.acc_out) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) w.acc_out[(size_t)b * w.ldacc + r0 + i] = ai[i];
+        }
+        continue;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int n = r0 + i;
+        if (n >= w.N) continue;
+        if (w.acc_out) w.acc_out[(size_t)b * w.ldacc + n] = ai[i];
+        float y = v[i];
+        if (w.resid) y = bf2f(w.resid[(size_t)b * w.ldr + n]) + y;
+        w.out[(size_t)b * w.ldo + n] = f2bf(y);
+      }
+    }
+  }
+}
+
+template <int WM, int WN, int FM, int FN, int NST, bool ROPE>
+int launch_ternary_tile(TernaryArgs& a, hipStream_t st) {
+  constexpr int TM = WM * FM * 16, TS = WN * FN, LDS = NST * (TM / 4 + TS) * 1024;
+  a.MT = (a.rows + TM - 1) / TM;
+  a.NT = 0;
+  for (TernarySet& s : a.set) {
+    s.tiles = ((s.N + 15) / 16 + TS - 1) / TS;
+    a.NT += s.tiles;
+  }
+  const int64_t tiles = (int64_t)a.MT * a.NT;
+  if (tiles > INT32_MAX - 8) return OHARA_ESIZE;
+  if (LDS > 64 * 1024)
+    (void)hipFuncSetAttribute((const void*)ternary_tile_kernel<WM, WN, FM, FN, NST, ROPE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  hipLaunchKernelGGL((ternary_tile_kernel<WM, WN, FM, FN, NST, ROPE>), dim3((unsigned)(tiles + 7) / 8 * 8), dim3(WM * WN * 64), LDS, st, a);
+  return ohara_launch_status();
+}
+
+// 64 x 64 while that leaves CUs with a tile or two, 128 x 128 (half the LDS traffic a product) for more.
+template <bool ROPE>
+int launch_ternary(TernaryArgs& a, hipStream_t st) {
+  int64_t strips = 0;
+  for (const TernarySet& s : a.set) strips += (s.N + 15) / 16;
+  if (((int64_t)a.rows + 127) / 128 * ((strips + 7) / 8) >= 384) return launch_ternary_tile<2, 4, 4, 2, 2, ROPE>(a, st);
+  return launch_ternary_tile<2, 2, 2, 2, 3, ROPE>(a, st);
+}
+
+// What the tiled kernel asks for: codes on 16 bytes, a tile of them addressed with 32 bits.
+bool ternary_tile_ok(const int8_t* q, int ldq) { return ((uintptr_t)q & 15) == 0 && (ldq & 15) == 0 && ldq >= 16 && ldq <= (1 << 23); }
+
 template <bool FUSED>
 int launch_bit(const BitArgs& a0, hipStream_t st) {
   const int strips = (a0.N + 15) / 16;
@@ -643,7 +891,69 @@ int ohara_gemv_ternary_i8(const int8_t* q, int ldq, const float* s, const int32_
   a.q = q; a.ldq = ldq; a.s = s; a.sumq = sumq;
   a.B = rows; a.N = n; a.K = k; a.out = out; a.ldo = ldo; a.resid = resid; a.ldr = ldr;
   a.acc_out = acc_out; a.ldacc = ldacc;
+  if (rows > 64 && (k & 7) == 0 && ternary_tile_ok(q, ldq)) {
+    TernaryArgs t{};
+    t.rows = rows; t.K = k; t.ldq = ldq;
+    t.set[0].wp = a.wp; t.set[0].q = q; t.set[0].s = s; t.set[0].sumq = sumq; t.set[0].gamma = gamma; t.set[0].N = n;
+    t.set[0].out = out; t.set[0].ldo = ldo; t.set[0].resid = resid; t.set[0].ldr = ldr; t.set[0].acc_out = acc_out; t.set[0].ldacc = ldacc;
+    t.wide = ((n | ldo | (resid ? ldr : 0)) & 3) == 0 && (((uintptr_t)out | (uintptr_t)resid) & 7) == 0;
+    return launch_ternary<false>(t, (hipStream_t)stream);
+  }
   return launch_bit<false>(a, (hipStream_t)stream);
+}
+
+int ohara_act_quant_sets_int8(const uint16_t* x, int ldx, const uint16_t* pre_norm_w, const uint16_t* const* norm_w, int sets,
+                              float eps, int rows, int k, int8_t* q, int ldq, float* s, int32_t* sumq, void* stream) {
+  if (!x || !norm_w || !q || !s || !sumq || rows < 1 || k < 1 || ldx < k || ldq < k || sets < 1 || sets > 3) return OHARA_EINVAL;
+  if ((k & 7) || (ldx & 7) || (ldq & 7)) return OHARA_EINVAL;  // 16-byte loads, 8-byte stores
+  if (k > BL_EPL * 64) return OHARA_ESIZE;
+  QuantSets w{};
+  for (int i = 0; i < sets; ++i) {
+    if (!norm_w[i]) return OHARA_EINVAL;
+    w.nw[i] = norm_w[i];
+  }
+  hipLaunchKernelGGL(act_quant_sets_kernel, dim3((rows + 3) / 4, sets), dim3(256), (size_t)4 * k * 2, (hipStream_t)stream, x, ldx,
+                     pre_norm_w, w, rows, k, eps, q, ldq, s, sumq);
+  return ohara_launch_status();
+}
+
+int ohara_gemm_ternary_sets_i8(const int8_t* q, int ldq, const float* s, const int32_t* sumq, const uint32_t* const* wp,
+                               const float* gamma, int sets, int n, int k, int rows, uint16_t* const* out, int ldo, void* stream) {
+  if (!q || !s || !sumq || !wp || !gamma || !out || sets < 1 || sets > 3 || n < 1 || k < 1 || rows < 1 || ldo < n) return OHARA_EINVAL;
+  if ((k & 7) || ldq < k || !ternary_tile_ok(q, ldq)) return OHARA_EINVAL;
+  TernaryArgs t{};
+  t.rows = rows; t.K = k; t.ldq = ldq;
+  t.wide = ((n | ldo) & 3) == 0;
+  for (int i = 0; i < sets; ++i) {
+    if (!wp[i] || !out[i]) return OHARA_EINVAL;
+    TernarySet& w = t.set[i];
+    w.wp = reinterpret_cast<const uint4*>(wp[i]); w.gamma = gamma[i]; w.N = n; w.out = out[i]; w.ldo = ldo;
+    w.q = q + (size_t)i * rows * ldq; w.s = s + (size_t)i * rows; w.sumq = sumq + (size_t)i * rows;
+    t.wide = t.wide && ((uintptr_t)out[i] & 7) == 0;
+  }
+  return launch_ternary<false>(t, (hipStream_t)stream);
+}
+
+int ohara_gemm_ternary_qkv_rope_append(const int8_t* q, int ldq, const float* s, const int32_t* sumq, const uint32_t* const* wp,
+                                       const float* gamma, int k, int batch, int seq_len, int h, int h_kv, int dh,
+                                       const uint16_t* cos, const uint16_t* sin, int pos, const int32_t* pos_dev, uint16_t* q_out,
+                                       uint16_t* kcache, uint16_t* vcache, int t_max, void* stream) {
+  if (!q || !s || !sumq || !wp || !gamma || !cos || !sin || !q_out || !kcache || !vcache) return OHARA_EINVAL;
+  if (batch < 1 || seq_len < 1 || h < 1 || h_kv < 1 || h % h_kv || dh < 4 || (dh & 3) || t_max < 1 || k < 1) return OHARA_EINVAL;
+  if ((k & 7) || ldq < k || !ternary_tile_ok(q, ldq)) return OHARA_EINVAL;
+  if (!pos_dev && (pos < 0 || pos + seq_len > t_max)) return OHARA_EINVAL;
+  if ((int64_t)batch * seq_len > INT32_MAX) return OHARA_ESIZE;
+  TernaryArgs t{};
+  t.rows = batch * seq_len; t.K = k; t.ldq = ldq;
+  bf16_t* outs[3] = {q_out, kcache, vcache};
+  for (int i = 0; i < 3; ++i) {
+    if (!wp[i]) return OHARA_EINVAL;
+    TernarySet& w = t.set[i];
+    w.wp = reinterpret_cast<const uint4*>(wp[i]); w.gamma = gamma[i]; w.N = (i ? h_kv : h) * dh; w.out = outs[i]; w.ldo = w.N;
+    w.q = q + (size_t)i * t.rows * ldq; w.s = s + (size_t)i * t.rows; w.sumq = sumq + (size_t)i * t.rows;
+  }
+  t.S = seq_len; t.Dh = dh; t.Tmax = t_max; t.pos = pos; t.pos_dev = pos_dev; t.cos = cos; t.sin = sin;
+  return launch_ternary<true>(t, (hipStream_t)stream);
 }
 
 int ohara_bitlinear_bf16(const uint16_t* x, int ldx, const uint16_t* pre_norm_w, const uint16_t* norm_w, float eps,

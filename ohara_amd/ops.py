@@ -430,6 +430,36 @@ def gemv_ternary(q, s, sumq, w: PackedTernary, residual=None, out=None, want_acc
     return (out, acc) if want_acc else out
 
 
+BIT_ROWS = 64  # rows that the fused BitLinear kernels quantise in their own LDS; more are quantised once, then multiplied in tiles
+
+
+def act_quant_sets(x, norm_ws, eps, pre_norm_w=None):
+    """Codes of x (rows, K) for each norm weight (at most three): q (sets, rows, K padded to 16), s and sum q (sets, rows)."""
+    _need(x, BF16, "x")
+    rows, k = x.shape
+    n, ldq = len(norm_ws), (k + 15) // 16 * 16
+    q = torch.empty(n, rows, ldq, dtype=torch.int8, device=x.device)
+    s = torch.empty(n, rows, dtype=torch.float32, device=x.device)
+    sq = torch.empty(n, rows, dtype=torch.int32, device=x.device)
+    nw = (C.c_void_p * n)(*[w.data_ptr() for w in norm_ws])
+    check(lib().ohara_act_quant_sets_int8(_ptr(x), x.stride(0), _ptr(pre_norm_w), nw, n, eps, rows, k, _ptr(q), ldq, _ptr(s),
+                                          _ptr(sq), _stream()), "act_quant_sets")
+    return q, s, sq
+
+
+def bitlinear_many(x, pre_norm_w, projs, eps=1e-5):
+    """Several BitLinears of one width on the same rows (any number), each row quantised once for each -> their outputs.
+    ``projs``: at most three (norm_w, PackedTernary) pairs."""
+    q, s, sq = act_quant_sets(x, [p[0] for p in projs], eps, pre_norm_w)
+    n, rows, width = len(projs), x.shape[0], projs[0][1].n
+    outs = [torch.empty(rows, width, dtype=BF16, device=x.device) for _ in projs]
+    wp = (C.c_void_p * n)(*[p[1].data.data_ptr() for p in projs])
+    gm = (C.c_float * n)(*[p[1].gamma for p in projs])
+    check(lib().ohara_gemm_ternary_sets_i8(_ptr(q), q.stride(1), _ptr(s), _ptr(sq), wp, gm, n, width, x.shape[1], rows,
+                                           (C.c_void_p * n)(*[t.data_ptr() for t in outs]), width, _stream()), "gemm_ternary_sets")
+    return outs
+
+
 def bitlinear(x, norm_w, w: PackedTernary, eps=1e-5, residual=None, out=None, want_acc=False, pre_norm_w=None):
     """Fused BitLinear.forward on rows of x (rows, K) bf16; ``pre_norm_w`` applies a block-level
     RMSNorm to x first, in the same pass."""
@@ -439,6 +469,9 @@ def bitlinear(x, norm_w, w: PackedTernary, eps=1e-5, residual=None, out=None, wa
         raise ValueError(f"x has {k} columns, weight expects {w.k}")
     if out is None:
         out = torch.empty(rows, w.n, dtype=BF16, device=x.device)
+    if rows > BIT_ROWS:
+        q, s, sq = act_quant_sets(x, [norm_w], eps, pre_norm_w)
+        return gemv_ternary(q[0], s[0], sq[0], w, residual, out, want_acc)
     acc = torch.empty(rows, w.n, dtype=torch.int32, device=x.device) if want_acc else None
     check(lib().ohara_bitlinear_bf16(_ptr(x), x.stride(0), _ptr(pre_norm_w), _ptr(norm_w), eps, _ptr(w.data), w.n, w.k, w.gamma, rows,
                                      _ptr(residual), 0 if residual is None else residual.stride(0), _ptr(out),
@@ -448,8 +481,8 @@ def bitlinear(x, norm_w, w: PackedTernary, eps=1e-5, residual=None, out=None, wa
 
 def bitlinear_qkv_rope_append(x, pre_norm_w, projs, eps, h, h_kv, dh, cos, sin, pos, kcache, vcache, q_out=None,
                               pos_dev=None, seq_len=1):
-    """The query / key / value BitLinears of one layer on rows of x (rows <= 64) in one launch, with
-    rotary + cache append.  ``projs``: three (norm_w, PackedTernary) pairs.  Returns q (rows, h*dh)."""
+    """The query / key / value BitLinears of one layer on rows of x in one launch (more than 64 rows: behind one that quantises
+    them), with rotary + cache append.  ``projs``: three (norm_w, PackedTernary) pairs.  Returns q (rows, h*dh)."""
     _need(x, BF16, "x")
     rows, k = x.shape
     if q_out is None:
@@ -457,6 +490,13 @@ def bitlinear_qkv_rope_append(x, pre_norm_w, projs, eps, h, h_kv, dh, cos, sin, 
     nw = (C.c_void_p * 3)(*[p[0].data_ptr() for p in projs])
     wp = (C.c_void_p * 3)(*[p[1].data.data_ptr() for p in projs])
     gm = (C.c_float * 3)(*[p[1].gamma for p in projs])
+    if rows > BIT_ROWS:
+        q, s, sq = act_quant_sets(x, [p[0] for p in projs], eps, pre_norm_w)
+        check(lib().ohara_gemm_ternary_qkv_rope_append(
+            _ptr(q), q.stride(1), _ptr(s), _ptr(sq), wp, gm, k, rows // seq_len, seq_len, h, h_kv, dh, _ptr(cos), _ptr(sin),
+            int(pos), _ptr(pos_dev), _ptr(q_out), _ptr(kcache), _ptr(vcache), kcache.shape[1], _stream()),
+            "gemm_ternary_qkv_rope_append")
+        return q_out
     check(lib().ohara_bitlinear_qkv_rope_append_bf16(
         _ptr(x), x.stride(0), _ptr(pre_norm_w), eps, k, nw, wp, gm, rows // seq_len, seq_len, h, h_kv, dh, _ptr(cos),
         _ptr(sin), int(pos), _ptr(pos_dev), _ptr(q_out), _ptr(kcache), _ptr(vcache), kcache.shape[1], _stream()),

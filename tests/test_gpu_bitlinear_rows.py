@@ -1,0 +1,69 @@
+"""BitLinears over many rows: quantised once and multiplied in tiles, against the same rows in calls of at most 64 (the kernels that
+quantise in their own LDS) and against whole-number products on the CPU.  Everything is compared bit for bit."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def _inputs(cuda, rows, n, k, seed):
+    g = torch.Generator(device=cuda).manual_seed(seed)
+    x = (torch.randn(rows, k, generator=g, device=cuda) * 2).to(BF)
+    t = torch.randint(-1, 2, (n, k), generator=g, device=cuda, dtype=torch.int8)
+    nw = (1 + 0.2 * torch.randn(k, generator=g, device=cuda)).to(BF)
+    pre = (1 + 0.2 * torch.randn(k, generator=g, device=cuda)).to(BF)
+    res = torch.randn(rows, n, generator=g, device=cuda).to(BF)
+    return x, t, nw, pre, res
+
+
+# one tile and parts of one, K below / at / past a step of 256 and off 16, columns off a strip and off four, both tile sizes
+@pytest.mark.parametrize("rows,n,k", [(66, 16, 8), (130, 70, 264), (100, 64, 256), (300, 2048, 5632), (193, 130, 1000),
+                                      (257, 96, 520), (2050, 5632, 2048), (1000, 6150, 136)])
+def test_rows_match_short_calls_and_whole_number_products(cuda, rows, n, k):
+    from ohara_amd import ops
+
+    x, t, nw, pre, res = _inputs(cuda, rows, n, k, rows + n + k)
+    w = ops.pack_ternary(t, 0.013)
+    got, acc = ops.bitlinear(x, nw, w, 1e-5, residual=res, want_acc=True, pre_norm_w=pre)
+    step = 60  # no call of one row: that one is quantised by a whole workgroup, with sums in another order
+    parts = [ops.bitlinear(x[r:r + step], nw, w, 1e-5, residual=res[r:r + step], want_acc=True, pre_norm_w=pre)
+             for r in range(0, rows, step)]
+    assert torch.equal(acc, torch.cat([p[1] for p in parts]))
+    assert torch.equal(got, torch.cat([p[0] for p in parts]))
+    q, s, sq = ops.act_quant_sets(x, [nw], 1e-5, pre)
+    at = torch.arange(0, rows, max(1, rows // 64), device=cuda)
+    codes = q[0, at, :k].cpu().to(torch.int32)
+    assert torch.equal(codes.sum(1).int(), sq[0, at].cpu())
+    assert torch.equal(acc[at].cpu(), codes @ t.cpu().to(torch.int32).t())
+
+
+def test_sets_share_rows_and_keep_their_own_codes(cuda):
+    from ohara_amd import ops
+
+    x, t, nw, pre, _ = _inputs(cuda, 211, 352, 264, 3)
+    x2, t2, nw2, _, _ = _inputs(cuda, 211, 352, 264, 4)
+    a, b = (ops.pack_ternary(t, 0.02), ops.pack_ternary(t2, 0.005))
+    one, two = ops.bitlinear_many(x, pre, [(nw, a), (nw2, b)], 1e-5)
+    assert torch.equal(one, ops.bitlinear(x, nw, a, 1e-5, pre_norm_w=pre))
+    assert torch.equal(two, ops.bitlinear(x, nw2, b, 1e-5, pre_norm_w=pre))
+
+
+@pytest.mark.parametrize("batch,seq,h,h_kv,dh", [(1, 70, 2, 2, 64), (3, 50, 4, 2, 128), (2, 129, 2, 1, 8)])
+def test_query_key_value_with_rotary_and_append(cuda, batch, seq, h, h_kv, dh):
+    from ohara_amd import ops
+    from ohara_amd.llama import rope_tables
+
+    k, t_max, pos = 264, 512, 37
+    x, _, _, pre, _ = _inputs(cuda, batch * seq, 8, k, 9)
+    projs = []
+    for i, heads in enumerate((h, h_kv, h_kv)):
+        _, t, nw, _, _ = _inputs(cuda, 1, heads * dh, k, 20 + i)
+        projs.append((nw, ops.pack_ternary(t, 0.01 * (i + 1))))
+    cos, sin = (c.to(cuda, BF) for c in rope_tables(dh, t_max, 10000.0))
+    kc, vc, kr, vr = (torch.zeros(batch, t_max, h_kv, dh, device=cuda, dtype=BF) for _ in range(4))
+    got = ops.bitlinear_qkv_rope_append(x, pre, projs, 1e-5, h, h_kv, dh, cos, sin, pos, kc, vc, seq_len=seq)
+    want, kk, vv = (ops.bitlinear(x, nw, w, 1e-5, pre_norm_w=pre) for nw, w in projs)
+    ops.rope_append(want, kk, vv, batch, seq, h, h_kv, dh, cos, sin, pos, kr, vr)
+    assert torch.equal(got, want) and torch.equal(kc, kr) and torch.equal(vc, vr)
