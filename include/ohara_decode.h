@@ -359,6 +359,13 @@ int ohara_moe_experts_gate_up(const uint16_t* x, int ldx, const uint16_t* wp_gat
 int ohara_moe_experts_down(const uint16_t* act, int ld_act, const uint16_t* wp_down, int64_t expert_stride_bytes,
                            int n_experts, int d, int hidden, int k, const int32_t* offsets, const int32_t* pair_of,
                            const uint16_t* expert_w, uint16_t* y, int ldy, void* stream);
+/* The same two for n_pairs pairs whose number the host knows: from 12 pairs an expert on, in tiles of an expert's pairs. */
+int ohara_moe_experts_gate_up_many(const uint16_t* x, int ldx, const uint16_t* wp_gate_up, int64_t expert_stride_bytes,
+                                   int n_experts, int hidden, int d, int k, int n_pairs, const int32_t* offsets,
+                                   const int32_t* pair_of, uint16_t* act, int ld_act, void* stream);
+int ohara_moe_experts_down_many(const uint16_t* act, int ld_act, const uint16_t* wp_down, int64_t expert_stride_bytes, int n_experts,
+                                int d, int hidden, int k, int n_pairs, const int32_t* offsets, const int32_t* pair_of,
+                                const uint16_t* expert_w, uint16_t* y, int ldy, void* stream);
 int ohara_moe_combine(const uint16_t* y, int ldy, const int32_t* expert_idx, const int32_t* pos_of, int n_tokens, int k,
                       const uint16_t* shared, int ld_shared, const uint16_t* resid, int ldr, uint16_t* out, int ldo, int d,
                       void* stream);

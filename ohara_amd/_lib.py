@@ -155,6 +155,8 @@ _PROTOS = {
     "ohara_moe_experts_gate_up_shared": (_i, [_p, _i, _p, _i64, _i, _i, _i, _i, _p, _p, _p, _i, _p, _i, _i, _p, _i, _p]),
     "ohara_moe_experts_down_shared": (_i, [_p, _i, _p, _i64, _i, _i, _i, _i, _p, _p, _p, _p, _i, _p, _i, _i, _p, _i, _p, _i,
                                            _p]),
+    "ohara_moe_experts_gate_up_many": (_i, [_p, _i, _p, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _i, _p]),
+    "ohara_moe_experts_down_many": (_i, [_p, _i, _p, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _p, _i, _p]),
     "ohara_moe_combine": (_i, [_p, _i, _p, _p, _i, _i, _p, _i, _p, _i, _p, _i, _i, _p]),
     "ohara_llama_forward": (_i, [C.POINTER(OharaModel), C.POINTER(OharaDecodeState), _i, _i, _i, _i, _i, _p]),
     "ohara_linear_bias_bf16": (_i, [_p, _i, _p, _i, _i, _p, _i, _i, _p, _i, _p, _i, _p, _i, _p]),

@@ -15,7 +15,7 @@
 // the chunk and carries, at bit 8*t + 2*r, the code T+1 of column 256*chunk + 64*j + 16*g + 4*r + t,
 // so "(dword >> 2r) & 0x03030303" is register r of the MFMA operand.  Codes are 0..2, hence
 // acc = sum q*code - sum q, the second term being one number per token.
-#include "common.h"
+#include "lds_tile.h"
 
 namespace {
 
@@ -582,7 +582,7 @@ __global__ __launch_bounds__(256) void rope_append_kernel(bf16_t* q, const bf16_
 }
 
 // ---- many rows ---------------------------------------------------------------------------------
-// Up to three BitLinears (their own codes, weights and outputs) as one launch of the tiled product of gemm_tile.hip on
+// Up to three BitLinears (their own codes, weights and outputs) as one launch of the tiled product of lds_tile.h on
 // v_mfma_i32_16x16x64_i8: a workgroup owns TM rows of codes x TS strips, steps of 256 columns travel straight into LDS
 // (codes: 256-byte row segments with their 16-byte pieces permuted by the row, weights: one 1 KiB tile a strip), a
 // wave unpacks a strip's tile into operands once for its FM row blocks.  The sums are whole numbers, so neither the tile nor the

@@ -302,17 +302,6 @@ __device__ __forceinline__ void wait_own_stores() {
   asm volatile("" ::: "memory");
 }
 
-// 16 bytes per lane from sbase + voff to LDS byte lds + 16 * lane.  (Assembly: behind the builtin the compiler waits for
-// every such load in flight before any LDS read, which would undo the ring.  No vector register is written; the waits
-// are wait_loads below; M0 holds nothing of the compiler's: none of the kernels that use this has another instruction that reads it.)
-__device__ __forceinline__ void load_lds16(uint32_t lds, const void* sbase, uint32_t voff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(sbase) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_loads() {  // until at most N of this wave's loads are in flight
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // x * sigmoid(x) with the hardware exponential and reciprocal (v_exp_f32, v_rcp_f32: about 1 ulp
 // each; every use rounds the result to bf16 right away).  The library expf and the IEEE division
 // are some forty instructions, which sixteen fragments per thread in the tiled GEMM's SwiGLU

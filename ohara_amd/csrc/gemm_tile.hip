@@ -1,16 +1,6 @@
 // Tiled MFMA GEMM for the batched (prefill) projections: y = epi(x W^T) with many rows.
 //
-// A workgroup owns a tile of TM activation rows x TS packed 16-row weight strips; its WM x WN waves own FM x FN
-// fragments of v_mfma_f32_16x16x32_bf16 each (weights = A operand, activations = B operand, exactly as in the skinny
-// kernel, so the epilogues are shared).  K is walked in order, KH MFMA steps of 32 at a time, so the sums do not depend
-// on the tile.  Both operands of a step travel straight from global memory into LDS (global_load_lds, 16 bytes a lane: no
-// registers held in flight, NST - 1 steps ahead) and every wave reads its fragments from there:
-//   * a packed weight tile (strip, k-step) is 1 KiB in lane order: one load, and a conflict-free 16-byte read;
-//   * a load of activations is 1 KiB of whole row segments of 64 KH bytes; the 16-byte pieces of a row are permuted by the
-//     row's number on their way in (each lane chooses its global address, the LDS side is always in lane order), which
-//     is what makes the fragment reads of sixteen rows conflict-free without padding.
-// One barrier per step: it says that the step's loads have arrived (every wave waits for its own first) and that the slot
-// of the step before is free for the next loads.
+// The walk over K is tile_product (lds_tile.h); the sums do not depend on the tile.
 //
 // What bounds it: in large tiles the LDS side and the matrix pipe together (a step of 128 x 192 x 64 takes 0.72 us where its
 // products alone take 0.41 us at the 2.0 GHz the chip holds under them); in small ones the chain barrier - read - multiply
@@ -27,29 +17,14 @@
 // Replaces the F.linear calls of ohara/models/llama.py:84-86,142,322 and
 // ohara/modules/mlp.py:152 when the call carries more than 64 rows.
 #include "gemm_epilogue.h"
-
-#include <type_traits>
+#include "lds_tile.h"
 
 namespace {
-
-template <int WM_, int WN_, int FM_, int FN_, int KH_, int NST_>
-struct Tile {
-  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, KH = KH_, NST = NST_;
-  static constexpr int NW = WM * WN;                       // waves
-  static constexpr int TM = WM * FM * 16, TS = WN * FN;    // rows, strips
-  static constexpr int RPL = 16 / KH;                      // activation rows of a 1 KiB load
-  static constexpr int XL = TM / RPL, WL = TS * KH;        // 1 KiB loads of a step
-  static constexpr int LPW = (XL + WL) / NW;               // of one wave
-  static constexpr int STAGE = (XL + WL) * 1024, LDS = NST * STAGE;
-  static_assert(XL % NW == 0 && WL % NW == 0, "loads split evenly over the waves");
-  static_assert((KH == 2 || KH == 4) && LDS <= 160 * 1024, "");
-};
 
 // ALIGNED: activation rows start on 16 bytes and a tile of them spans less than 4 GiB (false: through registers, any)
 template <int EPI, class C, bool ALIGNED>
 __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, int MT, int NT, int nstrips) {
-  constexpr int FM = C::FM, FN = C::FN, KH = C::KH, NST = C::NST, NW = C::NW, XL = C::XL, WL = C::WL, LPW = C::LPW;
-  constexpr int STAGE = C::STAGE, KB = 32 * KH, GM = 8;
+  constexpr int FM = C::FM, FN = C::FN, GM = 8;
   extern __shared__ __align__(16) unsigned char smem[];
   const int T = MT * NT;
   const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
@@ -62,89 +37,11 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / C::WN, wn = wave % C::WN;
   const int m = lane & 15, g = lane >> 4;
-  const int KS = (a.K + 31) >> 5, nsteps = (KS + KH - 1) / KH;
-  const bool tail = a.K % KB != 0;                         // the last step is not full
-
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
-  const char* xb = reinterpret_cast<const char*>(a.x + (size_t)row0 * a.ldx);
-  const char* wb = reinterpret_cast<const char*>(a.wp);
-  const uint32_t lane16 = lane * 16;
-  const int lrow = lane / (4 * KH);                        // this lane's row of a load
-  typedef typename std::conditional<ALIGNED, uint32_t, uint64_t>::type offset_t;
-  offset_t xoff[XL / NW];                                  // rows past the end read the last row
-  int piece[XL / NW];                                      // the 16-byte piece of its row that this lane fetches
+  XOffsets<C, ALIGNED> x;
 #pragma unroll
-  for (int i = 0; i < XL / NW; ++i) {
-    const int rr = (wave + i * NW) * C::RPL + lrow;
-    piece[i] = (lane & (4 * KH - 1)) ^ (rr & 7);
-    xoff[i] = ((offset_t)(min(row0 + rr, a.B - 1) - row0) * a.ldx + piece[i] * 8) * 2;
-  }
-  auto issue = [&](int s, uint32_t slot) {
-    const char* xs = xb + (size_t)s * (2 * KB);
-    const bool last = tail && s == nsteps - 1;
-#pragma unroll
-    for (int i = 0; i < XL / NW; ++i) {
-      const uint32_t dst = slot + (wave + i * NW) * 1024;
-      // pieces past K read the row's last piece and are multiplied by zero
-      const uint32_t back = last ? (uint32_t)max(0, s * KB + piece[i] * 8 - (a.K - 8)) * 2 : 0u;
-      if (ALIGNED) {
-        load_lds16(dst, xs, xoff[i] - back);
-      } else {
-        const uint4 v = ldg16(xs + xoff[i] - back);
-        *(OHARA_LDS u32x4*)(uintptr_t)(dst + lane16) = (u32x4){v.x, v.y, v.z, v.w};
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < WL / NW; ++i) {
-      const int t = wave + i * NW;  // strip t / KH, k-step t % KH; past the end: the last one, never used
-      const int strip = min(strip0 + t / KH, nstrips - 1), j = min(KH * s + t % KH, KS - 1);
-      load_lds16(slot + (XL + t) * 1024, wb + ((size_t)strip * KS + j) * 1024, lane16);
-    }
-  };
-
+  for (int i = 0; i < C::XPW; ++i) x.set(i, wave, lane, (typename XOffsets<C, ALIGNED>::type)(min(row0 + x.row(i, wave, lane), a.B - 1) - row0) * a.ldx);
   f32x4 acc[FN][FM];
-#pragma unroll
-  for (int u = 0; u < FN; ++u)
-#pragma unroll
-    for (int t = 0; t < FM; ++t) acc[u][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
-    if (s < nsteps) issue(s, lds0 + s * STAGE);
-  const uint32_t xrd = lds0 + (wm * FM * 16 + m) * (64 * KH);
-  const uint32_t wrd = lds0 + (XL + wn * FN * KH) * 1024 + lane16;
-  uint32_t so = 0, si = (NST - 1) * STAGE;
-  for (int s = 0; s < nsteps; ++s) {
-    if (!ALIGNED) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    else if (NST == 2 || s + NST - 2 >= nsteps) wait_loads<0>();
-    else wait_loads<(NST - 2) * LPW>();
-    __builtin_amdgcn_s_barrier();
-    if (s + NST - 1 < nsteps) issue(s + NST - 1, lds0 + si);
-#pragma unroll
-    for (int jj = 0; jj < KH; ++jj) {
-      // all fragments of a k-step into registers of their own before its products
-      uint4 xf[FM], wf[FN];
-      const uint32_t sw = (uint32_t)((4 * jj + g) ^ (m & 7)) * 16;
-#pragma unroll
-      for (int u = 0; u < FN; ++u) wf[u] = lds16_at(wrd + so + (u * KH + jj) * 1024);
-#pragma unroll
-      for (int t = 0; t < FM; ++t) xf[t] = lds16_at(xrd + so + t * (1024 * KH) + sw);
-      if (tail && s == nsteps - 1) {
-        const bool in = KB * s + 32 * jj + 8 * g < a.K;
-#pragma unroll
-        for (int t = 0; t < FM; ++t) xf[t] = in ? xf[t] : make_uint4(0, 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int t = 0; t < FM; ++t)
-#pragma unroll
-        for (int u = 0; u < FN; ++u)
-          acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[u]),
-                                                              __builtin_bit_cast(bf16x8, xf[t]), acc[u][t], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    so = so + STAGE == NST * STAGE ? 0 : so + STAGE;
-    si = si + STAGE == NST * STAGE ? 0 : si + STAGE;
-  }
+  tile_product<C, ALIGNED>(acc, reinterpret_cast<const char*>(a.x + (size_t)row0 * a.ldx), x, a.wp, strip0, nstrips, a.K, wave, lane, smem);
   const int rbase = row0 + wm * FM * 16, sbase = strip0 + wn * FN;
 
   // A thread finishes FM * FN fragments.  What their epilogues read (residual rows, biases, rotary

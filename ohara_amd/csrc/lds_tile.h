@@ -1,0 +1,139 @@
+// The tiled product of the many-row kernels (gemm_tile.hip, moe.hip): activations x packed weights on MFMA, both operands
+// through LDS.
+//
+// A workgroup owns a tile of TM activation rows x TS packed 16-row weight strips; its WM x WN waves own FM x FN
+// fragments of v_mfma_f32_16x16x32_bf16 each (weights = A operand, activations = B operand, as in the skinny kernels, so
+// the epilogues are shared).  K is walked in order, KH MFMA steps of 32 at a time.  Both operands of a step travel straight
+// from global memory into LDS (global_load_lds, 16 bytes a lane: no registers held in flight, NST - 1 steps ahead) and
+// every wave reads its fragments from there:
+//   * a packed weight tile (strip, k-step) is 1 KiB in lane order: one load, and a conflict-free 16-byte read;
+//   * a load of activations is 1 KiB of whole row segments of 64 KH bytes; the 16-byte pieces of a row are permuted by the
+//     row's number on their way in (each lane chooses its global address, the LDS side is always in lane order), which
+//     is what makes the fragment reads of sixteen rows conflict-free without padding.
+// One barrier per step: it says that the step's loads have arrived (every wave waits for its own first) and that the slot
+// of the step before is free for the next loads.
+#pragma once
+#include "common.h"
+
+#include <type_traits>
+
+namespace {
+
+// 16 bytes per lane from sbase + voff to LDS byte lds + 16 * lane.  (Assembly: behind the builtin the compiler waits for
+// every such load in flight before any LDS read, which would undo the ring.  No vector register is written; the waits
+// are wait_loads below; M0 holds nothing of the compiler's: none of the kernels that use this has another instruction that reads it.)
+__device__ __forceinline__ void load_lds16(uint32_t lds, const void* sbase, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(sbase) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() {  // until at most N of this wave's loads are in flight
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <int WM_, int WN_, int FM_, int FN_, int KH_, int NST_>
+struct Tile {
+  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, KH = KH_, NST = NST_;
+  static constexpr int NW = WM * WN;                       // waves
+  static constexpr int TM = WM * FM * 16, TS = WN * FN;    // rows, strips
+  static constexpr int RPL = 16 / KH;                      // activation rows of a 1 KiB load
+  static constexpr int XL = TM / RPL, WL = TS * KH;        // 1 KiB loads of a step
+  static constexpr int XPW = XL / NW, LPW = (XL + WL) / NW;  // of one wave
+  static constexpr int STAGE = (XL + WL) * 1024, LDS = NST * STAGE;
+  static_assert(XL % NW == 0 && WL % NW == 0, "loads split evenly over the waves");
+  static_assert((KH == 2 || KH == 4) && LDS <= 160 * 1024, "");
+};
+
+// Where a lane finds the activations it loads: a byte offset for each of its wave's loads (the caller gives the element offset
+// of the row), and the 16-byte piece of the row that is this lane's.
+template <class C, bool ALIGNED>
+struct XOffsets {
+  typedef typename std::conditional<ALIGNED, uint32_t, uint64_t>::type type;
+  type off[C::XPW];
+  int piece[C::XPW];
+  static __device__ __forceinline__ int row(int i, int wave, int lane) { return (wave + i * C::NW) * C::RPL + lane / (4 * C::KH); }
+  __device__ __forceinline__ void set(int i, int wave, int lane, type row_elements) {
+    piece[i] = (lane & (4 * C::KH - 1)) ^ (row(i, wave, lane) & 7);
+    off[i] = (row_elements + piece[i] * 8) * 2;
+  }
+};
+
+// acc[u][t]: strip u x row block t of this wave.  ALIGNED: activation rows start on 16 bytes (false: through registers, any).
+// K is a multiple of 8; what the last step reads past it are the row's last piece and the strip's last tile, multiplied by zero.
+template <class C, bool ALIGNED>
+__device__ __forceinline__ void tile_product(f32x4 (&acc)[C::FN][C::FM], const char* xb, const XOffsets<C, ALIGNED>& x, const uint4* wp,
+                                             int strip0, int nstrips, int K, int wave, int lane, unsigned char* smem) {
+  constexpr int FM = C::FM, FN = C::FN, KH = C::KH, NST = C::NST, NW = C::NW, XL = C::XL, WL = C::WL, LPW = C::LPW;
+  constexpr int STAGE = C::STAGE, KB = 32 * KH;
+  const int wm = wave / C::WN, wn = wave % C::WN;
+  const int m = lane & 15, g = lane >> 4;
+  const int KS = (K + 31) >> 5, nsteps = (KS + KH - 1) / KH;
+  const bool tail = K % KB != 0;                           // the last step is not full
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
+  const char* wb = reinterpret_cast<const char*>(wp);
+  const uint32_t lane16 = lane * 16;
+  auto issue = [&](int s, uint32_t slot) {
+    const char* xs = xb + (size_t)s * (2 * KB);
+    const bool last = tail && s == nsteps - 1;
+#pragma unroll
+    for (int i = 0; i < C::XPW; ++i) {
+      const uint32_t dst = slot + (wave + i * NW) * 1024;
+      const uint32_t back = last ? (uint32_t)max(0, s * KB + x.piece[i] * 8 - (K - 8)) * 2 : 0u;
+      if (ALIGNED) {
+        load_lds16(dst, xs, x.off[i] - back);
+      } else {
+        const uint4 v = ldg16(xs + x.off[i] - back);
+        *(OHARA_LDS u32x4*)(uintptr_t)(dst + lane16) = (u32x4){v.x, v.y, v.z, v.w};
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < WL / NW; ++i) {
+      const int t = wave + i * NW;  // strip t / KH, k-step t % KH; past the end: the last one, never used
+      const int strip = min(strip0 + t / KH, nstrips - 1), j = min(KH * s + t % KH, KS - 1);
+      load_lds16(slot + (XL + t) * 1024, wb + ((size_t)strip * KS + j) * 1024, lane16);
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < FN; ++u)
+#pragma unroll
+    for (int t = 0; t < FM; ++t) acc[u][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < nsteps) issue(s, lds0 + s * STAGE);
+  const uint32_t xrd = lds0 + (wm * FM * 16 + m) * (64 * KH);
+  const uint32_t wrd = lds0 + (XL + wn * FN * KH) * 1024 + lane16;
+  uint32_t so = 0, si = (NST - 1) * STAGE;
+  for (int s = 0; s < nsteps; ++s) {
+    if (!ALIGNED) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    else if (NST == 2 || s + NST - 2 >= nsteps) wait_loads<0>();
+    else wait_loads<(NST - 2) * LPW>();
+    __builtin_amdgcn_s_barrier();
+    if (s + NST - 1 < nsteps) issue(s + NST - 1, lds0 + si);
+#pragma unroll
+    for (int jj = 0; jj < KH; ++jj) {
+      // all fragments of a k-step into registers of their own before its products
+      uint4 xf[FM], wf[FN];
+      const uint32_t sw = (uint32_t)((4 * jj + g) ^ (m & 7)) * 16;
+#pragma unroll
+      for (int u = 0; u < FN; ++u) wf[u] = lds16_at(wrd + so + (u * KH + jj) * 1024);
+#pragma unroll
+      for (int t = 0; t < FM; ++t) xf[t] = lds16_at(xrd + so + t * (1024 * KH) + sw);
+      if (tail && s == nsteps - 1) {
+        const bool in = KB * s + 32 * jj + 8 * g < K;
+#pragma unroll
+        for (int t = 0; t < FM; ++t) xf[t] = in ? xf[t] : make_uint4(0, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < FM; ++t)
+#pragma unroll
+        for (int u = 0; u < FN; ++u)
+          acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[u]),
+                                                              __builtin_bit_cast(bf16x8, xf[t]), acc[u][t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    so = so + STAGE == NST * STAGE ? 0 : so + STAGE;
+    si = si + STAGE == NST * STAGE ? 0 : si + STAGE;
+  }
+}
+
+}  // namespace

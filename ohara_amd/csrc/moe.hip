@@ -18,6 +18,7 @@
 // The second half is a layer of another kind without a counterpart in the reference: fp32 router over experts and identity
 // outputs with groups, clamped gated units, fp32 weights.  It shares the sort and the expert kernel; its sum over the
 // chosen experts is part of the residual update (OharaMixture, residual_norm.hip).
+#include "lds_tile.h"
 #include "mfma_frag.h"
 
 namespace {
@@ -110,58 +111,9 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const bf16_t* logits, in
 
 // ---- counting sort of the (token, slot) pairs by expert -----------------------------------------
 // offs[e] .. offs[e+1]: pairs of expert e, in token order; pair_of[sorted position] = n*k + j;
-// pos_of[n*k + j] = sorted position.  One workgroup; N*k <= 65536, E <= 1024.
-__global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* idx, int NK, int E, int32_t* offs, int32_t* pair_of,
-                                                        int32_t* pos_of) {
-  __shared__ int cnt[1025];   // histogram, then the next free sorted position of every expert
-  __shared__ __align__(16) int sidx[1024];  // expert ids of the current block of 1024 pairs
-  const int tid = threadIdx.x;
-  for (int e = tid; e <= E; e += 1024) cnt[e] = 0;
-  __syncthreads();
-  for (int p = tid; p < NK; p += 1024) atomicAdd(&cnt[idx[p]], 1);
-  __syncthreads();
-  if (tid == 0) {
-    int run = 0;
-    for (int e = 0; e < E; ++e) {
-      const int c = cnt[e];
-      cnt[e] = run;
-      offs[e] = run;
-      run += c;
-    }
-    offs[E] = run;
-  }
-  __syncthreads();
-  // stable placement, 1024 pairs at a time: a pair's position is its expert's next free slot
-  // plus the number of earlier pairs of the block with the same expert (LDS broadcast reads)
-  for (int p0 = 0; p0 < NK; p0 += 1024) {
-    const int p = p0 + tid;
-    const int e = p < NK ? idx[p] : -1;
-    sidx[tid] = e;
-    __syncthreads();
-    // only earlier pairs count: a wave scans the entries below its last lane, and a wave without a
-    // valid pair scans nothing (entries past the end hold -1 and never match)
-    const int wave_first = tid & ~63;
-    const int n4 = p0 + wave_first < NK ? (min(wave_first + 64, NK - p0) + 3) >> 2 : 0;
-    int rank = 0;
-    const int4* s4 = reinterpret_cast<const int4*>(sidx);
-#pragma unroll 4
-    for (int t4 = 0; t4 < n4; ++t4) {
-      const int4 v = s4[t4];
-      const int t = 4 * t4;
-      rank += (t < tid && v.x == e) + (t + 1 < tid && v.y == e) + (t + 2 < tid && v.z == e) + (t + 3 < tid && v.w == e);
-    }
-    if (e >= 0) {
-      const int o = cnt[e] + rank;
-      pair_of[o] = p;
-      pos_of[p] = o;
-    }
-    __syncthreads();
-    if (e >= 0) atomicAdd(&cnt[e], 1);
-    __syncthreads();
-  }
-}
-
-// The same sort for at most 64 experts and 1024 pairs (decode): a pair's rank among the earlier pairs of
+// pos_of[n*k + j] = sorted position.
+//
+// At most 64 experts and 1024 pairs (decode), one workgroup: a pair's rank among the earlier pairs of
 // its expert is a ballot match inside its wave (six ballots for the six bits of an expert id) plus the
 // counts of the waves before it, instead of a scan over all earlier pairs; the offsets are one wave's scan.
 // COH: idx is read past the caches (other workgroups wrote it in this launch).  wcnt: pairs of expert e in wave w, then the first
@@ -698,7 +650,10 @@ __global__ __launch_bounds__(1024) void moe_router_kernel(RouterArgs<T> a) {
   if (is_last) sort_small_1024<true>(a.idx, a.N * a.top, a.E, a.offs, a.pair_of, a.pos_of, wcnt);
 }
 
-// The sort for many pairs on many workgroups: counts of every block of 1024 pairs, then every block places its own.
+// The sort for many pairs on many workgroups: every block of 1024 pairs places its own.  The counts that it needs - all pairs of an
+// expert, and those in blocks before it - come from a launch that counted each block (HIST), or, without memory for
+// them, from the block's own walk over all ids (30720 pairs: 11 us in all, where one workgroup that walked the blocks one
+// after the other took 700).
 __global__ __launch_bounds__(1024) void moe_count_kernel(const int32_t* idx, int NK, int E, int32_t* hist) {
   __shared__ int cnt[1024];
   const int tid = threadIdx.x, p = blockIdx.x * 1024 + tid;
@@ -709,15 +664,35 @@ __global__ __launch_bounds__(1024) void moe_count_kernel(const int32_t* idx, int
   if (tid < E) hist[(size_t)blockIdx.x * E + tid] = cnt[tid];
 }
 // A pair's rank among the earlier pairs of its expert: a ballot match inside its wave, and the counts of the waves before it.
+template <bool HIST>
 __global__ __launch_bounds__(1024) void moe_place_kernel(const int32_t* idx, int NK, int E, const int32_t* hist, int32_t* offs,
                                                          int32_t* pair_of, int32_t* pos_of) {
   extern __shared__ int wcnt[];  // [16][E]: pairs of an expert in a wave, then the sorted position of that wave's first
-  __shared__ int wsum[16];
+  __shared__ int wsum[16], tot[HIST ? 1 : 1024], bef[HIST ? 1 : 1024];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, blk = blockIdx.x, nb = gridDim.x;
   const int p = blk * 1024 + tid, e = p < NK ? idx[p] : -1;
   for (int i = tid; i < 16 * E; i += 1024) wcnt[i] = 0;
   int total = 0, before = 0;
-  if (tid < E) {
+  if (!HIST) {
+    tot[tid] = bef[tid] = 0;
+    __syncthreads();
+    for (int p0 = tid; p0 < NK; p0 += 4096) {  // four ids in flight
+      int id[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) id[u] = idx[min(p0 + 1024 * u, NK - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (p0 + 1024 * u < NK) {
+          atomicAdd(&tot[id[u]], 1);
+          if (p0 + 1024 * u < blk * 1024) atomicAdd(&bef[id[u]], 1);
+        }
+    }
+    __syncthreads();
+    if (tid < E) {
+      total = tot[tid];
+      before = bef[tid];
+    }
+  } else if (tid < E) {
     for (int b0 = 0; b0 < nb; b0 += 8) {  // eight blocks' counts in flight
       int c[8];
 #pragma unroll
@@ -763,9 +738,9 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(const int32_t* idx, int
   }
 }
 
-// ---- many pairs: tiles of 128 pairs of one expert x 128 packed weight rows -----------------------------
-// The structure of gemm_tile_kernel: weights straight from the packed layout, the activation rows (gathered by pair, or by
-// sorted position) through LDS, double-buffered.
+// ---- many pairs: tiles of pairs of one expert x packed weight rows -------------------------------------
+// tile_product (lds_tile.h) over rows gathered by pair (gated: the token's row) or by sorted position.  An XCD gets a contiguous
+// run of tiles, the weight tiles of one tile of pairs side by side, so an expert's weights and rows stay in its L2.
 struct ExpertTileArgs {
   const uint4* wp;
   size_t expert_stride;   // uint4 per expert
@@ -777,127 +752,134 @@ struct ExpertTileArgs {
   bf16_t* out;
   int ldo;
   OharaGlu glu;
-  const float* pair_w;
+  const float* pair_w;    // X_GLU: factor of a pair's input (null: none)
+  const bf16_t* w;        // X_DOWN: routing weights, pair order
 };
 
-template <int EPI>
-__global__ __launch_bounds__(256, 2) void moe_tile_kernel(ExpertTileArgs a, int NT, int nstrips) {
-  constexpr int TM = 128, TS = 8, KB = 64, LDX = KB + 8;
-  __shared__ __align__(16) bf16_t xs[2][TM][LDX];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m = lane & 15, g = lane >> 4;
-  const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
-  const int tn = q % NT;
-  int tile = (q / NT) * 8 + xcd, e = 0;  // the tile-th tile of pairs: which expert's
-  {
-    bool found = false;
-    for (int e0 = 0; e0 < a.E && !found; e0 += 64) {  // the same for all waves
-      const int c = e0 + lane < a.E ? (a.offs[e0 + lane + 1] - a.offs[e0 + lane] + TM - 1) / TM : 0;
-      const int incl = wave_incl_scan_i(c);
-      const unsigned long long past = __ballot(incl > tile);
-      if (past) {
-        const int l = __ffsll((long long)past) - 1;
-        tile -= __builtin_amdgcn_readlane(incl - c, l);
-        e = e0 + l;
-        found = true;
-      } else {
-        tile -= __builtin_amdgcn_readlane(incl, 63);
-      }
-    }
-    if (!found) return;
-  }
-  const int row0 = a.offs[e] + tile * TM, rows = min(TM, a.offs[e + 1] - row0);
-  const int strip0 = tn * TS + wave * 2, KS = (a.K + 31) >> 5, nsteps = (KS + 1) >> 1;
-  const int lr = tid >> 3, lc = (tid & 7) * 8;
-  const bf16_t* xp[4];
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const int r = row0 + min(p * 32 + lr, rows - 1);
-    xp[p] = a.x + (size_t)(EPI == X_GLU ? a.pair_of[r] / a.top : r) * a.ldx;
-  }
-  auto load_x = [&](int step, uint4* xr) {
-    const int k = step * KB + lc;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) xr[p] = k < a.K ? ldg16(xp[p] + k) : make_uint4(0, 0, 0, 0);
+template <int EPI, class C>
+__global__ __launch_bounds__(C::NW * 64, 2) void moe_tile_kernel(ExpertTileArgs a, int NT, int nstrips) {
+  constexpr bool GATED = EPI == X_SWIGLU || EPI == X_GLU;
+  constexpr int TM = C::TM, FM = C::FM, FN = C::FN;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // tiles of pairs there are (the grid is as large as there could be), and which of them is this workgroup's
+  auto scan = [&](int e0, int& c) {
+    c = e0 + lane < a.E ? (a.offs[e0 + lane + 1] - a.offs[e0 + lane] + TM - 1) / TM : 0;
+    return wave_incl_scan_i(c);
   };
-  auto store_x = [&](int buf, const uint4* xr) {
-#pragma unroll
-    for (int p = 0; p < 4; ++p) *reinterpret_cast<uint4*>(&xs[buf][p * 32 + lr][lc]) = xr[p];
-  };
-  const uint4* w0 = a.wp + (size_t)e * a.expert_stride + (size_t)strip0 * KS * 64 + lane;
-  const uint4* w1 = w0 + (size_t)KS * 64;
-  const bool live0 = strip0 < nstrips, live1 = strip0 + 1 < nstrips;
-  auto load_w = [&](int step, uint4* wv) {
-    const int j = step * 2;
-    wv[0] = (live0 && j < KS) ? ldg16(w0 + (size_t)j * 64) : make_uint4(0, 0, 0, 0);
-    wv[1] = (live0 && j + 1 < KS) ? ldg16(w0 + (size_t)(j + 1) * 64) : make_uint4(0, 0, 0, 0);
-    wv[2] = (live1 && j < KS) ? ldg16(w1 + (size_t)j * 64) : make_uint4(0, 0, 0, 0);
-    wv[3] = (live1 && j + 1 < KS) ? ldg16(w1 + (size_t)(j + 1) * 64) : make_uint4(0, 0, 0, 0);
-  };
-  f32x4 acc[2][8];
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
-#pragma unroll
-    for (int t = 0; t < 8; ++t) acc[u][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  uint4 xr[4], wv[4], wn[4];
-  load_x(0, xr);
-  load_w(0, wv);
-  store_x(0, xr);
-  __syncthreads();
-  for (int s = 0; s < nsteps; ++s) {
-    const int buf = s & 1;
-    const bool more = s + 1 < nsteps;
-    if (more) {
-      load_x(s + 1, xr);
-      load_w(s + 1, wn);
+  int total = 0, c;
+  for (int e0 = 0; e0 < a.E; e0 += 64) total += __builtin_amdgcn_readlane(scan(e0, c), 63);
+  const int T = total * NT;
+  const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3, base = T >> 3, rem = T & 7;
+  if (q >= base + (xcd < rem ? 1 : 0)) return;
+  const int pid = xcd * base + min(xcd, rem) + q;
+  int tile = pid / NT, e = 0;
+  const int tn = pid - tile * NT;
+  for (int e0 = 0; e0 < a.E; e0 += 64) {
+    const int incl = scan(e0, c);
+    const unsigned long long past = __ballot(incl > tile);
+    if (past) {
+      const int l = __ffsll((long long)past) - 1;
+      tile -= __builtin_amdgcn_readlane(incl - c, l);
+      e = e0 + l;
+      break;
     }
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      uint4 bv[8];
-#pragma unroll
-      for (int t = 0; t < 8; ++t) bv[t] = *reinterpret_cast<const uint4*>(&xs[buf][t * 16 + m][jj * 32 + 8 * g]);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        acc[0][t] = mma_bf(wv[jj], bv[t], acc[0][t]);
-        acc[1][t] = mma_bf(wv[2 + jj], bv[t], acc[1][t]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (more) {
-      store_x(buf ^ 1, xr);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) wv[i] = wn[i];
-    }
-    __syncthreads();
+    tile -= __builtin_amdgcn_readlane(incl, 63);
   }
+  e = __builtin_amdgcn_readfirstlane(e);
+  const int row0 = a.offs[e] + tile * TM, rows = min(TM, a.offs[e + 1] - row0), strip0 = tn * C::TS;
+  XOffsets<C, true> x;
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int strip = strip0 + u;
-    if (strip >= nstrips) continue;
+  for (int i = 0; i < C::XPW; ++i) {
+    const int r = row0 + min(x.row(i, wave, lane), rows - 1);
+    x.set(i, wave, lane, (uint32_t)(GATED ? a.pair_of[r] / a.top : r) * (uint32_t)a.ldx);
+  }
+  f32x4 acc[FN][FM];
+  tile_product<C, true>(acc, reinterpret_cast<const char*>(a.x), x, a.wp + (size_t)e * a.expert_stride, strip0, nstrips, a.K, wave, lane, smem);
+  const int r0 = wave / C::WN * FM * 16, sbase = strip0 + wave % C::WN * FN;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      if (t * 16 + m >= rows) continue;
-      bf16_t* o = a.out + (size_t)(row0 + t * 16 + m) * a.ldo;
-      f32x4 c = acc[u][t];
-      if (EPI == X_GLU && a.pair_w) {
-        const float w = a.pair_w[a.pair_of[row0 + t * 16 + m]];
+  for (int t = 0; t < FM; ++t) {
+    const int r = r0 + t * 16 + m;
+    if (r >= rows) continue;
+    bf16_t* o = a.out + (size_t)(row0 + r) * a.ldo;
+    float w = 1.f;
+    if (EPI == X_GLU && a.pair_w) w = a.pair_w[a.pair_of[row0 + r]];
+    if (EPI == X_DOWN) w = bf2f(a.w[a.pair_of[row0 + r]]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) c[i] *= w;
-      }
-      if (EPI == X_GLU) {  // N_out and ldo are multiples of 8
+    for (int u = 0; u < FN; ++u) {
+      const int strip = sbase + u;
+      if (strip >= nstrips) continue;
+      f32x4 c4 = acc[u][t];
+      if (GATED) {
         const int f = strip * 8 + 2 * g;
-        if (f < a.N_out)
-          *reinterpret_cast<uint32_t*>(o + f) = pack_bf(clamped_glu(c[0], c[2], a.glu.limit, a.glu.alpha, a.glu.offset),
-                                                        clamped_glu(c[1], c[3], a.glu.limit, a.glu.alpha, a.glu.offset));
+        float v0, v1;
+        if (EPI == X_GLU) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) c4[i] *= w;
+          v0 = clamped_glu(c4[0], c4[2], a.glu.limit, a.glu.alpha, a.glu.offset);
+          v1 = clamped_glu(c4[1], c4[3], a.glu.limit, a.glu.alpha, a.glu.offset);
+        } else {
+          v0 = rbf(silu_f(rbf(c4[0]))) * rbf(c4[2]);
+          v1 = rbf(silu_f(rbf(c4[1]))) * rbf(c4[3]);
+        }
+        if (f + 1 < a.N_out && !(a.ldo & 1)) {
+          *reinterpret_cast<uint32_t*>(o + f) = pack_bf(v0, v1);
+        } else {
+          if (f < a.N_out) o[f] = f2bf(v0);
+          if (f + 1 < a.N_out) o[f + 1] = f2bf(v1);
+        }
       } else {
         const int f = strip * 16 + 4 * g;
-        if (f < a.N_out) *reinterpret_cast<uint2*>(o + f) = make_uint2(pack_bf(c[0], c[1]), pack_bf(c[2], c[3]));
+        float v[4] = {c4[0], c4[1], c4[2], c4[3]};
+        if (EPI == X_DOWN) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = rbf(v[i]) * w;
+        }
+        if (f + 3 < a.N_out && !(a.ldo & 3)) {
+          *reinterpret_cast<uint2*>(o + f) = make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (f + i < a.N_out) o[f + i] = f2bf(v[i]);
+        }
       }
     }
   }
 }
 
-constexpr int TILE_PAIRS = 64;  // pairs per expert, on average, from which tiles beat streaming the weights per 16 pairs
+typedef Tile<2, 4, 2, 2, 2, 3> E64;   //  64 pairs x 128 packed rows
+typedef Tile<2, 4, 4, 2, 2, 2> E128;  // 128 x 128
+
+template <int EPI, class C>
+int launch_expert_tiles(const ExpertTileArgs& t, int n_pairs, int strips, hipStream_t st) {
+  const int64_t NT = (strips + C::TS - 1) / C::TS, blocks = ((int64_t)n_pairs / C::TM + t.E) * NT;
+  if (blocks > INT32_MAX - 8) return OHARA_ESIZE;
+  if (C::LDS > 64 * 1024)
+    (void)hipFuncSetAttribute((const void*)moe_tile_kernel<EPI, C>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+  hipLaunchKernelGGL((moe_tile_kernel<EPI, C>), dim3((unsigned)(blocks + 7) / 8 * 8), dim3(C::NW * 64), C::LDS, st, t, (int)NT, strips);
+  return ohara_launch_status();
+}
+
+// us for gate/up + down of 64 experts (1024 x 512) at so many pairs an expert, streaming the weights per 16 pairs / tiles of
+// 64 pairs / of 128:
+//     8    24 + 14    23 + 13    23 + 14        64   132 + 81    33 + 23    26 + 17
+//    16    40 + 25    23 + 14    23 + 14       256   504 + 296   66 + 44    57 + 41
+//    48   100 + 62    24 + 15    25 + 17       512   978 + 580  121 + 78    92 + 65
+// (tiles of 32 are behind everywhere: 27 + 18 at 32).  What bounds the tiles: the experts' weights (201 MB) up to 48 pairs, the
+// products' operands through LDS beyond.
+constexpr int TILE_PAIRS = 12;    // pairs an expert, on average, from which tiles beat streaming the weights
+constexpr int LARGE_PAIRS = 56;   // and from which tiles of 128 do those of 64
+
+// false: the rows are not on 16 bytes or not within 4 GiB of each other.
+template <int EPI>
+bool expert_tiles(const ExpertTileArgs& t, int rows, int n_pairs, int strips, hipStream_t st, int* rc) {
+  if (((uintptr_t)t.x & 15) || (t.ldx & 7) || (uint64_t)rows * t.ldx * 2 > UINT32_MAX) return false;
+  *rc = n_pairs >= (int64_t)LARGE_PAIRS * t.E ? launch_expert_tiles<EPI, E128>(t, n_pairs, strips, st)
+                                              : launch_expert_tiles<EPI, E64>(t, n_pairs, strips, st);
+  return true;
+}
+
 
 template <typename T>
 int launch_router(RouterArgs<T> a, int32_t* hist, hipStream_t st) {
@@ -924,24 +906,21 @@ int launch_router(RouterArgs<T> a, int32_t* hist, hipStream_t st) {
     const dim3 blocks((unsigned)((NK + 1023) / 1024));
     hipLaunchKernelGGL(moe_count_kernel, blocks, dim3(1024), 0, st, a.idx, NK, a.E, hist);
     const size_t lds = (size_t)16 * a.E * sizeof(int);
-    if (lds > 60 * 1024) (void)hipFuncSetAttribute((const void*)moe_place_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(moe_place_kernel, blocks, dim3(1024), lds, st, a.idx, NK, a.E, hist, a.offs, a.pair_of, a.pos_of);
+    if (lds > 60 * 1024) (void)hipFuncSetAttribute((const void*)moe_place_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(moe_place_kernel<true>, blocks, dim3(1024), lds, st, a.idx, NK, a.E, hist, a.offs, a.pair_of, a.pos_of);
   }
   return ohara_launch_status();
 }
 
 template <int EPI>
 int launch_experts(ExpertArgs a, int n_pairs, int n_sh, hipStream_t st) {
-  constexpr bool GATED = EPI == X_GLU;
+  constexpr bool GATED = EPI == X_GLU || EPI == X_SWIGLU;
   auto strips_of = [](int n) { return GATED ? 2 * ((n + 7) / 8 * 8) / 16 : (n + 15) / 16; };
   int strips = strips_of(a.N_out);
-  if (n_pairs >= TILE_PAIRS * a.E && !n_sh) {
-    const ExpertTileArgs t{a.wp, a.expert_stride, a.x, a.ldx, a.offs, a.pair_of, a.k, a.E, a.N_out, a.K, a.out, a.ldo, a.glu, a.pair_w};
-    const int NT = (strips + 7) / 8;
-    const int64_t tiles = (n_pairs + 127) / 128 + a.E, blocks = (tiles + 7) / 8 * 8 * NT;
-    if (blocks > INT32_MAX) return OHARA_ESIZE;
-    hipLaunchKernelGGL((moe_tile_kernel<EPI>), dim3((unsigned)blocks), dim3(256), 0, st, t, NT, strips);
-    return ohara_launch_status();
+  if (n_pairs >= (int64_t)TILE_PAIRS * a.E && !n_sh) {
+    const ExpertTileArgs t{a.wp, a.expert_stride, a.x, a.ldx, a.offs, a.pair_of, a.k, a.E, a.N_out, a.K, a.out, a.ldo, a.glu, a.pair_w, a.w};
+    int rc;
+    if (expert_tiles<EPI>(t, GATED ? n_pairs / a.k : n_pairs, n_pairs, strips, st, &rc)) return rc;
   }
   int rows = a.E, ks = (a.K + 31) / 32;
   if (n_sh) {
@@ -1062,9 +1041,12 @@ int ohara_moe_sort_pairs(const int32_t* expert_idx, int n_pairs, int n_experts, 
   if (n_experts <= 64 && n_pairs <= 1024)
     hipLaunchKernelGGL(moe_sort_small_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, expert_idx, n_pairs, n_experts,
                        offsets, pair_of, pos_of);
-  else
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, expert_idx, n_pairs, n_experts, offsets,
-                       pair_of, pos_of);
+  else {
+    const size_t lds = (size_t)16 * n_experts * sizeof(int);
+    if (lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)moe_place_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(moe_place_kernel<false>, dim3((n_pairs + 1023) / 1024), dim3(1024), lds, (hipStream_t)stream, expert_idx, n_pairs,
+                       n_experts, nullptr, offsets, pair_of, pos_of);
+  }
   return ohara_launch_status();
 }
 
@@ -1135,6 +1117,30 @@ int ohara_moe_experts_down(const uint16_t* act, int ld_act, const uint16_t* wp_d
                            const uint16_t* expert_w, uint16_t* y, int ldy, void* stream) {
   return ohara_moe_experts_down_shared(act, ld_act, wp_down, expert_stride_bytes, n_experts, d, hidden, k, offsets, pair_of,
                                        expert_w, y, ldy, nullptr, 0, 0, nullptr, 0, nullptr, 0, stream);
+}
+
+int ohara_moe_experts_gate_up_many(const uint16_t* x, int ldx, const uint16_t* wp_gate_up, int64_t expert_stride_bytes,
+                                   int n_experts, int hidden, int d, int k, int n_pairs, const int32_t* offsets,
+                                   const int32_t* pair_of, uint16_t* act, int ld_act, void* stream) {
+  if (!x || !wp_gate_up || !offsets || !pair_of || !act || n_experts < 1 || k < 1 || n_pairs < 1) return OHARA_EINVAL;
+  if (hidden < 1 || d < 8 || ((d | ldx) & 7) || ldx < d || ld_act < hidden) return OHARA_EINVAL;
+  ExpertArgs a{};
+  a.wp = reinterpret_cast<const uint4*>(wp_gate_up); a.expert_stride = (size_t)expert_stride_bytes / 16;
+  a.x = x; a.ldx = ldx; a.offs = offsets; a.pair_of = pair_of; a.k = k; a.N_out = hidden; a.K = d;
+  a.out = act; a.ldo = ld_act; a.E = n_experts;
+  return launch_experts<X_SWIGLU>(a, n_pairs, 0, (hipStream_t)stream);
+}
+
+int ohara_moe_experts_down_many(const uint16_t* act, int ld_act, const uint16_t* wp_down, int64_t expert_stride_bytes, int n_experts,
+                                int d, int hidden, int k, int n_pairs, const int32_t* offsets, const int32_t* pair_of,
+                                const uint16_t* expert_w, uint16_t* y, int ldy, void* stream) {
+  if (!act || !wp_down || !offsets || !pair_of || !expert_w || !y || n_experts < 1 || k < 1 || n_pairs < 1) return OHARA_EINVAL;
+  if (hidden < 8 || d < 1 || ((hidden | ld_act) & 7) || ld_act < hidden || ldy < d) return OHARA_EINVAL;
+  ExpertArgs a{};
+  a.wp = reinterpret_cast<const uint4*>(wp_down); a.expert_stride = (size_t)expert_stride_bytes / 16;
+  a.x = act; a.ldx = ld_act; a.offs = offsets; a.pair_of = pair_of; a.w = expert_w; a.k = k; a.N_out = d; a.K = hidden;
+  a.out = y; a.ldo = ldy; a.E = n_experts;
+  return launch_experts<X_DOWN>(a, n_pairs, 0, (hipStream_t)stream);
 }
 
 int ohara_moe_combine(const uint16_t* y, int ldy, const int32_t* expert_idx, const int32_t* pos_of, int n_tokens, int k,

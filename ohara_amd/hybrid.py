@@ -130,7 +130,7 @@ class RoutedExperts:
 
     A call returns an ``ops.Mixture``: the residual update sums it."""
 
-    TILE_PAIRS = 64  # pairs per expert from which the experts run in tiles and the shared expert in launches of its own
+    TILE_PAIRS = 16  # pairs per expert from which the experts run in tiles and the shared expert in launches of its own
 
     def __init__(self, experts, router, correction, *, top: int, limit: float, groups: int = 1, keep: int = 1, identity: int = 0, shared=None,
                  alpha: float = 1.702, offset: float = 1.0, sigmoid: bool = False, normalize: bool = True, weigh_input: bool = False,

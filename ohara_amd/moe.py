@@ -78,13 +78,13 @@ class GroupedMoE:
         pos_of = torch.empty(n * k, dtype=torch.int32, device=self.device)
         check(lib().ohara_moe_sort_pairs(_ptr(idx), n * k, E, _ptr(offs), _ptr(pair_of), _ptr(pos_of), st), "moe_sort")
         act = torch.empty(n * k, self.hidden, dtype=BF16, device=self.device)
-        check(lib().ohara_moe_experts_gate_up(_ptr(flat_x), flat_x.stride(0), _ptr(self.wp_gu),
-                                              self.wp_gu.stride(0) * 2, E, self.hidden, self.dim, k, _ptr(offs),
-                                              _ptr(pair_of), _ptr(act), self.hidden, st), "moe_gate_up")
+        check(lib().ohara_moe_experts_gate_up_many(_ptr(flat_x), flat_x.stride(0), _ptr(self.wp_gu),
+                                                   self.wp_gu.stride(0) * 2, E, self.hidden, self.dim, k, n * k, _ptr(offs),
+                                                   _ptr(pair_of), _ptr(act), self.hidden, st), "moe_gate_up")
         y = torch.empty(n * k, self.dim, dtype=BF16, device=self.device)
-        check(lib().ohara_moe_experts_down(_ptr(act), self.hidden, _ptr(self.wp_dn), self.wp_dn.stride(0) * 2, E,
-                                           self.dim, self.hidden, k, _ptr(offs), _ptr(pair_of), _ptr(w), _ptr(y),
-                                           self.dim, st), "moe_down")
+        check(lib().ohara_moe_experts_down_many(_ptr(act), self.hidden, _ptr(self.wp_dn), self.wp_dn.stride(0) * 2, E,
+                                                self.dim, self.hidden, k, n * k, _ptr(offs), _ptr(pair_of), _ptr(w), _ptr(y),
+                                                self.dim, st), "moe_down")
         sh = None
         if self.shared is not None:
             sh = ops.gemm_skinny(ops.gemm_skinny(flat_x, self.shared[0]), self.shared[1])

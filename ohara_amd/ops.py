@@ -99,9 +99,20 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float = 1e-5, out=None) -> to
     return out
 
 
+NORM_ROWS = 64  # rows whose norm the projection kernels redo in every workgroup; more are normed once, for the tiled kernel
+
+
+def _normed(x, norm_w, eps):
+    """(rows, norm weight) for a projection: many rows are normed here."""
+    if norm_w is not None and x.shape[0] > NORM_ROWS:
+        return rmsnorm(x, norm_w, eps), None
+    return x, norm_w
+
+
 def gemm_skinny(x, w: PackedLinear, norm_w=None, eps=1e-5, residual=None, out=None) -> torch.Tensor:
     """y = [rmsnorm(x)] @ W^T (+ residual / SwiGLU epilogue by the packing kind). x: (B, K)."""
     _need(x, BF16, "x")
+    x, norm_w = _normed(x, norm_w, eps)
     b, k = x.shape
     if k != w.k:
         raise ValueError(f"x has {k} columns, weight expects {w.k}")
@@ -149,6 +160,7 @@ def qkv_rope_append(x, wqkv: PackedLinear, norm_w, eps, h, h_kv, dh, cos, sin, p
     """x: (batch*seq_len, K) rows ordered (sequence, position).  ``seq_pos`` (int32, one entry per
     sequence, on the device) gives every sequence its own cache position instead of ``pos``."""
     _need(x, BF16, "x")
+    x, norm_w = _normed(x, norm_w, eps)
     rows = x.shape[0]
     b = rows // seq_len
     if q_out is None:
@@ -178,6 +190,7 @@ def qkv_rope(x, wqkv: PackedLinear, norm_w, eps, h, h_kv, dh, cos, sin, pos, t_m
     """As ``qkv_rope_append`` with the rotated keys and the values returned as (rows, h_kv*dh) row
     buffers instead of written into a cache -> (q, k, v)."""
     _need(x, BF16, "x")
+    x, norm_w = _normed(x, norm_w, eps)
     rows = x.shape[0]
     q = torch.empty(rows, h * dh, dtype=BF16, device=x.device)
     k = torch.empty(rows, h_kv * dh, dtype=BF16, device=x.device)
