@@ -648,7 +648,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void ternary_tile_kernel(TernaryAr
 #pragma unroll
   for (int i = 0; i < XL / NW; ++i) {
     const int rr = (wave + i * NW) * 4 + (lane >> 4);
-    piece[i] = (lane & 15) ^ (rr & 7);
+    piece[i] = (lane ^ rr) & 15;
     xoff[i] = (uint32_t)((min(row0 + rr, a.rows - 1) - row0) * a.ldq + piece[i] * 16);  // rows past the end: the last row
   }
   auto issue = [&](int s, uint32_t slot) {
@@ -689,7 +689,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void ternary_tile_kernel(TernaryAr
     for (int j = 0; j < 4; ++j) {
       uint4 xf[FM];
 #pragma unroll
-      for (int t = 0; t < FM; ++t) xf[t] = lds16_at(xrd + so + t * 4096 + (uint32_t)((4 * j + g) ^ (m & 7)) * 16);
+      for (int t = 0; t < FM; ++t) xf[t] = lds16_at(xrd + so + t * 4096 + (uint32_t)((4 * j + g) ^ m) * 16);
       if (tail && s == KC - 1) {
         const int left = a.K - (256 * s + 64 * j + 16 * g);  // codes of this piece inside the row (K: a multiple of 8)
 #pragma unroll

@@ -9,7 +9,8 @@
 //   * a packed weight tile (strip, k-step) is 1 KiB in lane order: one load, and a conflict-free 16-byte read;
 //   * a load of activations is 1 KiB of whole row segments of 64 KH bytes; the 16-byte pieces of a row are permuted by the
 //     row's number on their way in (each lane chooses its global address, the LDS side is always in lane order), which
-//     is what makes the fragment reads of sixteen rows conflict-free without padding.
+//     is what makes the fragment reads of sixteen rows conflict-free without padding (SQ_LDS_BANK_CONFLICT 0; with 256-byte
+//     segments and the low three bits of the row alone it was two cycles a read, 4 being what one takes).
 // One barrier per step: it says that the step's loads have arrived (every wave waits for its own first) and that the slot
 // of the step before is free for the next loads.
 #pragma once
@@ -52,7 +53,7 @@ struct XOffsets {
   int piece[C::XPW];
   static __device__ __forceinline__ int row(int i, int wave, int lane) { return (wave + i * C::NW) * C::RPL + lane / (4 * C::KH); }
   __device__ __forceinline__ void set(int i, int wave, int lane, type row_elements) {
-    piece[i] = (lane & (4 * C::KH - 1)) ^ (row(i, wave, lane) & 7);
+    piece[i] = (lane ^ row(i, wave, lane)) & (4 * C::KH - 1);
     off[i] = (row_elements + piece[i] * 8) * 2;
   }
 };
@@ -112,7 +113,7 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[C::FN][C::FM], const c
     for (int jj = 0; jj < KH; ++jj) {
       // all fragments of a k-step into registers of their own before its products
       uint4 xf[FM], wf[FN];
-      const uint32_t sw = (uint32_t)((4 * jj + g) ^ (m & 7)) * 16;
+      const uint32_t sw = (uint32_t)((4 * jj + g) ^ (m & (4 * KH - 1))) * 16;
 #pragma unroll
       for (int u = 0; u < FN; ++u) wf[u] = lds16_at(wrd + so + (u * KH + jj) * 1024);
 #pragma unroll
