@@ -4,18 +4,24 @@
 // (ohara/models/llama.py:100-135: the cache mask key_pos <= start_pos + q_idx :109-113, GQA head
 // mapping of repeat_interleave :101-103 by indexing, scale 1/sqrt(Dh), softmax in fp32).
 //
-// A workgroup (4 waves) owns 128 consecutive queries of one (sequence, head); a wave owns 32 of
-// them (two 16-query blocks).  Keys/values are walked in tiles of 64 positions:
-//   S^T = K Q^T   v_mfma_f32_16x16x32_bf16, A = K tile rows from LDS, B = Q rows held in
-//                 registers for the whole walk; a lane ends up with 16 scores of ONE query
-//                 (its column), so the row max/sum need two cross-lane steps only;
-//   O^T += V^T P  the probabilities go from the score accumulators straight into the B operand
-//                 (the k-slot -> position mapping is chosen so that no lane exchange is needed);
-//                 V is transposed on its way into LDS so that the A operand (8 positions of one
-//                 column) is two 8-byte reads.
-// The running max / sum / rescale are the usual online softmax; probabilities are rounded to
-// bf16 for the second product, sums are kept in fp32.
-#include "common.h"
+// A tile of 64 positions' keys and values travels straight into LDS (global_load_lds), tiles ahead, rows as they lie in the
+// cache with their 16-byte pieces permuted by the row's number; for 16 queries of one (sequence, head):
+//   S^T = K Q^T   v_mfma_f32_16x16x32_bf16, A = K rows from LDS, B = Q rows held in registers for the whole walk; a lane
+//                 ends up with 16 scores of ONE query (its column), so the row max/sum need two cross-lane
+//                 steps only;
+//   O^T += V^T P  the probabilities go from the scores straight into the B operand (the k-slot -> position
+//                 mapping is chosen so that no lane exchange is needed); the A operand - four positions of one
+//                 column - is what ds_read_b64_tr_b16 makes of four rows of V: within sixteen lanes, lane 4 r + c
+//                 reads columns 4 c .. 4 c + 3 of row r and lane n receives column n of the four rows.
+// The running max / sum / rescale are the usual online softmax; probabilities are rounded to bf16 for the second product,
+// sums are kept in fp32, positions are added in their order whatever the shape of the workgroup.
+//
+// Two kernels: one wave per 16 or 32 queries where there are many (attn_prefill_kernel), four waves per 16 where there are
+// few and the walk over the positions is a chain (attn_team_kernel).
+//
+// What bounds them: the softmax between the products, and where the keys and values come from.  A head's q blocks read
+// the same ones: spread round-robin over the XCDs every L2 held every head's, and the launch waited for memory.
+#include "lds_tile.h"
 
 namespace {
 
@@ -25,239 +31,405 @@ struct PrefillArgs {
   const bf16_t* v;
   bf16_t* out;       // (B*S, H*D)
   int B, S, H, Hkv, Tmax, pos;
-  int nqb;           // query blocks (of 128 or 64) per sequence
+  int nqb;           // query blocks per sequence
   float scale_log2e;
 };
 
-template <int D, int QW>  // QW: blocks of 16 queries per wave (2: 128 queries per workgroup, 1: 64)
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 lds_tr8(uint32_t addr) {
+  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((OHARA_LDS s16x4*)(uintptr_t)addr);
+  return __builtin_bit_cast(uint2, v);
+}
+
+// An XCD (ids go round-robin over the eight) gets whole heads, their late - longest - blocks first; where the heads do
+// not divide, an eighth of all blocks in the order of the heads, long and short ones in turn.
+__device__ __forceinline__ void my_block(const PrefillArgs& a, int& head, int& qblk) {
+  const int heads = a.H * a.B, x = blockIdx.x & 7, q = blockIdx.x >> 3;
+  if ((heads & 7) == 0) {
+    const int nh = heads >> 3;
+    head = x * nh + q % nh;
+    qblk = a.nqb - 1 - q / nh;
+  } else {
+    const int n = gridDim.x, p = x * (n >> 3) + min(x, n & 7) + q;
+    head = p / a.nqb;
+    const int r = p - head * a.nqb;
+    qblk = r & 1 ? r >> 1 : a.nqb - 1 - (r >> 1);
+  }
+}
+
+constexpr int KT = 64;                // positions of a tile
+constexpr int NKB = KT / 16, NWIN = KT / 32;
+
+// A tile in LDS: the keys' rows, then the values'.  How NW waves bring it there, and where a lane finds its fragments.
+template <int D>
+struct KvTile {
+  static constexpr int ROWB = 2 * D, PIECES = ROWB / 16, RPL = 1024 / ROWB;  // bytes and 16-byte pieces of a row, rows of a load
+  static constexpr int BYTES = KT * ROWB, SLOT = 2 * BYTES;
+  const char *kb, *vb;  // the sequence's first row of this head
+  uint32_t rowb;        // bytes from one position to the next
+  int len;              // positions that exist
+  int lane;
+
+  __device__ __forceinline__ KvTile(const PrefillArgs& a, int b, int kvh, int lane_) : lane(lane_) {
+    const size_t row = (size_t)a.Hkv * D;
+    kb = reinterpret_cast<const char*>(a.k + (size_t)b * a.Tmax * row + (size_t)kvh * D);
+    vb = reinterpret_cast<const char*>(a.v + (size_t)b * a.Tmax * row + (size_t)kvh * D);
+    rowb = (uint32_t)row * 2;
+    len = a.pos + a.S;
+  }
+  // ALIGNED: the caches start on 16 bytes (false: through registers, any)
+  template <int NW>
+  struct Offsets {
+    static_assert(KT / RPL % NW == 0, "loads split evenly over the waves");
+    static constexpr int N = KT / RPL / NW;
+    uint32_t k[N], v[N];
+  };
+  // this lane's of the loads of a tile that holds `rows` positions: past them, the last one (masked)
+  template <int NW>
+  __device__ __forceinline__ Offsets<NW> offsets(int rows, int wave) const {
+    Offsets<NW> o;
+    const int lr = lane / PIECES, lq = lane % PIECES;  // its row of a load, and its place in it
+#pragma unroll
+    for (int i = 0; i < o.N; ++i) {
+      const int r = (wave + i * NW) * RPL + lr;
+      const uint32_t ro = (uint32_t)min(r, rows - 1) * rowb;
+      o.k[i] = ro + (uint32_t)((lq ^ r) & (PIECES - 1)) * 16;
+      o.v[i] = ro + (uint32_t)(lq ^ ((r & (PIECES / 2 - 1)) << 1)) * 16;
+    }
+    return o;
+  }
+  template <int NW, bool ALIGNED>
+  __device__ __forceinline__ void issue(int t, uint32_t slot, int wave, const Offsets<NW>& full) const {
+    const char* kt = kb + (size_t)(t * KT) * rowb;
+    const char* vt = vb + (size_t)(t * KT) * rowb;
+    Offsets<NW> o = full;
+    if (t * KT + KT > len) o = offsets<NW>(len - t * KT, wave);
+#pragma unroll
+    for (int i = 0; i < o.N; ++i) {
+      const uint32_t dst = slot + (wave + i * NW) * 1024;
+      if (ALIGNED) {
+        load_lds16(dst, kt, o.k[i]);
+        load_lds16(dst + BYTES, vt, o.v[i]);
+      } else {
+        const uint4 kv = ldg16(kt + o.k[i]), vv = ldg16(vt + o.v[i]);
+        *(OHARA_LDS u32x4*)(uintptr_t)(dst + lane * 16) = (u32x4){kv.x, kv.y, kv.z, kv.w};
+        *(OHARA_LDS u32x4*)(uintptr_t)(dst + BYTES + lane * 16) = (u32x4){vv.x, vv.y, vv.z, vv.w};
+      }
+    }
+  }
+  // keys of positions 16 kb + (lane & 15), columns 32 j + 8 (lane >> 4) .. + 7
+  __device__ __forceinline__ uint4 keys(uint32_t slot, int kb_, int j) const {
+    const int m = lane & 15, g = lane >> 4;
+    return lds16_at(slot + (16 * kb_ + m) * ROWB + (uint32_t)((4 * j + g) ^ (m & (PIECES - 1))) * 16);
+  }
+  // column 16 d + (lane & 15) of the values of positions 32 w + 4 g .. + 3 and of those 16 later
+  __device__ __forceinline__ uint4 values(uint32_t slot, int w, int d) const {
+    const int m = lane & 15, row = 4 * (lane >> 4) + (m >> 2);
+    const uint32_t at = slot + BYTES + (32 * w + row) * ROWB + (m & 3) * 8 + (uint32_t)((row & (PIECES / 2 - 1)) ^ d) * 32;
+    const uint2 lo = lds_tr8(at), hi = lds_tr8(at + 16 * ROWB);
+    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+  }
+};
+
+template <bool ALIGNED, int LEFT>
+__device__ __forceinline__ void tile_barrier() {  // this wave's older loads have landed, and everyone's
+  if (ALIGNED) wait_loads<LEFT>();
+  else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+}
+
+// Online softmax over a tile, per query (= per lane column): s -> the B operand of the second product, and what the
+// accumulators so far are multiplied with.
+__device__ __forceinline__ float softmax_tile(f32x4 (&s)[NKB], uint4 (&pf)[NWIN], float& m_run, float& l_run, int t0, int first, int qpos,
+                                              int g, float scale_log2e) {
+  float tmax = -INFINITY;
+  float mul = 1.0f;  // what the stored scores still have to be multiplied with
+  if (t0 + KT - 1 > first) {  // (wave-uniform) the tile reaches past the wave's first query: mask
+#pragma unroll
+    for (int kk = 0; kk < NKB; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float v = s[kk][i] * scale_log2e;
+        if (t0 + kk * 16 + 4 * g + i > qpos) v = -INFINITY;
+        s[kk][i] = v;
+        tmax = fmaxf(tmax, v);
+      }
+  } else {
+#pragma unroll
+    for (int kk = 0; kk < NKB; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, s[kk][i]);
+    tmax *= scale_log2e;  // the scale is positive: the maximum of the products is the product of the maximum
+    mul = scale_log2e;    // and the scaling itself rides in the fused multiply-add of the exponent below
+  }
+  tmax = lane_xor_max<32>(lane_xor_max<16>(tmax));
+  // the running maximum is kept as an integer (log2 units): every rescale is then an exact power of
+  // two and the bf16 weights do not depend on which tile raised it (common.h: softmax bookkeeping)
+  const float mn = fmaxf(m_run, ceilf(tmax));
+  const float corr = pow2_neg_int(m_run - mn);
+  m_run = mn;
+  float ts = 0.f;
+  float p[NKB][4];
+#pragma unroll
+  for (int kk = 0; kk < NKB; ++kk)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[kk][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kk][i], mul, -mn));
+      ts += p[kk][i];
+    }
+  l_run = l_run * corr + ts;  // this lane's share; lanes g = 0..3 are added at the end
+  // k-slot 8 g + i of window w  <->  position 32 w + 4 g + i (i < 4), 32 w + 16 + 4 g + i - 4
+#pragma unroll
+  for (int w = 0; w < NWIN; ++w)
+    pf[w] = make_uint4(pack_bf(p[2 * w][0], p[2 * w][1]), pack_bf(p[2 * w][2], p[2 * w][3]),
+                       pack_bf(p[2 * w + 1][0], p[2 * w + 1][1]), pack_bf(p[2 * w + 1][2], p[2 * w + 1][3]));
+  return corr;
+}
+
+__device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// Queries wq0 + 16 qb + (lane & 15): lane g holds columns 32 j + 8 g .. + 7
+template <int D>
+__device__ __forceinline__ void load_queries(uint4 (&qf)[D / 32], int& qpos, const PrefillArgs& a, int b, int h, int qi, int g) {
+  qpos = qi < a.S ? a.pos + qi : 0x3fffffff;  // rows past the end: never masked, never stored
+#pragma unroll
+  for (int j = 0; j < D / 32; ++j)
+    qf[j] = qi < a.S ? ldg16(a.q + ((size_t)b * a.S + qi) * a.H * D + (size_t)h * D + 32 * j + 8 * g) : make_uint4(0, 0, 0, 0);
+}
+
+template <int D, int N>
+__device__ __forceinline__ void store_rows(const f32x4 (&o)[N], float l, const PrefillArgs& a, int b, int h, int qi, int g, int d0) {
+  l = lane_xor_sum<32>(lane_xor_sum<16>(l));
+  if (qi >= a.S) return;
+  const float inv = 1.0f / l;
+  bf16_t* dst = a.out + ((size_t)b * a.S + qi) * a.H * D + (size_t)h * D + 16 * d0 + 4 * g;
+#pragma unroll
+  for (int db = 0; db < N; ++db)
+    *reinterpret_cast<uint2*>(dst + db * 16) = make_uint2(pack_bf(o[db][0] * inv, o[db][1] * inv), pack_bf(o[db][2] * inv, o[db][3] * inv));
+}
+
+// Four waves of 16 QW queries, one tile ahead.
+template <int D, int QW, bool ALIGNED>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
-  constexpr int QB = 64 * QW, KT = 64;
-  constexpr int NK = D / 32;   // k-steps of the score product
-  constexpr int ND = D / 16;   // 16-column blocks of the output
-  constexpr int LDK = D + 8;   // K tile row stride (elements): 16-byte reads without bank conflicts
-  constexpr int LDV = KT + 4;  // V^T row stride (elements)
-  constexpr int RPT = KT * D / 8 / 256;  // 16-byte pieces of a tile per thread (K and V each)
-  constexpr int GP = RPT >= 4 ? 4 : 2;   // positions a thread transposes together
-  __shared__ __align__(16) bf16_t Ks[KT][LDK];
-  __shared__ __align__(16) bf16_t Vt[D][LDV];
-  // A column's 64 positions are rotated by four positions per group of eight columns (GP == 4): the sixteen
-  // threads that transpose one position group write columns eight apart, which would land on two banks.
-  auto vt_off = [](int col, int p) { return GP == 4 ? ((p + 4 * (col >> 3)) & (KT - 1)) : p; };
-
-  // heavy (late) query blocks first
-  const int qblk = a.nqb - 1 - (int)blockIdx.x;
-  const int h = blockIdx.y, b = blockIdx.z;
-  const int kvh = h / (a.H / a.Hkv);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int NW = 4, QB = 16 * QW * NW;
+  constexpr int NK = D / 32;             // k-steps of the score product
+  constexpr int ND = D / 16;             // 16-column blocks of the output
+  typedef KvTile<D> Tl;
+  extern __shared__ __align__(16) unsigned char smem[];
+  int head, qblk;
+  my_block(a, head, qblk);
+  const int b = head / a.H, h = head - b * a.H;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int m = lane & 15, g = lane >> 4;
-  const int q0 = qblk * QB;                       // first query of the workgroup
-  const int wq0 = q0 + wave * 16 * QW;            // first query of the wave
-  const size_t row = (size_t)a.Hkv * D;
-  const bf16_t* kb = a.k + (size_t)b * a.Tmax * row + (size_t)kvh * D;
-  const bf16_t* vb = a.v + (size_t)b * a.Tmax * row + (size_t)kvh * D;
-  const int Lall = a.pos + a.S;                   // cached positions that exist
-  const int kv_end = min(a.pos + q0 + QB, Lall);  // positions any query of the workgroup sees
+  const int q0 = qblk * QB;                              // first query of the workgroup
+  const int wq0 = q0 + wave * 16 * QW;                   // first query of the wave
+  const Tl tile(a, b, h / (a.H / a.Hkv), lane);
+  const typename Tl::template Offsets<NW> offs = tile.template offsets<NW>(KT, wave);
+  const int ntiles = (min(a.pos + q0 + QB, tile.len) + KT - 1) / KT;  // tiles any query of the workgroup sees
+  const int wave_last = min(a.pos + wq0 + 16 * QW - 1, tile.len - 1);  // last position any query of the wave sees
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
 
-  // Q fragments: lane (n = query within block, g) holds Q[q][32 j + 8 g .. +7]
   uint4 qf[QW][NK];
   int qpos[QW];
-#pragma unroll
-  for (int qb = 0; qb < QW; ++qb) {
-    const int qi = wq0 + qb * 16 + m;
-    qpos[qb] = qi < a.S ? a.pos + qi : 0x3fffffff;  // rows past the end: never masked, never stored
-#pragma unroll
-    for (int j = 0; j < NK; ++j)
-      qf[qb][j] = qi < a.S ? ldg16(a.q + ((size_t)b * a.S + qi) * a.H * D + (size_t)h * D + 32 * j + 8 * g)
-                           : make_uint4(0, 0, 0, 0);
-  }
-  const int wave_last = min(a.pos + wq0 + 16 * QW - 1, Lall - 1);  // last position any query of the wave sees
-
   f32x4 o[QW][ND];
   float m_run[QW], l_run[QW];
 #pragma unroll
   for (int qb = 0; qb < QW; ++qb) {
+    load_queries<D>(qf[qb], qpos[qb], a, b, h, wq0 + qb * 16 + m, g);
     m_run[qb] = -INFINITY;
     l_run[qb] = 0.f;
 #pragma unroll
     for (int db = 0; db < ND; ++db) o[qb][db] = (f32x4){0.f, 0.f, 0.f, 0.f};
   }
-
-  // tile loaders.  K: thread (r = tid / (D/8) + i * (256 / (D/8)), c = tid % (D/8)) one 16-byte
-  // piece.  V: thread (kq = tid / (D/8), c) takes rows 4 kq' .. with kq' = kq + i * (256/(D/8))
-  constexpr int CPR = D / 8;         // 16-byte pieces per row
-  constexpr int RPP = 256 / CPR;     // rows per pass
-  const int lr = tid / CPR, lc = tid % CPR;
-  uint4 kr[RPT], vr[RPT];
-  auto load_tile = [&](int t0) {
+  tile.template issue<NW, ALIGNED>(0, lds0, wave, offs);
+  uint32_t cur = lds0;
+  for (int t = 0; t < ntiles; ++t) {
+    tile_barrier<ALIGNED, 0>();  // the tile is there, and everyone is done with the one before
+    const uint32_t next = lds0 + Tl::SLOT - (cur - lds0);
+    if (t + 1 < ntiles) tile.template issue<NW, ALIGNED>(t + 1, next, wave, offs);
+    const int t0 = t * KT;
+    if (t0 <= wave_last) {  // else wholly masked for this wave (barriers stay uniform)
+      // all fragments read before the first product, and the products of different blocks in turn, so that none waits
+      // for the one before it
+      f32x4 s[QW][NKB];
+      uint4 kf[NKB][NK];
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const int p = t0 + lr + i * RPP;
-      kr[i] = p < Lall ? ldg16(kb + (size_t)p * row + lc * 8) : make_uint4(0, 0, 0, 0);
-    }
-    // V: GP consecutive positions per thread and group, so that the transposed write is wide
+      for (int kk = 0; kk < NKB; ++kk)
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const int p = t0 + GP * (lr + (i / GP) * RPP) + (i % GP);
-      vr[i] = p < Lall ? ldg16(vb + (size_t)p * row + lc * 8) : make_uint4(0, 0, 0, 0);
-    }
-  };
-  auto store_tile = [&]() {
-#pragma unroll
-    for (int i = 0; i < RPT; ++i) *reinterpret_cast<uint4*>(&Ks[lr + i * RPP][lc * 8]) = kr[i];
-    // transpose GP positions x 8 columns: per column one write of GP positions
-#pragma unroll
-    for (int grp = 0; grp < RPT / GP; ++grp) {
-      const int p0 = GP * (lr + grp * RPP);
-      uint32_t w[GP][4];
-#pragma unroll
-      for (int r = 0; r < GP; ++r) {
-        w[r][0] = vr[GP * grp + r].x; w[r][1] = vr[GP * grp + r].y;
-        w[r][2] = vr[GP * grp + r].z; w[r][3] = vr[GP * grp + r].w;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {  // column pair 2e, 2e+1 of this thread's 8 columns
-        const uint32_t lo01 = (w[0][e] & 0xffffu) | (w[1][e] << 16);
-        const uint32_t hi01 = (w[0][e] >> 16) | (w[1][e] & 0xffff0000u);
-        if (GP == 4) {
-          const uint32_t lo23 = (w[GP - 2][e] & 0xffffu) | (w[GP - 1][e] << 16);
-          const uint32_t hi23 = (w[GP - 2][e] >> 16) | (w[GP - 1][e] & 0xffff0000u);
-          *reinterpret_cast<uint2*>(&Vt[lc * 8 + 2 * e][vt_off(lc * 8 + 2 * e, p0)]) = make_uint2(lo01, lo23);
-          *reinterpret_cast<uint2*>(&Vt[lc * 8 + 2 * e + 1][vt_off(lc * 8 + 2 * e + 1, p0)]) = make_uint2(hi01, hi23);
-        } else {
-          *reinterpret_cast<uint32_t*>(&Vt[lc * 8 + 2 * e][p0]) = lo01;
-          *reinterpret_cast<uint32_t*>(&Vt[lc * 8 + 2 * e + 1][p0]) = hi01;
-        }
-      }
-    }
-  };
-
-  load_tile(0);
-  for (int t0 = 0; t0 < kv_end; t0 += KT) {
-    __syncthreads();  // everyone is done reading the previous tile
-    store_tile();
-    __syncthreads();
-    if (t0 + KT < kv_end) load_tile(t0 + KT);  // in flight during the products below
-    if (t0 > wave_last) continue;               // wholly masked for this wave (barriers stay uniform)
-
-    // scores: s[kb][qb] = D[16 positions x 16 queries]
-    // The K fragments of two 16-position blocks are read from LDS into registers of their own before
-    // their products (left to itself the compiler reuses one register quad: read, wait, product,
-    // sixteen times per tile, every LDS latency exposed - a quarter of a tile's time).
-    constexpr int KBB = QW == 1 ? 1 : 2;  // 16-position blocks whose fragments are read together (registers: three workgroups per CU with QW == 1)
-    f32x4 s[4][QW];
-#pragma unroll
-    for (int kb2 = 0; kb2 < 4; kb2 += KBB) {
-      uint4 kf[KBB][NK];
-#pragma unroll
-      for (int kk = 0; kk < KBB; ++kk)
-#pragma unroll
-        for (int j = 0; j < NK; ++j) kf[kk][j] = *reinterpret_cast<const uint4*>(&Ks[(kb2 + kk) * 16 + m][32 * j + 8 * g]);
+        for (int j = 0; j < NK; ++j) kf[kk][j] = tile.keys(cur, kk, j);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kk = 0; kk < KBB; ++kk) {
-        const int kbk = kb2 + kk;
+      for (int j = 0; j < NK; ++j)
 #pragma unroll
-        for (int qb = 0; qb < QW; ++qb) s[kbk][qb] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < NK; ++j)
+        for (int kk = 0; kk < NKB; ++kk)
 #pragma unroll
           for (int qb = 0; qb < QW; ++qb)
-            s[kbk][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[kk][j]),
-                                                                 __builtin_bit_cast(bf16x8, qf[qb][j]), s[kbk][qb], 0, 0, 0);
-      }
+            s[qb][kk] = mfma16(kf[kk][j], qf[qb][j], j ? s[qb][kk] : (f32x4){0.f, 0.f, 0.f, 0.f});
       __builtin_amdgcn_sched_barrier(0);
-    }
-    // online softmax per query (= per lane column)
-    uint4 pf[QW][2];  // [qb][32-position window]: B operand of the second product
+      uint4 pf[QW][NWIN];
 #pragma unroll
-    for (int qb = 0; qb < QW; ++qb) {
-      float tmax = -INFINITY;
-      float mul = 1.0f;  // what the stored scores still have to be multiplied with
-      if (t0 + KT - 1 > a.pos + wq0) {  // (wave-uniform) the tile reaches past the wave's first query: mask
+      for (int qb = 0; qb < QW; ++qb) {
+        const float corr = softmax_tile(s[qb], pf[qb], m_run[qb], l_run[qb], t0, a.pos + wq0, qpos[qb], g, a.scale_log2e);
+        if (__any(corr != 1.0f)) {  // most tiles leave the running maximum of every query of the wave alone
 #pragma unroll
-        for (int kbk = 0; kbk < 4; ++kbk)
+          for (int db = 0; db < ND; ++db)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float v = s[kbk][qb][i] * a.scale_log2e;
-            if (t0 + kbk * 16 + 4 * g + i > qpos[qb]) v = -INFINITY;
-            s[kbk][qb][i] = v;
-            tmax = fmaxf(tmax, v);
-          }
-      } else {
-#pragma unroll
-        for (int kbk = 0; kbk < 4; ++kbk)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, s[kbk][qb][i]);
-        tmax *= a.scale_log2e;  // the scale is positive: the maximum of the products is the product of the maximum
-        mul = a.scale_log2e;    // and the scaling itself rides in the fused multiply-add of the exponent below
-      }
-      tmax = lane_xor_max<32>(lane_xor_max<16>(tmax));
-      // the running maximum is kept as an integer (log2 units): every rescale is then an exact power of
-      // two and the bf16 weights do not depend on which tile raised it (common.h: softmax bookkeeping)
-      const float mn = fmaxf(m_run[qb], ceilf(tmax));  // finite: position 0 is visible to every query
-      const float corr = pow2_neg_int(m_run[qb] - mn);
-      m_run[qb] = mn;
-      float ts = 0.f;
-      float p[4][4];
-#pragma unroll
-      for (int kbk = 0; kbk < 4; ++kbk)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          p[kbk][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kbk][qb][i], mul, -mn));
-          ts += p[kbk][i];
+            for (int i = 0; i < 4; ++i) o[qb][db][i] *= corr;
         }
-      l_run[qb] = l_run[qb] * corr + ts;  // this lane's share; lanes g = 0..3 are added at the end
-      if (__any(corr != 1.0f)) {  // most tiles leave the running maximum of every query of the wave alone
+      }
+#pragma unroll
+      for (int w = 0; w < NWIN; ++w) {
+        uint4 vf[ND];  // all read before the first product, as above
+#pragma unroll
+        for (int db = 0; db < ND; ++db) vf[db] = tile.values(cur, w, db);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int db = 0; db < ND; ++db)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[qb][db][i] *= corr;
+          for (int qb = 0; qb < QW; ++qb) o[qb][db] = mfma16(vf[db], pf[qb][w], o[qb][db]);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      // k-slot 8 g + i of window w  <->  position 32 w + 4 g + i (i < 4), 32 w + 16 + 4 g + i - 4
-#pragma unroll
-      for (int w = 0; w < 2; ++w)
-        pf[qb][w] = make_uint4(pack_bf(p[2 * w][0], p[2 * w][1]), pack_bf(p[2 * w][2], p[2 * w][3]),
-                               pack_bf(p[2 * w + 1][0], p[2 * w + 1][1]), pack_bf(p[2 * w + 1][2], p[2 * w + 1][3]));
     }
-    // O^T[16 columns x 16 queries] += V^T[16 columns x 32 slots] P[32 slots x 16 queries]
-    constexpr int DBB = QW == 1 ? 4 : ND;  // 16-column blocks of V^T whose fragments are read together
-#pragma unroll
-    for (int w = 0; w < 2; ++w)
-#pragma unroll
-      for (int d0 = 0; d0 < ND; d0 += DBB) {
-        uint2 v0[DBB], v1[DBB];  // all read before the first product, as above
-#pragma unroll
-        for (int i = 0; i < DBB; ++i) {
-          const int db = d0 + i;
-          v0[i] = *reinterpret_cast<const uint2*>(&Vt[db * 16 + m][vt_off(db * 16 + m, 32 * w + 4 * g)]);
-          v1[i] = *reinterpret_cast<const uint2*>(&Vt[db * 16 + m][vt_off(db * 16 + m, 32 * w + 16 + 4 * g)]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < DBB; ++i) {
-          const uint4 vf = make_uint4(v0[i].x, v0[i].y, v1[i].x, v1[i].y);
-#pragma unroll
-          for (int qb = 0; qb < QW; ++qb)
-            o[qb][d0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, vf),
-                                                                    __builtin_bit_cast(bf16x8, pf[qb][w]), o[qb][d0 + i], 0, 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
+    cur = next;
   }
+#pragma unroll
+  for (int qb = 0; qb < QW; ++qb) store_rows<D>(o[qb], l_run[qb], a, b, h, wq0 + qb * 16 + m, g, 0);
+}
+
+// TEAMS teams of four waves, 16 queries each.  Wave w scores positions 16 w .. + 15 of every tile and owns a quarter of the output
+// columns; the scores go through LDS, and every wave of the team does the softmax of the whole tile.  In the round that works
+// off tile t the scores of t + 1 are made: one barrier a tile.
+template <int D, int TEAMS, int NST, bool ALIGNED>
+__global__ __launch_bounds__(TEAMS * 256, TEAMS) void attn_team_kernel(PrefillArgs a) {
+  constexpr int NW = 4 * TEAMS, QB = 16 * TEAMS;
+  constexpr int NK = D / 32, ND = D / 64;  // k-steps of the score product, 16-column blocks of a wave's output
+  typedef KvTile<D> Tl;
+  constexpr int LPW = 2 * KT / Tl::RPL / NW;  // a wave's loads of a tile
+  extern __shared__ __align__(16) unsigned char smem[];
+  int head, qblk;
+  my_block(a, head, qblk);
+  const int b = head / a.H, h = head - b * a.H;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w4 = wave & 3, team = wave >> 2;
+  const int m = lane & 15, g = lane >> 4;
+  const int q0 = qblk * QB, wq0 = q0 + 16 * team;
+  const Tl tile(a, b, h / (a.H / a.Hkv), lane);
+  const typename Tl::template Offsets<NW> offs = tile.template offsets<NW>(KT, wave);
+  const int ntiles = (min(a.pos + q0 + QB, tile.len) + KT - 1) / KT;
+  const int team_last = min(a.pos + wq0 + 15, tile.len - 1);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
+  const uint32_t sc0 = lds0 + NST * Tl::SLOT + team * 4096 + lane * 16;  // the team's scores: two tiles' in turn
+
+  uint4 qf[NK];
+  int qpos;
+  load_queries<D>(qf, qpos, a, b, h, wq0 + m, g);
+  f32x4 o[ND];
+#pragma unroll
+  for (int db = 0; db < ND; ++db) o[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+
+  auto scores = [&](const uint4 (&kf)[NK]) {
+    f32x4 s = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NK; ++j) s = mfma16(kf[j], qf[j], s);
+    return s;
+  };
+  auto put_scores = [&](int t, f32x4 s) { *(OHARA_LDS f32x4*)(uintptr_t)(sc0 + (t & 1) * (TEAMS * 4096) + w4 * 1024) = s; };
 
 #pragma unroll
-  for (int qb = 0; qb < QW; ++qb) {
-    const int qi = wq0 + qb * 16 + m;
-    float l = l_run[qb];
-    l = lane_xor_sum<32>(lane_xor_sum<16>(l));
-    if (qi >= a.S) continue;
-    const float inv = 1.0f / l;
-    bf16_t* dst = a.out + ((size_t)b * a.S + qi) * a.H * D + (size_t)h * D + 4 * g;
+  for (int t = 0; t < NST - 1; ++t)
+    if (t < ntiles) tile.template issue<NW, ALIGNED>(t, lds0 + t * Tl::SLOT, wave, offs);
+  if (NST - 2 < ntiles) tile_barrier<ALIGNED, (NST - 2) * LPW>();
+  else tile_barrier<ALIGNED, 0>();
+  uint4 kf[NK];
 #pragma unroll
-    for (int db = 0; db < ND; ++db)
-      *reinterpret_cast<uint2*>(dst + db * 16) = make_uint2(pack_bf(o[qb][db][0] * inv, o[qb][db][1] * inv),
-                                                            pack_bf(o[qb][db][2] * inv, o[qb][db][3] * inv));
+  for (int j = 0; j < NK; ++j) kf[j] = tile.keys(lds0, w4, j);
+  put_scores(0, scores(kf));
+  uint32_t cur = lds0;
+  for (int t = 0; t < ntiles; ++t) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the scores of this tile are written
+    if (t + NST - 2 < ntiles) tile_barrier<ALIGNED, (NST - 3) * LPW>();  // and the next tile is there
+    else tile_barrier<ALIGNED, 0>();
+    asm volatile("" ::: "memory");
+    const uint32_t next = cur + Tl::SLOT == lds0 + NST * Tl::SLOT ? lds0 : cur + Tl::SLOT;
+    if (t + NST - 1 < ntiles) tile.template issue<NW, ALIGNED>(t + NST - 1, cur == lds0 ? lds0 + (NST - 1) * Tl::SLOT : cur - Tl::SLOT, wave, offs);
+    const int t0 = t * KT;
+    // everything this round reads, then the products (past the last tile: of what the slot holds, unused)
+    f32x4 s[NKB];
+    uint4 vf[NWIN][ND];
+#pragma unroll
+    for (int kk = 0; kk < NKB; ++kk) s[kk] = *(OHARA_LDS f32x4*)(uintptr_t)(sc0 + (t & 1) * (TEAMS * 4096) + kk * 1024);
+#pragma unroll
+    for (int j = 0; j < NK; ++j) kf[j] = tile.keys(next, w4, j);
+#pragma unroll
+    for (int w = 0; w < NWIN; ++w)
+#pragma unroll
+      for (int db = 0; db < ND; ++db) vf[w][db] = tile.values(cur, w, w4 * ND + db);
+    __builtin_amdgcn_sched_barrier(0);
+    const f32x4 sn = scores(kf);
+    if (TEAMS == 1 || t0 <= team_last) {  // else wholly masked for this team
+      uint4 pf[NWIN];
+      const float corr = softmax_tile(s, pf, m_run, l_run, t0, a.pos + wq0, qpos, g, a.scale_log2e);
+#pragma unroll
+      for (int db = 0; db < ND; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[db][i] *= corr;
+#pragma unroll
+      for (int w = 0; w < NWIN; ++w)
+#pragma unroll
+        for (int db = 0; db < ND; ++db) o[db] = mfma16(vf[w][db], pf[w], o[db]);
+    }
+    put_scores(t + 1, sn);
+    cur = next;
   }
+  store_rows<D>(o, l_run, a, b, h, wq0 + m, g, w4 * ND);
+}
+
+template <int D, int QW, bool ALIGNED = true>
+int launch_waves(PrefillArgs a, hipStream_t st) {
+  a.nqb = (a.S + 64 * QW - 1) / (64 * QW);
+  const int64_t blocks = (int64_t)a.nqb * a.H * a.B;
+  if (blocks > INT32_MAX) return OHARA_ESIZE;
+  hipLaunchKernelGGL((attn_prefill_kernel<D, QW, ALIGNED>), dim3((unsigned)blocks), dim3(256), 2 * KvTile<D>::SLOT, st, a);
+  return ohara_launch_status();
+}
+
+template <int D, int TEAMS, int NST = 3>
+int launch_teams(PrefillArgs a, hipStream_t st) {
+  constexpr int LDS = NST * KvTile<D>::SLOT + 2 * TEAMS * 4096;
+  a.nqb = (a.S + 16 * TEAMS - 1) / (16 * TEAMS);
+  if (LDS > 64 * 1024)
+    (void)hipFuncSetAttribute((const void*)attn_team_kernel<D, TEAMS, NST, true>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  hipLaunchKernelGGL((attn_team_kernel<D, TEAMS, NST, true>), dim3((unsigned)(a.nqb * a.H * a.B)), dim3(TEAMS * 256), LDS, st, a);
+  return ohara_launch_status();
+}
+
+// Both kernels give the same bits; us with teams of 16 / 32 queries a workgroup and waves of 16 / 32 (64 / 128 a workgroup):
+//   heads of 128                                                 heads of 64, 16 heads
+//     128 queries x 6 heads   4.5 /  5.5 /  5.5 /  7.1             160 queries      4.3 /  5.0 /  4.6 /  5.8
+//     48 behind 1900, 4 x 16 24.7 / 27.8 / 34   / 49               500              7.6 /  8.5 /  8.4 / 11.7
+//     600 x 6                10.4 / 11.4 / 13.0 / 18.6             24 x 160         23  / 18   /  9.8 /  9.9
+//     1024 x 6               22   / 16.7 / 20   / 28               8 x 1024         122 / 90   / 34.9 / 36.1
+//     1024 x 16              31   / 20.3 / 20.2 / 28
+//     4001 x 16             364   / 214  / 110  / 122
+//     8 x 1024 x 6           97   / 62   / 28   / 36
+//     32 x 512 x 6          137   / 84   / 38   / 31
+//     16 x 700 x 16         269   / 173  / 74   / 68
+// so: teams while every workgroup is on a CU at once (two of the narrow ones' of 16), 128 queries from three workgroups a
+// CU on, else 64.  Before (one kernel, four waves, values through registers, the heads over all XCDs): 5.8, 45, 16.5, 25, 26, 167,
+// 50, 46, 92; 5.2, 10.4, 12, 64.
+template <int D>
+int launch_prefill_for(const PrefillArgs& a, hipStream_t st) {
+  constexpr int CUS = 256;
+  const int64_t heads = (int64_t)a.H * a.B;
+  auto blocks = [&](int queries) { return (a.S + queries - 1) / queries * heads; };
+  if (((uintptr_t)a.k | (uintptr_t)a.v) & 15) return launch_waves<D, 1, false>(a, st);
+  if (blocks(16) <= CUS * (D == 64 ? 2 : 1)) return launch_teams<D, 1>(a, st);
+  if (blocks(32) <= CUS) return launch_teams<D, 2>(a, st);
+  if (blocks(128) >= 3 * CUS) return launch_waves<D, 2>(a, st);
+  return launch_waves<D, 1>(a, st);
 }
 
 }  // namespace
@@ -274,25 +446,5 @@ extern "C" int ohara_attn_prefill_bf16(const uint16_t* q, const uint16_t* kcache
   a.q = q; a.k = kcache; a.v = vcache; a.out = out;
   a.B = batch; a.S = seq_len; a.H = h; a.Hkv = h_kv; a.Tmax = t_max; a.pos = pos;
   a.scale_log2e = (1.0f / sqrtf((float)dh)) * OHARA_LOG2E;  // the same constant as the decode kernels'
-  // A causal launch lasts as long as its last query block (sixteen tiles at 1024 tokens, twice the
-  // average), whatever the other workgroups do.  With fewer than two blocks of 128 queries per CU,
-  // blocks of 64 fit three workgroups on a CU and all of them are resident at once (8 x 1024 tokens,
-  // 6 heads: 56.1 -> 54.5 us; the tile of the last block, about 2.9 us, stays what bounds the launch).
-  static int cus = 0;
-  if (!cus) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      cus = 256;
-  }
-  const bool small = (int64_t)((seq_len + 127) / 128) * h * batch < 2 * (int64_t)cus;
-  a.nqb = small ? (seq_len + 63) / 64 : (seq_len + 127) / 128;
-  dim3 grid(a.nqb, h, batch), block(256);
-  if (dh == 128) {
-    if (small) hipLaunchKernelGGL((attn_prefill_kernel<128, 1>), grid, block, 0, (hipStream_t)stream, a);
-    else hipLaunchKernelGGL((attn_prefill_kernel<128, 2>), grid, block, 0, (hipStream_t)stream, a);
-  } else {
-    if (small) hipLaunchKernelGGL((attn_prefill_kernel<64, 1>), grid, block, 0, (hipStream_t)stream, a);
-    else hipLaunchKernelGGL((attn_prefill_kernel<64, 2>), grid, block, 0, (hipStream_t)stream, a);
-  }
-  return ohara_launch_status();
+  return dh == 128 ? launch_prefill_for<128>(a, (hipStream_t)stream) : launch_prefill_for<64>(a, (hipStream_t)stream);
 }

@@ -1,0 +1,83 @@
+"""Attention over many query positions in its four workgroup shapes: tile edges, queries and positions that do not fill them, heads that divide over the XCDs and heads that do not, caches that start on any element."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def _reference(q, k, v, pos):
+    """In 64 bits, with the bound: weights are rounded to bf16 (2^-9 of each, all of a query's in one direction at worst, against
+    a sum of unrounded ones), the result once more; a score is an fp32 sum of D products that are 16 together at most, which its
+    weight follows."""
+    B, S, H, D = q.shape
+    L = pos + S
+    k = k[:, :L].double().repeat_interleave(H // k.shape[2], 2)
+    v = v[:, :L].double().repeat_interleave(H // v.shape[2], 2)
+    s = torch.matmul(q.double().transpose(1, 2), k.permute(0, 2, 3, 1).contiguous()) / D ** 0.5
+    s.masked_fill_(torch.arange(L, device=q.device)[None, :] > pos + torch.arange(S, device=q.device)[:, None], float("-inf"))
+    p = torch.softmax(s, -1)
+    vt = v.transpose(1, 2).contiguous()
+    want = torch.matmul(p, vt).transpose(1, 2)
+    mass = torch.matmul(p, vt.abs()).transpose(1, 2)
+    return want, want.abs() * 2.0 ** -8 + mass * (2.0 ** -8 + D * 2.0 ** -20) + 1e-30
+
+
+# (batch, queries, heads, key heads, position before them): the comment names the workgroup that the rule picks at 128 columns
+SHAPES = [
+    (1, 16, 2, 1, 0), (1, 17, 6, 6, 15), (3, 33, 8, 2, 30), (4, 48, 16, 4, 1000), (1, 257, 8, 8, 31),   # a team of 16
+    (1, 1000, 7, 7, 0), (2, 513, 6, 2, 63), (8, 32, 24, 8, 97),                                         # two teams
+    (2, 1030, 12, 3, 1), (1, 577, 24, 24, 64), (5, 65, 64, 8, 0),                                       # waves of 16
+    (8, 520, 32, 4, 3), (3, 130, 131, 131, 63),                                                         # waves of 32
+]
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,S,H,Hkv,pos", SHAPES)
+def test_shapes_and_their_edges(cuda, B, S, H, Hkv, pos, D):
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(B + S * 3 + H * 7 + pos)
+    q = (torch.randn(B, S, H, D, generator=g, device=cuda) * 2).to(BF)
+    k, v = (torch.randn(B, pos + S + 3, Hkv, D, generator=g, device=cuda).to(BF) for _ in range(2))
+    want, bound = _reference(q, k, v, pos)
+    k[:, pos + S:] = float("nan")  # what lies behind the fed tokens is never used
+    v[:, pos + S:] = float("nan")
+    got = ops.attn_prefill(q.view(B * S, H * D), k, v, H, Hkv, D, pos, S).view(B, S, H, D)
+    assert ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,S,H,Hkv,pos", [(1, 40, 4, 2, 70), (2, 300, 6, 6, 5), (4, 200, 16, 4, 0)])
+@pytest.mark.parametrize("start", [2, 4])
+def test_caches_that_start_anywhere(cuda, B, S, H, Hkv, pos, D, start):
+    """Caches that are not on 16 bytes take the loads through registers."""
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(S)
+    shape = (B, pos + S, Hkv, D)
+    n = B * (pos + S) * Hkv * D
+    q = torch.randn(B, S, H, D, generator=g, device=cuda).to(BF)
+    k, v = (torch.randn(n + 16, generator=g, device=cuda).to(BF)[start:start + n].view(shape) for _ in range(2))
+    want, bound = _reference(q, k, v, pos)
+    got = ops.attn_prefill(q.view(B * S, H * D), k, v, H, Hkv, D, pos, S).view(B, S, H, D)
+    assert ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("B,S,H,pos", [(1, 256, 6, 100), (1, 700, 8, 0), (2, 900, 12, 7)])
+def test_infinities_reach_no_query_before_their_tile(cuda, B, S, H, pos):
+    """An infinite value at one position: what sees it is not finite, and every query whose walk ends before the position's tile
+    of 64 does not depend on it."""
+    from ohara_amd import ops
+
+    D = 128
+    g = torch.Generator(device=cuda).manual_seed(S)
+    q, k, v = (torch.randn(B, n, H, D, generator=g, device=cuda).to(BF) for n in (S, pos + S, pos + S))
+    at = pos + S // 2
+    clean = ops.attn_prefill(q.view(B * S, H * D), k, v, H, H, D, pos, S).view(B, S, H, D)
+    v[:, at] = float("inf")
+    got = ops.attn_prefill(q.view(B * S, H * D), k, v, H, H, D, pos, S).view(B, S, H, D)
+    first = max(0, at // 64 * 64 - 32 - pos)  # 32: queries of one wave
+    assert torch.equal(got[:, :first], clean[:, :first])
+    assert not got[:, at - pos:].isfinite().any()
