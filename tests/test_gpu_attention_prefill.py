@@ -8,7 +8,7 @@ BF = torch.bfloat16
 
 
 def _reference(q, k, v, pos):
-    """In 64 bits, with the bound: weights are rounded to bf16 (2^-9 of each, all of a query's in one direction at worst, against
+    """In 64 bits, with the bound: weights are rounded to bf16 (2^-8 of each, all of a query's in one direction at worst, against
     a sum of unrounded ones), the result once more; a score is an fp32 sum of D products that are 16 together at most, which its
     weight follows."""
     B, S, H, D = q.shape
