@@ -186,10 +186,6 @@ __device__ __forceinline__ float softmax_tile(f32x4 (&s)[NKB], uint4 (&pf)[NWIN]
   return corr;
 }
 
-__device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
 // Queries wq0 + 16 qb + (lane & 15): lane g holds columns 32 j + 8 g .. + 7
 template <int D>
 __device__ __forceinline__ void load_queries(uint4 (&qf)[D / 32], int& qpos, const PrefillArgs& a, int b, int h, int qi, int g) {

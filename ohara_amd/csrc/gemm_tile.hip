@@ -148,13 +148,13 @@ int launch_tile(const GemmArgs& a, int nstrips, hipStream_t st) {
   return ohara_launch_status();
 }
 
-//           waves fragments k-steps slots
-typedef Tile<2, 2, 1, 1, 4, 3> T32;       //  32 x  32
-typedef Tile<2, 2, 2, 2, 4, 2> T64;       //  64 x  64
-typedef Tile<2, 4, 2, 2, 2, 3> T64x128;
-typedef Tile<2, 4, 4, 2, 2, 2> T128;
-typedef Tile<2, 4, 4, 3, 2, 2> T128x192;
-typedef Tile<2, 4, 8, 4, 2, 2> T256;
+//           waves fragments k-steps slots ahead
+typedef Tile<2, 2, 1, 1, 4, 3, 1> T32;       //  32 x  32
+typedef Tile<2, 2, 2, 2, 4, 2, 0> T64;       //  64 x  64
+typedef Tile<2, 4, 2, 2, 2, 3, 1> T64x128;
+typedef Tile<2, 4, 4, 2, 2, 2, 0> T128;
+typedef Tile<2, 4, 4, 3, 2, 2, 0> T128x192;
+typedef Tile<2, 4, 8, 4, 2, 2, 0> T256;
 
 // Which tile: the one that should take least time.  A large tile needs less LDS traffic a product, a small one keeps more
 // CUs busy and its chain of steps is shorter.  The times are measured (33 shapes: 96 to 8192 rows, 768 to 17920 packed

@@ -13,6 +13,14 @@
 //     segments and the low three bits of the row alone it was two cycles a read, 4 being what one takes).
 // One barrier per step: it says that the step's loads have arrived (every wave waits for its own first) and that the slot
 // of the step before is free for the next loads.
+//
+// LA = 0: a k-step's fragments are read, then multiplied; the other waves of the CU fill the gap.  LA = 1, for the tiles with one or
+// two products a wave and activation fragment whose step is a chain: the fragments of the next group of products are read before
+// the present group's, across the barrier too.  us a call, 0 / 1: 32 x 32 tiles, 96 rows 768 x 3072 10.1 / 8.8; 64 x 128, 192 rows
+// 11264 x 2048 22.5 / 21.9; but 64 x 64, 192 rows 2048 x 5632 28.2 / 30.2; 128 x 192, 8192 rows 768 x 768 and 3072 (a mean) 37.0 / 39.5;
+// 256 x 256 with three groups ahead, 4001 rows 11264 x 2048 174 / 180.
+// What K leaves for a last step that is not full has its own code behind the loop: inside, its selects cost every step
+// (128 x 128, 4001 rows: 74.3 / 67.7).
 #pragma once
 #include "common.h"
 
@@ -31,9 +39,9 @@ __device__ __forceinline__ void wait_loads() {  // until at most N of this wave'
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int WM_, int WN_, int FM_, int FN_, int KH_, int NST_>
+template <int WM_, int WN_, int FM_, int FN_, int KH_, int NST_, int LA_>
 struct Tile {
-  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, KH = KH_, NST = NST_;
+  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, KH = KH_, NST = NST_, LA = LA_;
   static constexpr int NW = WM * WN;                       // waves
   static constexpr int TM = WM * FM * 16, TS = WN * FN;    // rows, strips
   static constexpr int RPL = 16 / KH;                      // activation rows of a 1 KiB load
@@ -60,6 +68,10 @@ struct XOffsets {
 
 // acc[u][t]: strip u x row block t of this wave.  ALIGNED: activation rows start on 16 bytes (false: through registers, any).
 // K is a multiple of 8; what the last step reads past it are the row's last piece and the strip's last tile, multiplied by zero.
+__device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
 template <class C, bool ALIGNED>
 __device__ __forceinline__ void tile_product(f32x4 (&acc)[C::FN][C::FM], const char* xb, const XOffsets<C, ALIGNED>& x, const uint4* wp,
                                              int strip0, int nstrips, int K, int wave, int lane, unsigned char* smem) {
@@ -97,43 +109,97 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[C::FN][C::FM], const c
   for (int u = 0; u < FN; ++u)
 #pragma unroll
     for (int t = 0; t < FM; ++t) acc[u][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
-    if (s < nsteps) issue(s, lds0 + s * STAGE);
   const uint32_t xrd = lds0 + (wm * FM * 16 + m) * (64 * KH);
   const uint32_t wrd = lds0 + (XL + wn * FN * KH) * 1024 + lane16;
-  uint32_t so = 0, si = (NST - 1) * STAGE;
-  for (int s = 0; s < nsteps; ++s) {
+  auto x_frag = [&](uint32_t slot, int jj, int t) {
+    return lds16_at(xrd + slot + t * (1024 * KH) + (uint32_t)((4 * jj + g) ^ (m & (4 * KH - 1))) * 16);
+  };
+  auto w_frag = [&](uint32_t slot, int jj, int u) { return lds16_at(wrd + slot + (u * KH + jj) * 1024); };
+  auto arrive = [&](bool all, auto left) {  // the loads of the next step have landed, everyone's
     if (!ALIGNED) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    else if (NST == 2 || s + NST - 2 >= nsteps) wait_loads<0>();
-    else wait_loads<(NST - 2) * LPW>();
+    else if (all) wait_loads<0>();
+    else wait_loads<decltype(left)::value>();
     __builtin_amdgcn_s_barrier();
-    if (s + NST - 1 < nsteps) issue(s + NST - 1, lds0 + si);
+  };
+  constexpr int LA = C::LA, G = KH * FM;
+  constexpr int AHEAD = LA ? NST : NST - 1;  // steps whose loads are in flight
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s)
+    if (s < nsteps) issue(s, lds0 + s * STAGE);
+  uint32_t so = 0;
+  const int nfull = nsteps - (tail ? 1 : 0);
+  if constexpr (LA == 0) {
+    uint32_t si = (NST - 1) * STAGE;
+    for (int s = 0; s < nsteps; ++s) {
+      arrive(NST == 2 || s + NST - 2 >= nsteps, std::integral_constant<int, (NST - 2) * LPW>());
+      if (s + NST - 1 < nsteps) issue(s + NST - 1, lds0 + si);
+      if (s == nfull) break;
+#pragma unroll
+      for (int jj = 0; jj < KH; ++jj) {
+        uint4 xf[FM], wf[FN];
+#pragma unroll
+        for (int u = 0; u < FN; ++u) wf[u] = w_frag(so, jj, u);
+#pragma unroll
+        for (int t = 0; t < FM; ++t) xf[t] = x_frag(so, jj, t);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < FM; ++t)
+#pragma unroll
+          for (int u = 0; u < FN; ++u) acc[u][t] = mfma16(wf[u], xf[t], acc[u][t]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      so = so + STAGE == NST * STAGE ? 0 : so + STAGE;
+      si = si + STAGE == NST * STAGE ? 0 : si + STAGE;
+    }
+  } else {
+    // A group is the products of one activation fragment.  Its fragments are read LA groups before, across the steps: the barrier
+    // stands LA groups before the end of a step, behind the last read of its slot.
+    constexpr int R = LA + 1, W = 2;
+    static_assert(G % R == 0 && KH % W == 0 && LA <= FM, "fragments stay where the unrolled groups expect them");
+    uint4 xf[R], wf[W][FN];
+    auto fetch = [&](uint32_t slot, int i) {
+      if (i % FM == 0) {
+#pragma unroll
+        for (int u = 0; u < FN; ++u) wf[i / FM % W][u] = w_frag(slot, i / FM, u);
+      }
+      xf[i % R] = x_frag(slot, i / FM, i % FM);
+    };
+    arrive(NST > nsteps, std::integral_constant<int, (NST - 1) * LPW>());
+#pragma unroll
+    for (int i = 0; i < LA; ++i) fetch(0, i);
+    for (int s = 0; s < nfull; ++s) {
+      const uint32_t next = so + STAGE == NST * STAGE ? 0 : so + STAGE;
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        if (i == G - LA) {
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          arrive(s + NST > nsteps, std::integral_constant<int, (NST - 2) * LPW>());
+          if (s + NST < nsteps) issue(s + NST, lds0 + so);
+        }
+        if (i + LA < G) fetch(so, i + LA);
+        else fetch(next, i + LA - G);  // (behind the last step: what the slot holds, unused)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < FN; ++u) acc[u][i % FM] = mfma16(wf[i / FM % W][u], xf[i % R], acc[u][i % FM]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      so = next;
+    }
+  }
+  if (tail) {
 #pragma unroll
     for (int jj = 0; jj < KH; ++jj) {
-      // all fragments of a k-step into registers of their own before its products
-      uint4 xf[FM], wf[FN];
-      const uint32_t sw = (uint32_t)((4 * jj + g) ^ (m & (4 * KH - 1))) * 16;
+      const bool in = KB * nfull + 32 * jj + 8 * g < K;
+      uint4 wt[FN];
 #pragma unroll
-      for (int u = 0; u < FN; ++u) wf[u] = lds16_at(wrd + so + (u * KH + jj) * 1024);
+      for (int u = 0; u < FN; ++u) wt[u] = w_frag(so, jj, u);
 #pragma unroll
-      for (int t = 0; t < FM; ++t) xf[t] = lds16_at(xrd + so + t * (1024 * KH) + sw);
-      if (tail && s == nsteps - 1) {
-        const bool in = KB * s + 32 * jj + 8 * g < K;
+      for (int t = 0; t < FM; ++t) {
+        const uint4 xt = in ? x_frag(so, jj, t) : make_uint4(0, 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < FM; ++t) xf[t] = in ? xf[t] : make_uint4(0, 0, 0, 0);
+        for (int u = 0; u < FN; ++u) acc[u][t] = mfma16(wt[u], xt, acc[u][t]);
       }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int t = 0; t < FM; ++t)
-#pragma unroll
-        for (int u = 0; u < FN; ++u)
-          acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[u]),
-                                                              __builtin_bit_cast(bf16x8, xf[t]), acc[u][t], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
     }
-    so = so + STAGE == NST * STAGE ? 0 : so + STAGE;
-    si = si + STAGE == NST * STAGE ? 0 : si + STAGE;
   }
 }
 

@@ -848,8 +848,8 @@ __global__ __launch_bounds__(C::NW * 64, 2) void moe_tile_kernel(ExpertTileArgs 
   }
 }
 
-typedef Tile<2, 4, 2, 2, 2, 3> E64;   //  64 pairs x 128 packed rows
-typedef Tile<2, 4, 4, 2, 2, 2> E128;  // 128 x 128
+typedef Tile<2, 4, 2, 2, 2, 3, 1> E64;   //  64 pairs x 128 packed rows
+typedef Tile<2, 4, 4, 2, 2, 2, 0> E128;  // 128 x 128
 
 template <int EPI, class C>
 int launch_expert_tiles(const ExpertTileArgs& t, int n_pairs, int strips, hipStream_t st) {
