@@ -2,14 +2,15 @@
 //
 // The walk over K is tile_product (lds_tile.h); the sums do not depend on the tile.
 //
-// What bounds it: in large tiles the LDS side and the matrix pipe together (a step of 128 x 192 x 64 takes 0.72 us where its
-// products alone take 0.41 us at the 2.0 GHz the chip holds under them); in small ones the chain barrier - read - multiply
-// of a step (0.135 to 0.34 us).  The kernel before this one (128 x 128, weights straight to registers) against this one,
-// us a call: 8192 rows 6144 x 768 with SwiGLU 114 / 93, 2304 x 768 44.4 / 36.8, 768 x 768 22.7 / 18.2, 768 x 3072 61 / 45;
-// 4001 rows 11264 x 2048 250 / 202, 2048 x 5632 115 / 94; 128 rows 6144 x 768 19.1 / 6.0, 768 x 3072 41.6 / 9.1.
-// Measured and dropped: fragments of the next half step read ahead into registers of their own (no gain at four
-// waves, spills at 256 x 256), the loads spread among the products (they then arrive late: 971 -> 1192 us at 8192^3), deeper
-// rings (no gain, fewer workgroups a CU), four waves a tile of 128 x 192 (99 / 52 us against 93 / 45).
+// What bounds it: in large tiles the loads into LDS, the LDS reads and the matrix pipe together (8192 x 8192 x 8192 on zeros: 815 us;
+// without the loads 615, without the reads 749, with neither 535; on random data the chip's clock falls under the products: 960), in
+// small ones the chain barrier - read - multiply of a step (0.14 to 0.36 us).  The kernel before this one (128 x 128, weights straight to
+// registers) against this one, us a call: 8192 rows 6144 x 768 with SwiGLU 114 / 76, 2304 x 768 44.4 / 31.8, 768 x 768 22.7 / 16.2,
+// 768 x 3072 61 / 44; 4001 rows 11264 x 2048 250 / 160, 2048 x 5632 115 / 86; 128 rows 6144 x 768 19.1 / 6.7, 768 x 3072 41.6 / 8.9.
+// Of that the epilogues (16 bytes a lane a store instead of 4 or 8, silu with a reciprocal of three instructions instead of eleven): 8192
+// rows 6144 x 768 83.5 / 76, 2304 x 768 33.5 / 31.8, 768 x 768 17.1 / 16.2; 4001 rows 11264 x 2048 170 / 160.
+// Measured and dropped: the loads spread among the products (8192^3: 961 -> 1001; with eight k-steps in flight 947, but 128-row tiles
+// 1035 -> 1152), deeper rings (no gain, fewer workgroups a CU), four waves a tile of 128 x 192 (99 / 52 us against 93 / 45 with eight).
 //
 // Workgroup ids go round-robin over the eight XCDs: an XCD gets a contiguous run of tiles, eight activation tiles side
 // by side, so that a run shares its operands in that XCD's L2.
@@ -68,15 +69,18 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
       qoff_t[t] = (size_t)grow * a.ldo;
       coff_t[t] = (((size_t)seq * a.Tmax + pos_t[t]) * a.Hkv) * a.Dh;
     }
+    const bool wide = ((a.ldo | (a.Hkv * a.Dh)) & 7) == 0 && (((uintptr_t)a.out | (uintptr_t)a.kcache | (uintptr_t)a.vcache) & 15) == 0;
+    uint2 left[FM];  // the strip before, where this one completes 16 bytes a lane with it
 #pragma unroll
     for (int u = 0; u < FN; ++u) {
       const int strip = sbase + u;
-      if (strip >= nstrips) continue;
       const int rr = strip * 16;  // uniform: the whole strip lies in one region and one head
-      if (rr >= nq + 2 * nk) continue;
-      const int region = rr < nq ? 0 : (rr < nq + nk ? 1 : 2);
-      const int rloc = rr - (region == 0 ? 0 : (region == 1 ? nq : nq + nk)) + 4 * g;  // column inside q, k or v
-      const int d = (rr - (region == 0 ? 0 : nq)) % a.Dh + 4 * g;
+      if (strip >= nstrips || rr >= nq + 2 * nk) continue;
+      const bool first = wide && !(u & 1) && u + 1 < FN && strip + 1 < nstrips && rr + 16 < nq + 2 * nk, second = wide && (u & 1);
+      auto column = [&](int r) { return r - (r < nq ? 0 : r < nq + nk ? nq : nq + nk); };  // inside q, k or v
+      auto region_of = [&](int r) { return r < nq ? 0 : r < nq + nk ? 1 : 2; };
+      const int region = region_of(rr);
+      const int d = column(rr) % a.Dh + 4 * g;
       uint32_t cv[FM], sv[FM];
       if (region < 2) {
 #pragma unroll
@@ -87,10 +91,13 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
         }
         __builtin_amdgcn_sched_barrier(0);
       }
+      // where this lane stores: its four columns of the strip, or eight of this strip or the one before
+      const int mine = second ? rr - (g & 1 ? 0 : 16) : rr;
+      const int reg = region_of(mine), col = column(mine) + (second ? 8 * (g >> 1) : 4 * g);
+      bf16_t* base = reg == 0 ? a.out : reg == 1 ? a.kcache : a.vcache;
 #pragma unroll
       for (int t = 0; t < FM; ++t) {
         const int b = rbase + t * 16 + m;
-        if (b >= a.B || pos_t[t] < 0 || pos_t[t] >= a.Tmax) continue;
         float v[4] = {rbf(acc[u][t][0]), rbf(acc[u][t][1]), rbf(acc[u][t][2]), rbf(acc[u][t][3])};
         if (region < 2) {
 #pragma unroll
@@ -102,8 +109,100 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
             v[2 * pr + 1] = __fadd_rn(__fmul_rn(e, sn), __fmul_rn(od, c));
           }
         }
-        bf16_t* o = region == 0 ? a.out + qoff_t[t] + rloc : (region == 1 ? a.kcache : a.vcache) + coff_t[t] + rloc;
-        *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
+        const uint2 w = make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
+        if (first) {
+          left[t] = w;
+          continue;
+        }
+        const bool in = b < a.B && pos_t[t] >= 0 && pos_t[t] < a.Tmax;
+        bf16_t* o = base + (reg == 0 ? qoff_t[t] : coff_t[t]) + col;
+        if (second) {
+          const u32x2 x = __builtin_amdgcn_permlane16_swap(left[t].x, w.x, false, false);
+          const u32x2 y = __builtin_amdgcn_permlane16_swap(left[t].y, w.y, false, false);
+          if (in) *reinterpret_cast<uint4*>(o) = make_uint4(x[0], y[0], x[1], y[1]);
+        } else if (in) {
+          *reinterpret_cast<uint2*>(o) = w;
+        }
+      }
+    }
+    return;
+  }
+  // Two strips' (four strips') columns lie side by side in a row of the output; exchanged among the lanes of a row they are stored,
+  // and a residual read, 16 bytes a lane.
+  const bool wide = ((a.N | a.ldo) & 7) == 0 && ((uintptr_t)a.out & 15) == 0;
+  if (EPI == EPI_SWIGLU && FN > 1 && wide) {
+#pragma unroll
+    for (int t = 0; t < FM; ++t) {
+      const int b = rbase + t * 16 + m;
+      float low = acc[0][t][0];
+#pragma unroll
+      for (int u = 0; u < FN; ++u) low = fminf(low, fminf(acc[u][t][0], acc[u][t][1]));
+      uint32_t w[FN];  // two columns of strip u
+      if (__any(low < -86.5f)) {  // (-87 after rounding)
+#pragma unroll
+        for (int u = 0; u < FN; ++u)
+          w[u] = pack_bf(rbf(silu_f(rbf(acc[u][t][0]))) * rbf(acc[u][t][2]), rbf(silu_f(rbf(acc[u][t][1]))) * rbf(acc[u][t][3]));
+      } else {
+#pragma unroll
+        for (int u = 0; u < FN; ++u)
+          w[u] = pack_bf(rbf(silu_from_m87(rbf(acc[u][t][0]))) * rbf(acc[u][t][2]),
+                         rbf(silu_from_m87(rbf(acc[u][t][1]))) * rbf(acc[u][t][3]));
+      }
+      bf16_t* o = a.out + (size_t)b * a.ldo + sbase * 8;
+      const int left = b < a.B ? a.N - sbase * 8 : 0;  // columns this row still has
+      int u = 0;
+      if constexpr (FN >= 4) {
+        const u32x2 p = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false), q = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+        const u32x2 c = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false), d = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+        if (8 * g < left) *reinterpret_cast<uint4*>(o + 8 * g) = make_uint4(c[0], c[1], d[0], d[1]);
+        u = 4;
+      } else {
+        const u32x2 c = __builtin_amdgcn_permlane16_swap(w[0], w[1], false, false);
+        const int at = 8 * (g & 1) + 4 * (g >> 1);
+        if (at < left) *reinterpret_cast<uint2*>(o + at) = make_uint2(c[0], c[1]);
+        u = 2;
+      }
+#pragma unroll
+      for (; u < FN; ++u)
+        if (8 * u + 2 * g < left) *reinterpret_cast<uint32_t*>(o + 8 * u + 2 * g) = w[u];
+    }
+    return;
+  }
+  if ((EPI == EPI_STORE || EPI == EPI_RESIDUAL) && FN > 1 && wide &&
+      (EPI == EPI_STORE || ((a.ldr & 7) == 0 && ((uintptr_t)a.resid & 15) == 0))) {
+#pragma unroll
+    for (int u = 0; u + 1 < FN; u += 2) {
+      const int col = (sbase + u + (g & 1)) * 16 + 8 * (g >> 1);
+      uint4 res[FM];
+      if (EPI == EPI_RESIDUAL) {
+#pragma unroll
+        for (int t = 0; t < FM; ++t)
+          res[t] = *reinterpret_cast<const uint4*>(a.resid + (size_t)min(rbase + t * 16 + m, a.B - 1) * a.ldr + min(col, a.N - 8));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int t = 0; t < FM; ++t) {
+        const int b = rbase + t * 16 + m;
+        const u32x2 c = __builtin_amdgcn_permlane16_swap(pack_bf(acc[u][t][0], acc[u][t][1]), pack_bf(acc[u + 1][t][0], acc[u + 1][t][1]), false, false);
+        const u32x2 d = __builtin_amdgcn_permlane16_swap(pack_bf(acc[u][t][2], acc[u][t][3]), pack_bf(acc[u + 1][t][2], acc[u + 1][t][3]), false, false);
+        uint4 v = make_uint4(c[0], d[0], c[1], d[1]);
+        if (EPI == EPI_RESIDUAL) {
+          auto sum = [](uint32_t r, uint32_t y) { return pack_bf(lo_bf(r) + lo_bf(y), hi_bf(r) + hi_bf(y)); };
+          v = make_uint4(sum(res[t].x, v.x), sum(res[t].y, v.y), sum(res[t].z, v.z), sum(res[t].w, v.w));
+        }
+        if (b < a.B && col < a.N) *reinterpret_cast<uint4*>(a.out + (size_t)b * a.ldo + col) = v;
+      }
+    }
+    if (FN & 1) {
+      constexpr int u = FN - 1;
+      EpiPre pre[FM];
+#pragma unroll
+      for (int t = 0; t < FM; ++t) gemm_epilogue_fetch<EPI>(a, rbase + t * 16 + m, min(sbase + u, nstrips - 1), g, pre[t]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < FM; ++t) {
+        const int b = rbase + t * 16 + m;
+        if (b < a.B && sbase + u < nstrips) gemm_epilogue<EPI, true>(a, b, sbase + u, g, acc[u][t], pre[t]);
       }
     }
     return;
@@ -157,8 +256,8 @@ typedef Tile<2, 4, 4, 3, 2, 2, 0> T128x192;
 typedef Tile<2, 4, 8, 4, 2, 2, 0> T256;
 
 // Which tile: the one that should take least time.  A large tile needs less LDS traffic a product, a small one keeps more
-// CUs busy and its chain of steps is shorter.  The times are measured (33 shapes: 96 to 8192 rows, 768 to 17920 packed
-// rows, K 768 to 10240); the choice they give is within 1 % of the best of the six on average, 20 % at worst.
+// CUs busy and its chain of steps is shorter.  The times are fitted to measurements (63 shapes: 96 to 11200 rows, 768 to 17920 packed
+// rows, K 768 to 10240); the choice they give is within 0.4 % of the best of the six on average, 13 % at worst.
 struct TileTime {
   int rows, strips;
   int slots;    // workgroups that share a CU
@@ -168,9 +267,9 @@ struct TileTime {
   float ends;   // us the start and the epilogue add
 };
 constexpr TileTime TIMES[6] = {
-    {T32::TM, T32::TS, 3, 0.135f, 0.25f, 0.10f, 0.9f},        {T64::TM, T64::TS, 2, 0.25f, 0.3f, 0.215f, 1.3f},
-    {T64x128::TM, T64x128::TS, 2, 0.335f, 0.4f, 0.37f, 1.6f}, {T128::TM, T128::TS, 2, 0.50f, 0.8f, 0.54f, 2.5f},
-    {T128x192::TM, T128x192::TS, 2, 0.74f, 0.75f, 0.72f, 3.0f}, {T256::TM, T256::TS, 1, 1.70f, 1.0f, 1.75f, 8.0f},
+    {T32::TM, T32::TS, 3, 0.14f, 0.376f, 0.079f, 0.43f},        {T64::TM, T64::TS, 2, 0.295f, 0.23f, 0.189f, 0.6f},
+    {T64x128::TM, T64x128::TS, 2, 0.363f, 0.61f, 0.312f, 1.3f}, {T128::TM, T128::TS, 2, 0.60f, 0.56f, 0.453f, 1.45f},
+    {T128x192::TM, T128x192::TS, 2, 0.747f, 0.64f, 0.6f, 3.15f}, {T256::TM, T256::TS, 1, 1.35f, 1.0f, 1.6f, 6.7f},
 };
 float tile_time(const TileTime& t, int rows, int strips, int K) {
   constexpr int CUS = 256;

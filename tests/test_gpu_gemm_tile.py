@@ -70,3 +70,87 @@ def test_infinities_stay_in_their_row(cuda):
     assert torch.equal(got[17].isnan(), want.isnan())
     at = ~want.isnan()
     assert torch.equal(got[17][at].double(), want[at])
+
+
+# 96 rows take tiles that are 32 rows high, 4100 tiles of 192 columns, 9000 tiles of 256
+@pytest.mark.parametrize("rows,f", [(96, 264), (300, 3072), (1100, 1544), (2100, 5632), (4100, 1160), (9000, 3080)])
+@pytest.mark.parametrize("pad", [0, 1, 4])
+def test_stores_of_16_bytes_and_less(cuda, rows, f, pad):
+    """Gates and sums stored 16 bytes a lane, and through rows that leave no room for that: the same bits; and the gates of the skinny
+    kernels, which have their reciprocal from another unit."""
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(rows + f)
+    k = 72
+    x = (torch.randn(rows, k, generator=g, device=cuda) * 4).to(BF)
+    wg, wu = ((torch.randn(f, k, generator=g, device=cuda)).to(BF) for _ in range(2))
+    gates, flat = ops.pack_gate_up(wg, wu), ops.pack_linear(wg)
+    odd = torch.full((rows, f + pad), 7.0, dtype=BF, device=cuda)
+    ops.gemm(x, gates, out=odd[:, :f])
+    skinny = torch.cat([ops.gemm_skinny(x[i:i + 64], gates) for i in range(0, min(rows, 320), 64)])[:320]
+    assert (odd[:320, :f] != skinny).float().mean() <= 0.01  # sums over K in another order: last places
+    gate, up = (x.double() @ w.double().t() for w in (wg, wu))
+    want = gate * torch.sigmoid(gate) * up
+    # silu, up and product are each rounded to bf16, and the gate, which silu follows with a slope of at most 1.1; sums are in fp32
+    err_gate, err_up = (k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) for w in (wg, wu))
+    silu = (gate * torch.sigmoid(gate)).abs()
+    bound = 1.02 * (silu * (up.abs() * 3 * 2.0 ** -8 + err_up) + 1.1 * (gate.abs() * 2.0 ** -8 + err_gate) * up.abs()) + 1e-30
+    assert ((odd[:, :f].double() - want).abs() <= bound).all()
+    assert (odd[:, f:] == 7.0).all()
+    res = torch.randn(rows, f + pad, generator=g, device=cuda).to(BF)
+    for resid in (None, res[:, :f]):
+        ops.gemm(x, flat, residual=resid, out=odd[:, :f])
+        assert torch.equal(odd[:, :f], ops.gemm(x, flat, residual=None if resid is None else resid.contiguous()))
+        assert (odd[:, f:] == 7.0).all()
+
+
+def test_gate_of_every_value(cuda):
+    """silu over every bf16 number, the ones where its short form does not hold among them, against the kernel of few rows."""
+    from ohara_amd import ops
+
+    v = torch.arange(-32768, 32768, dtype=torch.int32, device=cuda).to(torch.int16).view(BF)
+    v = v[v.isfinite()]
+    v = torch.cat([v, torch.zeros(-v.numel() % 64, dtype=BF, device=cuda)])
+    v = v.view(64, -1).t().contiguous().view(-1)  # rows of a fragment from all over the range
+    x = torch.zeros(v.numel(), 8, dtype=BF, device=cuda)
+    x[:, 0], x[:, 1] = v, 1.0
+    wg, wu = (torch.zeros(64, 8, dtype=BF, device=cuda) for _ in range(2))
+    wg[:, 0], wu[:, 1] = 1.0, 1.0
+    w = ops.pack_gate_up(wg, wu)
+    for part in (x, x[x[:, 0] > -87]):  # the second without a row that takes the long form
+        got = ops.gemm(part, w)
+        want = torch.cat([ops.gemm_skinny(part[i:i + 64].contiguous(), w) for i in range(0, part.shape[0], 64)])
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("B,S,H,Hkv,D,K", [(2, 100, 6, 6, 128, 768), (3, 90, 3, 1, 48, 64), (5, 300, 5, 5, 80, 136), (1, 2100, 9, 3, 64, 328),
+                                           (9, 1000, 16, 4, 128, 520)])
+def test_rotary_regions_and_their_edges(cuda, B, S, H, Hkv, D, K):
+    """Strips of q, k and v side by side in one store, also where the regions start on an odd strip, against 64 bits."""
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(S)
+    pos, T = 3, S + 8
+    x = torch.randn(B * S, K, generator=g, device=cuda).to(BF)
+    wq, wk, wv = ((torch.randn(n * D, K, generator=g, device=cuda) * 0.1).to(BF) for n in (H, Hkv, Hkv))
+    ang = torch.rand(T, D // 2, generator=g, device=cuda) * 6.28
+    cos, sin = ang.cos().to(BF), ang.sin().to(BF)
+    kc, vc = (torch.full((B, T, Hkv, D), 9.0, dtype=BF, device=cuda) for _ in range(2))
+    q = ops.qkv_rope_append(x, ops.pack_qkv(wq, wk, wv), None, 1e-5, H, Hkv, D, cos, sin, pos, kc, vc, seq_len=S).view(B, S, H, D)
+    assert (kc[:, :pos] == 9.0).all() and (kc[:, pos + S:] == 9.0).all()
+    assert (vc[:, :pos] == 9.0).all() and (vc[:, pos + S:] == 9.0).all()
+
+    def plain(w, n):
+        y, mass = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+        return y.view(B, S, n, D), (y.abs() * 2.0 ** -8 + K * 2.0 ** -24 * mass).view(B, S, n, D)
+
+    def turned(w, n):
+        y, e = plain(w, n)
+        c, s = (t[pos:pos + S].double()[None, :, None] for t in (cos, sin))
+        a, b, ea, eb = y[..., 0::2], y[..., 1::2], e[..., 0::2], e[..., 1::2]
+        want = torch.stack([a * c - b * s, a * s + b * c], -1).flatten(-2)
+        bound = torch.stack([ea * c.abs() + eb * s.abs(), ea * s.abs() + eb * c.abs()], -1).flatten(-2)
+        return want, bound + want.abs() * 2.0 ** -8 + bound * 2.0 ** -7
+
+    for got, (want, bound) in ((q, turned(wq, H)), (kc[:, pos:pos + S], turned(wk, Hkv)), (vc[:, pos:pos + S], plain(wv, Hkv))):
+        assert ((got.double() - want).abs() <= bound + 1e-30).all()
