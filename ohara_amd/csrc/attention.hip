@@ -26,10 +26,11 @@ struct AttnArgs {
   int B, S, H, Hkv, D, Tmax, start;  // query s of sequence b sees positions [0, start + s]
   const int32_t* pos_dev;            // when set: start = *pos_dev, or pos_dev[sequence] with pos_stride 1
   int pos_stride;
-  int nsplit;
+  int nsplit;        // chunks there is room for
+  int most;          // chunks that pay where the walk is what takes the time (0: where the memory is), see cut_context
   int* counters;     // (B*Hkv)
-  float* part_ml;    // (B, H, nsplit, 2)
-  float* part_acc;   // (B, H, nsplit, D)
+  float* part_ml;    // (B, Hkv, nsplit of room: G, chunks, 2)
+  float* part_acc;   // (B, Hkv, nsplit of room: G, chunks, D)
   float scale;
 };
 
@@ -60,13 +61,13 @@ __device__ __forceinline__ void stf_coh(float* p, float v) { st_coh4(p, __float_
 // Needs G * n_split <= OHARA_MERGE_CAP.
 #define OHARA_MERGE_CAP 2048
 template <int MAXD>
-__device__ void merge_partials(const AttnArgs& a, int b /* query row */, int kvh, int G) {
+__device__ void merge_partials(const AttnArgs& a, int b /* query row */, int kvh, int G, int ns) {
   __shared__ float s_w[OHARA_MERGE_CAP];   // max, then weight, of (head, chunk)
   __shared__ float s_ls[OHARA_MERGE_CAP];  // sum of (head, chunk)
   __shared__ float s_tot[64];              // per head: normaliser
-  const int D = a.D, ns = a.nsplit;
+  const int D = a.D;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const float* ml0 = a.part_ml + ((size_t)(b * a.H + kvh * G) * ns) * 2;  // heads of a group are adjacent
+  const float* ml0 = a.part_ml + ((size_t)(b * a.H + kvh * G) * a.nsplit) * 2;  // heads of a group are adjacent
   for (int i = tid; i < G * ns; i += blockDim.x) {
     const uint2 v = ld_coh8(ml0 + 2 * (size_t)i);
     s_w[i] = __uint_as_float(v.x);
@@ -91,7 +92,7 @@ __device__ void merge_partials(const AttnArgs& a, int b /* query row */, int kvh
   for (int idx = tid; idx < G * D; idx += blockDim.x) {
     const int hh = idx / D, d = idx - hh * D;
     const int h = kvh * G + hh;
-    const float* pa = a.part_acc + ((size_t)(b * a.H + h) * ns) * D + d;
+    const float* pa = a.part_acc + ((size_t)(b * a.H + kvh * G) * a.nsplit + (size_t)hh * ns) * D + d;
     const float* w = s_w + hh * ns;
     float o = 0.f;
     // Up to 32 chunks' values are in flight at once, every load unconditional (chunks past the last
@@ -108,6 +109,29 @@ __device__ void merge_partials(const AttnArgs& a, int b /* query row */, int kvh
     }
     a.out[(size_t)b * a.H * D + h * D + d] = f2bf(o * (1.0f / s_tot[hh]));
   }
+}
+
+// Into how many of the caller's n_split chunks a context of L positions is cut, from what is known only here (L may live on the
+// device): merging costs a launch about 3 us and every chunk 0.1 to 0.2 more, a workgroup walks 64 positions in 0.8, and with more
+// than 128 (row, head) pairs the memory is busy without a cut.  A call's workgroups all come to the same answer; the ones
+// without a chunk leave.  us a launch, 1 / 4 / 8 / 16 chunks, heads of 128 (the caller asks for about 1024 workgroups):
+//   64 pairs, 4 int8 heads each  100 positions 5.2 / 9.1 / 9.4 / 12.4;  300  9.4 / 10.0 / 10.2 / 13.0;  700  15.2 / 12.3 / 11.9 / 14.8;
+//                                1900  29.7 / 16.7 / 16.4 / 19.1;  4000  55 / 23.9 / 24.3 / 25.7
+//   64 pairs, 4 heads            700  16.0 / 12.3 / 13.8 / 16.1;  1900  34.9 / 18.3 / 20.3 / 22.2;  4000  68 / 28.8 / 31.0 / 33.0
+//   96 pairs (1 / 5 / 8 / 10)    100  4.9 / 7.0 / 7.5 / 8.2;  300  8.3 / 8.5 / 8.9 / 9.5;  530  12.0 / 10.7 / 10.8 / 11.3;
+//                                1500  27.6 / 17.6 / 17.0 / 17.5;  4000  65 / 37.4 / 36.3 / 39.8
+//   192 pairs (1 / 4 / 5)        100  5.0 / 7.8 / 7.8;  530  13.2 / 16.0 / 14.3;  700  16.4 / 17.4 / 17.7;  1500  30.5 / 28.7 / 29.4
+//   12 pairs (1 / 8 / 16 / 32)   300  6.6 / 6.8 / 7.3 / 9.8;  700  12.5 / 7.9 / 8.1 / 9.8;  4000  56 / 14.3 / 11.7 / 12.7
+struct Cut {
+  int chunk, used;
+};
+__device__ __forceinline__ Cut cut_context(const AttnArgs& a, int L, int unit /* positions of a workgroup's step */) {
+  const int n64 = (L + 63) >> 6;
+  int want = a.nsplit;
+  if (n64 <= 5 || (a.most == 0 && n64 <= 12)) want = 1;
+  else if (a.most) want = min(want, min((n64 + 1) >> 1, a.most));
+  const int chunk = max((L + want - 1) / want + unit - 1, unit) & ~(unit - 1);
+  return {chunk, max((L + chunk - 1) / chunk, 1)};
 }
 
 // Counts this workgroup's chunk as done and returns true in the workgroup that observes all
@@ -139,7 +163,8 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
   const int split = blockIdx.z, kvh = blockIdx.y, b = blockIdx.x;  // b: query row = seq * S + s
   const int seq = b / a.S;
   const int L = min((a.pos_dev ? a.pos_dev[(size_t)seq * a.pos_stride] : a.start) + (b - seq * a.S) + 1, a.Tmax);
-  const int chunk = (((L + a.nsplit - 1) / a.nsplit) + 63) & ~63;
+  const auto [chunk, used] = cut_context(a, L, 64);
+  if (split >= used) return;
   const int t0 = split * chunk;
   const int t1 = min(L, t0 + chunk);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -327,19 +352,19 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
       Ls += s_l[w][hh] * sc;
       o += s_acc[w][hh][d] * sc;
     }
-    if (a.nsplit == 1) {  // whole context in this workgroup: no partials
+    if (used == 1) {  // whole context in this workgroup: no partials
       a.out[(size_t)b * a.H * D + h * D + d] = f2bf(o * (1.0f / Ls));
       continue;
     }
-    const size_t pi = (size_t)(b * a.H + h) * a.nsplit + split;
+    const size_t pi = (size_t)(b * a.H + kvh * G) * a.nsplit + (size_t)hh * used + split;
     stf_coh(a.part_acc + pi * D + d, o);
     if (d == 0) {
       stf_coh(a.part_ml + pi * 2, M);
       stf_coh(a.part_ml + pi * 2 + 1, Ls);
     }
   }
-  if (a.nsplit == 1) return;
-  if (last_chunk_done(a.counters + b * a.Hkv + kvh, a.nsplit)) merge_partials<D>(a, b, kvh, G);
+  if (used == 1) return;
+  if (last_chunk_done(a.counters + b * a.Hkv + kvh, used)) merge_partials<D>(a, b, kvh, G, used);
 }
 
 
@@ -370,7 +395,8 @@ __global__ __launch_bounds__(256, (G == 1 ? 3 : 2)) void attn_decode_i8_kernel(A
   const int split = blockIdx.z, kvh = blockIdx.y, b = blockIdx.x;  // b: query row = seq * S + s
   const int seq = b / a.S;
   const int L = min((a.pos_dev ? a.pos_dev[(size_t)seq * a.pos_stride] : a.start) + (b - seq * a.S) + 1, a.Tmax);
-  const int chunk = (((L + a.nsplit - 1) / a.nsplit) + 127) & ~127;
+  const auto [chunk, used] = cut_context(a, L, 128);
+  if (split >= used) return;
   const int t0 = split * chunk;
   const int t1 = min(L, t0 + chunk);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -568,19 +594,19 @@ __global__ __launch_bounds__(256, (G == 1 ? 3 : 2)) void attn_decode_i8_kernel(A
       Ls += s_l[w][hh] * scw;
       o += s_acc[w][hh][d] * scw;
     }
-    if (a.nsplit == 1) {  // whole context in this workgroup: no partials
+    if (used == 1) {  // whole context in this workgroup: no partials
       a.out[(size_t)b * a.H * D + h * D + d] = f2bf(o * (1.0f / Ls));
       continue;
     }
-    const size_t pi = (size_t)(b * a.H + h) * a.nsplit + split;
+    const size_t pi = (size_t)(b * a.H + kvh * G) * a.nsplit + (size_t)hh * used + split;
     stf_coh(a.part_acc + pi * D + d, o);
     if (d == 0) {
       stf_coh(a.part_ml + pi * 2, M);
       stf_coh(a.part_ml + pi * 2 + 1, Ls);
     }
   }
-  if (a.nsplit == 1) return;
-  if (last_chunk_done(a.counters + b * a.Hkv + kvh, a.nsplit)) merge_partials<D>(a, b, kvh, G);
+  if (used == 1) return;
+  if (last_chunk_done(a.counters + b * a.Hkv + kvh, used)) merge_partials<D>(a, b, kvh, G, used);
 }
 
 // Head width 128 over the int8 cache with BOTH products on the matrix cores.  What a position costs in the
@@ -607,7 +633,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_i8_mfma_kernel(AttnArgs a)
   const int split = blockIdx.z, kvh = blockIdx.y, b = blockIdx.x;
   const int seq = b / a.S;
   const int L = min((a.pos_dev ? a.pos_dev[(size_t)seq * a.pos_stride] : a.start) + (b - seq * a.S) + 1, a.Tmax);
-  const int chunk = (((L + a.nsplit - 1) / a.nsplit) + 127) & ~127;
+  const auto [chunk, used] = cut_context(a, L, 128);
+  if (split >= used) return;
   const int t0 = split * chunk;
   const int t1 = min(L, t0 + chunk);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -777,19 +804,19 @@ __global__ __launch_bounds__(256, 2) void attn_decode_i8_mfma_kernel(AttnArgs a)
       Ls += s_l[w][hh] * scw;
       o += s_acc[w][hh][d] * scw;
     }
-    if (a.nsplit == 1) {  // whole context in this workgroup: no partials
+    if (used == 1) {  // whole context in this workgroup: no partials
       a.out[(size_t)b * a.H * D + h * D + d] = f2bf(o * (1.0f / Ls));
       continue;
     }
-    const size_t pi = (size_t)(b * a.H + h) * a.nsplit + split;
+    const size_t pi = (size_t)(b * a.H + kvh * G) * a.nsplit + (size_t)hh * used + split;
     stf_coh(a.part_acc + pi * D + d, o);
     if (d == 0) {
       stf_coh(a.part_ml + pi * 2, M);
       stf_coh(a.part_ml + pi * 2 + 1, Ls);
     }
   }
-  if (a.nsplit == 1) return;
-  if (last_chunk_done(a.counters + b * a.Hkv + kvh, a.nsplit)) merge_partials<D>(a, b, kvh, G);
+  if (used == 1) return;
+  if (last_chunk_done(a.counters + b * a.Hkv + kvh, used)) merge_partials<D>(a, b, kvh, G, used);
 }
 
 // Any even head width up to 256, any group size: one thread per position for q.k,
@@ -877,7 +904,7 @@ __global__ __launch_bounds__(256) void attn_decode_generic(AttnArgs a) {
     }
   }
   if (a.nsplit == 1) return;
-  if (last_chunk_done(a.counters + b * a.Hkv + kvh, a.nsplit)) merge_partials<256>(a, b, kvh, G);
+  if (last_chunk_done(a.counters + b * a.Hkv + kvh, a.nsplit)) merge_partials<256>(a, b, kvh, G, a.nsplit);
 }
 
 template <int D, bool I8>
@@ -942,6 +969,8 @@ static int attn_cached_impl(const uint16_t* q, const void* kcache, const void* v
   a.pos_stride = pos_stride;
   a.nsplit = n_split;
   batch *= seq_len;  // one workspace slot per query row
+  const int64_t pairs = (int64_t)batch * h_kv;
+  a.most = pairs <= 80 ? (int)(256 / pairs) : pairs <= 128 ? (int)(512 / pairs) : 0;  // one workgroup a CU where that is even, or two
   char* ws = reinterpret_cast<char*>(workspace);
   a.counters = reinterpret_cast<int*>(ws);
   ws += fixed_counter_bytes ? fixed_counter_bytes : align256((size_t)batch * h_kv * sizeof(int));
