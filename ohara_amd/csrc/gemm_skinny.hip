@@ -282,6 +282,128 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
   }
 }
 
+// Normed rows against 257 to 1024 strips, K <= 2048: S strips a workgroup, as many as make about one workgroup a CU of them.
+// Above, every strip's workgroup norms the rows again (48 vector instructions a lane and k-step: 704 strips at 32 rows kept the
+// chip busy for half of the launch) and its loads come in rounds.  Here NW waves split K so far that a wave's share is at
+// most SP k-steps: rows, norm weights and the weights of all S strips are requested before anything waits, and a normed
+// fragment is used S times.  The waves' sums meet in LDS and are added in the order of the waves, a wave to a fragment.
+template <int BT, int EPI, int S, int NW, int SP>
+__global__ __launch_bounds__(NW * 64) void group_kernel(GemmArgs a) {
+  extern __shared__ __align__(16) unsigned char group_smem[];
+  f32x4(*red)[S * BT][64] = reinterpret_cast<f32x4(*)[S * BT][64]>(group_smem);
+  __shared__ float ssq[NW][BT * 16];
+  const int strip0 = blockIdx.x * S, rbase = blockIdx.y * 16 * BT;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 15, g = lane >> 4;
+  const int KS = (a.K + 31) >> 5;
+  const int per_wave = (KS + NW - 1) / NW;
+  const int j0 = wave * per_wave, j1 = min(KS, j0 + per_wave);
+
+  uint4 xv[SP][BT], nw[SP], wv[SP][S];
+#pragma unroll
+  for (int c = 0; c < SP; ++c) {
+    const int k0 = 32 * (j0 + c) + 8 * g;
+#pragma unroll
+    for (int t = 0; t < BT; ++t) {
+      const int b = rbase + m + 16 * t;
+      const bool in = j0 + c < j1 && b < a.B && k0 < a.K;
+      xv[c][t] = ldg16(a.x + (in ? (size_t)b * a.ldx + k0 : (size_t)0));
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < SP; ++c) {
+    const int k0 = 32 * (j0 + c) + 8 * g;
+    nw[c] = ldg16(a.norm_w + (j0 + c < j1 && k0 < a.K ? k0 : 0));
+  }
+#pragma unroll
+  for (int u = 0; u < S; ++u)
+#pragma unroll
+    for (int c = 0; c < SP; ++c)
+      wv[c][u] = ldg16_nt(a.wp + ((size_t)min(strip0 + u, a.nstrips - 1) * KS + min(j0 + c, KS - 1)) * 64 + lane);
+  const bool pre_ok = EPI == EPI_ROPE && ((a.N | a.ldo) & 3) == 0;
+  EpiPre ep;
+  if (pre_ok && wave < S * BT) gemm_epilogue_fetch<EPI>(a, rbase + m + 16 * (wave % BT), min(strip0 + wave / BT, a.nstrips - 1), g, ep);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int t = 0; t < BT; ++t) {
+    float part = 0.f;
+#pragma unroll
+    for (int c = 0; c < SP; ++c)
+      if (j0 + c < j1 && rbase + m + 16 * t < a.B && 32 * (j0 + c) + 8 * g < a.K) part += sumsq8(xv[c][t]);
+    part = lanes_sum<32, 32>(lanes_sum<16, 16>(part));
+    if (g == 0) ssq[wave][16 * t + m] = part;
+  }
+  __syncthreads();
+  f32x4 acc[S][BT];
+#pragma unroll
+  for (int t = 0; t < BT; ++t) {
+    float tot = ssq[0][16 * t + m];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) tot += ssq[w][16 * t + m];
+    const float rinv = 1.0f / sqrtf(tot / (float)a.K + a.eps);
+#pragma unroll
+    for (int u = 0; u < S; ++u) acc[u][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < SP; ++c) {
+      const bool in = j0 + c < j1 && rbase + m + 16 * t < a.B && 32 * (j0 + c) + 8 * g < a.K;
+      const uint4 xn = in ? norm8(xv[c][t], nw[c], rinv) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < S; ++u)
+        acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[c][u]), __builtin_bit_cast(bf16x8, xn),
+                                                            acc[u][t], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < S; ++u)
+#pragma unroll
+    for (int t = 0; t < BT; ++t) red[wave][u * BT + t][lane] = acc[u][t];
+  __syncthreads();
+  if (wave >= S * BT) return;
+  const int strip = strip0 + wave / BT, b = rbase + m + 16 * (wave % BT);
+  f32x4 sum = red[0][wave][lane];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) sum += red[w][wave][lane];
+  if (strip >= a.nstrips || b >= a.B) return;
+  if (pre_ok) gemm_epilogue<EPI, true>(a, b, strip, g, sum, ep);
+  else gemm_epilogue<EPI>(a, b, strip, g, sum);
+}
+
+template <int BT, int EPI, int S, int NW, int SP>
+int launch_group_s(const GemmArgs& a, hipStream_t st) {
+  static_assert(S * BT <= NW, "a wave to a fragment");
+  constexpr int LDS = NW * S * BT * 1024;
+  if (LDS > 60 * 1024)
+    (void)hipFuncSetAttribute((const void*)group_kernel<BT, EPI, S, NW, SP>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  hipLaunchKernelGGL((group_kernel<BT, EPI, S, NW, SP>), dim3((a.nstrips + S - 1) / S, (a.B + 16 * BT - 1) / (16 * BT)), dim3(NW * 64), LDS, st, a);
+  return ohara_launch_status();
+}
+template <int BT, int EPI>
+int launch_group_bt(const GemmArgs& a, hipStream_t st) {
+  const int per_cu = (a.nstrips + 255) / 256;
+  if (a.K <= 1024) switch (per_cu) {
+    case 2: return launch_group_s<BT, EPI, 2, 8, 4>(a, st);
+    case 3: return launch_group_s<BT, EPI, 3, 8, 4>(a, st);
+    default: return launch_group_s<BT, EPI, 4, 8, 4>(a, st);
+  }
+  switch (per_cu) {
+    case 2: return launch_group_s<BT, EPI, 2, 16, 4>(a, st);
+    case 3: return launch_group_s<BT, EPI, 3, 16, 4>(a, st);
+    default: return launch_group_s<1, EPI, 4, 16, 4>(a, st);  // (four strips and 32 rows at once do not fit the registers)
+  }
+}
+// us a call, a strip's workgroup each (four waves) / this kernel, 1, 16, 32 and 64 rows:
+//   11264 x 2048  14.8 20.1 33.9 58 / 10.7 11.1 15.8 29.4      6144 x 768  5.25 6.2 7.6 11.4 / 4.65 5.0 6.5 9.4
+//   8192 x 1024    6.1  6.8  9.5 15.4 / 5.4  5.4  7.6 12.9
+// With fewer strips than CUs a group is one strip, and there it is no faster: 2304 x 768 3.7 4.3 5.7 7.2 / 3.8 4.2 5.6 7.8; 3072 x 2048
+// with eight waves a strip 6.0 6.9 11.9 16.9 / 6.8 7.0 10.7 19.6.
+bool group_applies(const GemmArgs& a, int epi, int strips) {
+  return a.norm_w && (epi == EPI_STORE || epi == EPI_SWIGLU || epi == EPI_ROPE) && strips > 256 && strips <= 1024 && a.K <= 2048;
+}
+template <int EPI>
+int launch_group(const GemmArgs& a, hipStream_t st) {  // past 32 rows, sixteen a workgroup where its K is short
+  return a.B <= 16 || (a.B > 32 && a.K <= 1024) ? launch_group_bt<1, EPI>(a, st) : launch_group_bt<2, EPI>(a, st);
+}
+
 // Many strips (the vocabulary projection): the activations are the stationary operand.  Every
 // workgroup normalises all rows once into LDS (up to 64 rows, zero-padded to
 // 16*BT rows and 32*KS columns), then each of its 8 waves walks whole strips - full K, no
@@ -467,6 +589,13 @@ int launch_epi(const GemmArgs& a, int epi, int strips, hipStream_t st) {
     }
     return ohara_launch_status();
   }
+  // Normed rows of 1025 to 2048 columns: eight waves, so that a wave's share of K is requested in one go (3072 x 2048, 1, 16, 32 and 64
+  // rows: 9.0, 10.2, 13.9, 18.7 us with four, 6.0, 6.9, 11.9, 16.9 with eight).
+  if (NORM && a.K > 1024 && a.K <= 2048 && (epi == EPI_STORE || epi == EPI_ROPE)) {
+    if (epi == EPI_STORE) hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_STORE, 8>), grid, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_ROPE, 8>), grid, dim3(512), 0, st, a);
+    return ohara_launch_status();
+  }
   switch (epi) {
     case EPI_STORE: hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_STORE>), grid, block, 0, st, a); break;
     case EPI_RESIDUAL: hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_RESIDUAL>), grid, block, 0, st, a); break;
@@ -505,6 +634,10 @@ int launch_chunk(const GemmArgs& a0, int epi, int strips, hipStream_t st) {
     else OHARA_PHI_IN(0);
 #undef OHARA_PHI_IN
     return ohara_launch_status();
+  }
+  if (group_applies(a, epi, strips)) {
+    if (epi == EPI_STORE) return launch_group<EPI_STORE>(a, st);
+    return epi == EPI_SWIGLU ? launch_group<EPI_SWIGLU>(a, st) : launch_group<EPI_ROPE>(a, st);
   }
   return a.norm_w ? launch_epi<1, true>(a, epi, strips, st) : launch_epi<1, false>(a, epi, strips, st);
 }

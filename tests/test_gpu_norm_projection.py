@@ -1,0 +1,70 @@
+"""Projections of up to 64 normed rows where several strips share a workgroup, and where eight waves share a strip: edges of K, of rows
+and of strips, against the norm and the projection as two calls."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def _check(got, x, w, nw, eps, plain):
+    """`plain`: the projection of rows normed before.  Only the two fp32 sums (of the squares, over K) are in another order: a normed value
+    may round to its neighbour (2^-8 of it at most), a result likewise."""
+    from ohara_amd import ops
+
+    xn = ops.rmsnorm(x, nw, eps).double()
+    mass = xn.abs() @ w.double().abs().t()
+    assert ((got.double() - xn @ w.double().t()).abs() <= (xn @ w.double().t()).abs() * 2.0 ** -8 + mass * (2.0 ** -8 + x.shape[1] * 2.0 ** -24)).all()
+    assert (got != plain).float().mean() <= 0.05
+
+
+# (columns, K): two, three and four strips a workgroup with eight waves (K up to 1024) and with sixteen, the last group not full; then one strip
+# with eight waves
+SHAPES = [(4112, 8), (8200, 1000), (12304, 1024), (4128, 1032), (11264, 2048), (12000, 1544), (16368, 2040), (3072, 2048), (40, 1032)]
+
+
+@pytest.mark.parametrize("n,k", SHAPES)
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64])
+def test_store_and_gates(cuda, rows, n, k):
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(rows + n + k)
+    x = (torch.randn(rows, k, generator=g, device=cuda) * torch.logspace(-2, 2, rows, device=cuda)[:, None]).to(BF)
+    nw = (1 + 0.3 * torch.randn(k, generator=g, device=cuda)).to(BF)
+    w = (torch.randn(n, k, generator=g, device=cuda) * 0.05).to(BF)
+    packed, xn = ops.pack_linear(w), ops.rmsnorm(x, nw, 1e-5)
+    _check(ops.gemm_skinny(x, packed, nw, 1e-5), x, w, nw, 1e-5, ops.gemm_skinny(xn, packed))
+    f = n // 2
+    gates = ops.pack_gate_up(w[:f], w[f:2 * f])
+    got, plain = ops.gemm_skinny(x, gates, nw, 1e-5), ops.gemm_skinny(xn, gates)
+    assert (got != plain).float().mean() <= 0.05
+    gate, up = (xn.double() @ t.double().t() for t in (w[:f], w[f:2 * f]))
+    mass_g, mass_u = (xn.double().abs() @ t.double().abs().t() for t in (w[:f], w[f:2 * f]))
+    silu = gate * torch.sigmoid(gate)
+    rel = 2.0 ** -8 + k * 2.0 ** -24
+    # three roundings of the product's factors and itself, the gate's through a slope of at most 1.1, and neighbours in the normed rows
+    bound = 1.02 * (silu.abs() * (up.abs() * 3 * 2.0 ** -8 + mass_u * rel) + 1.1 * (gate.abs() * 2.0 ** -8 + mass_g * rel) * (up.abs() + mass_u * rel))
+    assert ((got.double() - silu * up).abs() <= bound + 1e-30).all()
+
+
+@pytest.mark.parametrize("B,H,Hkv,D,K", [(1, 40, 8, 128, 1024), (17, 33, 33, 64, 776), (40, 48, 8, 64, 2048), (64, 16, 4, 128, 2048), (16, 16, 4, 128, 1288)])
+def test_rotary(cuda, B, H, Hkv, D, K):
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(B + K)
+    x = torch.randn(B, K, generator=g, device=cuda).to(BF)
+    nw = (1 + 0.3 * torch.randn(K, generator=g, device=cuda)).to(BF)
+    ws = [(torch.randn(n * D, K, generator=g, device=cuda) * 0.05).to(BF) for n in (H, Hkv, Hkv)]
+    ang = torch.rand(16, D // 2, generator=g, device=cuda) * 6.28
+    cos, sin = ang.cos().to(BF), ang.sin().to(BF)
+    wp, out = ops.pack_qkv(*ws), []
+    for rows, norm in ((x, nw), (ops.rmsnorm(x, nw, 1e-5), None)):
+        kc, vc = (torch.full((B, 16, Hkv, D), 9.0, dtype=BF, device=cuda) for _ in range(2))
+        q = ops.qkv_rope_append(rows, wp, norm, 1e-5, H, Hkv, D, cos, sin, 5, kc, vc)
+        assert (kc[:, :5] == 9.0).all() and (kc[:, 6:] == 9.0).all() and (vc[:, 6:] == 9.0).all()
+        out.append((q, kc[:, 5].reshape(B, -1), vc[:, 5].reshape(B, -1)))
+    _check(out[0][2], x, ws[2], nw, 1e-5, out[1][2])
+    for got, plain in zip(*out):  # the rotation adds two values that may each be a neighbour
+        assert (got != plain).float().mean() <= 0.05
+        assert (got.float() - plain.float()).abs().max() <= 2.0 ** -6 * plain.float().abs().max()
