@@ -39,11 +39,11 @@ class ContinuousBatcher:
         return [b for b in range(self.slots) if not self.active[b]]
 
     def _select(self, logits: torch.Tensor) -> torch.Tensor:
-        """logits (rows, V) -> ids (rows,) on the device."""
+        """logits (rows, V) -> ids (rows,) on the device, each drawn by a number of its own."""
         vv = self.valid_vocab or None
         if self.sampling is None:
             return ops.argmax(logits, valid_vocab=vv)
-        u = torch.rand(logits.shape[0], device=logits.device, dtype=torch.float32, generator=self.generator)
+        u = torch.cat([torch.rand(1, device=logits.device, dtype=torch.float32, generator=self.generator) for _ in logits])
         return ops.sample_topk_topp(logits, self.sampling.temperature, self.sampling.top_k, self.sampling.top_p, u,
                                     valid_vocab=vv)
 
@@ -68,10 +68,12 @@ class ContinuousBatcher:
             logits = self._padded_forward(slots, prompts, last_only)
             out = [row[: 1 if last_only else len(p)] for row, p in zip(logits, prompts)]
         else:
+            # one upload: a copy from the host waits for the stream, and behind a prompt it would for the prompt's whole pass
+            rows = torch.cat(prompts).to(self.model.device).split([len(p) for p in prompts])
             out = []
-            for b, ids in zip(slots, prompts):
+            for b, ids in zip(slots, rows):
                 views = [c._row_view(b) for c in self.cache]
-                out.append(self.model.forward(ids.view(1, -1).to(self.model.device), views, 0, last_only=last_only)[0])
+                out.append(self.model.forward(ids.view(1, -1), views, 0, last_only=last_only)[0])
         for b, ids in zip(slots, prompts):
             self._book(b, len(ids))
         return out
@@ -107,12 +109,13 @@ class ContinuousBatcher:
             raise RuntimeError("no free slot")
         prompts = [self._host_ids(p, start=1) for p in prompts]  # room for one generated token at least
         slots = free[: len(prompts)]
-        out = []
-        for b, logits in zip(slots, self._prefill(slots, prompts)):
-            tok = self._select(logits.reshape(1, -1))
-            self.last[b:b + 1] = tok
-            out.append((b, int(tok.item())))
-        return out
+        if not prompts:
+            return []
+        # one selection and one read-back for all of them (16 prompts of 100 to 800 tokens, d12: 20.5 -> NN ms with 15 steps)
+        toks = self._select(torch.cat([logits.reshape(1, -1) for logits in self._prefill(slots, prompts)]))
+        host = toks.tolist()
+        self.last[torch.tensor(slots, device=self.last.device)] = toks
+        return list(zip(slots, host))
 
     @torch.no_grad()
     def feed(self, entries) -> list[tuple[int, torch.Tensor]]:
