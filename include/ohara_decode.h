@@ -117,6 +117,11 @@ int ohara_qkv_rope_append_ragged_bf16(const uint16_t* x, int ldx, const uint16_t
                                       float eps, int batch, int seq_len, int h, int h_kv, int dh, const uint16_t* cos,
                                       const uint16_t* sin, const int32_t* seq_pos, uint16_t* q_out, uint16_t* kcache,
                                       uint16_t* vcache, int t_max, void* stream);
+/* Rows of prompts side by side (always the tiled kernel, no norm): `at` (device) holds the position of every row, then the
+ * row of the caches that its sequence is in. */
+int ohara_qkv_rope_append_rows_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int k, int rows, int h, int h_kv, int dh,
+                                    const uint16_t* cos, const uint16_t* sin, const int32_t* at, uint16_t* q_out, uint16_t* kcache,
+                                    uint16_t* vcache, int t_max, void* stream);
 int ohara_qkv_rope_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int k, const uint16_t* norm_w, float eps,
                         int batch, int seq_len, int h, int h_kv, int dh, const uint16_t* cos, const uint16_t* sin,
                         int pos, const int32_t* pos_dev, int t_max, uint16_t* q_out, uint16_t* k_out, uint16_t* v_out,
@@ -177,6 +182,12 @@ int ohara_attn_cached_bf16_noalloc(const uint16_t* q, const uint16_t* kcache, co
  * Needs no workspace.  (llama.py:100-135 with S > 1.) */
 int ohara_attn_prefill_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int batch,
                             int seq_len, int h, int h_kv, int dh, int t_max, int pos, uint16_t* out, void* stream);
+
+/* ohara_attn_prefill_bf16 over n prompts of their own lengths, their query rows side by side, each from position 0 of its row of the
+ * caches: `lengths` on the host; `seqs` on the device: n first query rows, n lengths, n rows of the caches. */
+int ohara_attn_prompts_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int n, const int32_t* lengths,
+                            const int32_t* seqs, int h, int h_kv, int dh, int t_max, uint16_t* out, void* stream);
+
 
 /* ---- int8 KV cache (ohara/modules/kv_cache.py:15-32, 67-73, 94-102, 116-118) ------------------
  * Every (sequence, position, head) row of dh values is stored as int8 with an fp32 scale and
@@ -477,6 +488,14 @@ typedef struct OharaDecodeState {
  * select_greedy != 0 (needs logits_mode LAST or seq_len == 1) appends the argmax. */
 int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* s, int seq_len, int pos, int use_pos_dev,
                         int logits_mode, int select_greedy, void* stream);
+
+/* ohara_llama_forward over n prompts of different lengths, each from position 0 into its own row of the caches (bf16 caches,
+ * head width 64 or 128); logits (n, vocab) of the last token of each.  s: ids, x, xn, q, attn and act for the rows of all prompts
+ * side by side.  `lengths` on the host; `table` on the device: n first rows, n lengths, n rows of the caches, then the position of
+ * every row and the row of the caches it belongs to. */
+int ohara_llama_prompts(const OharaModel* m, const OharaDecodeState* s, int n, const int32_t* lengths, const int32_t* table,
+                        void* stream);
+
 
 /* ---- one decode step as ONE persistent launch (batch <= 16) ------------------------
  * Same result as ohara_llama_forward(seq_len = 1, use_pos_dev = 1, LOGITS_LAST) but the

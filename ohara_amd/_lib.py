@@ -127,6 +127,8 @@ _PROTOS = {
     "ohara_qkv_rope_append_ragged_bf16": (_i, [_p, _i, _p, _i, _p, _f, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _p]),
     "ohara_advance_positions": (_i, [_p, _p, _i, _i, _p]),
     "ohara_advance_ragged": (_i, [_p, _p, _p, _p, _i, _i, _p]),
+    "ohara_qkv_rope_append_rows_bf16": (_i, [_p, _i, _p, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _p]),
+    "ohara_attn_prompts_bf16": (_i, [_p, _p, _p, _i, _p, _p, _i, _i, _i, _i, _p, _p]),
     "ohara_attn_prefill_bf16": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p]),
     "ohara_argmax_bf16": (_i, [_p, _i, _i, _i, _i, _p, _p, _i, _p, _p]),
     "ohara_sample_topk_topp": (_i, [_p, _i, _i, _i, _i, _i, _f, _i, _f, _p, _i, _p, _p, _i, _p, _p]),
@@ -158,6 +160,7 @@ _PROTOS = {
     "ohara_moe_experts_gate_up_many": (_i, [_p, _i, _p, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _i, _p]),
     "ohara_moe_experts_down_many": (_i, [_p, _i, _p, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _p, _i, _p]),
     "ohara_moe_combine": (_i, [_p, _i, _p, _p, _i, _i, _p, _i, _p, _i, _p, _i, _i, _p]),
+    "ohara_llama_prompts": (_i, [C.POINTER(OharaModel), C.POINTER(OharaDecodeState), _i, _p, _p, _p]),
     "ohara_llama_forward": (_i, [C.POINTER(OharaModel), C.POINTER(OharaDecodeState), _i, _i, _i, _i, _i, _p]),
     "ohara_linear_bias_bf16": (_i, [_p, _i, _p, _i, _i, _p, _i, _i, _p, _i, _p, _i, _p, _i, _p]),
     "ohara_phi_block_in_bf16": (_i, [_p, _i, _p, _p, _f, _p, _p, _i, _i, _i, _i, _i, _p, _p, _i, _p, _p, _i, _p, _i, _p]),

@@ -33,7 +33,16 @@ struct PrefillArgs {
   int B, S, H, Hkv, Tmax, pos;
   int nqb;           // query blocks per sequence
   float scale_log2e;
+  const int32_t* seqs;  // prompts of their own lengths, from position 0: B first rows, B lengths, B rows of the cache (S: the longest)
 };
+struct Sequence {
+  size_t row0;  // first query row
+  int S, cache;
+};
+__device__ __forceinline__ Sequence sequence(const PrefillArgs& a, int b) {
+  if (a.seqs) return {(size_t)a.seqs[b], a.seqs[a.B + b], a.seqs[2 * a.B + b]};
+  return {(size_t)b * a.S, a.S, b};
+}
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint2 lds_tr8(uint32_t addr) {
@@ -42,10 +51,15 @@ __device__ __forceinline__ uint2 lds_tr8(uint32_t addr) {
 }
 
 // An XCD (ids go round-robin over the eight) gets whole heads, their late - longest - blocks first; where the heads do
-// not divide, an eighth of all blocks in the order of the heads, long and short ones in turn.
+// not divide, an eighth of all blocks in the order of the heads, long and short ones in turn.  Where the sequences have lengths of
+// their own every eighth head, so that no XCD gets the long ones; the grid is rounded up to that (then head may be past the last).
 __device__ __forceinline__ void my_block(const PrefillArgs& a, int& head, int& qblk) {
   const int heads = a.H * a.B, x = blockIdx.x & 7, q = blockIdx.x >> 3;
-  if ((heads & 7) == 0) {
+  if (a.seqs) {
+    const int nh = (heads + 7) >> 3;
+    head = (q % nh) * 8 + x;
+    qblk = a.nqb - 1 - q / nh;
+  } else if ((heads & 7) == 0) {
     const int nh = heads >> 3;
     head = x * nh + q % nh;
     qblk = a.nqb - 1 - q / nh;
@@ -70,12 +84,12 @@ struct KvTile {
   int len;              // positions that exist
   int lane;
 
-  __device__ __forceinline__ KvTile(const PrefillArgs& a, int b, int kvh, int lane_) : lane(lane_) {
+  __device__ __forceinline__ KvTile(const PrefillArgs& a, const Sequence& sq, int kvh, int lane_) : lane(lane_) {
     const size_t row = (size_t)a.Hkv * D;
-    kb = reinterpret_cast<const char*>(a.k + (size_t)b * a.Tmax * row + (size_t)kvh * D);
-    vb = reinterpret_cast<const char*>(a.v + (size_t)b * a.Tmax * row + (size_t)kvh * D);
+    kb = reinterpret_cast<const char*>(a.k + (size_t)sq.cache * a.Tmax * row + (size_t)kvh * D);
+    vb = reinterpret_cast<const char*>(a.v + (size_t)sq.cache * a.Tmax * row + (size_t)kvh * D);
     rowb = (uint32_t)row * 2;
-    len = a.pos + a.S;
+    len = a.pos + sq.S;
   }
   // ALIGNED: the caches start on 16 bytes (false: through registers, any)
   template <int NW>
@@ -188,19 +202,19 @@ __device__ __forceinline__ float softmax_tile(f32x4 (&s)[NKB], uint4 (&pf)[NWIN]
 
 // Queries wq0 + 16 qb + (lane & 15): lane g holds columns 32 j + 8 g .. + 7
 template <int D>
-__device__ __forceinline__ void load_queries(uint4 (&qf)[D / 32], int& qpos, const PrefillArgs& a, int b, int h, int qi, int g) {
-  qpos = qi < a.S ? a.pos + qi : 0x3fffffff;  // rows past the end: never masked, never stored
+__device__ __forceinline__ void load_queries(uint4 (&qf)[D / 32], int& qpos, const PrefillArgs& a, const Sequence& sq, int h, int qi, int g) {
+  qpos = qi < sq.S ? a.pos + qi : 0x3fffffff;  // rows past the end: never masked, never stored
 #pragma unroll
   for (int j = 0; j < D / 32; ++j)
-    qf[j] = qi < a.S ? ldg16(a.q + ((size_t)b * a.S + qi) * a.H * D + (size_t)h * D + 32 * j + 8 * g) : make_uint4(0, 0, 0, 0);
+    qf[j] = qi < sq.S ? ldg16(a.q + (sq.row0 + qi) * a.H * D + (size_t)h * D + 32 * j + 8 * g) : make_uint4(0, 0, 0, 0);
 }
 
 template <int D, int N>
-__device__ __forceinline__ void store_rows(const f32x4 (&o)[N], float l, const PrefillArgs& a, int b, int h, int qi, int g, int d0) {
+__device__ __forceinline__ void store_rows(const f32x4 (&o)[N], float l, const PrefillArgs& a, const Sequence& sq, int h, int qi, int g, int d0) {
   l = lane_xor_sum<32>(lane_xor_sum<16>(l));
-  if (qi >= a.S) return;
+  if (qi >= sq.S) return;
   const float inv = 1.0f / l;
-  bf16_t* dst = a.out + ((size_t)b * a.S + qi) * a.H * D + (size_t)h * D + 16 * d0 + 4 * g;
+  bf16_t* dst = a.out + (sq.row0 + qi) * a.H * D + (size_t)h * D + 16 * d0 + 4 * g;
 #pragma unroll
   for (int db = 0; db < N; ++db)
     *reinterpret_cast<uint2*>(dst + db * 16) = make_uint2(pack_bf(o[db][0] * inv, o[db][1] * inv), pack_bf(o[db][2] * inv, o[db][3] * inv));
@@ -217,11 +231,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
   int head, qblk;
   my_block(a, head, qblk);
   const int b = head / a.H, h = head - b * a.H;
+  if (b >= a.B) return;
+  const Sequence sq = sequence(a, b);
+  if (qblk * QB >= sq.S) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int m = lane & 15, g = lane >> 4;
   const int q0 = qblk * QB;                              // first query of the workgroup
   const int wq0 = q0 + wave * 16 * QW;                   // first query of the wave
-  const Tl tile(a, b, h / (a.H / a.Hkv), lane);
+  const Tl tile(a, sq, h / (a.H / a.Hkv), lane);
   const typename Tl::template Offsets<NW> offs = tile.template offsets<NW>(KT, wave);
   const int ntiles = (min(a.pos + q0 + QB, tile.len) + KT - 1) / KT;  // tiles any query of the workgroup sees
   const int wave_last = min(a.pos + wq0 + 16 * QW - 1, tile.len - 1);  // last position any query of the wave sees
@@ -233,7 +250,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
   float m_run[QW], l_run[QW];
 #pragma unroll
   for (int qb = 0; qb < QW; ++qb) {
-    load_queries<D>(qf[qb], qpos[qb], a, b, h, wq0 + qb * 16 + m, g);
+    load_queries<D>(qf[qb], qpos[qb], a, sq, h, wq0 + qb * 16 + m, g);
     m_run[qb] = -INFINITY;
     l_run[qb] = 0.f;
 #pragma unroll
@@ -291,7 +308,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
     cur = next;
   }
 #pragma unroll
-  for (int qb = 0; qb < QW; ++qb) store_rows<D>(o[qb], l_run[qb], a, b, h, wq0 + qb * 16 + m, g, 0);
+  for (int qb = 0; qb < QW; ++qb) store_rows<D>(o[qb], l_run[qb], a, sq, h, wq0 + qb * 16 + m, g, 0);
 }
 
 // TEAMS teams of four waves, 16 queries each.  Wave w scores positions 16 w .. + 15 of every tile and owns a quarter of the output
@@ -307,11 +324,14 @@ __global__ __launch_bounds__(TEAMS * 256, TEAMS) void attn_team_kernel(PrefillAr
   int head, qblk;
   my_block(a, head, qblk);
   const int b = head / a.H, h = head - b * a.H;
+  if (b >= a.B) return;
+  const Sequence sq = sequence(a, b);
+  if (qblk * QB >= sq.S) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int w4 = wave & 3, team = wave >> 2;
   const int m = lane & 15, g = lane >> 4;
   const int q0 = qblk * QB, wq0 = q0 + 16 * team;
-  const Tl tile(a, b, h / (a.H / a.Hkv), lane);
+  const Tl tile(a, sq, h / (a.H / a.Hkv), lane);
   const typename Tl::template Offsets<NW> offs = tile.template offsets<NW>(KT, wave);
   const int ntiles = (min(a.pos + q0 + QB, tile.len) + KT - 1) / KT;
   const int team_last = min(a.pos + wq0 + 15, tile.len - 1);
@@ -320,7 +340,7 @@ __global__ __launch_bounds__(TEAMS * 256, TEAMS) void attn_team_kernel(PrefillAr
 
   uint4 qf[NK];
   int qpos;
-  load_queries<D>(qf, qpos, a, b, h, wq0 + m, g);
+  load_queries<D>(qf, qpos, a, sq, h, wq0 + m, g);
   f32x4 o[ND];
 #pragma unroll
   for (int db = 0; db < ND; ++db) o[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -380,13 +400,13 @@ __global__ __launch_bounds__(TEAMS * 256, TEAMS) void attn_team_kernel(PrefillAr
     put_scores(t + 1, sn);
     cur = next;
   }
-  store_rows<D>(o, l_run, a, b, h, wq0 + m, g, w4 * ND);
+  store_rows<D>(o, l_run, a, sq, h, wq0 + m, g, w4 * ND);
 }
 
 template <int D, int QW, bool ALIGNED = true>
 int launch_waves(PrefillArgs a, hipStream_t st) {
   a.nqb = (a.S + 64 * QW - 1) / (64 * QW);
-  const int64_t blocks = (int64_t)a.nqb * a.H * a.B;
+  const int64_t blocks = a.nqb * (a.seqs ? ((int64_t)a.H * a.B + 7) / 8 * 8 : (int64_t)a.H * a.B);
   if (blocks > INT32_MAX) return OHARA_ESIZE;
   hipLaunchKernelGGL((attn_prefill_kernel<D, QW, ALIGNED>), dim3((unsigned)blocks), dim3(256), 2 * KvTile<D>::SLOT, st, a);
   return ohara_launch_status();
@@ -398,7 +418,7 @@ int launch_teams(PrefillArgs a, hipStream_t st) {
   a.nqb = (a.S + 16 * TEAMS - 1) / (16 * TEAMS);
   if (LDS > 64 * 1024)
     (void)hipFuncSetAttribute((const void*)attn_team_kernel<D, TEAMS, NST, true>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  hipLaunchKernelGGL((attn_team_kernel<D, TEAMS, NST, true>), dim3((unsigned)(a.nqb * a.H * a.B)), dim3(TEAMS * 256), LDS, st, a);
+  hipLaunchKernelGGL((attn_team_kernel<D, TEAMS, NST, true>), dim3((unsigned)(a.nqb * (a.seqs ? (a.H * a.B + 7) / 8 * 8 : a.H * a.B))), dim3(TEAMS * 256), LDS, st, a);
   return ohara_launch_status();
 }
 
@@ -417,10 +437,14 @@ int launch_teams(PrefillArgs a, hipStream_t st) {
 // CU on, else 64.  Before (one kernel, four waves, values through registers, the heads over all XCDs): 5.8, 45, 16.5, 25, 26, 167,
 // 50, 46, 92; 5.2, 10.4, 12, 64.
 template <int D>
-int launch_prefill_for(const PrefillArgs& a, hipStream_t st) {
+int launch_prefill_for(const PrefillArgs& a, const int32_t* lengths, hipStream_t st) {  // lengths: on the host, where they differ
   constexpr int CUS = 256;
-  const int64_t heads = (int64_t)a.H * a.B;
-  auto blocks = [&](int queries) { return (a.S + queries - 1) / queries * heads; };
+  auto blocks = [&](int queries) {
+    if (!lengths) return (a.S + queries - 1) / queries * (int64_t)a.H * a.B;
+    int64_t n = 0;
+    for (int b = 0; b < a.B; ++b) n += (lengths[b] + queries - 1) / queries;
+    return n * a.H;
+  };
   if (((uintptr_t)a.k | (uintptr_t)a.v) & 15) return launch_waves<D, 1, false>(a, st);
   if (blocks(16) <= CUS * (D == 64 ? 2 : 1)) return launch_teams<D, 1>(a, st);
   if (blocks(32) <= CUS) return launch_teams<D, 2>(a, st);
@@ -442,5 +466,22 @@ extern "C" int ohara_attn_prefill_bf16(const uint16_t* q, const uint16_t* kcache
   a.q = q; a.k = kcache; a.v = vcache; a.out = out;
   a.B = batch; a.S = seq_len; a.H = h; a.Hkv = h_kv; a.Tmax = t_max; a.pos = pos;
   a.scale_log2e = (1.0f / sqrtf((float)dh)) * OHARA_LOG2E;  // the same constant as the decode kernels'
-  return dh == 128 ? launch_prefill_for<128>(a, (hipStream_t)stream) : launch_prefill_for<64>(a, (hipStream_t)stream);
+  return dh == 128 ? launch_prefill_for<128>(a, nullptr, (hipStream_t)stream) : launch_prefill_for<64>(a, nullptr, (hipStream_t)stream);
+}
+
+extern "C" int ohara_attn_prompts_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int n, const int32_t* lengths,
+                                       const int32_t* seqs, int h, int h_kv, int dh, int t_max, uint16_t* out, void* stream) {
+  if (!q || !kcache || !vcache || !lengths || !seqs || !out) return OHARA_EINVAL;
+  if (n < 1 || h < 1 || h_kv < 1 || h % h_kv || t_max < 1) return OHARA_EINVAL;
+  if (dh != 64 && dh != 128) return OHARA_ESIZE;
+  if (n > 65535 || h > 65535) return OHARA_ESIZE;
+  PrefillArgs a{};
+  a.q = q; a.k = kcache; a.v = vcache; a.out = out; a.seqs = seqs;
+  a.B = n; a.H = h; a.Hkv = h_kv; a.Tmax = t_max;
+  for (int b = 0; b < n; ++b) {
+    if (lengths[b] < 1 || lengths[b] > t_max) return OHARA_EINVAL;
+    if (lengths[b] > a.S) a.S = lengths[b];
+  }
+  a.scale_log2e = (1.0f / sqrtf((float)dh)) * OHARA_LOG2E;
+  return dh == 128 ? launch_prefill_for<128>(a, lengths, (hipStream_t)stream) : launch_prefill_for<64>(a, lengths, (hipStream_t)stream);
 }

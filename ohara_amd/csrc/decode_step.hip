@@ -130,6 +130,46 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
   return OHARA_OK;
 }
 
+// The last row of every prompt, 16 bytes a lane.
+static __global__ __launch_bounds__(64) void last_rows_kernel(const bf16_t* x, const int32_t* seqs, bf16_t* out, int d) {
+  const int b = blockIdx.x, n = gridDim.x;
+  const size_t row = (size_t)seqs[b] + seqs[n + b] - 1;
+  for (int i = threadIdx.x * 8; i < d; i += 512) *reinterpret_cast<uint4*>(out + (size_t)b * d + i) = ldg16(x + row * d + i);
+}
+
+// The same chain over prompts of different lengths, each from position 0 into its own row of the caches: the row-wise kernels
+// run once over all rows, side by side without padding.  16 prompts of 100 to 800 tokens, d12: 11.8 ms one by one, 4.1 together.
+extern "C" int ohara_llama_prompts(const OharaModel* m, const OharaDecodeState* s, int n, const int32_t* lengths, const int32_t* table,
+                                   void* stream) {
+  if (!m || !s || !m->layers || !s->kcache || !s->vcache || !lengths || !table || !s->xn || !s->logits) return OHARA_EINVAL;
+  if (s->kv_int8 || n < 1) return OHARA_EINVAL;
+  int64_t rows = 0;
+  for (int b = 0; b < n; ++b) {
+    if (lengths[b] < 1 || lengths[b] > m->t_max) return OHARA_EINVAL;
+    rows += lengths[b];
+  }
+  if (rows > s->rows_cap) return OHARA_ESIZE;
+  const int R = (int)rows, d = m->d_model, H = m->n_heads, Hkv = m->n_kv_heads, Dh = m->head_dim;
+  if (d & 7) return OHARA_ESIZE;
+  const int32_t* at = table + 3 * n;
+  int rc = ohara_embed_bf16(s->ids, m->token_emb, s->x, R, d, m->vocab, stream);
+  for (int l = 0; l < m->n_layers && !rc; ++l) {
+    const OharaLayer& L = m->layers[l];
+    rc = ohara_rmsnorm_bf16(s->x, L.norm1, s->xn, R, d, m->eps, stream);
+    if (!rc) rc = ohara_qkv_rope_append_rows_bf16(s->xn, d, L.wqkv, d, R, H, Hkv, Dh, m->cos, m->sin, at, s->q, s->kcache[l],
+                                                  s->vcache[l], m->t_max, stream);
+    if (!rc) rc = ohara_attn_prompts_bf16(s->q, s->kcache[l], s->vcache[l], n, lengths, table, H, Hkv, Dh, m->t_max, s->attn, stream);
+    if (!rc) rc = ohara_gemm_bf16(s->attn, H * Dh, L.wo, d, H * Dh, R, OHARA_EPI_RESIDUAL, s->x, d, s->x, d, stream);
+    if (!rc) rc = ohara_rmsnorm_bf16(s->x, L.norm2, s->xn, R, d, m->eps, stream);
+    if (!rc) rc = ohara_gemm_bf16(s->xn, d, L.wgu, m->d_ff, d, R, OHARA_EPI_SWIGLU, nullptr, 0, s->act, m->d_ff, stream);
+    if (!rc) rc = ohara_gemm_bf16(s->act, m->d_ff, L.wdown, d, m->d_ff, R, OHARA_EPI_RESIDUAL, s->x, d, s->x, d, stream);
+  }
+  if (rc) return rc;
+  hipLaunchKernelGGL(last_rows_kernel, dim3(n), dim3(64), 0, (hipStream_t)stream, s->x, table, s->xn, d);
+  return ohara_gemm_skinny_bf16(s->xn, d, m->w_vocab, m->vocab, d, m->final_norm, m->eps, n, OHARA_EPI_STORE, nullptr, 0, s->logits,
+                                m->vocab, stream);
+}
+
 extern "C" int ohara_event_create(void** event) {
   if (!event) return OHARA_EINVAL;
   hipEvent_t e;

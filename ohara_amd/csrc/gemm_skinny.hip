@@ -867,6 +867,22 @@ int ohara_qkv_rope_append_ragged_bf16(const uint16_t* x, int ldx, const uint16_t
                        vcache, t_max, 0, stream);
 }
 
+int ohara_qkv_rope_append_rows_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int k, int rows, int h, int h_kv, int dh,
+                                    const uint16_t* cos, const uint16_t* sin, const int32_t* at, uint16_t* q_out, uint16_t* kcache,
+                                    uint16_t* vcache, int t_max, void* stream) {
+  if (!x || !wp || !cos || !sin || !at || !q_out || !kcache || !vcache) return OHARA_EINVAL;
+  if (rows < 1 || h < 1 || h_kv < 1 || h % h_kv || dh < 4 || (dh & 3) || t_max < 1) return OHARA_EINVAL;
+  if ((k & 7) || (ldx & 7) || ldx < k) return OHARA_EINVAL;
+  GemmArgs a{};
+  a.wp = reinterpret_cast<const uint4*>(wp);
+  a.x = x; a.ldx = ldx;
+  a.B = rows; a.N = (h + 2 * h_kv) * dh; a.K = k; a.S = 1;
+  a.out = q_out; a.ldo = h * dh;
+  a.H = h; a.Hkv = h_kv; a.Dh = dh; a.Tmax = t_max; a.rows = at;
+  a.cos = cos; a.sin = sin; a.kcache = kcache; a.vcache = vcache;
+  return ohara_launch_gemm_tile(a, EPI_ROPE, (a.N + 15) / 16 * 16, (hipStream_t)stream);
+}
+
 int ohara_qkv_rope_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int k, const uint16_t* norm_w, float eps,
                         int batch, int seq_len, int h, int h_kv, int dh, const uint16_t* cos, const uint16_t* sin,
                         int pos, const int32_t* pos_dev, int t_max, uint16_t* q_out, uint16_t* k_out, uint16_t* v_out,

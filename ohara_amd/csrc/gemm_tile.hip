@@ -53,19 +53,25 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
   // long), the region (q / k / v) and the feature index inside the head on the strip alone (uniform
   // over the wave).  Worked out per fragment they were 40 % of this kernel's instructions.
   if (rbase >= a.B) return;
-  if (EPI == EPI_ROPE && a.S >= FM * 16 && ((a.ldo | a.Dh) & 15) == 0 && ((a.H * a.Dh) & 15) == 0 && !a.stage) {
+  if (EPI == EPI_ROPE && (a.rows || a.S >= FM * 16) && ((a.ldo | a.Dh) & 15) == 0 && ((a.H * a.Dh) & 15) == 0 && !a.stage) {
     const int nq = a.H * a.Dh, nk = a.Hkv * a.Dh;
     const int gbase = a.row0 + rbase;                          // global row of the wave's first row
-    const int seq0 = gbase / a.S, rem0 = gbase - seq0 * a.S;   // uniform over the wave
+    const int seq0 = a.rows ? 0 : gbase / a.S, rem0 = gbase - seq0 * a.S;   // uniform over the wave
     int pos_t[FM];
     size_t qoff_t[FM], coff_t[FM];
 #pragma unroll
     for (int t = 0; t < FM; ++t) {
       const int x = rem0 + min(t * 16 + m, a.B - 1 - rbase);  // rows past the end: the last row, never stored
-      const bool wrap = x >= a.S;
-      const int seq = seq0 + (wrap ? 1 : 0), sidx = x - (wrap ? a.S : 0);
       const int grow = gbase + t * 16 + m;
-      pos_t[t] = (a.pos_dev ? a.pos_dev[(size_t)seq * a.pos_stride] : a.pos) + sidx;
+      int seq;
+      if (a.rows) {
+        pos_t[t] = a.rows[x];
+        seq = a.rows[a.B + x];
+      } else {
+        const bool wrap = x >= a.S;
+        seq = seq0 + (wrap ? 1 : 0);
+        pos_t[t] = (a.pos_dev ? a.pos_dev[(size_t)seq * a.pos_stride] : a.pos) + x - (wrap ? a.S : 0);
+      }
       qoff_t[t] = (size_t)grow * a.ldo;
       coff_t[t] = (((size_t)seq * a.Tmax + pos_t[t]) * a.Hkv) * a.Dh;
     }

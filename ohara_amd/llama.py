@@ -433,6 +433,36 @@ class Llama:
 
     __call__ = forward
 
+    def takes_prompts(self, kv_cache: list) -> bool:
+        """Whether ``prompts`` serves this model over these caches."""
+        return self.head_dim in (64, 128) and self.config.hidden_size % 8 == 0 and not any(c.int8 for c in kv_cache)
+
+    def prompts(self, prompts: list, kv_cache: list, slots: list[int]) -> torch.Tensor:
+        """Prompts (1-D ids, on the host) of different lengths in one call, each from position 0 into its own row ``slots[i]`` of the
+        caches, which have to be empty there -> the logits (n, V) of the last token of each.  More than 64 tokens
+        together.  The books of the caches are the caller's."""
+        lens = [len(p) for p in prompts]
+        rows = sum(lens)
+        if rows <= 64 or min(lens) < 1 or max(lens) > self.config.max_sequence_length:
+            raise ValueError("prompts hold more than 64 tokens together, each at least one and at most max_sequence_length")
+        if len(set(slots)) != len(prompts) or min(slots) < 0 or max(slots) >= min(c.capacity for c in kv_cache):
+            raise ValueError("slots must be distinct rows of the cache")
+        n = len(prompts)
+        buf = self._get_buffers(n, rows)
+        length, slot = torch.tensor(lens, dtype=torch.int32), torch.tensor(slots, dtype=torch.int32)
+        first = length.cumsum(0, dtype=torch.int32) - length
+        at = torch.arange(rows, dtype=torch.int32) - first.repeat_interleave(length)
+        table = torch.cat([first, length, slot, at, slot.repeat_interleave(length)])
+        # one upload: ids as pairs of 32 bits in front
+        ids = torch.cat(prompts).to(torch.int64)
+        dev = torch.cat([ids.view(torch.int32), table]).to(self.device)
+        buf.ids.copy_(dev[:2 * rows].view(torch.int64))
+        logits = torch.empty(n, self.config.vocab_size, dtype=BF16, device=self.device)
+        st = self._state_struct(buf, kv_cache, logits)
+        check(lib().ohara_llama_prompts(C.byref(self._c_model), C.byref(st), n, length.data_ptr(), dev[2 * rows:].data_ptr(),
+                                        torch.cuda.current_stream().cuda_stream), "llama_prompts")
+        return logits
+
     # -- device-resident greedy loop --------------------------------------------------
 
     def session(self, batch: int, max_new_tokens: int, valid_vocab: int = 0, kv_cache: list | None = None,
