@@ -253,6 +253,8 @@ __global__ __launch_bounds__(256) void moe_route_fused_kernel(RouteFusedArgs a) 
   const int ldxs = KS * 32 + 8;
   bf16_t* xs = reinterpret_cast<bf16_t*>(route_smem);  // four normalised rows
   const int t0 = blockIdx.x * 4;
+  const uint4* wrow = a.wp + (size_t)min(wave, ((a.E + 15) >> 4) - 1) * KS * 64 + lane;  // (2.: strip `wave` of the router)
+  uint4 wv[32];
   // 1. RMSNorm, a row per wave (the row stays in registers between the sum and the scaling):
   //    y = bf16(bf16(x * rinv) * w), rinv = 1 / sqrt(mean(x^2) + eps)
   {
@@ -265,6 +267,10 @@ __global__ __launch_bounds__(256) void moe_route_fused_kernel(RouteFusedArgs a) 
       xv[c] = i < a.d ? ldg16(xr + i) : make_uint4(0, 0, 0, 0);
       gv[c] = i < a.d ? ldg16(a.norm_w + i) : make_uint4(0, 0, 0, 0);
     }
+    // the router's weights are asked for before anything waits, behind the row (24 tokens, 64 experts, d 1024: 14.4 -> 13.6 us)
+#pragma unroll
+    for (int c = 0; c < 32; ++c) wv[c] = ldg16_nt(wrow + (size_t)min(c, KS - 1) * 64);
+    __builtin_amdgcn_sched_barrier(0);
     float ss = 0.f;
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
@@ -294,20 +300,20 @@ __global__ __launch_bounds__(256) void moe_route_fused_kernel(RouteFusedArgs a) 
   }
   __syncthreads();
   // 2. the router product: wave s takes strip s (experts 16 s ..) over the whole contraction, the four tokens in
-  //    columns 0..3 (the other columns repeat them and are dropped), sixteen k-steps of weights in flight
+  //    columns 0..3 (the other columns repeat them and are dropped), 32 k-steps of weights in flight
   {
     const int m = lane & 15, g = lane >> 4;
     const int strips = (a.E + 15) >> 4;
     if (wave < strips) {
-      const uint4* wrow = a.wp + (size_t)wave * KS * 64 + lane;
       const bf16_t* xrow = xs + (size_t)(m & 3) * ldxs + 8 * g;
       f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
-      for (int jb = 0; jb < KS; jb += 16) {
-        uint4 wv[16];
+      for (int jb = 0; jb < KS; jb += 32) {
+        if (jb) {
 #pragma unroll
-        for (int c = 0; c < 16; ++c) wv[c] = ldg16_nt(wrow + (size_t)min(jb + c, KS - 1) * 64);
+          for (int c = 0; c < 32; ++c) wv[c] = ldg16_nt(wrow + (size_t)min(jb + c, KS - 1) * 64);
+        }
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
+        for (int c = 0; c < 32; ++c) {
           if (jb + c < KS) {
             const uint4 xv = *reinterpret_cast<const uint4*>(xrow + 32 * (jb + c));
             acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[c]), __builtin_bit_cast(bf16x8, xv),
