@@ -1330,38 +1330,41 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
   const float temp = a.temperature;
   const float u = a.u[(a.step_state && a.u_step_stride > 0 ? (size_t)a.step_state[1] * a.u_step_stride : 0) + b];
   const bf16_t* row = reinterpret_cast<const bf16_t*>(a.logits) + (size_t)b * a.ldl + base;
-  // One CU walks the whole row, so every instruction per id costs about half a microsecond.  The row
-  // is not kept in registers between the passes: each pass re-reads its 16 bytes per eight ids from
-  // the L2 and turns the two bf16 patterns of a register into order-preserving
-  // 16-bit keys with four integer instructions.  fn(id, key) is called for the thread's valid ids in
-  // id order; key 0 cannot occur for a number (it is the pattern of one NaN) and is skipped.
+  // One CU walks the whole row, so every instruction per id costs about half a microsecond: the two bf16 patterns of a
+  // register become order-preserving 16-bit keys with four integer instructions.  fn(id, key) is called for the valid ids among
+  // 8 id0 ..; key 0 cannot occur for a number (it is the pattern of one NaN) and is skipped.
+  // Where the order of a thread's ids does not matter - counting, and the search for a tie - it holds eighths NT chunks apart, `own`:
+  // a wave's load is 1 KiB in one piece, and they stay in registers from one pass to the next.  (64 ids in a row a thread, read again for the
+  // second pass, were sixty-four lines a load: 25.6 us a row of 65536 ids, 22.2 so, 18.7 with the counting below without a question per id.)
+  // The draw in vocabulary order adds up 64 ids in a row a thread and reads them so.
   // All loads of a pass go out before the first is used (addresses past the valid ids fall back on the
   // chunk of the last valid id, whose values are not looked at): one round trip to the L2 per pass.
   const bf16_t* row0 = reinterpret_cast<const bf16_t*>(a.logits) + (size_t)b * a.ldl;
   const int last_chunk = nvalid > 0 ? ((nvalid - 1) & ~7) : 0;
-  auto for_each_key = [&](auto&& fn) {
+  auto each_key = [&](uint4 v, int id0, auto&& fn) {
+    if (id0 >= nvalid) return;
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    const bool whole = id0 + 8 <= nvalid;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t neg = ((w[j] >> 15) & 0x00010001u) * 0xffffu;  // 0xffff in the halves that hold a negative value
+      const uint32_t kk = w[j] ^ (neg | 0x80008000u);                // negative: all bits flipped; else the sign bit set
+      const uint32_t klo = kk & 0xffffu, khi = kk >> 16;
+      if (klo && (whole || id0 + 2 * j < nvalid)) fn(id0 + 2 * j, klo);
+      if (khi && (whole || id0 + 2 * j + 1 < nvalid)) fn(id0 + 2 * j + 1, khi);
+    }
+  };
+  auto for_each_key = [&](auto&& fn) {  // the thread's EPT ids in a row, in id order
     uint4 vv[EPT / 8];
 #pragma unroll
     for (int c = 0; c < EPT / 8; ++c) vv[c] = ldg16(row0 + min(base + 8 * c, last_chunk));
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int c = 0; c < EPT / 8; ++c) {
-      const int id0 = base + 8 * c;
-      if (id0 < nvalid) {
-        const uint4 v = vv[c];
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-        const bool whole = id0 + 8 <= nvalid;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t neg = ((w[j] >> 15) & 0x00010001u) * 0xffffu;  // 0xffff in the halves that hold a negative value
-          const uint32_t kk = w[j] ^ (neg | 0x80008000u);                // negative: all bits flipped; else the sign bit set
-          const uint32_t klo = kk & 0xffffu, khi = kk >> 16;
-          if (klo && (whole || id0 + 2 * j < nvalid)) fn(id0 + 2 * j, klo);
-          if (khi && (whole || id0 + 2 * j + 1 < nvalid)) fn(id0 + 2 * j + 1, khi);
-        }
-      }
-    }
+    for (int c = 0; c < EPT / 8; ++c) each_key(vv[c], base + 8 * c, fn);
   };
+  uint4 own[EPT / 8];
+#pragma unroll
+  for (int c = 0; c < EPT / 8; ++c) own[c] = ldg16(row0 + min(8 * (c * NT + tid), last_chunk));
   auto xval = [&](uint32_t key) { return key16_value(key) / temp; };
   const bool nucleus = a.top_p > 0.f && a.top_p < 1.f;
   const bool want_table = a.top_k > 0 || nucleus;
@@ -1370,16 +1373,39 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
     for (int i = tid; i < HB / 4; i += NT) h4[i] = make_uint4(0, 0, 0, 0);
     __syncthreads();
   }
-  int tmax = 0, tmin = 0x10000, live = 0;
-  for_each_key([&](int, uint32_t kk) {
-    tmax = max(tmax, (int)kk);
-    tmin = min(tmin, (int)kk);
-    ++live;
-    if (want_table) atomicAdd(&hist[kk >> 1], (kk & 1u) ? 0x10000u : 1u);
-  });
-  int kmax = tmax, nkmin = -tmin, n_live = live;
-  block_max_max_sum_i(kmax, nkmin, n_live, s);  // (the barriers inside also complete the table)
+  // Counting and extremes, without a question per id: the key no number has is counted like the others (and left out of the list).
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  u16x2 hi2 = {0, 0}, lo2 = {0xffff, 0xffff};
+#pragma unroll
+  for (int c = 0; c < EPT / 8; ++c) {
+    const int id0 = 8 * (c * NT + tid);
+    const uint32_t w[4] = {own[c].x, own[c].y, own[c].z, own[c].w};
+    if (id0 + 8 <= nvalid) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t kk = w[j] ^ ((((w[j] >> 15) & 0x00010001u) * 0xffffu) | 0x80008000u);
+        hi2 = __builtin_elementwise_max(hi2, __builtin_bit_cast(u16x2, kk));
+        lo2 = __builtin_elementwise_min(lo2, __builtin_bit_cast(u16x2, kk));
+        if (want_table) {
+          atomicAdd(&hist[(kk & 0xffffu) >> 1], 1u << ((kk & 1u) << 4));
+          atomicAdd(&hist[kk >> 17], 1u << ((kk >> 12) & 16u));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (id0 + i < nvalid) {
+          const uint32_t v = (w[i >> 1] >> (16 * (i & 1))) & 0xffffu, key = v ^ ((v & 0x8000u) ? 0xffffu : 0x8000u);
+          hi2[0] = max((int)hi2[0], (int)key);
+          lo2[0] = min((int)lo2[0], (int)key);
+          if (want_table) atomicAdd(&hist[key >> 1], 1u << ((key & 1u) << 4));
+        }
+    }
+  }
+  int kmax = max((int)hi2[0], (int)hi2[1]), nkmin = -min((int)lo2[0], (int)lo2[1]), unused = 0;
+  block_max_max_sum_i(kmax, nkmin, unused, s);  // (the barriers inside also complete the table)
   const int kmin = -nkmin;
+  const int n_live = nvalid - (want_table ? (int)(hist[0] & 0xffffu) : 0);  // (asked for with the table only)
   int token = 0;
   if (kmax > 0) {
     const float m = xval((uint32_t)kmax);
@@ -1395,28 +1421,27 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
     int n_ent = 1;
     if (need_table) {
       const uint4* seg = reinterpret_cast<const uint4*>(hist + HB - 32 * (tid + 1));  // my 64 keys, ascending
-      uint4 sv[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) sv[q] = seg[q];
-      int nz = 0;
+      int nz = 0;  // counted with neighbouring lanes at different eighths of their 128 bytes (in step they meet on two banks' worth)
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        const uint32_t w[4] = {sv[q].x, sv[q].y, sv[q].z, sv[q].w};
+        const uint4 sv = seg[(q + tid) & 7];
+        const uint32_t w[4] = {tid == NT - 1 && ((q + tid) & 7) == 0 ? sv.x & 0xffff0000u : sv.x, sv.y, sv.z, sv.w};  // (not key 0)
 #pragma unroll
         for (int i = 0; i < 4; ++i) nz += ((w[i] >> 16) ? 1 : 0) + ((w[i] & 0xffffu) ? 1 : 0);
       }
       int off;
       n_ent = block_excl_scan_i(nz, off, s);
-      if (n_ent <= ENT_CAP && nz) {
+      if (n_ent <= ENT_CAP && nz) {  // few threads hold a key
         const int kbase = 65536 - 64 * (tid + 1);  // key of the low half of seg[0].x
 #pragma unroll
         for (int q = 7; q >= 0; --q) {
-          const uint32_t w[4] = {sv[q].x, sv[q].y, sv[q].z, sv[q].w};
+          const uint4 sv = seg[q];
+          const uint32_t w[4] = {sv.x, sv.y, sv.z, sv.w};
 #pragma unroll
           for (int i = 3; i >= 0; --i) {
             const int key = kbase + 8 * q + 2 * i;
             if (w[i] >> 16) ent[off++] = ((uint32_t)(key + 1) << 16) | (w[i] >> 16);
-            if (w[i] & 0xffffu) ent[off++] = ((uint32_t)key << 16) | (w[i] & 0xffffu);
+            if (key && (w[i] & 0xffffu)) ent[off++] = ((uint32_t)key << 16) | (w[i] & 0xffffu);
           }
         }
       }
@@ -1562,41 +1587,58 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
       __syncthreads();
       const uint32_t Td = (uint32_t)s.misc[7];
       const int r = s.misc[3];
-      // the r-th id, in id order, among the ids with key Td: one pass notes where in the thread's ids
-      // the key occurs (the bf16 pattern behind the key is compared as loaded: two instructions an id,
-      // on a CU that spends 0.44 us on every instruction per id), the thread that owns the r-th
-      // occurrence picks it from its own notes
+      // The r-th id, in id order, among the ids with key Td: the bf16 pattern behind the key is compared as loaded (two instructions an
+      // id), every thread notes where it occurs among its own, the totals of the NT-wide eighths say which of them holds the r-th, and a
+      // scan over that one which thread.
+      constexpr int NC = EPT / 8;
+      static_assert(NC <= 8, "one bit per id of the thread, one counter per eighth");
       unsigned long long where = 0;
       {
         const uint32_t pat = (Td & 0x8000u) ? (Td & 0x7fffu) : (~Td & 0xffffu);  // key -> bf16 bits
         const uint32_t pat2 = pat | (pat << 16);
-        uint4 vv[EPT / 8];
 #pragma unroll
-        for (int c = 0; c < EPT / 8; ++c) vv[c] = ldg16(row0 + min(base + 8 * c, last_chunk));
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int c = 0; c < EPT / 8; ++c) {
-          const uint32_t w[4] = {vv[c].x, vv[c].y, vv[c].z, vv[c].w};
+        for (int c = 0; c < NC; ++c) {
+          const uint32_t w[4] = {own[c].x, own[c].y, own[c].z, own[c].w};
+          uint32_t at = 0;
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const uint32_t x = w[j] ^ pat2;
-            if ((x & 0xffffu) == 0) where |= 1ull << (8 * c + 2 * j);
-            if ((x >> 16) == 0) where |= 1ull << (8 * c + 2 * j + 1);
+            if ((x & 0xffffu) == 0) at |= 1u << (2 * j);
+            if ((x >> 16) == 0) at |= 1u << (2 * j + 1);
           }
+          // ids at or past the end of the valid ones (and the chunks that stood in for them) do not count
+          const int nv = nvalid - 8 * (c * NT + tid);
+          at = nv >= 8 ? at : nv <= 0 ? 0u : at & ((1u << nv) - 1u);
+          where |= (unsigned long long)at << (8 * c);
         }
-        // ids at or past the end of the valid ones (and the chunks that stood in for them) do not count
-        const int nv = nvalid - base;
-        where = nv >= EPT ? where : (nv <= 0 ? 0ull : where & ((1ull << nv) - 1ull));
       }
-      static_assert(EPT <= 64, "one bit per id of the thread");
-      const int c = __popcll(where);
-      int off;
-      block_excl_scan_i(c, off, s);
+      if (tid < NC) s.hist[tid] = 0;
       if (tid == 0) s.misc[2] = -1;
       __syncthreads();
-      if (c > 0 && off <= r && r < off + c) {
-        for (int skip = r - off; skip > 0; --skip) where &= where - 1;  // drop the occurrences before the r-th
-        s.misc[2] = base + __ffsll((long long)where) - 1;
+#pragma unroll
+      for (int c = 0; c < NC; c += 2) {  // two eighths' counts in one word (a wave holds at most 512 of each)
+        const int both = __popc((uint32_t)(where >> (8 * c)) & 0xffu) | (__popc((uint32_t)(where >> (8 * c + 8)) & 0xffu) << 16);
+        const int sum = lanes_sum<32, 1>(c + 1 < NC ? both : both & 0xffff);
+        if ((tid & 63) == 0 && sum) {
+          atomicAdd(&s.hist[c], sum & 0xffff);
+          if (c + 1 < NC) atomicAdd(&s.hist[c + 1], sum >> 16);
+        }
+      }
+      __syncthreads();
+      int left = r, eighth = 0;
+#pragma unroll
+      for (int c = 0; c < NC - 1; ++c)
+        if (eighth == c && left >= (int)s.hist[c]) {
+          left -= (int)s.hist[c];
+          eighth = c + 1;
+        }
+      uint32_t mine = (uint32_t)(where >> (8 * eighth)) & 0xffu;
+      const int c = __popc(mine);
+      int off;
+      block_excl_scan_i(c, off, s);
+      if (c > 0 && off <= left && left < off + c) {
+        for (int skip = left - off; skip > 0; --skip) mine &= mine - 1;  // drop the occurrences before it
+        s.misc[2] = 8 * (eighth * NT + tid) + __ffs((int)mine) - 1;
       }
       __syncthreads();
       token = max(s.misc[2], 0);
@@ -1706,9 +1748,9 @@ int sample_dispatch(const void* logits, int logits_are_fp32, int ldl, int batch,
     return ohara_launch_status();
   }
   // bf16 rows: selection on the histogram of the 16-bit patterns, except for a small top-k, where sorting
-  // the few survivors is quicker (measured at 65536 ids: top-k 50 + top-p 0.9: 27 us sorted, 37 us by the
-  // table; top-p alone: 37 us (sharp row) to 139 us (flat row) with candidates / bisection, 37-38 us by
-  // the table whatever the row; plain multinomial 33 us either way)
+  // the few survivors is as quick or quicker (top-k 50 + top-p 0.9: 32000 ids 12.8 us sorted, 15.4 by the table; 51200 18.7 and 18.6;
+  // 65536 20.1 and 19.0, where the two add up in different orders; top-p alone: 37 us (sharp row) to 139 us (flat row) with
+  // candidates / bisection, 19 us by the table whatever the row; plain multinomial 25 us)
   const bool small_k = top_k > 0 && top_k <= CAP;
   if (!logits_are_fp32 && !small_k && vocab <= 65536 && (ldl & 7) == 0 &&
       (reinterpret_cast<uintptr_t>(logits) & 15) == 0) {
