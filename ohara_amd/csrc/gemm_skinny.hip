@@ -16,6 +16,8 @@
 //                               ohara/modules/kv_cache.py:104-105
 #include "gemm_epilogue.h"
 
+#include <type_traits>
+
 namespace {
 
 __device__ __forceinline__ float sumsq8(uint4 v) {
@@ -422,8 +424,11 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void wide_kernel(GemmArgs a) {
   const int ldxs = KS * 32 + 8;
   const int stride = gridDim.x * WIDE_WAVES;
   int strip = blockIdx.x * WIDE_WAVES + wave;
-  // two register buffers of WIDE_CH k-steps; the first strip's are requested before the
-  // activations are staged, so the weight stream starts with the kernel
+  // Two register buffers of WIDE_CH k-steps.  The first strip's are requested before the activations are staged, so the
+  // weight stream starts with the kernel, but behind the request for the rows, where those fit registers: loads return in
+  // order, so rows requested behind the weights wait for 24 KiB a wave before the norm can begin.  From a graph, weights in
+  // HBM, 1, 16, 32 and 64 rows: 32768 x 768 12.3 13.0 14.8 19.3 us (rows behind the weights 13.3 14.0 15.9 21.6; a copy's
+  // rate would take 9.9); 32000 x 2048, up to 32 rows, 26.4 26.6 28.0 (27.3 30.1 33.7, one row at a time; 25.9).
   uint4 wa[WIDE_CH], wb[WIDE_CH];
   // No branch around a load and nothing that touches the value: k-steps and strips outside the
   // matrix read a valid tile instead and are never multiplied (mul() skips k-steps >= KS, the strip
@@ -434,15 +439,11 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void wide_kernel(GemmArgs a) {
 #pragma unroll
     for (int c = 0; c < WIDE_CH; ++c) w[c] = ldg16_nt(wrow + (size_t)min(j + c, KS - 1) * 64);
   };
-  load(wa, strip, 0);
-  load(wb, strip, WIDE_CH);
-
-  if (a.K <= 1024) {
-    // every row of this wave is requested before any is used (K <= 1024: two 16-byte pieces per lane)
-    constexpr int RPW = 16 * BT / WIDE_WAVES;
-    uint4 v[RPW][2], nwv[2];
+  auto stage = [&](auto pieces) {  // every row of this wave in 16-byte pieces of 512 columns
+    constexpr int NP = decltype(pieces)::value, RPW = 16 * BT / WIDE_WAVES;
+    uint4 v[RPW][NP], nwv[NP];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < NP; ++c) {
       const int k = lane * 8 + 512 * c;
       nwv[c] = (NORM && k < a.K) ? ldg16(a.norm_w + k) : make_uint4(0, 0, 0, 0);
 #pragma unroll
@@ -451,19 +452,35 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void wide_kernel(GemmArgs a) {
         v[r][c] = (b < a.B && k < a.K) ? ldg16(a.x + (size_t)b * a.ldx + k) : make_uint4(0, 0, 0, 0);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    load(wa, strip, 0);
+    load(wb, strip, WIDE_CH);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
       const int b = wave + WIDE_WAVES * r;
       float rinv = 1.f;
-      if (NORM) rinv = 1.0f / sqrtf(wave_sum(sumsq8(v[r][0]) + sumsq8(v[r][1])) / (float)a.K + a.eps);
+      if (NORM) {
+        float ss = sumsq8(v[r][0]);
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
+        for (int c = 1; c < NP; ++c) ss += sumsq8(v[r][c]);
+        rinv = 1.0f / sqrtf(wave_sum(ss) / (float)a.K + a.eps);
+      }
+#pragma unroll
+      for (int c = 0; c < NP; ++c) {
         const int k = lane * 8 + 512 * c;
         if (k < KS * 32)
           *reinterpret_cast<uint4*>(xs + (size_t)b * ldxs + k) = NORM ? norm8(v[r][c], nwv[c], rinv) : v[r][c];
       }
     }
+  };
+  if (a.K <= 1024) {
+    stage(std::integral_constant<int, 2>());
+  } else if (BT <= 2 && a.K <= 2048) {
+    stage(std::integral_constant<int, 4>());
   } else {
+    load(wa, strip, 0);
+    load(wb, strip, WIDE_CH);
     for (int b = wave; b < 16 * BT; b += WIDE_WAVES) {
       float rinv = 1.f;
       if (NORM && b < a.B) {
