@@ -10,6 +10,7 @@
 // the online softmax are wavefront shuffle reductions.  Partial (max, sum, acc) triples of the chunks are
 // merged by whichever workgroup of the (sequence, KV head) finishes last, in chunk
 // order, so the result does not depend on scheduling.
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -28,6 +29,7 @@ struct AttnArgs {
   int pos_stride;
   int nsplit;        // chunks there is room for
   int most;          // chunks that pay where the walk is what takes the time (0: where the memory is), see cut_context
+  int most_long;     // the same for contexts of more than 4096 positions
   int* counters;     // (B*Hkv)
   float* part_ml;    // (B, Hkv, nsplit of room: G, chunks, 2)
   float* part_acc;   // (B, Hkv, nsplit of room: G, chunks, D)
@@ -122,6 +124,12 @@ __device__ void merge_partials(const AttnArgs& a, int b /* query row */, int kvh
 //                                1500  27.6 / 17.6 / 17.0 / 17.5;  4000  65 / 37.4 / 36.3 / 39.8
 //   192 pairs (1 / 4 / 5)        100  5.0 / 7.8 / 7.8;  530  13.2 / 16.0 / 14.3;  700  16.4 / 17.4 / 17.7;  1500  30.5 / 28.7 / 29.4
 //   12 pairs (1 / 8 / 16 / 32)   300  6.6 / 6.8 / 7.3 / 9.8;  700  12.5 / 7.9 / 8.1 / 9.8;  4000  56 / 14.3 / 11.7 / 12.7
+// 81 to 128 pairs, where the room is 8 to 11 chunks; chunks: us a launch, 768 / 1536 / 4096 / 16384 positions:
+//   heads of 128, 1 head each   96 pairs   5: 13.6 19.0 39.2 133   8: 13.7 18.2 37.8 128   10: 13.9 18.6 40.2 134;  int8 5: 13.6 17.6 29.8 85.6
+//                                          8: 10.8 16.6 27.4 80.9;  88 pairs, int8  5: 12.9 19.1 31.7 96.9   8: 10.6 16.1 28.2 87.1   11: 11.5 16.2 25.5 75.3
+//   heads of 128, 4 heads each  128 pairs  4: 17.8 25.8 54.3 193   8: 19.8 28.1 56.1 185;  int8 4: 17.3 22.2 41.8 129   8: 17.3 22.5 41.7 122
+//   heads of 64                 128 pairs, 4 heads each  4: 12.6 17.7 34.3 112   8: 13.2 18.4 34.9 113;  96 pairs, 8192 / 32768  8: 41.0 141   10: 42.7 150
+// so: one head each, eight; several, two workgroups a CU; with heads of 128 the room's four a CU from 4096 positions on.
 struct Cut {
   int chunk, used;
 };
@@ -129,7 +137,7 @@ __device__ __forceinline__ Cut cut_context(const AttnArgs& a, int L, int unit /*
   const int n64 = (L + 63) >> 6;
   int want = a.nsplit;
   if (n64 <= 5 || (a.most == 0 && n64 <= 12)) want = 1;
-  else if (a.most) want = min(want, min((n64 + 1) >> 1, a.most));
+  else if (a.most) want = min(want, min((n64 + 1) >> 1, n64 > 64 ? a.most_long : a.most));
   const int chunk = max((L + want - 1) / want + unit - 1, unit) & ~(unit - 1);
   return {chunk, max((L + chunk - 1) / chunk, 1)};
 }
@@ -970,7 +978,11 @@ static int attn_cached_impl(const uint16_t* q, const void* kcache, const void* v
   a.nsplit = n_split;
   batch *= seq_len;  // one workspace slot per query row
   const int64_t pairs = (int64_t)batch * h_kv;
-  a.most = pairs <= 80 ? (int)(256 / pairs) : pairs <= 128 ? (int)(512 / pairs) : 0;  // one workgroup a CU where that is even, or two
+  a.most = a.most_long = pairs <= 80 ? (int)(256 / pairs) : 0;  // one workgroup a CU
+  if (pairs > 80 && pairs <= 128) {
+    a.most = (int)(h == h_kv ? std::min<int64_t>(8, 1024 / pairs) : 512 / pairs);
+    a.most_long = dh == 128 ? (int)(1024 / pairs) : a.most;
+  }
   char* ws = reinterpret_cast<char*>(workspace);
   a.counters = reinterpret_cast<int*>(ws);
   ws += fixed_counter_bytes ? fixed_counter_bytes : align256((size_t)batch * h_kv * sizeof(int));

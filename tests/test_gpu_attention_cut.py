@@ -62,3 +62,18 @@ def test_lengths_where_the_cut_changes(cuda, B, H, Hkv, D, int8):
         for b, L in enumerate(lengths):
             scale = whole[L][b].float().abs().max().item()
             assert (got[b].float() - whole[L][b].float()).abs().max().item() <= scale * 2.0 ** -8
+
+
+@pytest.mark.parametrize("B,H,Hkv,D", [(16, 8, 8, 128), (12, 32, 8, 128), (12, 8, 8, 64)])
+def test_lengths_around_4096(cuda, B, H, Hkv, D):
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(B + H + D)
+    q = torch.randn(B, H * D, generator=g, device=cuda).to(BF)
+    k, v = (torch.randn(B, 4200, Hkv, D, generator=g, device=cuda).to(BF) for _ in range(2))
+    rooms = {ns: ops.attn_workspace(B, H, Hkv, D, ns, cuda) for ns in (8, 10, 33)}
+    for L in (4096, 4097, 4161):
+        want, bound = _exact(q.view(B, H, D), k, v, [L] * B)
+        for ns, ws in rooms.items():
+            got = ops.attn_cached(q, k, v, H, Hkv, D, L - 1, ns, ws)
+            assert ((got.view(B, H, D).double() - want).abs() <= bound).all()
