@@ -138,7 +138,8 @@ int ohara_qkv_rope_ragged_bf16(const uint16_t* x, int ldx, const uint16_t* wp, i
  * positions [0, pos + s] (the cache mask key_pos <= start_pos + q_idx, llama.py:109-113):
  *   out[b, s, h, :] = softmax(q[b,s,h,:] . K[b, 0:pos+s+1, h/(H/Hkv), :] / sqrt(dh)) V
  * (llama.py:100-135; GQA by head indexing instead of repeat_interleave :101-103).
- * seq_len = 1 is the decode case.  The context is split into `n_split` chunks;
+ * seq_len = 1 is the decode case.  The context is split into at most `n_split` chunks
+ * (dh 64 and 128: as many as its length at the call asks for; otherwise `n_split`);
  * partial (max, sum, acc) triples go to `workspace` and the last chunk to finish
  * merges them in chunk order.  workspace bytes = ohara_attn_workspace_bytes(
  * batch*seq_len, h, h_kv, dh, n_split); zero-fill it once before first use (the
@@ -177,7 +178,7 @@ int ohara_attn_cached_bf16_noalloc(const uint16_t* q, const uint16_t* kcache, co
                                    int n_split, uint16_t* out, void* stream);
 
 /* Same contract for many query positions per sequence (prefill), as a causal flash-style kernel
- * on MFMA: 128 queries per workgroup, keys/values walked in 64-position tiles through LDS,
+ * on MFMA: 16 to 128 queries per workgroup, keys/values walked in 64-position tiles through LDS,
  * online softmax in fp32, probabilities rounded to bf16 for the second product.  dh 64 or 128.
  * Needs no workspace.  (llama.py:100-135 with S > 1.) */
 int ohara_attn_prefill_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int batch,

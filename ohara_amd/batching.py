@@ -3,9 +3,10 @@ when a slot is free and leave when they finish.
 
 The reference drives `Llama.forward` with a single scalar position for the whole batch
 (ohara/models/llama.py:287-299, ohara/chat_engine.py:395-405), so all sequences of a batch must
-have the same length and start together.  Here every slot of the KV caches has its own length: a
-prompt is prefilled into its slot alone, and one decode step advances every active slot at its own
-position (`Llama.forward` with one position per sequence).  Selection is greedy or the fused
+have the same length and start together.  Here every slot of the KV caches has its own length: prompts
+are prefilled into their slots side by side where the model takes them so (`Llama.prompts`), one by one
+elsewhere, and one decode step advances every active slot at its own position (`Llama.forward` with
+one position per sequence).  Selection is greedy or the fused
 temperature / top-k / top-p sampler of ohara/chat_engine.py:51-82.
 """
 

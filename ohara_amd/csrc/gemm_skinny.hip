@@ -4,9 +4,10 @@
 // order whose every wave-load is one contiguous 1 KiB (64 lanes x 16 B), straight
 // into the A operand of v_mfma_f32_16x16x32_bf16; the activations are the B
 // operand (16 batch columns per MFMA), so batch 1..16 costs the same weight
-// stream.  One workgroup (4 waves) owns one 16-row strip; the waves split K and
-// their fp32 partial tiles are summed in a fixed order through LDS, so results do
-// not depend on scheduling.
+// stream.  One workgroup (4 to 16 waves) owns one 16-row strip (group_kernel: two to
+// four strips that share the normed rows; wide_kernel: whole strips per wave); the waves
+// split K and their fp32 partial tiles are summed in a fixed order through LDS, so
+// results do not depend on scheduling.
 //
 // Fusions (rounding points follow the reference's bf16 eager path):
 //   prologue  RMSNorm           ohara/modules/norm.py:16-21

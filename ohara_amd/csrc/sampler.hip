@@ -13,8 +13,8 @@
 // that order open).  Every reduction runs in a fixed order, so the result is a pure
 // function of (logits, parameters, u).
 //
-// A thread owns EPT consecutive vocabulary entries in registers; the 1024 threads cover up to
-// 1024*EPT ids.  Three routes from there:
+// bf16 rows without a small top-k go by a table of their patterns (sample_hist_kernel).  Otherwise a thread
+// owns EPT consecutive vocabulary entries in registers; the 1024 threads cover up to 1024*EPT ids.  Three routes from there:
 //   * top-p alone on bf16 rows (the reference's chat default, chat_engine.py:35-37): every id at or
 //     above the 256-th largest per-thread maximum is a candidate; if the candidates' share of the
 //     whole-row softmax exceeds top_p they are sorted and scanned like the survivors of a small

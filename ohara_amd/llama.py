@@ -298,10 +298,9 @@ class Llama:
                 for i in range(c.num_hidden_layers)]
 
     def default_n_split(self, batch: int) -> int:
-        """Context chunks per (sequence, KV head) so that decode attention launches about
-        four workgroups per CU (measured on d12, 6 KV heads, at batch 16 / 32 / 64: 6, 6 and 2-4
-        chunks are the fastest, twice as many are slower); a chunk is never shorter than 128
-        positions."""
+        """Most context chunks per (sequence, KV head), which is what the workspace has room for: about
+        four workgroups per CU, none shorter than 128 positions of a full window.  The kernel takes as
+        many of them as the context's length at the step asks for."""
         want = max(1, 1024 // max(1, batch * self.kv_heads))
         return max(1, min(want, self.config.max_sequence_length // 128, 64))
 
