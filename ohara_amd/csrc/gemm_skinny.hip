@@ -285,6 +285,60 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
   }
 }
 
+// Rows without a norm, K up to 6144: a wave's share of K is at most CH k-steps, all of them requested before anything waits.  Above, rounds
+// of six cost a round trip each; and a request costs what it costs whether its data are used, so CH is the share, rounded up to even.
+// H = 2: a workgroup takes half a strip (eight columns, in both halves of the product's sixteen), where strips leave CUs idle.
+// The sums are skinny_kernel's with as many waves.  us a call, from a graph with weights in HBM, skinny_kernel with four waves / this with H = 1
+// / H = 2, at 1, 8, 16, 32 and 64 rows (four waves up to K 3072, then eight):
+//    768 x 768   2.81 3.27 3.64 3.70 3.75 / 2.73 3.25 3.63 3.65 3.64 / 2.93 3.30 3.68 3.75 4.61
+//   1024 x 1024  3.77 4.15 4.40 4.38 4.38 / 3.10 3.33 3.69 3.69 3.71 / 3.19 3.35 3.69 3.73 4.90
+//   2048 x 2048  5.31 5.82 6.35 6.35 8.20 / 4.05 4.43 5.21 5.18 7.80 / 4.11 4.31 5.01 7.21 12.1
+//    768 x 3072  5.48 6.54 7.38 7.34 7.23 / 4.59 5.50 6.68 6.64 6.56 / 4.67 5.11 6.29 6.43 9.67
+//   1024 x 4096  7.00 8.10 9.04 8.93 8.89 / 5.18 6.32 7.92 7.80 7.76 / 5.24 5.94 7.53 7.65 13.3
+//   2048 x 5632  9.64 10.7 11.5 11.2 17.9 / 8.19 8.43 10.8 10.3 18.2 / 7.73 7.37 9.47 16.9 31.4
+//   4096 x 2048  6.33 6.60 6.76 8.71 14.2 / 4.99 5.10 5.77 8.14 12.8;  4096 x 4096  8.90 9.72 10.0 14.5 24.6 / 7.55 7.64 8.94 14.7 26.7
+// Sixteen waves are no faster (768 x 3072 4.59 5.68 7.04 6.87 6.75, 2048 x 5632 9.08 10.6 13.2 13.2 22.9).
+template <int EPI, int H, int NW, int CH>
+__global__ __launch_bounds__(NW * 64) void once_kernel(GemmArgs a) {
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int part = (local / a.ny) * 8 + xcd, strip = part / H, half = part % H;
+  const int rbase = (local % a.ny) * 16;
+  if (strip >= a.nstrips) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 15, g = lane >> 4;
+  const int KS = (a.K + 31) >> 5;
+  const int per_wave = (KS + NW - 1) / NW;
+  const int j0 = wave * per_wave, j1 = min(KS, j0 + per_wave);
+  const int b = rbase + m, q = H == 2 ? 2 * half + (g & 1) : g;  // q: which four of the strip's columns this lane finishes
+  __shared__ f32x4 red[NW - 1][64];
+  const bool pre_ok = ((a.N | a.ldo | a.ldr) & 3) == 0 && EPI == EPI_RESIDUAL;
+  EpiPre ep;
+  if (wave == 0 && pre_ok) gemm_epilogue_fetch<EPI>(a, b, strip, q, ep);
+  const uint4* wrow = a.wp + (size_t)strip * KS * 64 + (H == 2 ? 16 * g + 8 * half + (m & 7) : lane);
+  const bf16_t* xrow = a.x + (size_t)min(b, a.B - 1) * a.ldx;
+  uint4 wv[CH], xv[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    wv[c] = ldg16_nt(wrow + (size_t)min(j0 + c, KS - 1) * 64);
+    xv[c] = ldg16(xrow + min(32 * (j0 + c) + 8 * g, a.K - 8));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const uint4 xn = 32 * (j0 + c) + 8 * g < a.K ? xv[c] : make_uint4(0, 0, 0, 0);
+    if (j0 + c < j1) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[c]), __builtin_bit_cast(bf16x8, xn), acc, 0, 0, 0);
+  }
+  if (wave > 0) red[wave - 1][lane] = acc;
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int w = 0; w < NW - 1; ++w) acc += red[w][lane];
+  if (g >= 4 / H || b >= a.B) return;
+  if (pre_ok) gemm_epilogue<EPI, true>(a, b, strip, q, acc, ep);
+  else gemm_epilogue<EPI>(a, b, strip, q, acc);
+}
+
 // Normed rows against 257 to 1024 strips, K <= 2048: S strips a workgroup, as many as make about one workgroup a CU of them.
 // Above, every strip's workgroup norms the rows again (48 vector instructions a lane and k-step: 704 strips at 32 rows kept the
 // chip busy for half of the launch) and its loads come in rounds.  Here NW waves split K so far that a wave's share is at
@@ -580,6 +634,46 @@ int launch_wide(const GemmArgs& a0, int epi, int strips, hipStream_t st) {
   }
 }
 
+template <int EPI, int H, int NW, int CH>
+int launch_once_as(const GemmArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL((once_kernel<EPI, H, NW, CH>), dim3((unsigned)((H * a.nstrips + 7) / 8 * 8 * a.ny)), dim3(NW * 64), 0, st, a);
+  return ohara_launch_status();
+}
+template <int EPI, int H>
+int launch_once_h(const GemmArgs& a, hipStream_t st) {
+  const int KS = (a.K + 31) >> 5;
+  if (KS <= 96) switch ((KS + 7) / 8 * 2) {  // four waves' shares, even
+    case 2: case 4: case 6: return launch_once_as<EPI, H, 4, 6>(a, st);
+    case 8: return launch_once_as<EPI, H, 4, 8>(a, st);
+    case 10: return launch_once_as<EPI, H, 4, 10>(a, st);
+    case 12: return launch_once_as<EPI, H, 4, 12>(a, st);
+    case 14: return launch_once_as<EPI, H, 4, 14>(a, st);
+    case 16: return launch_once_as<EPI, H, 4, 16>(a, st);
+    case 18: return launch_once_as<EPI, H, 4, 18>(a, st);
+    case 20: return launch_once_as<EPI, H, 4, 20>(a, st);
+    case 22: return launch_once_as<EPI, H, 4, 22>(a, st);
+    default: return launch_once_as<EPI, H, 4, 24>(a, st);
+  }
+  switch ((KS + 15) / 16 * 2) {
+    case 14: return launch_once_as<EPI, H, 8, 14>(a, st);
+    case 16: return launch_once_as<EPI, H, 8, 16>(a, st);
+    case 18: return launch_once_as<EPI, H, 8, 18>(a, st);
+    case 20: return launch_once_as<EPI, H, 8, 20>(a, st);
+    case 22: return launch_once_as<EPI, H, 8, 22>(a, st);
+    default: return launch_once_as<EPI, H, 8, 24>(a, st);
+  }
+}
+// Past K 3072 while the workgroups are one to a CU (beyond, the eight waves' requests only queue: 4096 x 4096 above).
+bool once_applies(const GemmArgs& a, int epi, int strips) {
+  return !a.norm_w && (epi == EPI_STORE || epi == EPI_RESIDUAL) && (a.K <= 3072 || (a.K <= 6144 && strips * a.ny <= 256));
+}
+// Half a strip each while that is at most a workgroup to a CU; up to K 1024, and with few rows up to 4096, it gains nothing.
+template <int EPI>
+int launch_once(const GemmArgs& a, hipStream_t st) {
+  const bool half = 2 * a.nstrips * a.ny <= 256 && a.K > 1024 && (a.B >= 8 || a.K > 4096);
+  return half ? launch_once_h<EPI, 2>(a, st) : launch_once_h<EPI, 1>(a, st);
+}
+
 template <int BT, bool NORM>
 int launch_epi(const GemmArgs& a, int epi, int strips, hipStream_t st) {
   dim3 grid((unsigned)((strips + 7) / 8 * 8 * a.ny)), block(256);
@@ -657,6 +751,7 @@ int launch_chunk(const GemmArgs& a0, int epi, int strips, hipStream_t st) {
     if (epi == EPI_STORE) return launch_group<EPI_STORE>(a, st);
     return epi == EPI_SWIGLU ? launch_group<EPI_SWIGLU>(a, st) : launch_group<EPI_ROPE>(a, st);
   }
+  if (once_applies(a, epi, strips)) return epi == EPI_STORE ? launch_once<EPI_STORE>(a, st) : launch_once<EPI_RESIDUAL>(a, st);
   return a.norm_w ? launch_epi<1, true>(a, epi, strips, st) : launch_epi<1, false>(a, epi, strips, st);
 }
 
