@@ -71,7 +71,7 @@ __device__ __forceinline__ float sum8(uint4 v) {
 // NW waves per workgroup split K.  A workgroup keeps NW * CH KiB of weight loads in flight, so when
 // there are too few strips to put several workgroups on every CU (few output rows, long K) 16 waves
 // instead of 4 are what fills the memory pipeline.
-template <int BT, int NORM, int EPI, int NW = 4>
+template <int BT, int NORM, int EPI, int NW = 4, int SP = 8>
 __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
   // k-steps whose loads are issued back to back (the many-wave variants have no norm operands to hold)
   constexpr int CH = (NORM == 0 && NW > 4) ? 10 : (BT <= 2 ? 6 : 4);
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
   // and, where a wave's share of K is at most SP k-steps (K <= 1024 with four waves), the rows, the norm weights and
   // the weights of the whole share in one go - the rows arrive first (loads return in order), the norm's sums run
   // while the weights are still on their way, and the rows are not fetched a second time.
-  constexpr int SP = 8;
+  // (A request past the share costs as much as one that is used: SP is 6 where the share is.)
   const bool pre_ok = ((a.N | a.ldo | a.ldr | a.ldr2) & 3) == 0 && EPI != EPI_STORE && EPI != EPI_SWIGLU && EPI != EPI_SOFTCAP && EPI != EPI_GELU_LOOKUP && EPI != EPI_GLU;
   EpiPre ep[BT];
   if (wave == 0 && pre_ok) {
@@ -434,22 +434,23 @@ int launch_group_s(const GemmArgs& a, hipStream_t st) {
   hipLaunchKernelGGL((group_kernel<BT, EPI, S, NW, SP>), dim3((a.nstrips + S - 1) / S, (a.B + 16 * BT - 1) / (16 * BT)), dim3(NW * 64), LDS, st, a);
   return ohara_launch_status();
 }
-template <int BT, int EPI>
-int launch_group_bt(const GemmArgs& a, hipStream_t st) {
-  const int per_cu = (a.nstrips + 255) / 256;
-  if (a.K <= 1024) switch (per_cu) {
-    case 2: return launch_group_s<BT, EPI, 2, 8, 4>(a, st);
-    case 3: return launch_group_s<BT, EPI, 3, 8, 4>(a, st);
-    default: return launch_group_s<BT, EPI, 4, 8, 4>(a, st);
-  }
-  switch (per_cu) {
-    case 2: return launch_group_s<BT, EPI, 2, 16, 4>(a, st);
-    case 3: return launch_group_s<BT, EPI, 3, 16, 4>(a, st);
-    default: return launch_group_s<1, EPI, 4, 16, 4>(a, st);  // (four strips and 32 rows at once do not fit the registers)
+template <int BT, int EPI, int NW, int SP>
+int launch_group_nw(const GemmArgs& a, hipStream_t st) {
+  switch ((a.nstrips + 255) / 256) {
+    case 2: return launch_group_s<BT, EPI, 2, NW, SP>(a, st);
+    case 3: return launch_group_s<BT, EPI, 3, NW, SP>(a, st);
+    default: return launch_group_s<NW == 16 ? 1 : BT, EPI, 4, NW, SP>(a, st);  // (four strips and 32 rows at once do not fit sixteen waves' registers)
   }
 }
+// The waves' shares: three k-steps or four, and no request past them: 6144 x 768, 1, 16, 32 and 64 rows 4.63 4.85 6.61 9.60 us with four,
+// 4.48 4.59 6.05 8.30 with three; 8192 x 1536 8.40 8.47 11.5 21.0 / 7.82 7.96 10.6 19.5.
+template <int BT, int EPI>
+int launch_group_bt(const GemmArgs& a, hipStream_t st) {
+  if (a.K <= 1024) return a.K <= 768 ? launch_group_nw<BT, EPI, 8, 3>(a, st) : launch_group_nw<BT, EPI, 8, 4>(a, st);
+  return a.K <= 1536 ? launch_group_nw<BT, EPI, 16, 3>(a, st) : launch_group_nw<BT, EPI, 16, 4>(a, st);
+}
 // us a call, a strip's workgroup each (four waves) / this kernel, 1, 16, 32 and 64 rows:
-//   11264 x 2048  14.8 20.1 33.9 58 / 10.7 11.1 15.8 29.4      6144 x 768  5.25 6.2 7.6 11.4 / 4.65 5.0 6.5 9.4
+//   11264 x 2048  14.8 20.1 33.9 58 / 10.7 11.1 15.8 29.4      6144 x 768  5.25 6.2 7.6 11.4 / 4.48 4.6 6.05 8.3
 //   8192 x 1024    6.1  6.8  9.5 15.4 / 5.4  5.4  7.6 12.9
 // With fewer strips than CUs a group is one strip, and there it is no faster: 2304 x 768 3.7 4.3 5.7 7.2 / 3.8 4.2 5.6 7.8; 3072 x 2048
 // with eight waves a strip 6.0 6.9 11.9 16.9 / 6.8 7.0 10.7 19.6.
@@ -704,8 +705,19 @@ int launch_epi(const GemmArgs& a, int epi, int strips, hipStream_t st) {
   // Normed rows of 1025 to 2048 columns: eight waves, so that a wave's share of K is requested in one go (3072 x 2048, 1, 16, 32 and 64
   // rows: 9.0, 10.2, 13.9, 18.7 us with four, 6.0, 6.9, 11.9, 16.9 with eight).
   if (NORM && a.K > 1024 && a.K <= 2048 && (epi == EPI_STORE || epi == EPI_ROPE)) {
-    if (epi == EPI_STORE) hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_STORE, 8>), grid, dim3(512), 0, st, a);
+    const bool six = a.K <= 1536;
+    if (epi == EPI_STORE && six) hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_STORE, 8, 6>), grid, dim3(512), 0, st, a);
+    else if (epi == EPI_STORE) hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_STORE, 8>), grid, dim3(512), 0, st, a);
+    else if (six) hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_ROPE, 8, 6>), grid, dim3(512), 0, st, a);
     else hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_ROPE, 8>), grid, dim3(512), 0, st, a);
+    return ohara_launch_status();
+  }
+  // Four waves' shares of at most six k-steps.  2304 x 768, 1, 16, 32 and 64 rows: 3.76 3.98 5.62 7.28 us with eight requested, 3.54 3.75 4.96
+  // 6.29 with six (2304 x 1536 above, eight waves: 5.42 6.45 10.6 14.9 / 4.97 5.74 8.00 10.6).
+  if (NORM && a.K <= 768 && (epi == EPI_STORE || epi == EPI_SWIGLU || epi == EPI_ROPE)) {
+    if (epi == EPI_STORE) hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_STORE, 4, 6>), grid, block, 0, st, a);
+    else if (epi == EPI_SWIGLU) hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_SWIGLU, 4, 6>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_ROPE, 4, 6>), grid, block, 0, st, a);
     return ohara_launch_status();
   }
   switch (epi) {

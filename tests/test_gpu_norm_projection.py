@@ -68,3 +68,16 @@ def test_rotary(cuda, B, H, Hkv, D, K):
     for got, plain in zip(*out):  # the rotation adds two values that may each be a neighbour
         assert (got != plain).float().mean() <= 0.05
         assert (got.float() - plain.float()).abs().max() <= 2.0 ** -6 * plain.float().abs().max()
+
+
+@pytest.mark.parametrize("n,k", [(40, 760), (2304, 768), (2304, 776), (40, 1528), (2312, 1536), (2304, 1544), (4112, 768), (4112, 776), (8200, 1536), (8200, 1544)])
+@pytest.mark.parametrize("rows", [1, 17, 40])
+def test_shares_of_three_and_six_steps(cuda, rows, n, k):
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(rows + n + k)
+    x = torch.randn(rows, k, generator=g, device=cuda).to(BF)
+    nw = (1 + 0.3 * torch.randn(k, generator=g, device=cuda)).to(BF)
+    w = (torch.randn(n, k, generator=g, device=cuda) * 0.05).to(BF)
+    packed = ops.pack_linear(w)
+    _check(ops.gemm_skinny(x, packed, nw, 1e-5), x, w, nw, 1e-5, ops.gemm_skinny(ops.rmsnorm(x, nw, 1e-5), packed))
