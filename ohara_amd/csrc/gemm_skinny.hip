@@ -93,7 +93,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
   __shared__ float ssum[NORM == 2 ? NW : 1][BT * 16];
 
   // A launch of this kernel is a chain of memory round trips - the rows for the norm, the weights, what the epilogue
-  // adds or rotates with - and lasts about as long as their sum (6-9 us for 1-9 MB at 32 rows).  What does not depend
+  // adds or rotates with - and lasts about as long as their sum (5-8 us for 1-9 MB at 32 rows).  What does not depend
   // on anything computed here is therefore requested first: the epilogue's operands (wave 0 finishes the fragments),
   // and, where a wave's share of K is at most SP k-steps (K <= 1024 with four waves), the rows, the norm weights and
   // the weights of the whole share in one go - the rows arrive first (loads return in order), the norm's sums run
@@ -290,6 +290,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
 // H = 2: a workgroup takes half a strip (eight columns, in both halves of the product's sixteen), where strips leave CUs idle.
 // The sums are skinny_kernel's with as many waves.  us a call, from a graph with weights in HBM, skinny_kernel with four waves / this with H = 1
 // / H = 2, at 1, 8, 16, 32 and 64 rows (four waves up to K 3072, then eight):
+//   1024 x 512   3.16 3.42 3.54 3.57 3.63 / 2.68 2.87 3.07 3.06 3.06
 //    768 x 768   2.81 3.27 3.64 3.70 3.75 / 2.73 3.25 3.63 3.65 3.64 / 2.93 3.30 3.68 3.75 4.61
 //   1024 x 1024  3.77 4.15 4.40 4.38 4.38 / 3.10 3.33 3.69 3.69 3.71 / 3.19 3.35 3.69 3.73 4.90
 //   2048 x 2048  5.31 5.82 6.35 6.35 8.20 / 4.05 4.43 5.21 5.18 7.80 / 4.11 4.31 5.01 7.21 12.1
@@ -644,7 +645,9 @@ template <int EPI, int H>
 int launch_once_h(const GemmArgs& a, hipStream_t st) {
   const int KS = (a.K + 31) >> 5;
   if (KS <= 96) switch ((KS + 7) / 8 * 2) {  // four waves' shares, even
-    case 2: case 4: case 6: return launch_once_as<EPI, H, 4, 6>(a, st);
+    case 2: return launch_once_as<EPI, H, 4, 2>(a, st);
+    case 4: return launch_once_as<EPI, H, 4, 4>(a, st);
+    case 6: return launch_once_as<EPI, H, 4, 6>(a, st);
     case 8: return launch_once_as<EPI, H, 4, 8>(a, st);
     case 10: return launch_once_as<EPI, H, 4, 10>(a, st);
     case 12: return launch_once_as<EPI, H, 4, 12>(a, st);
@@ -678,8 +681,7 @@ int launch_once(const GemmArgs& a, hipStream_t st) {
 template <int BT, bool NORM>
 int launch_epi(const GemmArgs& a, int epi, int strips, hipStream_t st) {
   dim3 grid((unsigned)((strips + 7) / 8 * 8 * a.ny)), block(256);
-  // Linear-with-bias calls with a long K (2048 and up): 16 waves per workgroup.  (For the d12 Llama
-  // projections, K 768 / 2048 with 48 - 256 strips, 16 waves measured no faster than 4.)
+  // Linear-with-bias calls with a long K (2048 and up): 16 waves per workgroup.
   if (!NORM && ((epi >= EPI_BIAS && epi <= EPI_BIAS_ADD2) || epi == EPI_BIAS_XIELU) && a.K >= 2048) {
     if (strips * a.ny >= 400) {  // enough workgroups for four per CU: 8 waves each measured 5-9 % faster
       dim3 mid(512);
