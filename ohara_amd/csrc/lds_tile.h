@@ -67,7 +67,8 @@ struct XOffsets {
 };
 
 // acc[u][t]: strip u x row block t of this wave.  ALIGNED: activation rows start on 16 bytes (false: through registers, any).
-// K is a multiple of 8; what the last step reads past it are the row's last piece and the strip's last tile, multiplied by zero.
+// K is a multiple of 8; what the last step reads past it are the row's last piece, which the packed weights' zeros meet as a zero, and the
+// strip's last tile, which nothing multiplies (times zero an infinite weight would be a NaN).
 __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
@@ -189,6 +190,7 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[C::FN][C::FM], const c
   if (tail) {
 #pragma unroll
     for (int jj = 0; jj < KH; ++jj) {
+      if (KB * nfull + 32 * jj >= K) break;  // (uniform) k-steps past the end: what stands in for them is not multiplied, not even by zero
       const bool in = KB * nfull + 32 * jj + 8 * g < K;
       uint4 wt[FN];
 #pragma unroll

@@ -72,6 +72,21 @@ def test_infinities_stay_in_their_row(cuda):
     assert torch.equal(got[17][at].double(), want[at])
 
 
+@pytest.mark.parametrize("rows,n,k", SHAPES)
+def test_infinite_weights_of_a_last_step(cuda, rows, n, k):
+    """An infinite weight in the last columns makes its own column of the result infinite and no NaN, also where K ends inside a step."""
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(7)
+    x = torch.rand(rows, k, generator=g, device=cuda).add_(0.5).to(BF)
+    w = torch.randn(n, k, generator=g, device=cuda).to(BF)
+    w[3, k - 1], w[n - 2, k - 8] = float("inf"), -float("inf")
+    got = ops.gemm(x, ops.pack_linear(w))
+    assert (got[:, 3] == float("inf")).all() and (got[:, n - 2] == -float("inf")).all()
+    rest = [c for c in range(n) if c not in (3, n - 2)]
+    assert got[:, rest].isfinite().all()
+
+
 # 96 rows take tiles that are 32 rows high, 4100 tiles of 192 columns, 9000 tiles of 256
 @pytest.mark.parametrize("rows,f", [(96, 264), (300, 3072), (1100, 1544), (2100, 5632), (4100, 1160), (9000, 3080)])
 @pytest.mark.parametrize("pad", [0, 1, 4])
