@@ -351,7 +351,7 @@ __global__ __launch_bounds__(NW * 64) void group_kernel(GemmArgs a) {
   f32x4(*red)[S * BT][64] = reinterpret_cast<f32x4(*)[S * BT][64]>(group_smem);
   __shared__ float ssq[NW][BT * 16];
   const int strip0 = blockIdx.x * S, rbase = blockIdx.y * 16 * BT;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, g = lane >> 4;
   const int KS = (a.K + 31) >> 5;
   const int per_wave = (KS + NW - 1) / NW;
@@ -392,6 +392,13 @@ __global__ __launch_bounds__(NW * 64) void group_kernel(GemmArgs a) {
     if (g == 0) ssq[wave][16 * t + m] = part;
   }
   __syncthreads();
+  if (j1 - j0 < SP) {  // (uniform) what stands in for k-steps past the share: an infinite weight times zero would be a NaN
+#pragma unroll
+    for (int c = 0; c < SP; ++c)
+      if (j0 + c >= j1)
+#pragma unroll
+        for (int u = 0; u < S; ++u) wv[c][u] = make_uint4(0, 0, 0, 0);
+  }
   f32x4 acc[S][BT];
 #pragma unroll
   for (int t = 0; t < BT; ++t) {

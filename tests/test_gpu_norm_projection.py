@@ -81,3 +81,20 @@ def test_shares_of_three_and_six_steps(cuda, rows, n, k):
     w = (torch.randn(n, k, generator=g, device=cuda) * 0.05).to(BF)
     packed = ops.pack_linear(w)
     _check(ops.gemm_skinny(x, packed, nw, 1e-5), x, w, nw, 1e-5, ops.gemm_skinny(ops.rmsnorm(x, nw, 1e-5), packed))
+
+
+@pytest.mark.parametrize("n,k", SHAPES + [(4112, 576), (8200, 1352), (2304, 520)])
+@pytest.mark.parametrize("rows", [1, 17, 40])
+def test_infinite_weights_of_the_last_columns(cuda, rows, n, k):
+    """Waves whose share of K ends early, or that have none: an infinite weight makes its own column infinite and no NaN."""
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(8)
+    x = torch.rand(rows, k, generator=g, device=cuda).add_(0.5).to(BF)
+    nw = torch.ones(k, device=cuda, dtype=BF)
+    w = torch.randn(n, k, generator=g, device=cuda).to(BF)
+    w[3, k - 1], w[n - 2, k - 8] = float("inf"), -float("inf")
+    got = ops.gemm_skinny(x, ops.pack_linear(w), nw, 1e-5)
+    assert (got[:, 3] == float("inf")).all() and (got[:, n - 2] == -float("inf")).all()
+    rest = [c for c in range(n) if c not in (3, n - 2)]
+    assert got[:, rest].isfinite().all()
