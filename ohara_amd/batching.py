@@ -92,7 +92,7 @@ class ContinuousBatcher:
 
     def _prefill_group(self, slots: list[int], prompts: list) -> list[torch.Tensor]:
         if sum(len(p) for p in prompts) > 64:
-            return list(self.model.prompts(prompts, self.cache, slots).unsqueeze(1))
+            return list(self.model._prompts(prompts, self.cache, slots).unsqueeze(1))
         return [self.model.forward(p.view(1, -1).to(self.model.device), [c._row_view(b) for c in self.cache], 0, last_only=True)[0]
                 for b, p in zip(slots, prompts)]
 

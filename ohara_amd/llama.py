@@ -446,7 +446,13 @@ class Llama:
             raise ValueError("prompts hold more than 64 tokens together, each at least one and at most max_sequence_length")
         if len(set(slots)) != len(prompts) or min(slots) < 0 or max(slots) >= min(c.capacity for c in kv_cache):
             raise ValueError("slots must be distinct rows of the cache")
-        n = len(prompts)
+        _check_ids_on_host(torch.cat(prompts), self.config.vocab_size)
+        return self._prompts(prompts, kv_cache, slots)
+
+    def _prompts(self, prompts: list, kv_cache: list, slots: list[int]) -> torch.Tensor:
+        """``prompts`` without its checks; an id outside the vocabulary counts as 0, as in every call whose ids are on the device."""
+        lens = [len(p) for p in prompts]
+        n, rows = len(prompts), sum(lens)
         buf = self._get_buffers(n, rows)
         length, slot = torch.tensor(lens, dtype=torch.int32), torch.tensor(slots, dtype=torch.int32)
         first = length.cumsum(0, dtype=torch.int32) - length

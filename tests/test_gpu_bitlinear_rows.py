@@ -67,3 +67,25 @@ def test_query_key_value_with_rotary_and_append(cuda, batch, seq, h, h_kv, dh):
     want, kk, vv = (ops.bitlinear(x, nw, w, 1e-5, pre_norm_w=pre) for nw, w in projs)
     ops.rope_append(want, kk, vv, batch, seq, h, h_kv, dh, cos, sin, pos, kr, vr)
     assert torch.equal(got, want) and torch.equal(kc, kr) and torch.equal(vc, vr)
+
+
+@pytest.mark.parametrize("width,batch,seq", [(6, 1, 70), (10, 3, 40), (12, 2, 65)])
+def test_prompt_of_a_model_whose_heads_are_not_in_fours(cuda, width, batch, seq):
+    """More than 64 rows take any even head width: the tiled launch those in fours, three BitLinears and the rotary launch the others."""
+    from ohara_amd.bitnet import BitLlama
+    from ohara_amd.llama import Config
+    from oracle import bitlinear_ref as BL
+    from oracle import llama_ref as R
+
+    kw = dict(vocab_size=96, hidden_size=8 * width, intermediate_size=136, num_attention_heads=8, num_key_value_heads=4,
+              num_hidden_layers=2, max_sequence_length=80, rope_theta=10000.0)
+    rcfg = R.RefConfig(**kw)
+    w = BL.init_ternary_weights(rcfg, seed=3, dtype=BF, gamma=0.05)
+    ref, model = R.RefLlama(rcfg, w), BitLlama(Config(**kw), w, device=cuda)
+    ids = torch.randint(0, 96, (batch, seq), generator=torch.Generator().manual_seed(seq))
+    rc, cache = ref.build_kv_cache(batch), model.build_kv_cache(batch)
+    want, got = ref(ids, rc, 0).float(), model(ids.to(cuda), cache, 0).float().cpu()
+    # an int8 code that rounds the other way moves its whole row: the bounds of the small ternary models
+    scale, d = want.abs().max().item(), (got - want).abs()
+    assert d.max().item() <= 8e-2 * scale and d.mean().item() <= 1e-2 * scale
+    assert (cache[0].key[:, seq:] == 0).all() and (cache[0].key[:, :seq].float().abs().amax((2, 3)) > 0).all()

@@ -65,6 +65,24 @@ def test_what_is_refused(cuda):
     assert not m.takes_prompts(m.build_kv_cache(2, int8=True))
 
 
+@pytest.mark.parametrize("bad", [-1, 640])
+def test_ids_outside_the_vocabulary(cuda, bad):
+    m = _model(cuda, 4, 2, 512)
+    cache, prompts = m.build_kv_cache(2), _ids([60, 9])
+    prompts[1][4] = bad
+    with pytest.raises(IndexError):
+        m.prompts(prompts, cache, [0, 1])
+    assert all((c.key == 0).all() for c in cache)
+    from ohara_amd.batching import ContinuousBatcher
+
+    # a batcher takes it as 0, one prompt or several
+    together, apart, zero = (ContinuousBatcher(m, 2) for _ in range(3))
+    first = together.add_many(prompts)
+    assert first == [apart.add(p) for p in prompts]
+    prompts[1][4] = 0
+    assert first == zero.add_many(prompts)
+
+
 @pytest.mark.parametrize("int8", [False, True])
 @pytest.mark.parametrize("most", [100, 16384])
 def test_batcher_joins_many_at_once(cuda, monkeypatch, int8, most):
