@@ -144,6 +144,8 @@ class ContinuousBatcher:
         slots and lengths.  The next ``step`` continues from the last of the ids fed and the token after it is the
         caller's to select."""
         entries = [(b, self._host_ids(ids, 0 if b is None else self.lengths[b])) for b, ids in entries]
+        if not entries:
+            return []
         named = [b for b, _ in entries if b is not None]
         if any(not self.active[b] for b in named) or len(set(named)) != len(named):
             raise ValueError("entries must name distinct active slots")

@@ -99,3 +99,13 @@ def test_batcher_joins_many_at_once(cuda, monkeypatch, int8, most):
     assert [c.lengths for c in together.cache] == [c.lengths for c in apart.cache]
     assert together.steps(5) == apart.steps(5)
     assert together.add_many([]) == []
+
+
+def test_feed_of_nothing(cuda):
+    from ohara_amd.batching import ContinuousBatcher
+
+    b = ContinuousBatcher(_model(cuda, 4, 2, 512), 3)
+    assert b.feed([]) == []
+    slot, tok = b.add(_ids([70])[0])
+    assert b.feed([]) == [] and b.lengths[slot] == 70
+    assert [s for s, _ in b.feed([(slot, [tok])])] == [slot]
