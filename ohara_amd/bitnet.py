@@ -153,6 +153,10 @@ class BitLlama:
                 v = ops.bitlinear(h, L["attn.value"][1], L["attn.value"][0], self.eps, pre_norm_w=L["norm1"])
                 kr, vr = ops.rope_rows(q, k, v, B, S, H, Hkv, D, self.cos, self.sin, start)
                 ops.kv_quant_append(kr, vr, cache, start)
+            elif rows > ops.BIT_ROWS and D % 4:  # the tiled launch stores a head's columns four at a time
+                q, k, v = (ops.bitlinear(h, L[n][1], L[n][0], self.eps, pre_norm_w=L["norm1"])
+                           for n in ("attn.query", "attn.key", "attn.value"))
+                ops.rope_append(q, k, v, B, S, H, Hkv, D, self.cos, self.sin, start, cache.key, cache.value)
             else:  # one launch for q/k/v + rotary + append
                 q = ops.bitlinear_qkv_rope_append(
                     h, L["norm1"], [(L[n][1], L[n][0]) for n in ("attn.query", "attn.key", "attn.value")], self.eps,
