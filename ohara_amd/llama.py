@@ -441,10 +441,14 @@ class Llama:
         caches, which have to be empty there -> the logits (n, V) of the last token of each.  More than 64 tokens
         together.  The books of the caches are the caller's."""
         lens = [len(p) for p in prompts]
-        rows = sum(lens)
-        if rows <= 64 or min(lens) < 1 or max(lens) > self.config.max_sequence_length:
+        if sum(lens) <= 64 or min(lens) < 1 or max(lens) > self.config.max_sequence_length:
             raise ValueError("prompts hold more than 64 tokens together, each at least one and at most max_sequence_length")
-        if len(set(slots)) != len(prompts) or min(slots) < 0 or max(slots) >= min(c.capacity for c in kv_cache):
+        shape = (self.config.max_sequence_length, self.kv_heads, self.head_dim)
+        if len(kv_cache) != self.config.num_hidden_layers or any(tuple(c.key.shape[1:]) != shape for c in kv_cache):
+            raise ValueError("the KV cache must contain one entry per model layer, of the model's own shape")
+        if not self.takes_prompts(kv_cache):
+            raise ValueError("prompts side by side need bfloat16 caches and heads of 64 or 128")
+        if len(slots) != len(prompts) or len(set(slots)) != len(slots) or min(slots) < 0 or max(slots) >= min(c.capacity for c in kv_cache):
             raise ValueError("slots must be distinct rows of the cache")
         _check_ids_on_host(torch.cat(prompts), self.config.vocab_size)
         return self._prompts(prompts, kv_cache, slots)

@@ -62,6 +62,15 @@ def test_what_is_refused(cuda):
     for lens, slots in (([30, 30], [0, 1]), ([100, 0], [0, 1]), ([513, 1], [0, 1]), ([100, 1], [1, 1]), ([100, 1], [0, 3]), ([100], [0, 1])):
         with pytest.raises(ValueError):
             m.prompts(_ids(lens), cache, slots)
+    # (all refused on the host: the launches behind would follow pointers and strides that are not there)
+    short = _model(cuda, 4, 2, 512).build_kv_cache(3)
+    short[1].key, short[1].value = short[1].key[:, :256].contiguous(), short[1].value[:, :256].contiguous()
+    for caches in (cache[:1], cache + cache[:1], [], short, m.build_kv_cache(3, int8=True)):
+        with pytest.raises(ValueError):
+            m.prompts(_ids([70, 9]), caches, [0, 1])
+    with pytest.raises(ValueError):
+        m.prompts(_ids([70, 9]), cache, [0, 1, 1])
+    assert all((c.key == 0).all() for c in cache)
     assert not m.takes_prompts(m.build_kv_cache(2, int8=True))
 
 
