@@ -463,8 +463,10 @@ def act_quant_sets(x, norm_ws, eps, pre_norm_w=None):
 def bitlinear_many(x, pre_norm_w, projs, eps=1e-5):
     """Several BitLinears of one width on the same rows (any number), each row quantised once for each -> their outputs.
     ``projs``: at most three (norm_w, PackedTernary) pairs."""
-    q, s, sq = act_quant_sets(x, [p[0] for p in projs], eps, pre_norm_w)
     n, rows, width = len(projs), x.shape[0], projs[0][1].n
+    if any(w.n != width or w.k != x.shape[1] for _, w in projs):
+        raise ValueError(f"x has {x.shape[1]} columns, weights expect {[w.k for _, w in projs]} and give {[w.n for _, w in projs]}")
+    q, s, sq = act_quant_sets(x, [p[0] for p in projs], eps, pre_norm_w)
     outs = [torch.empty(rows, width, dtype=BF16, device=x.device) for _ in projs]
     wp = (C.c_void_p * n)(*[p[1].data.data_ptr() for p in projs])
     gm = (C.c_float * n)(*[p[1].gamma for p in projs])
@@ -504,6 +506,8 @@ def bitlinear_qkv_rope_append(x, pre_norm_w, projs, eps, h, h_kv, dh, cos, sin, 
     wp = (C.c_void_p * 3)(*[p[1].data.data_ptr() for p in projs])
     gm = (C.c_float * 3)(*[p[1].gamma for p in projs])
     if rows > BIT_ROWS:
+        if any(w.k != k or w.n != heads * dh for (_, w), heads in zip(projs, (h, h_kv, h_kv))):
+            raise ValueError(f"x has {k} columns and heads are {h}, {h_kv} x {dh}, weights expect {[w.k for _, w in projs]} and give {[w.n for _, w in projs]}")
         q, s, sq = act_quant_sets(x, [p[0] for p in projs], eps, pre_norm_w)
         check(lib().ohara_gemm_ternary_qkv_rope_append(
             _ptr(q), q.stride(1), _ptr(s), _ptr(sq), wp, gm, k, rows // seq_len, seq_len, h, h_kv, dh, _ptr(cos), _ptr(sin),

@@ -50,6 +50,21 @@ def test_sets_share_rows_and_keep_their_own_codes(cuda):
     assert torch.equal(two, ops.bitlinear(x, nw2, b, 1e-5, pre_norm_w=pre))
 
 
+def test_weights_of_another_width_are_refused(cuda):
+    """On the host: the launch would read past the weights' end."""
+    from ohara_amd import ops
+
+    x, t, nw, pre, _ = _inputs(cuda, 70, 64, 264, 5)
+    a, narrow, short = (ops.pack_ternary(w.contiguous(), 0.02) for w in (t, t[:32], t[:, :256]))
+    for w in (narrow, short):
+        with pytest.raises(ValueError):
+            ops.bitlinear_many(x, pre, [(nw, a), (nw, w)], 1e-5)
+        kc, vc, cs = torch.zeros(1, 80, 2, 32, dtype=BF, device=cuda), torch.zeros(1, 80, 2, 32, dtype=BF, device=cuda), torch.zeros(80, 16, dtype=BF, device=cuda)
+        with pytest.raises(ValueError):
+            ops.bitlinear_qkv_rope_append(x, pre, [(nw, a), (nw, w), (nw, a)], 1e-5, 2, 2, 32, cs, cs, 0, kc, vc, seq_len=70)
+        assert (kc == 0).all()
+
+
 @pytest.mark.parametrize("batch,seq,h,h_kv,dh", [(1, 70, 2, 2, 64), (3, 50, 4, 2, 128), (2, 129, 2, 1, 8)])
 def test_query_key_value_with_rotary_and_append(cuda, batch, seq, h, h_kv, dh):
     from ohara_amd import ops
