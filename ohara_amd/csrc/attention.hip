@@ -28,8 +28,8 @@ struct AttnArgs {
   const int32_t* pos_dev;            // when set: start = *pos_dev, or pos_dev[sequence] with pos_stride 1
   int pos_stride;
   int nsplit;        // chunks there is room for
-  int most;          // chunks that pay where the walk is what takes the time (0: where the memory is), see cut_context
-  int most_long;     // the same for contexts of more than 4096 positions
+  int one, few, some;         // 64s of positions up to which a context is one chunk, few_chunks or some_chunks, see cut_context
+  int few_chunks, some_chunks;
   int* counters;     // (B*Hkv)
   float* part_ml;    // (B, Hkv, nsplit of room: G, chunks, 2)
   float* part_acc;   // (B, Hkv, nsplit of room: G, chunks, D)
@@ -114,30 +114,17 @@ __device__ void merge_partials(const AttnArgs& a, int b /* query row */, int kvh
 }
 
 // Into how many of the caller's n_split chunks a context of L positions is cut, from what is known only here (L may live on the
-// device): merging costs a launch about 3 us and every chunk 0.1 to 0.2 more, a workgroup walks 64 positions in 0.8, and with more
-// than 128 (row, head) pairs the memory is busy without a cut.  A call's workgroups all come to the same answer; the ones
-// without a chunk leave.  us a launch, 1 / 4 / 8 / 16 chunks, heads of 128 (the caller asks for about 1024 workgroups):
-//   64 pairs, 4 int8 heads each  100 positions 5.2 / 9.1 / 9.4 / 12.4;  300  9.4 / 10.0 / 10.2 / 13.0;  700  15.2 / 12.3 / 11.9 / 14.8;
-//                                1900  29.7 / 16.7 / 16.4 / 19.1;  4000  55 / 23.9 / 24.3 / 25.7
-//   64 pairs, 4 heads            700  16.0 / 12.3 / 13.8 / 16.1;  1900  34.9 / 18.3 / 20.3 / 22.2;  4000  68 / 28.8 / 31.0 / 33.0
-//   96 pairs (1 / 5 / 8 / 10)    100  4.9 / 7.0 / 7.5 / 8.2;  300  8.3 / 8.5 / 8.9 / 9.5;  530  12.0 / 10.7 / 10.8 / 11.3;
-//                                1500  27.6 / 17.6 / 17.0 / 17.5;  4000  65 / 37.4 / 36.3 / 39.8
-//   192 pairs (1 / 4 / 5)        100  5.0 / 7.8 / 7.8;  530  13.2 / 16.0 / 14.3;  700  16.4 / 17.4 / 17.7;  1500  30.5 / 28.7 / 29.4
-//   12 pairs (1 / 8 / 16 / 32)   300  6.6 / 6.8 / 7.3 / 9.8;  700  12.5 / 7.9 / 8.1 / 9.8;  4000  56 / 14.3 / 11.7 / 12.7
-// 81 to 128 pairs, where the room is 8 to 11 chunks; chunks: us a launch, 768 / 1536 / 4096 / 16384 positions:
-//   heads of 128, 1 head each   96 pairs   5: 13.6 19.0 39.2 133   8: 13.7 18.2 37.8 128   10: 13.9 18.6 40.2 134;  int8 5: 13.6 17.6 29.8 85.6
-//                                          8: 10.8 16.6 27.4 80.9;  88 pairs, int8  5: 12.9 19.1 31.7 96.9   8: 10.6 16.1 28.2 87.1   11: 11.5 16.2 25.5 75.3
-//   heads of 128, 4 heads each  128 pairs  4: 17.8 25.8 54.3 193   8: 19.8 28.1 56.1 185;  int8 4: 17.3 22.2 41.8 129   8: 17.3 22.5 41.7 122
-//   heads of 64                 128 pairs, 4 heads each  4: 12.6 17.7 34.3 112   8: 13.2 18.4 34.9 113;  96 pairs, 8192 / 32768  8: 41.0 141   10: 42.7 150
-// so: one head each, eight; several, two workgroups a CU; with heads of 128 the room's four a CU from 4096 positions on.
+// device): merging costs a launch about 3 us and every chunk 0.1 more, a workgroup alone on a CU walks 64 positions in 0.5 to 1.2, and several
+// on one hide each other's waits until the memory is busy.  So with its length a context takes one chunk, chunks that
+// make one workgroup a CU of the launch, two, and all there is room for (which callers make four); chunks of 64 positions alone pay
+// nowhere.  CutRule, below, says up to which lengths.  A call's workgroups all come to the same answer; the ones without a chunk leave.
 struct Cut {
   int chunk, used;
 };
 __device__ __forceinline__ Cut cut_context(const AttnArgs& a, int L, int unit /* positions of a workgroup's step */) {
   const int n64 = (L + 63) >> 6;
-  int want = a.nsplit;
-  if (n64 <= 5 || (a.most == 0 && n64 <= 12)) want = 1;
-  else if (a.most) want = min(want, min((n64 + 1) >> 1, n64 > 64 ? a.most_long : a.most));
+  int want = n64 <= a.one ? 1 : n64 <= a.few ? a.few_chunks : n64 <= a.some ? a.some_chunks : a.nsplit;
+  want = max(min(want, min(a.nsplit, (n64 + 1) >> 1)), 1);
   const int chunk = max((L + want - 1) / want + unit - 1, unit) & ~(unit - 1);
   return {chunk, max((L + chunk - 1) / chunk, 1)};
 }
@@ -941,6 +928,52 @@ int launch_fast(const AttnArgs& a, int G, dim3 grid, hipStream_t st) {
   return 0;
 }
 
+// Up to how many 64s of positions a context is one chunk / chunks for one workgroup a CU / for two (cut_context), by kernel and number of
+// (row, key head) pairs.  Fitted to launches from a graph over caches out of HBM: 4 to 512 pairs, 320 to 32768 positions, 1, 2 and 4 heads a
+// pair, 28700 shapes, on average 0.9 % behind the best cut of each.  Some of them, chunks: us
+//   bf16, heads of 128, 1 each  12 pairs 1024  1: 16.5  8: 8.6  16: 9.1;  72 pairs 1536  1: 28.5  3: 16.6  6: 16.6  12: 16.5,
+//                               16384  1: 268  3: 113  7: 106  14: 103
+//                       4 each  64 pairs 4096  1: 70  4: 29.3  8: 31.1  16: 33.9;  80 pairs 16384  1: 272  3: 118  6: 117  12: 120
+//   int8, heads of 128, 1 each  72 pairs 768  1: 14.1  3: 11.3  6: 10.1,  16384  1: 191  3: 77  7: 69  13: 63;  144 pairs 640  1: 13.0  3: 13.1  5: 11.3
+//                       4 each  80 pairs 4096  1: 61  3: 31.7  6: 30.2  11: 30.5
+//   bf16, heads of 64, 1 each   40 pairs 16384  1: 171  6: 40.0  12: 36.2  24: 33.2;  56 pairs 16384  1: 172  4: 55.0  9: 46.7  18: 44.0
+//                       4 each  68 pairs 32768  1: 355  3: 135  7: 97  15: 97
+//   int8, heads of 64, 1 each   64 pairs 448  1: 7.2  4: 8.0;  192 pairs 960  1: 11.0  2: 12.8  4: 12.0
+// (Never more than one workgroup a CU up to 80 pairs, and one chunk up to 768 positions past 128, cost up to 40 % at 17 to 80 pairs over long
+// contexts and up to 17 % at 129 to 175.)
+struct CutRule {
+  short one, few, some;
+};
+constexpr int CUT_PAIRS[] = {16, 25, 32, 42, 51, 64, 73, 85, 102, 128, 146, 170, 204, 256, 341}, CUT_BANDS = 16;  // (where quotients change)
+constexpr short ANY = 32767;
+constexpr CutRule CUTS[8][CUT_BANDS] = {
+    // bf16, 128 wide: one head a pair, several
+    {{5, ANY, ANY}, {5, 192, ANY}, {5, 128, ANY}, {5, 96, 96}, {5, 32, ANY}, {5, 20, 128}, {5, 9, 48}, {5, 32, 96},
+     {6, 6, 6}, {6, 6, 6}, {8, 8, 8}, {8, 8, 9}, {12, 12, 12}, {48, 48, 48}, {7, 7, 7}, {8, 8, 8}},
+    {{5, ANY, ANY}, {5, ANY, ANY}, {5, ANY, ANY}, {5, ANY, ANY}, {5, 192, ANY}, {5, 256, 256}, {5, 64, 192}, {5, 192, 192},
+     {6, 16, 64}, {7, 48, 64}, {12, 12, 24}, {12, 12, 48}, {24, 24, 24}, {96, 96, 96}, {10, 10, 10}, {16, 16, 16}},
+    // int8, 128 wide: one head a pair, several
+    {{5, ANY, ANY}, {5, 256, ANY}, {5, 256, ANY}, {5, 5, 5}, {5, 5, 5}, {5, 5, 5}, {5, 5, 5}, {5, 5, 5},
+     {5, 5, 5}, {6, 6, 6}, {6, 6, 6}, {6, 6, 6}, {16, 16, 16}, {48, 48, 48}, {5, 5, 5}, {24, 24, 24}},
+    {{5, ANY, ANY}, {5, 192, ANY}, {5, 48, ANY}, {5, 96, ANY}, {5, 64, ANY}, {5, 24, 256}, {5, 5, 256}, {5, 5, 192},
+     {6, 6, 24}, {6, 6, 96}, {10, 10, 12}, {10, 10, 12}, {14, 14, 14}, {48, 48, 48}, {8, 8, 8}, {32, 32, 32}},
+    // bf16, 64 wide: one or two heads a pair, more
+    {{6, ANY, ANY}, {7, 256, ANY}, {7, ANY, ANY}, {7, 48, 192}, {7, 32, ANY}, {7, 20, 128}, {9, 14, ANY}, {8, 14, 96},
+     {9, 9, 20}, {9, 9, 20}, {10, 10, 10}, {10, 10, 14}, {12, 12, 12}, {32, 32, 32}, {14, 14, 14}, {32, 32, 32}},
+    {{5, ANY, ANY}, {6, 96, ANY}, {6, 48, ANY}, {6, 32, 256}, {6, 24, ANY}, {6, 24, ANY}, {7, 14, ANY}, {7, 20, ANY},
+     {8, 8, 96}, {8, 14, 192}, {10, 10, 24}, {10, 10, 96}, {16, 16, 20}, {24, 24, 48}, {20, 20, 20}, {64, 64, 64}},
+    // int8, 64 wide: one or two heads a pair, more
+    {{6, ANY, ANY}, {8, 192, ANY}, {8, ANY, ANY}, {8, 128, ANY}, {8, 128, ANY}, {10, ANY, ANY}, {12, 16, 256}, {12, 256, ANY},
+     {14, 16, 24}, {14, 24, 128}, {24, 24, 24}, {32, 32, ANY}, {32, 32, 32}, {ANY, ANY, ANY}, {12, 12, 12}, {16, 16, 16}},
+    {{5, ANY, ANY}, {5, 256, ANY}, {5, ANY, ANY}, {5, 128, ANY}, {5, 64, 256}, {5, 96, ANY}, {5, 32, 192}, {8, 128, ANY},
+     {8, 8, 8}, {10, 32, 128}, {16, 16, 16}, {20, 20, ANY}, {24, 24, 24}, {ANY, ANY, ANY}, {14, 14, 14}, {24, 24, 24}},
+};
+const CutRule& cut_rule(bool i8, int dh, int heads, int64_t pairs) {
+  int band = 0;
+  while (band < CUT_BANDS - 1 && pairs > CUT_PAIRS[band]) ++band;
+  return CUTS[(dh == 128 ? heads > 1 : 4 + (heads > 2)) + 2 * i8][band];
+}
+
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 }  // namespace
@@ -978,11 +1011,10 @@ static int attn_cached_impl(const uint16_t* q, const void* kcache, const void* v
   a.nsplit = n_split;
   batch *= seq_len;  // one workspace slot per query row
   const int64_t pairs = (int64_t)batch * h_kv;
-  a.most = a.most_long = pairs <= 80 ? (int)(256 / pairs) : 0;  // one workgroup a CU
-  if (pairs > 80 && pairs <= 128) {
-    a.most = (int)(h == h_kv ? std::min<int64_t>(8, 1024 / pairs) : 512 / pairs);
-    a.most_long = dh == 128 ? (int)(1024 / pairs) : a.most;
-  }
+  const CutRule& cut = cut_rule(i8, dh, h / h_kv, pairs);
+  a.one = cut.one; a.few = cut.few; a.some = cut.some;
+  a.few_chunks = (int)std::max<int64_t>(256 / pairs, 1);
+  a.some_chunks = (int)std::max<int64_t>(512 / pairs, 1);
   char* ws = reinterpret_cast<char*>(workspace);
   a.counters = reinterpret_cast<int*>(ws);
   ws += fixed_counter_bytes ? fixed_counter_bytes : align256((size_t)batch * h_kv * sizeof(int));

@@ -77,3 +77,29 @@ def test_lengths_around_4096(cuda, B, H, Hkv, D):
         for ns, ws in rooms.items():
             got = ops.attn_cached(q, k, v, H, Hkv, D, L - 1, ns, ws)
             assert ((got.view(B, H, D).double() - want).abs() <= bound).all()
+
+
+# a number of pairs of every kind of line (one workgroup a CU, two, all there is room for), the room that callers ask for
+@pytest.mark.parametrize("B,H,Hkv", [(4, 24, 6), (6, 8, 8), (9, 16, 8), (25, 4, 4), (25, 32, 8), (50, 6, 6)])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("int8", [False, True])
+def test_longer_contexts(cuda, B, H, Hkv, D, int8):
+    from ohara_amd import ops
+    from ohara_amd.llama import KVCache
+
+    T, ns = 3300, 1024 // (B * Hkv)
+    g = torch.Generator(device=cuda).manual_seed(B + H + D)
+    q = torch.randn(B, H * D, generator=g, device=cuda).to(BF)
+    k, v = (torch.randn(B, T, Hkv, D, generator=g, device=cuda).to(BF) for _ in range(2))
+    ws, one = (ops.attn_workspace(B, H, Hkv, D, n, cuda) for n in (ns, 1))
+    if int8:
+        cache = KVCache((B, T, Hkv, D), T, 0, device=cuda, dtype=BF, int8=True)
+        ops.kv_quant_append(k, v, cache, 0)
+    for L in (321, 449, 640, 1025, 1536, 3201):
+        if int8:
+            got, whole = (ops.attn_cached_int8(q, cache, H, Hkv, D, L - 1, n, w).float() for n, w in ((ns, ws), (1, one)))
+            # another order of fp32 sums: a value may round to its neighbour, 2^-7 of it at most
+            assert ((got - whole).abs() <= whole.abs() * 2.0 ** -7 + 2.0 ** -16).all()
+        else:
+            want, bound = _exact(q.view(B, H, D), k, v, [L] * B)
+            assert ((ops.attn_cached(q, k, v, H, Hkv, D, L - 1, ns, ws).view(B, H, D).double() - want).abs() <= bound).all()
