@@ -651,11 +651,15 @@ int launch_once_as(const GemmArgs& a, hipStream_t st) {
 template <int EPI, int H>
 int launch_once_h(const GemmArgs& a, hipStream_t st) {
   const int KS = (a.K + 31) >> 5;
+  if constexpr (H == 1) {  // (half strips start past K 1024)
+    switch ((KS + 7) / 8 * 2) {
+      case 2: return launch_once_as<EPI, H, 4, 2>(a, st);
+      case 4: return launch_once_as<EPI, H, 4, 4>(a, st);
+      case 6: return launch_once_as<EPI, H, 4, 6>(a, st);
+      case 8: return launch_once_as<EPI, H, 4, 8>(a, st);
+    }
+  }
   if (KS <= 96) switch ((KS + 7) / 8 * 2) {  // four waves' shares, even
-    case 2: return launch_once_as<EPI, H, 4, 2>(a, st);
-    case 4: return launch_once_as<EPI, H, 4, 4>(a, st);
-    case 6: return launch_once_as<EPI, H, 4, 6>(a, st);
-    case 8: return launch_once_as<EPI, H, 4, 8>(a, st);
     case 10: return launch_once_as<EPI, H, 4, 10>(a, st);
     case 12: return launch_once_as<EPI, H, 4, 12>(a, st);
     case 14: return launch_once_as<EPI, H, 4, 14>(a, st);
