@@ -1295,29 +1295,25 @@ __device__ __forceinline__ float key16_value(uint32_t key) {  // the bf16 value 
   return __uint_as_float(bits << 16);
 }
 
-// max of a, max of b and sum of c over the workgroup in one exchange (two barriers instead of six)
-__device__ __forceinline__ void block_max_max_sum_i(int& a, int& b, int& c, Smem& s) {
+// max of a and max of b over the workgroup in one exchange (two barriers instead of four)
+__device__ __forceinline__ void block_max_max_i(int& a, int& b, Smem& s) {
   a = lanes_max<32, 1>(a);
   b = lanes_max<32, 1>(b);
-  c = lanes_sum<32, 1>(c);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   __syncthreads();
   if (lane == 0) {
     s.wredi[w] = a;
     s.hist[w] = b;
-    s.hist[NW + w] = c;
   }
   __syncthreads();
-  int ra = s.wredi[0], rb = s.hist[0], rc = s.hist[NW];
+  int ra = s.wredi[0], rb = s.hist[0];
 #pragma unroll
   for (int i = 1; i < NW; ++i) {
     ra = max(ra, s.wredi[i]);
     rb = max(rb, s.hist[i]);
-    rc += s.hist[NW + i];
   }
   a = ra;
   b = rb;
-  c = rc;
 }
 
 template <int EPT>
@@ -1329,7 +1325,6 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
   const int base = tid * EPT;
   const float temp = a.temperature;
   const float u = a.u[(a.step_state && a.u_step_stride > 0 ? (size_t)a.step_state[1] * a.u_step_stride : 0) + b];
-  const bf16_t* row = reinterpret_cast<const bf16_t*>(a.logits) + (size_t)b * a.ldl + base;
   // One CU walks the whole row, so every instruction per id costs about half a microsecond: the two bf16 patterns of a
   // register become order-preserving 16-bit keys with four integer instructions.  fn(id, key) is called for the valid ids among
   // 8 id0 ..; key 0 cannot occur for a number (it is the pattern of one NaN) and is skipped.
@@ -1402,8 +1397,8 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
         }
     }
   }
-  int kmax = max((int)hi2[0], (int)hi2[1]), nkmin = -min((int)lo2[0], (int)lo2[1]), unused = 0;
-  block_max_max_sum_i(kmax, nkmin, unused, s);  // (the barriers inside also complete the table)
+  int kmax = max((int)hi2[0], (int)hi2[1]), nkmin = -min((int)lo2[0], (int)lo2[1]);
+  block_max_max_i(kmax, nkmin, s);  // (the barriers inside also complete the table)
   const int kmin = -nkmin;
   const int n_live = nvalid - (want_table ? (int)(hist[0] & 0xffffu) : 0);  // (asked for with the table only)
   int token = 0;
