@@ -87,12 +87,14 @@ int ohara_gemm_skinny_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n
 int ohara_swiglu_perm(int f, int32_t* perm_host);
 
 /* ---- tiled MFMA GEMM (batched prefill projections) ---------------------------
- * out = epi(x @ W^T) for any number of rows: 128 x 128 output tiles, K in steps of 64,
- * activations staged through LDS, packed weights streamed straight into the MFMA A operand.
+ * out = epi(x @ W^T) for any number of rows: output tiles of 32 x 32 to 256 x 256, the one that a model of the times
+ * says is fastest, K in steps of 64 or 128, activations and packed weights both straight into LDS.
  * Same packed `wp`, same epilogues and the same rounding points as ohara_gemm_skinny_bf16
  * (llama.py:84-86,142,322, mlp.py:152 with more than one position per call).  No fused norm. */
 int ohara_gemm_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, int rows, int epilogue,
                     const uint16_t* resid, int ldr, uint16_t* out, int ldo, void* stream);
+/* The tile of such a product over rows that start on 16 bytes: 1000 * its rows + its packed rows (SwiGLU packs two a column). */
+int ohara_gemm_tile_of(int rows, int packed_rows, int k);
 
 /* Fused q/k/v projection + rotary + KV-cache append: replaces Attention.forward's
  * three Linears, apply_rope and KVCache.forward (llama.py:84-98;
@@ -596,8 +598,8 @@ int ohara_bitnet_decode_persistent(const OharaBitModel* m, const OharaDecodeStat
                                    int init_workspace, int select_greedy, unsigned int spin_limit, void* stream);
 
 /* ---- Phi (ohara/models/phi.py): the parts of its cached decode path that differ from Llama ----
- * nn.Linear WITH bias on packed weights (phi.py:46-47, :63-66, :161), any number of rows (up to 128:
- * the weight-streaming strip kernel, 64 rows per pass; more: the tiled MFMA kernel of ohara_gemm_bf16,
+ * nn.Linear WITH bias on packed weights (phi.py:46-47, :63-66, :161), any number of rows (up to 64:
+ * the weight-streaming strip kernel; more: the tiled MFMA kernel of ohara_gemm_bf16,
  * same epilogues and rounding points).  n % 4 == 0, k % 8 == 0.
  *   OHARA_LIN_BIAS       out = bf16(x @ W^T + bias)
  *   OHARA_LIN_BIAS_GELU  out = new_gelu(bf16(x @ W^T + bias)), every op of phi.py:37-40 rounded to

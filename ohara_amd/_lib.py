@@ -111,6 +111,7 @@ _PROTOS = {
     "ohara_embed_bf16": (_i, [_p, _p, _p, _i, _i, _i, _p]),
     "ohara_rmsnorm_bf16": (_i, [_p, _p, _p, _i, _i, _f, _p]),
     "ohara_gemm_skinny_bf16": (_i, [_p, _i, _p, _i, _i, _p, _f, _i, _i, _p, _i, _p, _i, _p]),
+    "ohara_gemm_tile_of": (_i, [_i, _i, _i]),
     "ohara_gemm_bf16": (_i, [_p, _i, _p, _i, _i, _i, _i, _p, _i, _p, _i, _p]),
     "ohara_qkv_rope_append_bf16": (_i, [_p, _i, _p, _i, _p, _f, _i, _i, _i, _i, _i, _p, _p, _i, _p, _p, _p, _p, _i, _p]),
     "ohara_qkv_rope_bf16": (_i, [_p, _i, _p, _i, _p, _f, _i, _i, _i, _i, _i, _p, _p, _i, _p, _i, _p, _p, _p, _p]),

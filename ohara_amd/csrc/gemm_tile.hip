@@ -289,19 +289,23 @@ float tile_time(const TileTime& t, int rows, int strips, int K) {
   return step * K * (1.f / 64.f) + t.ends * (tiles > CUS ? tiles * (1.f / CUS) : 1.f);
 }
 
-template <int EPI>
-int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
-  if (((uintptr_t)a.x & 15) != 0 || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return launch_tile<EPI, T64, false>(a, nstrips, st);
+int fastest_tile(int rows, int strips, int K) {
   int best = 0;
-  float low = tile_time(TIMES[0], a.B, nstrips, a.K);
+  float low = tile_time(TIMES[0], rows, strips, K);
   for (int i = 1; i < 6; ++i) {
-    const float t = tile_time(TIMES[i], a.B, nstrips, a.K);
+    const float t = tile_time(TIMES[i], rows, strips, K);
     if (t < low) {
       low = t;
       best = i;
     }
   }
-  switch (best) {
+  return best;
+}
+
+template <int EPI>
+int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
+  if (((uintptr_t)a.x & 15) != 0 || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return launch_tile<EPI, T64, false>(a, nstrips, st);
+  switch (fastest_tile(a.B, nstrips, a.K)) {
     case 0: return launch_tile<EPI, T32>(a, nstrips, st);
     case 1: return launch_tile<EPI, T64>(a, nstrips, st);
     case 2: return launch_tile<EPI, T64x128>(a, nstrips, st);
@@ -331,6 +335,12 @@ int ohara_launch_gemm_tile(const GemmArgs& a, int epi, int packed_rows, hipStrea
     case EPI_GLU: return launch_epi<EPI_GLU>(a, nstrips, st);
     default: return OHARA_EINVAL;
   }
+}
+
+extern "C" int ohara_gemm_tile_of(int rows, int packed_rows, int k) {
+  if (rows < 1 || packed_rows < 1 || k < 1) return OHARA_EINVAL;
+  const TileTime& t = TIMES[fastest_tile(rows, (packed_rows + 15) / 16, k)];
+  return t.rows * 1000 + t.strips * 16;
 }
 
 extern "C" int ohara_gemm_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, int rows, int epilogue,

@@ -13,15 +13,80 @@ def _bound(x, w, y):
     return y.abs() * 2.0 ** -8 + x.shape[1] * 2.0 ** -24 * (x.abs() @ w.abs().t()) + 1e-30
 
 
-# (rows, columns, K): the comment names the tile that the rule picks
+# (rows, columns, K), edges of K and of strips among them (TILES below names tiles, and asserts that it runs them)
 SHAPES = [
-    (65, 16, 8), (97, 40, 72), (320, 768, 768), (129, 1000, 520), (257, 2048, 2056),  # 32 x 32; K below, at and past a step
-    (96, 6144, 768), (700, 1504, 1000), (193, 4100, 768),                             # 64 x 64
-    (320, 6144, 712),                                                                 # 64 x 128
-    (1000, 3096, 2008), (1030, 6104, 264),                                            # 128 x 128
-    (2049, 2304, 768), (700, 6160, 776), (2100, 11264, 520),                          # 128 x 192
-    (700, 17928, 1032),                                                               # 256 x 256
+    (65, 16, 8), (97, 40, 72), (320, 768, 768), (129, 1000, 520), (257, 2048, 2056), (96, 6144, 768),
+    (700, 1504, 1000), (193, 4100, 768), (320, 6144, 712),
+    (1000, 3096, 2008), (1030, 6104, 264), (2100, 11264, 520),
+    (2049, 2304, 768), (700, 6160, 776),
+    (700, 17928, 1032),
 ]
+
+# tile (rows, packed rows): (rows, packed rows, K) of products that run it, none of them whole tiles; K ends inside a step and with one
+TILES = {
+    (32, 32): [(97, 272, 136), (70, 272, 128)],
+    (64, 64): [(193, 2320, 136), (97, 4112, 128)],
+    (64, 128): [(130, 11280, 136), (450, 4112, 128), (450, 4112, 768)],
+    (128, 128): [(321, 6160, 136), (193, 11280, 64), (321, 6160, 128)],
+    (128, 192): [(700, 6160, 520), (1300, 3088, 768)],
+    (256, 256): [(1025, 11280, 520), (700, 17936, 1032), (1025, 11280, 768)],
+}
+
+
+@pytest.mark.parametrize("tile,rows,packed,k", [(t, *s) for t, shapes in TILES.items() for s in shapes])
+def test_every_tile_gives_the_same_bits(cuda, tile, rows, packed, k):
+    """The sums do not depend on the tile: all epilogues, stored 16 bytes a lane and less, against the same rows in calls of 32 to 96 that run
+    small tiles, and the plain product against 64 bits."""
+    from ohara_amd import ops
+    from ohara_amd._lib import check, lib
+
+    of = lib().ohara_gemm_tile_of
+    assert of(rows, packed, k) == 1000 * tile[0] + tile[1]
+    step = 32 if tile == (64, 64) else 96
+    assert tile == (32, 32) or of(step, packed, k) != 1000 * tile[0] + tile[1]
+    g = torch.Generator(device=cuda).manual_seed(rows + packed + k)
+    x = (torch.randn(rows, k, generator=g, device=cuda) * 3).to(BF)
+    w = (torch.randn(packed, k, generator=g, device=cuda) * 0.3).to(BF)
+    spans = [slice(r, min(r + step, rows)) for r in range(0, rows, step)]
+    for n in (packed, packed - 8, packed - 5):
+        wp, res = ops.pack_linear(w[:n].contiguous()), torch.randn(rows, n, generator=g, device=cuda).to(BF)
+        got, summed = ops.gemm(x, wp), ops.gemm(x, wp, residual=res)
+        assert torch.equal(got, torch.cat([ops.gemm(x[s], wp) for s in spans]))
+        assert torch.equal(summed, torch.cat([ops.gemm(x[s], wp, residual=res[s]) for s in spans]))
+        if n == packed - 5:
+            want = x.double() @ w[:n].double().t()
+            assert ((got.double() - want).abs() <= _bound(x.double(), w[:n].double(), want)).all()
+        wide = torch.full((rows, n + 4), 7.0, dtype=BF, device=cuda)
+        assert torch.equal(ops.gemm(x, wp, out=wide[:, :n]), got) and (wide[:, n:] == 7.0).all()
+    for f in (packed // 2, packed // 2 - 3):
+        gates = ops.pack_gate_up(w[:f].contiguous(), w[f:2 * f].contiguous())
+        got = ops.gemm(x, gates)
+        assert torch.equal(got, torch.cat([ops.gemm(x[s], gates) for s in spans]))
+        wide = torch.full((rows, f + 4), 7.0, dtype=BF, device=cuda)
+        assert torch.equal(ops.gemm(x, gates, out=wide[:, :f]), got) and (wide[:, f:] == 7.0).all()
+    # rotary: heads of 16, an odd number of query heads; positions in a row, and given row by row
+    H, D, T = packed // 16 - 2, 16, rows + 8
+    ang = torch.rand(T, D // 2, generator=g, device=cuda) * 6.28
+    cos, sin = ang.cos().to(BF), ang.sin().to(BF)
+    wq = ops.pack_qkv(w[:H * D], w[H * D:H * D + D], w[H * D + D:])
+    keys, values = (torch.full((4, T, 1, D), 9.0, dtype=BF, device=cuda) for _ in range(2))
+    q = ops.qkv_rope_append(x, wq, None, 1e-5, H, 1, D, cos, sin, 3, keys[:1], values[:1], seq_len=rows)
+    assert (keys[0, 3:3 + rows] != 9.0).any(-1).all() and (keys[0, :3] == 9.0).all() and (keys[0, 3 + rows:] == 9.0).all()
+    by_row = torch.empty_like(q)
+
+    def row_by_row(s, row):  # (always in tiles, also up to 64 rows)
+        n = s.stop - s.start
+        at = torch.cat([torch.arange(3 + s.start, 3 + s.stop), torch.full((n,), row)]).to(cuda, torch.int32)
+        check(lib().ohara_qkv_rope_append_rows_bf16(x[s].data_ptr(), k, wq.data.data_ptr(), k, n, H, 1, D, cos.data_ptr(), sin.data_ptr(),
+                                                    at.data_ptr(), by_row[s].data_ptr(), keys.data_ptr(), values.data_ptr(), T,
+                                                    torch.cuda.current_stream().cuda_stream), "rows")
+
+    for row, parts in ((1, [slice(0, rows)]), (3, spans)):
+        by_row.zero_()
+        for s in parts:
+            row_by_row(s, row)
+        assert torch.equal(by_row, q) and torch.equal(keys[row], keys[0]) and torch.equal(values[row], values[0])
+    assert (keys[2] == 9.0).all() and (values[2] == 9.0).all()
 
 
 @pytest.mark.parametrize("rows,n,k", SHAPES)
@@ -87,7 +152,7 @@ def test_infinite_weights_of_a_last_step(cuda, rows, n, k):
     assert got[:, rest].isfinite().all()
 
 
-# 96 rows take tiles that are 32 rows high, 4100 tiles of 192 columns, 9000 tiles of 256
+# 32 x 32 tiles, 64 x 64, then 128 x 128 (K is short)
 @pytest.mark.parametrize("rows,f", [(96, 264), (300, 3072), (1100, 1544), (2100, 5632), (4100, 1160), (9000, 3080)])
 @pytest.mark.parametrize("pad", [0, 1, 4])
 def test_stores_of_16_bytes_and_less(cuda, rows, f, pad):

@@ -35,6 +35,7 @@ def test_sort_of_many_pairs_is_stable(cuda, pairs, experts):
     ([3, 0, 1, 9], 72, 24, 1), ([64, 0, 1, 33, 100, 66], 136, 40, 2), ([65, 64, 0, 130, 255, 1, 200, 69], 264, 88, 4),
     ([20, 64, 65, 0, 1], 520, 264, 2),
     ([500, 0, 129, 128, 1, 400], 1024, 512, 1), ([256, 258], 520, 96, 2),
+    ([20, 33, 0, 40, 64, 1], 1024, 512, 1), ([30, 17, 65, 0], 64, 128, 2),  # tiles of 64, K of whole steps: many, one, two
 ])
 def test_experts_over_many_pairs(cuda, counts, d, hidden, top):
     from ohara_amd import ops
