@@ -929,8 +929,9 @@ int launch_fast(const AttnArgs& a, int G, dim3 grid, hipStream_t st) {
 }
 
 // Up to how many 64s of positions a context is one chunk / chunks for one workgroup a CU / for two (cut_context), by kernel and number of
-// (row, key head) pairs.  Fitted to launches from a graph over caches out of HBM: 4 to 512 pairs, 320 to 32768 positions, 1, 2 and 4 heads a
-// pair, 28700 shapes, on average 0.9 % behind the best cut of each.  Some of them, chunks: us
+// (row, key head) pairs.  Fitted to launches from a graph over caches out of HBM: 4 to 341 pairs, 320 to 32768 positions, 1, 2 and 4 heads a
+// pair, 1 to 32 key heads a position (sixteen and more, whose rows are 2 KiB and up apart, gain more from a cut), 34000 shapes, on average
+// 1 % behind the best cut of each.  Past that one chunk is within 10 % either way whatever the cut.  Some of them, chunks: us
 //   bf16, heads of 128, 1 each  12 pairs 1024  1: 16.5  8: 8.6  16: 9.1;  72 pairs 1536  1: 28.5  3: 16.6  6: 16.6  12: 16.5,
 //                               16384  1: 268  3: 113  7: 106  14: 103
 //                       4 each  64 pairs 4096  1: 70  4: 29.3  8: 31.1  16: 33.9;  80 pairs 16384  1: 272  3: 118  6: 117  12: 120
@@ -948,25 +949,25 @@ constexpr int CUT_PAIRS[] = {16, 25, 32, 42, 51, 64, 73, 85, 102, 128, 146, 170,
 constexpr short ANY = 32767;
 constexpr CutRule CUTS[8][CUT_BANDS] = {
     // bf16, 128 wide: one head a pair, several
-    {{5, ANY, ANY}, {5, 192, ANY}, {5, 128, ANY}, {5, 96, 96}, {5, 32, ANY}, {5, 20, 128}, {5, 9, 48}, {5, 32, 96},
-     {6, 6, 6}, {6, 6, 6}, {8, 8, 8}, {8, 8, 9}, {12, 12, 12}, {48, 48, 48}, {7, 7, 7}, {8, 8, 8}},
-    {{5, ANY, ANY}, {5, ANY, ANY}, {5, ANY, ANY}, {5, ANY, ANY}, {5, 192, ANY}, {5, 256, 256}, {5, 64, 192}, {5, 192, 192},
-     {6, 16, 64}, {7, 48, 64}, {12, 12, 24}, {12, 12, 48}, {24, 24, 24}, {96, 96, 96}, {10, 10, 10}, {16, 16, 16}},
+    {{5, ANY, ANY}, {5, 192, ANY}, {5, 256, ANY}, {5, 64, 128}, {5, 24, 24}, {5, 64, 256}, {5, 9, 48}, {5, 14, 14},
+     {5, 6, 6}, {5, 10, 10}, {8, 8, 8}, {8, 8, 9}, {12, 12, 12}, {64, 64, 64}, {5, 5, 5}, {12, 12, 12}},
+    {{5, ANY, ANY}, {5, ANY, ANY}, {5, ANY, ANY}, {5, ANY, ANY}, {5, 192, ANY}, {5, 192, 192}, {5, 32, ANY}, {5, 192, 192},
+     {6, 16, 64}, {7, 64, 64}, {12, 12, 24}, {12, 12, 48}, {20, 20, 20}, {96, 96, 96}, {9, 9, 9}, {12, 12, 12}},
     // int8, 128 wide: one head a pair, several
     {{5, ANY, ANY}, {5, 256, ANY}, {5, 256, ANY}, {5, 5, 5}, {5, 5, 5}, {5, 5, 5}, {5, 5, 5}, {5, 5, 5},
-     {5, 5, 5}, {6, 6, 6}, {6, 6, 6}, {6, 6, 6}, {16, 16, 16}, {48, 48, 48}, {5, 5, 5}, {24, 24, 24}},
-    {{5, ANY, ANY}, {5, 192, ANY}, {5, 48, ANY}, {5, 96, ANY}, {5, 64, ANY}, {5, 24, 256}, {5, 5, 256}, {5, 5, 192},
-     {6, 6, 24}, {6, 6, 96}, {10, 10, 12}, {10, 10, 12}, {14, 14, 14}, {48, 48, 48}, {8, 8, 8}, {32, 32, 32}},
+     {5, 5, 5}, {5, 5, 5}, {6, 6, 6}, {6, 6, 6}, {14, 14, 14}, {32, 32, 32}, {5, 5, 5}, {12, 12, 12}},
+    {{5, ANY, ANY}, {5, 256, ANY}, {5, 48, ANY}, {5, 96, ANY}, {5, 64, ANY}, {5, 24, 192}, {5, 5, 256}, {5, 5, 192},
+     {6, 6, 24}, {6, 6, 128}, {10, 10, 12}, {10, 10, 12}, {14, 14, 14}, {64, 64, 64}, {8, 8, 8}, {12, 12, 12}},
     // bf16, 64 wide: one or two heads a pair, more
-    {{6, ANY, ANY}, {7, 256, ANY}, {7, ANY, ANY}, {7, 48, 192}, {7, 32, ANY}, {7, 20, 128}, {9, 14, ANY}, {8, 14, 96},
-     {9, 9, 20}, {9, 9, 20}, {10, 10, 10}, {10, 10, 14}, {12, 12, 12}, {32, 32, 32}, {14, 14, 14}, {32, 32, 32}},
-    {{5, ANY, ANY}, {6, 96, ANY}, {6, 48, ANY}, {6, 32, 256}, {6, 24, ANY}, {6, 24, ANY}, {7, 14, ANY}, {7, 20, ANY},
-     {8, 8, 96}, {8, 14, 192}, {10, 10, 24}, {10, 10, 96}, {16, 16, 20}, {24, 24, 48}, {20, 20, 20}, {64, 64, 64}},
+    {{6, ANY, ANY}, {7, 192, ANY}, {7, ANY, ANY}, {7, 48, 192}, {7, 32, ANY}, {7, 32, 256}, {9, 14, ANY}, {8, 14, 24},
+     {9, 9, 24}, {9, 10, 20}, {10, 10, 10}, {10, 10, 14}, {12, 12, 12}, {24, 24, 24}, {10, 10, 10}, {12, 12, 12}},
+    {{5, ANY, ANY}, {6, 96, ANY}, {6, 64, ANY}, {6, 32, 256}, {6, 32, ANY}, {6, 32, ANY}, {7, 14, ANY}, {7, 20, ANY},
+     {8, 8, 192}, {8, 14, 96}, {10, 10, 24}, {10, 10, 96}, {16, 16, 16}, {24, 24, 64}, {20, 20, 20}, {12, 12, 12}},
     // int8, 64 wide: one or two heads a pair, more
-    {{6, ANY, ANY}, {8, 192, ANY}, {8, ANY, ANY}, {8, 128, ANY}, {8, 128, ANY}, {10, ANY, ANY}, {12, 16, 256}, {12, 256, ANY},
-     {14, 16, 24}, {14, 24, 128}, {24, 24, 24}, {32, 32, ANY}, {32, 32, 32}, {ANY, ANY, ANY}, {12, 12, 12}, {16, 16, 16}},
-    {{5, ANY, ANY}, {5, 256, ANY}, {5, ANY, ANY}, {5, 128, ANY}, {5, 64, 256}, {5, 96, ANY}, {5, 32, 192}, {8, 128, ANY},
-     {8, 8, 8}, {10, 32, 128}, {16, 16, 16}, {20, 20, ANY}, {24, 24, 24}, {ANY, ANY, ANY}, {14, 14, 14}, {24, 24, 24}},
+    {{6, ANY, ANY}, {8, 256, ANY}, {7, ANY, ANY}, {8, 128, ANY}, {8, 128, ANY}, {10, ANY, ANY}, {12, 32, 256}, {12, 96, ANY},
+     {14, 14, 24}, {14, 24, 96}, {20, 20, 20}, {20, 20, 24}, {24, 24, 24}, {96, 96, 96}, {12, 12, 12}, {12, 12, 12}},
+    {{5, ANY, ANY}, {5, 256, ANY}, {5, ANY, ANY}, {5, 128, ANY}, {5, 128, 256}, {5, 128, ANY}, {5, 48, 192}, {8, 128, ANY},
+     {10, 32, 192}, {10, 48, 256}, {16, 16, 16}, {20, 20, ANY}, {24, 24, 24}, {ANY, ANY, ANY}, {16, 16, 16}, {12, 12, 12}},
 };
 const CutRule& cut_rule(bool i8, int dh, int heads, int64_t pairs) {
   int band = 0;

@@ -16,9 +16,9 @@
 //
 // LA = 0: a k-step's fragments are read, then multiplied; the other waves of the CU fill the gap.  LA = 1, for the tiles with one or
 // two products a wave and activation fragment whose step is a chain: the fragments of the next group of products are read before
-// the present group's, across the barrier too.  us a call, 0 / 1: 32 x 32 tiles, 96 rows 768 x 3072 10.1 / 8.8; 64 x 128, 192 rows
-// 11264 x 2048 22.5 / 21.9; but 64 x 64, 192 rows 2048 x 5632 28.2 / 30.2; 128 x 192, 8192 rows 768 x 768 and 3072 (a mean) 37.0 / 39.5;
-// 256 x 256 with three groups ahead, 4001 rows 11264 x 2048 174 / 180.
+// the present group's, across the barrier too.  us a call, 0 / 1, from a graph over one set of operands: 32 x 32 tiles, 96 rows
+// 768 x 3072 10.1 / 8.8; 64 x 128, 192 rows 11264 x 2048 22.5 / 21.9; but 64 x 64, 192 rows 2048 x 5632 28.2 / 30.2; 128 x 192, 8192 rows
+// 768 x 768 and 3072 (a mean) 37.0 / 39.5; 256 x 256 with three groups ahead, 4001 rows 11264 x 2048 174 / 180.
 // What K leaves for a last step that is not full has its own code behind the loop: inside, its selects cost every step
 // (128 x 128, 4001 rows: 74.3 / 67.7).
 #pragma once
