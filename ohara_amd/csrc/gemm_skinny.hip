@@ -716,8 +716,10 @@ int launch_epi(const GemmArgs& a, int epi, int strips, hipStream_t st) {
     return ohara_launch_status();
   }
   // Normed rows of 1025 to 2048 columns: eight waves, so that a wave's share of K is requested in one go (3072 x 2048, 1, 16, 32 and 64
-  // rows: 9.0, 10.2, 13.9, 18.7 us with four, 6.0, 6.9, 11.9, 16.9 with eight).
-  if (NORM && a.K > 1024 && a.K <= 2048 && (epi == EPI_STORE || epi == EPI_ROPE)) {
+  // rows: 9.0, 10.2, 13.9, 18.7 us with four, 6.0, 6.9, 11.9, 16.9 with eight), where the CUs have not more strips than that hides
+  // anyway (33 and 64 rows, which wide_kernel cannot hold: 32000 x 2048 108, 155 us with four, 116, 161 with eight; 128256 x 2048 409, 596 and
+  // 452, 627; 257 to 1024 strips are group_kernel's).
+  if (NORM && a.K > 1024 && a.K <= 2048 && strips <= 256 && (epi == EPI_STORE || epi == EPI_ROPE)) {
     const bool six = a.K <= 1536;
     if (epi == EPI_STORE && six) hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_STORE, 8, 6>), grid, dim3(512), 0, st, a);
     else if (epi == EPI_STORE) hipLaunchKernelGGL((skinny_kernel<BT, NORM, EPI_STORE, 8>), grid, dim3(512), 0, st, a);
