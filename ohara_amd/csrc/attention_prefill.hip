@@ -433,9 +433,17 @@ int launch_teams(PrefillArgs a, hipStream_t st) {
 //     8 x 1024 x 6           97   / 62   / 28   / 36
 //     32 x 512 x 6          137   / 84   / 38   / 31
 //     16 x 700 x 16         269   / 173  / 74   / 68
-// so: teams while every workgroup is on a CU at once (two of the narrow ones' of 16), 128 queries from three workgroups a
-// CU on, else 64.  Before (one kernel, four waves, values through registers, the heads over all XCDs): 5.8, 45, 16.5, 25, 26, 167,
-// 50, 46, 92; 5.2, 10.4, 12, 64.
+// so: teams of 16 while every one has a CU to itself, and over more than two tiles while every two have one (with heads of 128
+// as teams of 32).  A shorter walk does not pay for the teams' barriers: us, teams / waves: heads of 64, 8 x 24 queries x 32 heads
+// 5.2 / 4.8; heads of 128, 8 x 33 x 16 6.2 / 5.4; over four tiles, 200 x 32 7.1 / 7.5.
+// 128 queries a workgroup read each position once where 64 read it twice, and are slower by a quarter where there are few of
+// them or the second half of the last one is empty (heads of 128, 32 x 300 x 6 behind 1500: 90 / 109 us, 64 / 128 queries).  So
+// from three a CU on, if at least half of their second halves hold queries; from fewer on where 64 queries need a second round:
+// with heads of 64 from the sixth workgroup of 64 queries a CU (28 x 112 x 24 behind 2000: 119 / 96; five: 20 x 128 x 32 behind 250
+// 18.7 / 20.6), with heads of 128 from the third, there if nearly every half holds queries and the walks are of about one length
+// (48 x 65 x 6 behind 1500: 77 / 62; but 4 x 1000 x 16 from the start: 33 / 35).
+// Before (one kernel, four waves, values through registers, the heads over all XCDs), for the table's lines: 5.8, 45, 16.5, 25,
+// 26, 167, 50, 46, 92; 5.2, 10.4, 12, 64.
 template <int D>
 int launch_prefill_for(const PrefillArgs& a, const int32_t* lengths, hipStream_t st) {  // lengths: on the host, where they differ
   constexpr int CUS = 256;
@@ -446,9 +454,14 @@ int launch_prefill_for(const PrefillArgs& a, const int32_t* lengths, hipStream_t
     return n * a.H;
   };
   if (((uintptr_t)a.k | (uintptr_t)a.v) & 15) return launch_waves<D, 1, false>(a, st);
-  if (blocks(16) <= CUS * (D == 64 ? 2 : 1)) return launch_teams<D, 1>(a, st);
-  if (blocks(32) <= CUS) return launch_teams<D, 2>(a, st);
-  if (blocks(128) >= 3 * CUS) return launch_waves<D, 2>(a, st);
+  const bool long_walk = a.pos + a.S > 128;
+  if (blocks(16) <= CUS * (D == 64 && long_walk ? 2 : 1)) return launch_teams<D, 1>(a, st);
+  if constexpr (D == 128)
+    if (long_walk && blocks(32) <= CUS) return launch_teams<D, 2>(a, st);
+  const int64_t wide = blocks(128), halves = blocks(64);
+  const bool even = 5 * halves >= 9 * wide && (a.S <= 128 || a.pos >= a.S);
+  const bool second_round = D == 64 ? halves > 5 * CUS : wide > CUS && even;
+  if ((wide >= 3 * CUS || second_round) && 2 * halves >= 3 * wide) return launch_waves<D, 2>(a, st);
   return launch_waves<D, 1>(a, st);
 }
 

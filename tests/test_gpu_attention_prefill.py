@@ -28,8 +28,10 @@ def _reference(q, k, v, pos):
 SHAPES = [
     (1, 16, 2, 1, 0), (1, 17, 6, 6, 15), (3, 33, 8, 2, 30), (4, 48, 16, 4, 1000), (1, 257, 8, 8, 31),   # a team of 16
     (1, 1000, 7, 7, 0), (2, 513, 6, 2, 63), (8, 32, 24, 8, 97),                                         # two teams
-    (2, 1030, 12, 3, 1), (1, 577, 24, 24, 64), (5, 65, 64, 8, 0),                                       # waves of 16
+    (2, 1030, 12, 3, 1), (1, 577, 24, 24, 64), (8, 32, 24, 8, 96),                                      # waves of 16
+    (3, 60, 300, 300, 10), (3, 129, 70, 70, 130), (3, 250, 70, 70, 249),                                # waves of 16
     (8, 520, 32, 4, 3), (3, 130, 131, 131, 63),                                                         # waves of 32
+    (5, 65, 64, 8, 0), (3, 128, 86, 43, 5), (3, 250, 70, 70, 250), (2, 200, 170, 34, 9),                # waves of 32
 ]
 
 
