@@ -8,7 +8,7 @@
 // registers) against this one, us a call from a graph over twelve sets of random operands in turn: 8192 rows 6144 x 768 with SwiGLU 114 / 85,
 // 2304 x 768 49 / 43, 768 x 768 with a residual 26.9 / 22.7, 768 x 3072 with a residual 65 / 57; 4001 rows 11264 x 2048 with SwiGLU 225 / 169,
 // 2048 x 5632 with a residual 116 / 97; 128 rows 6144 x 768 18.4 / 6.9, 768 x 3072 40.9 / 9.4 (one set again and again, out of the caches: 83,
-// 40, 17.6, 50; 167, 94; 6.2, 8.8).  Of that the epilogues (16 bytes a lane a store instead of 4 or 8, silu with a reciprocal of three
+// 38, 17.6, 50; 167, 94; 6.2, 8.8).  Of that the epilogues (16 bytes a lane a store instead of 4 or 8, silu with a reciprocal of three
 // instructions instead of eleven) took 5 to 9 %.
 // Measured and dropped: the loads spread among the products (8192^3: 961 -> 1001; with eight k-steps in flight 947, but 128-row tiles
 // 1035 -> 1152), deeper rings (no gain, fewer workgroups a CU), four waves a tile of 128 x 192 (99 / 52 us against 93 / 45 with eight).

@@ -20,8 +20,9 @@ def _check(got, x, w, nw, eps, plain):
 
 
 # (columns, K): two, three and four strips a workgroup with eight waves (K up to 1024) and with sixteen, the last group not full; then one strip
-# with eight waves
-SHAPES = [(4112, 8), (8200, 1000), (12304, 1024), (4128, 1032), (11264, 2048), (12000, 1544), (16368, 2040), (3072, 2048), (40, 1032)]
+# with eight waves; then more strips than groups take, where rows that wide_kernel cannot hold have a strip and four waves
+SHAPES = [(4112, 8), (8200, 1000), (12304, 1024), (4128, 1032), (11264, 2048), (12000, 1544), (16368, 2040), (3072, 2048), (40, 1032),
+          (16400, 1032), (16416, 2048)]
 
 
 @pytest.mark.parametrize("n,k", SHAPES)
