@@ -650,8 +650,8 @@ def phase_timeline(dev, prompt_len, steps=32, batch=1, int8=False):
 def bitnet_phase_timeline(dev, batch=1, steps=16):
     """Per-phase timeline of the single-launch BitNet decode step (C4 size, context 2047 -> 2048):
     workgroup 0's shader-clock samples at every grid barrier (six per barrier: phase work issued, own
-    stores complete, workgroup barrier passed, arrival issued, prefetch issued, barrier passed),
-    averaged over `steps` launches and over the layers after the first."""
+    stores complete, workgroup barrier passed, arrival issued, prefetch issued, barrier passed) or, for
+    a single sequence, behind every poll and every phase, averaged over `steps` launches and over the layers after the first."""
     from ohara_amd.bitnet import BitLlama
 
     cfg, st = bitnet_c4_state(dev)
@@ -679,6 +679,17 @@ def bitnet_phase_timeline(dev, batch=1, steps=16):
     sess.check_error()
     c = acc / steps
     kernel_us = total_ms / steps * 1e3
+    if batch == 1:  # ten samples a layer (100 MHz clock) of workgroup 0 and, 512 words on, of the first one of the down projection
+        first, down = c[: nl * 10].view(nl, 10), c[512 : 512 + nl * 10].view(nl, 10)
+        us = lambda t, a, b: round(float((t[1:, b] - t[1:, a]).mean()) / 100, 2)  # noqa: E731
+        return {"batch": 1, "kernel_us_hip_events": round(kernel_us, 1), "layers": nl,
+                "per_layer_us": round(float((first[1:, 9] - first[:-1, 9]).mean()) / 100, 2),
+                "after_last_layer_us (final norm + vocabulary projection + selection)": round(float(c[nl * 10 + 7] - first[-1, 9]) / 100, 1),
+                "us": {"stream polled for (q/k/v)": round(float((down[1:, 0] - down[:-1, 9]).mean()) / 100, 2),
+                       "q/k/v + rotary + append": us(down, 0, 1), "attention: q polled for, partials": us(down, 1, 2),
+                       "merge of a head": us(down, 2, 3), "merged row polled for": us(first, 3, 4), "output projection": us(first, 4, 5),
+                       "stream polled for (gate/up)": us(first, 5, 6), "gate/up + SwiGLU": us(first, 6, 7),
+                       "activations polled for": us(down, 7, 8), "down projection": us(down, 8, 9)}}
     per = c[: nl * 30].view(nl, 30)
     n_tail = 8  # after the last barrier of the layers: vocabulary projection (2), selection arrive (4) / wait (2)
     ticks_per_us = float(c[nl * 30 + n_tail - 1] - c[0]) / kernel_us  # within a few us of the whole launch

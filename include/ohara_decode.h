@@ -590,7 +590,9 @@ typedef struct OharaBitModel {
 int64_t ohara_bitnet_persistent_workspace_bytes(const OharaBitModel* m, int batch, int n_workgroups);
 int64_t ohara_bitnet_persistent_error_offset(const OharaBitModel* m, int batch, int n_workgroups);
 /* 1024 x uint64 shader-clock samples of workgroup 0 (six per grid barrier: phase work issued, own
- * stores complete, workgroup barrier passed, arrival issued, prefetch issued, barrier passed), taken
+ * stores complete, workgroup barrier passed, arrival issued, prefetch issued, barrier passed; a single
+ * sequence: ten per layer, behind every poll and phase, and those of the down projection's first
+ * workgroup 512 words on), taken
  * when s->prof_kernel == -2 (measurement only; a separate build of the kernel that exists for
  * head_dim 128 only, other shapes leave the slots untouched). */
 int64_t ohara_bitnet_persistent_profile_offset(const OharaBitModel* m, int batch, int n_workgroups);

@@ -1,8 +1,8 @@
-// Persistent decode kernel of the BitNet-b1.58 Llama: one launch computes a whole decode step (one
+// Persistent decode kernels of the BitNet-b1.58 Llama: one launch computes a whole decode step (one
 // new token per sequence, batch <= 8) of the Llama of ohara/models/llama.py:279-323 whose seven
-// per-layer projections are BitLinears (experiments/bitnet/bitnet.py:29-95).
+// per-layer projections are BitLinears (experiments/bitnet/bitnet.py:29-95).  A single sequence: bitnet_one.h.
 //
-// Same skeleton as the bf16 persistent kernel (one resident workgroup per CU, grid-wide barriers
+// Two to eight sequences: same skeleton as the bf16 persistent kernel (one resident workgroup per CU, grid-wide barriers
 // between phases, write-once mailboxes written with device-scope stores), with integer GEMM phases:
 //   P1  [embedding] + norm1 + per-projection BitLinear norm / int8 codes + Q, K, V on
 //       v_mfma_i32_16x16x64_i8 + rotary + cache append
@@ -12,10 +12,8 @@
 //   P5  codes + ff.down, K split over two groups of workgroups; the int32 partial sums are exact, so
 //       whoever needs the residual stream next adds them, scales and rounds as one BitLinear would
 // then final norm + vocabulary projection (bf16, the bf16 kernel's phase) and the arg-max.
-// A single sequence: every workgroup derives the codes of the row it multiplies itself (a row is 2-11 KB;
-// the three passes over it, spread over the workgroup, cost about as much as one hand-off).  Two to eight
-// sequences: each (BitLinear, row) pair is quantised once, by one workgroup, and handed to the others
-// through a code mailbox and one more grid barrier per GEMM phase.  Either way the reduction orders are
+// Each (BitLinear, row) pair is quantised once, by one workgroup, and handed to the others
+// through a code mailbox and one more grid barrier per GEMM phase.  The reduction orders are
 // those of the stand-alone BitLinear kernels, so the integer accumulators are those kernels' accumulators.
 #include <vector>
 
@@ -47,7 +45,7 @@ struct BitMegaArgs {
   char* am;        // NL act-mailboxes
   float* pm;       // NL attention-partial mailboxes
   int32_t* dm;     // NL mailboxes of the down projection's int32 partial sums [part][strip][row][16]
-  int8_t* cq;      // NL code mailboxes (batch > 1): the code rows of the seven BitLinears, each quantised by one workgroup
+  int8_t* cq;      // NL code mailboxes: the code rows of the seven BitLinears, each quantised by one workgroup
   float* cs;       // NL x [7][16] {s, sum q} pairs of those rows (eight used)
   size_t cq_stride;
   float* ds;       // NL x 32 floats (a 128-byte line per layer: one writer, written before it is read):
@@ -55,6 +53,7 @@ struct BitMegaArgs {
   size_t xm_stride, qm_stride, am_stride, pm_stride, dm_stride;
   float* cand_val;
   int* cand_idx;
+  char* tg;        // a single sequence: two sets of polled mailboxes (bitnet_one.h)
   bf16_t* logits;
   int32_t* step_state;
   int64_t* history;
@@ -211,11 +210,9 @@ __device__ __forceinline__ uint2 bit_codes8(uint4 xh, float s, uint32_t& sq) {
 // the sum of the codes from the sum of `n` raw words
 __device__ __forceinline__ int bit_code_sum(uint32_t sq, int n) { return (int)(sq - (uint32_t)n * BIT_RINT_MAGIC_BITS); }
 
-// ---- batch 1: the row in registers -------------------------------------------------------------
+// ---- a row over the workgroup ------------------------------------------------------------------
 // Thread t owns the 8-value pieces t, t + 256, ... (NP of them; pieces beyond the row are zero and
-// change no sum or maximum); the row never goes through LDS, all loads (row, norm weights) are
-// in flight together, and the sum of the codes - needed only after the product - is left as four
-// per-wave partial sums.
+// change no sum or maximum); the row never goes through LDS, and all its loads are in flight together.
 template <int NP, typename F>
 __device__ __forceinline__ void row1_load(uint4 (&r)[NP], int pieces, F f) {
 #pragma unroll
@@ -224,126 +221,13 @@ __device__ __forceinline__ void row1_load(uint4 (&r)[NP], int pieces, F f) {
     r[i] = p < pieces ? f(p) : make_uint4(0, 0, 0, 0);
   }
 }
-__device__ __forceinline__ float row1_sum(float v, float* red) {
-  v = wave_sum(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return ((red[0] + red[1]) + red[2]) + red[3];
-}
-// block-level RMSNorm (norm.py:16-21) of the row, in place
-template <int NP>
-__device__ __forceinline__ void row1_block_norm(uint4 (&v)[NP], const uint4 (&w)[NP], int K, float eps, float* red) {
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < NP; ++i) ss += bit_sumsq8(v[i]);
-  const float rinv0 = 1.0f / sqrtf(row1_sum(ss, red) / (float)K + eps);
-#pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const uint32_t uu[4] = {v[i].x, v[i].y, v[i].z, v[i].w}, ww[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
-    uint32_t o[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      o[j] = pack_bf(rbf(lo_bf(uu[j]) * rinv0) * lo_bf(ww[j]), rbf(hi_bf(uu[j]) * rinv0) * hi_bf(ww[j]));
-    v[i] = make_uint4(o[0], o[1], o[2], o[3]);
-  }
-}
-// the BitLinear's own norm, scale and codes of the row h (bitnet.py:29-33, 49-53) -> xq (LDS);
-// thread 0 leaves the scale in *s_out, every wave its share of the sum of the codes in sumw[wave]
-template <int NP>
-__device__ __forceinline__ void row1_codes(const uint4 (&h)[NP], const uint4 (&nw)[NP], int pieces, int K, float eps,
-                                           int8_t* xq, float* red, float* s_out, int* sumw) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < NP; ++i) ss += bit_sumsq8(h[i]);
-  const float rinv = 1.0f / sqrtf(row1_sum(ss, red) / (float)K + eps);
-  uint4 xh[NP];
-  uint32_t mg = 0u;
-#pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    xh[i] = bit_xhat8(h[i], nw[i], rinv);
-    mg = bit_mag_max8(mg, xh[i]);
-  }
-  float mx = wave_max(bit_mag_float(mg));
-  __syncthreads();
-  if (lane == 0) red[wave] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  const float s = 127.0f / fmaxf(mx, 1e-5f);
-  uint32_t sqw = 0u;
-#pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const uint2 pk = bit_codes8(xh[i], s, sqw);
-    const int p = tid + 256 * i;
-    if (p < pieces) sts8(xq + (size_t)p * 8, pk);
-  }
-  int sq = bit_code_sum(sqw, NP * 8);
-  sq = lanes_sum<32, 1>(sq);
-  if (lane == 0) sumw[wave] = sq;
-  if (tid == 0) *s_out = s;
-}
-
-// Batch 1: one row from `load(piece) -> uint4` into one or two code sets (two BitLinears that share
-// the input and the block norm: ff.gate and ff.up).  Every thread of the workgroup calls.
-template <int NP, typename Load>
-__device__ __forceinline__ void bit_stage_row1(const BitLds& L, int nsets, int K, const bf16_t* pre_w, const bf16_t* nw0,
-                                               const bf16_t* nw1, float eps, Load load) {
-  const int tid = threadIdx.x;
-  const int pieces = K >> 3;
-  uint4 x[NP], pw[NP], n0[NP], n1[NP];
-  row1_load(x, pieces, load);
-  if (pre_w) row1_load(pw, pieces, [&](int p) { return ldg16(pre_w + (size_t)p * 8); });
-  row1_load(n0, pieces, [&](int p) { return ldg16(nw0 + (size_t)p * 8); });
-  if (nsets == 2) row1_load(n1, pieces, [&](int p) { return ldg16(nw1 + (size_t)p * 8); });
-  __syncthreads();  // whoever still reads the previous codes or scales is done
-  {
-    const int pad8 = (L.ldq - K) >> 3;
-    for (int i = tid; i < nsets * pad8; i += 256) {
-      const int st = i / pad8, c = i - st * pad8;
-      sts8(L.codes + (size_t)st * L.set + K + c * 8, make_uint2(0, 0));
-    }
-  }
-  if (pre_w) row1_block_norm(x, pw, K, eps, L.red);
-  row1_codes(x, n0, pieces, K, eps, L.codes, L.red, L.s_s, L.sumw);
-  if (nsets == 2) row1_codes(x, n1, pieces, K, eps, L.codes + L.set, L.red, L.s_s + 16, L.sumw + 4);
-  __syncthreads();
-  if (tid < nsets) L.s_sum[tid * 16] = (L.sumw[tid * 4] + L.sumw[tid * 4 + 1]) + (L.sumw[tid * 4 + 2] + L.sumw[tid * 4 + 3]);
-  // the product that follows passes a workgroup barrier before anyone reads s_sum
-}
-// The norm weights of a row's staging (block norm `pre_w`, the BitLinears' own norms `nw0` / `nw1`) do not
-// depend on the phase before it: row1_norm_fetch issues their loads - in the barrier window, next to the
-// phase's weight prefetch, where a cold HBM read costs nothing - and bit_stage_row1_pre takes them from
-// registers.  Pieces past the row read the last piece and multiply values that are zero.
+// A norm's weights for those pieces.  Pieces past the row read the last piece and multiply values that are zero.
 template <int NP>
 __device__ __forceinline__ void row1_norm_fetch(uint4 (&r)[NP], int pieces, const bf16_t* w) {
 #pragma unroll
   for (int i = 0; i < NP; ++i) r[i] = ldg16(w + (size_t)min((int)threadIdx.x + 256 * i, pieces - 1) * 8);
 }
-template <int NP, typename Load>
-__device__ __forceinline__ void bit_stage_row1_pre(const BitLds& L, int nsets, int K, bool block_norm, const uint4 (&pw)[NP],
-                                                   const uint4 (&n0)[NP], const uint4 (&n1)[NP], float eps, Load load) {
-  const int tid = threadIdx.x;
-  const int pieces = K >> 3;
-  uint4 x[NP];
-  row1_load(x, pieces, load);
-  __syncthreads();  // whoever still reads the previous codes or scales is done
-  {
-    const int pad8 = (L.ldq - K) >> 3;
-    for (int i = tid; i < nsets * pad8; i += 256) {
-      const int st = i / pad8, c = i - st * pad8;
-      sts8(L.codes + (size_t)st * L.set + K + c * 8, make_uint2(0, 0));
-    }
-  }
-  if (block_norm) row1_block_norm(x, pw, K, eps, L.red);
-  row1_codes(x, n0, pieces, K, eps, L.codes, L.red, L.s_s, L.sumw);
-  if (nsets == 2) row1_codes(x, n1, pieces, K, eps, L.codes + L.set, L.red, L.s_s + 16, L.sumw + 4);
-  __syncthreads();
-  if (tid < nsets) L.s_sum[tid * 16] = (L.sumw[tid * 4] + L.sumw[tid * 4 + 1]) + (L.sumw[tid * 4 + 2] + L.sumw[tid * 4 + 3]);
-  // the product that follows passes a workgroup barrier before anyone reads s_sum
-}
-
-// ---- batch > 1: every (BitLinear, row) pair is quantised once ---------------------------------
+// ---- every (BitLinear, row) pair is quantised once ---------------------------------
 // With B rows a workgroup that derived all the codes itself would spend 8 - 17 us per phase on them at eight rows
 // (the three passes are instruction-bound with one wave per SIMD), 256 times over.  Instead ONE workgroup
 // per (BitLinear, row) pair derives the row's codes with all its threads (thread t owns the pieces t, t + 256, ...),
@@ -589,18 +473,83 @@ __device__ void bit_stage_final_norm(bf16_t* xs, int ldxs, const BitX& x, const 
   }
 }
 
+// The arg-max over the grid of every row's logits (lane l of a wave holds the best of column l & 15) -> ids, history.
+// Every thread of the grid calls.
+template <class PROF>
+__device__ __forceinline__ void bit_select(const BitMegaArgs& a, float* red, GridSync& gs, float best_v, int best_i, int B, int step, PROF& pf) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwg = gridDim.x;
+#pragma unroll
+  for (int o = 16; o < 64; o <<= 1) {
+    const float ov = __shfl_xor(best_v, o, WAVE);
+    const int oi = __shfl_xor(best_i, o, WAVE);
+    if (ov > best_v || (ov == best_v && oi < best_i)) {
+      best_v = ov;
+      best_i = oi;
+    }
+  }
+  __syncthreads();
+  float* cv = red;
+  int* ci = reinterpret_cast<int*>(red + 64);
+  if (lane < 16) {
+    cv[wave * 16 + lane] = best_v;
+    ci[wave * 16 + lane] = best_i;
+  }
+  __syncthreads();
+  if (tid < B) {
+    float bv = cv[tid];
+    int bi = ci[tid];
+    for (int w = 1; w < 4; ++w) {
+      const float ov = cv[w * 16 + tid];
+      const int oi = ci[w * 16 + tid];
+      if (ov > bv || (ov == bv && oi < bi)) {
+        bv = ov;
+        bi = oi;
+      }
+    }
+    st_coh4(a.cand_val + (size_t)blockIdx.x * B + tid, __float_as_uint(bv));
+    st_coh4(a.cand_idx + (size_t)blockIdx.x * B + tid, (uint32_t)bi);
+  }
+  gs.arrive(pf);
+  gs.wait(pf);
+  if (blockIdx.x == 0) {
+    for (int b = wave; b < B; b += 4) {
+      float bv = -INFINITY;
+      int bi = 0x7fffffff;
+      for (int w = lane; w < nwg; w += 64) {
+        const float ov = __uint_as_float(ld_coh4(a.cand_val + (size_t)w * B + b));
+        const int oi = (int)ld_coh4(a.cand_idx + (size_t)w * B + b);
+        if (ov > bv || (ov == bv && oi < bi)) {
+          bv = ov;
+          bi = oi;
+        }
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        const float ov = __shfl_xor(bv, o, WAVE);
+        const int oi = __shfl_xor(bi, o, WAVE);
+        if (ov > bv || (ov == bv && oi < bi)) {
+          bv = ov;
+          bi = oi;
+        }
+      }
+      if (lane == 0) {
+        if (bi == 0x7fffffff) bi = 0;
+        a.ids[b] = bi;
+        if (a.history && step < a.hist_cap) a.history[(size_t)step * B + b] = bi;
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------------------
 // the kernel
 // ---------------------------------------------------------------------------------------
-// ONE: a single sequence.  The staging of the workgroup's own row is then the only one compiled in, the
-// quantise-once sub-phases and the code fetch otherwise, which keeps either kernel's layer loop much smaller
-// than one that holds both.
 // PROFILE: with the phase stamps (measurement builds of the head-dim-128 kernels only).
-template <int D, int G, bool ONE, bool PROFILE = false>
+template <int D, int G, bool PROFILE = false>
 __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const OharaBitModel& m = a.m;
-  const int d = m.d_model, H = m.n_heads, Hkv = m.n_kv_heads, F = m.d_ff, V = m.vocab, B = ONE ? 1 : a.B;
+  const int d = m.d_model, H = m.n_heads, Hkv = m.n_kv_heads, F = m.d_ff, V = m.vocab, B = a.B;
   const int nwg = gridDim.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int mm = lane & 15, gg = lane >> 4;
@@ -690,13 +639,6 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
     rope_s = ldg4(m.sin + (size_t)pos * (D >> 1) + (dd >> 1));
   }
   bit_prefetch<2>(reinterpret_cast<const uint4*>(gptr(ltab[0].w[p1_which])), KCd, p1_strip0, 0, KCd, p1_strip0 < p1_nstr, wpre);
-  // batch-1 build: the norm weights of the next phase's staging, fetched in the barrier windows
-  uint4 npw[1], nn0[3], nn1[1];
-  npw[0] = nn0[0] = nn0[1] = nn0[2] = nn1[0] = make_uint4(0, 0, 0, 0);
-  if (ONE && 2 * p1_gi < p1_nstr) {
-    row1_norm_fetch<1>(npw, d >> 3, reinterpret_cast<const bf16_t*>(gptr(ltab[0].norm1)));
-    row1_norm_fetch<1>(reinterpret_cast<uint4(&)[1]>(nn0), d >> 3, reinterpret_cast<const bf16_t*>(gptr(ltab[0].nw[p1_which])));
-  }
 
   for (int l = 0; l < m.n_layers; ++l) {
     const BitLayerDev& LY = ltab[l];
@@ -730,7 +672,7 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
       bitx_load<8>(xin, b, p * 8, w);
       return make_uint4(w[0], w[1], w[2], w[3]);
     };
-    if (!ONE) {
+    {
       bit_for_units(3 * B, nwg, [&](int u) {
         const int which = u / B, b = u - which * B;
         bit_quant_once<1>(L, d, norm1, reinterpret_cast<const bf16_t*>(gptr(LY.nw[which])), m.eps,
@@ -742,12 +684,7 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
     if (2 * p1_gi < p1_nstr) {
       const int which = p1_which;
       const uint4* wp = reinterpret_cast<const uint4*>(gptr(LY.w[which]));
-      if (ONE) {
-        auto load0 = [&](int p) { return load_in(0, p); };
-        bit_stage_row1_pre<1>(L, 1, d, true, npw, reinterpret_cast<const uint4(&)[1]>(nn0), nn1, m.eps, load0);
-      } else {
-        bit_codes_fetch(L, 1, B, cq_l + (size_t)which * B * ldq_d, cs_l + which * 32, 0, KCd, true);
-      }
+      bit_codes_fetch(L, 1, B, cq_l + (size_t)which * B * ldq_d, cs_l + which * 32, 0, KCd, true);
       for (int s0 = 2 * p1_gi; s0 < p1_nstr; s0 += 2 * p1_gsz) {
         const bool first = s0 == 2 * p1_gi;
         const int strip = s0 + sub2;
@@ -791,8 +728,6 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
     gs.arrive(pf);
     const uint4* wo = reinterpret_cast<const uint4*>(gptr(LY.w[BO]));
     bit_prefetch<4>(wo, KCo, blockIdx.x, 0, KCo, (int)blockIdx.x < ns_d, wpre);
-    if (ONE && (int)blockIdx.x < ns_d)
-      row1_norm_fetch<1>(reinterpret_cast<uint4(&)[1]>(nn0), HD >> 3, reinterpret_cast<const bf16_t*>(gptr(LY.nw[BO])));
     // the residual of this lane's outputs in the first strip: known since the previous layer
     uint32_t rpre[2] = {0u, 0u};
     if ((int)blockIdx.x < ns_d && wave == 0 && mm < B && (int)blockIdx.x * 16 + 4 * gg < d)
@@ -800,7 +735,7 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
     gs.wait(pf);
     // ---- P3: merge + attn.proj + residual ----
     L.shape(B, HD);
-    if (!ONE) {  // one workgroup per row merges the row's chunks and derives its codes
+    {  // one workgroup per row merges the row's chunks and derives its codes
       bit_for_units(B, nwg, [&](int b) {
         bf16_t* xs = L.stage;
         __syncthreads();
@@ -814,21 +749,7 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
     }
     for (int strip = blockIdx.x; strip < ns_d; strip += nwg) {
       const bool first = strip == (int)blockIdx.x;
-      if (first) {
-        if (ONE) {
-          bf16_t* xs = L.stage;
-          const int ldxs = L.ldm;
-          // a single sequence always runs with 16 chunks unless there are more than 16 KV heads: that
-          // merge is part of the kernel (a call would wait for the weights already in flight)
-          if (a.ns == 16 && B * HD > 4 * 256) stage_attn_merge<16>(xs, ldxs, p_l, B, H, D, mrg_w, mrg_l);
-          else stage_attn_merge_any<false>(a.ns, xs, ldxs, p_l, B, H, D, mrg_w, mrg_l);
-          __syncthreads();
-          auto load0 = [&](int p) { return lds16(xs + p * 8); };
-          bit_stage_row1_pre<1>(L, 1, HD, false, npw, reinterpret_cast<const uint4(&)[1]>(nn0), nn1, m.eps, load0);
-        } else {
-          bit_codes_fetch(L, 1, B, cq_l + cq_o, cs_l + BO * 32, 0, KCo, true);
-        }
-      }
+      if (first) bit_codes_fetch(L, 1, B, cq_l + cq_o, cs_l + BO * 32, 0, KCo, true);
       i32x4 acc;
       if (bit_strip<4>(wo, KCo, strip, 0, KCo, true, wpre, first, L.codes, L.ldq, B,
                        reinterpret_cast<int*>(L.red), acc) && mm < B) {
@@ -852,11 +773,6 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
       bit_prefetch<2>(wg, KCd, strip, 0, KCd, strip < ns_f, wpre);
       bit_prefetch<2>(wu, KCd, strip, 0, KCd, strip < ns_f, wpre2);
     }
-    if (ONE && 2 * (int)blockIdx.x < ns_f) {
-      row1_norm_fetch<1>(npw, d >> 3, norm2);
-      row1_norm_fetch<1>(reinterpret_cast<uint4(&)[1]>(nn0), d >> 3, reinterpret_cast<const bf16_t*>(gptr(LY.nw[BG])));
-      row1_norm_fetch<1>(nn1, d >> 3, reinterpret_cast<const bf16_t*>(gptr(LY.nw[BU])));
-    }
     gs.wait(pf);
     // ---- P4: norm2 + ff.gate, ff.up + SwiGLU; two strips at a time, two waves each ----
     L.shape(B, d);
@@ -867,7 +783,7 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
       bitx_load<8>(xmid, b, p * 8, w);
       return make_uint4(w[0], w[1], w[2], w[3]);
     };
-    if (!ONE) {
+    {
       bit_for_units(2 * B, nwg, [&](int u) {
         const int set = u / B, b = u - set * B;
         bit_quant_once<1>(L, d, norm2, reinterpret_cast<const bf16_t*>(gptr(LY.nw[BG + set])), m.eps,
@@ -878,12 +794,7 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
       gs.wait(nopf);
     }
     if (2 * (int)blockIdx.x < ns_f) {
-      if (ONE) {
-        auto load0 = [&](int p) { return load_mid(0, p); };
-        bit_stage_row1_pre<1>(L, 2, d, true, npw, reinterpret_cast<const uint4(&)[1]>(nn0), nn1, m.eps, load0);
-      } else {
-        bit_codes_fetch(L, 2, B, cq_l + cq_g, cs_l + BG * 32, 0, KCd, true);
-      }
+      bit_codes_fetch(L, 2, B, cq_l + cq_g, cs_l + BG * 32, 0, KCd, true);
       for (int s0 = 2 * (int)blockIdx.x; s0 < ns_f; s0 += 2 * nwg) {
         const bool first = s0 == 2 * (int)blockIdx.x;
         const int strip = s0 + sub2;
@@ -912,18 +823,13 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
     {
       const int unit = blockIdx.x, part = unit / ns_d, strip = unit - part * ns_d;
       bit_prefetch<4>(wd, KCf, strip, part * per_part, min(KCf, (part + 1) * per_part), unit < ns_d * OHARA_BIT_DOWN_SPLIT, wpre);
-      if (ONE && unit < ns_d * OHARA_BIT_DOWN_SPLIT) {
-        const bf16_t* nwd = reinterpret_cast<const bf16_t*>(gptr(LY.nw[BD]));
-        if (F <= 2048) row1_norm_fetch<1>(reinterpret_cast<uint4(&)[1]>(nn0), F >> 3, nwd);
-        else row1_norm_fetch<3>(nn0, F >> 3, nwd);
-      }
     }
     gs.wait(pf);
     // ---- P5: ff.down, K split over OHARA_BIT_DOWN_SPLIT groups of workgroups ----
     {
       const int nunits = ns_d * OHARA_BIT_DOWN_SPLIT;
       L.shape(B, F);
-      if (!ONE) {
+      {
         const bf16_t* nwd = reinterpret_cast<const bf16_t*>(gptr(LY.nw[BD]));
         bit_for_units(B, nwg, [&](int b) {
           auto loadq = [&](int p) { return ldg16(am_addr(a_l, a.blk_a, b, p * 8)); };
@@ -938,15 +844,10 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
         const bool first = unit == (int)blockIdx.x;
         const int part = unit / ns_d, strip = unit - part * ns_d;
         if (!staged) {
-          if (ONE) {
-            auto load0 = [&](int p) { return ldg16(am_addr(a_l, a.blk_a, 0, p * 8)); };
-            if (F <= 2048) bit_stage_row1_pre<1>(L, 1, F, false, npw, reinterpret_cast<const uint4(&)[1]>(nn0), nn1, m.eps, load0);
-            else bit_stage_row1_pre<3>(L, 1, F, false, nn0, nn0, nn0, m.eps, load0);
-          } else {  // the codes of this workgroup's K partition (its units all lie in one partition or take whole rows)
-            const bool one_part = (int)blockIdx.x + nwg >= nunits;
-            if (one_part) bit_codes_fetch(L, 1, B, cq_l + cq_dn, cs_l + BD * 32, part * per_part, min(KCf, (part + 1) * per_part), false);
-            else bit_codes_fetch(L, 1, B, cq_l + cq_dn, cs_l + BD * 32, 0, KCf, true);
-          }
+          // the codes of this workgroup's K partition (its units all lie in one partition or take whole rows)
+          const bool one_part = (int)blockIdx.x + nwg >= nunits;
+          if (one_part) bit_codes_fetch(L, 1, B, cq_l + cq_dn, cs_l + BD * 32, part * per_part, min(KCf, (part + 1) * per_part), false);
+          else bit_codes_fetch(L, 1, B, cq_l + cq_dn, cs_l + BD * 32, 0, KCf, true);
           staged = true;
         }
         i32x4 acc;
@@ -968,10 +869,6 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
     if (l + 1 == m.n_layers) break;  // the last barrier's wait follows the loop, behind another prefetch
     bit_prefetch<2>(reinterpret_cast<const uint4*>(gptr(ltab[l + 1].w[p1_which])), KCd, p1_strip0, 0, KCd,
                     p1_strip0 < p1_nstr, wpre);
-    if (ONE && 2 * p1_gi < p1_nstr) {
-      row1_norm_fetch<1>(npw, d >> 3, reinterpret_cast<const bf16_t*>(gptr(ltab[l + 1].norm1)));
-      row1_norm_fetch<1>(reinterpret_cast<uint4(&)[1]>(nn0), d >> 3, reinterpret_cast<const bf16_t*>(gptr(ltab[l + 1].nw[p1_which])));
-    }
     gs.wait(pf);
   }
   GemmPre lpre;
@@ -991,69 +888,7 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
     __syncthreads();
     lm_phase(lm, lpre, xs, ldxs, B, best_v, best_i, pf);
   }
-  if (a.select) {
-#pragma unroll
-    for (int o = 16; o < 64; o <<= 1) {
-      const float ov = __shfl_xor(best_v, o, WAVE);
-      const int oi = __shfl_xor(best_i, o, WAVE);
-      if (ov > best_v || (ov == best_v && oi < best_i)) {
-        best_v = ov;
-        best_i = oi;
-      }
-    }
-    __syncthreads();
-    float* cv = L.red;
-    int* ci = reinterpret_cast<int*>(L.red + 64);
-    if (lane < 16) {
-      cv[wave * 16 + lane] = best_v;
-      ci[wave * 16 + lane] = best_i;
-    }
-    __syncthreads();
-    if (tid < B) {
-      float bv = cv[tid];
-      int bi = ci[tid];
-      for (int w = 1; w < 4; ++w) {
-        const float ov = cv[w * 16 + tid];
-        const int oi = ci[w * 16 + tid];
-        if (ov > bv || (ov == bv && oi < bi)) {
-          bv = ov;
-          bi = oi;
-        }
-      }
-      st_coh4(a.cand_val + (size_t)blockIdx.x * B + tid, __float_as_uint(bv));
-      st_coh4(a.cand_idx + (size_t)blockIdx.x * B + tid, (uint32_t)bi);
-    }
-    gs.arrive(pf);
-    gs.wait(pf);
-    if (blockIdx.x == 0) {
-      for (int b = wave; b < B; b += 4) {
-        float bv = -INFINITY;
-        int bi = 0x7fffffff;
-        for (int w = lane; w < nwg; w += 64) {
-          const float ov = __uint_as_float(ld_coh4(a.cand_val + (size_t)w * B + b));
-          const int oi = (int)ld_coh4(a.cand_idx + (size_t)w * B + b);
-          if (ov > bv || (ov == bv && oi < bi)) {
-            bv = ov;
-            bi = oi;
-          }
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-          const float ov = __shfl_xor(bv, o, WAVE);
-          const int oi = __shfl_xor(bi, o, WAVE);
-          if (ov > bv || (ov == bv && oi < bi)) {
-            bv = ov;
-            bi = oi;
-          }
-        }
-        if (lane == 0) {
-          if (bi == 0x7fffffff) bi = 0;
-          a.ids[b] = bi;
-          if (a.history && step < a.hist_cap) a.history[(size_t)step * B + b] = bi;
-        }
-      }
-    }
-  }
+  if (a.select) bit_select(a, L.red, gs, best_v, best_i, B, step, pf);
   if (blockIdx.x == 0 && tid == 0) {
     *gs.done = gs.k - 1;
     if (a.select) {
@@ -1063,13 +898,21 @@ __global__ __launch_bounds__(256) void bitnet_mega_kernel(BitMegaArgs a) {
   }
 }
 
+}  // namespace
+
+#include "bitnet_one.h"
+
+namespace {
+
 // ---- workspace layout ------------------------------------------------------------------
-#define OHARA_BIT_BAR_WORDS(nwg) ((((nwg) + OHARA_BAR_GROUP - 1) / OHARA_BAR_GROUP + 12) * 64)
+// (two words behind GridSync's: the launches since the workspace was cleared - a single sequence's hand-offs alternate between two
+// sets of mailboxes by it - and the workgroups that have finished, which tells the last one out that it is the one to count on)
+#define OHARA_BIT_BAR_WORDS(nwg) ((((nwg) + OHARA_BAR_GROUP - 1) / OHARA_BAR_GROUP + 14) * 64)
 
 size_t bit_al(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct BitLayout {
-  size_t layers, xm, qm, am, pm, dm, ds, cq, cs, candv, candi, prof, bar, total;
+  size_t layers, xm, qm, am, pm, dm, ds, cq, cs, candv, candi, prof, bar, tg, total;
   size_t xm_stride, qm_stride, am_stride, pm_stride, dm_stride, cq_stride;
   int blk_x, blk_a;
 };
@@ -1093,11 +936,11 @@ BitLayout bit_layout(const OharaBitModel* m, int B, int nwg) {
   L.pm = o; o += L.pm_stride * sizeof(float) * NL;
   L.dm = o; o += L.dm_stride * sizeof(int32_t) * NL;
   L.ds = o; o += bit_al((size_t)NL * 32 * sizeof(float));
-  {  // batch > 1: code rows of the seven BitLinears (K padded to 256 columns + 16), B rows each; {s, sum q} pairs
+  {  // code rows of the seven BitLinears (K padded to 256 columns + 16), B rows each; {s, sum q} pairs
     const int ldq_d = (((m->d_model + 255) >> 8) << 8) + 16, ldq_o = (((hd + 255) >> 8) << 8) + 16;
     const int ldq_f = (((m->d_ff + 255) >> 8) << 8) + 16;
     const size_t o_ = bit_cq_al((size_t)3 * B * ldq_d), g_ = bit_cq_al(o_ + (size_t)B * ldq_o), dn_ = bit_cq_al(g_ + (size_t)2 * B * ldq_d);
-    L.cq_stride = B > 1 ? bit_cq_al(dn_ + (size_t)B * ldq_f) : 0;
+    L.cq_stride = bit_cq_al(dn_ + (size_t)B * ldq_f);
   }
   L.cq = o; o += L.cq_stride * NL;
   L.cs = o; o += bit_al((size_t)NL * 256 * sizeof(float));
@@ -1105,6 +948,8 @@ BitLayout bit_layout(const OharaBitModel* m, int B, int nwg) {
   L.candi = o; o += bit_al((size_t)nwg * B * sizeof(int));
   L.prof = o; o += bit_al(1024 * sizeof(unsigned long long));
   L.bar = o; o += bit_al(OHARA_BIT_BAR_WORDS(nwg) * sizeof(unsigned int));
+  L.tg = o;  // a single sequence: the two sets of polled mailboxes, filled with 0xFF ("not written yet")
+  if (B == 1) o += 2 * one_boxes(*m).stride * NL;
   L.total = o;
   return L;
 }
@@ -1180,7 +1025,8 @@ int ohara_bitnet_decode_persistent(const OharaBitModel* m, const OharaDecodeStat
     }
     if (hipMemcpyAsync((void*)a.layers_dev, tab.data(), sizeof(BitLayerDev) * m->n_layers, hipMemcpyHostToDevice, st) !=
             hipSuccess ||
-        hipMemsetAsync((void*)(ws + L.bar), 0, L.total - L.bar, st) != hipSuccess ||
+        hipMemsetAsync((void*)(ws + L.bar), 0, L.tg - L.bar, st) != hipSuccess ||
+        (L.total > L.tg && hipMemsetAsync((void*)(ws + L.tg), 0xFF, L.total - L.tg, st) != hipSuccess) ||
         hipStreamSynchronize(st) != hipSuccess)
       return OHARA_ELAUNCH;
     return OHARA_OK;
@@ -1191,6 +1037,7 @@ int ohara_bitnet_decode_persistent(const OharaBitModel* m, const OharaDecodeStat
   a.dm_stride = L.dm_stride;
   a.cq = reinterpret_cast<int8_t*>(ws + L.cq); a.cs = reinterpret_cast<float*>(ws + L.cs); a.cq_stride = L.cq_stride;
   a.blk_x = L.blk_x; a.blk_a = L.blk_a;
+  a.tg = ws + L.tg;
   a.cand_val = reinterpret_cast<float*>(ws + L.candv);
   a.cand_idx = reinterpret_cast<int*>(ws + L.candi);
   a.bar = reinterpret_cast<unsigned int*>(ws + L.bar);
@@ -1204,43 +1051,26 @@ int ohara_bitnet_decode_persistent(const OharaBitModel* m, const OharaDecodeStat
   ns = ns < 1 ? 1 : (ns > OHARA_MEGA_NS ? OHARA_MEGA_NS : ns);
   while (ns & (ns - 1)) ns &= ns - 1;
   a.ns = ns;
-  const size_t smem = bit_smem_bytes(m, s->batch, ns);
+  // A single sequence: the polled build, where each phase's units have workgroups of their own and the layer table fits LDS beside
+  // the weights of the layer ahead.
+  const size_t smem_one = one_smem_bytes(m);
+  const int ns_d = m->d_model / 16, ns_q = m->n_heads * D / 16, ns_kv = m->n_kv_heads * D / 16;
+  const bool one = s->batch == 1 && smem_one <= 160 * 1024 && (ns_q + 1) / 2 + 2 * ((ns_kv + 1) / 2) <= n_workgroups &&
+                   ns_d <= n_workgroups && (m->d_ff / 16 + 1) / 2 <= n_workgroups && m->n_heads <= n_workgroups;
+  const size_t smem = one ? smem_one : bit_smem_bytes(m, s->batch, ns);
   if (smem > 160 * 1024) return OHARA_ESIZE;
-  dim3 grid(n_workgroups), block(256);
-#define OHARA_BITMEGA_B(DD, ONE_)                                                                            \
-  do {                                                                                                       \
-    if (smem > 64 * 1024)                                                                                    \
-      (void)hipFuncSetAttribute((const void*)bitnet_mega_kernel<DD, 1, ONE_>,                                \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);                      \
-    static ResidencySlot slot;                                                                               \
-    if (!ohara_grid_fits(slot, (const void*)bitnet_mega_kernel<DD, 1, ONE_>, smem, n_workgroups))            \
-      return OHARA_ESIZE; /* the workgroups could not all be resident: the grid barrier would expire */      \
-    hipLaunchKernelGGL((bitnet_mega_kernel<DD, 1, ONE_>), grid, block, smem, st, a);                         \
-  } while (0)
-#define OHARA_BITMEGA(DD)                                                                                    \
-  do {                                                                                                       \
-    if (s->batch == 1) OHARA_BITMEGA_B(DD, true);                                                            \
-    else OHARA_BITMEGA_B(DD, false);                                                                         \
-  } while (0)
-#define OHARA_BITMEGA_PROF(ONE_)                                                                             \
-  do {                                                                                                       \
-    if (smem > 64 * 1024)                                                                                    \
-      (void)hipFuncSetAttribute((const void*)bitnet_mega_kernel<128, 1, ONE_, true>,                         \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);                      \
-    static ResidencySlot slot;                                                                               \
-    if (!ohara_grid_fits(slot, (const void*)bitnet_mega_kernel<128, 1, ONE_, true>, smem, n_workgroups))     \
-      return OHARA_ESIZE;                                                                                    \
-    hipLaunchKernelGGL((bitnet_mega_kernel<128, 1, ONE_, true>), grid, block, smem, st, a);                  \
-  } while (0)
-  if (a.prof && D == 128) {  // the stamps exist in these two instantiations only
-    if (s->batch == 1) OHARA_BITMEGA_PROF(true);
-    else OHARA_BITMEGA_PROF(false);
-  } else if (D == 128) OHARA_BITMEGA(128);
-  else OHARA_BITMEGA(64);
-#undef OHARA_BITMEGA
-#undef OHARA_BITMEGA_B
-#undef OHARA_BITMEGA_PROF
-  return ohara_launch_status();
+  auto launch = [&](auto kernel, ResidencySlot& slot) {
+    if (smem > 64 * 1024) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    // (workgroups that cannot all be resident would be waited for until the spin limit)
+    if (!ohara_grid_fits(slot, (const void*)kernel, smem, n_workgroups)) return OHARA_ESIZE;
+    hipLaunchKernelGGL(kernel, dim3(n_workgroups), dim3(256), smem, st, a);
+    return ohara_launch_status();
+  };
+  static ResidencySlot slots[6];
+  if (a.prof && D == 128)  // the stamps exist in these two instantiations only
+    return one ? launch(bitnet_one_kernel<128, true>, slots[0]) : launch(bitnet_mega_kernel<128, 1, true>, slots[1]);
+  if (D == 128) return one ? launch(bitnet_one_kernel<128>, slots[2]) : launch(bitnet_mega_kernel<128, 1>, slots[3]);
+  return one ? launch(bitnet_one_kernel<64>, slots[4]) : launch(bitnet_mega_kernel<64, 1>, slots[5]);
 }
 
 }  // extern "C"

@@ -1473,14 +1473,16 @@ __device__ __forceinline__ void attn_new_row_i8(const uint32_t* w, int8_t* kq, i
 // I8 (with TAG only): kc / vc are the int8 caches, `stats` their (sequence, KV head, position) records.
 // AHEAD (with TAG only): a wave's second tile is requested before the poll for q (the single-sequence build: with more
 // sequences a chunk is many tiles and the registers the request holds across the poll are spilled).
-template <int D, int G, bool TAG = false, bool I8 = false, bool AHEAD = false>
+// PPOLL (with TAG only): the partials go to a polled mailbox themselves, `other` bytes from its twin in the other set.
+template <int D, int G, bool TAG = false, bool I8 = false, bool AHEAD = false, bool PPOLL = false>
 __device__ __forceinline__ void attn_phase(int B, int H, int Hkv, int Tmax, int blk_x, int ns, const AttnPre<D>& pre,
                                            const char* qm, float* pm, const bf16_t* kc, const bf16_t* vc, int L,
                                            float* lds, const char* qt = nullptr, const char* kvt = nullptr,
                                            const Poll pc = Poll{0, 0, nullptr}, bool announce = false, int q_row = 0,
                                            int kv_row = 0,  // q_row, kv_row: bytes between the sequences' rows of qt, kvt
                                            float* stats = nullptr,
-                                           float* wave_lds = nullptr) {  // TAG: 1 KB of LDS per wave, free during this phase
+                                           float* wave_lds = nullptr,  // TAG: 1 KB of LDS per wave, free during this phase
+                                           ptrdiff_t other = 0) {
   static_assert(!I8 || TAG, "the int8 cache is served by the polled builds");
   constexpr int NC = D / 32, DC = D / 8, PP = 64 / DC, NV = 16 / PP;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1739,9 +1741,12 @@ __device__ __forceinline__ void attn_phase(int B, int H, int Hkv, int Tmax, int 
         o1 += s_acc[(w * G + hh) * D + d + 1] * sc;
       }
       float* dst = pm + ((size_t)(b * H + h) * OHARA_MEGA_NS + split) * PS;
-      st_coh8(dst + d, make_uint2(__float_as_uint(o0), __float_as_uint(o1)));
+      if (PPOLL) mb_st8(reinterpret_cast<char*>(dst), other, 2 * d, __float_as_uint(o0), __float_as_uint(o1));
+      else st_coh8(dst + d, make_uint2(__float_as_uint(o0), __float_as_uint(o1)));
       if (d == 0) {
-        if (TAG && announce) {
+        if (PPOLL) {
+          mb_st8(reinterpret_cast<char*>(dst), other, 2 * D, __float_as_uint(M), __float_as_uint(Ls));
+        } else if (TAG && announce) {
           ann = dst + D;
           ann_m = M;
           ann_l = Ls;
