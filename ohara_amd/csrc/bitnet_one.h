@@ -84,9 +84,10 @@ __device__ __forceinline__ void one_request(uint32_t base, int first, const uint
   for (int c = 0; c0 + c < c1; ++c)
     load_lds16(dst + c * 1024, wp + ((size_t)st * KC + c0 + c) * 64, (threadIdx.x & 63) * 16);
 }
+template <int NP = 1>  // pieces past the row: its last one again, which meets zeros
 __device__ __forceinline__ void one_request_norm(uint32_t base, const bf16_t* w, int pieces) {
   const uint32_t dst = __builtin_amdgcn_readfirstlane(base + (threadIdx.x >> 6) * 1024);
-  for (int i = 0; i * 256 < pieces; ++i)
+  for (int i = 0; i < NP; ++i)
     load_lds16(dst + i * 4096, w, min((int)threadIdx.x + 256 * i, pieces - 1) * 16);
 }
 
@@ -376,7 +377,7 @@ __global__ __launch_bounds__(256) void bitnet_one_kernel(BitMegaArgs a) {
   auto ask5 = [&](int l) {
     if (!has5) return;
     one_request<4, ONE_T5>(t5, 0, weights(l, BD), KCf, i5, true);
-    one_request_norm(n5, norms(ltab[l].nw[BD]), F >> 3);
+    one_request_norm<ONE_N5>(n5, norms(ltab[l].nw[BD]), F >> 3);
   };
   AttnPre<D> apre;
   auto ask_kv = [&](int l) {
@@ -515,12 +516,12 @@ __global__ __launch_bounds__(256) void bitnet_one_kernel(BitMegaArgs a) {
     if (has5) {
       L.shape(1, F);
       const int r0 = i5 * 16 + 4 * gg;
-      uint4 x[3];
-      one_poll<3>(x, xt + bx.act, F >> 3, pc);
+      uint4 x[ONE_N5];
+      one_poll<ONE_N5>(x, xt + bx.act, F >> 3, pc);
       pf.stamp();
       uint2 r = make_uint2(0, 0);
       if (wave == 0) r = ld_coh8(xt + (size_t)r0 * 2);
-      one_codes<3, 1, false>(x, n5, F, m.eps, L, red, s);
+      one_codes<ONE_N5, 1, false>(x, n5, F, m.eps, L, red, s);
       one_leave(one_product<4, ONE_T5, ONE_T5>(t5, 0, KCf, true, L.codes), fold);
       __syncthreads();
       if (wave == 0) {
