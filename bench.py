@@ -566,7 +566,7 @@ def bench_phi(dev):
 # hand-off is polled for, so a step's critical path runs from role to role.
 _GEMM = ["activations in LDS -> MFMAs issued", "cross-wave sum"]
 PHASE_STAMPS = (
-    ["P1 staged"] + ["P1 " + x for x in _GEMM] + ["P1 epilogue", "P2 chunk announced", "P2 requests issued", "P3 merged"]
+    ["P1 staged"] + ["P1 " + x for x in _GEMM] + ["P1 epilogue", "P2 partials stored", "P2 requests issued", "P3 merged"]
     + ["P3 " + x for x in _GEMM] + ["P3 epilogue", "P4 staged"] + ["P4 " + x for x in _GEMM]
     + ["P4 epilogue", "P4 requests issued", "P5 staged"] + ["P5 " + x for x in _GEMM] + ["P5 epilogue", "P5 requests issued"]
 )
@@ -625,8 +625,8 @@ def phase_timeline(dev, prompt_len, steps=32, batch=1, int8=False):
         return float(acc[list(roles[role]), layer * per + idx[name]].max())
 
     chain = [("qkv", "P1 staged", "stream polled for, norm1 in LDS"), ("qkv", "P1 epilogue", "q/k/v product, rotary, q and new k/v rows stored"),
-             ("attention", "P2 chunk announced", "q polled for, chunk, partials stored and announced"),
-             ("wo", "P3 merged", "chunks polled for, partials fetched and merged"), ("wo", "P3 epilogue", "output projection + residual stored"),
+             ("attention", "P2 partials stored", "q polled for, chunk, partials stored"),
+             ("wo", "P3 merged", "heads merged, their rows polled for"), ("wo", "P3 epilogue", "output projection + residual stored"),
              ("gate/up", "P4 staged", "stream polled for, norm2 in LDS"), ("gate/up", "P4 epilogue", "gate/up product, SwiGLU stored"),
              ("down", "P5 staged", "activations polled for, in LDS"), ("down", "P5 epilogue", "down projection + residual stored")]
     seg = torch.zeros(len(chain) + 1, dtype=torch.float64)

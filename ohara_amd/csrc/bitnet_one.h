@@ -232,55 +232,6 @@ __device__ __forceinline__ float one_value(uint2 four) {  // this lane's of four
   return threadIdx.x & 1 ? hi_bf(w) : lo_bf(w);
 }
 
-// The partials of a head's chunks, polled for and merged in chunk order (the sums of stage_attn_merge) -> the head's part of the row.
-template <int D>
-__device__ __forceinline__ void one_merge(const char* part, int ns, float* sm, char* row, ptrdiff_t other, const Poll& pc) {
-  constexpr int CG = D / 4, RG = 256 / CG, R = (OHARA_MEGA_NS + RG - 1) / RG, PS = D + 32;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int c = tid % CG, r = tid / CG;
-  float* sw = sm + OHARA_MEGA_NS * D;  // weights and the sum
-  const MbRsrc rs = mb_rsrc(part);
-  const int sp = lane & 15;            // every wave looks at the (maximum, sum) pairs itself
-  uint4 v[R];
-  u32x2 ml;
-  unsigned int spins = 0;
-  for (;;) {
-    bool ok = true;
-#pragma unroll
-    for (int i = 0; i < R; ++i) ok = mb_ld16(rs, (min(r + i * RG, ns - 1) * PS + c * 4) * 2, v[i]) && ok;
-    ml = __builtin_amdgcn_raw_buffer_load_b64(rs, (uint32_t)(min(sp, ns - 1) * PS + D) * 4u, 0, 16);
-    ok = ok && ml.x != OHARA_UNWRITTEN && ml.y != OHARA_UNWRITTEN;
-    if (__all(ok) || poll_expired(pc, spins)) break;
-  }
-  const float ms = sp < ns ? __uint_as_float(ml.x) : -INFINITY, ls = sp < ns ? __uint_as_float(ml.y) : 0.f;
-  const float M = lane_xor_max<1>(lane_xor_max<2>(lane_xor_max<4>(lane_xor_max<8>(ms))));
-  const float w = (ms == -INFINITY) ? 0.f : pow2_neg_int(ms - M);
-  const float Ls = lane_xor_sum<1>(lane_xor_sum<2>(lane_xor_sum<4>(lane_xor_sum<8>(ls * w))));
-#pragma unroll
-  for (int i = 0; i < R; ++i)
-    if (r + i * RG < ns) sts16(sm + (r + i * RG) * D + c * 4, v[i]);
-  if (tid < 16) sw[tid] = w;
-  if (tid == 0) sw[16] = Ls;
-  __syncthreads();
-  if (tid < D / 2) {
-    float o0 = 0.f, o1 = 0.f, ws[OHARA_MEGA_NS];
-    f32x2_t av[OHARA_MEGA_NS];
-#pragma unroll
-    for (int s = 0; s < OHARA_MEGA_NS; ++s) {
-      ws[s] = sw[s];
-      av[s] = *reinterpret_cast<const f32x2_t*>(sm + min(s, ns - 1) * D + 2 * tid);  // (past the last chunk: again, of weight zero)
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int s = 0; s < OHARA_MEGA_NS; ++s) {
-      o0 += av[s][0] * ws[s];
-      o1 += av[s][1] * ws[s];
-    }
-    const float inv = 1.0f / sw[16];
-    mb_st4(row, other, 2 * tid, pack_bf(o0 * inv, o1 * inv));
-  }
-}
-
 template <int D, bool PROFILE = false>
 __global__ __launch_bounds__(256) void bitnet_one_kernel(BitMegaArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -308,7 +259,7 @@ __global__ __launch_bounds__(256) void bitnet_one_kernel(BitMegaArgs a) {
   OneRed red{reinterpret_cast<float*>(take(64)), 0};
   int* fold = reinterpret_cast<int*>(take(512));  // gate's and up's parts, or one product's
   float* att = reinterpret_cast<float*>(take((size_t)(8 + 4 * D) * sizeof(float)));
-  float* mrg = reinterpret_cast<float*>(take((size_t)(OHARA_MEGA_NS * D + 32) * sizeof(float)));
+  float* mrg = reinterpret_cast<float*>(take(merge_head_lds(D)));
   BitLayerDev* ltab = reinterpret_cast<BitLayerDev*>(take(0));
   {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(a.layers_dev);
@@ -329,7 +280,7 @@ __global__ __launch_bounds__(256) void bitnet_one_kernel(BitMegaArgs a) {
   gs.init(a.bar, nwg, a.spin_limit);
   unsigned int* launches = a.bar + (gs.ng + 12) * 64;
   const unsigned int nth = *launches + 1u;  // the last workgroup out advances it
-  const Poll pc{nth, a.spin_limit, gs.err};
+  const Poll pc{a.spin_limit, gs.err};
   const OneBoxes bx = one_boxes(m);
   const size_t set_bytes = bx.stride * m.n_layers;
   char* const boxes = a.tg + (size_t)(nth & 1u) * set_bytes;
@@ -455,10 +406,10 @@ __global__ __launch_bounds__(256) void bitnet_one_kernel(BitMegaArgs a) {
     }
     pf.stamp();
     // ---- P2: attention partials, then the merge of a head's by one workgroup ----
-    attn_phase<D, 1, true, false, true, true>(1, H, Hkv, m.t_max, 0, a.ns, apre, nullptr, reinterpret_cast<float*>(xt + bx.part), kc, vc, Lc,
-                                              att, xt + bx.q, xt + bx.kv, pc, false, 0, 0, nullptr, L.red, other);
+    attn_phase<D, 1, true, false, true>(1, H, Hkv, m.t_max, 0, a.ns, apre, nullptr, reinterpret_cast<float*>(xt + bx.part), kc, vc, Lc,
+                                              att, xt + bx.q, xt + bx.kv, pc, 0, 0, nullptr, L.red, other);
     pf.stamp();
-    if (merges) one_merge<D>(xt + bx.part + (size_t)ih * OHARA_MEGA_NS * (D + 32) * 4, a.ns, mrg, xt + bx.row + ih * D * 2, other, pc);
+    if (merges) merge_head<D>(xt + bx.part + (size_t)ih * OHARA_MEGA_NS * (D + 32) * 4, a.ns, mrg, xt + bx.row + ih * D * 2, other, pc);
     pf.stamp();
     ask1(l + 1);
     ask5(l);
@@ -590,7 +541,7 @@ size_t one_smem_bytes(const OharaBitModel* m) {
   take(64);
   take(512);
   take((size_t)(8 + 4 * D) * sizeof(float));
-  take((size_t)(OHARA_MEGA_NS * D + 32) * sizeof(float));
+  take(merge_head_lds(D));
   return o + sizeof(BitLayerDev) * m->n_layers;
 }
 

@@ -13,55 +13,6 @@ namespace {
 
 size_t mega_al(size_t v) { return (v + 255) & ~(size_t)255; }
 
-struct MegaLayout {
-  size_t layers, kptr, vptr, sptr, xm, qm, am, pm, dm, candv, candi, prof, bar, tg, total;
-  size_t xm_stride, qm_stride, am_stride, pm_stride, dm_stride, tg_stride, tg_set;
-  int blk_x, blk_a, tg_n, tg_q, tg_kv, tg_a, tg_rx, tg_rq, tg_rkv, tg_ra;
-};
-
-MegaLayout mega_layout(const OharaModel* m, int B, int nwg) {
-  MegaLayout L{};
-  const int NL = m->n_layers, D = m->head_dim;
-  L.blk_x = (B * 32 + 127) / 128 * 128;
-  L.blk_a = (B * 16 + 127) / 128 * 128;
-  const int nq_rows = (m->n_heads + 2 * m->n_kv_heads) * D;
-  L.xm_stride = mega_al((size_t)((m->d_model + 15) / 16) * L.blk_x);
-  L.qm_stride = mega_al((size_t)((nq_rows + 15) / 16) * L.blk_x);
-  L.am_stride = mega_al((size_t)((m->d_ff + 7) / 8) * L.blk_a);
-  L.pm_stride = mega_al((size_t)B * m->n_heads * OHARA_MEGA_NS * (D + 32) * sizeof(float)) / sizeof(float);
-  size_t o = 0;
-  L.layers = o; o += mega_al(sizeof(OharaLayer) * NL);
-  L.kptr = o; o += mega_al(sizeof(void*) * NL);
-  L.vptr = o; o += mega_al(sizeof(void*) * NL);
-  L.sptr = o; o += mega_al(sizeof(void*) * NL);
-  L.xm = o; o += L.xm_stride * NL;
-  L.qm = o; o += L.qm_stride * NL;
-  L.am = o; o += L.am_stride * NL;
-  L.dm_stride = mega_al((size_t)OHARA_DOWN_SPLIT * ((m->d_model + 15) / 16) * ((B * 64 + 127) / 128 * 128)) / sizeof(float);
-  L.dm = o; o += L.dm_stride * sizeof(float) * NL;
-  L.candv = o; o += mega_al((size_t)nwg * B * sizeof(float));
-  L.candi = o; o += mega_al((size_t)nwg * B * sizeof(int));
-  L.prof = o; o += mega_al((size_t)nwg * OHARA_PROF_SLOTS * sizeof(unsigned long long));
-  L.bar = o; o += mega_al(OHARA_BAR_WORDS(nwg) * sizeof(unsigned int));
-  // behind the barrier words, cleared with them: the attention partials (batch 1: a tag follows each (max, sum) pair);
-  // then the two sets of polled mailboxes (batch 1), filled with 0xFF ("not written yet")
-  L.pm = o; o += L.pm_stride * sizeof(float) * NL;
-  L.tg_rx = (int)mega_al((size_t)m->d_model * 2);
-  L.tg_rq = (int)mega_al((size_t)m->n_heads * D * 2);
-  L.tg_rkv = (int)mega_al((size_t)2 * m->n_kv_heads * D * 2);
-  L.tg_ra = (int)mega_al((size_t)((m->d_ff + 7) / 8 * 8) * 2);
-  const int PB = B <= 8 ? B : 1;  // (the polled builds serve up to eight sequences)
-  L.tg_n = PB * L.tg_rx;
-  L.tg_q = 2 * L.tg_n;
-  L.tg_kv = L.tg_q + PB * L.tg_rq;
-  L.tg_a = L.tg_kv + PB * L.tg_rkv;
-  L.tg_stride = L.tg_a + (size_t)PB * L.tg_ra;
-  L.tg_set = L.tg_stride * NL;
-  L.tg = o; o += 2 * L.tg_set;
-  L.total = o;
-  return L;
-}
-
 // What a launch looks like for (model, batch, grid): chunks per (sequence, KV head), which build, its LDS bytes.
 struct MegaPlan {
   int ns, mode;
@@ -88,15 +39,67 @@ MegaPlan mega_plan(const OharaModel* m, int batch, int n_workgroups) {
   // The polled builds (batch 1; up to eight sequences) park the down projection's tiles in LDS (4 waves x
   // OHARA_LDS_PF KB) and want gate/up, the output projection and the down projection on workgroups of their own.
   const int n_dn = (m->d_model + 15) / 16, n_gu = (2 * ((m->d_ff + 7) / 8 * 8) / 16 + 1) / 2;
-  const size_t smem0 = xs_bytes + 4096 + (size_t)(8 + 4 * D) * G * sizeof(float) + mrg + (size_t)m->n_layers * 72;
-  const size_t smem_polled = smem0 + 256 + (size_t)4 * OHARA_LDS_PF * 1024;
+  const size_t rest = 4096 + (size_t)(8 + 4 * D) * G * sizeof(float) + (size_t)m->n_layers * 72;
+  const size_t smem0 = xs_bytes + rest + mrg;
+  const size_t merge_bytes = (merge_head_lds(D) + 255) & ~(size_t)255, smem1 = (xs_bytes > merge_bytes ? xs_bytes : merge_bytes) + rest;
+  const size_t smem_polled = smem1 + 256 + (size_t)4 * OHARA_LDS_PF * 1024;
   const bool roles = n_gu + n_dn <= n_workgroups && 2 * n_dn <= n_workgroups;
   const int mode = !roles ? 0 : (batch == 1 ? 1 : (batch <= 8 && smem_polled <= 160 * 1024 ? 2 : 0));
   // A single sequence leaves LDS free: the workgroups that park their waves' second vocabulary strip add half of the
   // third (12 more tiles per wave) where that fits.
-  const size_t smem_more = smem0 + 256 + (size_t)4 * (OHARA_LDS_PF + 12) * 1024;
+  const size_t smem_more = smem1 + 256 + (size_t)4 * (OHARA_LDS_PF + 12) * 1024;
   if (mode == 1 && smem_more <= 160 * 1024) return MegaPlan{ns, 1, smem_more, OHARA_LDS_PF + 12};
   return MegaPlan{ns, mode, mode ? smem_polled : smem0, OHARA_LDS_PF};
+}
+
+struct MegaLayout {
+  size_t layers, kptr, vptr, sptr, xm, qm, am, pm, dm, candv, candi, prof, bar, tg, total;
+  size_t xm_stride, qm_stride, am_stride, pm_stride, dm_stride, tg_stride, tg_set;
+  int blk_x, blk_a, tg_n, tg_q, tg_kv, tg_a, tg_m, tg_p, tg_rx, tg_rq, tg_rkv, tg_ra;
+};
+
+MegaLayout mega_layout(const OharaModel* m, int B, int nwg) {
+  MegaLayout L{};
+  const int NL = m->n_layers, D = m->head_dim;
+  L.blk_x = (B * 32 + 127) / 128 * 128;
+  L.blk_a = (B * 16 + 127) / 128 * 128;
+  const int nq_rows = (m->n_heads + 2 * m->n_kv_heads) * D;
+  L.xm_stride = mega_al((size_t)((m->d_model + 15) / 16) * L.blk_x);
+  L.qm_stride = mega_al((size_t)((nq_rows + 15) / 16) * L.blk_x);
+  L.am_stride = mega_al((size_t)((m->d_ff + 7) / 8) * L.blk_a);
+  L.pm_stride = mega_al((size_t)B * m->n_heads * OHARA_MEGA_NS * (D + 32) * sizeof(float)) / sizeof(float);
+  size_t o = 0;
+  L.layers = o; o += mega_al(sizeof(OharaLayer) * NL);
+  L.kptr = o; o += mega_al(sizeof(void*) * NL);
+  L.vptr = o; o += mega_al(sizeof(void*) * NL);
+  L.sptr = o; o += mega_al(sizeof(void*) * NL);
+  const bool polled = mega_plan(m, B, nwg).mode != 0;  // the polled builds have mailboxes of their own
+  L.xm = o; o += polled ? 0 : L.xm_stride * NL;
+  L.qm = o; o += polled ? 0 : L.qm_stride * NL;
+  L.am = o; o += polled ? 0 : L.am_stride * NL;
+  L.pm = o; o += polled ? 0 : L.pm_stride * sizeof(float) * NL;
+  L.dm_stride = mega_al((size_t)OHARA_DOWN_SPLIT * ((m->d_model + 15) / 16) * ((B * 64 + 127) / 128 * 128)) / sizeof(float);
+  L.dm = o; o += polled ? 0 : L.dm_stride * sizeof(float) * NL;
+  L.candv = o; o += mega_al((size_t)nwg * B * sizeof(float));
+  L.candi = o; o += mega_al((size_t)nwg * B * sizeof(int));
+  L.prof = o; o += mega_al((size_t)nwg * OHARA_PROF_SLOTS * sizeof(unsigned long long));
+  L.bar = o; o += mega_al(OHARA_BAR_WORDS(nwg) * sizeof(unsigned int));
+  // then the two sets of polled mailboxes, filled with 0xFF ("not written yet")
+  L.tg_rx = (int)mega_al((size_t)m->d_model * 2);
+  L.tg_rq = (int)mega_al((size_t)m->n_heads * D * 2);
+  L.tg_rkv = (int)mega_al((size_t)2 * m->n_kv_heads * D * 2);
+  L.tg_ra = (int)mega_al((size_t)((m->d_ff + 7) / 8 * 8) * 2);
+  L.tg_n = B * L.tg_rx;
+  L.tg_q = 2 * L.tg_n;
+  L.tg_kv = L.tg_q + B * L.tg_rq;
+  L.tg_a = L.tg_kv + B * L.tg_rkv;
+  L.tg_m = L.tg_a + B * L.tg_ra;
+  L.tg_p = L.tg_m + B * L.tg_rq;
+  L.tg_stride = L.tg_p + mega_al((size_t)B * m->n_heads * OHARA_MEGA_NS * (D + 32) * sizeof(float));
+  L.tg_set = L.tg_stride * NL;
+  L.tg = o; o += polled ? 2 * L.tg_set : 0;
+  L.total = o;
+  return L;
 }
 
 }  // namespace
@@ -156,6 +159,7 @@ int ohara_llama_decode_persistent(const OharaModel* m, const OharaDecodeState* s
   a.cand_idx = reinterpret_cast<int*>(ws + L.candi);
   a.bar = reinterpret_cast<unsigned int*>(ws + L.bar);
   a.tg = ws + L.tg; a.tg_stride = L.tg_stride; a.tg_set = L.tg_set; a.tg_n = L.tg_n; a.tg_q = L.tg_q; a.tg_kv = L.tg_kv; a.tg_a = L.tg_a;
+  a.tg_m = L.tg_m; a.tg_p = L.tg_p;
   a.tg_rx = L.tg_rx; a.tg_rq = L.tg_rq; a.tg_rkv = L.tg_rkv; a.tg_ra = L.tg_ra;
   if (init_workspace) {
     // small synchronous copies: done once per (model, cache) binding, outside any capture
@@ -168,7 +172,7 @@ int ohara_llama_decode_persistent(const OharaModel* m, const OharaDecodeState* s
         (s->kv_int8 && hipMemcpyAsync((void*)a.kvstats_dev, s->kvstats, sizeof(void*) * m->n_layers,
                                       hipMemcpyHostToDevice, st) != hipSuccess) ||
         hipMemsetAsync((void*)a.bar, 0, L.tg - L.bar, st) != hipSuccess ||
-        hipMemsetAsync((void*)a.tg, 0xFF, L.total - L.tg, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
+        (L.total > L.tg && hipMemsetAsync((void*)a.tg, 0xFF, L.total - L.tg, st) != hipSuccess) || hipStreamSynchronize(st) != hipSuccess)
       return OHARA_ELAUNCH;
     return OHARA_OK;
   }

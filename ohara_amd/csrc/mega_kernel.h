@@ -29,12 +29,14 @@
 // The one exception is the KV-cache row appended in this step (its lines are shared by
 // several writers): attention reads that single row with device-scope loads.
 //
-// Batch 1 (the ONE builds): three of the five hand-offs of a layer carry one short row - the q row and
-// the new key / value rows (P1 -> P2), the residual stream (P3 -> P4), the activations (P4 -> P5) - and
-// go through TAGGED mailboxes that the consumers poll for (persistent.h) instead of a barrier; two grid
-// barriers per layer remain (after the attention partials, after the down projection's sums).  The
-// weights of P4 and P5 are requested around the first of them, where a workgroup is idle anyway, so that
-// no weight load is in flight ahead of a poll (a wave's loads return in order).
+// The polled builds (batch 1, and up to eight sequences) have no grid barrier inside the layers: every hand-off is a row in a mailbox
+// whose words the consumers poll for (persistent.h).  So are the attention partials: one workgroup a (sequence, head) polls for its
+// chunks', merges them and hands on the head's part of the row.  (Before, a chunk waited for its own stores, then announced them, and
+// each of the 48 workgroups of the output projection read all partials, 49 KB a sequence: d12 layers at context 1050 took 14.6 us at
+// batch 1, 26.5 at 8, 16.6 over an int8 cache; 14.2, 24.7 and 16.3 now, with gate/up's weights where they delay nobody's chunk.
+// Replies of 40 tokens behind 700: batch 2 9.63 -> 9.09 ms, 8 14.7 -> 13.95, 6 over an int8 cache 15.5 -> 15.0; 64 behind 1024 at batch 1
+// 13.3 -> 13.0; one sequence over an int8 cache 9.01 -> 9.10: its last chunk quantises the new row and hid the wait for the stores.)
+// Weights are requested where a workgroup is idle, so that no weight load is in flight ahead of a poll (a wave's loads return in order).
 //
 // Every barrier wait is bounded: a workgroup that spins longer than the limit raises a
 // sticky error word and moves on, all later waits return at once, and the grid drains.
@@ -68,7 +70,8 @@ struct MegaArgs {
   int64_t* history;
   char* tg;             // batch 1: two sets of NL blocks of polled mailboxes, tg_stride bytes a block, tg_set bytes a set
   size_t tg_stride, tg_set;
-  int tg_n, tg_q, tg_kv, tg_a;  // byte offsets inside a layer's block: stream after the layer | q | new k, v | activations
+  int tg_n, tg_q, tg_kv, tg_a, tg_m, tg_p;  // byte offsets inside a layer's block: stream after the layer | q | new k, v | activations | merged
+                                            // attention rows | attention partials ([b*H + h][chunk][Dh + 32] floats)
   int tg_rx, tg_rq, tg_rkv, tg_ra;  // bytes between the sequences' rows of those mailboxes
   unsigned int* bar;    // barrier words, see GridSync
   unsigned long long* prof;  // optional: clock of every workgroup's thread 0 at every phase boundary (OHARA_PROF_SLOTS each)
@@ -95,13 +98,16 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
   const int kmax = max(d, max(F, H * D));
   const int ldxs = kmax + 8;
   bf16_t* xs = reinterpret_cast<bf16_t*>(smem);
-  float* red = reinterpret_cast<float*>(smem + (((size_t)B * ldxs * 2 + 255) & ~(size_t)255));  // 4 KiB
+  // (polled builds: a workgroup that merges a head's partials does it where it stages rows)
+  const size_t xs_bytes = ((max((size_t)B * ldxs * 2, POLLED ? merge_head_lds(D) : 0)) + 255) & ~(size_t)255;
+  float* red = reinterpret_cast<float*>(smem + xs_bytes);  // 4 KiB
   float* att = red + 1024;                                                                      // (8 + 4*D)*G floats
   // per-layer pointers (6 weights/norms + K and V cache), copied once to LDS so that no phase
   // starts with a chain of dependent global loads
-  float* mrg_w = att + (8 + 4 * D) * G;       // B*H*ns chunk weights
-  float* mrg_l = mrg_w + ((B * H * attn_merge_width(a.ns) + 1) & ~1);  // B*H*(merge width) chunk weights before it
-  unsigned long long* ptab = reinterpret_cast<unsigned long long*>(mrg_l + ((B * H * attn_merge_width(a.ns) + 1) & ~1));
+  const int mrg = POLLED ? 0 : (B * H * attn_merge_width(a.ns) + 1) & ~1;
+  float* mrg_w = att + (8 + 4 * D) * G;       // B*H*(merge width) chunk weights
+  float* mrg_l = mrg_w + mrg;                 // and their sums
+  unsigned long long* ptab = reinterpret_cast<unsigned long long*>(mrg_l + mrg);
   // (polled builds: the ids of the rows this wave embeds are the first thing requested - their rows are what the first
   // layer's q/k/v workgroups wait for, and a wave's loads return in the order they were issued)
   // (the single-sequence build only: with more rows the registers this holds across the prefetches are spilled)
@@ -157,7 +163,7 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
   if constexpr (POLLED) {
    {
     // ---- polled hand-offs, no grid barrier inside the layers ------------------------------------------
-    const Poll pc{nth, a.spin_limit, gs.err};
+    const Poll pc{a.spin_limit, gs.err};
     const int nwg = (int)gridDim.x;
     // this launch's set of mailboxes, and the way from there to the other set
     char* const tgs = a.tg + (size_t)(nth & 1u) * a.tg_set;
@@ -167,9 +173,11 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
     // (a CU takes in ~55 GB/s) - so the phases are spread over the grid such that a workgroup's next
     // weights can be on their way while it has nothing else to do, long before the poll that precedes
     // their use (a wave's loads return in order: a poll issued behind a batch of weights comes back after
-    // it).  Attention chunks, the output projection and gate/up start at workgroup 0; q/k/v sits at the far
-    // end; the down projection (whole K per strip: 24 k-step tiles per wave from LDS, no partial sums)
-    // follows the output projection, clear of the workgroups that the next layer starts on.
+    // it).  Attention chunks, the output projection and gate/up start at workgroup 0; q/k/v and the down projection (whole K per
+    // strip: 24 k-step tiles per wave from LDS, no partial sums) end with the grid, the latter clear of gate/up, so that its
+    // workgroups have nothing to request between its stores and the next layer's stream.  (Behind the output projection, on
+    // workgroups with attention chunks, those were 0.5 us late each layer: their first tiles came behind 72 KB of weights.)  The heads'
+    // partials are merged just below the down projection, by workgroups that have had their part with q/k/v.
     dn.nstrips = (d + 15) / 16;
     qkv.wg0 = max(0, nwg - qkv.nstrips);
     dn.wg0 = prj.nstrips + dn.nstrips <= nwg ? prj.nstrips : max(0, nwg - dn.nstrips);
@@ -177,17 +185,20 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
     const bool has_attn = (int)blockIdx.x < n_chunks;
     const bool has_dn = phase_block(dn) < dn.nstrips;
     const bool has_qkv = phase_block(qkv) < qkv.nstrips;
+    const bool has_gu = phase_block(gu) * 2 < gu.nstrips;
+    // Gate/up's weights (72 KB a workgroup) are requested behind the attention phase by the workgroups of the down projection: between its
+    // stores and the next layer's first tiles they made those workgroups' chunks 0.5 us late.  A single sequence: by all (registers:
+    // where one kernel holds both places it spills over an int8 cache).
+    const bool gate_late = ONE || has_dn;
     qkv.kv_i8 = I8;  // (the attention phase quantises the appended row itself)
     // ahead of the first layer: gate/up and output projection weights, the first K/V tile, q/k/v weights
     // (q/k/v last: its prefetch leaves norm1's weights in pre.g and the rotary pair in pre.r)
     prj.tout = tgs;  // (marks the polled mode for the prefetch: the residual is fetched by the phase itself)
-    gu.wp = lds_ptr<const uint4>(ptab, 2); gu.norm_w = lds_ptr<const bf16_t>(ptab, 5);
     uint4 g1[2], g2[2];  // norm1's and norm2's weights, the rotary pair: each prefetch writes its own
     uint2 r1, r_unused;
     if constexpr (ONE) {
       if (has_qkv) embed_request_rows<2>(m.token_emb, V, d, emb);  // (ahead of the weights: see above)
     }
-    gemm_prefetch<2, 12, E_SWIGLU, 6>(gu, pre, B, g2, r_unused);
     prj.wp = lds_ptr<const uint4>(ptab, 1);
     gemm_prefetch<4, 6, E_RESID, 18>(prj, pre, B, g2, r_unused);
     gemm_prefetch<4, 6, E_ROPE>(qkv, pre, B, g1, r1);
@@ -211,25 +222,24 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
     for (int l = 0; l < m.n_layers; ++l) {
       auto lm_stage = [&]() {
         if (!lm_staged) return;
-        const int c0 = l * lm_per, c1 = min(lm_tiles, c0 + lm_per);
-        char* dst = wl + ((size_t)(threadIdx.x >> 6) * lm_park + c0) * 1024;
+        const int c0 = __builtin_amdgcn_readfirstlane(l * lm_per), c1 = __builtin_amdgcn_readfirstlane(min(lm_tiles, l * lm_per + lm_per));
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lm_staged_addr);
+        const int strip1 = __builtin_amdgcn_readfirstlane(lm_strip1), strip2 = __builtin_amdgcn_readfirstlane(lm_strip2);
 #pragma unroll 1
         for (int c = c0; c < c1; ++c) {  // tile c of the second strip, then (a single sequence) tile c - KSL of the third
           const bool third = ONE && !I8 && !PROFILE && c >= KSL;
-          const uint4* src = lm.wp + ((size_t)(third ? lm_strip2 : lm_strip1) * KSL + (third ? c - KSL : c)) * 64 + (threadIdx.x & 63);
-          __builtin_amdgcn_global_load_lds((const OHARA_GLOBAL void*)src, (OHARA_LDS void*)dst, 16, 0, 0);
-          dst += 1024;
+          load_lds16(dst + c * 1024, lm.wp + ((size_t)(third ? strip2 : strip1) * KSL + (third ? c - KSL : c)) * 64, (threadIdx.x & 63) * 16);
         }
       };
       const unsigned long long* pl = ptab + l * 8;
       bf16_t* kc = lds_ptr<bf16_t>(pl, 6);
       bf16_t* vc = lds_ptr<bf16_t>(pl, 7);
-      float* p_l = a.pm + (size_t)l * a.pm_stride;
       char* xt = tgs + (size_t)l * a.tg_stride;    // the stream after the attention block
       char* xn = xt + a.tg_n;                       // the stream after the layer
       char* qt = xt + a.tg_q;
       char* kvt = xt + a.tg_kv;
       char* at = xt + a.tg_a;
+      char* mt = xt + a.tg_m;
       const char* xn_prev = xn - a.tg_stride;       // (l > 0)
       const bool more = l + 1 < m.n_layers;
       // the first K/V tile of this workgroup's attention chunk (the attention workgroups have no q/k/v strip: nothing
@@ -246,11 +256,22 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
       pre.r = r1;
       gemm_phase<4, 6, E_ROPE, ProfT<PROFILE>, 0, true>(qkv, pre, xs, ldxs, B, red, best_v, best_i, pf);  // 2 stamps
       pf.stamp();  // 4: rotary epilogue, tagged stores issued
-      // P2: attention partials (polls for q; the chunk that holds the new position polls for its k / v rows); each chunk
-      // leaves the launch's tag behind its (max, sum) pair
-      attn_phase<D, G, true, I8, ONE>(B, H, Hkv, m.t_max, a.blk_x, a.ns, apre, nullptr, p_l, kc, vc, L, att, qt, kvt, pc, true,
-                                 a.tg_rq, a.tg_rkv, I8 ? lds_ptr<float>(stab, l) : nullptr, red);
-      pf.stamp();  // 5: partials stored, flag raised
+      // P2: attention partials (polls for q; the chunk that holds the new position polls for its k / v rows)
+      attn_phase<D, G, true, I8, ONE>(B, H, Hkv, m.t_max, a.blk_x, a.ns, apre, nullptr, reinterpret_cast<float*>(xt + a.tg_p), kc, vc, L, att,
+                                 qt, kvt, pc, a.tg_rq, a.tg_rkv, I8 ? lds_ptr<float>(stab, l) : nullptr, red, qkv.tother);
+      pf.stamp();  // 5: partials stored
+      // ... and their merge
+      for (int u = nwg - 1 - (int)blockIdx.x; u < B * H; u += nwg) {
+        const int b = u / H, h = u - b * H;
+        merge_head<D>(xt + a.tg_p + (size_t)u * OHARA_MEGA_NS * (D + 32) * 4, a.ns, reinterpret_cast<float*>(xs), mt + (size_t)b * a.tg_rq + h * D * 2,
+                      qkv.tother, pc);
+        __syncthreads();
+      }
+      auto gate_weights = [&](int from) {
+        gu.wp = lds_ptr<const uint4>(pl, 2 + from); gu.norm_w = lds_ptr<const bf16_t>(pl, 5 + from);
+        gemm_prefetch<2, 12, E_SWIGLU, 6>(gu, pre, B, g2, r_unused);
+      };
+      if (gate_late || l == 0) gate_weights(0);
       // the next layer's q/k/v weights (+ norm1's, the rotary pair): their registers are free again (behind the attention
       // phase, which needs many: a workgroup without a chunk - at the usual sizes those with q/k/v strips - is here at once)
       if (has_qkv && more) {
@@ -261,35 +282,27 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
       if (has_qkv) lm_stage();  // (the next thing a q/k/v workgroup polls for is a phase or more away)
       // the down projection's weights (98 KB a workgroup) into LDS: on their way from here, used after P4
       dn.wp = lds_ptr<const uint4>(pl, 3); dn.tout = xn; dn.tresid = xt; dn.trow = dn.tres_row = a.tg_rx;
-      if (has_dn) {
-        // (not before the chunk's flag has reached memory: behind the other waves' 72 KB of requests it was seen 1.5 us late)
-        if (has_attn) {
-          wait_own_stores();
-          __syncthreads();
-        }
-        gemm_prefetch_lds<4, E_XNEXT>(dn, wl);
-      }
+      if (has_dn) gemm_prefetch_lds<4, E_XNEXT>(dn, wl);
       pf.stamp();  // 6: requests issued
-      // P3: polls for every chunk's tag; merge + output projection + residual
+      // P3: polls for the merged rows, output projection + residual
       prj.tout = xt; prj.tresid = l > 0 ? xn_prev : nullptr; prj.resid_embed = l == 0; prj.trow = prj.tres_row = a.tg_rx;
-      if ((int)blockIdx.x < prj.nstrips) stage_attn_merge_any<!ONE, true>(a.ns, xs, ldxs, p_l, B, H, D, mrg_w, mrg_l, pc);
+      if ((int)blockIdx.x < prj.nstrips) stage_act_tagged(xs, mt, pc, 0, H * D, B, ldxs, a.tg_rq);
       __syncthreads();
-      pf.stamp();  // 7: merge in LDS
+      pf.stamp();  // 7: merged rows in LDS
       gemm_phase<4, 6, E_RESID, ProfT<PROFILE>, 18, true>(prj, pre, xs, ldxs, B, red, best_v, best_i, pf);  // 2 stamps
       pf.stamp();  // 10: residual epilogue
       // P4: polls for the stream, norm2 + gate/up + SwiGLU; the activations are left tagged
       gu.out = nullptr; gu.tout = at; gu.trow = a.tg_ra;
-      if (phase_block(gu) * 2 < gu.nstrips) stage_norm_tagged<2>(xs, xt, pc, m.eps, d, g2, B, ldxs, a.tg_rx);
+      if (has_gu) stage_norm_tagged<2>(xs, xt, pc, m.eps, d, g2, B, ldxs, a.tg_rx);
       __syncthreads();
       pf.stamp();  // 11: stream polled for + norm2 in LDS
       gemm_phase<2, 12, E_SWIGLU, ProfT<PROFILE>, 6, true>(gu, pre, xs, ldxs, B, red, best_v, best_i, pf);  // 2 stamps
       // What the next layer needs of this workgroup besides q/k/v is requested now, a phase and a half before its use:
-      // output projection and gate/up weights (+ norm2's); after the last layer, the vocabulary projection's first tiles.
+      // output projection and (not behind attention) gate/up weights (+ norm2's); after the last layer, the vocabulary projection's first tiles.
       // (the workgroups of the down projection do this after it: the wait for their LDS tiles would wait for these too)
       auto next_weights = [&]() {
         if (more) {
-          gu.wp = lds_ptr<const uint4>(pl, 10); gu.norm_w = lds_ptr<const bf16_t>(pl, 13);
-          gemm_prefetch<2, 12, E_SWIGLU, 6>(gu, pre, B, g2, r_unused);
+          if (!gate_late) gate_weights(8);
           prj.wp = lds_ptr<const uint4>(pl, 9);
           gemm_prefetch<4, 6, E_RESID, 18>(prj, pre, B, g2, r_unused);
         } else {

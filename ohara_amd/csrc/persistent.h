@@ -3,7 +3,7 @@
 // strips, and the split-context attention phase.  Included by the kernels that are built from them
 // (the bf16 Llama step and the BitNet ternary step); everything here is file-local to its includer.
 #pragma once
-#include "common.h"
+#include "lds_tile.h"
 
 // Host side: can `n_workgroups` workgroups of `kernel` (256 threads, `smem` bytes of dynamic LDS) be
 // resident on the current device at the same time?  The grid barrier of the persistent kernels needs
@@ -188,11 +188,11 @@ __device__ __forceinline__ float dot8m(uint4 a, uint4 b, float s) {
 // the number of pollers.  That is against ~1.6 us for a grid barrier plus the producers' wait for
 // their stores before it plus fetching the data cold.  Every poll loop is bounded like the barrier's
 // spins.  Only worth it where a consumer needs little (a row, a head's 128 values).
-// The attention partials (fp32, 48 KB per consumer) go another way: see stage_attn_merge.
+// The attention partials (fp32) travel the same way to one workgroup a head, which merges them (merge_head): a chunk's are then
+// neither waited for by their writer before it may announce them nor read by every consumer of the row.
 // ---------------------------------------------------------------------------------------
 #define OHARA_UNWRITTEN 0xFFFFFFFFu
 struct Poll {
-  uint32_t tag;   // the number of this launch since the workspace was cleared
   unsigned int limit;
   unsigned int* err;
 };
@@ -566,7 +566,8 @@ __device__ __forceinline__ void stage_act_fly(bf16_t* xs, const char* at, const 
 __device__ __forceinline__ void stage_act_tagged(bf16_t* xs, const char* at, const Poll& pc, int f0, int f1, int B = 1,
                                                  int ldxs = 0, int row_bytes = 0) {
   const int n8 = (f1 - f0) >> 3, total = B * n8;
-  if (total <= 2 * (int)blockDim.x) stage_act_fly<2>(xs, at, pc, f0, n8, total, ldxs, row_bytes);
+  if (total <= (int)blockDim.x) stage_act_fly<1>(xs, at, pc, f0, n8, total, ldxs, row_bytes);
+  else if (total <= 2 * (int)blockDim.x) stage_act_fly<2>(xs, at, pc, f0, n8, total, ldxs, row_bytes);
   else stage_act_fly<6>(xs, at, pc, f0, n8, total, ldxs, row_bytes);
 }
 
@@ -577,13 +578,9 @@ __device__ __forceinline__ void stage_act_tagged(bf16_t* xs, const char* at, con
 // columns per pass and issues the accumulator loads of 16 / NS passes - 16 loads - before it uses
 // any, so the number of dependent load rounds does not grow with the chunk count times the batch.
 // `mw`: B*H*NS floats, `ml`: B*H floats of LDS.
-// TAGGED (batch-1 kernels without a barrier ahead of the merge): a chunk's maximum and sum are stored as
-// {max, tag, sum, tag} - each value in one 8-byte word with the tag of the launch - once the chunk's accumulators
-// have reached memory; they are polled for, one lane per chunk, and the accumulators are fetched only after
-// every chunk of the workgroup has been seen.
-template <int NS, bool TAGGED = false>  // NS: a power of two; `used` <= NS chunks hold partials (the others weigh nothing)
+template <int NS>  // NS: a power of two; `used` <= NS chunks hold partials (the others weigh nothing)
 __device__ __forceinline__ void stage_attn_merge(bf16_t* xs, int ldxs, const float* pm, int B, int H, int Dh, float* mw_, float* ml_,
-                                                 int used = NS, const Poll pc = Poll{0, 0, nullptr}) {
+                                                 int used = NS) {
   constexpr int NSM = OHARA_MEGA_NS, PR = 16 / NS;
   const int HD = H * Dh, PS = Dh + 32;
   const int nbh = B * H, total = B * HD;
@@ -604,7 +601,7 @@ __device__ __forceinline__ void stage_attn_merge(bf16_t* xs, int ldxs, const flo
   };
   // the accumulator loads of the first round go out first: they do not depend on the chunk
   // weights, which are formed while they are in flight
-  if (!TAGGED) load((int)threadIdx.x * 4);
+  load((int)threadIdx.x * 4);
   // NS lanes per (sequence, head): lane sp holds chunk sp's (max, sum); max and weighted sum by
   // shuffles inside the group
   for (int i0 = 0; i0 < nbh * NS; i0 += blockDim.x) {
@@ -613,18 +610,9 @@ __device__ __forceinline__ void stage_attn_merge(bf16_t* xs, int ldxs, const flo
     const bool in = bh < nbh && sp < used;
     float ms = -INFINITY, ls = 0.f;
     if (in) {
-      if (TAGGED) {
-        uint4 v;
-        unsigned int spins = 0;
-        do v = ld_coh16(pm + ((size_t)bh * NSM + sp) * PS + Dh);  // {max, tag}, {sum, tag}: two 8-byte loads
-        while ((v.y != pc.tag || v.w != pc.tag) && !poll_expired(pc, spins));
-        ms = __uint_as_float(v.x);
-        ls = __uint_as_float(v.z);
-      } else {
-        const uint2 v = ldg8(pm + ((size_t)bh * NSM + sp) * PS + Dh);
-        ms = __uint_as_float(v.x);
-        ls = __uint_as_float(v.y);
-      }
+      const uint2 v = ldg8(pm + ((size_t)bh * NSM + sp) * PS + Dh);
+      ms = __uint_as_float(v.x);
+      ls = __uint_as_float(v.y);
     }
     float M = ms;
     if (NS > 8) M = lane_xor_max<8>(M);
@@ -641,9 +629,8 @@ __device__ __forceinline__ void stage_attn_merge(bf16_t* xs, int ldxs, const flo
     if (in && sp == 0) ml[bh] = Ls;
   }
   __syncthreads();
-  asm volatile("" ::: "memory");  // compiler only (TAGGED): the accumulator loads stay behind the polls
   for (int e0 = threadIdx.x * 4; e0 < total; e0 += pass * PR) {
-    if (TAGGED || e0 != (int)threadIdx.x * 4) load(e0);
+    if (e0 != (int)threadIdx.x * 4) load(e0);
 #pragma unroll
     for (int r = 0; r < PR; ++r) {
       const int e = e0 + r * pass;
@@ -703,10 +690,10 @@ __device__ __forceinline__ void stage_attn_merge_small(bf16_t* xs, int ldxs, con
 }
 
 // Out-of-line copies of the merge, for kernels that want to keep their own code compact.
-template <int NS, bool TAGGED = false>
+template <int NS>
 __device__ __noinline__ void stage_attn_merge_call(bf16_t* xs, int ldxs, const float* pm, int B, int H, int Dh, float* mw,
-                                                   float* ml, int used, uint32_t tag = 0, unsigned int limit = 0, unsigned int* err = nullptr) {
-  stage_attn_merge<NS, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, used, Poll{tag, limit, err});  // (a struct would travel through memory)
+                                                   float* ml, int used) {
+  stage_attn_merge<NS>(xs, ldxs, pm, B, H, Dh, mw, ml, used);
 }
 
 // The power of two that the merge of `ns` chunks is specialised for (the chunk weights in LDS are laid
@@ -722,27 +709,75 @@ __host__ __device__ inline int attn_merge_width(int ns) {
 // caller (no call in the layer loop: a call makes the caller wait for every load it has in flight, the
 // weights fetched ahead included); otherwise they stay outside it, which keeps a kernel whose usual case
 // is the small merge within the instruction cache.
-template <bool INLINE, bool TAGGED = false>
+template <bool INLINE>
 __device__ __forceinline__ void stage_attn_merge_any(int ns, bf16_t* xs, int ldxs, const float* pm, int B, int H, int Dh,
-                                                     float* mw, float* ml, const Poll pc = Poll{0, 0, nullptr}) {
+                                                     float* mw, float* ml) {
   const int w = attn_merge_width(ns);
-  if (!TAGGED && ns == OHARA_MEGA_NS && B * H * Dh <= 4 * 256) {  // (TAGGED: one lane polls one chunk's pair)
+  if (ns == OHARA_MEGA_NS && B * H * Dh <= 4 * 256) {
     stage_attn_merge_small(xs, ldxs, pm, B, H, Dh);
-  } else if (TAGGED && w == 16) {
-    // the usual width at batch 1, inline: a call would park the caller's prefetched weights in scratch memory
-    stage_attn_merge<16, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc);
   } else if (INLINE) {
-    if (w == 16) stage_attn_merge<16, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc);
-    else if (w == 8) stage_attn_merge<8, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc);
-    else if (w == 4) stage_attn_merge<4, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc);
-    else if (w == 2) stage_attn_merge<2, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc);
-    else stage_attn_merge<1, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc);
+    if (w == 16) stage_attn_merge<16>(xs, ldxs, pm, B, H, Dh, mw, ml, ns);
+    else if (w == 8) stage_attn_merge<8>(xs, ldxs, pm, B, H, Dh, mw, ml, ns);
+    else if (w == 4) stage_attn_merge<4>(xs, ldxs, pm, B, H, Dh, mw, ml, ns);
+    else if (w == 2) stage_attn_merge<2>(xs, ldxs, pm, B, H, Dh, mw, ml, ns);
+    else stage_attn_merge<1>(xs, ldxs, pm, B, H, Dh, mw, ml, ns);
   } else {
-    if (w == 16) stage_attn_merge_call<16, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc.tag, pc.limit, pc.err);
-    else if (w == 8) stage_attn_merge_call<8, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc.tag, pc.limit, pc.err);
-    else if (w == 4) stage_attn_merge_call<4, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc.tag, pc.limit, pc.err);
-    else if (w == 2) stage_attn_merge_call<2, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc.tag, pc.limit, pc.err);
-    else stage_attn_merge_call<1, TAGGED>(xs, ldxs, pm, B, H, Dh, mw, ml, ns, pc.tag, pc.limit, pc.err);
+    if (w == 16) stage_attn_merge_call<16>(xs, ldxs, pm, B, H, Dh, mw, ml, ns);
+    else if (w == 8) stage_attn_merge_call<8>(xs, ldxs, pm, B, H, Dh, mw, ml, ns);
+    else if (w == 4) stage_attn_merge_call<4>(xs, ldxs, pm, B, H, Dh, mw, ml, ns);
+    else if (w == 2) stage_attn_merge_call<2>(xs, ldxs, pm, B, H, Dh, mw, ml, ns);
+    else stage_attn_merge_call<1>(xs, ldxs, pm, B, H, Dh, mw, ml, ns);
+  }
+}
+
+// LDS of merge_head.
+__host__ __device__ inline size_t merge_head_lds(int D) { return (size_t)(OHARA_MEGA_NS * D + 32) * sizeof(float); }
+// The partials of a head's chunks, polled for and merged in chunk order (the sums of stage_attn_merge) -> the head's part of the row.
+template <int D>
+__device__ __forceinline__ void merge_head(const char* part, int ns, float* sm, char* row, ptrdiff_t other, const Poll& pc) {
+  constexpr int CG = D / 4, RG = 256 / CG, R = (OHARA_MEGA_NS + RG - 1) / RG, PS = D + 32;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int c = tid % CG, r = tid / CG;
+  float* sw = sm + OHARA_MEGA_NS * D;  // weights and the sum
+  const MbRsrc rs = mb_rsrc(part);
+  const int sp = lane & 15;            // every wave looks at the (maximum, sum) pairs itself
+  uint4 v[R];
+  u32x2 ml;
+  unsigned int spins = 0;
+  for (;;) {
+    bool ok = true;
+#pragma unroll
+    for (int i = 0; i < R; ++i) ok = mb_ld16(rs, (min(r + i * RG, ns - 1) * PS + c * 4) * 2, v[i]) && ok;
+    ml = __builtin_amdgcn_raw_buffer_load_b64(rs, (uint32_t)(min(sp, ns - 1) * PS + D) * 4u, 0, 16);
+    ok = ok && ml.x != OHARA_UNWRITTEN && ml.y != OHARA_UNWRITTEN;
+    if (__all(ok) || poll_expired(pc, spins)) break;
+  }
+  const float ms = sp < ns ? __uint_as_float(ml.x) : -INFINITY, ls = sp < ns ? __uint_as_float(ml.y) : 0.f;
+  const float M = lane_xor_max<1>(lane_xor_max<2>(lane_xor_max<4>(lane_xor_max<8>(ms))));
+  const float w = (ms == -INFINITY) ? 0.f : pow2_neg_int(ms - M);
+  const float Ls = lane_xor_sum<1>(lane_xor_sum<2>(lane_xor_sum<4>(lane_xor_sum<8>(ls * w))));
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+    if (r + i * RG < ns) sts16(sm + (r + i * RG) * D + c * 4, v[i]);
+  if (tid < 16) sw[tid] = w;
+  if (tid == 0) sw[16] = Ls;
+  __syncthreads();
+  if (tid < D / 2) {
+    float o0 = 0.f, o1 = 0.f, ws[OHARA_MEGA_NS];
+    f32x2_t av[OHARA_MEGA_NS];
+#pragma unroll
+    for (int s = 0; s < OHARA_MEGA_NS; ++s) {
+      ws[s] = sw[s];
+      av[s] = *reinterpret_cast<const f32x2_t*>(sm + min(s, ns - 1) * D + 2 * tid);  // (past the last chunk: again, of weight zero)
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < OHARA_MEGA_NS; ++s) {
+      o0 += av[s][0] * ws[s];
+      o1 += av[s][1] * ws[s];
+    }
+    const float inv = 1.0f / sw[16];
+    mb_st4(row, other, 2 * tid, pack_bf(o0 * inv, o1 * inv));
   }
 }
 
@@ -909,17 +944,14 @@ __device__ __forceinline__ void gemm_prefetch_lds(const GemmP& p, char* wl) {
   int strip, j0, j1;
   const bool live = gemm_unit<KP, EPI>(p, phase_block(p) * SPW + sub, kpart, KS, strip, j0, j1);
   if (!live) return;
-  // a rolled loop with a running address: unrolled, the compiler computed all 24 addresses first, spilled
-  // them, and waited for every earlier load before each reload
-  const uint4* src = p.wp + ((size_t)strip * KS + j0) * 64 + lane;
-  char* dst = wl + (size_t)wave * OHARA_LDS_PF * 1024;
-  const int n = min(j1 - j0, OHARA_LDS_PF);
+  // (load_lds16 and not the builtin: behind that the compiler waits for every load in flight before it reads LDS, and in this loop it
+  // waited for the load before)
+  const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(OHARA_LDS char*)wl + wave * (OHARA_LDS_PF * 1024));
+  const int st = __builtin_amdgcn_readfirstlane(strip), first = __builtin_amdgcn_readfirstlane(j0);
+  const uint4* src = p.wp + ((size_t)st * KS + first) * 64;
+  const int n = __builtin_amdgcn_readfirstlane(min(j1 - j0, OHARA_LDS_PF));
 #pragma unroll 1
-  for (int c = 0; c < n; ++c) {
-    __builtin_amdgcn_global_load_lds((const OHARA_GLOBAL void*)src, (OHARA_LDS void*)dst, 16, 0, 0);
-    src += 64;
-    dst += 1024;
-  }
+  for (int c = 0; c < n; ++c) load_lds16(dst + c * 1024, src + c * 64, lane * 16);
 }
 
 template <int KP, int PF, int EPI, class PROF, int PO = 0, bool TAG = false>
@@ -1473,12 +1505,12 @@ __device__ __forceinline__ void attn_new_row_i8(const uint32_t* w, int8_t* kq, i
 // I8 (with TAG only): kc / vc are the int8 caches, `stats` their (sequence, KV head, position) records.
 // AHEAD (with TAG only): a wave's second tile is requested before the poll for q (the single-sequence build: with more
 // sequences a chunk is many tiles and the registers the request holds across the poll are spilled).
-// PPOLL (with TAG only): the partials go to a polled mailbox themselves, `other` bytes from its twin in the other set.
-template <int D, int G, bool TAG = false, bool I8 = false, bool AHEAD = false, bool PPOLL = false>
+// TAG: the partials go to a polled mailbox too, `other` bytes from its twin in the other set.
+template <int D, int G, bool TAG = false, bool I8 = false, bool AHEAD = false>
 __device__ __forceinline__ void attn_phase(int B, int H, int Hkv, int Tmax, int blk_x, int ns, const AttnPre<D>& pre,
                                            const char* qm, float* pm, const bf16_t* kc, const bf16_t* vc, int L,
                                            float* lds, const char* qt = nullptr, const char* kvt = nullptr,
-                                           const Poll pc = Poll{0, 0, nullptr}, bool announce = false, int q_row = 0,
+                                           const Poll pc = Poll{0, nullptr}, int q_row = 0,
                                            int kv_row = 0,  // q_row, kv_row: bytes between the sequences' rows of qt, kvt
                                            float* stats = nullptr,
                                            float* wave_lds = nullptr,  // TAG: 1 KB of LDS per wave, free during this phase
@@ -1725,8 +1757,6 @@ __device__ __forceinline__ void attn_phase(int B, int H, int Hkv, int Tmax, int 
       }
     }
     __syncthreads();
-    float* ann = nullptr;  // the thread that holds a head's maximum and sum: where they go
-    float ann_m = 0.f, ann_l = 0.f;
     for (int idx = tid * 2; idx < G * D; idx += 512) {
       const int hh = idx / D, d = idx - hh * D;
       const int h = kvh * G + hh;
@@ -1741,28 +1771,14 @@ __device__ __forceinline__ void attn_phase(int B, int H, int Hkv, int Tmax, int 
         o1 += s_acc[(w * G + hh) * D + d + 1] * sc;
       }
       float* dst = pm + ((size_t)(b * H + h) * OHARA_MEGA_NS + split) * PS;
-      if (PPOLL) mb_st8(reinterpret_cast<char*>(dst), other, 2 * d, __float_as_uint(o0), __float_as_uint(o1));
+      if (TAG) mb_st8(reinterpret_cast<char*>(dst), other, 2 * d, __float_as_uint(o0), __float_as_uint(o1));
       else st_coh8(dst + d, make_uint2(__float_as_uint(o0), __float_as_uint(o1)));
       if (d == 0) {
-        if (PPOLL) {
-          mb_st8(reinterpret_cast<char*>(dst), other, 2 * D, __float_as_uint(M), __float_as_uint(Ls));
-        } else if (TAG && announce) {
-          ann = dst + D;
-          ann_m = M;
-          ann_l = Ls;
-        } else {
-          st_coh8(dst + D, make_uint2(__float_as_uint(M), __float_as_uint(Ls)));
-        }
+        if (TAG) mb_st8(reinterpret_cast<char*>(dst), other, 2 * D, __float_as_uint(M), __float_as_uint(Ls));
+        else st_coh8(dst + D, make_uint2(__float_as_uint(M), __float_as_uint(Ls)));
       }
     }
-    // `announce`: the merge polls for the head's maximum and sum, which are stored - each in an 8-byte word of its own
-    // together with the launch's tag, {max, tag, sum, tag} - once the item's accumulators have reached memory
-    if (TAG && announce) wait_own_stores();
     __syncthreads();
-    if (TAG && announce && ann) {
-      st_coh8(ann, make_uint2(__float_as_uint(ann_m), pc.tag));
-      st_coh8(ann + 2, make_uint2(__float_as_uint(ann_l), pc.tag));
-    }
   }
 }
 
