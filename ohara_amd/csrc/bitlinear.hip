@@ -891,7 +891,7 @@ int ohara_gemv_ternary_i8(const int8_t* q, int ldq, const float* s, const int32_
   a.q = q; a.ldq = ldq; a.s = s; a.sumq = sumq;
   a.B = rows; a.N = n; a.K = k; a.out = out; a.ldo = ldo; a.resid = resid; a.ldr = ldr;
   a.acc_out = acc_out; a.ldacc = ldacc;
-  if (rows > 64 && (k & 7) == 0 && ternary_tile_ok(q, ldq)) {
+  if (rows > 12 && (k & 7) == 0 && ternary_tile_ok(q, ldq)) {  // (a few rows: a strip a workgroup, no tile of 64 for them)
     TernaryArgs t{};
     t.rows = rows; t.K = k; t.ldq = ldq;
     t.set[0].wp = a.wp; t.set[0].q = q; t.set[0].s = s; t.set[0].sumq = sumq; t.set[0].gamma = gamma; t.set[0].N = n;

@@ -104,3 +104,28 @@ def test_prompt_of_a_model_whose_heads_are_not_in_fours(cuda, width, batch, seq)
     scale, d = want.abs().max().item(), (got - want).abs()
     assert d.max().item() <= 8e-2 * scale and d.mean().item() <= 1e-2 * scale
     assert (cache[0].key[:, seq:] == 0).all() and (cache[0].key[:, :seq].float().abs().amax((2, 3)) > 0).all()
+
+
+@pytest.mark.parametrize("rows", [12, 13, 17, 64, 65])
+def test_rows_around_the_change_of_kernel(cuda, rows):
+    """A few rows are quantised by every workgroup, more once and multiplied in tiles: the same codes and whole sums, so the same bits
+    as the rows give a few at a time."""
+    from ohara_amd import ops
+
+    g = torch.Generator().manual_seed(rows)
+    H, D, K, N = 2, 64, 264, 200
+    x = torch.randn(rows, K, generator=g).to(torch.bfloat16).to(cuda)
+    nw = (1 + 0.1 * torch.randn(4, K, generator=g)).to(torch.bfloat16).to(cuda)
+    ws = [ops.pack_ternary(torch.randint(-1, 2, (n, K), generator=g, dtype=torch.int8).to(cuda), 0.02) for n in (H * D, H * D, H * D, N)]
+    res = torch.randn(rows, N, generator=g).to(torch.bfloat16).to(cuda)
+    got = ops.bitlinear(x, nw[3], ws[3], residual=res)
+    want = torch.cat([ops.bitlinear(x[i:i + 6], nw[3], ws[3], residual=res[i:i + 6]) for i in range(0, rows, 6)])
+    assert torch.equal(got, want)
+    angle = torch.rand(128, D // 2, generator=g)
+    cos, sin = angle.cos().to(torch.bfloat16).to(cuda), angle.sin().to(torch.bfloat16).to(cuda)
+    kc, vc, kp, vp = (torch.zeros(1, 80, H, D, dtype=torch.bfloat16, device=cuda) for _ in range(4))
+    projs = [(nw[i], ws[i]) for i in range(3)]
+    q = ops.bitlinear_qkv_rope_append(x, nw[3], projs, 1e-5, H, H, D, cos, sin, 3, kc, vc, seq_len=rows)
+    parts = [ops.bitlinear_qkv_rope_append(x[i:i + 6], nw[3], projs, 1e-5, H, H, D, cos, sin, 3 + i, kp, vp, seq_len=min(6, rows - i))
+             for i in range(0, rows, 6)]
+    assert torch.equal(q, torch.cat(parts)) and torch.equal(kc, kp) and torch.equal(vc, vp)
