@@ -63,8 +63,8 @@ int ohara_rmsnorm_bf16(const uint16_t* x, const uint16_t* w, uint16_t* out, int 
 /* ---- skinny GEMM (decode projections) ------------------------------------------
  * y = [rmsnorm(x; norm_w, eps)] @ W^T  with one of three epilogues.  `wp` is W in
  * the packed layout; n / k are the logical sizes of W.  norm_w may be NULL.
- * `batch` rows of x.  More than 64 rows without a fused norm go to the tiled MFMA
- * kernel of ohara_gemm_bf16; with a fused norm they are processed 64 at a time, each
+ * `batch` rows of x.  More than 64 rows without a fused norm (without a residual and with
+ * k > 1024: more than 16) go to the tiled MFMA kernel of ohara_gemm_bf16; with a fused norm they are processed 64 at a time, each
  * chunk streaming W once.
  *
  * OHARA_EPI_STORE      out[b, n] = bf16(y)                      (any Linear)
@@ -299,7 +299,7 @@ int ohara_gemv_ternary_i8(const int8_t* q, int ldq, const float* s, const int32_
                           int k, float gamma, int rows, const uint16_t* resid, int ldr, uint16_t* out, int ldo,
                           int32_t* acc_out, int ldacc, void* stream);
 /* Many rows: each row quantised once for each of `sets` (at most three) BitLinears that read it and differ in their norm
- * weight; q: (sets, rows, ldq), s and sumq: (sets, rows).  ohara_gemv_ternary_i8 (more than 64 rows, q on 16 bytes),
+ * weight; q: (sets, rows, ldq), s and sumq: (sets, rows).  ohara_gemv_ternary_i8 (more than 12 rows, q on 16 bytes),
  * ohara_gemm_ternary_sets_i8 (`sets` weights of n columns, one output each) and ohara_gemm_ternary_qkv_rope_append (query, key,
  * value: rotary + append as in ohara_bitlinear_qkv_rope_append_bf16, any number of rows) multiply the codes in tiles; the
  * accumulators are those of ohara_bitlinear_bf16.  ldq a multiple of 16, q on 16 bytes, k a multiple of 8. */
@@ -454,9 +454,9 @@ typedef struct OharaDecodeState {
   uint16_t* q;           /* (rows, h*dh)                                                  */
   uint16_t* attn;        /* (rows, h*dh)                                                  */
   uint16_t* act;         /* (rows, f)                                                     */
-  uint16_t* xn;          /* (rows, d) normalised rows for calls with > 64 rows; may be NULL when
-                            rows_cap <= 64 (NULL with more rows: the skinny kernel runs 64 rows at
-                            a time instead of the tiled MFMA kernel)                           */
+  uint16_t* xn;          /* (rows, d) normalised rows for calls with > 64 rows (> 16 where d > 1024);
+                            may be NULL (the skinny kernel then norms the rows itself, 64 at a
+                            time, instead of the tiled MFMA kernel)                            */
   uint16_t* logits;      /* (batch, vocab) or (rows, vocab), see logits_mode              */
   void* attn_ws;         /* ohara_attn_workspace_bytes(batch, h, h_kv, dh, n_split)       */
   int32_t* step_state;   /* 4 x int32 {pos, step, done, pad}, may be NULL                 */
@@ -600,8 +600,8 @@ int ohara_bitnet_decode_persistent(const OharaBitModel* m, const OharaDecodeStat
                                    int init_workspace, int select_greedy, unsigned int spin_limit, void* stream);
 
 /* ---- Phi (ohara/models/phi.py): the parts of its cached decode path that differ from Llama ----
- * nn.Linear WITH bias on packed weights (phi.py:46-47, :63-66, :161), any number of rows (up to 64:
- * the weight-streaming strip kernel; more: the tiled MFMA kernel of ohara_gemm_bf16,
+ * nn.Linear WITH bias on packed weights (phi.py:46-47, :63-66, :161), any number of rows (up to 64,
+ * or 16 where k > 1024: the weight-streaming strip kernel; more: the tiled MFMA kernel of ohara_gemm_bf16,
  * same epilogues and rounding points).  n % 4 == 0, k % 8 == 0.
  *   OHARA_LIN_BIAS       out = bf16(x @ W^T + bias)
  *   OHARA_LIN_BIAS_GELU  out = new_gelu(bf16(x @ W^T + bias)), every op of phi.py:37-40 rounded to

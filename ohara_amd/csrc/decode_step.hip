@@ -8,7 +8,7 @@
 // then final norm + vocabulary projection (:321-322) and, optionally, greedy
 // selection feeding the next step.  No host synchronisation, no allocation: the
 // chain can be captured once into a HIP graph and replayed per token.
-#include "common.h"
+#include "gemm_epilogue.h"
 
 extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* s, int seq_len, int pos,
                                    int use_pos_dev, int logits_mode, int select_greedy, void* stream) {
@@ -40,7 +40,7 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
     if (rc) return rc;                                                                      \
   } while (0)
   int rc = 0;
-  const bool tiled = R > 64 && s->xn != nullptr;
+  const bool tiled = s->xn != nullptr && ohara_tiles_win(R, d);
   OHARA_RUN(ohara_embed_bf16(s->ids, m->token_emb, s->x, R, d, m->vocab, stream));
   for (int l = 0; l < m->n_layers; ++l) {
     const OharaLayer& L = m->layers[l];

@@ -60,6 +60,15 @@ struct GemmArgs {
 // gemm_tile.hip: the tiled kernel for calls with many rows (a.B rows, no fused norm).
 int ohara_launch_gemm_tile(const GemmArgs& a, int epi, int packed_rows, hipStream_t st);
 
+// Rows from which on rows that are normed once and multiplied in tiles are the quicker way, where the strip kernels norm them in every
+// workgroup (or, without a norm, read them there) - 17 at wide models, 65 at narrow ones.  us, normed strips / a norm and tiles, cold
+// weights, at 16, 17, 32, 33 and 64 rows: 3072 x 2048 7.1 11.9 12.4 16.1 17.6 / 9.4 9.5 9.6 9.7 9.8; 11264 x 2048 with SwiGLU 12.5 15.2 16.3
+// 26.9 30.0 / 15.7 15.5 16.9 18.1 20.5; 32000 x 2048 26.8 28.7 29.1 109 156 / 29.4 29.4 29.6 29.7 29.3; but 6144 x 768 4.8 5.7 6.2 7.5 8.4 / 7.0
+// 7.0 7.0 7.7 7.7, 2304 x 768 3.8 4.9 5.2 4.9 6.4 / 6.6 6.6 6.7 6.8 6.8, 3072 x 1024 4.5 6.1 6.3 7.2 8.2 / 7.2 7.2 7.3 7.4 7.3.  With a
+// bias: 17920 x 2560 24.7 40.3 35.7 46.2 64.1 / 23.1 23.2 24.7 24.3 28.7, 2560 x 2560 7.2 11.1 11.7 10.1 12.8 / 7.5 7.7 7.7 7.7 7.7, 2560 x
+// 10240 20.7 34.7 33.3 33.6 43.8 / 31.4 31.5 31.7 31.2 31.4.  (A residual's product has nothing to norm: 65 rows, see its entry point.)
+inline bool ohara_tiles_win(int rows, int k) { return rows > (k > 1024 ? 16 : 64); }
+
 namespace {
 
 // What an epilogue reads besides the accumulators, fetched ahead: a kernel that finishes many fragments

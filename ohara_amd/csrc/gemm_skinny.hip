@@ -883,7 +883,7 @@ int ohara_linear_bias_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n
   a.B = rows; a.N = n; a.K = k;
   a.out = out; a.ldo = ldo; a.bias = bias;
   a.resid = add1; a.ldr = ld1; a.resid2 = add2; a.ldr2 = ld2;
-  if (rows > 64) return ohara_launch_gemm_tile(a, epi, (n + 15) / 16 * 16, (hipStream_t)stream);
+  if (ohara_tiles_win(rows, k)) return ohara_launch_gemm_tile(a, epi, (n + 15) / 16 * 16, (hipStream_t)stream);
   return launch_skinny(a, epi, (n + 15) / 16 * 16, (hipStream_t)stream);
 }
 
@@ -903,7 +903,7 @@ int ohara_phi_block_in_bf16(const uint16_t* x, int ldx, const uint16_t* ln_w, co
   a.B = batch * seq_len; a.N = 3 * d + ff; a.K = d;
   a.out = q; a.ldo = ldq; a.out2 = act; a.ldo2 = ldact; a.split_n = 3 * d; a.bias = bias;
   a.S = seq_len; a.Tmax = t_max; a.pos = pos; a.pos_dev = pos_dev; a.kcache = kcache; a.vcache = vcache;
-  if (a.B > 64 && !ln_w) return ohara_launch_gemm_tile(a, EPI_PHI_IN, (a.N + 15) / 16 * 16, (hipStream_t)stream);  // prefill
+  if (!ln_w && ohara_tiles_win(a.B, a.K)) return ohara_launch_gemm_tile(a, EPI_PHI_IN, (a.N + 15) / 16 * 16, (hipStream_t)stream);  // prefill
   return launch_skinny(a, EPI_PHI_IN, (a.N + 15) / 16 * 16, (hipStream_t)stream);
 }
 
@@ -969,7 +969,8 @@ int ohara_gemm_skinny_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n
   int packed_rows;
   if (epilogue == OHARA_EPI_SWIGLU) packed_rows = 2 * ((n + 7) / 8 * 8);
   else packed_rows = (n + 15) / 16 * 16;
-  if (batch > 64 && !norm_w) return ohara_launch_gemm_tile(a, epilogue, packed_rows, (hipStream_t)stream);
+  // (a residual, 17, 33 and 64 rows, strips / tiles: 2048 x 2048 5.6 7.6 7.9 / 6.9 6.9 7.0; 2048 x 5632 11.1 18.7 18.1 / 18.5 18.4 18.6 us)
+  if (!norm_w && (epilogue == OHARA_EPI_RESIDUAL ? batch > 64 : ohara_tiles_win(batch, k))) return ohara_launch_gemm_tile(a, epilogue, packed_rows, (hipStream_t)stream);
   return launch_skinny(a, epilogue, packed_rows, (hipStream_t)stream);
 }
 
@@ -991,7 +992,7 @@ static int qkv_rope_impl(const uint16_t* x, int ldx, const uint16_t* wp, int k, 
   a.out = q_out; a.ldo = h * dh;
   a.H = h; a.Hkv = h_kv; a.Dh = dh; a.Tmax = t_max; a.pos = pos; a.pos_dev = pos_dev; a.pos_stride = pos_stride;
   a.cos = cos; a.sin = sin; a.kcache = kcache; a.vcache = vcache; a.stage = stage;
-  if (a.B > 64 && !norm_w) return ohara_launch_gemm_tile(a, EPI_ROPE, (a.N + 15) / 16 * 16, (hipStream_t)stream);
+  if (!norm_w && ohara_tiles_win(a.B, k)) return ohara_launch_gemm_tile(a, EPI_ROPE, (a.N + 15) / 16 * 16, (hipStream_t)stream);
   return launch_skinny(a, EPI_ROPE, (a.N + 15) / 16 * 16, (hipStream_t)stream);
 }
 

@@ -156,7 +156,7 @@ class _Buffers:
         self.q = torch.empty(rows, hd, dtype=BF16, device=dev)
         self.attn = torch.empty(rows, hd, dtype=BF16, device=dev)
         self.act = torch.empty(rows, model.act_width, dtype=BF16, device=dev)
-        self.xn = torch.empty(rows, c.hidden_size, dtype=BF16, device=dev) if rows > 64 else None
+        self.xn = torch.empty(rows, c.hidden_size, dtype=BF16, device=dev) if rows > ops.norm_rows(c.hidden_size) else None
         self.attn_ws = ops.attn_workspace(batch, c.num_attention_heads, model.kv_heads, model.head_dim, n_split, dev)
         self.step_state = torch.zeros(4, dtype=torch.int32, device=dev)
         self.logits = None

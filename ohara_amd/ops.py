@@ -99,12 +99,14 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float = 1e-5, out=None) -> to
     return out
 
 
-NORM_ROWS = 64  # rows whose norm the projection kernels redo in every workgroup; more are normed once, for the tiled kernel
+def norm_rows(k: int) -> int:
+    """Rows whose norm the projection kernels redo in every workgroup; more are normed once, for the tiled kernel (ohara_tiles_win)."""
+    return 16 if k > 1024 else 64
 
 
 def _normed(x, norm_w, eps):
     """(rows, norm weight) for a projection: many rows are normed here."""
-    if norm_w is not None and x.shape[0] > NORM_ROWS:
+    if norm_w is not None and x.shape[0] > norm_rows(x.shape[1]):
         return rmsnorm(x, norm_w, eps), None
     return x, norm_w
 

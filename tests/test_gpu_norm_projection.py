@@ -99,3 +99,41 @@ def test_infinite_weights_of_the_last_columns(cuda, rows, n, k):
     assert (got[:, 3] == float("inf")).all() and (got[:, n - 2] == -float("inf")).all()
     rest = [c for c in range(n) if c not in (3, n - 2)]
     assert got[:, rest].isfinite().all()
+
+
+@pytest.mark.parametrize("n,k", [(11264, 2048), (3072, 2048), (16416, 1032)])
+@pytest.mark.parametrize("rows", [17, 33, 64])
+def test_norm_inside_the_projection_at_wide_models(cuda, rows, n, k):
+    """Python norms these rows ahead of the tiles; a caller without room for normed rows (the last rows' logits of a batch) gets the
+    kernels that norm them themselves."""
+    from ohara_amd import _lib, ops
+
+    g = torch.Generator(device=cuda).manual_seed(rows + n)
+    x, nw = torch.randn(rows, k, generator=g, device=cuda).to(BF), (1 + 0.3 * torch.randn(k, generator=g, device=cuda)).to(BF)
+    w = (torch.randn(n, k, generator=g, device=cuda) * 0.05).to(BF)
+    packed, out = ops.pack_linear(w), torch.empty(rows, n, dtype=BF, device=cuda)
+    _lib.check(_lib.lib().ohara_gemm_skinny_bf16(x.data_ptr(), k, packed.data.data_ptr(), n, k, nw.data_ptr(), 1e-5, rows, _lib.EPI_STORE, None, 0,
+                                                 out.data_ptr(), n, torch.cuda.current_stream().cuda_stream), "gemm_skinny")
+    _check(out, x, w, nw, 1e-5, ops.gemm_skinny(x, packed, nw, 1e-5))
+
+
+@pytest.mark.parametrize("batch,seq", [(17, 1), (64, 1), (3, 11), (1, 16), (1, 17)])
+def test_rotary_rows_around_the_change_of_kernel(cuda, batch, seq):
+    """Rows 16 | 17 at a wide model: the same rows one sequence at a time (strips) and together (tiles from 17 on)."""
+    from ohara_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(batch + seq)
+    H, G, D, K, T, pos = 4, 2, 64, 1032, 40, 5
+    x, nw = torch.randn(batch * seq, K, generator=g, device=cuda).to(BF), (1 + 0.3 * torch.randn(K, generator=g, device=cuda)).to(BF)
+    wqkv = ops.pack_qkv(*((torch.randn(h * D, K, generator=g, device=cuda) * 0.05).to(BF) for h in (H, G, G)))
+    angle = torch.rand(2 * T, D // 2, generator=g, device=cuda)
+    cos, sin = angle.cos().to(BF), angle.sin().to(BF)
+    kc, vc = (torch.zeros(batch, T, G, D, dtype=BF, device=cuda) for _ in range(2))
+    k1, v1 = torch.zeros_like(kc), torch.zeros_like(vc)
+    q = ops.qkv_rope_append(x, wqkv, nw, 1e-5, H, G, D, cos, sin, pos, kc, vc, seq_len=seq)
+    each = [ops.qkv_rope_append(x[b * seq:(b + 1) * seq][:16], wqkv, nw, 1e-5, H, G, D, cos, sin, pos, k1[b:b + 1], v1[b:b + 1],
+                                seq_len=min(seq, 16)) for b in range(batch)]
+    for got, want in ((q.view(batch, seq, -1)[:, :16], torch.stack(each)), (kc[:, :pos + 16], k1[:, :pos + 16]), (vc[:, :pos + 16], v1[:, :pos + 16])):
+        # two bf16 roundings (the projection's and the rotation's) and a normed value that rounds to its neighbour, of values up to 8
+        assert (got.float() - want.float()).abs().max() <= 8 * 2.0 ** -7 and (got != want).float().mean() <= 0.1
+    assert (kc[:, pos + seq:] == 0).all() and (kc[:, :pos] == 0).all()
