@@ -185,6 +185,11 @@ int ohara_attn_cached_bf16_noalloc(const uint16_t* q, const uint16_t* kcache, co
  * Needs no workspace.  (llama.py:100-135 with S > 1.) */
 int ohara_attn_prefill_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int batch,
                             int seq_len, int h, int h_kv, int dh, int t_max, int pos, uint16_t* out, void* stream);
+/* The same with room for partial results (16-byte aligned; ohara_attn_prefill_ws_bytes of `pos` or a later one, 0: none needed): few
+ * queries behind a long context are then cut into chunks of positions over more workgroups.  Too little room or NULL: as without. */
+int64_t ohara_attn_prefill_ws_bytes(int batch, int seq_len, int h, int h_kv, int dh, int pos);
+int ohara_attn_prefill_ws_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int batch, int seq_len, int h,
+                               int h_kv, int dh, int t_max, int pos, uint16_t* out, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ohara_attn_prefill_bf16 over n prompts of their own lengths, their query rows side by side, each from position 0 of its row of the
  * caches: `lengths` on the host; `seqs` on the device: n first query rows, n lengths, n rows of the caches. */
@@ -458,7 +463,9 @@ typedef struct OharaDecodeState {
                             may be NULL (the skinny kernel then norms the rows itself, 64 at a
                             time, instead of the tiled MFMA kernel)                            */
   uint16_t* logits;      /* (batch, vocab) or (rows, vocab), see logits_mode              */
-  void* attn_ws;         /* ohara_attn_workspace_bytes(batch, h, h_kv, dh, n_split)       */
+  void* attn_ws;         /* ohara_attn_workspace_bytes(batch, h, h_kv, dh, n_split); calls with
+                            seq_len > 1 keep partial results there (ohara_attn_prefill_ws_bytes)
+                            where the room behind its counters, align256(4 batch h_kv) bytes, is enough */
   int32_t* step_state;   /* 4 x int32 {pos, step, done, pad}, may be NULL                 */
   int64_t* history;      /* (hist_cap, batch) generated ids, may be NULL                  */
   uint16_t* const* kcache; /* host array [n_layers] of (batch_cap, t_max, h_kv, dh)       */

@@ -16,12 +16,15 @@
 // The running max / sum / rescale are the usual online softmax; probabilities are rounded to bf16 for the second product,
 // sums are kept in fp32, positions are added in their order whatever the shape of the workgroup.
 //
-// Two kernels: one wave per 16 or 32 queries where there are many (attn_prefill_kernel), four waves per 16 where there are
-// few and the walk over the positions is a chain (attn_team_kernel).
+// Three kernels: one wave per 16 or 32 queries where there are many (attn_prefill_kernel), four waves per 16 where there are
+// few and the walk over the positions is a chain (attn_team_kernel), and for few queries behind a long context - with room for partial
+// results from the caller - the positions in chunks, each a workgroup's (attn_chunk_kernel).
 //
 // What bounds them: the softmax between the products, and where the keys and values come from.  A head's q blocks read
 // the same ones: spread round-robin over the XCDs every L2 held every head's, and the launch waited for memory.
 #include "lds_tile.h"
+
+#include <algorithm>
 
 namespace {
 
@@ -182,13 +185,14 @@ __device__ __forceinline__ float softmax_tile(f32x4 (&s)[NKB], uint4 (&pf)[NWIN]
   const float mn = fmaxf(m_run, ceilf(tmax));
   const float corr = pow2_neg_int(m_run - mn);
   m_run = mn;
+  const float off = mn == -INFINITY ? 0.f : mn;  // (a chunk may begin behind the last position of a query: all its weights are zeros)
   float ts = 0.f;
   float p[NKB][4];
 #pragma unroll
   for (int kk = 0; kk < NKB; ++kk)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[kk][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kk][i], mul, -mn));
+      p[kk][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kk][i], mul, -off));
       ts += p[kk][i];
     }
   l_run = l_run * corr + ts;  // this lane's share; lanes g = 0..3 are added at the end
@@ -403,6 +407,177 @@ __global__ __launch_bounds__(TEAMS * 256, TEAMS) void attn_team_kernel(PrefillAr
   store_rows<D>(o, l_run, a, sq, h, wq0 + m, g, w4 * ND);
 }
 
+// Few queries behind a long context.  What bounds the kernels above there is a CU's rate of taking in keys and values, 50 GB/s: 1.5 MB a
+// head at 3000 positions are 31 us, however its waves share them.  So a workgroup takes a chunk of the positions, for four tasks of
+// one KV head - a task is 16 queries of one head; the heads of a group come first, they see the same positions - a wave each, and leaves
+// partial sums for attn_chunks_merge_kernel.  us with both launches, the kernels above / these: 16 queries x 16 heads (4 KV heads) of
+// 128 behind 3000 34.5 / 10.8, 48 queries 35.1 / 13.0, 200 38.4 / 22.5; 4 x 48 behind 1900 25.1 / 17.3; 200 x 16 heads of 64 behind
+// 2000 21.6 / 13.5.
+struct Cut {
+  int tasks, ntb, chunks, tiles;  // tasks of a (sequence, KV head) and fours of them; chunks, and tiles of one
+};
+struct ChunkArgs {
+  PrefillArgs p;
+  Cut cut;
+  int group;    // heads a KV head
+  float* part;  // [task][chunk]: 16 D sums in lane order, 16 maxima, 16 sums of the weights
+};
+
+template <int D>
+__global__ __launch_bounds__(256, 2) void attn_chunk_kernel(ChunkArgs c) {
+  constexpr int NW = 4, NK = D / 32, ND = D / 16, PS = 16 * D + 32;
+  typedef KvTile<D> Tl;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const PrefillArgs& a = c.p;
+  // an XCD gets neighbouring workgroups: the chunks and fours of one KV head share its L2
+  const int n = c.p.B * c.p.Hkv * c.cut.ntb * c.cut.chunks, xcd = blockIdx.x & 7, share = (n + 7) >> 3;
+  const int id = xcd * share + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= share || id >= n) return;
+  const int tb = id % c.cut.ntb, chunk = id / c.cut.ntb % c.cut.chunks, bh = id / (c.cut.ntb * c.cut.chunks), b = bh / a.Hkv, kvh = bh - b * a.Hkv;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  const int task = tb * NW + wave, last_task = min(tb * NW + NW, c.cut.tasks) - 1;
+  const int wq0 = task / c.group * 16, h = kvh * c.group + task % c.group;
+  const Sequence sq = sequence(a, b);
+  const Tl tile(a, sq, kvh, lane);
+  const typename Tl::template Offsets<NW> offs = tile.template offsets<NW>(KT, wave);
+  const int first = chunk * c.cut.tiles, seen = (min(a.pos + last_task / c.group * 16 + 16, tile.len) + KT - 1) / KT;
+  const int end = min(first + c.cut.tiles, seen);                           // tiles any task of the workgroup sees
+  const int wave_last = task < c.cut.tasks ? min(a.pos + wq0 + 15, tile.len - 1) : -1;  // last position any query of the wave sees
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
+
+  uint4 qf[NK];
+  int qpos;
+  load_queries<D>(qf, qpos, a, sq, h, task < c.cut.tasks ? wq0 + m : sq.S, g);
+  f32x4 o[ND];
+#pragma unroll
+  for (int db = 0; db < ND; ++db) o[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  if (first < end) tile.template issue<NW, true>(first, lds0, wave, offs);
+  uint32_t cur = lds0;
+  for (int t = first; t < end; ++t) {
+    tile_barrier<true, 0>();
+    const uint32_t next = lds0 + Tl::SLOT - (cur - lds0);
+    if (t + 1 < end) tile.template issue<NW, true>(t + 1, next, wave, offs);
+    const int t0 = t * KT;
+    if (t0 <= wave_last) {
+      f32x4 s[NKB];
+      uint4 kf[NKB][NK];
+#pragma unroll
+      for (int kk = 0; kk < NKB; ++kk)
+#pragma unroll
+        for (int j = 0; j < NK; ++j) kf[kk][j] = tile.keys(cur, kk, j);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < NK; ++j)
+#pragma unroll
+        for (int kk = 0; kk < NKB; ++kk) s[kk] = mfma16(kf[kk][j], qf[j], j ? s[kk] : (f32x4){0.f, 0.f, 0.f, 0.f});
+      __builtin_amdgcn_sched_barrier(0);
+      uint4 pf[NWIN];
+      const float corr = softmax_tile(s, pf, m_run, l_run, t0, a.pos + wq0, qpos, g, a.scale_log2e);
+      if (__any(corr != 1.0f)) {
+#pragma unroll
+        for (int db = 0; db < ND; ++db)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[db][i] *= corr;
+      }
+#pragma unroll
+      for (int w = 0; w < NWIN; ++w) {
+        uint4 vf[ND];
+#pragma unroll
+        for (int db = 0; db < ND; ++db) vf[db] = tile.values(cur, w, db);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int db = 0; db < ND; ++db) o[db] = mfma16(vf[db], pf[w], o[db]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    cur = next;
+  }
+  if (task >= c.cut.tasks) return;
+  l_run = lane_xor_sum<32>(lane_xor_sum<16>(l_run));
+  float* part = c.part + ((size_t)(bh * c.cut.tasks + task) * c.cut.chunks + chunk) * PS;
+#pragma unroll
+  for (int db = 0; db < ND; ++db) *reinterpret_cast<f32x4*>(part + (db * 64 + lane) * 4) = o[db];
+  if (g == 0) {
+    part[16 * D + m] = m_run;
+    part[16 * D + 16 + m] = l_run;
+  }
+}
+
+// The chunks' sums of a task, in their order: a wave takes sixteen columns of its sixteen queries.
+template <int D>
+__global__ __launch_bounds__(D * 4) void attn_chunks_merge_kernel(ChunkArgs c) {
+  constexpr int PS = 16 * D + 32;
+  const PrefillArgs& a = c.p;
+  const int lane = threadIdx.x & 63, db = threadIdx.x >> 6, m = lane & 15, g = lane >> 4;
+  const int bh = blockIdx.x / c.cut.tasks, task = blockIdx.x - bh * c.cut.tasks, b = bh / a.Hkv;
+  const int qi = task / c.group * 16 + m, h = (bh - b * a.Hkv) * c.group + task % c.group;
+  const float* part = c.part + (size_t)blockIdx.x * c.cut.chunks * PS;
+  float M = -INFINITY, l = 0.f;
+  f32x4 sum = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int i0 = 0; i0 < c.cut.chunks; i0 += 8) {  // eight chunks' loads in flight; the maxima are whole powers of two, so is every rescaling
+    float mx[8], ls[8];
+    f32x4 pv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float* p = part + (size_t)min(i0 + i, c.cut.chunks - 1) * PS;
+      mx[i] = i0 + i < c.cut.chunks ? p[16 * D + m] : -INFINITY;
+      ls[i] = p[16 * D + 16 + m];
+      pv[i] = *reinterpret_cast<const f32x4*>(p + (db * 64 + lane) * 4);
+    }
+    float mn = M;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mn = fmaxf(mn, mx[i]);
+    const float back = pow2_neg_int(M - mn);
+    l *= back;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum[e] *= back;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float w = mx[i] == -INFINITY ? 0.f : pow2_neg_int(mx[i] - mn);
+      l += ls[i] * w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[e] += pv[i][e] * w;
+    }
+    M = mn;
+  }
+  if (qi >= a.S) return;
+  const float inv = 1.0f / l;
+  *reinterpret_cast<uint2*>(a.out + ((size_t)b * a.S + qi) * a.H * D + (size_t)h * D + 16 * db + 4 * g) =
+      make_uint2(pack_bf(sum[0] * inv, sum[1] * inv), pack_bf(sum[2] * inv, sum[3] * inv));
+}
+
+// How a call would be cut: no chunks (0) where the kernels above are the better ones, which is where the walk is no longer than 512
+// positions and two more for every task (the more tasks, the more CUs they keep, and the more partial sums).  us, uncut / cut:
+//   16 x 6 heads behind 500    9.1 /  8.2  (not cut)     8 x 24 x 16 (4) behind 1000 14.5 / 14.7  (not cut)
+//   behind 1000               13.6 /  8.4                8 x 48 x 16 (4) behind 1000 18.2 / 18.5  (not cut)
+//   2 x 128 x 16 (4), 400      9.5 / 12.2  (not cut)     8 x 100 x 6 behind 3000     44.8 / 26.2
+//   1024 x 6 from the start   16.7 / 18.3  (not cut)     8 x 100 x 16 (4) behind 3000 66.6 / 45.7
+// A workgroup a CU, so as not to write more partial sums than that takes (48 a KV head: 4 x 48 x 16 (4) behind 1900 17.3 us, with two a
+// CU 18.3); two from 65 on, where one leaves CUs idle (96: 8 x 100 x 6 39.7, with two 26.2).  None under three tiles.
+// One or two tasks over many KV heads read their positions at the rate of HBM as they are: 16 queries behind 1500, 192 heads of 128 25.7 /
+// 28.2, 128 22.5 / 23.0, but 32 queries and 96 heads 20.9 / 19.6; 192 heads of 64 17.4 / 18.4, but 144 16.6 / 14.8.
+inline Cut cut(int B, int S, int H, int Hkv, int D, int pos, bool most = false) {  // most: the chunks of any call at `pos` or before
+  constexpr int CUS = 256;
+  const int64_t tasks = (int64_t)((S + 15) / 16) * (H / Hkv), ntb = (tasks + 3) / 4, wgs = ntb * B * Hkv;
+  const int ntiles = (int)((pos + (int64_t)S + KT - 1) / KT);
+  if (wgs > CUS || pos + (int64_t)S <= 512 + 2 * tasks * B * Hkv) return Cut{};
+  if (tasks < 3 && (int64_t)B * Hkv > (D == 128 ? 112 : 160)) return Cut{};
+  const int want = (int)((wgs <= 64 ? CUS : 2 * CUS) / wgs);
+  const int tiles = std::max((ntiles + want - 1) / want, 3);
+  return Cut{(int)tasks, (int)ntb, most ? std::min(want, (ntiles + 2) / 3) : (ntiles + tiles - 1) / tiles, tiles};
+}
+
+template <int D>
+int launch_chunks(const PrefillArgs& a, const Cut& cut, float* part, hipStream_t st) {
+  const ChunkArgs c{a, cut, a.H / a.Hkv, part};
+  const int n = c.p.B * c.p.Hkv * c.cut.ntb * c.cut.chunks;
+  hipLaunchKernelGGL((attn_chunk_kernel<D>), dim3((n + 7) / 8 * 8), dim3(256), 2 * KvTile<D>::SLOT, st, c);
+  hipLaunchKernelGGL((attn_chunks_merge_kernel<D>), dim3(c.p.B * c.p.Hkv * c.cut.tasks), dim3(D * 4), 0, st, c);
+  return ohara_launch_status();
+}
+
 template <int D, int QW, bool ALIGNED = true>
 int launch_waves(PrefillArgs a, hipStream_t st) {
   a.nqb = (a.S + 64 * QW - 1) / (64 * QW);
@@ -467,19 +642,50 @@ int launch_prefill_for(const PrefillArgs& a, const int32_t* lengths, hipStream_t
 
 }  // namespace
 
-extern "C" int ohara_attn_prefill_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int batch,
-                                       int seq_len, int h, int h_kv, int dh, int t_max, int pos, uint16_t* out,
-                                       void* stream) {
+static int prefill_args(PrefillArgs& a, const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int batch, int seq_len, int h, int h_kv,
+                        int dh, int t_max, int pos, uint16_t* out) {
   if (!q || !kcache || !vcache || !out) return OHARA_EINVAL;
   if (batch < 1 || seq_len < 1 || h < 1 || h_kv < 1 || h % h_kv || t_max < 1) return OHARA_EINVAL;
   if (pos < 0 || pos + seq_len > t_max) return OHARA_EINVAL;
   if (dh != 64 && dh != 128) return OHARA_ESIZE;
   if (batch > 65535 || h > 65535) return OHARA_ESIZE;
-  PrefillArgs a{};
   a.q = q; a.k = kcache; a.v = vcache; a.out = out;
   a.B = batch; a.S = seq_len; a.H = h; a.Hkv = h_kv; a.Tmax = t_max; a.pos = pos;
   a.scale_log2e = (1.0f / sqrtf((float)dh)) * OHARA_LOG2E;  // the same constant as the decode kernels'
+  return OHARA_OK;
+}
+
+extern "C" int ohara_attn_prefill_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int batch,
+                                       int seq_len, int h, int h_kv, int dh, int t_max, int pos, uint16_t* out,
+                                       void* stream) {
+  PrefillArgs a{};
+  const int rc = prefill_args(a, q, kcache, vcache, batch, seq_len, h, h_kv, dh, t_max, pos, out);
+  if (rc) return rc;
   return dh == 128 ? launch_prefill_for<128>(a, nullptr, (hipStream_t)stream) : launch_prefill_for<64>(a, nullptr, (hipStream_t)stream);
+}
+
+// The partial results of a call that is cut into chunks: task x chunk blocks of 16 dh sums and 32 statistics.
+static int64_t chunk_bytes(const Cut& c, int batch, int h_kv, int dh) {
+  return (int64_t)batch * h_kv * c.tasks * c.chunks * (16 * dh + 32) * (int64_t)sizeof(float);
+}
+
+extern "C" int64_t ohara_attn_prefill_ws_bytes(int batch, int seq_len, int h, int h_kv, int dh, int pos) {
+  if (batch < 1 || seq_len < 1 || h < 1 || h_kv < 1 || h % h_kv || (dh != 64 && dh != 128) || pos < 0) return OHARA_EINVAL;
+  return chunk_bytes(cut(batch, seq_len, h, h_kv, dh, pos, true), batch, h_kv, dh);
+}
+
+extern "C" int ohara_attn_prefill_ws_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int batch, int seq_len, int h,
+                                          int h_kv, int dh, int t_max, int pos, uint16_t* out, void* workspace, int64_t workspace_bytes,
+                                          void* stream) {
+  PrefillArgs a{};
+  const int rc = prefill_args(a, q, kcache, vcache, batch, seq_len, h, h_kv, dh, t_max, pos, out);
+  if (rc) return rc;
+  const hipStream_t st = (hipStream_t)stream;
+  const Cut c = cut(batch, seq_len, h, h_kv, dh, pos);
+  if (c.chunks > 1 && workspace && workspace_bytes >= chunk_bytes(c, batch, h_kv, dh) &&
+      !(((uintptr_t)workspace | (uintptr_t)kcache | (uintptr_t)vcache) & 15))
+    return dh == 128 ? launch_chunks<128>(a, c, (float*)workspace, st) : launch_chunks<64>(a, c, (float*)workspace, st);
+  return dh == 128 ? launch_prefill_for<128>(a, nullptr, st) : launch_prefill_for<64>(a, nullptr, st);
 }
 
 extern "C" int ohara_attn_prompts_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int n, const int32_t* lengths,

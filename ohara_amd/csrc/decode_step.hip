@@ -10,6 +10,8 @@
 // chain can be captured once into a HIP graph and replayed per token.
 #include "gemm_epilogue.h"
 
+#include <algorithm>
+
 extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* s, int seq_len, int pos,
                                    int use_pos_dev, int logits_mode, int select_greedy, void* stream) {
   if (!m || !s || !m->layers || !s->kcache || !s->vcache) return OHARA_EINVAL;
@@ -28,6 +30,10 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
   const int32_t* pos_dev = use_pos_dev ? s->step_state : nullptr;  // first field is pos
   const int n_split = seq_len == 1 ? s->n_split : 1;
   hipStream_t hs = (hipStream_t)stream;
+  // of attn_ws, what lies behind the counters of decode attention (which stay zero) is room for a prompt's partial results
+  const int64_t counters = ((int64_t)B * Hkv * 4 + 255) / 256 * 256;
+  const int64_t room = s->attn_ws ? std::max<int64_t>(0, ohara_attn_workspace_bytes(B, H, Hkv, Dh, s->n_split) - counters) : 0;
+  void* const room_at = s->attn_ws ? (unsigned char*)s->attn_ws + counters : nullptr;
   int launch = 0;
   // Brackets launch number s->prof_kernel with the caller's events.
 #define OHARA_RUN(call)                                                                     \
@@ -73,8 +79,8 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
                                            seq_len, H, Hkv, Dh, m->cos, m->sin, pos, pos_dev, s->q, s->kcache[l],
                                            s->vcache[l], m->t_max, stream));
       if (seq_len >= 16 && (Dh == 64 || Dh == 128))
-        OHARA_RUN(ohara_attn_prefill_bf16(s->q, s->kcache[l], s->vcache[l], B, seq_len, H, Hkv, Dh, m->t_max, pos,
-                                          s->attn, stream));
+        OHARA_RUN(ohara_attn_prefill_ws_bf16(s->q, s->kcache[l], s->vcache[l], B, seq_len, H, Hkv, Dh, m->t_max, pos,
+                                             s->attn, room_at, room, stream));
       else
         OHARA_RUN(ohara_attn_cached_bf16(s->q, s->kcache[l], s->vcache[l], B, seq_len, H, Hkv, Dh, m->t_max, pos,
                                          pos_dev, n_split, s->attn_ws, s->attn, stream));
@@ -93,7 +99,7 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
         rc = ohara_kv_dequant_int8(kq, s->kvstats[l], 0, B, len, Hkv, Dh, m->t_max, s->kdeq, stream);
         if (!rc) rc = ohara_kv_dequant_int8(vq, s->kvstats[l], 1, B, len, Hkv, Dh, m->t_max, s->vdeq, stream);
         if (rc) return rc;
-        OHARA_RUN(ohara_attn_prefill_bf16(s->q, s->kdeq, s->vdeq, B, seq_len, H, Hkv, Dh, len, pos, s->attn, stream));
+        OHARA_RUN(ohara_attn_prefill_ws_bf16(s->q, s->kdeq, s->vdeq, B, seq_len, H, Hkv, Dh, len, pos, s->attn, room_at, room, stream));
       } else {
         OHARA_RUN(ohara_attn_cached_int8(s->q, kq, vq, s->kvstats[l], B, seq_len, H, Hkv, Dh, m->t_max, pos, pos_dev,
                                          n_split, s->attn_ws, s->attn, stream));

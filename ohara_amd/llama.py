@@ -311,7 +311,12 @@ class Llama:
             # keep at most one prefill-sized set alive
             for k in [k for k in self._buffers if k[1] > k[0] and k != key]:
                 del self._buffers[k]
-            buf = _Buffers(self, batch, rows, self.default_n_split(batch))
+            n_split, c = self.default_n_split(batch), self.config
+            if rows > batch:  # several tokens a sequence: the workspace holds their partial results (at most 17 MB)
+                h, dh, S = c.num_attention_heads, self.head_dim, rows // batch
+                room = ops.lib().ohara_attn_prefill_ws_bytes(batch, S, h, self.kv_heads, dh, max(0, c.max_sequence_length - S))
+                n_split = max(n_split, -(-room // (batch * h * (4 * dh + 8))))
+            buf = _Buffers(self, batch, rows, n_split)
             self._buffers[key] = buf
         return buf
 

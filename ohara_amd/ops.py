@@ -243,15 +243,17 @@ def attn_cached(q, kcache, vcache, h, h_kv, dh, pos, n_split, workspace, out=Non
 
 def attn_prefill(q, kcache, vcache, h, h_kv, dh, pos, seq_len, out=None):
     """q: (batch*seq_len, h*dh); causal attention of seq_len queries per sequence over cache
-    positions [0, pos + s] on the MFMA prefill kernel."""
+    positions [0, pos + s] on the MFMA prefill kernels."""
     _need(q, BF16, "q")
     rows = q.shape[0]
     if out is None:
         out = torch.empty(rows, h * dh, dtype=BF16, device=q.device)
+    room = max(0, lib().ohara_attn_prefill_ws_bytes(rows // seq_len, seq_len, h, h_kv, dh, int(pos)))  # < 0: refused below
+    workspace = torch.empty(room, dtype=torch.uint8, device=q.device) if room else None
     check(
-        lib().ohara_attn_prefill_bf16(
-            _ptr(q), _ptr(kcache), _ptr(vcache), rows // seq_len, seq_len, h, h_kv, dh, kcache.shape[1], int(pos),
-            _ptr(out), _stream(),
+        lib().ohara_attn_prefill_ws_bf16(
+            _ptr(q), _ptr(kcache), _ptr(vcache), rows // seq_len, seq_len, h, h_kv, dh, kcache.shape[1],
+            int(pos), _ptr(out), _ptr(workspace), room, _stream(),
         ),
         "attn_prefill",
     )

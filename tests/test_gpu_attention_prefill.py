@@ -83,3 +83,37 @@ def test_infinities_reach_no_query_before_their_tile(cuda, B, S, H, pos):
     first = max(0, at // 64 * 64 - 32 - pos)  # 32: queries of one wave
     assert torch.equal(got[:, :first], clean[:, :first])
     assert not got[:, at - pos:].isfinite().any()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,S,H,Hkv,pos", [
+    (1, 16, 6, 6, 509), (1, 17, 16, 4, 700), (1, 1, 4, 4, 1500), (2, 100, 6, 6, 765), (1, 33, 12, 4, 1000),    # three tiles a chunk and more
+    (1, 200, 16, 4, 1400), (8, 100, 6, 6, 1200), (1, 1100, 2, 1, 0), (3, 190, 1, 1, 3000),                    # chunks some queries do not see
+    (1, 700, 3, 1, 129), (1, 250, 6, 2, 1030),
+])
+def test_chunks_of_a_long_context(cuda, B, S, H, Hkv, pos, D):
+    """Few queries behind many positions are cut into chunks; without room for their partial results they are not."""
+    from ohara_amd import ops
+    from ohara_amd._lib import check, lib
+
+    g = torch.Generator(device=cuda).manual_seed(B + S * 3 + H * 7 + pos)
+    q = (torch.randn(B, S, H, D, generator=g, device=cuda) * 2).to(BF)
+    k, v = (torch.randn(B, pos + S + 3, Hkv, D, generator=g, device=cuda).to(BF) for _ in range(2))
+    want, bound = _reference(q, k, v, pos)
+    k[:, pos + S:] = float("nan")
+    v[:, pos + S:] = float("nan")
+    room = lib().ohara_attn_prefill_ws_bytes(B, S, H, Hkv, D, pos)
+    assert room > 0 and lib().ohara_attn_prefill_ws_bytes(B, S, H, Hkv, D, pos + 2000) >= room
+    whole = torch.empty(B * S, H * D, dtype=BF, device=cuda)
+
+    def run(at, size):
+        check(lib().ohara_attn_prefill_ws_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), B, S, H, Hkv, D, k.shape[1], pos,
+                                               whole.data_ptr(), at, size, torch.cuda.current_stream().cuda_stream), "attn_prefill")
+        return whole.view(B, S, H, D)
+
+    ws = torch.full((room + 64,), 0xFF, dtype=torch.uint8, device=cuda)  # NaNs: what no chunk wrote is never used
+    for got in (ops.attn_prefill(q.view(B * S, H * D), k, v, H, Hkv, D, pos, S).view(B, S, H, D), run(ws.data_ptr(), room)):
+        assert ((got.double() - want).abs() <= bound).all()
+    assert (ws[room:] == 0xFF).all()
+    for at, size in ((None, 0), (None, room), (ws.data_ptr(), 16)):
+        assert ((run(at, size).double() - want).abs() <= bound).all()
