@@ -78,7 +78,7 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
       OHARA_RUN(ohara_qkv_rope_append_bf16(tiled ? s->xn : s->x, d, L.wqkv, d, tiled ? nullptr : L.norm1, m->eps, B,
                                            seq_len, H, Hkv, Dh, m->cos, m->sin, pos, pos_dev, s->q, s->kcache[l],
                                            s->vcache[l], m->t_max, stream));
-      if (seq_len >= 16 && (Dh == 64 || Dh == 128))
+      if (ohara_attn_prefill_wins(B, seq_len, H, Hkv, Dh, pos))
         OHARA_RUN(ohara_attn_prefill_ws_bf16(s->q, s->kcache[l], s->vcache[l], B, seq_len, H, Hkv, Dh, m->t_max, pos,
                                              s->attn, room_at, room, stream));
       else

@@ -261,8 +261,8 @@ def attn_prefill(q, kcache, vcache, h, h_kv, dh, pos, seq_len, out=None):
 
 
 def attn_auto(q, kcache, vcache, h, h_kv, dh, pos, n_split, workspace, seq_len, out=None):
-    """The MFMA prefill kernel for calls with many positions per sequence, else the decode kernel."""
-    if seq_len >= 16 and dh in (64, 128):
+    """The MFMA prefill kernels where they win, which is for many positions per sequence, else the decode kernel."""
+    if lib().ohara_attn_prefill_wins(q.shape[0] // seq_len, seq_len, h, h_kv, dh, int(pos)):
         return attn_prefill(q, kcache, vcache, h, h_kv, dh, pos, seq_len, out)
     return attn_cached(q, kcache, vcache, h, h_kv, dh, pos, n_split if seq_len == 1 else 1, workspace, out, None, seq_len)
 

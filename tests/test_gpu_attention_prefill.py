@@ -117,3 +117,27 @@ def test_chunks_of_a_long_context(cuda, B, S, H, Hkv, pos, D):
     assert (ws[room:] == 0xFF).all()
     for at, size in ((None, 0), (None, room), (ws.data_ptr(), 16)):
         assert ((run(at, size).double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,S,H,Hkv,pos,wins", [
+    (1, 2, 6, 6, 400, (0, 0)), (1, 2, 6, 6, 900, (1, 1)), (1, 15, 6, 6, 368, (0, 0)), (3, 7, 5, 5, 376, (0, 0)), (3, 7, 5, 5, 377, (1, 1)),
+    (2, 8, 16, 16, 119, (0, 0)), (2, 8, 16, 16, 120, (0, 1)), (4, 8, 16, 16, 0, (1, 1)), (8, 9, 8, 4, 300, (0, 1)), (8, 9, 4, 2, 300, (0, 0)),
+    (1, 2, 6, 2, 0, (1, 1)), (2, 5, 16, 4, 33, (1, 1)), (1, 3, 20, 4, 700, (1, 1)), (8, 15, 6, 6, 3000, (1, 1)),
+])
+def test_a_few_tokens_a_sequence(cuda, B, S, H, Hkv, pos, wins, D):
+    """Either kernel within the bound on both sides of the lines between them (wins: with heads of 64, of 128), and the one that is taken."""
+    from ohara_amd import ops
+    from ohara_amd._lib import lib
+
+    assert lib().ohara_attn_prefill_wins(B, S, H, Hkv, D, pos) == wins[D == 128]
+    g = torch.Generator(device=cuda).manual_seed(B + S * 3 + H * 7 + pos)
+    q = (torch.randn(B, S, H, D, generator=g, device=cuda) * 2).to(BF)
+    k, v = (torch.randn(B, pos + S + 3, Hkv, D, generator=g, device=cuda).to(BF) for _ in range(2))
+    want, bound = _reference(q, k, v, pos)
+    rows = q.view(B * S, H * D)
+    assert ((ops.attn_cached(rows, k, v, H, Hkv, D, pos, 1, None, None, None, S).view(B, S, H, D).double() - want).abs() <= bound).all()
+    k[:, pos + S:] = float("nan")
+    v[:, pos + S:] = float("nan")
+    assert ((ops.attn_prefill(rows, k, v, H, Hkv, D, pos, S).view(B, S, H, D).double() - want).abs() <= bound).all()
+    assert ((ops.attn_auto(rows, k, v, H, Hkv, D, pos, 1, None, S).view(B, S, H, D).double() - want).abs() <= bound).all()
