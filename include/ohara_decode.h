@@ -501,6 +501,39 @@ typedef struct OharaDecodeState {
 int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* s, int seq_len, int pos, int use_pos_dev,
                         int logits_mode, int select_greedy, void* stream);
 
+/* The same for a model whose feed-forwards are grouped experts (moe_grouped.py:209-228) or dense, over caches of bfloat16 or int8.
+ * `scratch`: ohara_moe_forward_bytes of the same arguments, 256-byte aligned, used by this call alone; attn_ws:
+ * ohara_attn_workspace_bytes(batch, h, h_kv, dh, n_split), zero between calls.  logits: (batch, vocab) of the last tokens, or
+ * (batch * seq_len, vocab). */
+typedef struct OharaMoeLayer {
+  const uint16_t *wqkv, *wo, *norm1, *norm2;
+  const uint16_t *wgu, *wdown;               /* packed: the dense feed-forward's, or the shared expert's (NULL: none), ff wide */
+  const uint16_t *router, *router_bias;      /* router NULL: a dense layer                       */
+  const uint16_t *experts_gu, *experts_down; /* as ohara_moe_experts_gate_up_shared / _down_shared */
+  int64_t gu_stride, down_stride;            /* bytes from expert to expert                      */
+  int32_t* counter;
+  int32_t ff, n_experts, hidden, k, biased_topk, gate_sigmoid, normalize, reserved;
+} OharaMoeLayer;
+
+typedef struct OharaMoeCall {
+  int32_t n_layers, d_model, n_heads, n_kv_heads, head_dim, vocab, t_max;
+  int32_t batch, seq_len, pos, n_split, last_only;
+  float eps;
+  int32_t reserved;
+  const uint16_t *token_emb, *final_norm, *w_vocab, *cos, *sin;
+  const OharaMoeLayer* layers;               /* host array [n_layers]                            */
+  const int64_t* ids;                        /* (batch, seq_len)                                 */
+  void* const* kcache;                       /* host arrays [n_layers]                           */
+  void* const* vcache;
+  void* const* kvstats;                      /* int8 caches; NULL: bfloat16                      */
+  uint16_t* logits;
+  void *attn_ws, *scratch;
+  int64_t scratch_bytes;
+} OharaMoeCall;
+
+int64_t ohara_moe_forward_bytes(const OharaMoeCall* c);
+int ohara_moe_forward(const OharaMoeCall* c, void* stream);
+
 /* ohara_llama_forward over n prompts of different lengths, each from position 0 into its own row of the caches (bf16 caches,
  * head width 64 or 128); logits (n, vocab) of the last token of each.  s: ids, x, xn, q, attn and act for the rows of all prompts
  * side by side.  `lengths` on the host; `table` on the device: n first rows, n lengths, n rows of the caches, then the position of

@@ -61,6 +61,25 @@ class OharaDecodeState(C.Structure):
     ]
 
 
+class OharaMoeLayer(C.Structure):
+    _fields_ = [
+        ("wqkv", _p), ("wo", _p), ("norm1", _p), ("norm2", _p), ("wgu", _p), ("wdown", _p), ("router", _p), ("router_bias", _p),
+        ("experts_gu", _p), ("experts_down", _p), ("gu_stride", _i64), ("down_stride", _i64), ("counter", _p),
+        ("ff", _i), ("n_experts", _i), ("hidden", _i), ("k", _i), ("biased_topk", _i), ("gate_sigmoid", _i), ("normalize", _i),
+        ("reserved", _i),
+    ]
+
+
+class OharaMoeCall(C.Structure):
+    _fields_ = [
+        ("n_layers", _i), ("d_model", _i), ("n_heads", _i), ("n_kv_heads", _i), ("head_dim", _i), ("vocab", _i), ("t_max", _i),
+        ("batch", _i), ("seq_len", _i), ("pos", _i), ("n_split", _i), ("last_only", _i), ("eps", _f), ("reserved", _i),
+        ("token_emb", _p), ("final_norm", _p), ("w_vocab", _p), ("cos", _p), ("sin", _p), ("layers", C.POINTER(OharaMoeLayer)),
+        ("ids", _p), ("kcache", C.POINTER(_p)), ("vcache", C.POINTER(_p)), ("kvstats", C.POINTER(_p)), ("logits", _p),
+        ("attn_ws", _p), ("scratch", _p), ("scratch_bytes", _i64),
+    ]
+
+
 class OharaSeq(C.Structure):
     _fields_ = [("batch", _i), ("seq_len", _i), ("pos", _i), ("pos_stride", _i), ("pos_dev", _p), ("lens", _p), ("slots", _p)]
 
@@ -163,6 +182,8 @@ _PROTOS = {
                                            _p]),
     "ohara_moe_experts_gate_up_many": (_i, [_p, _i, _p, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _i, _p]),
     "ohara_moe_experts_down_many": (_i, [_p, _i, _p, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _p, _i, _p]),
+    "ohara_moe_forward_bytes": (_i64, [_p]),
+    "ohara_moe_forward": (_i, [_p, _p]),
     "ohara_moe_combine": (_i, [_p, _i, _p, _p, _i, _i, _p, _i, _p, _i, _p, _i, _i, _p]),
     "ohara_llama_prompts": (_i, [C.POINTER(OharaModel), C.POINTER(OharaDecodeState), _i, _p, _p, _p]),
     "ohara_llama_forward": (_i, [C.POINTER(OharaModel), C.POINTER(OharaDecodeState), _i, _i, _i, _i, _i, _p]),

@@ -4,10 +4,12 @@ mode and the Llama whose feed-forwards are GroupedMoE layers (ohara/models/llama
 
 from __future__ import annotations
 
+import ctypes as C
+
 import torch
 
 from . import ops
-from ._lib import check, lib
+from ._lib import OharaMoeCall, OharaMoeLayer, check, lib
 from .llama import BF16, Config, KVCache, _validate_config, rope_tables
 
 
@@ -204,6 +206,7 @@ class MoeLlama:
                 L["wdown"] = ops.pack_linear(dev(state[p + "ff.down.weight"]))
             self.layers.append(L)
         self._ws = {}
+        self._table = None, None
 
     def eval(self):
         return self
@@ -219,6 +222,64 @@ class MoeLlama:
         shape = (batch_size, c.max_sequence_length, self.kv_heads, self.head_dim)
         return [KVCache(shape, c.max_sequence_length, i, device=self.device, dtype=BF16, int8=int8)
                 for i in range(c.num_hidden_layers)]
+
+    def _layer_table(self):
+        """The layers for the C chain, from the tensors that they hold now: laid out again where one of them is another."""
+        held = []
+        for L in self.layers:
+            moe = L.get("moe")
+            held += [L["wqkv"].data, L["wo"].data, L["norm1"], L["norm2"]]
+            if moe is None:
+                held += [L["wgu"].data, L["wdown"].data] + [None] * 5
+            else:
+                sh = moe.shared
+                held += [sh and sh[0].data, sh and sh[1].data, moe.router.data, moe.router_bias, moe.wp_gu, moe.wp_dn, moe._counter]
+        at = [0 if t is None else t.data_ptr() for t in held]
+        at += [(m.k, m.biased, m.gate_fn, m.normalize) for m in (L.get("moe") for L in self.layers) if m is not None]
+        table, table_of = self._table
+        if at != table_of:
+            table = (OharaMoeLayer * len(self.layers))()
+            for i, L in enumerate(self.layers):
+                c, moe = table[i], L.get("moe")
+                (c.wqkv, c.wo, c.norm1, c.norm2, c.wgu, c.wdown, c.router, c.router_bias, c.experts_gu, c.experts_down,
+                 c.counter) = at[11 * i:11 * i + 11]
+                if moe is None:
+                    c.ff = L["wgu"].n
+                else:
+                    c.ff = moe.shared[0].n if moe.shared is not None else 0
+                    c.n_experts, c.hidden, c.k = moe.E, moe.hidden, moe.k
+                    c.gu_stride, c.down_stride = moe.wp_gu.stride(0) * 2, moe.wp_dn.stride(0) * 2
+                    c.biased_topk, c.gate_sigmoid, c.normalize = int(moe.biased), int(moe.gate_fn == "sigmoid"), int(moe.normalize)
+            self._table = table, at
+        return table
+
+    def _chain(self, x, kv_cache, start: int, n_split: int, ws, last_only: bool):
+        """The call as one C call, which launches what the loop of ``forward`` does; None where it does not take it."""
+        c, (B, S) = self.config, x.shape
+        if last_only and S > 1 and B > ops.norm_rows(c.hidden_size):
+            return None
+        if any(L["moe"].trace is not None for L in self.layers if "moe" in L) or any(
+                cc.key.shape[1] != c.max_sequence_length for cc in kv_cache):
+            return None
+        n = len(self.layers)
+        call = OharaMoeCall(n, c.hidden_size, c.num_attention_heads, self.kv_heads, self.head_dim, c.vocab_size,
+                            c.max_sequence_length, B, S, start, n_split, int(last_only), self.eps)
+        call.layers = self._layer_table()
+        if kv_cache[0].int8:
+            call.kvstats = (C.c_void_p * n)(*[cc.stats.data_ptr() for cc in kv_cache])
+        size = lib().ohara_moe_forward_bytes(C.byref(call))
+        if size < 0:
+            return None
+        ids = x.to(self.device).reshape(-1).contiguous()
+        scratch = torch.empty(size, dtype=torch.uint8, device=self.device)
+        logits = torch.empty(B, 1 if last_only else S, c.vocab_size, dtype=BF16, device=self.device)
+        call.token_emb, call.final_norm, call.w_vocab = _ptr(self.token_emb), _ptr(self.final_norm), _ptr(self.w_vocab.data)
+        call.cos, call.sin, call.ids, call.logits = _ptr(self.cos), _ptr(self.sin), _ptr(ids), _ptr(logits)
+        call.kcache = (C.c_void_p * n)(*[cc.key.data_ptr() for cc in kv_cache])
+        call.vcache = (C.c_void_p * n)(*[cc.value.data_ptr() for cc in kv_cache])
+        call.attn_ws, call.scratch, call.scratch_bytes = _ptr(ws), _ptr(scratch), size
+        check(lib().ohara_moe_forward(C.byref(call), ops._stream()), "moe_forward")
+        return logits
 
     @torch.no_grad()
     def forward(self, x, kv_cache=None, position_ids=None, *, last_only: bool = False):
@@ -254,6 +315,11 @@ class MoeLlama:
         ws = self._ws.get((B, n_split))
         if ws is None:
             ws = self._ws[(B, n_split)] = ops.attn_workspace(B, H, Hkv, D, n_split, self.device)
+        logits = self._chain(x, kv_cache, start, n_split, ws, last_only)
+        if logits is not None:
+            for cc, end in zip(kv_cache, ends):
+                cc._commit(B, end)
+            return logits
         h = ops.embed(x.to(self.device), self.token_emb)
         for L, cache in zip(self.layers, kv_cache):
             if int8:

@@ -209,3 +209,47 @@ def test_moe_block_in_four_launches(cuda, N, d, E, hidden, k, shared, gate):
         dd = (got.float() - want.float()).cpu()[same].abs()
         assert dd.max().item() <= 2e-2 * scale and dd.mean().item() <= 2e-3 * scale, (dd.max().item(), dd.mean().item(), scale)
     moe.trace = None
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("B,S,start,last", [(1, 1, 5, False), (1, 1, 700, True), (3, 2, 0, False), (2, 5, 30, True), (20, 1, 9, False),
+                                            (70, 1, 200, True), (1, 40, 600, False), (2, 33, 0, True), (70, 2, 3, True),
+                                            (3, 200, 11, False)])
+@pytest.mark.parametrize("kind", ["shared", "alternating", "wide heads"])
+def test_one_call_for_all_layers(cuda, B, S, start, last, int8, kind):
+    """The C chain against the loop over the layers, bit for bit, logits and caches; what it does not take goes through the loop."""
+    from ohara_amd.llama import Config
+    from ohara_amd.moe import MoeLlama
+
+    kw = dict(vocab_size=256, hidden_size=128, intermediate_size=64, num_attention_heads=2, num_key_value_heads=0, num_hidden_layers=3,
+              max_sequence_length=768, dropout=0.0, moe_num_experts=16, moe_experts_per_tok=4, moe_layer_interval=1, moe_grouped=True,
+              moe_num_shared_experts=1, moe_gate_fn="softmax")
+    if kind == "alternating":
+        kw.update(moe_layer_interval=2, moe_num_shared_experts=0, moe_gate_fn="sigmoid", moe_experts_per_tok=3)
+    if kind == "wide heads":
+        kw.update(hidden_size=1536, num_attention_heads=12, num_key_value_heads=2, moe_num_experts=5, moe_experts_per_tok=1)
+    model = MoeLlama(Config(**kw), R.init_weights(R.RefConfig(**kw), seed=9, dtype=BF, std=0.06, norm_jitter=0.1), device=cuda)
+    g = torch.Generator().manual_seed(B * S + start)
+    before = torch.randint(0, 256, (B, start), generator=g).to(cuda)
+    ids = torch.randint(0, 256, (B, S), generator=g).to(cuda)
+    took, chain = [], model._chain
+    results = []
+    for fused in (False, True):
+        model._chain = lambda *a: None
+        cache = model.build_kv_cache(B, int8=int8)
+        if start:
+            model(before, cache, 0, last_only=True)
+        if fused:
+            model._chain = lambda *a: took.append(chain(*a)) or took[-1]
+        logits = model(ids, cache, start, last_only=last)
+        results.append([logits] + [t for c in cache for t in ((c.key, c.value, c.stats) if int8 else (c.key, c.value))])
+    for a, b in zip(*results):
+        assert a.shape == b.shape and torch.equal(a, b)
+    assert (took[0] is None) == (last and S > 1 and B > (16 if kind == "wide heads" else 64))
+    layer = next(L for L in model.layers if "moe" in L)["moe"]  # tensors that are replaced are seen
+    layer.router_bias = layer.router_bias + torch.arange(layer.E, device=cuda).to(BF)
+    model._chain = lambda *a: None
+    want = model(ids, model.build_kv_cache(B), 0)
+    model._chain = chain
+    assert torch.equal(model(ids, model.build_kv_cache(B), 0), want)
+
