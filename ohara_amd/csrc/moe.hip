@@ -29,39 +29,56 @@ namespace {
 template <int MAXPL>
 __device__ __forceinline__ void route_core(float (&sel)[MAXPL], const float (&raw)[MAXPL], int E, int k, int sigmoid,
                                            int normalize, int lane, int& my_id, float& wt) {
-  // Winner j is kept by lane j; the arg-max butterfly runs on DPP moves and row swaps.
+  // Winner j is kept by lane j.
   float my_raw = 0.f;
   my_id = 0;
-  for (int j = 0; j < k; ++j) {
-    // lane-local best (lowest id on ties), then across the wave
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
+  if constexpr (MAXPL == 1) {
+    // An expert a lane: its rank is how many come before it, counted over the 64 keys, and the lanes swap places by rank.  (64 times
+    // four instructions where k arg-max butterflies are k times six dependent steps; with the product's
+    // reads below, 64 experts, 8 chosen, d 1024: 24 tokens 12.7 -> 10.6 us, one 10.9 -> 8.4)
+    const float v = sel[0] + 0.f;  // (-0 is 0)
+    const uint32_t bits = __float_as_uint(v);
+    uint32_t key = bits ^ (bits >> 31 ? 0xffffffffu : 0x80000000u);  // ascending as v is
+    if (v != v) key = 2;  // NaN: behind every number
+    if (lane >= E) key = 1;
+    int rank = 0;
 #pragma unroll
-    for (int i = 0; i < MAXPL; ++i) {
-      const int e = i * 64 + lane;
-      if (e < E && (sel[i] > bv || (sel[i] == bv && e < bi))) {
-        bv = sel[i];
-        bi = e;
-      }
-    }
-    lane_xor_argmax<32>(bv, bi);
-    lane_xor_argmax<16>(bv, bi);
-    lane_xor_argmax<8>(bv, bi);
-    lane_xor_argmax<4>(bv, bi);
-    lane_xor_argmax<2>(bv, bi);
-    lane_xor_argmax<1>(bv, bi);
-    // fetch the unbiased logit of the winner and retire it
-    float r = 0.f;
+    for (int j = 0; j < 64; ++j) rank += (uint32_t)__builtin_amdgcn_readlane((int)key, j) > key - (j < lane ? 1u : 0u);  // (ties: the lower id)
+    my_id = __builtin_amdgcn_ds_permute(rank * 4, lane);
+    my_raw = __uint_as_float((uint32_t)__builtin_amdgcn_ds_permute(rank * 4, (int)__float_as_uint(raw[0])));
+  } else {
+    // the arg-max butterfly runs on DPP moves and row swaps
+    for (int j = 0; j < k; ++j) {
+      // lane-local best (lowest id on ties), then across the wave
+      float bv = -INFINITY;
+      int bi = 0x7fffffff;
 #pragma unroll
-    for (int i = 0; i < MAXPL; ++i)
-      if (i * 64 + lane == bi) {
-        r = raw[i];
-        sel[i] = -INFINITY;
+      for (int i = 0; i < MAXPL; ++i) {
+        const int e = i * 64 + lane;
+        if (e < E && (sel[i] > bv || (sel[i] == bv && e < bi))) {
+          bv = sel[i];
+          bi = e;
+        }
       }
-    r = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(r), bi & 63));
-    if (lane == j) {
-      my_raw = r;
-      my_id = bi;
+      lane_xor_argmax<32>(bv, bi);
+      lane_xor_argmax<16>(bv, bi);
+      lane_xor_argmax<8>(bv, bi);
+      lane_xor_argmax<4>(bv, bi);
+      lane_xor_argmax<2>(bv, bi);
+      lane_xor_argmax<1>(bv, bi);
+      // fetch the unbiased logit of the winner and retire it
+      float r = 0.f;
+#pragma unroll
+      for (int i = 0; i < MAXPL; ++i)
+        if (i * 64 + lane == bi) {
+          r = raw[i];
+          sel[i] = -INFINITY;
+        }
+      r = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(r), bi & 63));
+      if (lane == j) {
+        my_raw = r;
+        my_id = bi;
+      }
     }
   }
   // weights: every lane below k holds one; the sums run in slot order, as a loop over the slots would
@@ -313,11 +330,24 @@ __global__ __launch_bounds__(256) void moe_route_fused_kernel(RouteFusedArgs a) 
           for (int c = 0; c < 32; ++c) wv[c] = ldg16_nt(wrow + (size_t)min(jb + c, KS - 1) * 64);
         }
 #pragma unroll
-        for (int c = 0; c < 32; ++c) {
-          if (jb + c < KS) {
-            const uint4 xv = *reinterpret_cast<const uint4*>(xrow + 32 * (jb + c));
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[c]), __builtin_bit_cast(bf16x8, xv),
-                                                          acc, 0, 0, 0);
+        for (int cb = 0; cb < 32; cb += 8) {  // eight steps' reads together (a branch a step waited for each)
+          if (jb + cb + 8 <= KS) {
+            uint4 xv[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) xv[c] = *reinterpret_cast<const uint4*>(xrow + 32 * (jb + cb + c));
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[cb + c]), __builtin_bit_cast(bf16x8, xv[c]),
+                                                            acc, 0, 0, 0);
+          } else {
+#pragma unroll
+            for (int c = 0; c < 7; ++c) {
+              if (jb + cb + c < KS) {
+                const uint4 xv = *reinterpret_cast<const uint4*>(xrow + 32 * (jb + cb + c));
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[cb + c]), __builtin_bit_cast(bf16x8, xv),
+                                                              acc, 0, 0, 0);
+              }
+            }
           }
         }
       }

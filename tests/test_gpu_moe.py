@@ -253,3 +253,24 @@ def test_one_call_for_all_layers(cuda, B, S, start, last, int8, kind):
     model._chain = chain
     assert torch.equal(model(ids, model.build_kv_cache(B), 0), want)
 
+
+@pytest.mark.parametrize("E,k", [(1, 1), (2, 1), (5, 5), (17, 16), (63, 8), (64, 1), (64, 16), (65, 8)])
+def test_selection_among_ties(cuda, E, k):
+    """Up to 64 experts the chosen are found by rank, past them by k searches: ties to the lowest id, zeros of either sign alike,
+    -inf before nothing else is left."""
+    from ohara_amd._lib import check, lib
+
+    g = torch.Generator().manual_seed(E * 31 + k)
+    n = 37
+    logits = torch.randint(-2, 3, (n, E), generator=g).float() / 2
+    logits[torch.rand(n, E, generator=g) < 0.1] = -0.0
+    if k < E:
+        logits[:, :E - k][torch.rand(n, E - k, generator=g) < 0.2] = float("-inf")
+    idx = torch.full((n, k), -1, dtype=torch.int32, device=cuda)
+    w = torch.zeros(n, k, dtype=BF, device=cuda)
+    dev = logits.to(BF).to(cuda)
+    check(lib().ohara_moe_route_topk(dev.data_ptr(), E, None, n, E, k, 0, 1, 0, idx.data_ptr(), w.data_ptr(),
+                                     torch.cuda.current_stream().cuda_stream), "moe_route")
+    want = torch.sort(-logits, dim=-1, stable=True).indices[:, :k]
+    assert torch.equal(idx.cpu().long(), want)
+    assert ((w.float().cpu() - torch.sigmoid(logits.gather(1, want))).abs() <= 2.0 ** -8).all()  # bf16 of a value below one
