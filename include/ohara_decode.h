@@ -224,6 +224,11 @@ int ohara_kv_dequant_int8(const int8_t* q, const float* stats, int which, int ba
 int ohara_attn_cached_int8(const uint16_t* q, const int8_t* kcache, const int8_t* vcache, const float* stats, int batch,
                            int seq_len, int h, int h_kv, int dh, int t_max, int pos, const int32_t* pos_dev, int n_split,
                            void* workspace, uint16_t* out, void* stream);
+/* ohara_kv_quant_append_int8 of one position a sequence (pos_stride 1: ohara_kv_quant_append_ragged_int8's, pos_dev the positions) and the
+ * attention of its queries, in one launch where heads are 64 or 128 wide, in groups of 1, 2 or 4. */
+int ohara_attn_append_int8(const uint16_t* q, const uint16_t* k, const uint16_t* v, int8_t* kcache, int8_t* vcache, float* stats, int batch,
+                           int h, int h_kv, int dh, int t_max, int pos, const int32_t* pos_dev, int pos_stride, int n_split, void* workspace,
+                           uint16_t* out, void* stream);
 
 /* The append and the attention with one cache position per sequence (seq_pos: device array, `batch`
  * entries; token s of sequence b goes to / sits at seq_pos[b] + s).  No counterpart in the reference,

@@ -136,6 +136,7 @@ _PROTOS = {
     "ohara_qkv_rope_bf16": (_i, [_p, _i, _p, _i, _p, _f, _i, _i, _i, _i, _i, _p, _p, _i, _p, _i, _p, _p, _p, _p]),
     "ohara_kv_quant_append_int8": (_i, [_p, _p, _i, _i, _i, _i, _i, _p, _p, _p, _p, _i, _p]),
     "ohara_kv_dequant_int8": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _p, _p]),
+    "ohara_attn_append_int8": (_i, [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _i, _i, _p, _p, _p]),
     "ohara_attn_cached_int8": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _i, _p, _p, _p]),
     "ohara_attn_workspace_bytes": (_i64, [_i, _i, _i, _i, _i]),
     "ohara_attn_cached_bf16": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _i, _p, _p, _p]),

@@ -34,6 +34,8 @@ struct AttnArgs {
   float* part_ml;    // (B, Hkv, nsplit of room: G, chunks, 2)
   float* part_acc;   // (B, Hkv, nsplit of room: G, chunks, D)
   float scale;
+  const bf16_t* k_new;  // int8 mode, one query a sequence: (B, Hkv, D) rows of the queries' own positions, quantised into the cache
+  const bf16_t* v_new;  // by the call (null: they are there)
 };
 
 __device__ __forceinline__ float dot8(uint4 a, uint4 b, float s) {
@@ -378,6 +380,47 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
 // permutation of the head dimension, the same one on both sides), NC products of 16x16x32 per sub-tile;
 // lanes 0..15 end up with the scores of position n for every head.  The value product stays on the
 // vector units (its operand would have to be transposed).
+// The query's own position, quantised by the workgroup that walks the end of the context (as kv_quant_append_kernel would, whose launch
+// is 4.5 us of a layer): into the cache, and through LDS into the last tile, so that nothing waits for the stores.  Waves 0 and 1 take
+// the key and the value row; their loads are asked for before the first tile's.
+template <int D>
+struct NewRow {
+  __align__(16) int8_t k[D], v[D];
+  float st[4];  // key scale, key minimum, value scale, value minimum
+};
+template <int D>
+struct NewLoad {
+  bf16_t x[D / 64];
+};
+template <int D>
+__device__ __forceinline__ NewLoad<D> load_new(const AttnArgs& a, int seq, int kvh, int wave, int lane) {
+  NewLoad<D> l;
+  const bf16_t* src = (wave ? a.v_new : a.k_new) + ((size_t)seq * a.Hkv + kvh) * D;
+#pragma unroll
+  for (int i = 0; i < D / 64; ++i) l.x[i] = src[lane + 64 * i];
+  return l;
+}
+template <int D>
+__device__ __forceinline__ void put_new(const AttnArgs& a, const NewLoad<D>& l, int seq, int kvh, int pos, int wave, int lane, NewRow<D>& row) {
+  float x[D / 64], scale, mn;
+#pragma unroll
+  for (int i = 0; i < D / 64; ++i) x[i] = bf2f(l.x[i]);
+  int8_t code[D / 64];
+  kv_quant_row(x, D, lane, scale, mn, code);
+  int8_t* dst = reinterpret_cast<int8_t*>(const_cast<bf16_t*>(wave ? a.v : a.k)) + (((size_t)seq * a.Tmax + pos) * a.Hkv + kvh) * D;
+#pragma unroll
+  for (int i = 0; i < D / 64; ++i) {
+    (wave ? row.v : row.k)[lane + 64 * i] = code[i];
+    dst[lane + 64 * i] = code[i];
+  }
+  if (lane == 0) {
+    row.st[2 * wave] = scale;
+    row.st[2 * wave + 1] = mn;
+    float* rec = const_cast<float*>(a.stats) + (((size_t)seq * a.Hkv + kvh) * a.Tmax + pos) * 4 + 2 * wave;
+    *reinterpret_cast<float2*>(rec) = make_float2(scale, mn);
+  }
+}
+
 template <int D, int G>
 __global__ __launch_bounds__(256, (G == 1 ? 3 : 2)) void attn_decode_i8_kernel(AttnArgs a) {
   constexpr int NC = D / 32;        // bf16 uint4 of a K quarter-row after expansion
@@ -394,6 +437,8 @@ __global__ __launch_bounds__(256, (G == 1 ? 3 : 2)) void attn_decode_i8_kernel(A
   if (split >= used) return;
   const int t0 = split * chunk;
   const int t1 = min(L, t0 + chunk);
+  const int own = a.pos_dev ? a.pos_dev[(size_t)seq * a.pos_stride] : a.start;
+  const bool append = a.k_new && split == used - 1 && own >= 0 && own < a.Tmax;  // (then own == t1 - 1)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int p = lane & 15, dq = lane >> 4;  // position of the sub-tile, quarter of its K row (the B operand's column and k group)
   const int pp = lane / DC, dc = lane % DC;
@@ -401,6 +446,7 @@ __global__ __launch_bounds__(256, (G == 1 ? 3 : 2)) void attn_decode_i8_kernel(A
 
   __shared__ float s_m[4][G], s_l[4][G];
   __shared__ float s_acc[4][G][D];
+  __shared__ NewRow<D> s_new;
 
   uint4 qa[NC];  // A operand: row (lane & 15) = head of the group (rows past the group are zero), this lane's quarter dq
 #pragma unroll
@@ -445,6 +491,20 @@ __global__ __launch_bounds__(256, (G == 1 ? 3 : 2)) void attn_decode_i8_kernel(A
     }
   };
   Tile cur, nxt;
+  // the row of the last position (which the loads past it repeat) into the tile that a wave takes last
+  auto patch = [&](int tb, Tile& cur) {
+    if (!append || tb + 32 < t1) return;
+#pragma unroll
+    for (int sb = 0; sb < 2; ++sb)
+      if (tb + 16 * sb + p >= t1 - 1) {
+        cur.st[sb] = make_uint4(__float_as_uint(s_new.st[0]), __float_as_uint(s_new.st[1]), __float_as_uint(s_new.st[2]), __float_as_uint(s_new.st[3]));
+#pragma unroll
+        for (int c = 0; c < NCB; ++c) cur.k[sb][c] = *reinterpret_cast<const uint4*>(s_new.k + dq * (D / 4) + 16 * c);
+      }
+#pragma unroll
+    for (int c = 0; c < NV; ++c)
+      if (tb + c * PP + pp >= t1 - 1) cur.v[c] = *reinterpret_cast<const uint2*>(s_new.v + dc * 8);
+  };
   auto consume = [&](int tb, const Tile& cur) {
     // One sub-tile of 16 positions at a time (both at once would need the registers of two expanded K
     // tiles); within it the heads of the group advance together, as in the bf16 kernel.
@@ -532,22 +592,29 @@ __global__ __launch_bounds__(256, (G == 1 ? 3 : 2)) void attn_decode_i8_kernel(A
     }
   };
   int tb = t0 + wave * 32;
+  NewLoad<D> fresh;
+  if (append && wave < 2) fresh = load_new<D>(a, seq, kvh, wave, lane);
+  if (tb < t1) load_tile(tb, cur);
+  if (append) {
+    if (wave < 2) put_new<D>(a, fresh, seq, kvh, own, wave, lane, s_new);
+    __syncthreads();
+  }
   if (tb < t1) {
-    load_tile(tb, cur);
     if constexpr (G >= 4) {  // two tiles taking turns do not fit the registers of four heads
       for (; tb + 128 < t1; tb += 128) {
         load_tile(tb + 128, nxt);
         consume(tb, cur);
         cur = nxt;
       }
+      patch(tb, cur);
       consume(tb, cur);
     } else {
       for (;;) {
-        if (tb + 128 >= t1) { consume(tb, cur); break; }
+        if (tb + 128 >= t1) { patch(tb, cur); consume(tb, cur); break; }
         load_tile(tb + 128, nxt);
         consume(tb, cur);
         tb += 128;
-        if (tb + 128 >= t1) { consume(tb, nxt); break; }
+        if (tb + 128 >= t1) { patch(tb, nxt); consume(tb, nxt); break; }
         load_tile(tb + 128, cur);
         consume(tb, nxt);
         tb += 128;
@@ -632,12 +699,15 @@ __global__ __launch_bounds__(256, 2) void attn_decode_i8_mfma_kernel(AttnArgs a)
   if (split >= used) return;
   const int t0 = split * chunk;
   const int t1 = min(L, t0 + chunk);
+  const int own = a.pos_dev ? a.pos_dev[(size_t)seq * a.pos_stride] : a.start;
+  const bool append = a.k_new && split == used - 1 && own >= 0 && own < a.Tmax;  // (then own == t1 - 1)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = lane & 15, rg = lane >> 4;  // K side: position n of a sub-tile, quarter rg; scores: head n, position group rg
   const float scale_l2 = a.scale * OHARA_LOG2E;
 
   __shared__ float s_m[4][G], s_l[4][G];
   __shared__ float s_acc[4][G][D];
+  __shared__ NewRow<D> s_new;
   __shared__ __align__(16) bf16_t s_vt[4][D][LDV];
 
   uint4 qa[NC];
@@ -679,6 +749,30 @@ __global__ __launch_bounds__(256, 2) void attn_decode_i8_mfma_kernel(AttnArgs a)
     }
   };
   bf16_t* vt = &s_vt[wave][0][0];
+  // the row of the last position (which the loads past it repeat) into the tile that a wave takes last
+  auto patch = [&](int tb, Tile& cur) {
+    if (!append || tb + 32 < t1) return;
+    int me = threadIdx.x;  // (taken anew: addresses kept over the loop would be registers too many)
+    asm volatile("" : "+v"(me));
+    const int n = me & 15, rg = (me & 63) >> 4;
+#pragma unroll
+    for (int sb = 0; sb < 2; ++sb)
+      if (tb + 16 * sb + n >= t1 - 1) {
+        cur.ks[sb] = make_uint2(__float_as_uint(s_new.st[0]), __float_as_uint(s_new.st[1]));
+#pragma unroll
+        for (int c = 0; c < 2; ++c) cur.k[sb][c] = *reinterpret_cast<const uint4*>(s_new.k + rg * 32 + 16 * c);
+      }
+    const uint2 v = *reinterpret_cast<const uint2*>(s_new.v + n * 8);
+    const float vs = s_new.st[2], vm = s_new.st[3];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const bool own_row = tb + 8 * rg + c >= t1 - 1;
+      cur.v[c].x = own_row ? v.x : cur.v[c].x;
+      cur.v[c].y = own_row ? v.y : cur.v[c].y;
+      cur.vs[c].x = own_row ? __float_as_uint(vs) : cur.vs[c].x;
+      cur.vs[c].y = own_row ? __float_as_uint(vm) : cur.vs[c].y;
+    }
+  };
   auto consume = [&](int tb, const Tile& cur) {
     // ---- V: dequantise 8 positions x 8 columns, transpose, park as V^T ---------------------------------
     {
@@ -761,14 +855,20 @@ __global__ __launch_bounds__(256, 2) void attn_decode_i8_mfma_kernel(AttnArgs a)
   };
   Tile cur, nxt;
   int tb = t0 + wave * 32;
+  NewLoad<D> fresh;
+  if (append && wave < 2) fresh = load_new<D>(a, seq, kvh, wave, lane);
+  if (tb < t1) load_tile(tb, cur);
+  if (append) {
+    if (wave < 2) put_new<D>(a, fresh, seq, kvh, own, wave, lane, s_new);
+    __syncthreads();
+  }
   if (tb < t1) {
-    load_tile(tb, cur);
     for (;;) {
-      if (tb + 128 >= t1) { consume(tb, cur); break; }
+      if (tb + 128 >= t1) { patch(tb, cur); consume(tb, cur); break; }
       load_tile(tb + 128, nxt);
       consume(tb, cur);
       tb += 128;
-      if (tb + 128 >= t1) { consume(tb, nxt); break; }
+      if (tb + 128 >= t1) { patch(tb, nxt); consume(tb, nxt); break; }
       load_tile(tb + 128, cur);
       consume(tb, nxt);
       tb += 128;
@@ -994,7 +1094,8 @@ int64_t ohara_attn_workspace_bytes(int batch, int h, int h_kv, int dh, int n_spl
 static int attn_cached_impl(const uint16_t* q, const void* kcache, const void* vcache, const float* stats, bool i8,
                             int batch, int seq_len,
                             int h, int h_kv, int dh, int t_max, int pos, const int32_t* pos_dev, int pos_stride, int n_split,
-                            void* workspace, uint16_t* out, void* stream, size_t fixed_counter_bytes = 0) {
+                            void* workspace, uint16_t* out, void* stream, size_t fixed_counter_bytes = 0,
+                            const uint16_t* k_new = nullptr, const uint16_t* v_new = nullptr) {
   if (!q || !kcache || !vcache || !out) return OHARA_EINVAL;
   if (i8 && !stats) return OHARA_EINVAL;
   if (batch < 1 || seq_len < 1 || h < 1 || h_kv < 1 || h % h_kv || dh < 2 || (dh & 1) || dh > 256)
@@ -1007,6 +1108,7 @@ static int attn_cached_impl(const uint16_t* q, const void* kcache, const void* v
   AttnArgs a{};
   a.q = q; a.k = reinterpret_cast<const bf16_t*>(kcache); a.v = reinterpret_cast<const bf16_t*>(vcache); a.out = out;
   a.stats = stats;
+  a.k_new = k_new; a.v_new = v_new;
   a.B = batch; a.S = seq_len; a.H = h; a.Hkv = h_kv; a.D = dh; a.Tmax = t_max; a.start = pos; a.pos_dev = pos_dev;
   a.pos_stride = pos_stride;
   a.nsplit = n_split;
@@ -1067,6 +1169,22 @@ int ohara_attn_cached_ragged_int8(const uint16_t* q, const int8_t* kcache, const
   if (!seq_pos) return OHARA_EINVAL;
   return attn_cached_impl(q, kcache, vcache, stats, true, batch, seq_len, h, h_kv, dh, t_max, 0, seq_pos, 1, n_split,
                           workspace, out, stream);
+}
+
+// The append of one position a sequence (ohara_kv_quant_append_int8, or _ragged with pos_stride 1) and attention over the codes: one
+// launch where a kernel for the heads is there.
+int ohara_attn_append_int8(const uint16_t* q, const uint16_t* k, const uint16_t* v, int8_t* kcache, int8_t* vcache, float* stats, int batch,
+                           int h, int h_kv, int dh, int t_max, int pos, const int32_t* pos_dev, int pos_stride, int n_split, void* workspace,
+                           uint16_t* out, void* stream) {
+  const int G = h_kv > 0 ? h / h_kv : 0;
+  const bool together = k && v && h_kv > 0 && h % h_kv == 0 && (dh == 64 || dh == 128) && (G == 1 || G == 2 || G == 4);
+  if (!together) {
+    const int rc = pos_stride ? ohara_kv_quant_append_ragged_int8(k, v, batch, 1, h_kv, dh, pos_dev, kcache, vcache, stats, t_max, stream)
+                              : ohara_kv_quant_append_int8(k, v, batch, 1, h_kv, dh, pos, pos_dev, kcache, vcache, stats, t_max, stream);
+    if (rc) return rc;
+  }
+  return attn_cached_impl(q, kcache, vcache, stats, true, batch, 1, h, h_kv, dh, t_max, pos, pos_dev, pos_stride, n_split, workspace, out, stream, 0,
+                          together ? k : nullptr, together ? v : nullptr);
 }
 
 // ---- the same attention for callers that cannot allocate -------------------------------------

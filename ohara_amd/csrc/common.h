@@ -245,6 +245,28 @@ __device__ __forceinline__ float lanes_min(float v) {
   else return v;
 }
 
+// A row of D values affine-quantised by a wave, lane l holding columns l, l + 64, ... (kv_cache.py:23-26 in the cache dtype, every
+// operation rounded to bf16: (max - min) / 255 clamped at bf16(1e-8); ((x - min) / scale - 128).round().clamp(-128, 127)).
+template <int N>
+__device__ __forceinline__ void kv_quant_row(const float (&x)[N], int D, int lane, float& scale, float& mn, int8_t (&code)[N]) {
+  float mx = -INFINITY;
+  mn = INFINITY;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (lane + 64 * i < D) {
+      mn = fminf(mn, x[i]);
+      mx = fmaxf(mx, x[i]);
+    }
+  mn = lanes_min<32, 1>(mn);
+  mx = lanes_max<32, 1>(mx);
+  scale = fmaxf(rbf(rbf(mx - mn) / 255.0f), rbf(1e-8f));
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float t = rbf(rbf(rbf(x[i] - mn) / scale) - 128.0f);
+    code[i] = (int8_t)(int)fminf(fmaxf(rintf(t), -128.f), 127.f);
+  }
+}
+
 // Sum / maximum over the wave, every lane gets the result; the order of the adds is that of the
 // butterfly 32, 16, 8, 4, 2, 1.
 __device__ __forceinline__ float wave_sum(float v) {

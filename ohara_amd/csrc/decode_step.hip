@@ -64,11 +64,16 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
       OHARA_RUN(ohara_qkv_rope_ragged_bf16(tiled ? s->xn : s->x, d, L.wqkv, d, tiled ? nullptr : L.norm1, m->eps, B,
                                            seq_len, H, Hkv, Dh, m->cos, m->sin, s->seq_pos, m->t_max, s->q, s->kstage,
                                            s->vstage, stream));
-      rc = ohara_kv_quant_append_ragged_int8(s->kstage, s->vstage, B, seq_len, Hkv, Dh, s->seq_pos, kq, vq, s->kvstats[l],
-                                             m->t_max, stream);
-      if (rc) return rc;
-      OHARA_RUN(ohara_attn_cached_ragged_int8(s->q, kq, vq, s->kvstats[l], B, seq_len, H, Hkv, Dh, m->t_max, s->seq_pos,
-                                              n_split, s->attn_ws, s->attn, stream));
+      if (seq_len == 1) {
+        OHARA_RUN(ohara_attn_append_int8(s->q, s->kstage, s->vstage, kq, vq, s->kvstats[l], B, H, Hkv, Dh, m->t_max, 0, s->seq_pos, 1,
+                                         n_split, s->attn_ws, s->attn, stream));
+      } else {
+        rc = ohara_kv_quant_append_ragged_int8(s->kstage, s->vstage, B, seq_len, Hkv, Dh, s->seq_pos, kq, vq, s->kvstats[l],
+                                               m->t_max, stream);
+        if (rc) return rc;
+        OHARA_RUN(ohara_attn_cached_ragged_int8(s->q, kq, vq, s->kvstats[l], B, seq_len, H, Hkv, Dh, m->t_max, s->seq_pos,
+                                                n_split, s->attn_ws, s->attn, stream));
+      }
     } else if (ragged) {
       // one position per sequence; attention of any length through the split-context kernel
       OHARA_RUN(ohara_qkv_rope_append_ragged_bf16(tiled ? s->xn : s->x, d, L.wqkv, d, tiled ? nullptr : L.norm1, m->eps,
@@ -93,10 +98,15 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
       int8_t* vq = reinterpret_cast<int8_t*>(s->vcache[l]);
       OHARA_RUN(ohara_qkv_rope_bf16(tiled ? s->xn : s->x, d, L.wqkv, d, tiled ? nullptr : L.norm1, m->eps, B, seq_len, H,
                                     Hkv, Dh, m->cos, m->sin, pos, pos_dev, m->t_max, s->q, s->kstage, s->vstage, stream));
-      rc = ohara_kv_quant_append_int8(s->kstage, s->vstage, B, seq_len, Hkv, Dh, pos, pos_dev, kq, vq, s->kvstats[l],
-                                      m->t_max, stream);
-      if (rc) return rc;
-      if (seq_len >= 16 && (Dh == 64 || Dh == 128) && s->kdeq && s->vdeq) {
+      if (seq_len > 1) {
+        rc = ohara_kv_quant_append_int8(s->kstage, s->vstage, B, seq_len, Hkv, Dh, pos, pos_dev, kq, vq, s->kvstats[l],
+                                        m->t_max, stream);
+        if (rc) return rc;
+      }
+      if (seq_len == 1) {
+        OHARA_RUN(ohara_attn_append_int8(s->q, s->kstage, s->vstage, kq, vq, s->kvstats[l], B, H, Hkv, Dh, m->t_max, pos, pos_dev, 0,
+                                         n_split, s->attn_ws, s->attn, stream));
+      } else if (seq_len >= 16 && (Dh == 64 || Dh == 128) && s->kdeq && s->vdeq) {
         const int len = pos + seq_len;
         rc = ohara_kv_dequant_int8(kq, s->kvstats[l], 0, B, len, Hkv, Dh, m->t_max, s->kdeq, stream);
         if (!rc) rc = ohara_kv_dequant_int8(vq, s->kvstats[l], 1, B, len, Hkv, Dh, m->t_max, s->vdeq, stream);
@@ -289,8 +299,10 @@ extern "C" int ohara_moe_forward(const OharaMoeCall* cp, void* stream) {
       int8_t *kq = (int8_t*)c.kcache[l], *vq = (int8_t*)c.vcache[l];
       float* stats = (float*)c.kvstats[l];
       rc = ohara_qkv_rope_bf16(rows, d, L.wqkv, d, norm, c.eps, B, S, H, Hkv, Dh, c.cos, c.sin, c.pos, nullptr, c.t_max, s.q, s.k, s.v, stream);
-      if (!rc) rc = ohara_kv_quant_append_int8(s.k, s.v, B, S, Hkv, Dh, c.pos, nullptr, kq, vq, stats, c.t_max, stream);
-      if (s.dequantise) {
+      if (!rc && S > 1) rc = ohara_kv_quant_append_int8(s.k, s.v, B, S, Hkv, Dh, c.pos, nullptr, kq, vq, stats, c.t_max, stream);
+      if (S == 1) {
+        if (!rc) rc = ohara_attn_append_int8(s.q, s.k, s.v, kq, vq, stats, B, H, Hkv, Dh, c.t_max, c.pos, nullptr, 0, n_split, c.attn_ws, s.attn, stream);
+      } else if (s.dequantise) {
         const int len = c.pos + S;
         if (!rc) rc = ohara_kv_dequant_int8(kq, stats, 0, B, len, Hkv, Dh, c.t_max, s.kd, stream);
         if (!rc) rc = ohara_kv_dequant_int8(vq, stats, 1, B, len, Hkv, Dh, c.t_max, s.vd, stream);

@@ -30,30 +30,14 @@ __global__ __launch_bounds__(256) void kv_quant_append_kernel(const bf16_t* k, c
   const bf16_t* src = (which ? v : k) + ((size_t)row * Hkv + h) * D;
   const size_t slot = ((size_t)seq * Tmax + pos) * Hkv + h;
   int8_t* dst = (which ? vq : kq) + slot * D;
-  float x[8];
-  float mn = INFINITY, mx = -INFINITY;
+  float x[8], scale, mn;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int d = lane + 64 * i;
-    x[i] = d < D ? bf2f(src[d]) : 0.f;
-    if (d < D) {
-      mn = fminf(mn, x[i]);
-      mx = fmaxf(mx, x[i]);
-    }
-  }
-  mn = lanes_min<32, 1>(mn);
-  mx = lanes_max<32, 1>(mx);
-  // kv_cache.py:23-24 in the cache dtype: (max - min) -> bf16, / 255 -> bf16, clamp at bf16(1e-8)
-  const float scale = fmaxf(rbf(rbf(mx - mn) / 255.0f), rbf(1e-8f));
+  for (int i = 0; i < 8; ++i) x[i] = lane + 64 * i < D ? bf2f(src[lane + 64 * i]) : 0.f;
+  int8_t code[8];
+  kv_quant_row(x, D, lane, scale, mn, code);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int d = lane + 64 * i;
-    if (d < D) {
-      // kv_cache.py:26: ((x - min) / scale - 128).round().clamp(-128, 127), each op rounded to bf16
-      const float t = rbf(rbf(rbf(x[i] - mn) / scale) - 128.0f);
-      dst[d] = (int8_t)(int)fminf(fmaxf(rintf(t), -128.f), 127.f);
-    }
-  }
+  for (int i = 0; i < 8; ++i)
+    if (lane + 64 * i < D) dst[lane + 64 * i] = code[i];
   if (lane == 0) {
     float* rec = stats + (((size_t)seq * Hkv + h) * Tmax + pos) * 4 + 2 * which;
     *reinterpret_cast<float2*>(rec) = make_float2(scale, mn);

@@ -435,3 +435,55 @@ def test_bitnet_model_with_int8_caches(cuda, P):
     mixed = [model.build_kv_cache(1, int8=True)[0]] + model.build_kv_cache(1)[1:]
     with pytest.raises(ValueError, match="same KV cache mode"):
         model(ids[:1, :2].to(cuda), mixed, 0)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,Hkv", [(4, 4), (4, 2), (8, 2), (6, 2), (16, 1)])
+@pytest.mark.parametrize("positions", [(0,), (31, 32, 33), (127, 128, 0, 126), (511, 4, 600), (639, 640, 3), (2900,)])
+def test_append_and_attention_in_one_launch(cuda, D, H, Hkv, positions):
+    """Bit for bit the two launches: codes, statistics and attention, positions at the edges of tiles and chunks and past the cache, one
+    position for all sequences and one each."""
+    from ohara_amd._lib import check, lib
+
+    B, T = len(positions), 640 if max(positions) < 700 else 3000
+    g = torch.Generator(device=cuda).manual_seed(D + H + sum(positions))
+    stream = torch.cuda.current_stream().cuda_stream
+    q = torch.randn(B, H * D, generator=g, device=cuda).to(torch.bfloat16)
+    k, v = (torch.randn(B, Hkv, D, generator=g, device=cuda).to(torch.bfloat16) for _ in range(2))
+    codes = [torch.randint(-128, 128, (B, T, Hkv, D), generator=g, device=cuda, dtype=torch.int32).to(torch.int8) for _ in range(2)]
+    stats = torch.rand(B, Hkv, T, 4, generator=g, device=cuda) / 50
+    for b, pos in enumerate(positions):
+        stats[b, :, min(pos, T):] = float("nan")  # nothing is there yet (a position past the cache is not appended)
+    pos_dev = torch.tensor(positions, dtype=torch.int32, device=cuda)
+    for n_split in (1, 7):
+        for ragged in (True, False):
+            if not ragged and positions[0] >= T:
+                continue
+            pos = 0 if ragged else positions[0]
+            ends = None if ragged else stats.clone()
+            if ends is not None:
+                ends[:, :, :pos] = torch.nan_to_num(ends[:, :, :pos])
+                ends[:, :, pos:] = float("nan")
+            results = []
+            for together in (False, True):
+                kq, vq, st = codes[0].clone(), codes[1].clone(), (stats if ragged else ends).clone()
+                ws = torch.zeros(lib().ohara_attn_workspace_bytes(B, H, Hkv, D, n_split), dtype=torch.uint8, device=cuda)
+                out = torch.empty(B, H * D, dtype=torch.bfloat16, device=cuda)
+                cache = (kq.data_ptr(), vq.data_ptr(), st.data_ptr())
+                if together:
+                    check(lib().ohara_attn_append_int8(q.data_ptr(), k.data_ptr(), v.data_ptr(), *cache, B, H, Hkv, D, T, pos,
+                                                       pos_dev.data_ptr() if ragged else None, int(ragged), n_split, ws.data_ptr(),
+                                                       out.data_ptr(), stream), "append")
+                elif ragged:
+                    check(lib().ohara_kv_quant_append_ragged_int8(k.data_ptr(), v.data_ptr(), B, 1, Hkv, D, pos_dev.data_ptr(), *cache, T,
+                                                                  stream), "append")
+                    check(lib().ohara_attn_cached_ragged_int8(q.data_ptr(), *cache, B, 1, H, Hkv, D, T, pos_dev.data_ptr(), n_split,
+                                                              ws.data_ptr(), out.data_ptr(), stream), "attention")
+                else:
+                    check(lib().ohara_kv_quant_append_int8(k.data_ptr(), v.data_ptr(), B, 1, Hkv, D, pos, None, *cache, T, stream), "append")
+                    check(lib().ohara_attn_cached_int8(q.data_ptr(), *cache, B, 1, H, Hkv, D, T, pos, None, n_split, ws.data_ptr(),
+                                                       out.data_ptr(), stream), "attention")
+                results.append((out.view(torch.int16), kq, vq, st.view(torch.int32)))
+            for a, b in zip(*results):
+                assert torch.equal(a, b)
+            assert not results[1][0].view(torch.bfloat16).isnan().any()
