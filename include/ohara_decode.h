@@ -662,6 +662,15 @@ int ohara_bitnet_decode_persistent(const OharaBitModel* m, const OharaDecodeStat
 int ohara_linear_bias_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, const uint16_t* bias, int rows,
                            int epilogue, const uint16_t* add1, int ld1, const uint16_t* add2, int ld2, uint16_t* out,
                            int ldo, void* stream);
+/* OHARA_LIN_BIAS_ADD2 with room (16-byte aligned, _bytes; 0: none needed) for a product in parts of its depth, where rows are too few to
+ * keep the CUs busy over all of it.  Too little room or NULL: as without. */
+int64_t ohara_linear_bias_add2_bytes(int rows, int n, int k);
+int ohara_linear_bias_add2_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, const uint16_t* bias, int rows, const uint16_t* add1,
+                                int ld1, const uint16_t* add2, int ld2, uint16_t* out, int ldo, void* workspace, int64_t workspace_bytes, void* stream);
+/* resid (rows, n) += x W^T, then, where norm_w is given, xn = its RMSNorm (ohara_rmsnorm_bf16); room as above. */
+int64_t ohara_gemm_residual_norm_bytes(int rows, int n, int k);
+int ohara_gemm_residual_norm_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, int rows, uint16_t* resid, const uint16_t* norm_w,
+                                  float eps, uint16_t* xn, void* workspace, int64_t workspace_bytes, void* stream);
 /* The head of a Phi block in one launch (phi.py:150, :81-87, :95, :50-51): h = LayerNorm(x), then
  * [q; k; v; fc1] = h @ W^T + bias with W the packed vertical concatenation of q_proj, k_proj, v_proj
  * (d rows each) and mlp.fc1 (ff rows): q rows -> q (leading dimension ldq), k / v rows -> the

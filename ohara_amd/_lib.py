@@ -129,6 +129,10 @@ _PROTOS = {
     "ohara_swiglu_perm": (_i, [_i, _p]),
     "ohara_embed_bf16": (_i, [_p, _p, _p, _i, _i, _i, _p]),
     "ohara_rmsnorm_bf16": (_i, [_p, _p, _p, _i, _i, _f, _p]),
+    "ohara_linear_bias_add2_bytes": (_i64, [_i, _i, _i]),
+    "ohara_linear_bias_add2_bf16": (_i, [_p, _i, _p, _i, _i, _p, _i, _p, _i, _p, _i, _p, _i, _p, _i64, _p]),
+    "ohara_gemm_residual_norm_bytes": (_i64, [_i, _i, _i]),
+    "ohara_gemm_residual_norm_bf16": (_i, [_p, _i, _p, _i, _i, _i, _p, _p, _f, _p, _p, _i64, _p]),
     "ohara_gemm_skinny_bf16": (_i, [_p, _i, _p, _i, _i, _p, _f, _i, _i, _p, _i, _p, _i, _p]),
     "ohara_gemm_tile_of": (_i, [_i, _i, _i]),
     "ohara_gemm_bf16": (_i, [_p, _i, _p, _i, _i, _i, _i, _p, _i, _p, _i, _p]),

@@ -52,7 +52,8 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
   OHARA_RUN(ohara_embed_bf16(s->ids, m->token_emb, s->x, R, d, m->vocab, stream));
   for (int l = 0; l < m->n_layers; ++l) {
     const OharaLayer& L = m->layers[l];
-    if (tiled) {  // many rows: normalise once, then the tiled MFMA kernel (launches are not numbered)
+    if (tiled && l == 0) {  // many rows: normalise once, then the tiled MFMA kernel (launches are not numbered); later layers' norms
+                            // come with the residual before them
       rc = ohara_rmsnorm_bf16(s->x, L.norm1, s->xn, R, d, m->eps, stream);
       if (rc) return rc;
     }
@@ -117,22 +118,19 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
                                          n_split, s->attn_ws, s->attn, stream));
       }
     }
-    OHARA_RUN(ohara_gemm_skinny_bf16(s->attn, H * Dh, L.wo, d, H * Dh, nullptr, m->eps, R, OHARA_EPI_RESIDUAL, s->x, d,
-                                s->x, d, stream));
-    if (tiled) {
-      rc = ohara_rmsnorm_bf16(s->x, L.norm2, s->xn, R, d, m->eps, stream);
-      if (rc) return rc;
-    }
+    if (tiled)
+      OHARA_RUN(ohara_gemm_residual_norm_bf16(s->attn, H * Dh, L.wo, d, H * Dh, R, s->x, L.norm2, m->eps, s->xn, room_at, room, stream));
+    else
+      OHARA_RUN(ohara_gemm_skinny_bf16(s->attn, H * Dh, L.wo, d, H * Dh, nullptr, m->eps, R, OHARA_EPI_RESIDUAL, s->x, d, s->x, d, stream));
     OHARA_RUN(ohara_gemm_skinny_bf16(tiled ? s->xn : s->x, d, L.wgu, m->d_ff, d, tiled ? nullptr : L.norm2, m->eps, R,
                                      OHARA_EPI_SWIGLU, nullptr, 0, s->act, m->d_ff, stream));
-    OHARA_RUN(ohara_gemm_skinny_bf16(s->act, m->d_ff, L.wdown, d, m->d_ff, nullptr, m->eps, R, OHARA_EPI_RESIDUAL, s->x, d,
-                                s->x, d, stream));
+    const uint16_t* after = l + 1 < m->n_layers ? m->layers[l + 1].norm1 : logits_mode == OHARA_LOGITS_ALL ? m->final_norm : nullptr;
+    if (tiled)
+      OHARA_RUN(ohara_gemm_residual_norm_bf16(s->act, m->d_ff, L.wdown, d, m->d_ff, R, s->x, after, m->eps, s->xn, room_at, room, stream));
+    else
+      OHARA_RUN(ohara_gemm_skinny_bf16(s->act, m->d_ff, L.wdown, d, m->d_ff, nullptr, m->eps, R, OHARA_EPI_RESIDUAL, s->x, d, s->x, d, stream));
   }
   if (logits_mode == OHARA_LOGITS_ALL) {
-    if (tiled) {
-      rc = ohara_rmsnorm_bf16(s->x, m->final_norm, s->xn, R, d, m->eps, stream);
-      if (rc) return rc;
-    }
     OHARA_RUN(ohara_gemm_skinny_bf16(tiled ? s->xn : s->x, d, m->w_vocab, m->vocab, d, tiled ? nullptr : m->final_norm,
                                      m->eps, R, OHARA_EPI_STORE, nullptr, 0, s->logits, m->vocab, stream));
   } else if (logits_mode == OHARA_LOGITS_LAST) {

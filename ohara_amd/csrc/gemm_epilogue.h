@@ -59,6 +59,8 @@ struct GemmArgs {
 
 // gemm_tile.hip: the tiled kernel for calls with many rows (a.B rows, no fused norm).
 int ohara_launch_gemm_tile(const GemmArgs& a, int epi, int packed_rows, hipStream_t st);
+int ohara_depth_parts(int rows, int packed_rows, int k, float merge_us);
+int ohara_launch_gemm_parts(const GemmArgs& a, int packed_rows, int parts, float* sums, hipStream_t st);
 
 // Rows from which on rows that are normed once and multiplied in tiles are the quicker way, where the strip kernels norm them in every
 // workgroup (or, without a norm, read them there) - 17 at wide models, 65 at narrow ones.  us, normed strips / a norm and tiles, cold

@@ -15,6 +15,8 @@
 //             SwiGLU            ohara/modules/mlp.py:152
 //             rotary + KV append ohara/embeddings_pos/rotary.py:55-93,
 //                               ohara/modules/kv_cache.py:104-105
+#include <algorithm>
+
 #include "gemm_epilogue.h"
 
 #include <type_traits>
@@ -830,6 +832,88 @@ __global__ void pack_rows_kernel(const bf16_t* w, int n, int k, int ldw, const i
   dst[idx] = make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
 }
 
+// Eight columns of a row, the parts' sums added in their order.
+template <int P>
+__device__ __forceinline__ void merged8(const float* sums, int rows, int n, int row, int c, float (&f)[8]) {
+  f32x4 lo[P], hi[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const float* at = sums + ((size_t)p * rows + row) * n + c;
+    lo[p] = *reinterpret_cast<const f32x4*>(at);
+    hi[p] = *reinterpret_cast<const f32x4*>(at + 4);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f[i] = lo[0][i];
+    f[4 + i] = hi[0][i];
+#pragma unroll
+    for (int p = 1; p < P; ++p) {
+      f[i] += lo[p][i];
+      f[4 + i] += hi[p][i];
+    }
+  }
+}
+
+// resid += the product (EPI_RESIDUAL's rounding), a row a workgroup, and its RMSNorm (ohara/modules/norm.py:16-21) where the next
+// projection wants it.  n % 16 == 0, n <= 4096: at most two columns of eight a thread.
+template <int P>
+__global__ __launch_bounds__(256) void merge_norm_kernel(const float* sums, int rows, int n, bf16_t* resid, const bf16_t* norm_w, bf16_t* xn, float eps) {
+  __shared__ float red[4];
+  const int row = blockIdx.x, step = 8 * blockDim.x;
+  bf16_t* x = resid + (size_t)row * n;
+  uint4 v[2], w[2];
+  float ss = 0.f;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int c = 8 * threadIdx.x + t * step;
+    if (c >= n) continue;
+    float f[8];
+    const uint4 r = ldg16(x + c);
+    if (norm_w) w[t] = ldg16(norm_w + c);
+    merged8<P>(sums, rows, n, row, c, f);
+    const uint32_t u[4] = {r.x, r.y, r.z, r.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o[i] = pack_bf(lo_bf(u[i]) + rbf(f[2 * i]), hi_bf(u[i]) + rbf(f[2 * i + 1]));
+      ss = __builtin_fmaf(lo_bf(o[i]), lo_bf(o[i]), ss);
+      ss = __builtin_fmaf(hi_bf(o[i]), hi_bf(o[i]), ss);
+    }
+    v[t] = make_uint4(o[0], o[1], o[2], o[3]);
+    *reinterpret_cast<uint4*>(x + c) = v[t];
+  }
+  if (!norm_w) return;
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  ss = red[0];
+  for (int i = 1; i < (int)(blockDim.x >> 6); ++i) ss += red[i];
+  const float rinv = 1.0f / sqrtf(ss / (float)n + eps);
+  auto two = [&](uint32_t xx, uint32_t ww) { return pack_bf(rbf(lo_bf(xx) * rinv) * lo_bf(ww), rbf(hi_bf(xx) * rinv) * hi_bf(ww)); };
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int c = 8 * threadIdx.x + t * step;
+    if (c < n) *reinterpret_cast<uint4*>(xn + (size_t)row * n + c) = make_uint4(two(v[t].x, w[t].x), two(v[t].y, w[t].y), two(v[t].z, w[t].z), two(v[t].w, w[t].w));
+  }
+}
+
+// EPI_BIAS_ADD2 of the merged product.
+template <int P>
+__global__ __launch_bounds__(256) void merge_add2_kernel(GemmArgs a, const float* sums) {
+  const int row = blockIdx.x;
+  for (int c = 8 * threadIdx.x; c < a.N; c += 2048) {
+    float f[8];
+    const uint4 b = ldg16(a.bias + c), r1 = ldg16(a.resid + (size_t)row * a.ldr + c), r2 = ldg16(a.resid2 + (size_t)row * a.ldr2 + c);
+    merged8<P>(sums, a.B, a.N, row, c, f);
+    const uint32_t bu[4] = {b.x, b.y, b.z, b.w}, u1[4] = {r1.x, r1.y, r1.z, r1.w}, u2[4] = {r2.x, r2.y, r2.z, r2.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      o[i] = pack_bf(rbf(lo_bf(u1[i]) + rbf(f[2 * i] + lo_bf(bu[i]))) + lo_bf(u2[i]), rbf(hi_bf(u1[i]) + rbf(f[2 * i + 1] + hi_bf(bu[i]))) + hi_bf(u2[i]));
+    *reinterpret_cast<uint4*>(a.out + (size_t)row * a.ldo + c) = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
 }  // namespace
 
 extern "C" {
@@ -885,6 +969,72 @@ int ohara_linear_bias_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n
   a.resid = add1; a.ldr = ld1; a.resid2 = add2; a.ldr2 = ld2;
   if (ohara_tiles_win(rows, k)) return ohara_launch_gemm_tile(a, epi, (n + 15) / 16 * 16, (hipStream_t)stream);
   return launch_skinny(a, epi, (n + 15) / 16 * 16, (hipStream_t)stream);
+}
+
+// ---- products in parts of the depth (ohara_depth_parts), merged by rows ---------------------------------------------------------
+// The merge of a residual is the norm behind it too: 1 us more than that norm's launch; the other one is a launch of its own, 3.  (Up to 32
+// rows a strip's workgroup over the whole depth is the faster one.)
+static int residual_parts(int rows, int n, int k) {
+  return rows > 32 && (n & 15) == 0 && n <= 4096 ? ohara_depth_parts(rows, n, k, 1.f) : 1;
+}
+static int bias_parts(int rows, int n, int k) { return rows > 32 && (n & 15) == 0 ? ohara_depth_parts(rows, n, k, 3.f) : 1; }
+static int64_t parts_bytes(int parts, int rows, int n) { return parts > 1 ? (int64_t)parts * rows * n * (int64_t)sizeof(float) : 0; }
+
+int64_t ohara_gemm_residual_norm_bytes(int rows, int n, int k) {
+  if (rows < 1 || n < 1 || k < 1) return OHARA_EINVAL;
+  return parts_bytes(residual_parts(rows, n, k), rows, n);
+}
+
+int ohara_gemm_residual_norm_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, int rows, uint16_t* resid, const uint16_t* norm_w,
+                                  float eps, uint16_t* xn, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!x || !wp || !resid || n < 1 || k < 1 || rows < 1 || (norm_w && !xn)) return OHARA_EINVAL;
+  const int parts = residual_parts(rows, n, k);
+  const bool aligned = !(((uintptr_t)x | (uintptr_t)resid | (uintptr_t)norm_w | (uintptr_t)xn | (uintptr_t)workspace) & 15) && !(ldx & 7) && ldx >= k;
+  if (parts > 1 && aligned && workspace && workspace_bytes >= parts_bytes(parts, rows, n)) {
+    GemmArgs a{};
+    a.wp = reinterpret_cast<const uint4*>(wp);
+    a.x = x; a.ldx = ldx; a.B = rows; a.N = n; a.K = k;
+    float* sums = (float*)workspace;
+    const int rc = ohara_launch_gemm_parts(a, n, parts, sums, (hipStream_t)stream);
+    if (rc) return rc;
+    const dim3 grid(rows), block(std::min(256, (n / 8 + 63) / 64 * 64));
+#define OHARA_MERGE(P) hipLaunchKernelGGL(merge_norm_kernel<P>, grid, block, 0, (hipStream_t)stream, sums, rows, n, resid, norm_w, xn, eps)
+    if (parts == 2) OHARA_MERGE(2);
+    else if (parts == 4) OHARA_MERGE(4);
+    else OHARA_MERGE(8);
+#undef OHARA_MERGE
+    return ohara_launch_status();
+  }
+  const int rc = ohara_gemm_skinny_bf16(x, ldx, wp, n, k, nullptr, eps, rows, OHARA_EPI_RESIDUAL, resid, n, resid, n, stream);
+  return rc || !norm_w ? rc : ohara_rmsnorm_bf16(resid, norm_w, xn, rows, n, eps, stream);
+}
+
+int64_t ohara_linear_bias_add2_bytes(int rows, int n, int k) {
+  if (rows < 1 || n < 1 || k < 1) return OHARA_EINVAL;
+  return parts_bytes(bias_parts(rows, n, k), rows, n);
+}
+
+int ohara_linear_bias_add2_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, const uint16_t* bias, int rows, const uint16_t* add1,
+                                int ld1, const uint16_t* add2, int ld2, uint16_t* out, int ldo, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!x || !wp || !bias || !add1 || !add2 || !out || n < 1 || k < 1 || rows < 1 || ldx < k || ld1 < n || ld2 < n || ldo < n) return OHARA_EINVAL;
+  const int parts = bias_parts(rows, n, k);
+  const bool aligned = !(((uintptr_t)x | (uintptr_t)bias | (uintptr_t)add1 | (uintptr_t)add2 | (uintptr_t)out | (uintptr_t)workspace) & 15) &&
+                       !((ldx | ld1 | ld2 | ldo) & 7);
+  if (parts == 1 || !aligned || !workspace || workspace_bytes < parts_bytes(parts, rows, n))
+    return ohara_linear_bias_bf16(x, ldx, wp, n, k, bias, rows, OHARA_LIN_BIAS_ADD2, add1, ld1, add2, ld2, out, ldo, stream);
+  GemmArgs a{};
+  a.wp = reinterpret_cast<const uint4*>(wp);
+  a.x = x; a.ldx = ldx; a.B = rows; a.N = n; a.K = k;
+  a.bias = bias; a.resid = add1; a.ldr = ld1; a.resid2 = add2; a.ldr2 = ld2; a.out = out; a.ldo = ldo;
+  float* sums = (float*)workspace;
+  const int rc = ohara_launch_gemm_parts(a, n, parts, sums, (hipStream_t)stream);
+  if (rc) return rc;
+#define OHARA_MERGE(P) hipLaunchKernelGGL(merge_add2_kernel<P>, dim3(rows), dim3(256), 0, (hipStream_t)stream, a, sums)
+  if (parts == 2) OHARA_MERGE(2);
+  else if (parts == 4) OHARA_MERGE(4);
+  else OHARA_MERGE(8);
+#undef OHARA_MERGE
+  return ohara_launch_status();
 }
 
 int ohara_phi_block_in_bf16(const uint16_t* x, int ldx, const uint16_t* ln_w, const uint16_t* ln_b, float eps,

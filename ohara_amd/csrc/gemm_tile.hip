@@ -1,6 +1,6 @@
 // Tiled MFMA GEMM for the batched (prefill) projections: y = epi(x W^T) with many rows.
 //
-// The walk over K is tile_product (lds_tile.h); the sums do not depend on the tile.
+// The walk over K is tile_product (lds_tile.h); the sums do not depend on the tile, but on the parts of the depth they are made of.
 //
 // What bounds it: in large tiles the loads into LDS, the LDS reads and the matrix pipe together (8192 x 8192 x 8192 on zeros: 815 us;
 // without the loads 615, without the reads 749, with neither 535; on random data the chip's clock falls under the products: 960), in
@@ -254,6 +254,47 @@ int launch_tile(const GemmArgs& a, int nstrips, hipStream_t st) {
   return ohara_launch_status();
 }
 
+// A part of the depth a workgroup, its fp32 sums to [part][row][16 nstrips]: where tiles over the whole depth are too few for the CUs or
+// each of them takes in too much (50 GB/s a CU: 32 x 32 over 5632 are 720 KB).
+template <class C>
+__global__ __launch_bounds__(C::NW * 64, 2) void gemm_part_kernel(GemmArgs a, int MT, int NT, int nstrips, int parts, float* out) {
+  constexpr int FM = C::FM, FN = C::FN;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int T = MT * NT * parts, xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+  const int base = T >> 3, rem = T & 7;
+  if (q >= base + (xcd < rem ? 1 : 0)) return;
+  const int id = xcd * base + min(xcd, rem) + q, part = id / (MT * NT), pid = id - part * MT * NT;  // (an XCD: a part or two)
+  const int row0 = (pid % MT) * C::TM, strip0 = (pid / MT) * C::TS;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / C::WN, wn = wave % C::WN, m = lane & 15, g = lane >> 4;
+  const int depth = a.K / parts;  // a multiple of 128
+  XOffsets<C, true> x;
+#pragma unroll
+  for (int i = 0; i < C::XPW; ++i) x.set(i, wave, lane, (typename XOffsets<C, true>::type)(min(row0 + x.row(i, wave, lane), a.B - 1) - row0) * a.ldx);
+  f32x4 acc[FN][FM];
+  tile_product<C, true>(acc, reinterpret_cast<const char*>(a.x + (size_t)row0 * a.ldx + (size_t)part * depth), x, a.wp + (size_t)part * (depth / 32) * 64,
+                        strip0, nstrips, depth, wave, lane, smem, a.K / 32);
+  const int rbase = row0 + wm * FM * 16, sbase = strip0 + wn * FN;
+#pragma unroll
+  for (int u = 0; u < FN; ++u)
+#pragma unroll
+    for (int t = 0; t < FM; ++t) {
+      const int b = rbase + t * 16 + m;
+      if (b < a.B && sbase + u < nstrips)
+        *reinterpret_cast<f32x4*>(out + (((size_t)part * a.B + b) * nstrips + sbase + u) * 16 + 4 * g) = acc[u][t];
+    }
+}
+
+template <class C>
+int launch_part(const GemmArgs& a, int nstrips, int parts, float* out, hipStream_t st) {
+  const int64_t MT = (a.B + C::TM - 1) / C::TM, NT = (nstrips + C::TS - 1) / C::TS;
+  if (MT * NT * parts > INT32_MAX - 8) return OHARA_ESIZE;
+  if (C::LDS > 64 * 1024) (void)hipFuncSetAttribute((const void*)gemm_part_kernel<C>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+  hipLaunchKernelGGL((gemm_part_kernel<C>), dim3((unsigned)(MT * NT * parts + 7) / 8 * 8), dim3(C::NW * 64), C::LDS, st, a, (int)MT, (int)NT, nstrips,
+                     parts, out);
+  return ohara_launch_status();
+}
+
 //           waves fragments k-steps slots ahead
 typedef Tile<2, 2, 1, 1, 4, 3, 1> T32;       //  32 x  32
 typedef Tile<2, 2, 2, 2, 4, 2, 0> T64;       //  64 x  64
@@ -316,7 +357,45 @@ int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
   }
 }
 
+float least_time(int rows, int strips, int K) { return tile_time(TIMES[fastest_tile(rows, strips, K)], rows, strips, K); }
+
 }  // namespace
+
+// In how many parts the depth is multiplied: those of least time, the tiles' (as above) and the merge's, which is the sums written and
+// read at 8 TB/s (they stay in the caches) and merge_us.  us with what follows the product, whole / in parts:
+//   2048 x 5632, residual and norm, 33, 65, 192, 400, 700, 1500 rows  21.1 21.6 26.8 41.2 42.2 58.8 / 11.2 14.6 19.0 28.6 33.2 54.5
+//   768 x 3072                      65, 128, 256, 512, 700            11.9 11.9 12.0 13.7 17.6      /  7.5  8.0  9.9 12.3 14.2
+//   2560 x 10240, bias and addends  33, 128, 256, 700, 1000           31.7 43.0 59.4 72.3 116       / 20.1 28.3 32.7 52.8 71.1
+// and 2048 x 2048 in parts at 33 rows (10.3 / 7.6), whole from 700 on (17.1).  (At 4 TB/s the rule left 512 x 768 x 3072 and 700 rows of
+// the other two whole.)
+int ohara_depth_parts(int rows, int packed_rows, int k, float merge_us) {
+  const int strips = packed_rows / 16;
+  int best = 1;
+  float low = 0.95f * least_time(rows, strips, k);
+  for (int p = 2; p <= 8; p *= 2) {
+    if (k % (128 * p) || k / p < 512 || (int64_t)strips * p > INT32_MAX / 16) continue;
+    const float t = least_time(rows, strips * p, k / p) + (float)p * rows * strips * 16 * 8 * (1.f / 8e6f) + merge_us;
+    if (t < low) {
+      low = t;
+      best = p;
+    }
+  }
+  return best;
+}
+
+// a.x on 16 bytes, its rows a.ldx % 8 == 0 apart; parts as ohara_depth_parts; sums: [part][row][packed_rows].
+int ohara_launch_gemm_parts(const GemmArgs& a, int packed_rows, int parts, float* sums, hipStream_t st) {
+  const int nstrips = packed_rows / 16;
+  if (parts < 2 || a.K % (128 * parts) || ((uintptr_t)a.x & 15) || (a.ldx & 7) || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return OHARA_EINVAL;
+  switch (fastest_tile(a.B, nstrips * parts, a.K / parts)) {
+    case 0: return launch_part<T32>(a, nstrips, parts, sums, st);
+    case 1: return launch_part<T64>(a, nstrips, parts, sums, st);
+    case 2: return launch_part<T64x128>(a, nstrips, parts, sums, st);
+    case 3: return launch_part<T128>(a, nstrips, parts, sums, st);
+    case 4: return launch_part<T128x192>(a, nstrips, parts, sums, st);
+    default: return launch_part<T256>(a, nstrips, parts, sums, st);
+  }
+}
 
 // Launcher shared with the skinny entry points (declared there).
 int ohara_launch_gemm_tile(const GemmArgs& a, int epi, int packed_rows, hipStream_t st) {

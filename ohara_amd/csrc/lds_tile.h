@@ -75,13 +75,14 @@ __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
 
 template <class C, bool ALIGNED>
 __device__ __forceinline__ void tile_product(f32x4 (&acc)[C::FN][C::FM], const char* xb, const XOffsets<C, ALIGNED>& x, const uint4* wp,
-                                             int strip0, int nstrips, int K, int wave, int lane, unsigned char* smem) {
+                                             int strip0, int nstrips, int K, int wave, int lane, unsigned char* smem, int strip_steps = 0) {
   constexpr int FM = C::FM, FN = C::FN, KH = C::KH, NST = C::NST, NW = C::NW, XL = C::XL, WL = C::WL, LPW = C::LPW;
   constexpr int STAGE = C::STAGE, KB = 32 * KH;
   const int wm = wave / C::WN, wn = wave % C::WN;
   const int m = lane & 15, g = lane >> 4;
   const int KS = (K + 31) >> 5, nsteps = (KS + KH - 1) / KH;
   const bool tail = K % KB != 0;                           // the last step is not full
+  const int SS = strip_steps ? strip_steps : KS;           // k-steps from strip to strip (more than KS: a part of the depth)
   const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
   const char* wb = reinterpret_cast<const char*>(wp);
   const uint32_t lane16 = lane * 16;
@@ -103,7 +104,7 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[C::FN][C::FM], const c
     for (int i = 0; i < WL / NW; ++i) {
       const int t = wave + i * NW;  // strip t / KH, k-step t % KH; past the end: the last one, never used
       const int strip = min(strip0 + t / KH, nstrips - 1), j = min(KH * s + t % KH, KS - 1);
-      load_lds16(slot + (XL + t) * 1024, wb + ((size_t)strip * KS + j) * 1024, lane16);
+      load_lds16(slot + (XL + t) * 1024, wb + ((size_t)strip * SS + j) * 1024, lane16);
     }
   };
 #pragma unroll

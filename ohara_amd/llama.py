@@ -157,7 +157,8 @@ class _Buffers:
         self.attn = torch.empty(rows, hd, dtype=BF16, device=dev)
         self.act = torch.empty(rows, model.act_width, dtype=BF16, device=dev)
         self.xn = torch.empty(rows, c.hidden_size, dtype=BF16, device=dev) if rows > ops.norm_rows(c.hidden_size) else None
-        self.attn_ws = ops.attn_workspace(batch, c.num_attention_heads, model.kv_heads, model.head_dim, n_split, dev)
+        self.attn_ws = ops.attn_workspace(batch, c.num_attention_heads, model.kv_heads, model.head_dim, n_split, dev,
+                                          4 * batch * model.kv_heads if rows > batch else None)
         self.step_state = torch.zeros(4, dtype=torch.int32, device=dev)
         self.logits = None
         self.history = None
@@ -312,9 +313,11 @@ class Llama:
             for k in [k for k in self._buffers if k[1] > k[0] and k != key]:
                 del self._buffers[k]
             n_split, c = self.default_n_split(batch), self.config
-            if rows > batch:  # several tokens a sequence: the workspace holds their partial results (at most 17 MB)
+            if rows > batch:  # several tokens a sequence: the workspace holds their partial results
                 h, dh, S = c.num_attention_heads, self.head_dim, rows // batch
                 room = ops.lib().ohara_attn_prefill_ws_bytes(batch, S, h, self.kv_heads, dh, max(0, c.max_sequence_length - S))
+                if rows > ops.norm_rows(c.hidden_size):
+                    room = max(room, *(ops.lib().ohara_gemm_residual_norm_bytes(rows, c.hidden_size, k) for k in (h * dh, self.act_width)))
                 n_split = max(n_split, -(-room // (batch * h * (4 * dh + 8))))
             buf = _Buffers(self, batch, rows, n_split)
             self._buffers[key] = buf

@@ -207,11 +207,14 @@ def qkv_rope(x, wqkv: PackedLinear, norm_w, eps, h, h_kv, dh, cos, sin, pos, t_m
     return q, k, v
 
 
-def attn_workspace(batch, h, h_kv, dh, n_split, device) -> torch.Tensor:
+def attn_workspace(batch, h, h_kv, dh, n_split, device, zeros=None) -> torch.Tensor:
+    """``zeros``: how many bytes at the start are cleared (the counters; all of it by default)."""
     n = lib().ohara_attn_workspace_bytes(batch, h, h_kv, dh, n_split)
     if n < 0:
         raise ValueError("bad attention workspace shape")
-    return torch.zeros(n, dtype=torch.uint8, device=device)
+    ws = torch.empty(n, dtype=torch.uint8, device=device)
+    ws[:zeros].zero_()
+    return ws
 
 
 def attn_cached(q, kcache, vcache, h, h_kv, dh, pos, n_split, workspace, out=None, pos_dev=None, seq_len=1,
@@ -587,6 +590,14 @@ def linear_bias(x, w: PackedLinear, bias, epilogue: str = "bias", add1=None, add
     for t in (add1, add2):
         if t is not None and (t.dtype != BF16 or t.stride(1) != 1):
             raise ValueError("addends must be bf16 with unit column stride")
+    if epilogue == "add2" and add1 is not None and add2 is not None:
+        room = lib().ohara_linear_bias_add2_bytes(rows, w.n, w.k)
+        if room > 0:  # few rows for the depth: a product in parts
+            workspace = torch.empty(room, dtype=torch.uint8, device=x.device)
+            check(lib().ohara_linear_bias_add2_bf16(
+                _ptr(x), x.stride(0), _ptr(w.data), w.n, w.k, _ptr(bias), rows, _ptr(add1), add1.stride(0), _ptr(add2),
+                add2.stride(0), _ptr(out), out.stride(0), _ptr(workspace), room, _stream()), "linear_bias")
+            return out
     check(
         lib().ohara_linear_bias_bf16(
             _ptr(x), x.stride(0), _ptr(w.data), w.n, w.k, _ptr(bias), rows, _LIN_EPI[epilogue],

@@ -234,3 +234,51 @@ def test_rotary_regions_and_their_edges(cuda, B, S, H, Hkv, D, K):
 
     for got, (want, bound) in ((q, turned(wq, H)), (kc[:, pos:pos + S], turned(wk, Hkv)), (vc[:, pos:pos + S], plain(wv, Hkv))):
         assert ((got.double() - want).abs() <= bound + 1e-30).all()
+
+
+@pytest.mark.parametrize("n,k,rows", [(768, 3072, 65), (768, 3072, 129), (768, 3072, 400), (2048, 5632, 33), (2048, 5632, 192), (2048, 5632, 401),
+                                      (2560, 10240, 65), (2560, 10240, 301), (2560, 10240, 1000), (16, 4096, 97), (4096, 4096, 70)])
+def test_products_in_parts_of_the_depth(cuda, n, k, rows):
+    """The residual product with the norm behind it, and the one with a bias and two addends, in parts of the depth against 64 bits: an
+    fp32 sum of k products in any order, rounded where the products over the whole depth are; without room those are taken."""
+    from ohara_amd import ops
+    from ohara_amd._lib import check, lib
+
+    g = torch.Generator(device=cuda).manual_seed(n + k + rows)
+    x, w = (torch.randn(r, k, generator=g, device=cuda).to(torch.bfloat16) for r in (rows, n))
+    res, add2 = (torch.randn(rows, n, generator=g, device=cuda).to(torch.bfloat16) for _ in range(2))
+    bias, norm = (torch.randn(n, generator=g, device=cuda).to(torch.bfloat16) for _ in range(2))
+    y, mass = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    sum_err = mass * k * 2.0 ** -24
+    packed, stream = ops.pack_linear(w), torch.cuda.current_stream().cuda_stream
+
+    def half(v, e):  # a value known to e, rounded to bf16: its error
+        return e + (v.abs() + e) * 2.0 ** -8
+
+    y_err = half(y, sum_err)
+    want, want_err = res.double() + y, half(res.double() + y, y_err)
+    room = lib().ohara_gemm_residual_norm_bytes(rows, n, k)
+    assert room > 0 or n in (2560, 16)
+    for size in {room, 0}:
+        ws = torch.full((size + 64,), 0xFF, dtype=torch.uint8, device=cuda)
+        out, xn = res.clone(), torch.empty_like(res)
+        check(lib().ohara_gemm_residual_norm_bf16(x.data_ptr(), k, packed.data.data_ptr(), n, k, rows, out.data_ptr(), norm.data_ptr(), 1e-5,
+                                                  xn.data_ptr(), ws.data_ptr(), size, stream), "residual_norm")
+        assert ((out.double() - want).abs() <= want_err).all()
+        o = out.double()
+        v = o / (o.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+        assert ((xn.double() - v * norm.double()).abs() <= (v * norm.double()).abs() * 2.0 ** -7 + 1e-6).all()  # rounded twice
+        assert (ws[size:] == 0xFF).all()
+        plain = res.clone()
+        check(lib().ohara_gemm_residual_norm_bf16(x.data_ptr(), k, packed.data.data_ptr(), n, k, rows, plain.data_ptr(), None, 1e-5, None,
+                                                  ws.data_ptr(), size, stream), "residual_norm")
+        assert torch.equal(plain, out)
+    with_bias = y + bias.double()
+    b_err = half(with_bias, sum_err)
+    first, first_err = with_bias + res.double(), half(with_bias + res.double(), b_err)
+    total, total_err = first + add2.double(), half(first + add2.double(), first_err)
+    got = ops.linear_bias(x, packed, bias, "add2", add1=res, add2=add2)
+    assert ((got.double() - total).abs() <= total_err).all()
+    odd = torch.empty(rows, n + 4, dtype=torch.bfloat16, device=cuda)[:, 4:]  # not on 16 bytes: over the whole depth
+    ops.linear_bias(x, packed, bias, "add2", add1=res, add2=add2, out=odd)
+    assert ((odd.double() - total).abs() <= total_err).all()
