@@ -258,15 +258,17 @@ __global__ __launch_bounds__(256) void phi_attn_kernel(PhiAttnArgs a) {
   }
   __syncthreads();
   if (tid < D) {
-    float M = -INFINITY;
+    float M = -INFINITY, gv[16];
+#pragma unroll
+    for (int g = 0; g < 16; ++g) gv[g] = gacc[g][tid];
 #pragma unroll
     for (int g = 0; g < 16; ++g) M = fmaxf(M, gm[g]);
     float num = 0.f, den = 0.f;
 #pragma unroll
-    for (int g = 0; g < 16; ++g) {
-      if (gm[g] == -INFINITY) continue;  // a group that saw no position
-      const float wg = expf(gm[g] - M);
-      num += wg * gacc[g][tid];
+    for (int g = 0; g < 16; ++g) {  // (no branch: every read would be waited for behind it; with the merge's below, whose values are asked for
+                                    // with the maxima: 32 heads of 80 behind 700 13.1 -> 11.2 us)
+      const float wg = gm[g] == -INFINITY ? 0.f : expf(gm[g] - M);  // (a group that saw no position holds zeros)
+      num += wg * gv[g];
       den += wg * gl[g];
     }
     if (a.ns > 1) {
@@ -299,7 +301,13 @@ __global__ __launch_bounds__(256) void phi_attn_kernel(PhiAttnArgs a) {
   __syncthreads();
   if (!is_last) return;
   const float* p = a.ws + ((size_t)row * a.H + h) * a.ns * (D + 2);
-  if (tid < a.ns) {  // ns <= 64: one round of loads for all (max, sum) pairs
+  // ns <= 64: one round of loads for all (max, sum) pairs and the first sixteen chunks' values
+  float av[16];
+  if (tid < D) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) av[i] = __uint_as_float(ld_coh4(p + (size_t)min(i, a.ns - 1) * (D + 2) + tid));
+  }
+  if (tid < a.ns) {
     // qr and gacc are free again: chunk maxima and sums go there
     qr[tid] = __uint_as_float(ld_coh4(p + (size_t)tid * (D + 2) + D));
     gacc[0][tid] = __uint_as_float(ld_coh4(p + (size_t)tid * (D + 2) + D + 1));
@@ -310,16 +318,23 @@ __global__ __launch_bounds__(256) void phi_attn_kernel(PhiAttnArgs a) {
     for (int c = 0; c < a.ns; ++c) M = fmaxf(M, qr[c]);
     float num = 0.f, den = 0.f;
     for (int c0 = 0; c0 < a.ns; c0 += 16) {  // sixteen chunks' values in flight, every load unconditional
-      float av[16];
+      if (c0) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) av[i] = __uint_as_float(ld_coh4(p + (size_t)min(c0 + i, a.ns - 1) * (D + 2) + tid));
-      __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < 16; ++i) av[i] = __uint_as_float(ld_coh4(p + (size_t)min(c0 + i, a.ns - 1) * (D + 2) + tid));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float mc[16], lc[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        if (c0 + i >= a.ns || qr[c0 + i] == -INFINITY) continue;
-        const float wg = expf(qr[c0 + i] - M);
-        num += wg * av[i];
-        den += wg * gacc[0][c0 + i];
+        mc[i] = qr[min(c0 + i, a.ns - 1)];
+        lc[i] = gacc[0][min(c0 + i, a.ns - 1)];
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const bool in = c0 + i < a.ns && mc[i] != -INFINITY;
+        const float wg = expf(mc[i] - M);
+        num += in ? wg * av[i] : 0.f;
+        den += in ? wg * lc[i] : 0.f;
       }
     }
     a.out[(size_t)row * hd + (size_t)h * D + tid] = f2bf(num / den);
