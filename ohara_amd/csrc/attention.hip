@@ -64,55 +64,76 @@ __device__ __forceinline__ void stf_coh(float* p, float v) { st_coh4(p, __float_
 // accumulator columns are then summed in chunk order with the loads of up to 32 chunks issued together.
 // Needs G * n_split <= OHARA_MERGE_CAP.
 #define OHARA_MERGE_CAP 2048
-template <int MAXD>
-__device__ void merge_partials(const AttnArgs& a, int b /* query row */, int kvh, int G, int ns) {
-  __shared__ float s_w[OHARA_MERGE_CAP];   // max, then weight, of (head, chunk)
-  __shared__ float s_ls[OHARA_MERGE_CAP];  // sum of (head, chunk)
-  __shared__ float s_tot[64];              // per head: normaliser
-  const int D = a.D;
+struct MergeRoom {
+  float w[OHARA_MERGE_CAP];   // max, then weight, of (head, chunk)
+  float ls[OHARA_MERGE_CAP];  // sum of (head, chunk)
+  float tot[64];              // per head: normaliser
+};
+// A thread's first column is asked for with the statistics, N chunks of it and of every other in one round (the next N behind it),
+// every load and LDS read unconditional: behind a test each was waited for by itself.  Chunks past the last read the last one again and
+// are not added; N is near their number, for they come from memory all the same.  (0.6 us
+// of a launch's 12.8 for 16 sequences of 4 x 4 heads of 128 behind 700, int8; 12 sequences of 6 heads behind 800, a step 1.9 % less.)
+template <int D, int N>
+__device__ __forceinline__ void merge_columns(const AttnArgs& a, int b, int kvh, int G, int ns, int dim, MergeRoom& r) {
+  const int width = D ? D : dim;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  float av[N];
+  auto load = [&](int idx, int s0) {
+    const int hh = idx / width, d = idx - hh * width;
+    const float* pa = a.part_acc + ((size_t)(b * a.H + kvh * G) * a.nsplit + (size_t)hh * ns) * width + d;
+#pragma unroll
+    for (int i = 0; i < N; ++i) av[i] = ldf_coh(pa + (size_t)min(s0 + i, ns - 1) * width);
+  };
+  if (tid < G * width) load(tid, 0);
   const float* ml0 = a.part_ml + ((size_t)(b * a.H + kvh * G) * a.nsplit) * 2;  // heads of a group are adjacent
   for (int i = tid; i < G * ns; i += blockDim.x) {
     const uint2 v = ld_coh8(ml0 + 2 * (size_t)i);
-    s_w[i] = __uint_as_float(v.x);
-    s_ls[i] = __uint_as_float(v.y);
+    r.w[i] = __uint_as_float(v.x);
+    r.ls[i] = __uint_as_float(v.y);
   }
   __syncthreads();
   for (int hh = wave; hh < G; hh += 4) {
     float M = -INFINITY;
-    for (int s0 = lane; s0 < ns; s0 += 64) M = fmaxf(M, s_w[hh * ns + s0]);
+    for (int s0 = lane; s0 < ns; s0 += 64) M = fmaxf(M, r.w[hh * ns + s0]);
     M = wave_max(M);
     float L = 0.f;
     for (int s0 = lane; s0 < ns; s0 += 64) {
-      const float ms = s_w[hh * ns + s0];
+      const float ms = r.w[hh * ns + s0];
       const float w = (ms == -INFINITY) ? 0.f : pow2_neg_int(ms - M);  // maxima are integers (log2 units): exact
-      s_w[hh * ns + s0] = w;
-      L += s_ls[hh * ns + s0] * w;
+      r.w[hh * ns + s0] = w;
+      L += r.ls[hh * ns + s0] * w;
     }
     L = wave_sum(L);
-    if (lane == 0) s_tot[hh] = L;
+    if (lane == 0) r.tot[hh] = L;
   }
   __syncthreads();
-  for (int idx = tid; idx < G * D; idx += blockDim.x) {
-    const int hh = idx / D, d = idx - hh * D;
-    const int h = kvh * G + hh;
-    const float* pa = a.part_acc + ((size_t)(b * a.H + kvh * G) * a.nsplit + (size_t)hh * ns) * D + d;
-    const float* w = s_w + hh * ns;
+  for (int idx = tid; idx < G * width; idx += blockDim.x) {
+    const int hh = idx / width;
+    const float* w = r.w + hh * ns;
     float o = 0.f;
-    // Up to 32 chunks' values are in flight at once, every load unconditional (chunks past the last
-    // read the last one again and are not added): with eight at a time behind a test each, 32 chunks
-    // were four dependent round trips and more than half of a batch-1 launch.
-    for (int s0 = 0; s0 < ns; s0 += 32) {
-      float av[32];
+    for (int s0 = 0; s0 < ns; s0 += N) {
+      if (s0 || idx != tid) {
+        load(idx, s0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float wv[N];
 #pragma unroll
-      for (int i = 0; i < 32; ++i) av[i] = ldf_coh(pa + (size_t)min(s0 + i, ns - 1) * D);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int i = 0; i < N; ++i) wv[i] = w[min(s0 + i, ns - 1)];
 #pragma unroll
-      for (int i = 0; i < 32; ++i)
-        if (s0 + i < ns) o += av[i] * w[s0 + i];
+      for (int i = 0; i < N; ++i) {
+        const float more = __builtin_fmaf(av[i], wv[i], o);
+        o = s0 + i < ns ? more : o;
+      }
     }
-    a.out[(size_t)b * a.H * D + h * D + d] = f2bf(o * (1.0f / s_tot[hh]));
+    a.out[(size_t)b * a.H * width + (size_t)kvh * G * width + idx] = f2bf(o * (1.0f / r.tot[hh]));
   }
+}
+template <int D>  // 0: a.D
+__device__ void merge_partials(const AttnArgs& a, int b /* query row */, int kvh, int G, int ns) {
+  __shared__ MergeRoom room;
+  if (ns <= 4) merge_columns<D, 4>(a, b, kvh, G, ns, a.D, room);
+  else if (ns <= 16) merge_columns<D, 16>(a, b, kvh, G, ns, a.D, room);
+  else merge_columns<D, 32>(a, b, kvh, G, ns, a.D, room);
 }
 
 // Into how many of the caller's n_split chunks a context of L positions is cut, from what is known only here (L may live on the
@@ -999,7 +1020,7 @@ __global__ __launch_bounds__(256) void attn_decode_generic(AttnArgs a) {
     }
   }
   if (a.nsplit == 1) return;
-  if (last_chunk_done(a.counters + b * a.Hkv + kvh, a.nsplit)) merge_partials<256>(a, b, kvh, G, a.nsplit);
+  if (last_chunk_done(a.counters + b * a.Hkv + kvh, a.nsplit)) merge_partials<0>(a, b, kvh, G, a.nsplit);
 }
 
 template <int D, bool I8>
