@@ -157,8 +157,8 @@ class _Buffers:
         self.attn = torch.empty(rows, hd, dtype=BF16, device=dev)
         self.act = torch.empty(rows, model.act_width, dtype=BF16, device=dev)
         self.xn = torch.empty(rows, c.hidden_size, dtype=BF16, device=dev) if rows > ops.norm_rows(c.hidden_size) else None
-        self.attn_ws = ops.attn_workspace(batch, c.num_attention_heads, model.kv_heads, model.head_dim, n_split, dev,
-                                          4 * batch * model.kv_heads if rows > batch else None)
+        # (several tokens a sequence: room, whose counters no kernel reads)
+        self.attn_ws = ops.attn_workspace(batch, c.num_attention_heads, model.kv_heads, model.head_dim, n_split, dev, rows <= batch)
         self.step_state = torch.zeros(4, dtype=torch.int32, device=dev)
         self.logits = None
         self.history = None
@@ -305,15 +305,15 @@ class Llama:
         want = max(1, 1024 // max(1, batch * self.kv_heads))
         return max(1, min(want, self.config.max_sequence_length // 128, 64))
 
-    def _get_buffers(self, batch: int, rows: int) -> _Buffers:
-        key = (batch, rows)
+    def _get_buffers(self, batch: int, rows: int, side_by_side: bool = False) -> _Buffers:
+        key = (batch, rows, side_by_side)
         buf = self._buffers.get(key)
         if buf is None:
             # keep at most one prefill-sized set alive
             for k in [k for k in self._buffers if k[1] > k[0] and k != key]:
                 del self._buffers[k]
             n_split, c = self.default_n_split(batch), self.config
-            if rows > batch:  # several tokens a sequence: the workspace holds their partial results
+            if rows > batch and not side_by_side:  # several tokens a sequence: the workspace holds their partial results
                 h, dh, S = c.num_attention_heads, self.head_dim, rows // batch
                 room = ops.lib().ohara_attn_prefill_ws_bytes(batch, S, h, self.kv_heads, dh, max(0, c.max_sequence_length - S))
                 if rows > ops.norm_rows(c.hidden_size):
@@ -465,7 +465,7 @@ class Llama:
         """``prompts`` without its checks; an id outside the vocabulary counts as 0, as in every call whose ids are on the device."""
         lens = [len(p) for p in prompts]
         n, rows = len(prompts), sum(lens)
-        buf = self._get_buffers(n, rows)
+        buf = self._get_buffers(n, rows, True)  # (that chain needs no room for partial results)
         length, slot = torch.tensor(lens, dtype=torch.int32), torch.tensor(slots, dtype=torch.int32)
         first = length.cumsum(0, dtype=torch.int32) - length
         at = torch.arange(rows, dtype=torch.int32) - first.repeat_interleave(length)

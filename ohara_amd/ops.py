@@ -207,14 +207,11 @@ def qkv_rope(x, wqkv: PackedLinear, norm_w, eps, h, h_kv, dh, cos, sin, pos, t_m
     return q, k, v
 
 
-def attn_workspace(batch, h, h_kv, dh, n_split, device, zeros=None) -> torch.Tensor:
-    """``zeros``: how many bytes at the start are cleared (the counters; all of it by default)."""
+def attn_workspace(batch, h, h_kv, dh, n_split, device, zeros: bool = True) -> torch.Tensor:
     n = lib().ohara_attn_workspace_bytes(batch, h, h_kv, dh, n_split)
     if n < 0:
         raise ValueError("bad attention workspace shape")
-    ws = torch.empty(n, dtype=torch.uint8, device=device)
-    ws[:zeros].zero_()
-    return ws
+    return (torch.zeros if zeros else torch.empty)(n, dtype=torch.uint8, device=device)
 
 
 def attn_cached(q, kcache, vcache, h, h_kv, dh, pos, n_split, workspace, out=None, pos_dev=None, seq_len=1,
