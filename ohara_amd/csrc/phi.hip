@@ -267,9 +267,10 @@ __global__ __launch_bounds__(256) void phi_attn_kernel(PhiAttnArgs a) {
 #pragma unroll
     for (int g = 0; g < 16; ++g) {  // (no branch: every read would be waited for behind it; with the merge's below, whose values are asked for
                                     // with the maxima: 32 heads of 80 behind 700 13.1 -> 11.2 us)
-      const float wg = gm[g] == -INFINITY ? 0.f : expf(gm[g] - M);  // (a group that saw no position holds zeros)
-      num += wg * gv[g];
-      den += wg * gl[g];
+      const bool in = gm[g] != -INFINITY;  // (not a group that saw no position, nor one whose scores are all -inf, which holds NaN)
+      const float wg = expf(gm[g] - M);
+      num += in ? wg * gv[g] : 0.f;
+      den += in ? wg * gl[g] : 0.f;
     }
     if (a.ns > 1) {
       // write-through stores: the workgroup that merges may sit on another XCD

@@ -114,6 +114,27 @@ def test_kv_append_and_attention_against_the_oracle(cuda):
                 _ulp_close(got3.view(B, S, H, D), want, ulps=0.6, floor=2.0 ** -6)
 
 
+@pytest.mark.parametrize("L0", [5, 15])
+def test_a_position_that_scores_minus_infinity_has_no_weight(cuda, L0):
+    """Up to sixteen positions are one to a lane group: the group of such a position is left out, whatever its sums are."""
+    from ohara_amd import ops
+    from ohara_amd.phi import rope_cos_sin
+
+    H, D, rot = 2, 80, 32
+    g = torch.Generator().manual_seed(L0)
+    q, k, v = (torch.randn(1, n, H, D, generator=g).to(BF) for n in (1, L0 + 1, L0 + 1))
+    q[..., D - 1] = 1.0  # (the last feature is not rotated)
+    k[:, 3, :, D - 1] = float("-inf")
+    cos, sin = rope_cos_sin(32, rot)
+    want = P.attention(q, k, v, L0, rot, torch.float32)
+    assert want.isfinite().all()
+    for ns in (1, 2):
+        ws = ops.phi_attn_workspace(1, H, D, ns, cuda) if ns > 1 else None
+        got = ops.phi_attn(q.view(1, H * D).to(cuda), k.to(cuda), v.to(cuda), cos.to(cuda), sin.to(cuda), rot, 1, 1, H, D, L0, n_split=ns,
+                           workspace=ws)
+        _ulp_close(got.view(1, 1, H, D), want, ulps=0.6, floor=2.0 ** -6)
+
+
 def _pair(cuda, dtype=BF, seed=5, **kw):
     from ohara_amd.phi import Phi, PhiConfig
 
