@@ -538,7 +538,7 @@ __global__ __launch_bounds__(D * 4) void attn_chunks_merge_kernel(ChunkArgs c) {
       const float w = mx[i] == -INFINITY ? 0.f : pow2_neg_int(mx[i] - mn);
       l += ls[i] * w;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sum[e] += pv[i][e] * w;
+      for (int e = 0; e < 4; ++e) sum[e] = i0 + i < c.cut.chunks ? __builtin_fmaf(pv[i][e], w, sum[e]) : sum[e];  // (an infinity: not twice)
     }
     M = mn;
   }

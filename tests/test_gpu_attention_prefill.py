@@ -141,3 +141,21 @@ def test_a_few_tokens_a_sequence(cuda, B, S, H, Hkv, pos, wins, D):
     v[:, pos + S:] = float("nan")
     assert ((ops.attn_prefill(rows, k, v, H, Hkv, D, pos, S).view(B, S, H, D).double() - want).abs() <= bound).all()
     assert ((ops.attn_auto(rows, k, v, H, Hkv, D, pos, 1, None, S).view(B, S, H, D).double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S,pos", [(16, 700), (40, 2500)])  # four chunks, and more than one round of eight
+def test_an_infinite_value_in_the_last_chunk_stays_infinite(cuda, S, pos, D):
+    """The merge reads the last chunk again where its round of eight has no more: those sums are not added, not even times zero."""
+    from ohara_amd import ops
+    from ohara_amd._lib import lib
+
+    H = 6
+    assert lib().ohara_attn_prefill_ws_bytes(1, S, H, H, D, pos) > 0
+    g = torch.Generator(device=cuda).manual_seed(S + D)
+    q, k, v = (torch.randn(1, n, H, D, generator=g, device=cuda).to(BF) for n in (S, pos + S, pos + S))
+    want, bound = _reference(q, k, v, pos)
+    v[:, pos - 1, :, 0] = float("inf")
+    got = ops.attn_prefill(q.view(S, H * D), k, v, H, H, D, pos, S).view(1, S, H, D)
+    assert (got[..., 0] == float("inf")).all()
+    assert ((got.double() - want).abs() <= bound)[..., 1:].all()
