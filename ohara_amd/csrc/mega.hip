@@ -28,23 +28,23 @@ MegaPlan mega_plan(const OharaModel* m, int batch, int n_workgroups) {
   // one attention item per workgroup where the batch allows it
   int ns = n_workgroups / (batch * m->n_kv_heads);
   ns = ns < 1 ? 1 : (ns > OHARA_MEGA_NS ? OHARA_MEGA_NS : ns);
-  // A power of two unless the exact count keeps at least half as many workgroups again busy and its
-  // merge stays narrow (the merge reads the next power of two of chunk slots): 7 chunks of 36 pairs
-  // instead of 4 took batch 6 from 0.397 to 0.379 ms per step, 5 instead of 4 at batch 8 lost what the
-  // attention phase gained to the wider merge.
-  int p2 = ns;
-  while (p2 & (p2 - 1)) p2 &= p2 - 1;
-  if (!(2 * ns >= 3 * p2 && attn_merge_width(ns) <= 8)) ns = p2;
-  const size_t mrg = (size_t)2 * ((batch * m->n_heads * attn_merge_width(ns) + 1) & ~1) * sizeof(float);
   // The polled builds (batch 1; up to eight sequences) park the down projection's tiles in LDS (4 waves x
   // OHARA_LDS_PF KB) and want gate/up, the output projection and the down projection on workgroups of their own.
   const int n_dn = (m->d_model + 15) / 16, n_gu = (2 * ((m->d_ff + 7) / 8 * 8) / 16 + 1) / 2;
   const size_t rest = 4096 + (size_t)(8 + 4 * D) * G * sizeof(float) + (size_t)m->n_layers * 72;
-  const size_t smem0 = xs_bytes + rest + mrg;
   const size_t merge_bytes = (merge_head_lds(D) + 255) & ~(size_t)255, smem1 = (xs_bytes > merge_bytes ? xs_bytes : merge_bytes) + rest;
   const size_t smem_polled = smem1 + 256 + (size_t)4 * OHARA_LDS_PF * 1024;
   const bool roles = n_gu + n_dn <= n_workgroups && 2 * n_dn <= n_workgroups;
   const int mode = !roles ? 0 : (batch == 1 ? 1 : (batch <= 8 && smem_polled <= 160 * 1024 ? 2 : 0));
+  // The polled builds take as many chunks as there are workgroups: one workgroup merges a head, whatever their number.  us a step of 6 heads
+  // of 128, powers of two (8, 8, 4) / as many (14, 10, 5): 3 sequences behind 200 202.5 / 202.7, 1000 228 / 216, 3000 290 / 256; 4 behind 700
+  // 221 / 219, 3000 296 / 280; 8 behind 100 258 / 258, 700 292 / 287, 3000 442 / 412; int8 caches, 3 behind 700 251 / 240, 8 348 / 342.
+  // With grid barriers, where every merge reads the next power of two of chunk slots, a power of two unless the exact count keeps at least
+  // half as many workgroups again busy and its merge stays narrow.
+  int p2 = ns;
+  while (p2 & (p2 - 1)) p2 &= p2 - 1;
+  if (!mode && !(2 * ns >= 3 * p2 && attn_merge_width(ns) <= 8)) ns = p2;
+  const size_t smem0 = xs_bytes + rest + (size_t)2 * ((batch * m->n_heads * attn_merge_width(ns) + 1) & ~1) * sizeof(float);
   // A single sequence leaves LDS free: the workgroups that park their waves' second vocabulary strip add half of the
   // third (12 more tiles per wave) where that fits.
   const size_t smem_more = smem1 + 256 + (size_t)4 * (OHARA_LDS_PF + 12) * 1024;

@@ -339,6 +339,31 @@ def test_d12_persistent_kernel_batch8_prompt1024(cuda, batch):
         sess.check_error()
 
 
+@pytest.mark.parametrize("batch,P", [(3, 9), (3, 230), (4, 70), (5, 200), (8, 33)])  # 14, 14, 10, 8 and 5 chunks of six heads' contexts
+def test_persistent_kernel_with_as_many_chunks_as_fit(cuda, batch, P):
+    """Counts of chunks that are no powers of two, and chunks without a position: teacher-forced logits against the oracle."""
+    from ohara_amd.llama import Llama
+
+    rcfg, cfg = _cfg_pair(vocab_size=512, hidden_size=768, intermediate_size=512, num_attention_heads=6,
+                          num_key_value_heads=0, num_hidden_layers=2, max_sequence_length=256, dropout=0.0)
+    w = R.init_weights(rcfg, seed=batch, dtype=BF)
+    ref, model = R.RefLlama(rcfg, w), Llama(cfg, w, device=cuda)
+    steps = 4
+    prompt = torch.randint(0, 512, (batch, P), generator=torch.Generator().manual_seed(P))
+    rc = ref.build_kv_cache(batch)
+    want, fed = [ref(prompt, rc, 0)[:, -1]], []
+    for s in range(steps):
+        fed.append(want[-1].float().argmax(-1))
+        want.append(ref(fed[-1].view(batch, 1), rc, P + s)[:, -1])
+    sess = model.session(batch, steps + 1, persistent=True)
+    sess.prefill(prompt.to(cuda))
+    for s in range(steps):
+        sess.feed(fed[s])
+        sess.step()
+        _assert_logits_close(sess.logits, want[s + 1], 2e-2, 2e-3)  # (as for the twelve layers of this width)
+    sess.check_error()
+
+
 @pytest.mark.parametrize("persistent", [True, False])
 def test_sampled_decode_session(cuda, persistent):
     """Temperature 0.8 / top-k 50 / top-p 0.9 decode driven by a pre-drawn uniform tensor, with no
