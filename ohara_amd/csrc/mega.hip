@@ -21,6 +21,7 @@ struct MegaPlan {
 };
 
 MegaPlan mega_plan(const OharaModel* m, int batch, int n_workgroups) {
+  if (m->n_kv_heads < 1) return MegaPlan{1, 0, 0, OHARA_LDS_PF};  // (the sizes of a workspace are asked for ahead of any check; no launch)
   const int D = m->head_dim, G = m->n_heads / m->n_kv_heads;
   const int kmax = m->d_model > m->d_ff ? m->d_model : m->d_ff;
   const int kmax2 = kmax > m->n_heads * D ? kmax : m->n_heads * D;
@@ -138,6 +139,7 @@ int ohara_llama_decode_persistent(const OharaModel* m, const OharaDecodeState* s
   if (s->batch < 1 || s->batch > 16) return OHARA_ESIZE;
   if (n_workgroups < 1 || n_workgroups > 1024) return OHARA_EINVAL;
   if (s->n_split != OHARA_MEGA_NS) return OHARA_EINVAL;
+  if (m->n_kv_heads < 1) return OHARA_EINVAL;
   const int D = m->head_dim, G = m->n_heads / m->n_kv_heads;
   if (!(D == 128 || D == 64) || !(G == 1 || G == 2 || G == 4) || m->n_heads % m->n_kv_heads) return OHARA_ESIZE;
   if ((m->d_model & 7) || (m->d_ff & 7) || m->d_model > 1024) return OHARA_ESIZE;

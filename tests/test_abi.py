@@ -74,3 +74,33 @@ def test_argument_checks_need_no_gpu():
     # packed row 0..3 of strip 0: gate 0, gate 1, up 0, up 1 (up rows follow the 12 gate rows)
     assert list(buf[:4]) == [0, 1, 12, 13]
     assert list(buf[16:20]) == [8, 9, 20, 21] and buf[28] == -1
+
+
+def test_sizes_of_a_model_without_key_heads():
+    """The persistent step's size and offset entries answer for any numbers (a division by zero would end the process), and the step
+    itself refuses a model without key heads ahead of its division by them."""
+    import subprocess
+    import sys
+
+    code = """
+import ctypes as C
+from ohara_amd import _lib
+lib = _lib.lib()
+for kv in (0, -1):
+    m = _lib.OharaModel(2, 256, 4, kv, 64, 128, 100, 32)
+    for batch in (1, 3, 9):
+        sizes = [f(C.byref(m), batch, 16, 64) for f in (lib.ohara_persistent_barrier_offset, lib.ohara_persistent_error_offset,
+                                                       lib.ohara_persistent_profile_offset, lib.ohara_persistent_workspace_bytes)]
+        assert 0 < min(sizes) and max(sizes) == sizes[-1], sizes
+        assert lib.ohara_persistent_polled(C.byref(m), batch, 64) == -1
+    layers = (_lib.OharaLayer * 2)()
+    m.layers = layers
+    ptrs = (C.c_void_p * 2)()
+    s = _lib.OharaDecodeState()
+    s.batch, s.n_split, s.step_state = 1, 16, 1
+    s.kcache = s.vcache = C.cast(ptrs, type(s.kcache))
+    assert lib.ohara_llama_decode_persistent(C.byref(m), C.byref(s), 1, 64, 0, 0, 0, 0) == -1
+print("ok")
+"""
+    run = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0 and run.stdout.strip() == "ok", (run.returncode, run.stderr[-2000:])
