@@ -235,7 +235,10 @@ class MoeLlama:
                 sh = moe.shared
                 held += [sh and sh[0].data, sh and sh[1].data, moe.router.data, moe.router_bias, moe.wp_gu, moe.wp_dn, moe._counter]
         at = [0 if t is None else t.data_ptr() for t in held]
-        at += [(m.k, m.biased, m.gate_fn, m.normalize) for m in (L.get("moe") for L in self.layers) if m is not None]
+        for L in self.layers:  # (and whatever else the table holds: other widths may come to lie at the same addresses)
+            m = L.get("moe")
+            at.append(L["wgu"].n if m is None else (m.E, m.hidden, m.k, m.biased, m.gate_fn, m.normalize, m.wp_gu.stride(0), m.wp_dn.stride(0),
+                                                    m.shared and m.shared[0].n))
         table, table_of = self._table
         if at != table_of:
             table = (OharaMoeLayer * len(self.layers))()

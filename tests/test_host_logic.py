@@ -366,3 +366,37 @@ def test_phi_checkpoint_name_mapping_and_local_shards(tmp_path):
         load_huggingface_state_dict(str(empty), 2)
     with pytest.raises(KeyError, match="missing expected tensors"):
         load_huggingface_state_dict(str(tmp_path), 3)
+
+
+def test_expert_layer_table_follows_widths_as_well_as_addresses():
+    """Weights that are replaced by others of other widths may lie where the old ones lay: the C chain's table is laid out anew."""
+    from types import SimpleNamespace
+
+    from ohara_amd.moe import MoeLlama
+
+    room = torch.zeros(4096, dtype=torch.bfloat16)
+    packed = lambda n: SimpleNamespace(data=room, n=n)  # noqa: E731
+    moe = SimpleNamespace(shared=(packed(32), packed(64)), router=packed(8), router_bias=room, _counter=room, E=8, hidden=16, k=2, biased=True,
+                          gate_fn="softmax", normalize=True, wp_gu=room[:1024].view(8, 128), wp_dn=room[:512].view(8, 64))
+    model = MoeLlama.__new__(MoeLlama)
+    dense = dict(wqkv=packed(192), wo=packed(64), norm1=room, norm2=room, wgu=packed(48), wdown=packed(64))
+    model.layers = [dense, dict(wqkv=packed(192), wo=packed(64), norm1=room, norm2=room, moe=moe)]
+    model._table = None, None
+
+    def held():
+        a, b = model._layer_table()
+        return a.ff, b.ff, b.n_experts, b.hidden, b.gu_stride, b.down_stride, a.wgu, b.experts_gu
+
+    first = held()
+    assert first == (48, 32, 8, 16, 256, 128, room.data_ptr(), room.data_ptr()) and held() == first
+    table = model._layer_table()
+    assert model._layer_table() is table
+    dense["wgu"] = packed(24)
+    moe.shared = (packed(40), packed(64))
+    moe.E, moe.hidden, moe.wp_gu, moe.wp_dn = 4, 40, room[:2048].view(4, 512), room[:1024].view(4, 256)
+    assert held() == (24, 40, 4, 40, 1024, 512, room.data_ptr(), room.data_ptr())
+    for change in (dict(E=3), dict(hidden=24), dict(wp_gu=room[:2052].view(4, 513)), dict(wp_dn=room[:1028].view(4, 257)), dict(shared=None)):
+        before = model._layer_table()
+        for name, value in change.items():
+            setattr(moe, name, value)
+        assert model._layer_table() is not before
