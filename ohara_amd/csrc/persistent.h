@@ -756,9 +756,9 @@ __device__ __forceinline__ void merge_head(const char* part, int ns, float* sm, 
   const float M = lane_xor_max<1>(lane_xor_max<2>(lane_xor_max<4>(lane_xor_max<8>(ms))));
   const float w = (ms == -INFINITY) ? 0.f : pow2_neg_int(ms - M);
   const float Ls = lane_xor_sum<1>(lane_xor_sum<2>(lane_xor_sum<4>(lane_xor_sum<8>(ls * w))));
+  static_assert(R * RG == OHARA_MEGA_NS, "");
 #pragma unroll
-  for (int i = 0; i < R; ++i)
-    if (r + i * RG < ns) sts16(sm + (r + i * RG) * D + c * 4, v[i]);
+  for (int i = 0; i < R; ++i) sts16(sm + (r + i * RG) * D + c * 4, r + i * RG < ns ? v[i] : make_uint4(0, 0, 0, 0));
   if (tid < 16) sw[tid] = w;
   if (tid == 0) sw[16] = Ls;
   __syncthreads();
@@ -768,7 +768,8 @@ __device__ __forceinline__ void merge_head(const char* part, int ns, float* sm, 
 #pragma unroll
     for (int s = 0; s < OHARA_MEGA_NS; ++s) {
       ws[s] = sw[s];
-      av[s] = *reinterpret_cast<const f32x2_t*>(sm + min(s, ns - 1) * D + 2 * tid);  // (past the last chunk: again, of weight zero)
+      av[s] = *reinterpret_cast<const f32x2_t*>(sm + s * D + 2 * tid);  // (past the last chunk zeros: of that one's sums an infinity, times
+                                                                        // a weight of zero, would be a NaN)
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

@@ -364,6 +364,44 @@ def test_persistent_kernel_with_as_many_chunks_as_fit(cuda, batch, P):
     sess.check_error()
 
 
+@pytest.mark.parametrize("H,D,batch", [(6, 128, 3), (6, 128, 5), (12, 64, 4), (2, 64, 1), (6, 128, 8)])  # 14, 8, 5, 16 and 5 chunks
+def test_persistent_merge_of_an_infinite_value(cuda, H, D, batch):
+    """An infinite value in a context's last chunk leaves its column of the head's merged row infinite and touches nothing else: the merge
+    runs over sixteen slots, and those past the last chunk hold no sums of it."""
+    import ctypes as C
+
+    from ohara_amd._lib import lib
+    from ohara_amd.llama import Llama
+
+    layers, P, F = 2, 200, 512
+    rcfg, cfg = _cfg_pair(vocab_size=512, hidden_size=H * D, intermediate_size=F, num_attention_heads=H, num_key_value_heads=0,
+                          num_hidden_layers=layers, max_sequence_length=256, dropout=0.0)
+    model = Llama(cfg, R.init_weights(rcfg, seed=batch, dtype=BF), device=cuda)
+    prompt = torch.randint(0, 512, (batch, P), generator=torch.Generator().manual_seed(1)).to(cuda)
+    al = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    x, q, kv, a = al(2 * H * D), al(2 * H * D), al(4 * H * D), al(2 * F)  # a sequence's rows in the mailboxes
+    merged = batch * (2 * x + q + kv + a)                                  # ... of a layer, and the merged rows behind them
+    block = merged + batch * q + al(batch * H * 16 * (D + 32) * 4)
+
+    def rows(infinite):
+        sess = model.session(batch, 4, persistent=True)
+        sess.prefill(prompt)
+        if infinite:
+            sess.cache[0].value[batch - 1, P - 1, 1, 5] = float("inf")
+        sess.step()
+        torch.cuda.synchronize()
+        sess.check_error()
+        size = lib().ohara_persistent_workspace_bytes(C.byref(model._c_model), batch, 16, sess._nwg)
+        at = size - block * layers + merged  # the first step's set of mailboxes is the second one; layer 0
+        return sess._pws[at:at + batch * q].view(batch, q)[:, :2 * H * D].contiguous().view(BF)
+
+    clean, got = rows(False), rows(True)
+    assert clean.isfinite().all() and clean.float().abs().max() > 0
+    assert got[batch - 1, D + 5] == float("inf")
+    got[batch - 1, D + 5] = clean[batch - 1, D + 5]
+    assert torch.equal(got, clean)
+
+
 @pytest.mark.parametrize("persistent", [True, False])
 def test_sampled_decode_session(cuda, persistent):
     """Temperature 0.8 / top-k 50 / top-p 0.9 decode driven by a pre-drawn uniform tensor, with no
