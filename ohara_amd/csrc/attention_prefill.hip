@@ -224,10 +224,79 @@ __device__ __forceinline__ void store_rows(const f32x4 (&o)[N], float l, const P
     *reinterpret_cast<uint2*>(dst + db * 16) = make_uint2(pack_bf(o[db][0] * inv, o[db][1] * inv), pack_bf(o[db][2] * inv, o[db][3] * inv));
 }
 
+// Two to fifteen tokens a call (FEW).  A masked position weighs zero in a tile, and zero times an infinity is a NaN, for queries that do not
+// see it: calls of more tokens live with that (so does softmax(...) @ v); these went through kernels that walk each token's own positions
+// and still give such kernels' results.  So a query whose sums are not finite walks its positions once more, by itself: the weights are
+// the same bits times a power of two (common.h: softmax bookkeeping).  That costs nothing where sums are finite; taking the masked values out of
+// the products, where a product with zeros says that it is needed, cost every call 0.3 to 0.6 us, or a tenth (8 x 15 behind 3000).
+__device__ __forceinline__ unsigned int not_finite(float sum) {  // of a lane's sums; bit m: query m of the wave
+  const unsigned long long l = __ballot(!(fabsf(sum) < INFINITY));
+  const unsigned int f = (unsigned int)l | (unsigned int)(l >> 32);
+  return (f | f >> 16) & 0xffffu;
+}
+// The queries q0 + m with a bit in `which` -> columns c0 .. c0 + cols - 1 of their rows.
+template <int D>
+__device__ __forceinline__ void walk_rows(const PrefillArgs& a, const Sequence& sq, int h, int q0, unsigned int which, int c0, int cols, int lane) {
+  constexpr int N = D / 64, AT = 8;  // columns of a lane, positions at a time
+  const size_t row = (size_t)a.Hkv * D, at0 = (size_t)sq.cache * a.Tmax * row + (size_t)(h / (a.H / a.Hkv)) * D + lane;
+#pragma unroll 1
+  for (int m = 0; m < 16 && q0 + m < sq.S; ++m) {
+    if (!(which >> m & 1)) continue;
+    const size_t mine = (sq.row0 + q0 + m) * a.H * D + (size_t)h * D + lane;
+    const int last = a.pos + q0 + m;
+    float x[N], o[N], top = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      x[i] = bf2f(a.q[mine + 64 * i]);
+      o[i] = 0.f;
+    }
+#pragma unroll 1
+    for (int p0 = 0; p0 <= last; p0 += AT) {
+      bf16_t k[AT][N], v[AT][N];
+#pragma unroll
+      for (int j = 0; j < AT; ++j)
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const size_t at = at0 + (size_t)min(p0 + j, last) * row + 64 * i;
+          k[j][i] = a.k[at];
+          v[j][i] = a.v[at];
+        }
+#pragma unroll
+      for (int j = 0; j < AT; ++j) {
+        if (p0 + j > last) break;
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < N; ++i) s = __builtin_fmaf(x[i], bf2f(k[j][i]), s);
+        s = wave_sum(s) * a.scale_log2e;
+        const float higher = fmaxf(top, ceilf(s)), back = pow2_neg_int(top - higher);
+        top = higher;
+        const float w = __builtin_amdgcn_exp2f(s - (top == -INFINITY ? 0.f : top));
+        l = l * back + w;
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = o[i] * back + rbf(w) * bf2f(v[j][i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (lane + 64 * i >= c0 && lane + 64 * i < c0 + cols) a.out[mine + 64 * i] = f2bf(o[i] * (1.0f / l));
+  }
+}
+// ... and the rest as they are.
+template <int D, int N>
+__device__ __forceinline__ void store_few(const f32x4 (&o)[N], float l, const PrefillArgs& a, const Sequence& sq, int h, int q0, int lane, int d0) {
+  float sum = 0.f;
+#pragma unroll
+  for (int db = 0; db < N; ++db) sum += (o[db][0] + o[db][1]) + (o[db][2] + o[db][3]);
+  const unsigned int odd = not_finite(sum);
+  store_rows<D>(o, l, a, sq, h, odd >> (lane & 15) & 1 ? sq.S : q0 + (lane & 15), lane >> 4, d0);
+  if (odd) walk_rows<D>(a, sq, h, q0, odd, 16 * d0, 16 * N, lane);
+}
+
 // Four waves of 16 QW queries, one tile ahead.
-template <int D, int QW, bool ALIGNED>
+template <int D, int QW, bool ALIGNED, bool FEW>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
   constexpr int NW = 4, QB = 16 * QW * NW;
+  static_assert(!FEW || QW == 1, "sixteen queries a wave");
   constexpr int NK = D / 32;             // k-steps of the score product
   constexpr int ND = D / 16;             // 16-column blocks of the output
   typedef KvTile<D> Tl;
@@ -311,6 +380,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
     }
     cur = next;
   }
+  if constexpr (FEW) return store_few<D>(o[0], l_run[0], a, sq, h, wq0, lane, 0);
 #pragma unroll
   for (int qb = 0; qb < QW; ++qb) store_rows<D>(o[qb], l_run[qb], a, sq, h, wq0 + qb * 16 + m, g, 0);
 }
@@ -318,7 +388,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
 // TEAMS teams of four waves, 16 queries each.  Wave w scores positions 16 w .. + 15 of every tile and owns a quarter of the output
 // columns; the scores go through LDS, and every wave of the team does the softmax of the whole tile.  In the round that works
 // off tile t the scores of t + 1 are made: one barrier a tile.
-template <int D, int TEAMS, int NST, bool ALIGNED>
+template <int D, int TEAMS, int NST, bool ALIGNED, bool FEW>
 __global__ __launch_bounds__(TEAMS * 256, TEAMS) void attn_team_kernel(PrefillArgs a) {
   constexpr int NW = 4 * TEAMS, QB = 16 * TEAMS;
   constexpr int NK = D / 32, ND = D / 64;  // k-steps of the score product, 16-column blocks of a wave's output
@@ -404,6 +474,7 @@ __global__ __launch_bounds__(TEAMS * 256, TEAMS) void attn_team_kernel(PrefillAr
     put_scores(t + 1, sn);
     cur = next;
   }
+  if constexpr (FEW) return store_few<D>(o, l_run, a, sq, h, wq0, lane, w4 * ND);
   store_rows<D>(o, l_run, a, sq, h, wq0 + m, g, w4 * ND);
 }
 
@@ -506,7 +577,7 @@ __global__ __launch_bounds__(256, 2) void attn_chunk_kernel(ChunkArgs c) {
 }
 
 // The chunks' sums of a task, in their order: a wave takes sixteen columns of its sixteen queries.
-template <int D>
+template <int D, bool FEW>
 __global__ __launch_bounds__(D * 4) void attn_chunks_merge_kernel(ChunkArgs c) {
   constexpr int PS = 16 * D + 32;
   const PrefillArgs& a = c.p;
@@ -542,10 +613,13 @@ __global__ __launch_bounds__(D * 4) void attn_chunks_merge_kernel(ChunkArgs c) {
     }
     M = mn;
   }
-  if (qi >= a.S) return;
-  const float inv = 1.0f / l;
-  *reinterpret_cast<uint2*>(a.out + ((size_t)b * a.S + qi) * a.H * D + (size_t)h * D + 16 * db + 4 * g) =
-      make_uint2(pack_bf(sum[0] * inv, sum[1] * inv), pack_bf(sum[2] * inv, sum[3] * inv));
+  const unsigned int odd = FEW ? not_finite((sum[0] + sum[1]) + (sum[2] + sum[3])) : 0;
+  if (qi < a.S && !(odd >> m & 1)) {
+    const float inv = 1.0f / l;
+    *reinterpret_cast<uint2*>(a.out + ((size_t)b * a.S + qi) * a.H * D + (size_t)h * D + 16 * db + 4 * g) =
+        make_uint2(pack_bf(sum[0] * inv, sum[1] * inv), pack_bf(sum[2] * inv, sum[3] * inv));
+  }
+  if (FEW && odd) walk_rows<D>(a, sequence(a, b), h, 0, odd, 16 * db, 16, lane);
 }
 
 // How a call would be cut: no chunks (0) where the kernels above are the better ones, which is where the walk is no longer than 512
@@ -574,26 +648,28 @@ int launch_chunks(const PrefillArgs& a, const Cut& cut, float* part, hipStream_t
   const ChunkArgs c{a, cut, a.H / a.Hkv, part};
   const int n = c.p.B * c.p.Hkv * c.cut.ntb * c.cut.chunks;
   hipLaunchKernelGGL((attn_chunk_kernel<D>), dim3((n + 7) / 8 * 8), dim3(256), 2 * KvTile<D>::SLOT, st, c);
-  hipLaunchKernelGGL((attn_chunks_merge_kernel<D>), dim3(c.p.B * c.p.Hkv * c.cut.tasks), dim3(D * 4), 0, st, c);
+  const dim3 tasks(c.p.B * c.p.Hkv * c.cut.tasks);
+  if (a.S < 16) hipLaunchKernelGGL((attn_chunks_merge_kernel<D, true>), tasks, dim3(D * 4), 0, st, c);
+  else hipLaunchKernelGGL((attn_chunks_merge_kernel<D, false>), tasks, dim3(D * 4), 0, st, c);
   return ohara_launch_status();
 }
 
-template <int D, int QW, bool ALIGNED = true>
+template <int D, int QW, bool ALIGNED = true, bool FEW = false>
 int launch_waves(PrefillArgs a, hipStream_t st) {
   a.nqb = (a.S + 64 * QW - 1) / (64 * QW);
   const int64_t blocks = a.nqb * (a.seqs ? ((int64_t)a.H * a.B + 7) / 8 * 8 : (int64_t)a.H * a.B);
   if (blocks > INT32_MAX) return OHARA_ESIZE;
-  hipLaunchKernelGGL((attn_prefill_kernel<D, QW, ALIGNED>), dim3((unsigned)blocks), dim3(256), 2 * KvTile<D>::SLOT, st, a);
+  hipLaunchKernelGGL((attn_prefill_kernel<D, QW, ALIGNED, FEW>), dim3((unsigned)blocks), dim3(256), 2 * KvTile<D>::SLOT, st, a);
   return ohara_launch_status();
 }
 
-template <int D, int TEAMS, int NST = 3>
+template <int D, int TEAMS, bool FEW = false, int NST = 3>
 int launch_teams(PrefillArgs a, hipStream_t st) {
   constexpr int LDS = NST * KvTile<D>::SLOT + 2 * TEAMS * 4096;
   a.nqb = (a.S + 16 * TEAMS - 1) / (16 * TEAMS);
   if (LDS > 64 * 1024)
-    (void)hipFuncSetAttribute((const void*)attn_team_kernel<D, TEAMS, NST, true>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  hipLaunchKernelGGL((attn_team_kernel<D, TEAMS, NST, true>), dim3((unsigned)(a.nqb * (a.seqs ? (a.H * a.B + 7) / 8 * 8 : a.H * a.B))), dim3(TEAMS * 256), LDS, st, a);
+    (void)hipFuncSetAttribute((const void*)attn_team_kernel<D, TEAMS, NST, true, FEW>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  hipLaunchKernelGGL((attn_team_kernel<D, TEAMS, NST, true, FEW>), dim3((unsigned)(a.nqb * (a.seqs ? (a.H * a.B + 7) / 8 * 8 : a.H * a.B))), dim3(TEAMS * 256), LDS, st, a);
   return ohara_launch_status();
 }
 
@@ -628,8 +704,12 @@ int launch_prefill_for(const PrefillArgs& a, const int32_t* lengths, hipStream_t
     for (int b = 0; b < a.B; ++b) n += (lengths[b] + queries - 1) / queries;
     return n * a.H;
   };
-  if (((uintptr_t)a.k | (uintptr_t)a.v) & 15) return launch_waves<D, 1, false>(a, st);
-  const bool long_walk = a.pos + a.S > 128;
+  const bool aligned = !(((uintptr_t)a.k | (uintptr_t)a.v) & 15), long_walk = a.pos + a.S > 128;
+  if (a.S < 16 && !a.seqs) {  // (a call's own tokens; the rules below come to the same kernels)
+    if (!aligned) return launch_waves<D, 1, false, true>(a, st);
+    return blocks(16) <= CUS * (D == 64 && long_walk ? 2 : 1) ? launch_teams<D, 1, true>(a, st) : launch_waves<D, 1, true, true>(a, st);
+  }
+  if (!aligned) return launch_waves<D, 1, false>(a, st);
   if (blocks(16) <= CUS * (D == 64 && long_walk ? 2 : 1)) return launch_teams<D, 1>(a, st);
   if constexpr (D == 128)
     if (long_walk && blocks(32) <= CUS) return launch_teams<D, 2>(a, st);

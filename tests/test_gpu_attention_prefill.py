@@ -159,3 +159,31 @@ def test_an_infinite_value_in_the_last_chunk_stays_infinite(cuda, S, pos, D):
     got = ops.attn_prefill(q.view(S, H * D), k, v, H, H, D, pos, S).view(1, S, H, D)
     assert (got[..., 0] == float("inf")).all()
     assert ((got.double() - want).abs() <= bound)[..., 1:].all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,S,H,Hkv,pos", [
+    (1, 2, 6, 6, 900), (2, 15, 16, 4, 1000), (1, 9, 20, 4, 700), (1, 15, 6, 2, 570),  # chunks, the new tokens in one tile and across two
+    (4, 8, 16, 16, 0), (2, 5, 16, 4, 33), (1, 15, 6, 2, 56),                         # a team of four waves
+    (40, 3, 16, 16, 20), (20, 15, 32, 8, 60), (70, 2, 8, 8, 126),                    # waves
+])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_a_few_tokens_do_not_see_values_behind_them(cuda, B, S, H, Hkv, pos, D, value):
+    """Two to fifteen tokens a sequence: a value that is not finite reaches the tokens from its own on, in its own column, and no others."""
+    from ohara_amd import ops
+    from ohara_amd._lib import lib
+
+    assert lib().ohara_attn_prefill_wins(B, S, H, Hkv, 128, pos)
+    g = torch.Generator(device=cuda).manual_seed(B + S + H + pos)
+    q, k, v = (torch.randn(B, n, h, D, generator=g, device=cuda).to(BF) for n, h in ((S, H), (pos + S, Hkv), (pos + S, Hkv)))
+    want, bound = _reference(q, k, v, pos)
+    odd = torch.empty(v.numel() + 2, dtype=BF, device=cuda)[2:].view(v.shape)  # (a cache that is not on 16 bytes)
+    for cache in (v.clone(), odd):
+        for at in {1, S // 2, S - 1}:
+            cache.copy_(v)
+            cache[:, pos + at, Hkv - 1, 5] = value
+            got = ops.attn_prefill(q.view(B * S, H * D), k, cache, H, Hkv, D, pos, S).view(B, S, H, D)
+            seen = (slice(None), slice(at, None), slice(H - H // Hkv, None), 5)
+            assert got[seen].isnan().all() if value != value else (got[seen] == value).all()
+            got[seen] = want[seen].to(BF)
+            assert ((got.double() - want).abs() <= bound).all()
