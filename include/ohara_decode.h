@@ -190,8 +190,10 @@ int ohara_attn_prefill_bf16(const uint16_t* q, const uint16_t* kcache, const uin
 int64_t ohara_attn_prefill_ws_bytes(int batch, int seq_len, int h, int h_kv, int dh, int pos);
 int ohara_attn_prefill_ws_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int batch, int seq_len, int h,
                                int h_kv, int dh, int t_max, int pos, uint16_t* out, void* workspace, int64_t workspace_bytes, void* stream);
-/* 1 where they are the faster ones of the two (and take the sizes): ohara_attn_cached_bf16 reads the context once for every token. */
+/* 1 where they are the faster ones of the two (and take the sizes): ohara_attn_cached_bf16 reads the context once for every token.
+ * _with: for a call that has this much room; the other one for one that has what it asks for. */
 int ohara_attn_prefill_wins(int batch, int seq_len, int h, int h_kv, int dh, int pos);
+int ohara_attn_prefill_wins_with(int batch, int seq_len, int h, int h_kv, int dh, int pos, int64_t workspace_bytes);
 
 /* ohara_attn_prefill_bf16 over n prompts of their own lengths, their query rows side by side, each from position 0 of its row of the
  * caches: `lengths` on the host; `seqs` on the device: n first query rows, n lengths, n rows of the caches. */

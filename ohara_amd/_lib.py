@@ -155,6 +155,7 @@ _PROTOS = {
     "ohara_qkv_rope_append_rows_bf16": (_i, [_p, _i, _p, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _p]),
     "ohara_attn_prompts_bf16": (_i, [_p, _p, _p, _i, _p, _p, _i, _i, _i, _i, _p, _p]),
     "ohara_attn_prefill_wins": (_i, [_i, _i, _i, _i, _i, _i]),
+    "ohara_attn_prefill_wins_with": (_i, [_i, _i, _i, _i, _i, _i, _i64]),
     "ohara_attn_prefill_ws_bytes": (_i64, [_i, _i, _i, _i, _i, _i]),
     "ohara_attn_prefill_ws_bf16": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _i64, _p]),
     "ohara_attn_prefill_bf16": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p]),

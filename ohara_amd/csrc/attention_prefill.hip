@@ -762,13 +762,19 @@ extern "C" int64_t ohara_attn_prefill_ws_bytes(int batch, int seq_len, int h, in
 //     8 behind 3000            49 /  9.7   8 x 15 behind 3000 184 / 21.3   2 x 4 behind 200   5.4 /  5.7   8 x 15 behind 3000   459 / 40.7
 //   16 heads of 64: 2 x 8 behind 200 4.2 / 4.9; 4 x 8 8.8 / 4.9; 8 x 2 behind 500 9.1 / 6.9; 2 x 2 5.0 / 6.8
 //   16 heads of 128 on 4 of keys: 2 behind 30 4.7 / 3.8; 8 behind 3000 55 / 10.7; 8 x 15 124 / 18.5
-extern "C" int ohara_attn_prefill_wins(int batch, int seq_len, int h, int h_kv, int dh, int pos) {
+// (2 behind 1000 in one walk, without room: 13.6 us)
+extern "C" int ohara_attn_prefill_wins_with(int batch, int seq_len, int h, int h_kv, int dh, int pos, int64_t workspace_bytes) {
   if (batch < 1 || seq_len < 2 || h < 1 || h_kv < 1 || h % h_kv || (dh != 64 && dh != 128) || pos < 0) return 0;
   if (seq_len >= 16) return 1;
   if (batch > 65535 || h > 65535) return 0;
   const int64_t walks = (int64_t)batch * seq_len * h_kv, far = (int64_t)pos + seq_len;
-  return h / h_kv > 2 || cut(batch, seq_len, h, h_kv, dh, pos).chunks > 1 || walks >= 512 || (walks >= 256 * 128 / dh && far >= 128) ||
-         (walks >= 96 && far >= 384);
+  const Cut c = cut(batch, seq_len, h, h_kv, dh, pos);
+  return h / h_kv > 2 || (c.chunks > 1 && workspace_bytes >= chunk_bytes(c, batch, h_kv, dh)) || walks >= 512 ||
+         (walks >= 256 * 128 / dh && far >= 128) || (walks >= 96 && far >= 384);
+}
+
+extern "C" int ohara_attn_prefill_wins(int batch, int seq_len, int h, int h_kv, int dh, int pos) {
+  return ohara_attn_prefill_wins_with(batch, seq_len, h, h_kv, dh, pos, INT64_MAX);
 }
 
 extern "C" int ohara_attn_prefill_ws_bf16(const uint16_t* q, const uint16_t* kcache, const uint16_t* vcache, int batch, int seq_len, int h,

@@ -34,7 +34,7 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
   hipStream_t hs = (hipStream_t)stream;
   // of attn_ws, what lies behind the counters of decode attention (which stay zero) is room for a prompt's partial results
   const int64_t counters = ((int64_t)B * Hkv * 4 + 255) / 256 * 256;
-  const int64_t room = s->attn_ws ? std::max<int64_t>(0, ohara_attn_workspace_bytes(B, H, Hkv, Dh, s->n_split) - counters) : 0;
+  const int64_t room = s->attn_ws && !((uintptr_t)s->attn_ws & 15) ? std::max<int64_t>(0, ohara_attn_workspace_bytes(B, H, Hkv, Dh, s->n_split) - counters) : 0;
   void* const room_at = s->attn_ws ? (unsigned char*)s->attn_ws + counters : nullptr;
   int launch = 0;
   // Brackets launch number s->prof_kernel with the caller's events.
@@ -86,7 +86,7 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
       OHARA_RUN(ohara_qkv_rope_append_bf16(tiled ? s->xn : s->x, d, L.wqkv, d, tiled ? nullptr : L.norm1, m->eps, B,
                                            seq_len, H, Hkv, Dh, m->cos, m->sin, pos, pos_dev, s->q, s->kcache[l],
                                            s->vcache[l], m->t_max, stream));
-      if (ohara_attn_prefill_wins(B, seq_len, H, Hkv, Dh, pos))
+      if (ohara_attn_prefill_wins_with(B, seq_len, H, Hkv, Dh, pos, room))
         OHARA_RUN(ohara_attn_prefill_ws_bf16(s->q, s->kcache[l], s->vcache[l], B, seq_len, H, Hkv, Dh, m->t_max, pos,
                                              s->attn, room_at, room, stream));
       else
