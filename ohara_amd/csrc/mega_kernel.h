@@ -182,7 +182,14 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
     qkv.wg0 = max(0, nwg - qkv.nstrips);
     dn.wg0 = prj.nstrips + dn.nstrips <= nwg ? prj.nstrips : max(0, nwg - dn.nstrips);
     const int n_chunks = B * Hkv * a.ns;
-    const bool has_attn = (int)blockIdx.x < n_chunks;
+    // One sequence: the chunks on workgroups with no other part, if those are enough; else from workgroup 0 on, the ends of the heads'
+    // contexts first.  The chunk with the new position, over an int8 cache quantised there, is the late one, and behind its chunk a workgroup
+    // of the down projection requests 170 KB, one of the output projection 72.  us a step, a head's chunks together / so (in brackets with
+    // partials merged by every reader of the row): d12 over an int8 cache behind 128 202.9 / 200.2 (201.4), 1024 213.3 / 209.9 (210.7), 3000
+    // 233.3 / 230.4 (230.7); bf16 behind 1024 188.6 / 184.3; 8 heads on 2, 32 workgroups free, int8 210.2 / 197.8 (204.8; not on those 207.3).
+    const int idle0 = max(dn.wg0 + dn.nstrips, (gu.nstrips + 1) >> 1), first_attn = ONE && qkv.wg0 - idle0 >= n_chunks ? idle0 : 0;
+    const int item0 = (int)blockIdx.x - first_attn + ((int)blockIdx.x < first_attn ? nwg : 0);
+    const bool has_attn = item0 < n_chunks;
     const bool has_dn = phase_block(dn) < dn.nstrips;
     const bool has_qkv = phase_block(qkv) < qkv.nstrips;
     const bool has_gu = phase_block(gu) * 2 < gu.nstrips;
@@ -244,7 +251,7 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
       const bool more = l + 1 < m.n_layers;
       // the first K/V tile of this workgroup's attention chunk (the attention workgroups have no q/k/v strip: nothing
       // of theirs is polled for until q is)
-      if (has_attn && !I8) attn_prefetch<D>(B, Hkv, m.t_max, a.ns, kc, vc, L, apre);
+      if (has_attn && !I8) attn_prefetch<D, ONE>(B, Hkv, m.t_max, a.ns, kc, vc, L, apre, item0);
       // P1: [embedding | poll for the stream] + norm1 + QKV + rotary + append; q and the new k / v rows are left tagged
       qkv.kc = kc; qkv.vc = vc; qkv.out = nullptr; qkv.tout = qt; qkv.tkv = kvt; qkv.trow = a.tg_rq; qkv.tkv_row = a.tg_rkv;
       if (has_qkv) {
@@ -257,8 +264,8 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
       gemm_phase<4, 6, E_ROPE, ProfT<PROFILE>, 0, true>(qkv, pre, xs, ldxs, B, red, best_v, best_i, pf);  // 2 stamps
       pf.stamp();  // 4: rotary epilogue, tagged stores issued
       // P2: attention partials (polls for q; the chunk that holds the new position polls for its k / v rows)
-      attn_phase<D, G, true, I8, ONE>(B, H, Hkv, m.t_max, a.blk_x, a.ns, apre, nullptr, reinterpret_cast<float*>(xt + a.tg_p), kc, vc, L, att,
-                                 qt, kvt, pc, a.tg_rq, a.tg_rkv, I8 ? lds_ptr<float>(stab, l) : nullptr, red, qkv.tother);
+      attn_phase<D, G, true, I8, ONE, ONE>(B, H, Hkv, m.t_max, a.blk_x, a.ns, apre, nullptr, reinterpret_cast<float*>(xt + a.tg_p), kc, vc, L, att,
+                                 qt, kvt, pc, a.tg_rq, a.tg_rkv, I8 ? lds_ptr<float>(stab, l) : nullptr, red, qkv.tother, item0);
       pf.stamp();  // 5: partials stored
       // ... and their merge
       for (int u = nwg - 1 - (int)blockIdx.x; u < B * H; u += nwg) {

@@ -1359,12 +1359,20 @@ __device__ __forceinline__ void attn_tile_load_u(const bf16_t* kb, const bf16_t*
   }
 }
 
+// LAST_FIRST (one sequence): the last chunks of all key heads come first.
+template <bool LAST_FIRST = false>
 __device__ __forceinline__ void attn_item_range(int item, int ns, int Hkv, int L, int& b, int& kvh, int& split, int& t0,
                                                 int& t1) {
   const int chunk = (((L + ns - 1) / ns) + 15) & ~15;
-  split = item % ns;
-  kvh = (item / ns) % Hkv;
-  b = item / (ns * Hkv);
+  if (LAST_FIRST) {
+    split = ns - 1 - item / Hkv;
+    kvh = item % Hkv;
+    b = 0;
+  } else {
+    split = item % ns;
+    kvh = (item / ns) % Hkv;
+    b = item / (ns * Hkv);
+  }
   t0 = split * chunk;
   t1 = min(L, t0 + chunk);
 }
@@ -1376,14 +1384,14 @@ __device__ __forceinline__ bool attn_first_tile_prefetchable(int t0, int t1, int
   return tb + 16 <= min(t1, L - 1);
 }
 
-template <int D>
+template <int D, bool LAST_FIRST = false>
 __device__ __forceinline__ void attn_prefetch(int B, int Hkv, int Tmax, int ns, const bf16_t* kc, const bf16_t* vc,
-                                              int L, AttnPre<D>& pre) {
+                                              int L, AttnPre<D>& pre, int item = blockIdx.x) {
   const int wave = threadIdx.x >> 6;
   const size_t row = (size_t)Hkv * D;
   int b, kvh, split, t0, t1;
-  attn_item_range(blockIdx.x, ns, Hkv, L, b, kvh, split, t0, t1);
-  const bool has = (int)blockIdx.x < B * Hkv * ns && attn_first_tile_prefetchable<D>(t0, t1, L);
+  attn_item_range<LAST_FIRST>(item, ns, Hkv, L, b, kvh, split, t0, t1);
+  const bool has = item < B * Hkv * ns && attn_first_tile_prefetchable<D>(t0, t1, L);
   const bf16_t* kb = kc + (size_t)b * Tmax * row + (size_t)kvh * D;
   const bf16_t* vb = vc + (size_t)b * Tmax * row + (size_t)kvh * D;
   attn_tile_load<D>(kb, vb, row, t0 + wave * 16, has ? t1 : 0, -1, pre.k, pre.v);
@@ -1507,7 +1515,7 @@ __device__ __forceinline__ void attn_new_row_i8(const uint32_t* w, int8_t* kq, i
 // AHEAD (with TAG only): a wave's second tile is requested before the poll for q (the single-sequence build: with more
 // sequences a chunk is many tiles and the registers the request holds across the poll are spilled).
 // TAG: the partials go to a polled mailbox too, `other` bytes from its twin in the other set.
-template <int D, int G, bool TAG = false, bool I8 = false, bool AHEAD = false>
+template <int D, int G, bool TAG = false, bool I8 = false, bool AHEAD = false, bool LAST_FIRST = false>
 __device__ __forceinline__ void attn_phase(int B, int H, int Hkv, int Tmax, int blk_x, int ns, const AttnPre<D>& pre,
                                            const char* qm, float* pm, const bf16_t* kc, const bf16_t* vc, int L,
                                            float* lds, const char* qt = nullptr, const char* kvt = nullptr,
@@ -1515,7 +1523,7 @@ __device__ __forceinline__ void attn_phase(int B, int H, int Hkv, int Tmax, int 
                                            int kv_row = 0,  // q_row, kv_row: bytes between the sequences' rows of qt, kvt
                                            float* stats = nullptr,
                                            float* wave_lds = nullptr,  // TAG: 1 KB of LDS per wave, free during this phase
-                                           ptrdiff_t other = 0) {
+                                           ptrdiff_t other = 0, int item0 = blockIdx.x) {  // item0: this workgroup's first item
   static_assert(!I8 || TAG, "the int8 cache is served by the polled builds");
   constexpr int NC = D / 32, DC = D / 8, PP = 64 / DC, NV = 16 / PP;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1530,9 +1538,9 @@ __device__ __forceinline__ void attn_phase(int B, int H, int Hkv, int Tmax, int 
   const size_t row = (size_t)Hkv * D;
   const int PS = D + 32;
   bool first = true;
-  for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
+  for (int item = item0; item < nitems; item += gridDim.x) {
     int b, kvh, split, t0, t1;
-    attn_item_range(item, ns, Hkv, L, b, kvh, split, t0, t1);
+    attn_item_range<LAST_FIRST>(item, ns, Hkv, L, b, kvh, split, t0, t1);
     if (B == 1) b = 0;  // (a single sequence: the row offsets below fold away)
     const bf16_t* kb = kc + (size_t)b * Tmax * row + (size_t)kvh * D;
     const bf16_t* vb = vc + (size_t)b * Tmax * row + (size_t)kvh * D;

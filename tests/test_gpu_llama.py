@@ -402,6 +402,39 @@ def test_persistent_merge_of_an_infinite_value(cuda, H, D, batch):
     assert torch.equal(got, clean)
 
 
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("workgroups,P", [(96, 40), (95, 40), (95, 300), (96, 300), (40, 300)])
+def test_single_sequence_chunks_on_free_workgroups(cuda, workgroups, P, int8):
+    """Attention's 32 chunks on the 32 workgroups with no other part, and, where there are fewer, from the first one on, the last chunks of all
+    heads ahead: steps of both sets of mailboxes against the kernel chain."""
+    import ctypes as C
+
+    from ohara_amd._lib import lib
+    from ohara_amd.llama import Llama
+
+    rcfg, cfg = _cfg_pair(vocab_size=333, hidden_size=256, intermediate_size=256, num_attention_heads=4, num_key_value_heads=2,
+                          num_hidden_layers=3, max_sequence_length=512, dropout=0.0)
+    model = Llama(cfg, R.init_weights(rcfg, seed=9, dtype=BF), device=cuda)
+    ids = torch.randint(0, 333, (1, P), generator=torch.Generator().manual_seed(1)).to(cuda)
+    sess = model.session(1, 8, persistent=True, kv_cache=model.build_kv_cache(1, int8=int8))
+    sess._nwg = workgroups
+    assert lib().ohara_persistent_polled(C.byref(model._c_model), 1, workgroups) == 1
+    sess.prefill(ids)
+    cache = model.build_kv_cache(1, int8=int8)
+    model(ids, cache, 0, last_only=True)
+    for i in range(5):
+        token = torch.tensor([[7 + 31 * i]], device=cuda)
+        want = model(token, cache, P + i, last_only=True)[:, 0]
+        sess.feed(token)
+        sess.step()
+        torch.cuda.synchronize()
+        sess.check_error()
+        _assert_logits_close(sess.logits, want.cpu())
+        for mine, ref in zip(sess.cache, cache):  # what follows compares a step, not what earlier roundings grew to
+            for name in ("key", "value") + (("stats",) if int8 else ()):
+                getattr(mine, name).copy_(getattr(ref, name))
+
+
 @pytest.mark.parametrize("persistent", [True, False])
 def test_sampled_decode_session(cuda, persistent):
     """Temperature 0.8 / top-k 50 / top-p 0.9 decode driven by a pre-drawn uniform tensor, with no
