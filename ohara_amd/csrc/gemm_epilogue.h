@@ -60,6 +60,7 @@ struct GemmArgs {
 // gemm_tile.hip: the tiled kernel for calls with many rows (a.B rows, no fused norm).
 int ohara_launch_gemm_tile(const GemmArgs& a, int epi, int packed_rows, hipStream_t st);
 int ohara_depth_parts(int rows, int packed_rows, int k, float merge_us);
+constexpr int OHARA_PARTS_LDX = (1 << 23) - 1;  // rows further apart: a tile's (256 rows) are not addressed with 32 bits; not in parts
 int ohara_launch_gemm_parts(const GemmArgs& a, int packed_rows, int parts, float* sums, hipStream_t st);
 
 // Rows from which on rows that are normed once and multiplied in tiles are the quicker way, where the strip kernels norm them in every

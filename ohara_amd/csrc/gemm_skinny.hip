@@ -989,7 +989,8 @@ int ohara_gemm_residual_norm_bf16(const uint16_t* x, int ldx, const uint16_t* wp
                                   float eps, uint16_t* xn, void* workspace, int64_t workspace_bytes, void* stream) {
   if (!x || !wp || !resid || n < 1 || k < 1 || rows < 1 || (norm_w && !xn)) return OHARA_EINVAL;
   const int parts = residual_parts(rows, n, k);
-  const bool aligned = !(((uintptr_t)x | (uintptr_t)resid | (uintptr_t)norm_w | (uintptr_t)xn | (uintptr_t)workspace) & 15) && !(ldx & 7) && ldx >= k;
+  const bool aligned = !(((uintptr_t)x | (uintptr_t)resid | (uintptr_t)norm_w | (uintptr_t)xn | (uintptr_t)workspace) & 15) && !(ldx & 7) &&
+                       ldx >= k && ldx <= OHARA_PARTS_LDX;
   if (parts > 1 && aligned && workspace && workspace_bytes >= parts_bytes(parts, rows, n)) {
     GemmArgs a{};
     a.wp = reinterpret_cast<const uint4*>(wp);
@@ -1019,7 +1020,7 @@ int ohara_linear_bias_add2_bf16(const uint16_t* x, int ldx, const uint16_t* wp, 
   if (!x || !wp || !bias || !add1 || !add2 || !out || n < 1 || k < 1 || rows < 1 || ldx < k || ld1 < n || ld2 < n || ldo < n) return OHARA_EINVAL;
   const int parts = bias_parts(rows, n, k);
   const bool aligned = !(((uintptr_t)x | (uintptr_t)bias | (uintptr_t)add1 | (uintptr_t)add2 | (uintptr_t)out | (uintptr_t)workspace) & 15) &&
-                       !((ldx | ld1 | ld2 | ldo) & 7);
+                       !((ldx | ld1 | ld2 | ldo) & 7) && ldx <= OHARA_PARTS_LDX;
   if (parts == 1 || !aligned || !workspace || workspace_bytes < parts_bytes(parts, rows, n))
     return ohara_linear_bias_bf16(x, ldx, wp, n, k, bias, rows, OHARA_LIN_BIAS_ADD2, add1, ld1, add2, ld2, out, ldo, stream);
   GemmArgs a{};

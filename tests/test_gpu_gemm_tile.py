@@ -282,3 +282,30 @@ def test_products_in_parts_of_the_depth(cuda, n, k, rows):
     odd = torch.empty(rows, n + 4, dtype=torch.bfloat16, device=cuda)[:, 4:]  # not on 16 bytes: over the whole depth
     ops.linear_bias(x, packed, bias, "add2", add1=res, add2=add2, out=odd)
     assert ((odd.double() - total).abs() <= total_err).all()
+
+
+def test_rows_far_apart_are_multiplied_whole(cuda):
+    """Rows whose distance the parts of the depth do not address (views into very wide buffers) take the product over the whole depth."""
+    from ohara_amd import ops
+    from ohara_amd._lib import check, lib
+
+    ldx = 1 << 23  # 2^23 elements: a tile of 256 such rows is 4 GiB
+    rows, far = 33, torch.empty(33 * ldx, dtype=torch.bfloat16, device=cuda)
+    g = torch.Generator(device=cuda).manual_seed(1)
+    for n, k in ((2560, 10240), (2048, 5632)):
+        assert lib().ohara_linear_bias_add2_bytes(rows, n, k) > 0 and lib().ohara_gemm_residual_norm_bytes(rows, n, k) > 0
+        x, w = (torch.randn(r, k, generator=g, device=cuda).to(torch.bfloat16) for r in (rows, n))
+        a1, a2 = (torch.randn(rows, n, generator=g, device=cuda).to(torch.bfloat16) for _ in range(2))
+        bias, norm = (torch.randn(n, generator=g, device=cuda).to(torch.bfloat16) for _ in range(2))
+        wide = far.view(rows, ldx)[:, :k]
+        wide.copy_(x)
+        packed, stream = ops.pack_linear(w), torch.cuda.current_stream().cuda_stream
+        whole = torch.empty(rows, n + 4, dtype=torch.bfloat16, device=cuda)[:, 4:]  # (not on 16 bytes: over the whole depth too)
+        ops.linear_bias(x, packed, bias, "add2", add1=a1, add2=a2, out=whole)
+        assert torch.equal(ops.linear_bias(wide, packed, bias, "add2", add1=a1, add2=a2), whole)
+        out, xn = a1.clone(), torch.empty_like(a1)
+        ws = torch.empty(lib().ohara_gemm_residual_norm_bytes(rows, n, k), dtype=torch.uint8, device=cuda)
+        check(lib().ohara_gemm_residual_norm_bf16(wide.data_ptr(), ldx, packed.data.data_ptr(), n, k, rows, out.data_ptr(), norm.data_ptr(), 1e-5,
+                                                  xn.data_ptr(), ws.data_ptr(), ws.numel(), stream), "residual_norm")
+        want = ops.gemm_skinny(x, packed, residual=a1, out=a1.clone())
+        assert torch.equal(out, want) and torch.equal(xn, ops.rmsnorm(want, norm))
