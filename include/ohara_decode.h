@@ -93,6 +93,9 @@ int ohara_swiglu_perm(int f, int32_t* perm_host);
  * (llama.py:84-86,142,322, mlp.py:152 with more than one position per call).  No fused norm. */
 int ohara_gemm_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, int rows, int epilogue,
                     const uint16_t* resid, int ldr, uint16_t* out, int ldo, void* stream);
+/* 1 where rows are best normed ahead of their projection (norm_w then NULL) and not by it: more than 64, more than 32 where k > 1024 and the
+ * packed rows are many, more than 16 where k > 2048.  What ohara_llama_forward does by itself. */
+int ohara_projection_norm_ahead(int rows, int k, int packed_rows);
 /* The tile of such a product over rows that start on 16 bytes: 1000 * its rows + its packed rows (SwiGLU packs two a column). */
 int ohara_gemm_tile_of(int rows, int packed_rows, int k);
 
@@ -468,8 +471,8 @@ typedef struct OharaDecodeState {
   uint16_t* q;           /* (rows, h*dh)                                                  */
   uint16_t* attn;        /* (rows, h*dh)                                                  */
   uint16_t* act;         /* (rows, f)                                                     */
-  uint16_t* xn;          /* (rows, d) normalised rows for calls with > 64 rows (> 16 where d > 1024);
-                            may be NULL (the skinny kernel then norms the rows itself, 64 at a
+  uint16_t* xn;          /* (rows, d) normalised rows for calls with > 64 rows (> 32 where d > 1024, > 16
+                            where d > 2048); may be NULL (the skinny kernel then norms the rows itself, 64 at a
                             time, instead of the tiled MFMA kernel)                            */
   uint16_t* logits;      /* (batch, vocab) or (rows, vocab), see logits_mode              */
   void* attn_ws;         /* ohara_attn_workspace_bytes(batch, h, h_kv, dh, n_split); calls with

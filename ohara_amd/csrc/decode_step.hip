@@ -48,12 +48,14 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
     if (rc) return rc;                                                                      \
   } while (0)
   int rc = 0;
-  const bool tiled = s->xn != nullptr && ohara_tiles_win(R, d);
+  // many rows: normed once, then the tiled MFMA kernel (launches are not numbered)
+  auto normed = [&](int n) { return s->xn != nullptr && ohara_norm_ahead(R, d, (n + 15) / 16 * 16); };
+  const bool qkv_normed = normed((H + 2 * Hkv) * Dh), gu_normed = normed(2 * ((m->d_ff + 7) / 8 * 8));
+  const bool logits_normed = logits_mode == OHARA_LOGITS_ALL && normed(m->vocab);
   OHARA_RUN(ohara_embed_bf16(s->ids, m->token_emb, s->x, R, d, m->vocab, stream));
   for (int l = 0; l < m->n_layers; ++l) {
     const OharaLayer& L = m->layers[l];
-    if (tiled && l == 0) {  // many rows: normalise once, then the tiled MFMA kernel (launches are not numbered); later layers' norms
-                            // come with the residual before them
+    if (qkv_normed && l == 0) {  // later layers' norms come with the residual before them
       rc = ohara_rmsnorm_bf16(s->x, L.norm1, s->xn, R, d, m->eps, stream);
       if (rc) return rc;
     }
@@ -62,7 +64,7 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
       // own position, attention straight over the codes (the extra launch is not numbered)
       int8_t* kq = reinterpret_cast<int8_t*>(s->kcache[l]);
       int8_t* vq = reinterpret_cast<int8_t*>(s->vcache[l]);
-      OHARA_RUN(ohara_qkv_rope_ragged_bf16(tiled ? s->xn : s->x, d, L.wqkv, d, tiled ? nullptr : L.norm1, m->eps, B,
+      OHARA_RUN(ohara_qkv_rope_ragged_bf16(qkv_normed ? s->xn : s->x, d, L.wqkv, d, qkv_normed ? nullptr : L.norm1, m->eps, B,
                                            seq_len, H, Hkv, Dh, m->cos, m->sin, s->seq_pos, m->t_max, s->q, s->kstage,
                                            s->vstage, stream));
       if (seq_len == 1) {
@@ -77,13 +79,13 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
       }
     } else if (ragged) {
       // one position per sequence; attention of any length through the split-context kernel
-      OHARA_RUN(ohara_qkv_rope_append_ragged_bf16(tiled ? s->xn : s->x, d, L.wqkv, d, tiled ? nullptr : L.norm1, m->eps,
+      OHARA_RUN(ohara_qkv_rope_append_ragged_bf16(qkv_normed ? s->xn : s->x, d, L.wqkv, d, qkv_normed ? nullptr : L.norm1, m->eps,
                                                   B, seq_len, H, Hkv, Dh, m->cos, m->sin, s->seq_pos, s->q, s->kcache[l],
                                                   s->vcache[l], m->t_max, stream));
       OHARA_RUN(ohara_attn_cached_ragged_bf16(s->q, s->kcache[l], s->vcache[l], B, seq_len, H, Hkv, Dh, m->t_max,
                                               s->seq_pos, n_split, s->attn_ws, s->attn, stream));
     } else if (!s->kv_int8) {
-      OHARA_RUN(ohara_qkv_rope_append_bf16(tiled ? s->xn : s->x, d, L.wqkv, d, tiled ? nullptr : L.norm1, m->eps, B,
+      OHARA_RUN(ohara_qkv_rope_append_bf16(qkv_normed ? s->xn : s->x, d, L.wqkv, d, qkv_normed ? nullptr : L.norm1, m->eps, B,
                                            seq_len, H, Hkv, Dh, m->cos, m->sin, pos, pos_dev, s->q, s->kcache[l],
                                            s->vcache[l], m->t_max, stream));
       if (ohara_attn_prefill_wins_with(B, seq_len, H, Hkv, Dh, pos, room))
@@ -97,7 +99,7 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
       // dequantised values (the extra launches are not numbered)
       int8_t* kq = reinterpret_cast<int8_t*>(s->kcache[l]);
       int8_t* vq = reinterpret_cast<int8_t*>(s->vcache[l]);
-      OHARA_RUN(ohara_qkv_rope_bf16(tiled ? s->xn : s->x, d, L.wqkv, d, tiled ? nullptr : L.norm1, m->eps, B, seq_len, H,
+      OHARA_RUN(ohara_qkv_rope_bf16(qkv_normed ? s->xn : s->x, d, L.wqkv, d, qkv_normed ? nullptr : L.norm1, m->eps, B, seq_len, H,
                                     Hkv, Dh, m->cos, m->sin, pos, pos_dev, m->t_max, s->q, s->kstage, s->vstage, stream));
       if (seq_len > 1) {
         rc = ohara_kv_quant_append_int8(s->kstage, s->vstage, B, seq_len, Hkv, Dh, pos, pos_dev, kq, vq, s->kvstats[l],
@@ -118,20 +120,23 @@ extern "C" int ohara_llama_forward(const OharaModel* m, const OharaDecodeState* 
                                          n_split, s->attn_ws, s->attn, stream));
       }
     }
-    if (tiled)
-      OHARA_RUN(ohara_gemm_residual_norm_bf16(s->attn, H * Dh, L.wo, d, H * Dh, R, s->x, L.norm2, m->eps, s->xn, room_at, room, stream));
+    const bool parts = qkv_normed || gu_normed;
+    if (parts)
+      OHARA_RUN(ohara_gemm_residual_norm_bf16(s->attn, H * Dh, L.wo, d, H * Dh, R, s->x, gu_normed ? L.norm2 : nullptr, m->eps, s->xn, room_at,
+                                              room, stream));
     else
       OHARA_RUN(ohara_gemm_skinny_bf16(s->attn, H * Dh, L.wo, d, H * Dh, nullptr, m->eps, R, OHARA_EPI_RESIDUAL, s->x, d, s->x, d, stream));
-    OHARA_RUN(ohara_gemm_skinny_bf16(tiled ? s->xn : s->x, d, L.wgu, m->d_ff, d, tiled ? nullptr : L.norm2, m->eps, R,
+    OHARA_RUN(ohara_gemm_skinny_bf16(gu_normed ? s->xn : s->x, d, L.wgu, m->d_ff, d, gu_normed ? nullptr : L.norm2, m->eps, R,
                                      OHARA_EPI_SWIGLU, nullptr, 0, s->act, m->d_ff, stream));
-    const uint16_t* after = l + 1 < m->n_layers ? m->layers[l + 1].norm1 : logits_mode == OHARA_LOGITS_ALL ? m->final_norm : nullptr;
-    if (tiled)
+    const bool last = l + 1 == m->n_layers;
+    const uint16_t* after = last ? (logits_normed ? m->final_norm : nullptr) : qkv_normed ? m->layers[l + 1].norm1 : nullptr;
+    if (parts || after)
       OHARA_RUN(ohara_gemm_residual_norm_bf16(s->act, m->d_ff, L.wdown, d, m->d_ff, R, s->x, after, m->eps, s->xn, room_at, room, stream));
     else
       OHARA_RUN(ohara_gemm_skinny_bf16(s->act, m->d_ff, L.wdown, d, m->d_ff, nullptr, m->eps, R, OHARA_EPI_RESIDUAL, s->x, d, s->x, d, stream));
   }
   if (logits_mode == OHARA_LOGITS_ALL) {
-    OHARA_RUN(ohara_gemm_skinny_bf16(tiled ? s->xn : s->x, d, m->w_vocab, m->vocab, d, tiled ? nullptr : m->final_norm,
+    OHARA_RUN(ohara_gemm_skinny_bf16(logits_normed ? s->xn : s->x, d, m->w_vocab, m->vocab, d, logits_normed ? nullptr : m->final_norm,
                                      m->eps, R, OHARA_EPI_STORE, nullptr, 0, s->logits, m->vocab, stream));
   } else if (logits_mode == OHARA_LOGITS_LAST) {
     // row b*seq_len + seq_len-1 of x for every sequence: a strided view, no gather
@@ -284,14 +289,15 @@ extern "C" int ohara_moe_forward(const OharaMoeCall* cp, void* stream) {
   if (!c.scratch || ((uintptr_t)c.scratch & 255) || c.scratch_bytes < s.bytes) return OHARA_EINVAL;
   const int B = c.batch, S = c.seq_len, R = B * S, d = c.d_model, H = c.n_heads, Hkv = c.n_kv_heads, Dh = c.head_dim;
   const int n_split = S == 1 ? c.n_split : 1;
-  const bool tiled = ohara_tiles_win(R, d);
+  auto ahead = [&](int n) { return ohara_norm_ahead(R, d, (n + 15) / 16 * 16); };
+  const bool qkv_normed = ahead((H + 2 * Hkv) * Dh);
   uint16_t *x = s.x, *next = s.y;
   int rc = ohara_embed_bf16(c.ids, c.token_emb, x, R, d, c.vocab, stream);
   for (int l = 0; l < c.n_layers && !rc; ++l) {
     const OharaMoeLayer& L = c.layers[l];
-    const uint16_t* rows = tiled ? s.xn : x;
-    const uint16_t* norm = tiled ? nullptr : L.norm1;
-    if (tiled) rc = ohara_rmsnorm_bf16(x, L.norm1, s.xn, R, d, c.eps, stream);
+    const uint16_t* rows = qkv_normed ? s.xn : x;
+    const uint16_t* norm = qkv_normed ? nullptr : L.norm1;
+    if (qkv_normed) rc = ohara_rmsnorm_bf16(x, L.norm1, s.xn, R, d, c.eps, stream);
     if (rc) return rc;
     if (c.kvstats) {
       int8_t *kq = (int8_t*)c.kcache[l], *vq = (int8_t*)c.vcache[l];
@@ -319,8 +325,9 @@ extern "C" int ohara_moe_forward(const OharaMoeCall* cp, void* stream) {
     if (!rc) rc = ohara_gemm_skinny_bf16(s.attn, H * Dh, L.wo, d, H * Dh, nullptr, c.eps, R, OHARA_EPI_RESIDUAL, x, d, x, d, stream);
     if (rc) return rc;
     if (!L.router) {
-      if (tiled) rc = ohara_rmsnorm_bf16(x, L.norm2, s.xn, R, d, c.eps, stream);
-      if (!rc) rc = ohara_gemm_skinny_bf16(rows, d, L.wgu, L.ff, d, tiled ? nullptr : L.norm2, c.eps, R, OHARA_EPI_SWIGLU, nullptr, 0, s.act, L.ff, stream);
+      const bool gu_normed = ahead(2 * ((L.ff + 7) / 8 * 8));
+      if (gu_normed) rc = ohara_rmsnorm_bf16(x, L.norm2, s.xn, R, d, c.eps, stream);
+      if (!rc) rc = ohara_gemm_skinny_bf16(gu_normed ? s.xn : x, d, L.wgu, L.ff, d, gu_normed ? nullptr : L.norm2, c.eps, R, OHARA_EPI_SWIGLU, nullptr, 0, s.act, L.ff, stream);
       if (!rc) rc = ohara_gemm_skinny_bf16(s.act, L.ff, L.wdown, d, L.ff, nullptr, c.eps, R, OHARA_EPI_RESIDUAL, x, d, x, d, stream);
       continue;
     }
@@ -351,7 +358,7 @@ extern "C" int ohara_moe_forward(const OharaMoeCall* cp, void* stream) {
   if (rc) return rc;
   // the last token of every sequence: a strided view, normed by the projection
   const bool last = c.last_only && S > 1;
-  const bool normed = !last && tiled;
+  const bool normed = !last && ahead(c.vocab);
   if (normed) rc = ohara_rmsnorm_bf16(x, c.final_norm, s.xn, R, d, c.eps, stream);
   if (rc) return rc;
   return ohara_gemm_skinny_bf16(normed ? s.xn : last ? x + (size_t)(S - 1) * d : x, last ? S * d : d, c.w_vocab, c.vocab, d,

@@ -63,14 +63,29 @@ int ohara_depth_parts(int rows, int packed_rows, int k, float merge_us);
 constexpr int OHARA_PARTS_LDX = (1 << 23) - 1;  // rows further apart: a tile's (256 rows) are not addressed with 32 bits; not in parts
 int ohara_launch_gemm_parts(const GemmArgs& a, int packed_rows, int parts, float* sums, hipStream_t st);
 
-// Rows from which on rows that are normed once and multiplied in tiles are the quicker way, where the strip kernels norm them in every
-// workgroup (or, without a norm, read them there) - 17 at wide models, 65 at narrow ones.  us, normed strips / a norm and tiles, cold
-// weights, at 16, 17, 32, 33 and 64 rows: 3072 x 2048 7.1 11.9 12.4 16.1 17.6 / 9.4 9.5 9.6 9.7 9.8; 11264 x 2048 with SwiGLU 12.5 15.2 16.3
-// 26.9 30.0 / 15.7 15.5 16.9 18.1 20.5; 32000 x 2048 26.8 28.7 29.1 109 156 / 29.4 29.4 29.6 29.7 29.3; but 6144 x 768 4.8 5.7 6.2 7.5 8.4 / 7.0
-// 7.0 7.0 7.7 7.7, 2304 x 768 3.8 4.9 5.2 4.9 6.4 / 6.6 6.6 6.7 6.8 6.8, 3072 x 1024 4.5 6.1 6.3 7.2 8.2 / 7.2 7.2 7.3 7.4 7.3.  With a
-// bias: 17920 x 2560 24.7 40.3 35.7 46.2 64.1 / 23.1 23.2 24.7 24.3 28.7, 2560 x 2560 7.2 11.1 11.7 10.1 12.8 / 7.5 7.7 7.7 7.7 7.7, 2560 x
-// 10240 20.7 34.7 33.3 33.6 43.8 / 31.4 31.5 31.7 31.2 31.4.  (A residual's product has nothing to norm: 65 rows, see its entry point.)
-inline bool ohara_tiles_win(int rows, int k) { return rows > (k > 1024 ? 16 : 64); }
+// Up to 64 rows: where a product in tiles is the quicker one, and where it is with the norm ahead of it as a launch of its own, than the strip
+// kernels, which take a workgroup for every 16 rows of a strip (and norm them there).  W: those workgroups.  us, cold weights, at 17, 32, 33 and
+// 64 rows (W: strips x 2, 2, 3, 4):
+//   plain, strips / tiles   1024 x 2048 5.0 5.1 5.1 5.4 / 6.7 6.8 6.8 6.8;  2048 x 2048 5.5 5.5 7.8 8.0 / 6.8 6.9 6.9 6.9;  6144 x 2048 12.3 11.2 14.8
+//     18.2 / 9.5 9.3 10.0 11.6;  2048 x 1152 4.2 4.6 5.6 6.2 / 5.1 5.2 5.2 5.2;  2560 x 1152 5.9 5.9 5.7 7.6 / 5.2;  1024 x 4096 7.6 7.5 7.9 8.0 / 10.7
+//     10.7 10.7 10.8;  2048 x 4096 8.6 8.1 14.0 13.9 / 14.1 14.0 13.9 13.9;  with rotary, bias, gelu or SwiGLU alike: W > 256, a workgroup a CU
+//   normed strips / norm and tiles   K to 1536: 2048 x 1280 5.6 5.9 7.4 8.2 / 7.9 8.0 8.0 8.1;  2560 x 1536 7.9 8.5 8.0 11.0 / 8.4 8.4 8.5 8.5;
+//     6144 x 1280 9.4 10.2 15.4 18.3 / 9.7 9.8 10.5 11.7;  11264 x 1536 with SwiGLU 12.7 13.2 21.4 23.5 / 13.9 14.9 15.2 17.1: W > 512, from 33 rows.
+//     K to 2048: 2048 x 1792 6.7 6.9 11.3 12.1 / 9.0 9.0 9.1 9.2;  6144 x 2048 12.5 13.2 19.9 23.2 / 12.2 12.1 12.8 14.3;  11264 x 2048 with SwiGLU 16.5 17.6
+//     28.0 30.7 / 16.1 17.4 17.6 20.1;  32000 x 2048 30.9 31.3 112 161 / 30.8 31.1 30.9 31.3: W > 256, from 33 rows (up to 32 they are even alone; a
+//     forward of eight layers, 17, 24 and 32 sequences a token: 2048 wide, 16 heads on 4 461 455 465 / 467 462 466, 1792, 14 on 2 1475 1480 1496 /
+//     1556 1562 1563).  Deeper: 1024 x 2560 11.6 12.5 12.0 12.4, 7680 x 2560 33.8 32.3 40.5 54.2 / 16.8 15.6 16.4 19.2, a forward 1045 1022 995 /
+//     662 661 657: always, from 17.
+// To 1024: 6144 x 768 5.7 6.2 7.5 8.4 / 7.0 7.0 7.7 7.7, 3072 x 1024 6.1 6.3 7.2 8.2 / 7.2 7.3 7.3 7.4: 65 rows.  (By K alone, 17 rows past 1024, narrow
+// projections lost up to 70 % and forwards of 17 to 32 rows up to 10.  A residual's product has nothing to norm: 65 rows, see its entry point.)
+inline int64_t ohara_strip_workgroups(int rows, int packed_rows) { return (int64_t)((rows + 15) / 16) * (packed_rows / 16); }
+inline bool ohara_tiles_win(int rows, int k, int packed_rows) {
+  return rows > 64 || (rows > 16 && k > 1024 && ohara_strip_workgroups(rows, packed_rows) > 256);
+}
+inline bool ohara_norm_ahead(int rows, int k, int packed_rows) {
+  if (rows > 64 || k > 2048) return rows > 16;
+  return rows > 32 && k > 1024 && ohara_strip_workgroups(rows, packed_rows) > (k > 1536 ? 256 : 512);
+}
 
 namespace {
 

@@ -934,6 +934,8 @@ int ohara_pack_rows_bf16(const uint16_t* w, int n, int k, int ldw, const int32_t
   return ohara_launch_status();
 }
 
+int ohara_projection_norm_ahead(int rows, int k, int packed_rows) { return rows > 0 && k > 0 && packed_rows > 0 && ohara_norm_ahead(rows, k, packed_rows); }
+
 int ohara_swiglu_perm(int f, int32_t* perm_host) {
   if (f < 1 || !perm_host) return OHARA_EINVAL;
   const int fp = (f + 7) / 8 * 8;
@@ -967,8 +969,9 @@ int ohara_linear_bias_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n
   a.B = rows; a.N = n; a.K = k;
   a.out = out; a.ldo = ldo; a.bias = bias;
   a.resid = add1; a.ldr = ld1; a.resid2 = add2; a.ldr2 = ld2;
-  if (ohara_tiles_win(rows, k)) return ohara_launch_gemm_tile(a, epi, (n + 15) / 16 * 16, (hipStream_t)stream);
-  return launch_skinny(a, epi, (n + 15) / 16 * 16, (hipStream_t)stream);
+  const int packed_rows = (n + 15) / 16 * 16;
+  if (ohara_tiles_win(rows, k, packed_rows)) return ohara_launch_gemm_tile(a, epi, packed_rows, (hipStream_t)stream);
+  return launch_skinny(a, epi, packed_rows, (hipStream_t)stream);
 }
 
 // ---- products in parts of the depth (ohara_depth_parts), merged by rows ---------------------------------------------------------
@@ -1054,8 +1057,9 @@ int ohara_phi_block_in_bf16(const uint16_t* x, int ldx, const uint16_t* ln_w, co
   a.B = batch * seq_len; a.N = 3 * d + ff; a.K = d;
   a.out = q; a.ldo = ldq; a.out2 = act; a.ldo2 = ldact; a.split_n = 3 * d; a.bias = bias;
   a.S = seq_len; a.Tmax = t_max; a.pos = pos; a.pos_dev = pos_dev; a.kcache = kcache; a.vcache = vcache;
-  if (!ln_w && ohara_tiles_win(a.B, a.K)) return ohara_launch_gemm_tile(a, EPI_PHI_IN, (a.N + 15) / 16 * 16, (hipStream_t)stream);  // prefill
-  return launch_skinny(a, EPI_PHI_IN, (a.N + 15) / 16 * 16, (hipStream_t)stream);
+  const int packed_rows = (a.N + 15) / 16 * 16;
+  if (!ln_w && ohara_tiles_win(a.B, a.K, packed_rows)) return ohara_launch_gemm_tile(a, EPI_PHI_IN, packed_rows, (hipStream_t)stream);  // prefill
+  return launch_skinny(a, EPI_PHI_IN, packed_rows, (hipStream_t)stream);
 }
 
 int ohara_gemm_softcap_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, float cap, int rows,
@@ -1121,7 +1125,8 @@ int ohara_gemm_skinny_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n
   if (epilogue == OHARA_EPI_SWIGLU) packed_rows = 2 * ((n + 7) / 8 * 8);
   else packed_rows = (n + 15) / 16 * 16;
   // (a residual, 17, 33 and 64 rows, strips / tiles: 2048 x 2048 5.6 7.6 7.9 / 6.9 6.9 7.0; 2048 x 5632 11.1 18.7 18.1 / 18.5 18.4 18.6 us)
-  if (!norm_w && (epilogue == OHARA_EPI_RESIDUAL ? batch > 64 : ohara_tiles_win(batch, k))) return ohara_launch_gemm_tile(a, epilogue, packed_rows, (hipStream_t)stream);
+  if (!norm_w && (epilogue == OHARA_EPI_RESIDUAL ? batch > 64 : ohara_tiles_win(batch, k, packed_rows)))
+    return ohara_launch_gemm_tile(a, epilogue, packed_rows, (hipStream_t)stream);
   return launch_skinny(a, epilogue, packed_rows, (hipStream_t)stream);
 }
 
@@ -1143,8 +1148,9 @@ static int qkv_rope_impl(const uint16_t* x, int ldx, const uint16_t* wp, int k, 
   a.out = q_out; a.ldo = h * dh;
   a.H = h; a.Hkv = h_kv; a.Dh = dh; a.Tmax = t_max; a.pos = pos; a.pos_dev = pos_dev; a.pos_stride = pos_stride;
   a.cos = cos; a.sin = sin; a.kcache = kcache; a.vcache = vcache; a.stage = stage;
-  if (!norm_w && ohara_tiles_win(a.B, k)) return ohara_launch_gemm_tile(a, EPI_ROPE, (a.N + 15) / 16 * 16, (hipStream_t)stream);
-  return launch_skinny(a, EPI_ROPE, (a.N + 15) / 16 * 16, (hipStream_t)stream);
+  const int packed_rows = (a.N + 15) / 16 * 16;
+  if (!norm_w && ohara_tiles_win(a.B, k, packed_rows)) return ohara_launch_gemm_tile(a, EPI_ROPE, packed_rows, (hipStream_t)stream);
+  return launch_skinny(a, EPI_ROPE, packed_rows, (hipStream_t)stream);
 }
 
 int ohara_qkv_rope_append_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int k, const uint16_t* norm_w,

@@ -100,21 +100,23 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float = 1e-5, out=None) -> to
 
 
 def norm_rows(k: int) -> int:
-    """Rows whose norm the projection kernels redo in every workgroup; more are normed once, for the tiled kernel (ohara_tiles_win)."""
-    return 16 if k > 1024 else 64
+    """Up to so many rows of this width every projection norms them itself; more may be normed ahead (ohara_projection_norm_ahead)."""
+    return 64 if k <= 1024 else 32 if k <= 2048 else 16
 
 
-def _normed(x, norm_w, eps):
+def _normed(x, norm_w, eps, w: PackedLinear):
     """(rows, norm weight) for a projection: many rows are normed here."""
     if norm_w is not None and x.shape[0] > norm_rows(x.shape[1]):
-        return rmsnorm(x, norm_w, eps), None
+        packed_rows = 2 * ((w.n + 7) // 8 * 8) if w.kind == "swiglu" else (w.n + 15) // 16 * 16
+        if lib().ohara_projection_norm_ahead(x.shape[0], x.shape[1], packed_rows):
+            return rmsnorm(x, norm_w, eps), None
     return x, norm_w
 
 
 def gemm_skinny(x, w: PackedLinear, norm_w=None, eps=1e-5, residual=None, out=None) -> torch.Tensor:
     """y = [rmsnorm(x)] @ W^T (+ residual / SwiGLU epilogue by the packing kind). x: (B, K)."""
     _need(x, BF16, "x")
-    x, norm_w = _normed(x, norm_w, eps)
+    x, norm_w = _normed(x, norm_w, eps, w)
     b, k = x.shape
     if k != w.k:
         raise ValueError(f"x has {k} columns, weight expects {w.k}")
@@ -162,7 +164,7 @@ def qkv_rope_append(x, wqkv: PackedLinear, norm_w, eps, h, h_kv, dh, cos, sin, p
     """x: (batch*seq_len, K) rows ordered (sequence, position).  ``seq_pos`` (int32, one entry per
     sequence, on the device) gives every sequence its own cache position instead of ``pos``."""
     _need(x, BF16, "x")
-    x, norm_w = _normed(x, norm_w, eps)
+    x, norm_w = _normed(x, norm_w, eps, wqkv)
     rows = x.shape[0]
     b = rows // seq_len
     if q_out is None:
@@ -192,7 +194,7 @@ def qkv_rope(x, wqkv: PackedLinear, norm_w, eps, h, h_kv, dh, cos, sin, pos, t_m
     """As ``qkv_rope_append`` with the rotated keys and the values returned as (rows, h_kv*dh) row
     buffers instead of written into a cache -> (q, k, v)."""
     _need(x, BF16, "x")
-    x, norm_w = _normed(x, norm_w, eps)
+    x, norm_w = _normed(x, norm_w, eps, wqkv)
     rows = x.shape[0]
     q = torch.empty(rows, h * dh, dtype=BF16, device=x.device)
     k = torch.empty(rows, h_kv * dh, dtype=BF16, device=x.device)

@@ -402,6 +402,34 @@ def test_persistent_merge_of_an_infinite_value(cuda, H, D, batch):
     assert torch.equal(got, clean)
 
 
+@pytest.mark.parametrize("hidden,ff,vocab,kv,ahead", [
+    (1280, 1408, 640, 2, (False, True, False)),   # q/k/v 112 strips, gate/up 176, logits 40: at 33 rows more than 512 workgroups or not
+    (1280, 264, 9008, 2, (False, False, True)),
+    (1792, 1024, 640, 1, (True, True, False)),
+    (1280, 264, 640, 10, (True, False, False)),
+])
+@pytest.mark.parametrize("B,S", [(3, 11), (40, 1), (1, 64)])
+def test_norms_ahead_of_some_projections(cuda, hidden, ff, vocab, kv, ahead, B, S):
+    """33 to 64 rows at wide models: each projection's rows are normed ahead of it or by it, whatever its neighbours do."""
+    from ohara_amd._lib import lib
+    from ohara_amd.llama import Llama
+
+    rcfg, cfg = _cfg_pair(vocab_size=vocab, hidden_size=hidden, intermediate_size=ff, num_attention_heads=hidden // 128, num_key_value_heads=kv,
+                          num_hidden_layers=2, max_sequence_length=96, dropout=0.0)
+    sizes = (hidden + 256 * kv, 2 * ff, vocab)
+    assert tuple(bool(lib().ohara_projection_norm_ahead(33, hidden, n)) for n in sizes) == ahead
+    w = R.init_weights(rcfg, seed=B + S, dtype=BF)
+    ref, model = R.RefLlama(rcfg, w), Llama(cfg, w, device=cuda)
+    ids = torch.randint(0, vocab, (B, 5 + S), generator=torch.Generator().manual_seed(S))
+    rc, cache = ref.build_kv_cache(B), model.build_kv_cache(B)
+    ref(ids[:, :5], rc, 0)
+    model(ids[:, :5].to(cuda), cache, 0)
+    for mine, theirs in zip(cache, rc):
+        mine.key[:, :5].copy_(theirs.key[:B, :5])
+        mine.value[:, :5].copy_(theirs.value[:B, :5])
+    _assert_logits_close(model(ids[:, 5:].to(cuda), cache, 5), ref(ids[:, 5:], rc, 5))
+
+
 @pytest.mark.parametrize("int8", [False, True])
 @pytest.mark.parametrize("workgroups,P", [(96, 40), (95, 40), (95, 300), (96, 300), (40, 300)])
 def test_single_sequence_chunks_on_free_workgroups(cuda, workgroups, P, int8):

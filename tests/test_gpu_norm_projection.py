@@ -101,12 +101,14 @@ def test_infinite_weights_of_the_last_columns(cuda, rows, n, k):
     assert got[:, rest].isfinite().all()
 
 
-@pytest.mark.parametrize("n,k", [(11264, 2048), (3072, 2048), (16416, 1032)])
+@pytest.mark.parametrize("n,k", [(11264, 2048), (3072, 2048), (16416, 1032), (7680, 2560), (512, 2056)])
 @pytest.mark.parametrize("rows", [17, 33, 64])
 def test_norm_inside_the_projection_at_wide_models(cuda, rows, n, k):
-    """Python norms these rows ahead of the tiles; a caller without room for normed rows (the last rows' logits of a batch) gets the
-    kernels that norm them themselves."""
+    """Python norms these rows ahead of the product where the rule says so (from 33 rows here, from 17 past 2048 columns); a caller without
+    room for normed rows (the last rows' logits of a batch) gets the kernels that norm them themselves."""
     from ohara_amd import _lib, ops
+
+    assert _lib.lib().ohara_projection_norm_ahead(rows, k, n) == (rows > (16 if k > 2048 else 32))
 
     g = torch.Generator(device=cuda).manual_seed(rows + n)
     x, nw = torch.randn(rows, k, generator=g, device=cuda).to(BF), (1 + 0.3 * torch.randn(k, generator=g, device=cuda)).to(BF)
@@ -117,13 +119,15 @@ def test_norm_inside_the_projection_at_wide_models(cuda, rows, n, k):
     _check(out, x, w, nw, 1e-5, ops.gemm_skinny(x, packed, nw, 1e-5))
 
 
+@pytest.mark.parametrize("H,G,K", [(4, 2, 1032), (24, 12, 2056)])
 @pytest.mark.parametrize("batch,seq", [(17, 1), (64, 1), (3, 11), (1, 16), (1, 17)])
-def test_rotary_rows_around_the_change_of_kernel(cuda, batch, seq):
-    """Rows 16 | 17 at a wide model: the same rows one sequence at a time (strips) and together (tiles from 17 on)."""
+def test_rotary_rows_around_the_change_of_kernel(cuda, batch, seq, H, G, K):
+    """Rows 16 | 17 at wide models: the same rows one sequence at a time (strips) and together, in tiles from 17 on where the projection is
+    wide too, in strips where it is narrow."""
     from ohara_amd import ops
 
     g = torch.Generator(device=cuda).manual_seed(batch + seq)
-    H, G, D, K, T, pos = 4, 2, 64, 1032, 40, 5
+    D, T, pos = 64, 40, 5
     x, nw = torch.randn(batch * seq, K, generator=g, device=cuda).to(BF), (1 + 0.3 * torch.randn(K, generator=g, device=cuda)).to(BF)
     wqkv = ops.pack_qkv(*((torch.randn(h * D, K, generator=g, device=cuda) * 0.05).to(BF) for h in (H, G, G)))
     angle = torch.rand(2 * T, D // 2, generator=g, device=cuda)

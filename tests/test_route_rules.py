@@ -1,0 +1,30 @@
+"""Which kernel a call takes, on both sides of the lines (no GPU)."""
+
+import pytest
+
+
+@pytest.mark.parametrize("B,S,H,Hkv,D,pos", [(1, 2, 6, 6, 128, 1000), (1, 8, 6, 6, 128, 3000), (1, 2, 16, 16, 64, 2000)])
+def test_a_few_tokens_without_room_for_chunks(B, S, H, Hkv, D, pos):
+    """What wins only in chunks does not without room for their partial results; sixteen tokens, or walks enough, do either way."""
+    from ohara_amd._lib import lib
+
+    room = lib().ohara_attn_prefill_ws_bytes(B, S, H, Hkv, D, pos)
+    assert room > 0 and lib().ohara_attn_prefill_wins(B, S, H, Hkv, D, pos) == 1
+    assert [lib().ohara_attn_prefill_wins_with(B, S, H, Hkv, D, pos, n) for n in (room, room // 2, 0)] == [1, 0, 0]
+    for b, s in ((B, 16), (40, 15)):
+        assert lib().ohara_attn_prefill_wins_with(b, s, H, Hkv, D, pos, 0) == lib().ohara_attn_prefill_wins(b, s, H, Hkv, D, pos) == 1
+
+
+@pytest.mark.parametrize("rows,k,packed_rows,ahead", [
+    (64, 1024, 65536, 0), (65, 1024, 16, 1), (65, 4096, 16, 1),                    # narrow models; many rows
+    (32, 1025, 65536, 0), (33, 1032, 2720, 0), (33, 1032, 2736, 1), (48, 1536, 2736, 1), (49, 1536, 2048, 0), (64, 1536, 2064, 1),
+    (32, 1544, 65536, 0), (33, 1544, 1360, 0), (33, 2048, 1376, 1), (48, 2048, 1360, 0), (48, 2048, 1376, 1), (64, 2048, 1024, 0), (64, 2048, 1040, 1),
+    (16, 2056, 65536, 0), (17, 2056, 16, 1),
+])
+def test_norms_ahead_of_a_projection(rows, k, packed_rows, ahead):
+    from ohara_amd import ops
+    from ohara_amd._lib import lib
+
+    assert lib().ohara_projection_norm_ahead(rows, k, packed_rows) == ahead
+    assert not ahead or rows > ops.norm_rows(k)
+    assert lib().ohara_projection_norm_ahead(0, k, packed_rows) == lib().ohara_projection_norm_ahead(rows, k, 0) == 0
