@@ -236,9 +236,21 @@ def test_rotary_regions_and_their_edges(cuda, B, S, H, Hkv, D, K):
         assert ((got.double() - want).abs() <= bound + 1e-30).all()
 
 
-@pytest.mark.parametrize("n,k,rows", [(768, 3072, 65), (768, 3072, 129), (768, 3072, 400), (2048, 5632, 33), (2048, 5632, 192), (2048, 5632, 401),
-                                      (2560, 10240, 65), (2560, 10240, 301), (2560, 10240, 1000), (16, 4096, 97), (4096, 4096, 70)])
-def test_products_in_parts_of_the_depth(cuda, n, k, rows):
+# width, depth, rows; the parts of the residual's product and of the one with two addends, and their tiles (1000 rows + columns)
+PARTS = [
+    (768, 3072, 65, (4, 32032), (4, 32032)), (768, 3072, 129, (4, 32032), (4, 32032)), (768, 3072, 400, (4, 64064), None),
+    (768, 3072, 673, (2, 64064), None), (768, 3072, 1281, (2, 64128), None), (2048, 2048, 300, None, None), (2048, 2048, 410, (2, 64064), None),
+    (2048, 5632, 33, (4, 32032), (4, 32032)), (2048, 5632, 192, (4, 64064), (4, 64064)), (2048, 5632, 401, (4, 128128), (4, 128128)),
+    (2048, 5632, 1408, (2, 128192), (2, 128192)), (2048, 5632, 1500, (4, 256256), None), (2048, 5632, 3000, (2, 256256), None),
+    (2560, 10240, 33, (8, 64064), (8, 64064)), (2560, 10240, 65, (8, 64128), (8, 64128)), (2560, 10240, 301, (8, 128128), (8, 128128)),
+    (2560, 10240, 513, (8, 256256), (8, 256256)), (2560, 10240, 1000, (4, 128192), (4, 128192)), (2560, 10240, 2400, (2, 256256), (2, 256256)),
+    (16, 4096, 97, (8, 32032), (8, 32032)), (4096, 4096, 70, (4, 64128), (4, 64128)), (4096, 4096, 228, (2, 64128), (2, 64128)),
+    (4096, 14336, 986, (2, 128128), (2, 128128)),
+]
+
+
+@pytest.mark.parametrize("n,k,rows,residual,add2s", PARTS)
+def test_products_in_parts_of_the_depth(cuda, n, k, rows, residual, add2s):
     """The residual product with the norm behind it, and the one with a bias and two addends, in parts of the depth against 64 bits: an
     fp32 sum of k products in any order, rounded where the products over the whole depth are; without room those are taken."""
     from ohara_amd import ops
@@ -258,7 +270,9 @@ def test_products_in_parts_of_the_depth(cuda, n, k, rows):
     y_err = half(y, sum_err)
     want, want_err = res.double() + y, half(res.double() + y, y_err)
     room = lib().ohara_gemm_residual_norm_bytes(rows, n, k)
-    assert room > 0 or n in (2560, 16)
+    for size, parts in ((room, residual), (lib().ohara_linear_bias_add2_bytes(rows, n, k), add2s)):
+        assert size == (4 * parts[0] * rows * n if parts else 0)
+        assert not parts or lib().ohara_gemm_tile_of(rows, n * parts[0], k // parts[0]) == parts[1]
     for size in {room, 0}:
         ws = torch.full((size + 64,), 0xFF, dtype=torch.uint8, device=cuda)
         out, xn = res.clone(), torch.empty_like(res)
