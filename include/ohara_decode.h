@@ -565,8 +565,8 @@ int ohara_llama_prompts(const OharaModel* m, const OharaDecodeState* s, int n, c
  * what a step relies on, every other slot a step reads was written earlier in the same step, and
  * the merge of the attention chunks never uses a chunk no workgroup wrote).  Call once with
  * init_workspace = 1 (copies the layer table and the cache pointers to the device, zeroes the
- * barrier words, the launch counters and the attention partials behind them and fills the
- * hand-off rows of the polled builds (batch <= 8) with 0xFF, their "not written yet"; synchronises the stream;
+ * barrier words and the launch counters and fills the hand-off rows and the attention partials of the
+ * polled builds (batch <= 8) with 0xFF, their "not written yet"; synchronises the stream;
  * do it outside graph capture) whenever the model or the caches change, and before the workspace
  * is used for the first time or after its memory has been used for anything else; then each call
  * with init_workspace = 0 enqueues one step.  Steps on one workspace must not overlap (each

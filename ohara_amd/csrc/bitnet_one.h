@@ -109,8 +109,9 @@ __device__ __forceinline__ void one_poll(uint4 (&v)[NP], const char* row, int pi
 }
 
 // The codes of a row (bitnet.py:29-33, 49-53) for one BitLinear or two that share it, behind the block's own norm where there is one
-// (norm.py:16-21): the arithmetic of row1_block_norm and row1_codes.  `nw`: this thread's pieces of the norm weights in LDS, those
-// of the block first.  Scales to every thread; each wave leaves its share of the sums of the codes in sumw.
+// (norm.py:16-21).  A sum of squares is a thread's pieces in their order (t, t + 256, ...), the wave's butterfly, then the four waves in
+// theirs; scale, codes and their sum from the same values in the same steps as everywhere (bit_xhat8, bit_mag_max8, bit_codes8).
+// `nw`: this thread's pieces of the norm weights in LDS, those of the block first.  Scales to every thread; each wave leaves its share of the sums of the codes in sumw.
 template <int NP, int NSETS, bool BLOCK>
 __device__ __forceinline__ void one_codes(uint4 (&x)[NP], uint32_t nw, int K, float eps, const BitLds& L, OneRed& red, float (&scale)[2]) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, pieces = K >> 3;

@@ -173,11 +173,11 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
     // (a CU takes in ~55 GB/s) - so the phases are spread over the grid such that a workgroup's next
     // weights can be on their way while it has nothing else to do, long before the poll that precedes
     // their use (a wave's loads return in order: a poll issued behind a batch of weights comes back after
-    // it).  Attention chunks, the output projection and gate/up start at workgroup 0; q/k/v and the down projection (whole K per
-    // strip: 24 k-step tiles per wave from LDS, no partial sums) end with the grid, the latter clear of gate/up, so that its
-    // workgroups have nothing to request between its stores and the next layer's stream.  (Behind the output projection, on
-    // workgroups with attention chunks, those were 0.5 us late each layer: their first tiles came behind 72 KB of weights.)  The heads'
-    // partials are merged just below the down projection, by workgroups that have had their part with q/k/v.
+    // it).  The output projection and gate/up start at workgroup 0, attention's chunks there or on workgroups with no other part (below); q/k/v
+    // ends with the grid; the down projection (whole K per strip: 24 k-step tiles per wave from LDS, no partial sums) follows the output
+    // projection, among gate/up's workgroups.  (At the far end of the grid, clear of both, attention's last chunk was there 0.5 us earlier,
+    // but the activations 0.9 us later.)  The heads' partials are merged by the last workgroups of the grid, which have had their part with
+    // q/k/v.
     dn.nstrips = (d + 15) / 16;
     qkv.wg0 = max(0, nwg - qkv.nstrips);
     dn.wg0 = prj.nstrips + dn.nstrips <= nwg ? prj.nstrips : max(0, nwg - dn.nstrips);
@@ -249,8 +249,8 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
       char* mt = xt + a.tg_m;
       const char* xn_prev = xn - a.tg_stride;       // (l > 0)
       const bool more = l + 1 < m.n_layers;
-      // the first K/V tile of this workgroup's attention chunk (the attention workgroups have no q/k/v strip: nothing
-      // of theirs is polled for until q is)
+      // the first K/V tile of this workgroup's attention chunk (one with a q/k/v strip too - with several sequences chunks reach those -
+      // polls for the stream behind that tile's 8 KB a wave; the others poll for nothing until q)
       if (has_attn && !I8) attn_prefetch<D, ONE>(B, Hkv, m.t_max, a.ns, kc, vc, L, apre, item0);
       // P1: [embedding | poll for the stream] + norm1 + QKV + rotary + append; q and the new k / v rows are left tagged
       qkv.kc = kc; qkv.vc = vc; qkv.out = nullptr; qkv.tout = qt; qkv.tkv = kvt; qkv.trow = a.tg_rq; qkv.tkv_row = a.tg_rkv;
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(256) void decode_mega_kernel(MegaArgs a) {
       };
       if (gate_late || l == 0) gate_weights(0);
       // the next layer's q/k/v weights (+ norm1's, the rotary pair): their registers are free again (behind the attention
-      // phase, which needs many: a workgroup without a chunk - at the usual sizes those with q/k/v strips - is here at once)
+      // phase, which needs many: a workgroup without a chunk - with one sequence, at the usual sizes, those with q/k/v strips - is here at once)
       if (has_qkv && more) {
         qkv.wp = lds_ptr<const uint4>(pl, 8);
         qkv.norm_w = lds_ptr<const bf16_t>(pl, 12);

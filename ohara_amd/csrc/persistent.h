@@ -228,12 +228,6 @@ __device__ __forceinline__ bool mb_ld16(MbRsrc r, int col, uint4& out) {
   return v.x != OHARA_UNWRITTEN && v.y != OHARA_UNWRITTEN && v.z != OHARA_UNWRITTEN && v.w != OHARA_UNWRITTEN;
 }
 
-// two values starting at column `col` (even); true when they have been written
-__device__ __forceinline__ bool mb_ld4(MbRsrc r, int col, uint32_t& out) {
-  out = __builtin_amdgcn_raw_buffer_load_b32(r, (uint32_t)col * 2u, 0, 16);
-  return out != OHARA_UNWRITTEN;
-}
-
 // Strip-blocked mailbox of a (B, N) bf16 matrix: the 16 columns [16s, 16s+16) of all rows
 // form block s of `blk` bytes (a multiple of 128), row b at byte b*32 inside it.
 __device__ __forceinline__ const char* xm_addr(const char* base, int blk, int b, int n) {
