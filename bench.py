@@ -573,21 +573,20 @@ PHASE_STAMPS = (
 PHASE_TAIL = 13  # samples after the layers: three around the final norm, vocabulary projection (2), its end, selection (6), the end
 
 
-def _batch1_roles(cfg, nwg, batch=1):
-    """Which workgroups take which phase of the batch-1 kernel (mirrors the assignment in csrc/mega.hip)."""
+def _polled_roles(cfg, nwg, batch=1):
+    """Which workgroups take which phase of the polled builds (mirrors the assignment in csrc/mega_kernel.h)."""
     d, F = cfg.hidden_size, cfg.intermediate_size
     H = cfg.num_attention_heads
     Hkv = cfg.num_key_value_heads or H
     D = d // H
     n_qkv, n_wo, n_dn = (H + 2 * Hkv) * D // 16, d // 16, d // 16
     n_gu = (2 * ((F + 7) // 8 * 8) // 16 + 1) // 2
-    ns = max(1, min(16, nwg // (batch * Hkv)))
-    p2 = 1 << (ns.bit_length() - 1)
-    if not (2 * ns >= 3 * p2 and ns <= 8):
-        ns = p2
+    chunks = batch * Hkv * max(1, min(16, nwg // (batch * Hkv)))
     dn0 = n_wo if n_wo + n_dn <= nwg else nwg - n_dn
-    return {"qkv": range(nwg - n_qkv, nwg), "attention": range(0, batch * Hkv * ns), "wo": range(0, n_wo),
-            "gate/up": range(0, n_gu), "down": range(dn0, dn0 + n_dn)}
+    free = max(dn0 + n_dn, n_gu)
+    at0 = free if batch == 1 and nwg - n_qkv - free >= chunks else 0
+    return {"qkv": range(nwg - n_qkv, nwg), "attention": range(at0, at0 + min(chunks, nwg)), "merge": range(max(0, nwg - batch * H), nwg),
+            "wo": range(0, n_wo), "gate/up": range(0, n_gu), "down": range(dn0, dn0 + n_dn)}
 
 
 def phase_timeline(dev, prompt_len, steps=32, batch=1, int8=False):
@@ -605,7 +604,7 @@ def phase_timeline(dev, prompt_len, steps=32, batch=1, int8=False):
         sess.step()
     nl = cfg.num_hidden_layers
     per = len(PHASE_STAMPS)
-    roles = _batch1_roles(cfg, sess._nwg, batch)
+    roles = _polled_roles(cfg, sess._nwg, batch)
     acc, total_ms = None, 0.0
     for _ in range(steps):
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -626,7 +625,8 @@ def phase_timeline(dev, prompt_len, steps=32, batch=1, int8=False):
 
     chain = [("qkv", "P1 staged", "stream polled for, norm1 in LDS"), ("qkv", "P1 epilogue", "q/k/v product, rotary, q and new k/v rows stored"),
              ("attention", "P2 partials stored", "q polled for, chunk, partials stored"),
-             ("wo", "P3 merged", "heads merged, their rows polled for"), ("wo", "P3 epilogue", "output projection + residual stored"),
+             ("merge", "P2 requests issued", "a head's partials polled for and merged (and the next q/k/v weights requested)"),
+             ("wo", "P3 merged", "merged rows polled for"), ("wo", "P3 epilogue", "output projection + residual stored"),
              ("gate/up", "P4 staged", "stream polled for, norm2 in LDS"), ("gate/up", "P4 epilogue", "gate/up product, SwiGLU stored"),
              ("down", "P5 staged", "activations polled for, in LDS"), ("down", "P5 epilogue", "down projection + residual stored")]
     seg = torch.zeros(len(chain) + 1, dtype=torch.float64)
