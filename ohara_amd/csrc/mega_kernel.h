@@ -33,9 +33,9 @@
 // whose words the consumers poll for (persistent.h).  So are the attention partials: one workgroup a (sequence, head) polls for its
 // chunks', merges them and hands on the head's part of the row.  (Before, a chunk waited for its own stores, then announced them, and
 // each of the 48 workgroups of the output projection read all partials, 49 KB a sequence: d12 layers at context 1050 took 14.6 us at
-// batch 1, 26.5 at 8, 16.6 over an int8 cache; 14.2, 24.7 and 16.3 now, with gate/up's weights where they delay nobody's chunk.
-// Replies of 40 tokens behind 700: batch 2 9.63 -> 9.09 ms, 8 14.7 -> 13.95, 6 over an int8 cache 15.5 -> 15.0; 64 behind 1024 at batch 1
-// 13.3 -> 13.0; one sequence over an int8 cache 9.01 -> 9.10: its last chunk quantises the new row and hid the wait for the stores.)
+// batch 1, 26.5 at 8, 16.6 over an int8 cache; 13.8, 23.5 and 16.1 now, with gate/up's weights where they delay nobody's chunk and one
+// sequence's late chunks where nobody's weights wait for them.  Replies of 40 tokens behind 700: batch 2 9.63 -> 9.09 ms, 8 14.7 -> 13.95, 6 over an
+// int8 cache 15.5 -> 15.0; 64 behind 1024 at batch 1 13.3 -> 12.75.)
 // Weights are requested where a workgroup is idle, so that no weight load is in flight ahead of a poll (a wave's loads return in order).
 //
 // Every barrier wait is bounded: a workgroup that spins longer than the limit raises a

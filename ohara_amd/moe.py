@@ -225,27 +225,30 @@ class MoeLlama:
 
     def _layer_table(self):
         """The layers for the C chain, from the tensors that they hold now: laid out again where one of them is another."""
-        held = []
+        at = []  # a layer's eleven addresses, and what else the table holds: other widths may come to lie at the same addresses
         for L in self.layers:
             moe = L.get("moe")
-            held += [L["wqkv"].data, L["wo"].data, L["norm1"], L["norm2"]]
+            at += L["wqkv"].data.data_ptr(), L["wo"].data.data_ptr(), L["norm1"].data_ptr(), L["norm2"].data_ptr()
             if moe is None:
-                held += [L["wgu"].data, L["wdown"].data] + [None] * 5
+                wgu = L["wgu"]
+                at += wgu.data.data_ptr(), L["wdown"].data.data_ptr(), 0, 0, 0, 0, 0, wgu.n
+                continue
+            sh, bias = moe.shared, moe.router_bias
+            gu, dn, up = moe.wp_gu, moe.wp_dn, 0
+            if sh is None:
+                at += 0, 0
             else:
-                sh = moe.shared
-                held += [sh and sh[0].data, sh and sh[1].data, moe.router.data, moe.router_bias, moe.wp_gu, moe.wp_dn, moe._counter]
-        at = [0 if t is None else t.data_ptr() for t in held]
-        for L in self.layers:  # (and whatever else the table holds: other widths may come to lie at the same addresses)
-            m = L.get("moe")
-            at.append(L["wgu"].n if m is None else (m.E, m.hidden, m.k, m.biased, m.gate_fn, m.normalize, m.wp_gu.stride(0), m.wp_dn.stride(0),
-                                                    m.shared and m.shared[0].n))
+                at += sh[0].data.data_ptr(), sh[1].data.data_ptr()
+                up = sh[0].n
+            at += (moe.router.data.data_ptr(), 0 if bias is None else bias.data_ptr(), gu.data_ptr(), dn.data_ptr(), moe._counter.data_ptr(),
+                   (moe.E, moe.hidden, moe.k, moe.biased, moe.gate_fn, moe.normalize, gu.stride(0), dn.stride(0), up))
         table, table_of = self._table
         if at != table_of:
             table = (OharaMoeLayer * len(self.layers))()
             for i, L in enumerate(self.layers):
                 c, moe = table[i], L.get("moe")
                 (c.wqkv, c.wo, c.norm1, c.norm2, c.wgu, c.wdown, c.router, c.router_bias, c.experts_gu, c.experts_down,
-                 c.counter) = at[11 * i:11 * i + 11]
+                 c.counter) = at[12 * i:12 * i + 11]
                 if moe is None:
                     c.ff = L["wgu"].n
                 else:
