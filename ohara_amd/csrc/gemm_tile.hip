@@ -2,16 +2,15 @@
 //
 // The walk over K is tile_product (lds_tile.h); the sums do not depend on the tile, but on the parts of the depth they are made of.
 //
-// What bounds it: in large tiles the loads into LDS, the LDS reads and the matrix pipe together (8192 x 8192 x 8192 on zeros: 815 us;
-// without the loads 615, without the reads 749, with neither 535; on random data the chip's clock falls under the products: 960), in
-// small ones the chain barrier - read - multiply of a step (0.14 to 0.36 us).  The kernel before this one (128 x 128, weights straight to
-// registers) against this one, us a call from a graph over twelve sets of random operands in turn: 8192 rows 6144 x 768 with SwiGLU 114 / 85,
-// 2304 x 768 49 / 43, 768 x 768 with a residual 26.9 / 22.7, 768 x 3072 with a residual 65 / 57; 4001 rows 11264 x 2048 with SwiGLU 225 / 169,
-// 2048 x 5632 with a residual 116 / 97; 128 rows 6144 x 768 18.4 / 6.9, 768 x 3072 40.9 / 9.4 (one set again and again, out of the caches: 83,
-// 38, 17.6, 50; 167, 94; 6.2, 8.8).  Of that the epilogues (16 bytes a lane a store instead of 4 or 8, silu with a reciprocal of three
-// instructions instead of eleven) took 5 to 9 %.
-// Measured and dropped: the loads spread among the products (8192^3: 961 -> 1001; with eight k-steps in flight 947, but 128-row tiles
-// 1035 -> 1152), deeper rings (no gain, fewer workgroups a CU), four waves a tile of 128 x 192 (99 / 52 us against 93 / 45 with eight).
+// What bounds it: in the large tiles, whose waves work in two halves (lds_tile.h), the chip's clock under the products (8192 x 8192 x 8192 on
+// zeros 571 us, on random data 715 = 1.54 PFLOP/s; with all waves reading, then all multiplying, and 64 KB in flight 745 and 863), at K of 768
+// a tile's start and epilogue (9 of 25 us a round); in small ones the chain barrier - read - multiply of a step (0.14 to 0.36 us).  us a call, that
+// walk over K / halves, sets of random operands in turn: 256 x 256: 8192 rows 6144 x 768 with SwiGLU 82 / 75, 4001 rows 11264 x 2048 with
+// SwiGLU 179 / 149, 11200 rows 459 / 387, 704 rows 17920 x 2560 77 / 59;  the best of the tiles before / of all: 8192 rows 768 x 3072 with a
+// residual 46 / 38, 768 x 768 17.5 / 15.9, 4001 rows 2048 x 5632 90 / 77, 2048 x 2048 38 / 35.
+// Measured and dropped there: loads among the products (4001 rows 151 / 165), s_setprio around them (even), four waves of 128 x 128 each (160 /
+// 209), 64-byte pieces of activations five steps ahead (151 / 154), halves on 128 x 128 (90 / 94) and on 192-row tiles.  In the small tiles:
+// loads spread among the products, deeper rings (no gain, fewer workgroups a CU), four waves a tile of 128 x 192 (99 / 52 us against 93 / 45).
 //
 // Workgroup ids go round-robin over the eight XCDs: an XCD gets a contiguous run of tiles, eight activation tiles side
 // by side, so that a run shares its operands in that XCD's L2.
@@ -20,6 +19,8 @@
 // ohara/modules/mlp.py:152 when the call carries more than 64 rows.
 #include "gemm_epilogue.h"
 #include "lds_tile.h"
+
+#include <algorithm>
 
 namespace {
 
@@ -77,6 +78,92 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
       coff_t[t] = (((size_t)seq * a.Tmax + pos_t[t]) * a.Hkv) * a.Dh;
     }
     const bool wide = ((a.ldo | (a.Hkv * a.Dh)) & 7) == 0 && (((uintptr_t)a.out | (uintptr_t)a.kcache | (uintptr_t)a.vcache) & 15) == 0;
+    auto column = [&](int r) { return r - (r < nq ? 0 : r < nq + nk ? nq : nq + nk); };  // inside q, k or v
+    auto region_of = [&](int r) { return r < nq ? 0 : r < nq + nk ? 1 : 2; };
+    auto table_row = [&](int t) { return (size_t)min(max(pos_t[t], 0), a.Tmax - 1) * (a.Dh >> 1); };
+    auto turned = [&](f32x4 y, uint32_t cv, uint32_t sv) {
+      float v[4] = {rbf(y[0]), rbf(y[1]), rbf(y[2]), rbf(y[3])};
+#pragma unroll
+      for (int pr = 0; pr < 2; ++pr) {
+        const float c = pr ? hi_bf(cv) : lo_bf(cv), sn = pr ? hi_bf(sv) : lo_bf(sv);
+        const float e = v[2 * pr], od = v[2 * pr + 1];
+        // separate fp32 multiplies and add/sub, as the reference's eager ops round
+        v[2 * pr] = __fsub_rn(__fmul_rn(e, c), __fmul_rn(od, sn));
+        v[2 * pr + 1] = __fadd_rn(__fmul_rn(e, sn), __fmul_rn(od, c));
+      }
+      return make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
+    };
+    // 16 bytes a lane of the left and the right strip of a pair: lanes of even g the left one's, of odd g the right one's
+    auto paired = [&](uint2 l, uint2 r) {
+      const u32x2 x = __builtin_amdgcn_permlane16_swap(l.x, r.x, false, false), y = __builtin_amdgcn_permlane16_swap(l.y, r.y, false, false);
+      return make_uint4(x[0], y[0], x[1], y[1]);
+    };
+    if constexpr (FN == 2 || FN == 4) {
+      // A wave's strips in one head, as heads of whole 16 FN features have them: a row's table values are 16 FN bytes, a quarter a lane in one
+      // load and exchanged, all rows' in one round trip.  (A load of 4 bytes for every strip and row, a round trip a strip: 8192 rows
+      // 2304 x 768, 256 x 256 70.3 us against 49.2 for the plain store, now 50.7 / 44.7; 128 x 256 50.5 / 46.7, now 42.7 / 42.0.)
+      if (wide && a.Dh % (16 * FN) == 0 && nstrips - sbase >= FN && sbase * 16 < nq + 2 * nk && (((uintptr_t)a.cos | (uintptr_t)a.sin) & 15) == 0) {
+        const int rr = sbase * 16, region = region_of(rr), col = column(rr);  // uniform
+        size_t at[FM];
+#pragma unroll
+        for (int t = 0; t < FM; ++t) at[t] = region == 0 ? qoff_t[t] : coff_t[t];
+        constexpr int NB = FM < 4 ? FM : 4;  // rows ahead: all of them are 64 registers more than there are in a tile of 256 x 256
+        uint32_t cv[NB][FN], sv[NB][FN];
+        const int d = col % a.Dh / 2 + 2 * FN * g;
+        auto fetch = [&](int t) {
+          auto quarter = [](const bf16_t* p, uint32_t (&v)[FN]) {
+            if constexpr (FN == 4) {
+              const uint4 q = ldg16(p);
+              v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
+            } else {
+              const uint2 q = ldg8(p);
+              v[0] = q.x, v[1] = q.y;
+            }
+          };
+          quarter(a.cos + table_row(t) + d, cv[t % NB]);
+          quarter(a.sin + table_row(t) + d, sv[t % NB]);
+        };
+        if (region < 2) {
+#pragma unroll
+          for (int t = 0; t < NB; ++t) fetch(t);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        bf16_t* base = (region == 0 ? a.out : region == 1 ? a.kcache : a.vcache) + col + 16 * (g & 1) + 8 * (g >> 1);
+        auto by_strip = [](uint32_t (&v)[FN]) {  // lane group g: from its quarter of the row to its own values of every strip
+          if constexpr (FN == 4) {
+            const u32x2 p = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false), q = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
+            const u32x2 c = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false), d = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+            v[0] = c[0], v[1] = c[1], v[2] = d[0], v[3] = d[1];
+          } else {
+            const u32x2 p = __builtin_amdgcn_permlane16_swap(v[0], v[1], false, false), c = __builtin_amdgcn_permlane32_swap(p[0], p[1], false, false);
+            v[0] = c[0], v[1] = c[1];
+          }
+        };
+#pragma unroll
+        for (int t = 0; t < FM; ++t) {
+          uint2 w[FN];
+          if (region < 2) {
+            by_strip(cv[t % NB]);
+            by_strip(sv[t % NB]);
+#pragma unroll
+            for (int u = 0; u < FN; ++u) w[u] = turned(acc[u][t], cv[t % NB][u], sv[t % NB][u]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (t + NB < FM) fetch(t + NB);
+          } else {
+#pragma unroll
+            for (int u = 0; u < FN; ++u) w[u] = make_uint2(pack_bf(acc[u][t][0], acc[u][t][1]), pack_bf(acc[u][t][2], acc[u][t][3]));
+          }
+          const bool in = rbase + t * 16 + m < a.B && pos_t[t] >= 0 && pos_t[t] < a.Tmax;
+          bf16_t* o = base + at[t];
+#pragma unroll
+          for (int u = 0; u < FN; u += 2) {
+            const uint4 both = paired(w[u], w[u + 1]);
+            if (in) *reinterpret_cast<uint4*>(o + 16 * u) = both;
+          }
+        }
+        return;
+      }
+    }
     uint2 left[FM];  // the strip before, where this one completes 16 bytes a lane with it
 #pragma unroll
     for (int u = 0; u < FN; ++u) {
@@ -84,17 +171,14 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
       const int rr = strip * 16;  // uniform: the whole strip lies in one region and one head
       if (strip >= nstrips || rr >= nq + 2 * nk) continue;
       const bool first = wide && !(u & 1) && u + 1 < FN && strip + 1 < nstrips && rr + 16 < nq + 2 * nk, second = wide && (u & 1);
-      auto column = [&](int r) { return r - (r < nq ? 0 : r < nq + nk ? nq : nq + nk); };  // inside q, k or v
-      auto region_of = [&](int r) { return r < nq ? 0 : r < nq + nk ? 1 : 2; };
       const int region = region_of(rr);
-      const int d = column(rr) % a.Dh + 4 * g;
       uint32_t cv[FM], sv[FM];
       if (region < 2) {
+        const int d = column(rr) % a.Dh + 4 * g;
 #pragma unroll
         for (int t = 0; t < FM; ++t) {
-          const int pc = min(max(pos_t[t], 0), a.Tmax - 1);
-          cv[t] = *reinterpret_cast<const uint32_t*>(a.cos + (size_t)pc * (a.Dh >> 1) + (d >> 1));
-          sv[t] = *reinterpret_cast<const uint32_t*>(a.sin + (size_t)pc * (a.Dh >> 1) + (d >> 1));
+          cv[t] = ldg4(a.cos + table_row(t) + (d >> 1));
+          sv[t] = ldg4(a.sin + table_row(t) + (d >> 1));
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -105,18 +189,8 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
 #pragma unroll
       for (int t = 0; t < FM; ++t) {
         const int b = rbase + t * 16 + m;
-        float v[4] = {rbf(acc[u][t][0]), rbf(acc[u][t][1]), rbf(acc[u][t][2]), rbf(acc[u][t][3])};
-        if (region < 2) {
-#pragma unroll
-          for (int pr = 0; pr < 2; ++pr) {
-            const float c = pr ? hi_bf(cv[t]) : lo_bf(cv[t]), sn = pr ? hi_bf(sv[t]) : lo_bf(sv[t]);
-            const float e = v[2 * pr], od = v[2 * pr + 1];
-            // separate fp32 multiplies and add/sub, as the reference's eager ops round
-            v[2 * pr] = __fsub_rn(__fmul_rn(e, c), __fmul_rn(od, sn));
-            v[2 * pr + 1] = __fadd_rn(__fmul_rn(e, sn), __fmul_rn(od, c));
-          }
-        }
-        const uint2 w = make_uint2(pack_bf(v[0], v[1]), pack_bf(v[2], v[3]));
+        const f32x4 y = acc[u][t];
+        const uint2 w = region < 2 ? turned(y, cv[t], sv[t]) : make_uint2(pack_bf(y[0], y[1]), pack_bf(y[2], y[3]));
         if (first) {
           left[t] = w;
           continue;
@@ -124,9 +198,8 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
         const bool in = b < a.B && pos_t[t] >= 0 && pos_t[t] < a.Tmax;
         bf16_t* o = base + (reg == 0 ? qoff_t[t] : coff_t[t]) + col;
         if (second) {
-          const u32x2 x = __builtin_amdgcn_permlane16_swap(left[t].x, w.x, false, false);
-          const u32x2 y = __builtin_amdgcn_permlane16_swap(left[t].y, w.y, false, false);
-          if (in) *reinterpret_cast<uint4*>(o) = make_uint4(x[0], y[0], x[1], y[1]);
+          const uint4 both = paired(left[t], w);
+          if (in) *reinterpret_cast<uint4*>(o) = both;
         } else if (in) {
           *reinterpret_cast<uint2*>(o) = w;
         }
@@ -295,13 +368,15 @@ int launch_part(const GemmArgs& a, int nstrips, int parts, float* out, hipStream
   return ohara_launch_status();
 }
 
-//           waves fragments k-steps slots ahead
+//           waves fragments k-steps slots ahead (in halves: k-steps a phase, slots of activations and weights)
 typedef Tile<2, 2, 1, 1, 4, 3, 1> T32;       //  32 x  32
 typedef Tile<2, 2, 2, 2, 4, 2, 0> T64;       //  64 x  64
 typedef Tile<2, 4, 2, 2, 2, 3, 1> T64x128;
 typedef Tile<2, 4, 4, 2, 2, 2, 0> T128;
 typedef Tile<2, 4, 4, 3, 2, 2, 0> T128x192;
-typedef Tile<2, 4, 8, 4, 2, 2, 0> T256;
+typedef HalvesTile<2, 4, 8, 4, 1, 3, 4> T256;
+typedef HalvesTile<2, 4, 4, 4, 2, 3, 3> H128x256;
+typedef HalvesTile<2, 4, 4, 3, 2, 3, 3> H128x192;
 
 // Which tile: the one that should take least time.  A large tile needs less LDS traffic a product, a small one keeps more
 // CUs busy and its chain of steps is shorter.  The times are fitted to measurements (63 shapes: 96 to 11200 rows, 768 to 17920 packed
@@ -310,14 +385,24 @@ struct TileTime {
   int rows, strips;
   int slots;    // workgroups that share a CU
   float alone;  // us a step of 64 takes one workgroup on a CU
-  float more;   // what another one beside it adds, as a share of that
+  float more;   // what another one beside it adds, as a share of that (one slot: what a whole round of them adds)
   float full;   // us a step takes each of the workgroups of a full chip
   float ends;   // us the start and the epilogue add
 };
 constexpr TileTime TIMES[6] = {
     {T32::TM, T32::TS, 3, 0.14f, 0.376f, 0.079f, 0.43f},        {T64::TM, T64::TS, 2, 0.295f, 0.23f, 0.189f, 0.6f},
     {T64x128::TM, T64x128::TS, 2, 0.363f, 0.61f, 0.312f, 1.3f}, {T128::TM, T128::TS, 2, 0.60f, 0.56f, 0.453f, 1.45f},
-    {T128x192::TM, T128x192::TS, 2, 0.747f, 0.64f, 0.6f, 3.15f}, {T256::TM, T256::TS, 1, 1.35f, 1.0f, 1.6f, 6.7f},
+    {T128x192::TM, T128x192::TS, 2, 0.747f, 0.64f, 0.6f, 3.15f}, {T256::TM, T256::TS, 1, 1.35f, 0.0f, 1.6f, 6.7f},
+};
+// From 1024 rows on, the tiles in halves among them: fitted to 117 products of 1024 to 16384 rows, 768 to 17920 packed rows, K 768 to 10240,
+// as they stand in a model (the activations just written, weights and caches of other layers before and after): the choice is within
+// 0.4 % of the best on average, 8 % at worst; the six with the times above take 9 % longer on average.  Fewer rows are a round of small
+// tiles or parts of the depth, to which those are fitted.
+constexpr TileTime MANY[8] = {
+    {T32::TM, T32::TS, 3, 0.14f, 0.376f, 0.079f, 2.2f},             {T64::TM, T64::TS, 2, 0.295f, 0.23f, 0.189f, 2.5f},
+    {T64x128::TM, T64x128::TS, 2, 0.481f, 0.529f, 0.372f, 2.13f},   {T128::TM, T128::TS, 2, 0.76f, 0.313f, 0.431f, 3.81f},
+    {T128x192::TM, T128x192::TS, 2, 0.843f, 0.597f, 0.585f, 4.44f}, {T256::TM, T256::TS, 1, 0.859f, 0.501f, 1.342f, 12.6f},
+    {H128x256::TM, H128x256::TS, 1, 0.556f, 0.374f, 0.82f, 8.04f},  {H128x192::TM, H128x192::TS, 1, 0.512f, 0.368f, 0.569f, 6.81f},
 };
 float tile_time(const TileTime& t, int rows, int strips, int K) {
   constexpr int CUS = 256;
@@ -325,17 +410,23 @@ float tile_time(const TileTime& t, int rows, int strips, int K) {
   const int64_t waves = tiles / (CUS * t.slots), rest = tiles % (CUS * t.slots);
   float step = waves * t.slots * t.full;
   if (rest) {
-    const float chain = t.alone * (1.f + t.more * ((rest + CUS - 1) / CUS - 1)), chip = rest * (1.f / CUS) * t.full;
+    const float others = t.slots == 1 ? rest * (1.f / CUS) : (float)((rest + CUS - 1) / CUS - 1);
+    const float chain = t.alone * (1.f + t.more * others), chip = rest * (1.f / CUS) * t.full;
     step += rest <= CUS || chain > chip ? chain : chip;
   }
   return step * K * (1.f / 64.f) + t.ends * (tiles > CUS ? tiles * (1.f / CUS) : 1.f);
 }
 
-int fastest_tile(int rows, int strips, int K) {
+// rotary: the epilogue of three strips a wave reads the tables in pieces of 4 bytes, and among many rows those tiles are not taken for it
+// (2048 rows 2304 x 768 128 x 192 20.7 us, 128 x 256 17.4; 8192 rows 53.1, 256 x 256 52.8)
+int fastest_tile(int rows, int strips, int K, bool rotary = false) {
+  const bool many = rows >= 1024;
+  const TileTime* times = many ? MANY : TIMES;
   int best = 0;
-  float low = tile_time(TIMES[0], rows, strips, K);
-  for (int i = 1; i < 6; ++i) {
-    const float t = tile_time(TIMES[i], rows, strips, K);
+  float low = tile_time(times[0], rows, strips, K);
+  for (int i = 1; i < (K < 64 ? 5 : many ? 8 : 6); ++i) {  // (halves walk whole steps)
+    if (many && rotary && times[i].strips == 12) continue;
+    const float t = tile_time(times[i], rows, strips, K);
     if (t < low) {
       low = t;
       best = i;
@@ -347,17 +438,23 @@ int fastest_tile(int rows, int strips, int K) {
 template <int EPI>
 int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
   if (((uintptr_t)a.x & 15) != 0 || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return launch_tile<EPI, T64, false>(a, nstrips, st);
-  switch (fastest_tile(a.B, nstrips, a.K)) {
+  switch (fastest_tile(a.B, nstrips, a.K, EPI == EPI_ROPE)) {
     case 0: return launch_tile<EPI, T32>(a, nstrips, st);
     case 1: return launch_tile<EPI, T64>(a, nstrips, st);
     case 2: return launch_tile<EPI, T64x128>(a, nstrips, st);
     case 3: return launch_tile<EPI, T128>(a, nstrips, st);
     case 4: return launch_tile<EPI, T128x192>(a, nstrips, st);
-    default: return launch_tile<EPI, T256>(a, nstrips, st);
+    case 5: return launch_tile<EPI, T256>(a, nstrips, st);
+    case 6: return launch_tile<EPI, H128x256>(a, nstrips, st);
+    default: return launch_tile<EPI, H128x192>(a, nstrips, st);
   }
 }
 
-float least_time(int rows, int strips, int K) { return tile_time(TIMES[fastest_tile(rows, strips, K)], rows, strips, K); }
+float least_time(int rows, int strips, int K) {
+  float low = tile_time(TIMES[0], rows, strips, K);
+  for (int i = 1; i < 6; ++i) low = std::min(low, tile_time(TIMES[i], rows, strips, K));
+  return low;
+}
 
 }  // namespace
 
@@ -393,7 +490,9 @@ int ohara_launch_gemm_parts(const GemmArgs& a, int packed_rows, int parts, float
     case 2: return launch_part<T64x128>(a, nstrips, parts, sums, st);
     case 3: return launch_part<T128>(a, nstrips, parts, sums, st);
     case 4: return launch_part<T128x192>(a, nstrips, parts, sums, st);
-    default: return launch_part<T256>(a, nstrips, parts, sums, st);
+    case 5: return launch_part<T256>(a, nstrips, parts, sums, st);
+    case 6: return launch_part<H128x256>(a, nstrips, parts, sums, st);
+    default: return launch_part<H128x192>(a, nstrips, parts, sums, st);
   }
 }
 
@@ -419,7 +518,7 @@ int ohara_launch_gemm_tile(const GemmArgs& a, int epi, int packed_rows, hipStrea
 
 extern "C" int ohara_gemm_tile_of(int rows, int packed_rows, int k) {
   if (rows < 1 || packed_rows < 1 || k < 1) return OHARA_EINVAL;
-  const TileTime& t = TIMES[fastest_tile(rows, (packed_rows + 15) / 16, k)];
+  const TileTime& t = MANY[fastest_tile(rows, (packed_rows + 15) / 16, k)];  // (its sizes are those of both)
   return t.rows * 1000 + t.strips * 16;
 }
 

@@ -18,7 +18,7 @@
 // two products a wave and activation fragment whose step is a chain: the fragments of the next group of products are read before
 // the present group's, across the barrier too.  us a call, 0 / 1, from a graph over one set of operands: 32 x 32 tiles, 96 rows
 // 768 x 3072 10.1 / 8.8; 64 x 128, 192 rows 11264 x 2048 22.5 / 21.9; but 64 x 64, 192 rows 2048 x 5632 28.2 / 30.2; 128 x 192, 8192 rows
-// 768 x 768 and 3072 (a mean) 37.0 / 39.5; 256 x 256 with three groups ahead, 4001 rows 11264 x 2048 174 / 180.
+// 768 x 768 and 3072 (a mean) 37.0 / 39.5.
 // What K leaves for a last step that is not full has its own code behind the loop: inside, its selects cost every step
 // (128 x 128, 4001 rows: 74.3 / 67.7).
 #pragma once
@@ -41,6 +41,7 @@ __device__ __forceinline__ void wait_loads() {  // until at most N of this wave'
 
 template <int WM_, int WN_, int FM_, int FN_, int KH_, int NST_, int LA_>
 struct Tile {
+  static constexpr bool HALVES = false;
   static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, KH = KH_, NST = NST_, LA = LA_;
   static constexpr int NW = WM * WN;                       // waves
   static constexpr int TM = WM * FM * 16, TS = WN * FN;    // rows, strips
@@ -50,6 +51,21 @@ struct Tile {
   static constexpr int STAGE = (XL + WL) * 1024, LDS = NST * STAGE;
   static_assert(XL % NW == 0 && WL % NW == 0, "loads split evenly over the waves");
   static_assert((KH == 2 || KH == 4) && LDS <= 160 * 1024, "");
+};
+
+// A tile whose waves work in two halves (halves_product): PU k-steps of 32 a phase, the activations in a ring of XS slots of 64 columns,
+// the weights in one of WS slots of a phase.
+template <int WM_, int WN_, int FM_, int FN_, int PU_, int XS_, int WS_>
+struct HalvesTile {
+  static constexpr bool HALVES = true;
+  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, KH = 2, PU = PU_, XS = XS_, WS = WS_, LA = 0;
+  static constexpr int NW = WM * WN, TM = WM * FM * 16, TS = WN * FN;
+  static constexpr int RPL = 8, XL = TM / RPL, WL = TS * PU, XPW = XL / NW, WPW = WL / NW;
+  static constexpr int XPP = XPW * PU / 2;                 // activation loads of a wave in a phase
+  static constexpr int XSLOT = XL * 1024, WSLOT = WL * 1024, LDS = XS * XSLOT + WS * WSLOT;
+  static_assert(XL % NW == 0 && WL % NW == 0 && XPW * PU % 2 == 0 && NW == 8, "loads split evenly over the waves and phases; two waves a SIMD");
+  static_assert((PU == 1 && WS == XS + 1) || (PU == 2 && WS == XS), "both rings as far ahead");
+  static_assert(LDS <= 160 * 1024, "");
 };
 
 // Where a lane finds the activations it loads: a byte offset for each of its wave's loads (the caller gives the element offset
@@ -73,9 +89,141 @@ __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
+// The product by two halves of the waves, four each, one wave a SIMD: while one half reads its fragments of a phase from LDS and asks for
+// loads, the other multiplies; a barrier, and they change places.  So a SIMD's matrix pipe has products from one of its two waves and the
+// reads of the other travel under them (before, all eight read first and then all multiplied).  K a phase: 32 where that is 32 products a
+// wave, 64 where it would be 12 or 16 (a phase costs a barrier).  Without its loads the walk takes 478 of 728 us (8192^3, zeros), without its
+// reads 758: what a CU takes in is the bound.  So the activations go by 64 columns, whole 128-byte lines (loads alone: 59 GB/s a CU in
+// 64-byte pieces, 90 in lines; the walk 728 / 571), the weights by phases, both as far ahead as LDS allows.
+// Which slot is free: a phase's loads go into the slots of the phase (activations: the step) before, which the other half has read in the
+// phase between.  What has landed: a wave waits for its own loads of the next phase before the barrier in front of it.
+// Bits: those of tile_product.  K >= 64.
+template <class C>
+__device__ __forceinline__ void halves_product(f32x4 (&acc)[C::FN][C::FM], const char* xb, const XOffsets<C, true>& x, const uint4* wp, int strip0,
+                                               int nstrips, int K, int wave, int lane, unsigned char* smem, int strip_steps) {
+  constexpr int FM = C::FM, FN = C::FN, NW = C::NW, PU = C::PU, PH = 2 / PU, XS = C::XS, WS = C::WS, WPW = C::WPW, XPP = C::XPP;
+  const int wm = wave / C::WN, wn = wave % C::WN, m = lane & 15, g = lane >> 4;
+  const int KS = (K + 31) >> 5, SS = strip_steps ? strip_steps : KS;
+  const int nfull = K >> 6, tail = K & 63;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem, ldsw = lds0 + XS * C::XSLOT;
+  const uint32_t lane16 = lane * 16;
+  const char* wb[WPW];
+#pragma unroll
+  for (int i = 0; i < WPW; ++i)
+    wb[i] = reinterpret_cast<const char*>(wp) + (size_t)min(strip0 + (wave + i * NW) / PU, nstrips - 1) * SS * 1024;
+  // Past the last step the last full one is loaded again, unused: the loads in flight stay the same number.
+  auto load_x = [&](int s, uint32_t slot, int i) {
+    const uint32_t dst = lds0 + slot + (wave + i * NW) * 1024;
+    if (tail && s == nfull) load_lds16(dst, xb + (size_t)s * 128, x.off[i] - (uint32_t)max(0, s * 64 + x.piece[i] * 8 - (K - 8)) * 2);
+    else load_lds16(dst, xb + (size_t)min(s, nfull - 1) * 128, x.off[i]);
+  };
+  auto load_w = [&](int p, uint32_t slot, int i) {
+    const int t = wave + i * NW;
+    load_lds16(ldsw + slot + t * 1024, wb[i] + (size_t)min(p * PU + t % PU, KS - 1) * 1024, lane16);
+  };
+#pragma unroll
+  for (int u = 0; u < FN; ++u)
+#pragma unroll
+    for (int t = 0; t < FM; ++t) acc[u][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const uint32_t xrd = lds0 + (wm * FM * 16 + m) * 128, wrd = ldsw + wn * FN * PU * 1024 + lane16;
+  auto x_frag = [&](uint32_t slot, int jj, int t) { return lds16_at(xrd + slot + t * 2048 + (uint32_t)((4 * jj + g) ^ (m & 7)) * 16); };
+  auto w_frag = [&](uint32_t slot, int j, int u) { return lds16_at(wrd + slot + (u * PU + j) * 1024); };
+  // As many phases' loads ahead as the rings hold, in the order of the phases.
+#pragma unroll
+  for (int i = 0; i < C::XPW; ++i) load_x(0, 0, i);
+#pragma unroll
+  for (int p = 0; p < WS - 1; ++p) {
+    if (p > 0) {
+#pragma unroll
+      for (int i = 0; i < XPP; ++i) {
+        const int l = (p - 1) * XPP + i;  // of the activations' loads behind the first step's
+        load_x(1 + l / C::XPW, (1 + l / C::XPW) * C::XSLOT, l % C::XPW);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < WPW; ++i) load_w(p, p * C::WSLOT, i);
+  }
+  wait_loads<(WS - 2) * (WPW + XPP)>();
+  __builtin_amdgcn_s_barrier();
+  const bool late = wave >= NW / 2;
+  if (late) __builtin_amdgcn_s_barrier();
+  uint32_t xo = 0, xi = (XS - 1) * C::XSLOT, wo = 0, wi = (WS - 1) * C::WSLOT;
+  auto step = [&](int s, auto whole) {  // whole: it asks for whole steps (past the last one, for that)
+#pragma unroll
+    for (int h = 0; h < PH; ++h) {
+      uint4 xf[PU][FM], wf[PU][FN];
+#pragma unroll
+      for (int j = 0; j < PU; ++j) {
+#pragma unroll
+        for (int u = 0; u < FN; ++u) wf[j][u] = w_frag(wo, j, u);
+#pragma unroll
+        for (int t = 0; t < FM; ++t) xf[j][t] = x_frag(xo, h * PU + j, t);
+      }
+      // Into the slots of the phase (the step) before: the other half has read them, a barrier ago.
+      const int p = s * PH + h + WS - 1;
+#pragma unroll
+      for (int i = 0; i < XPP; ++i) {
+        if (decltype(whole)::value) load_lds16(lds0 + xi + (wave + (h * XPP + i) * NW) * 1024, xb + (size_t)min(s + XS - 1, nfull - 1) * 128, x.off[h * XPP + i]);
+        else load_x(s + XS - 1, xi, h * XPP + i);
+      }
+#pragma unroll
+      for (int i = 0; i < WPW; ++i) {
+        const int t = wave + i * NW;
+        if (decltype(whole)::value) load_lds16(ldsw + wi + t * 1024, wb[i] + (size_t)(min(p, nfull * PH - 1) * PU + t % PU) * 1024, lane16);
+        else load_w(p, wi, i);
+      }
+      wait_loads<(WS - 2) * (WPW + XPP)>();  // the next phase's have landed
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < PU; ++j)
+#pragma unroll
+        for (int t = 0; t < FM; ++t)
+#pragma unroll
+          for (int u = 0; u < FN; ++u) acc[u][t] = mfma16(wf[j][u], xf[j][t], acc[u][t]);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      wo = wo + C::WSLOT == WS * C::WSLOT ? 0 : wo + C::WSLOT;
+      wi = wi + C::WSLOT == WS * C::WSLOT ? 0 : wi + C::WSLOT;
+    }
+    xo = xo + C::XSLOT == XS * C::XSLOT ? 0 : xo + C::XSLOT;
+    xi = xi + C::XSLOT == XS * C::XSLOT ? 0 : xi + C::XSLOT;
+  };
+  int s = 0;
+  for (const int n = tail ? nfull - XS + 1 : nfull; s < n; ++s) step(s, std::true_type());
+  for (; s < nfull; ++s) step(s, std::false_type());
+  if (!late) __builtin_amdgcn_s_barrier();
+  wait_loads<0>();
+  if (tail) {
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      if (64 * nfull + 32 * jj >= K) break;  // (uniform) as behind tile_product's loop
+      const bool in = 64 * nfull + 32 * jj + 8 * g < K;
+      const uint32_t slot = PU == 2 || !jj ? wo : wo + C::WSLOT == WS * C::WSLOT ? 0 : wo + C::WSLOT;
+      uint4 wt[FN];
+#pragma unroll
+      for (int u = 0; u < FN; ++u) wt[u] = w_frag(slot, PU == 2 ? jj : 0, u);
+#pragma unroll
+      for (int t = 0; t < FM; ++t) {
+        const uint4 xt = in ? x_frag(xo, jj, t) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < FN; ++u) acc[u][t] = mfma16(wt[u], xt, acc[u][t]);
+      }
+    }
+  }
+}
+
 template <class C, bool ALIGNED>
 __device__ __forceinline__ void tile_product(f32x4 (&acc)[C::FN][C::FM], const char* xb, const XOffsets<C, ALIGNED>& x, const uint4* wp,
                                              int strip0, int nstrips, int K, int wave, int lane, unsigned char* smem, int strip_steps = 0) {
+  if constexpr (C::HALVES) {
+    static_assert(ALIGNED, "");
+    halves_product<C>(acc, xb, x, wp, strip0, nstrips, K, wave, lane, smem, strip_steps);
+  } else {
   constexpr int FM = C::FM, FN = C::FN, KH = C::KH, NST = C::NST, NW = C::NW, XL = C::XL, WL = C::WL, LPW = C::LPW;
   constexpr int STAGE = C::STAGE, KB = 32 * KH;
   const int wm = wave / C::WN, wn = wave % C::WN;
@@ -203,6 +351,7 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[C::FN][C::FM], const c
         for (int u = 0; u < FN; ++u) acc[u][t] = mfma16(wt[u], xt, acc[u][t]);
       }
     }
+  }
   }
 }
 
