@@ -274,3 +274,47 @@ def test_selection_among_ties(cuda, E, k):
     want = torch.sort(-logits, dim=-1, stable=True).indices[:, :k]
     assert torch.equal(idx.cpu().long(), want)
     assert ((w.float().cpu() - torch.sigmoid(logits.gather(1, want))).abs() <= 2.0 ** -8).all()  # bf16 of a value below one
+
+
+@pytest.mark.parametrize("N,d,E,hidden,k", [
+    (180, 72, 6, 64, 2), (200, 264, 6, 40, 2),                        # tiles of 128 pairs
+    (560, 72, 8, 72, 2), (330, 200, 4, 136, 2), (400, 64, 6, 328, 2),  # of 256, one an expert
+    (2100, 136, 5, 72, 2), (1200, 520, 3, 64, 2), (1550, 72, 4, 40, 2),  # and several
+])
+def test_tiles_of_pairs_equal_each_experts_dense_products(cuda, N, d, E, hidden, k):
+    """An expert's pairs in tiles, against its rows by themselves through the dense tiled products, bit for bit: uneven numbers of pairs, an
+    expert without any, depths that end inside a step; rows stored 16 bytes a lane and less."""
+    from ohara_amd import ops
+    from ohara_amd._lib import check, lib
+    from ohara_amd.moe import GroupedMoE
+
+    w, _, x = _make(N, d, E, hidden, k, 0, seed=N + d, std=0.2)
+    w["w_gate"][0] *= 40  # (gates below -87 among them)
+    x = x.to(cuda)
+    moe = GroupedMoE(w["w_gate"], w["w_up"], w["w_down"], w["router"], w["bias"], k, device=cuda)
+    g = torch.Generator().manual_seed(N)
+    share = torch.rand(E, generator=g) + 0.7
+    share[E - 1] = 1e-9  # (no pairs)
+    idx = torch.multinomial(share.expand(N, E), k, generator=g).int().to(cuda)
+    wt = torch.rand(N, k, generator=g).to(BF).to(cuda)
+    offs, pair_of, pos_of = (torch.empty(n, dtype=torch.int32, device=cuda) for n in (E + 1, N * k, N * k))
+    st = torch.cuda.current_stream().cuda_stream
+    check(lib().ohara_moe_sort_pairs(idx.data_ptr(), N * k, E, offs.data_ptr(), pair_of.data_ptr(), pos_of.data_ptr(), st), "sort")
+    for pad in (0, 2):
+        act = torch.full((N * k, hidden + pad), 7.0, dtype=BF, device=cuda)
+        y = torch.full((N * k, d + pad), 7.0, dtype=BF, device=cuda)
+        check(lib().ohara_moe_experts_gate_up_many(x.data_ptr(), d, moe.wp_gu.data_ptr(), moe.wp_gu.stride(0) * 2, E, hidden, d, k, N * k,
+                                                   offs.data_ptr(), pair_of.data_ptr(), act.data_ptr(), hidden + pad, st), "gate_up")
+        rows = act[:, :hidden].contiguous()
+        check(lib().ohara_moe_experts_down_many(rows.data_ptr(), hidden, moe.wp_dn.data_ptr(), moe.wp_dn.stride(0) * 2, E, d, hidden, k, N * k,
+                                                offs.data_ptr(), pair_of.data_ptr(), wt.data_ptr(), y.data_ptr(), d + pad, st), "down")
+        bounds = offs.tolist()
+        assert bounds[E - 1] == bounds[E] == N * k
+        for e in range(E - 1):
+            span = slice(bounds[e], bounds[e + 1])
+            pairs = pair_of[span].long()
+            gates = ops.pack_gate_up(w["w_gate"][e].t().contiguous().to(cuda), w["w_up"][e].t().contiguous().to(cuda))
+            assert torch.equal(rows[span], ops.gemm(x[pairs // k].contiguous(), gates))
+            down = ops.gemm(rows[span].contiguous(), ops.pack_linear(w["w_down"][e].t().contiguous().to(cuda)))
+            assert torch.equal(y[span, :d], (down.float() * wt.view(-1)[pairs].float()[:, None]).to(BF))
+        assert (act[:, hidden:] == 7.0).all() and (y[:, d:] == 7.0).all()
