@@ -167,6 +167,11 @@ int ohara_advance_positions(int32_t* seq_pos, const uint8_t* active, int batch, 
  * an idle slot (it rides along at position 0).  No counterpart in the reference (one position for the batch). */
 int ohara_advance_ragged(int32_t* seq_pos, const uint8_t* active, const int64_t* new_ids, int64_t* next_ids, int batch,
                          int by, void* stream);
+/* Slots of a ragged batch that are taken or left, in one launch: seq_pos[slots[i]] = positions[i] (NULL: 0), active_flags[slots[i]] = active,
+ * next_ids[slots[i]] = ids[i] (NULL: as it is if active, else 0).  slots and positions lie on the host and may change when the call returns;
+ * ids, next_ids, seq_pos and active_flags on the device.  No counterpart in the reference (one position for the batch). */
+int ohara_set_slots(const int32_t* slots, const int32_t* positions, int n, int active, const int64_t* ids, int64_t* next_ids,
+                    int32_t* seq_pos, uint8_t* active_flags, int batch, void* stream);
 
 /* ohara_attn_cached_bf16 for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the

@@ -153,6 +153,7 @@ _PROTOS = {
     "ohara_qkv_rope_append_ragged_bf16": (_i, [_p, _i, _p, _i, _p, _f, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _p]),
     "ohara_advance_positions": (_i, [_p, _p, _i, _i, _p]),
     "ohara_advance_ragged": (_i, [_p, _p, _p, _p, _i, _i, _p]),
+    "ohara_set_slots": (_i, [_p, _p, _i, _i, _p, _p, _p, _p, _i, _p]),
     "ohara_qkv_rope_append_rows_bf16": (_i, [_p, _i, _p, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _p]),
     "ohara_attn_prompts_bf16": (_i, [_p, _p, _p, _i, _p, _p, _i, _i, _i, _i, _p, _p]),
     "ohara_attn_prefill_wins": (_i, [_i, _i, _i, _i, _i, _i]),

@@ -191,6 +191,20 @@ __global__ void advance_ragged_kernel(int32_t* seq_pos, const uint8_t* active, c
   if (on) seq_pos[b] += by;
   next_ids[b] = on ? new_ids[b] : 0;
 }
+// Slots that are taken or left; the host's numbers travel with the launch (a copy of each was a wait for the stream: 16 us, 48 of them
+// for 16 sequences that leave, 32 behind the prompts of 16 that join; 16 prompts with 15 steps 10.7 -> 9.7 ms).
+constexpr int SLOTS = 128;  // of a launch
+struct Slots {
+  int32_t slot[SLOTS], pos[SLOTS];
+};
+__global__ void set_slots_kernel(Slots s, int n, int active, const int64_t* ids, int64_t* next_ids, int32_t* seq_pos, uint8_t* flags) {
+  const int i = threadIdx.x;
+  if (i >= n) return;
+  const int b = s.slot[i];
+  seq_pos[b] = s.pos[i];
+  flags[b] = (uint8_t)active;
+  if (ids || !active) next_ids[b] = ids ? ids[i] : 0;
+}
 }  // namespace
 
 extern "C" {
@@ -240,5 +254,23 @@ extern "C" int ohara_advance_ragged(int32_t* seq_pos, const uint8_t* active, con
   if (!seq_pos || !new_ids || !next_ids || batch < 1) return OHARA_EINVAL;
   hipLaunchKernelGGL(advance_ragged_kernel, dim3((batch + 255) / 256), dim3(256), 0, (hipStream_t)stream, seq_pos,
                      active, new_ids, next_ids, batch, by);
+  return ohara_launch_status();
+}
+
+extern "C" int ohara_set_slots(const int32_t* slots, const int32_t* positions, int n, int active, const int64_t* ids, int64_t* next_ids,
+                               int32_t* seq_pos, uint8_t* active_flags, int batch, void* stream) {
+  if (!slots || !next_ids || !seq_pos || !active_flags || n < 1 || batch < 1) return OHARA_EINVAL;
+  for (int i = 0; i < n; ++i)
+    if (slots[i] < 0 || slots[i] >= batch) return OHARA_EINVAL;
+  for (int i0 = 0; i0 < n; i0 += SLOTS) {
+    const int m = n - i0 < SLOTS ? n - i0 : SLOTS;
+    Slots s{};
+    for (int i = 0; i < m; ++i) {
+      s.slot[i] = slots[i0 + i];
+      s.pos[i] = positions ? positions[i0 + i] : 0;
+    }
+    hipLaunchKernelGGL(set_slots_kernel, dim3(1), dim3(SLOTS), 0, (hipStream_t)stream, s, m, active ? 1 : 0, ids ? ids + i0 : nullptr, next_ids,
+                       seq_pos, active_flags);
+  }
   return ohara_launch_status();
 }

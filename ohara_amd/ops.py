@@ -341,6 +341,22 @@ def advance_ragged(seq_pos: torch.Tensor, active: torch.Tensor | None, new_ids: 
                                      _stream()), "advance_ragged")
 
 
+def set_slots(slots: list[int], positions: list[int] | None, seq_pos: torch.Tensor, active: torch.Tensor, next_ids: torch.Tensor,
+              ids: torch.Tensor | None = None) -> None:
+    """In one launch: seq_pos[slots[i]] = positions[i], active[slots[i]] = 1 and, with ``ids``, next_ids[slots[i]] = ids[i]; without
+    ``positions`` the slots are left: all three 0."""
+    _need(seq_pos, torch.int32, "seq_pos")
+    _need(active, torch.uint8, "active")
+    _need(next_ids, torch.int64, "next_ids")
+    if ids is not None:
+        _need(ids, torch.int64, "ids")
+    n = len(slots)
+    if active.numel() != seq_pos.numel() or next_ids.numel() != seq_pos.numel() or any(len(t) != n for t in (positions, ids) if t is not None):
+        raise ValueError("one position and id per slot are required")
+    check(lib().ohara_set_slots((C.c_int32 * n)(*slots), None if positions is None else (C.c_int32 * n)(*positions), n, int(positions is not None),
+                                _ptr(ids), _ptr(next_ids), _ptr(seq_pos), _ptr(active), seq_pos.numel(), _stream()), "set_slots")
+
+
 _zero_draws: dict = {}  # (rows, device) -> fp32 zeros
 
 
