@@ -327,6 +327,9 @@ int ohara_gemv_ternary_i8(const int8_t* q, int ldq, const float* s, const int32_
  * accumulators are those of ohara_bitlinear_bf16.  ldq a multiple of 16, q on 16 bytes, k a multiple of 8. */
 int ohara_act_quant_sets_int8(const uint16_t* x, int ldx, const uint16_t* pre_norm_w, const uint16_t* const* norm_w, int sets,
                               float eps, int rows, int k, int8_t* q, int ldq, float* s, int32_t* sumq, void* stream);
+/* The same for one BitLinear whose input rows are bf16(bf16(silu(gate)) * up) (ohara/modules/mlp.py:152); gate and up: rows ld apart. */
+int ohara_act_quant_swiglu_int8(const uint16_t* gate, const uint16_t* up, int ld, const uint16_t* norm_w, float eps, int rows, int k,
+                                int8_t* q, int ldq, float* s, int32_t* sumq, void* stream);
 int ohara_gemm_ternary_sets_i8(const int8_t* q, int ldq, const float* s, const int32_t* sumq, const uint32_t* const* wp,
                                const float* gamma, int sets, int n, int k, int rows, uint16_t* const* out, int ldo, void* stream);
 int ohara_gemm_ternary_qkv_rope_append(const int8_t* q, int ldq, const float* s, const int32_t* sumq, const uint32_t* const* wp,

@@ -169,6 +169,7 @@ _PROTOS = {
     "ohara_bitlinear_pack_ternary": (_i, [_p, _i, _i, _i, _p, C.POINTER(_i64), _p]),
     "ohara_act_quant_int8": (_i, [_p, _i, _p, _f, _i, _i, _p, _i, _p, _p, _p]),
     "ohara_gemv_ternary_i8": (_i, [_p, _i, _p, _p, _p, _i, _i, _f, _i, _p, _i, _p, _i, _p, _i, _p]),
+    "ohara_act_quant_swiglu_int8": (_i, [_p, _p, _i, _p, _f, _i, _i, _p, _i, _p, _p, _p]),
     "ohara_act_quant_sets_int8": (_i, [_p, _i, _p, _p, _i, _f, _i, _i, _p, _i, _p, _p, _p]),
     "ohara_gemm_ternary_sets_i8": (_i, [_p, _i, _p, _p, _p, _p, _i, _i, _i, _i, _p, _i, _p]),
     "ohara_gemm_ternary_qkv_rope_append": (_i, [_p, _i, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _p, _i, _p, _p, _p, _p, _i,

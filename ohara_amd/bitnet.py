@@ -172,9 +172,10 @@ class BitLlama:
             if rows <= ops.BIT_ROWS:  # one launch for gate/up + SwiGLU
                 act = ops.bitlinear_gate_up(h, L["norm2"], (L["ff.gate"][1], L["ff.gate"][0]),
                                             (L["ff.up"][1], L["ff.up"][0]), self.eps)
+                h = ops.bitlinear(act, L["ff.down"][1], L["ff.down"][0], self.eps, residual=h)
             else:
-                act = ops.silu_mul(*ops.bitlinear_many(h, L["norm2"], [(L[n][1], L[n][0]) for n in ("ff.gate", "ff.up")], self.eps))
-            h = ops.bitlinear(act, L["ff.down"][1], L["ff.down"][0], self.eps, residual=h)
+                gate, up = ops.bitlinear_many(h, L["norm2"], [(L[n][1], L[n][0]) for n in ("ff.gate", "ff.up")], self.eps)
+                h = ops.bitlinear_swiglu(gate, up, L["ff.down"][1], L["ff.down"][0], self.eps, residual=h)
         if last_only:
             h = h.view(B, S, -1)[:, -1].contiguous()
         logits = ops.gemm_skinny(h, self.w_vocab, norm_w=self.final_norm, eps=self.eps)

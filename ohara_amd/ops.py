@@ -486,6 +486,22 @@ def act_quant_sets(x, norm_ws, eps, pre_norm_w=None):
     return q, s, sq
 
 
+def bitlinear_swiglu(gate, up, norm_w, w: PackedTernary, eps=1e-5, residual=None):
+    """BitLinear on rows silu(gate) * up (rows, K) each, quantised as they are multiplied out, in tiles."""
+    _need(gate, BF16, "gate")
+    _need(up, BF16, "up")
+    rows, k = gate.shape
+    if k != w.k or up.shape != gate.shape:
+        raise ValueError(f"gate and up have {k} and {up.shape[1]} columns, weight expects {w.k}")
+    ldq = (k + 15) // 16 * 16
+    q = torch.empty(rows, ldq, dtype=torch.int8, device=gate.device)
+    s = torch.empty(rows, dtype=torch.float32, device=gate.device)
+    sq = torch.empty(rows, dtype=torch.int32, device=gate.device)
+    check(lib().ohara_act_quant_swiglu_int8(_ptr(gate), _ptr(up), k, _ptr(norm_w), eps, rows, k, _ptr(q), ldq, _ptr(s), _ptr(sq), _stream()),
+          "act_quant_swiglu")
+    return gemv_ternary(q, s, sq, w, residual)
+
+
 def bitlinear_many(x, pre_norm_w, projs, eps=1e-5):
     """Several BitLinears of one width on the same rows (any number), each row quantised once for each -> their outputs.
     ``projs``: at most three (norm_w, PackedTernary) pairs."""
