@@ -374,6 +374,8 @@ typedef Tile<2, 2, 2, 2, 4, 2, 0> T64;       //  64 x  64
 typedef Tile<2, 4, 2, 2, 2, 3, 1> T64x128;
 typedef Tile<2, 4, 4, 2, 2, 2, 0> T128;
 typedef Tile<2, 4, 4, 3, 2, 2, 0> T128x192;
+typedef Tile<4, 1, 1, 3, 4, 3, 1> T64x48;
+typedef Tile<2, 2, 2, 3, 4, 3, 0> T64x96;
 typedef HalvesTile<2, 4, 8, 4, 1, 3, 4> T256;
 typedef HalvesTile<2, 4, 4, 4, 2, 3, 3> H128x256;
 typedef HalvesTile<2, 4, 4, 3, 2, 3, 3> H128x192;
@@ -398,12 +400,25 @@ constexpr TileTime TIMES[6] = {
 // as they stand in a model (the activations just written, weights and caches of other layers before and after): the choice is within
 // 0.4 % of the best on average, 8 % at worst; the six with the times above take 9 % longer on average.  Fewer rows are a round of small
 // tiles or parts of the depth, to which those are fitted.
-constexpr TileTime MANY[8] = {
+constexpr TileTime MANY[10] = {
     {T32::TM, T32::TS, 3, 0.14f, 0.376f, 0.079f, 2.2f},             {T64::TM, T64::TS, 2, 0.295f, 0.23f, 0.189f, 2.5f},
     {T64x128::TM, T64x128::TS, 2, 0.481f, 0.529f, 0.372f, 2.13f},   {T128::TM, T128::TS, 2, 0.76f, 0.313f, 0.431f, 3.81f},
     {T128x192::TM, T128x192::TS, 2, 0.843f, 0.597f, 0.585f, 4.44f}, {T256::TM, T256::TS, 1, 0.859f, 0.501f, 1.342f, 12.6f},
     {H128x256::TM, H128x256::TS, 1, 0.556f, 0.374f, 0.82f, 8.04f},  {H128x192::TM, H128x192::TS, 1, 0.512f, 0.368f, 0.569f, 6.81f},
+    {T64x48::TM, T64x48::TS}, {T64x96::TM, T64x96::TS},  // (by the rule below)
 };
+// Fewer than 1024 rows: 64 x 48 and 64 x 96 where such tiles fill the chip once and those of 32 or 64 would a third round or half of one more:
+// a CU takes in 50 to 90 GB/s, and one tile of 64 x 48 reads 112 rows of operands for the 3072 results of three of 32 x 32, which read 192.
+// us, the best of the six / 64 x 48: 128 rows 6144 x 768 with SwiGLU 6.8 / 5.9, 96 rows 6.0 / 5.7, 33 rows 11264 x 2048 14.2 / 11.8, 192 rows
+// 3072 x 2048 with rotary 13.7 / 11.7, 256 rows 14.8 / 12.1, 320 rows 2048 x 2048 12.6 / 11.5 (two rounds of 32 x 32: 160 rows 3072 x 2048
+// 10.8 / 11.4);  / 64 x 96: 65 to 128 rows 11264 x 2048 17.2 to 18.0 / 15.0 to 15.7, 512 rows 3072 x 2048 19.2 / 17.8 (192 rows 6144 x 768 7.6 / 7.4,
+// 160 rows 6.8 / 7.0).
+int one_round_tile(int rows, int strips, int K) {
+  auto tiles = [&](int r, int s) { return ((int64_t)rows + r - 1) / r * ((strips + s - 1) / s); };
+  const int64_t narrow = tiles(T64x48::TM, T64x48::TS), wide = tiles(T64x96::TM, T64x96::TS);
+  if (K >= 512 && narrow >= 192 && narrow <= 256 && tiles(32, 2) > 512) return 8;
+  return rows > 64 && K >= 1024 && wide >= 192 && wide <= 256 ? 9 : -1;
+}
 float tile_time(const TileTime& t, int rows, int strips, int K) {
   constexpr int CUS = 256;
   const int64_t tiles = ((int64_t)rows + t.rows - 1) / t.rows * ((strips + t.strips - 1) / t.strips);
@@ -421,6 +436,7 @@ float tile_time(const TileTime& t, int rows, int strips, int K) {
 // (2048 rows 2304 x 768 128 x 192 20.7 us, 128 x 256 17.4; 8192 rows 53.1, 256 x 256 52.8)
 int fastest_tile(int rows, int strips, int K, bool rotary = false) {
   const bool many = rows >= 1024;
+  if (const int i = one_round_tile(rows, strips, K); !many && i >= 0) return i;
   const TileTime* times = many ? MANY : TIMES;
   int best = 0;
   float low = tile_time(times[0], rows, strips, K);
@@ -446,7 +462,9 @@ int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
     case 4: return launch_tile<EPI, T128x192>(a, nstrips, st);
     case 5: return launch_tile<EPI, T256>(a, nstrips, st);
     case 6: return launch_tile<EPI, H128x256>(a, nstrips, st);
-    default: return launch_tile<EPI, H128x192>(a, nstrips, st);
+    case 7: return launch_tile<EPI, H128x192>(a, nstrips, st);
+    case 8: return launch_tile<EPI, T64x48>(a, nstrips, st);
+    default: return launch_tile<EPI, T64x96>(a, nstrips, st);
   }
 }
 
@@ -492,7 +510,9 @@ int ohara_launch_gemm_parts(const GemmArgs& a, int packed_rows, int parts, float
     case 4: return launch_part<T128x192>(a, nstrips, parts, sums, st);
     case 5: return launch_part<T256>(a, nstrips, parts, sums, st);
     case 6: return launch_part<H128x256>(a, nstrips, parts, sums, st);
-    default: return launch_part<H128x192>(a, nstrips, parts, sums, st);
+    case 7: return launch_part<H128x192>(a, nstrips, parts, sums, st);
+    case 8: return launch_part<T64x48>(a, nstrips, parts, sums, st);
+    default: return launch_part<T64x96>(a, nstrips, parts, sums, st);
   }
 }
 

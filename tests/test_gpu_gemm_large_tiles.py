@@ -1,5 +1,5 @@
-"""The tiles whose waves work in two halves, and the rotary epilogue by whole rows of the tables: depths that end inside a step, with one
-and before the ring is full, against the same rows in calls of 32 that run small tiles, bit for bit, and against 64 bits; rotated rows
+"""The tiles whose waves work in two halves, those that fill the chip once with few rows, and the rotary epilogue by whole rows of the tables:
+depths that end inside a step, with one and before the ring is full, against the same rows in calls of 32 that run small tiles, bit for bit, and against 64 bits; rotated rows
 against the plain product's, rotated here."""
 
 import pytest
@@ -14,11 +14,12 @@ CASES = [
     (128192, 1024, 6144, 776), (128256, 3000, 2320, 328), (128256, 2049, 3088, 520), (128256, 1537, 4112, 544), (128256, 2049, 3088, 768),
     (256256, 3000, 8208, 168), (256256, 3000, 8208, 192), (256256, 3000, 8208, 200), (256256, 2049, 6160, 296), (256256, 2049, 6160, 320),
     (256256, 1537, 8208, 360),
+    (64048, 128, 6128, 520), (64048, 190, 3056, 776), (64048, 65, 6128, 544), (64096, 100, 11280, 1032), (64096, 500, 3056, 1096), (64096, 470, 3056, 1024),
 ]
 
 
 @pytest.mark.parametrize("tile,rows,packed,k", CASES)
-def test_tiles_in_halves(cuda, tile, rows, packed, k):
+def test_tiles_and_small_ones(cuda, tile, rows, packed, k):
     from ohara_amd import ops
     from ohara_amd._lib import lib
 
@@ -34,6 +35,9 @@ def test_tiles_in_halves(cuda, tile, rows, packed, k):
     assert torch.equal(got, torch.cat([ops.gemm(x[s], wp) for s in spans]))
     assert torch.equal(summed, torch.cat([ops.gemm(x[s], wp, residual=res[s]) for s in spans]))
     assert (got[:, 5] == float("inf")).all()
+    for f in (packed // 2, packed // 2 - 3):
+        gates = ops.pack_gate_up(w[:f].contiguous(), w[f:2 * f].contiguous())
+        assert torch.equal(ops.gemm(x, gates), torch.cat([ops.gemm(x[s], gates) for s in spans]))
     cols = torch.cat([torch.arange(5), torch.arange(6, packed)])
     xd, wd = x.double(), w[cols.to(cuda)].double()
     want = xd @ wd.t()
