@@ -29,7 +29,8 @@ struct GemmArgs {
   int S, row0;  // rows are (sequence, position) pairs: row = seq * S + s, position = pos + s
   int ny, nstrips;  // skinny kernel: 16-row chunks per strip (workgroups of a strip share an XCD) and strips
   const int32_t* pos_dev;
-  const int32_t* rows;  // when set: the position of every row, then (B of them each) the row of the cache its sequence is in
+  const int32_t* rows;  // when set: the position of every row, then (nrows of them each) the row of the cache its sequence is in
+  int nrows;
   int pos_stride;  // 0: *pos_dev is the position of every sequence; 1: pos_dev[seq] (ragged batches)
   const bf16_t* cos;
   const bf16_t* sin;
@@ -259,7 +260,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, int b, int stri
     }
   } else {  // EPI_ROPE: rows [q (H*Dh); k (Hkv*Dh); v (Hkv*Dh)], one position per sequence
     const int grow = a.row0 + b;
-    const int seq = a.rows ? a.rows[a.B + grow] : grow / a.S;
+    const int seq = a.rows ? a.rows[a.nrows + grow] : grow / a.S;
     const int pos = PRE ? p.pos : a.rows ? a.rows[grow] : (a.pos_dev ? a.pos_dev[(size_t)seq * a.pos_stride] : a.pos) + (grow - seq * a.S);
     const int nq = a.H * a.Dh, nk = a.Hkv * a.Dh;
     if (r0 >= nq + 2 * nk || pos < 0 || pos >= a.Tmax) return;

@@ -1181,7 +1181,7 @@ int ohara_qkv_rope_append_rows_bf16(const uint16_t* x, int ldx, const uint16_t* 
   a.x = x; a.ldx = ldx;
   a.B = rows; a.N = (h + 2 * h_kv) * dh; a.K = k; a.S = 1;
   a.out = q_out; a.ldo = h * dh;
-  a.H = h; a.Hkv = h_kv; a.Dh = dh; a.Tmax = t_max; a.rows = at;
+  a.H = h; a.Hkv = h_kv; a.Dh = dh; a.Tmax = t_max; a.rows = at; a.nrows = rows;
   a.cos = cos; a.sin = sin; a.kcache = kcache; a.vcache = vcache;
   return ohara_launch_gemm_tile(a, EPI_ROPE, (a.N + 15) / 16 * 16, (hipStream_t)stream);
 }

@@ -68,7 +68,7 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
       int seq;
       if (a.rows) {
         pos_t[t] = a.rows[x];
-        seq = a.rows[a.B + x];
+        seq = a.rows[a.nrows + x];
       } else {
         const bool wrap = x >= a.S;
         seq = seq0 + (wrap ? 1 : 0);
@@ -398,13 +398,13 @@ constexpr TileTime TIMES[6] = {
 };
 // From 1024 rows on, the tiles in halves among them: fitted to 117 products of 1024 to 16384 rows, 768 to 17920 packed rows, K 768 to 10240,
 // as they stand in a model (the activations just written, weights and caches of other layers before and after): the choice is within
-// 0.4 % of the best on average, 8 % at worst; the six with the times above take 9 % longer on average.  Fewer rows are a round of small
-// tiles or parts of the depth, to which those are fitted.
+// 0.3 % of the best on average, 8 % at worst; the six with the times above take 9 % longer on average.  A tile alone on its CU pays its ends
+// once in every round.  Fewer rows are a round of small tiles or parts of the depth, to which those are fitted.
 constexpr TileTime MANY[10] = {
     {T32::TM, T32::TS, 3, 0.14f, 0.376f, 0.079f, 2.2f},             {T64::TM, T64::TS, 2, 0.295f, 0.23f, 0.189f, 2.5f},
-    {T64x128::TM, T64x128::TS, 2, 0.481f, 0.529f, 0.372f, 2.13f},   {T128::TM, T128::TS, 2, 0.76f, 0.313f, 0.431f, 3.81f},
-    {T128x192::TM, T128x192::TS, 2, 0.843f, 0.597f, 0.585f, 4.44f}, {T256::TM, T256::TS, 1, 0.859f, 0.501f, 1.342f, 12.6f},
-    {H128x256::TM, H128x256::TS, 1, 0.556f, 0.374f, 0.82f, 8.04f},  {H128x192::TM, H128x192::TS, 1, 0.512f, 0.368f, 0.569f, 6.81f},
+    {T64x128::TM, T64x128::TS, 2, 0.405f, 0.529f, 0.346f, 2.13f},   {T128::TM, T128::TS, 2, 0.76f, 0.313f, 0.497f, 3.81f},
+    {T128x192::TM, T128x192::TS, 2, 0.94f, 0.575f, 0.633f, 4.81f},  {T256::TM, T256::TS, 1, 0.843f, 0.571f, 1.252f, 12.19f},
+    {H128x256::TM, H128x256::TS, 1, 0.561f, 0.53f, 0.762f, 7.48f},  {H128x192::TM, H128x192::TS, 1, 0.429f, 0.533f, 0.6f, 6.73f},
     {T64x48::TM, T64x48::TS}, {T64x96::TM, T64x96::TS},  // (by the rule below)
 };
 // Fewer than 1024 rows: 64 x 48 and 64 x 96 where such tiles fill the chip once and those of 32 or 64 would a third round or half of one more:
@@ -429,7 +429,8 @@ float tile_time(const TileTime& t, int rows, int strips, int K) {
     const float chain = t.alone * (1.f + t.more * others), chip = rest * (1.f / CUS) * t.full;
     step += rest <= CUS || chain > chip ? chain : chip;
   }
-  return step * K * (1.f / 64.f) + t.ends * (tiles > CUS ? tiles * (1.f / CUS) : 1.f);
+  const float rounds = t.slots == 1 ? (float)((tiles + CUS - 1) / CUS) : tiles > CUS ? tiles * (1.f / CUS) : 1.f;
+  return step * K * (1.f / 64.f) + t.ends * rounds;
 }
 
 // rotary: the epilogue of three strips a wave reads the tables in pieces of 4 bytes, and among many rows those tiles are not taken for it
@@ -451,10 +452,40 @@ int fastest_tile(int rows, int strips, int K, bool rotary = false) {
   return best;
 }
 
+// A part of the rows in whole rounds of large tiles, one a CU, and the rest by itself, where the last round would be nearly empty: how many
+// rows and which tile (0 rows: all in one launch).  The times of two launches are those of MANY, added; taken from 8 % on.  us, one / two
+// launches: 2304 x 768 with rotary, 7600, 8192, 16384 rows 48.0 57.4 82.8 / 39.9 44.4 73.2; 6144 x 768 with SwiGLU, 5500, 11200 rows 66.2 117 /
+// 58.1 107; 3072 x 2048 with rotary, 5500, 11200 rows 87.8 144 / 65.1 125; 11264 x 2048 with SwiGLU, 3000 rows 142 / 125; 2048 x 5632, 11200
+// rows 226 / 204; 2560 x 10240, 8192 rows 375 / 326.  (At 7 % and less the model is not that good: 6144 x 768, 3000 rows 37.5 / 40.4.)
+struct Split {
+  int rows, tile;
+};
+Split split_rows(int rows, int strips, int K, bool rotary) {
+  Split best{0, 0};
+  if (rows < 1024 || K < 64) return best;
+  auto least = [&](int r) {
+    float low = tile_time(MANY[0], r, strips, K);
+    for (int i = 1; i < 8; ++i)
+      if (!rotary || MANY[i].strips != 12) low = std::min(low, tile_time(MANY[i], r, strips, K));
+    return low;
+  };
+  float low = 0.92f * least(rows);
+  for (int i = 5; i < 7; ++i) {  // 256 x 256, 128 x 256
+    const int64_t across = (strips + MANY[i].strips - 1) / MANY[i].strips, down = ((int64_t)rows + MANY[i].rows - 1) / MANY[i].rows;
+    const int64_t first = across * down / 256 * 256 / across * MANY[i].rows;
+    if (first < 1 || first >= rows) continue;
+    const float t = tile_time(MANY[i], (int)first, strips, K) + least(rows - (int)first);
+    if (t < low) {
+      low = t;
+      best = {(int)first, i};
+    }
+  }
+  return best;
+}
+
 template <int EPI>
-int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
-  if (((uintptr_t)a.x & 15) != 0 || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return launch_tile<EPI, T64, false>(a, nstrips, st);
-  switch (fastest_tile(a.B, nstrips, a.K, EPI == EPI_ROPE)) {
+int launch_of(int tile, const GemmArgs& a, int nstrips, hipStream_t st) {
+  switch (tile) {
     case 0: return launch_tile<EPI, T32>(a, nstrips, st);
     case 1: return launch_tile<EPI, T64>(a, nstrips, st);
     case 2: return launch_tile<EPI, T64x128>(a, nstrips, st);
@@ -466,6 +497,25 @@ int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
     case 8: return launch_tile<EPI, T64x48>(a, nstrips, st);
     default: return launch_tile<EPI, T64x96>(a, nstrips, st);
   }
+}
+template <int EPI>
+int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
+  if (((uintptr_t)a.x & 15) != 0 || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return launch_tile<EPI, T64, false>(a, nstrips, st);
+  const Split split = split_rows(a.B, nstrips, a.K, EPI == EPI_ROPE);
+  if (!split.rows) return launch_of<EPI>(fastest_tile(a.B, nstrips, a.K, EPI == EPI_ROPE), a, nstrips, st);
+  GemmArgs first = a, rest = a;
+  first.B = split.rows;
+  rest.B = a.B - split.rows;
+  rest.x += (size_t)split.rows * a.ldx;
+  rest.row0 += split.rows;
+  if (EPI != EPI_ROPE && EPI != EPI_PHI_IN) {  // (those find their rows from row0)
+    rest.out += (size_t)split.rows * a.ldo;
+    if (a.resid) rest.resid += (size_t)split.rows * a.ldr;
+    if (a.resid2) rest.resid2 += (size_t)split.rows * a.ldr2;
+    if (a.ids) rest.ids += split.rows;
+  }
+  const int rc = launch_of<EPI>(split.tile, first, nstrips, st);
+  return rc ? rc : launch_of<EPI>(fastest_tile(rest.B, nstrips, a.K, EPI == EPI_ROPE), rest, nstrips, st);
 }
 
 float least_time(int rows, int strips, int K) {
