@@ -16,7 +16,7 @@
 // The running max / sum / rescale are the usual online softmax; probabilities are rounded to bf16 for the second product,
 // sums are kept in fp32, positions are added in their order whatever the shape of the workgroup.
 //
-// Three kernels: one wave per 16 or 32 queries where there are many (attn_prefill_kernel), four waves per 16 where there are
+// Four kernels: one wave per 16 or 32 queries where there are many (attn_flow_kernel, attn_prefill_kernel), four waves per 16 where there are
 // few and the walk over the positions is a chain (attn_team_kernel), and for few queries behind a long context - with room for partial
 // results from the caller - the positions in chunks, each a workgroup's (attn_chunk_kernel).
 //
@@ -134,6 +134,23 @@ struct KvTile {
       }
     }
   }
+  // one half of a tile, its keys or its values, whose first load of a full tile is at `off`
+  template <int NW, bool KEYS>
+  __device__ __forceinline__ void issue_half(int t, uint32_t at, int wave, uint32_t off) const {
+    constexpr int N = KT / RPL / NW, STEP = NW * RPL;  // a wave's loads, positions between them: whole periods of the permutation
+    static_assert(STEP % PIECES == 0, "");
+    const char* from = (KEYS ? kb : vb) + (size_t)(t * KT) * rowb;
+    if (t * KT + KT <= len) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) load_lds16(at + (wave + i * NW) * 1024, from + (size_t)(i * STEP) * rowb, off);
+    } else {
+      int rows = len - t * KT;
+      asm volatile("" : "+s"(rows));  // (else every tile works these out, for the last one)
+      const Offsets<NW> o = offsets<NW>(rows, wave);
+#pragma unroll
+      for (int i = 0; i < N; ++i) load_lds16(at + (wave + i * NW) * 1024, from, KEYS ? o.k[i] : o.v[i]);
+    }
+  }
   // keys of positions 16 kb + (lane & 15), columns 32 j + 8 (lane >> 4) .. + 7
   __device__ __forceinline__ uint4 keys(uint32_t slot, int kb_, int j) const {
     const int m = lane & 15, g = lane >> 4;
@@ -155,53 +172,60 @@ __device__ __forceinline__ void tile_barrier() {  // this wave's older loads hav
   __builtin_amdgcn_s_barrier();
 }
 
-// Online softmax over a tile, per query (= per lane column): s -> the B operand of the second product, and what the
-// accumulators so far are multiplied with.
-__device__ __forceinline__ float softmax_tile(f32x4 (&s)[NKB], uint4 (&pf)[NWIN], float& m_run, float& l_run, int t0, int first, int qpos,
-                                              int g, float scale_log2e) {
-  float tmax = -INFINITY;
-  float mul = 1.0f;  // what the stored scores still have to be multiplied with
-  if (t0 + KT - 1 > first) {  // (wave-uniform) the tile reaches past the wave's first query: mask
-#pragma unroll
-    for (int kk = 0; kk < NKB; ++kk)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v = s[kk][i] * scale_log2e;
-        if (t0 + kk * 16 + 4 * g + i > qpos) v = -INFINITY;
-        s[kk][i] = v;
-        tmax = fmaxf(tmax, v);
-      }
-  } else {
-#pragma unroll
-    for (int kk = 0; kk < NKB; ++kk)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, s[kk][i]);
-    tmax *= scale_log2e;  // the scale is positive: the maximum of the products is the product of the maximum
-    mul = scale_log2e;    // and the scaling itself rides in the fused multiply-add of the exponent below
-  }
+// Online softmax over a tile, per query (= per lane column).  The running maximum is kept as an integer (log2 units): every rescale
+// is then an exact power of two and the bf16 weights do not depend on which tile raised it (common.h: softmax bookkeeping).
+struct Shift {
+  float off, corr;  // a weight's exponent is score * mul - off; what the sums so far are multiplied with
+};
+__device__ __forceinline__ Shift softmax_shift(float tmax, float& m_run) {  // tmax: this lane's
   tmax = lane_xor_max<32>(lane_xor_max<16>(tmax));
-  // the running maximum is kept as an integer (log2 units): every rescale is then an exact power of
-  // two and the bf16 weights do not depend on which tile raised it (common.h: softmax bookkeeping)
   const float mn = fmaxf(m_run, ceilf(tmax));
   const float corr = pow2_neg_int(m_run - mn);
   m_run = mn;
-  const float off = mn == -INFINITY ? 0.f : mn;  // (a chunk may begin behind the last position of a query: all its weights are zeros)
+  return {mn == -INFINITY ? 0.f : mn, corr};  // (a chunk may begin behind the last position of a query: all its weights are zeros)
+}
+__device__ __forceinline__ void softmax_mask(f32x4 (&s)[NKB], int t0, int qpos, int g, float scale_log2e) {
+#pragma unroll
+  for (int kk = 0; kk < NKB; ++kk)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float v = s[kk][i] * scale_log2e;
+      s[kk][i] = t0 + kk * 16 + 4 * g + i > qpos ? -INFINITY : v;
+    }
+}
+__device__ __forceinline__ void softmax_weights(const f32x4 (&s)[NKB], float mul, const Shift& x, uint4 (&pf)[NWIN], float& l_run) {
   float ts = 0.f;
   float p[NKB][4];
 #pragma unroll
   for (int kk = 0; kk < NKB; ++kk)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[kk][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kk][i], mul, -off));
+      p[kk][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kk][i], mul, -x.off));
       ts += p[kk][i];
     }
-  l_run = l_run * corr + ts;  // this lane's share; lanes g = 0..3 are added at the end
+  l_run = l_run * x.corr + ts;  // this lane's share; lanes g = 0..3 are added at the end
   // k-slot 8 g + i of window w  <->  position 32 w + 4 g + i (i < 4), 32 w + 16 + 4 g + i - 4
 #pragma unroll
   for (int w = 0; w < NWIN; ++w)
     pf[w] = make_uint4(pack_bf(p[2 * w][0], p[2 * w][1]), pack_bf(p[2 * w][2], p[2 * w][3]),
                        pack_bf(p[2 * w + 1][0], p[2 * w + 1][1]), pack_bf(p[2 * w + 1][2], p[2 * w + 1][3]));
-  return corr;
+}
+// s -> the B operand of the second product; the result multiplies the accumulators
+__device__ __forceinline__ float softmax_tile(f32x4 (&s)[NKB], uint4 (&pf)[NWIN], float& m_run, float& l_run, int t0, int first, int qpos,
+                                              int g, float scale_log2e) {
+  float mul = scale_log2e;        // what the stored scores still have to be multiplied with: in the exponent's fused multiply-add
+  if (t0 + KT - 1 > first) {      // (wave-uniform) the tile reaches past the wave's first query
+    softmax_mask(s, t0, qpos, g, scale_log2e);
+    mul = 1.0f;
+  }
+  float tmax = -INFINITY;
+#pragma unroll
+  for (int kk = 0; kk < NKB; ++kk)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, s[kk][i]);
+  const Shift x = softmax_shift(tmax * mul, m_run);  // the scale is positive: the maximum of the products is the product of the maximum
+  softmax_weights(s, mul, x, pf, l_run);
+  return x.corr;
 }
 
 // Queries wq0 + 16 qb + (lane & 15): lane g holds columns 32 j + 8 g .. + 7
@@ -292,7 +316,9 @@ __device__ __forceinline__ void store_few(const f32x4 (&o)[N], float l, const Pr
   if (odd) walk_rows<D>(a, sq, h, q0, odd, 16 * d0, 16 * N, lane);
 }
 
-// Four waves of 16 QW queries, one tile ahead.
+// Four waves of 16 QW queries, one tile ahead, scores, softmax and values one after the other.  With heads of 128 a wave that adds values goes
+// before the other of its SIMD, which keeps the two apart: 32 queries a wave, us without / with: 4001 x 32 heads (8 KV heads) 189 / 180, 4 x 2048
+// x 16 (4) 100.5 / 93, 16 x 700 x 16 (4) 74.1 / 71.6 (heads of 64: no difference).
 template <int D, int QW, bool ALIGNED, bool FEW>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
   constexpr int NW = 4, QB = 16 * QW * NW;
@@ -365,6 +391,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
             for (int i = 0; i < 4; ++i) o[qb][db][i] *= corr;
         }
       }
+      if (D == 128) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int w = 0; w < NWIN; ++w) {
         uint4 vf[ND];  // all read before the first product, as above
@@ -377,12 +404,158 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
           for (int qb = 0; qb < QW; ++qb) o[qb][db] = mfma16(vf[db], pf[qb][w], o[qb][db]);
         __builtin_amdgcn_sched_barrier(0);
       }
+      if (D == 128) __builtin_amdgcn_s_setprio(0);
     }
     cur = next;
   }
   if constexpr (FEW) return store_few<D>(o[0], l_run[0], a, sq, h, wq0, lane, 0);
 #pragma unroll
   for (int qb = 0; qb < QW; ++qb) store_rows<D>(o[qb], l_run[qb], a, sq, h, wq0 + qb * 16 + m, g, 0);
+}
+
+// Four waves of 16 queries.  While tile t + 1 is scored the weights of tile t are made, and while the values of t are added the maxima of t + 1
+// are found: in one wave the products and the softmax keep both units busy, where one after the other (the kernel above) they leave each
+// idle in turn and only another wave fills in.  All of a round's fragments are read before its first product; in the second half, which
+// is mostly products, a wave goes before the other of its SIMD, so that the two fall into different halves (4001 x 16 heads, 4 KV
+// heads, of 128: 93.2 us without, 91.5 with).  us, one after the other / this: 1024 x 16 25.8 / 21.9, 2048 x 6 45.7 / 36.0, 2048 x 16
+// 48.6 / 40.3, 3001 x 16 71.7 / 58.4, 4001 x 16 103.9 / 91.5, 32 x 300 x 6 behind 1500 115 / 92; heads of 64, 4001 x 16 68.8 / 55.7.
+// 238 VGPRs: 32 queries a wave do not fit (with fragments in parts of two they spill ten: 2048 x 6 55.6).
+template <int D>
+__global__ __launch_bounds__(256, 2) void attn_flow_kernel(PrefillArgs a) {
+  constexpr int NW = 4, QB = 16 * NW, NK = D / 32, ND = D / 16;
+  typedef KvTile<D> Tl;
+  constexpr int BY = Tl::BYTES, LOADS = KT / Tl::RPL / NW;
+  extern __shared__ __align__(16) unsigned char smem[];
+  int head, qblk;
+  my_block(a, head, qblk);
+  const int b = head / a.H, h = head - b * a.H;
+  if (b >= a.B) return;
+  const Sequence sq = sequence(a, b);
+  if (qblk * QB >= sq.S) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  const int q0 = qblk * QB, wq0 = q0 + wave * 16;
+  const Tl tile(a, sq, h / (a.H / a.Hkv), lane);
+  const typename Tl::template Offsets<NW> offs = tile.template offsets<NW>(KT, wave);
+  const uint32_t koff = offs.k[0], voff = offs.v[0];
+  const int ntiles = (min(a.pos + q0 + QB, tile.len) + KT - 1) / KT;   // tiles any query of the workgroup sees
+  const int wave_last = min(a.pos + wq0 + 15, tile.len - 1);           // last position any query of the wave sees
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;  // keys of even and of odd tiles, then their values
+
+  uint4 qf[NK];
+  int qpos;
+  load_queries<D>(qf, qpos, a, sq, h, wq0 + m, g);
+  f32x4 o[ND];
+#pragma unroll
+  for (int db = 0; db < ND; ++db) o[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  tile.template issue_half<NW, true>(0, lds0, wave, koff);
+  tile.template issue_half<NW, false>(0, lds0 + 2 * BY, wave, voff);
+  if (1 < ntiles) tile.template issue_half<NW, true>(1, lds0 + BY, wave, koff);
+
+  // where this lane's fragments lie (KvTile::keys and ::values): the permutations are an exclusive or
+  const uint32_t kp = m * Tl::ROWB + (uint32_t)(g ^ (m & (Tl::PIECES - 1))) * 16;
+  const int vr = 4 * g + (m >> 2);
+  const uint32_t vp = vr * Tl::ROWB + (m & 3) * 8 + (uint32_t)(vr & (Tl::PIECES / 2 - 1)) * 32;
+  auto read_keys = [&](uint4 (&kf)[NK][NKB], uint32_t at) {
+#pragma unroll
+    for (int j = 0; j < NK; ++j)
+#pragma unroll
+      for (int kk = 0; kk < NKB; ++kk) kf[j][kk] = lds16_at((kp ^ (j * 64)) + (at + kk * (16 * Tl::ROWB)));
+  };
+  auto read_values = [&](uint4 (&vf)[NWIN][ND], uint32_t at) {
+#pragma unroll
+    for (int w = 0; w < NWIN; ++w)
+#pragma unroll
+      for (int db = 0; db < ND; ++db) {
+        const uint32_t p = vp ^ (db * 32), from = at + w * (32 * Tl::ROWB);
+        const uint2 lo = lds_tr8(p + from), hi = lds_tr8(p + (from + 16 * Tl::ROWB));
+        vf[w][db] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+      }
+  };
+  auto score = [&](f32x4 (&r)[NKB], const uint4 (&kf)[NK][NKB]) {
+#pragma unroll
+    for (int j = 0; j < NK; ++j)
+#pragma unroll
+      for (int kk = 0; kk < NKB; ++kk) r[kk] = mfma16(kf[j][kk], qf[j], j ? r[kk] : (f32x4){0.f, 0.f, 0.f, 0.f});
+  };
+  f32x4 s[NKB];  // tile t's scores, what they have to be multiplied with, and their maximum's shift
+  float mul;
+  Shift x;
+  auto shift = [&] {
+    float top = -INFINITY;
+#pragma unroll
+    for (int kk = 0; kk < NKB; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) top = fmaxf(top, s[kk][i]);
+    x = softmax_shift(top * mul, m_run);
+  };
+  auto add = [&](const uint4 (&vf)[NWIN][ND], const uint4 (&pf)[NWIN]) {
+#pragma unroll
+    for (int w = 0; w < NWIN; ++w)
+#pragma unroll
+      for (int db = 0; db < ND; ++db) o[db] = mfma16(vf[w][db], pf[w], o[db]);
+  };
+
+  if (1 < ntiles) tile_barrier<true, 2 * LOADS>();
+  else tile_barrier<true, LOADS>();
+  {
+    uint4 kf[NK][NKB];
+    read_keys(kf, lds0);
+    score(s, kf);
+    const bool masked = KT - 1 > a.pos + wq0;
+    if (masked) softmax_mask(s, 0, qpos, g, a.scale_log2e);
+    mul = masked ? 1.0f : a.scale_log2e;
+    shift();
+  }
+  auto round = [&](int t, auto parity) {
+    constexpr int P = decltype(parity)::value;
+    tile_barrier<true, 0>();  // the next keys and these values are there, and everyone is done with those before
+    if (t + 2 < ntiles) tile.template issue_half<NW, true>(t + 2, lds0 + P * BY, wave, koff);
+    if (t + 1 < ntiles) tile.template issue_half<NW, false>(t + 1, lds0 + (3 - P) * BY, wave, voff);
+    const int t1 = (t + 1) * KT;
+    uint4 vf[NWIN][ND], pf[NWIN];
+    auto flow = [&](auto masked) {  // masked: not every query of the wave sees the whole of tile t + 1
+      uint4 kf[NK][NKB];
+      f32x4 sn[NKB];
+      read_keys(kf, lds0 + (1 - P) * BY);
+      read_values(vf, lds0 + (2 + P) * BY);
+      __builtin_amdgcn_sched_barrier(0);
+      score(sn, kf);
+      softmax_weights(s, mul, x, pf, l_run);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kk = 0; kk < NKB; ++kk) s[kk] = sn[kk];
+      mul = decltype(masked)::value ? 1.0f : a.scale_log2e;
+      if (decltype(masked)::value) softmax_mask(s, t1, qpos, g, a.scale_log2e);
+      __builtin_amdgcn_s_setprio(1);
+      __builtin_amdgcn_sched_barrier(0);
+      add(vf, pf);
+      shift();
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(0);
+      if (__any(x.corr != 1.0f)) {  // most tiles leave the running maximum of every query of the wave alone
+#pragma unroll
+        for (int db = 0; db < ND; ++db)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[db][i] *= x.corr;
+      }
+    };
+    if (t1 + KT - 1 <= a.pos + wq0) {  // (wave-uniform)
+      flow(std::false_type());
+    } else if (t1 <= wave_last) {
+      flow(std::true_type());
+    } else if (t * KT <= wave_last) {  // the wave's last tile
+      read_values(vf, lds0 + (2 + P) * BY);
+      softmax_weights(s, mul, x, pf, l_run);
+      add(vf, pf);
+    }
+  };
+  for (int t = 0; t < ntiles; t += 2) {
+    round(t, std::integral_constant<int, 0>());
+    if (t + 1 < ntiles) round(t + 1, std::integral_constant<int, 1>());
+  }
+  store_rows<D>(o, l_run, a, sq, h, wq0 + m, g, 0);
 }
 
 // TEAMS teams of four waves, 16 queries each.  Wave w scores positions 16 w .. + 15 of every tile and owns a quarter of the output
@@ -663,6 +836,15 @@ int launch_waves(PrefillArgs a, hipStream_t st) {
   return ohara_launch_status();
 }
 
+template <int D>
+int launch_flow(PrefillArgs a, hipStream_t st) {
+  a.nqb = (a.S + 63) / 64;
+  const int64_t blocks = a.nqb * (a.seqs ? ((int64_t)a.H * a.B + 7) / 8 * 8 : (int64_t)a.H * a.B);
+  if (blocks > INT32_MAX) return OHARA_ESIZE;
+  hipLaunchKernelGGL((attn_flow_kernel<D>), dim3((unsigned)blocks), dim3(256), 2 * KvTile<D>::SLOT, st, a);
+  return ohara_launch_status();
+}
+
 template <int D, int TEAMS, bool FEW = false, int NST = 3>
 int launch_teams(PrefillArgs a, hipStream_t st) {
   constexpr int LDS = NST * KvTile<D>::SLOT + 2 * TEAMS * 4096;
@@ -673,7 +855,9 @@ int launch_teams(PrefillArgs a, hipStream_t st) {
   return ohara_launch_status();
 }
 
-// Both kernels give the same bits; us with teams of 16 / 32 queries a workgroup and waves of 16 / 32 (64 / 128 a workgroup):
+// All kernels of 16 queries a wave give the same bits, those of 32 where `pos` is a multiple of 32 (else a tile's scores are scaled before the
+// exponent for sixteen queries that need no mask); us with teams of 16 / 32 queries a workgroup and
+// attn_prefill_kernel's waves of 16 / 32 (64 / 128 a workgroup):
 //   heads of 128                                                 heads of 64, 16 heads
 //     128 queries x 6 heads   4.5 /  5.5 /  5.5 /  7.1             160 queries      4.3 /  5.0 /  4.6 /  5.8
 //     48 behind 1900, 4 x 16 24.7 / 27.8 / 34   / 49               500              7.6 /  8.5 /  8.4 / 11.7
@@ -687,12 +871,14 @@ int launch_teams(PrefillArgs a, hipStream_t st) {
 // so: teams of 16 while every one has a CU to itself, and over more than two tiles while every two have one (with heads of 128
 // as teams of 32).  A shorter walk does not pay for the teams' barriers: us, teams / waves: heads of 64, 8 x 24 queries x 32 heads
 // 5.2 / 4.8; heads of 128, 8 x 33 x 16 6.2 / 5.4; over four tiles, 200 x 32 7.1 / 7.5.
+// 64 queries a workgroup: attn_flow_kernel, but one after the other where there are two tiles at most, which leaves little to overlap
+// (12 x 100 x 16 9.4 / 9.8, 16 x 64 x 32 11.3 / 11.6; three tiles, 8 x 192 x 32 17.3 / 16.5).
 // 128 queries a workgroup read each position once where 64 read it twice, and are slower by a quarter where there are few of
-// them or the second half of the last one is empty (heads of 128, 32 x 300 x 6 behind 1500: 90 / 109 us, 64 / 128 queries).  So
-// from three a CU on, if at least half of their second halves hold queries; from fewer on where 64 queries need a second round:
-// with heads of 64 from the sixth workgroup of 64 queries a CU (28 x 112 x 24 behind 2000: 119 / 96; five: 20 x 128 x 32 behind 250
-// 18.7 / 20.6), with heads of 128 from the third, there if nearly every half holds queries and the walks are of about one length
-// (48 x 65 x 6 behind 1500: 77 / 62; but 4 x 1000 x 16 from the start: 33 / 35).
+// them or the second half of the last one is empty (heads of 128, 32 x 300 x 6 behind 1500: 92 / 126 us, 64 / 128 queries).  So
+// from three a CU on, if at least half of their second halves hold queries (2 x 4001 x 16 188 / 164, 16 x 500 x 12 39.5 / 35.5, 8 x 700
+// x 16 37.4 / 35.1, 16 x 1024 x 6 52.8 / 50.5; 8 x 2048 x 6 80.9 / 84.9; two a CU, 12 x 1024 x 6 41.8 / 44.7); with heads of 64 also from
+// the sixth workgroup of 64 queries a CU (28 x 112 x 24 behind 2000: 139 / 105; 4 x 2048 x 16 is both, 60.7 / 57.4; three, 3 x 2048 x 16 49.7 /
+// 54.0; 20 x 128 x 32 behind 250 27.6 / 27.7).
 // Before (one kernel, four waves, values through registers, the heads over all XCDs), for the table's lines: 5.8, 45, 16.5, 25,
 // 26, 167, 50, 46, 92; 5.2, 10.4, 12, 64.
 template <int D>
@@ -714,10 +900,8 @@ int launch_prefill_for(const PrefillArgs& a, const int32_t* lengths, hipStream_t
   if constexpr (D == 128)
     if (long_walk && blocks(32) <= CUS) return launch_teams<D, 2>(a, st);
   const int64_t wide = blocks(128), halves = blocks(64);
-  const bool even = 5 * halves >= 9 * wide && (a.S <= 128 || a.pos >= a.S);
-  const bool second_round = D == 64 ? halves > 5 * CUS : wide > CUS && even;
-  if ((wide >= 3 * CUS || second_round) && 2 * halves >= 3 * wide) return launch_waves<D, 2>(a, st);
-  return launch_waves<D, 1>(a, st);
+  if ((wide >= 3 * CUS || (D == 64 && halves > 5 * CUS)) && 2 * halves >= 3 * wide) return launch_waves<D, 2>(a, st);
+  return long_walk ? launch_flow<D>(a, st) : launch_waves<D, 1>(a, st);
 }
 
 }  // namespace
