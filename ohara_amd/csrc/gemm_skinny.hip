@@ -18,6 +18,7 @@
 #include <algorithm>
 
 #include "gemm_epilogue.h"
+#include "phi_attn.h"
 
 #include <type_traits>
 
@@ -73,13 +74,13 @@ __device__ __forceinline__ float sum8(uint4 v) {
 // NW waves per workgroup split K.  A workgroup keeps NW * CH KiB of weight loads in flight, so when
 // there are too few strips to put several workgroups on every CU (few output rows, long K) 16 waves
 // instead of 4 are what fills the memory pipeline.
-template <int BT, int NORM, int EPI, int NW = 4, int SP = 8>
-__global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
+template <int BT, int NORM, int EPI, int NW, int SP>
+__device__ __forceinline__ void skinny(const GemmArgs& a, int block) {
   // k-steps whose loads are issued back to back (the many-wave variants have no norm operands to hold)
   constexpr int CH = (NORM == 0 && NW > 4) ? 10 : (BT <= 2 ? 6 : 4);
   // workgroup id -> (strip, chunk of 16*BT rows).  Ids go round-robin over the 8 XCDs; the chunks of
   // one strip get ids 8 apart, so they run on the same XCD and share its L2 copy of the weights.
-  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int xcd = block & 7, local = block >> 3;
   const int strip = (local / a.ny) * 8 + xcd;
   const int rbase = (local % a.ny) * 16 * BT;
   if (strip >= a.nstrips) return;
@@ -285,6 +286,19 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
       else gemm_epilogue<EPI>(a, b, strip, g, acc[t]);
     }
   }
+}
+
+template <int BT, int NORM, int EPI, int NW = 4, int SP = 8>
+__global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
+  skinny<BT, NORM, EPI, NW, SP>(a, blockIdx.x);
+}
+
+// Phi's attention of single tokens beside the second product of its MLP, which does not wait for it: neither fills the chip - 352 teams of four waves,
+// whose chain of round trips bounds them, and 160 strips - and one after the other they took the sum of their times.  The attention's go first: its
+// chain is the longer one.  (Fewer of the product's loads in flight, 2 to 7 k-steps instead of 10, leave the times as they are.)
+__global__ __launch_bounds__(1024) void phi_attn_linear_kernel(PhiAttnArgs t, GemmArgs a, int fours) {
+  if ((int)blockIdx.x < fours) phi_attend<4, true>(t, blockIdx.x);
+  else skinny<1, 0, EPI_BIAS, 16, 8>(a, blockIdx.x - fours);
 }
 
 // Rows without a norm, K up to 6144: a wave's share of K is at most CH k-steps, all of them requested before anything waits.  Above, rounds
@@ -1038,6 +1052,35 @@ int ohara_linear_bias_add2_bf16(const uint16_t* x, int ldx, const uint16_t* wp, 
   else if (parts == 4) OHARA_MERGE(4);
   else OHARA_MERGE(8);
 #undef OHARA_MERGE
+  return ohara_launch_status();
+}
+
+int ohara_phi_attn_linear_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, const uint16_t* vcache, const float* cos, const float* sin, int rot,
+                               int batch, int h, int dh, int t_max, int pos, const int32_t* pos_dev, int n_split, void* workspace, uint16_t* out,
+                               const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, const uint16_t* bias, uint16_t* y, int ldy, void* stream) {
+  PhiAttnArgs t;
+  const int rc = phi_attn_args(t, q, ldq, kcache, vcache, cos, sin, rot, batch, 1, h, dh, t_max, pos, pos_dev, n_split, workspace, out);
+  if (rc) return rc;
+  if (!x || !wp || !bias || !y || n < 1 || k < 1 || (k & 7) || (ldx & 7) || ldx < k || (n & 3) || (ldy & 3) || ldy < n) return OHARA_EINVAL;
+  const int strips = (n + 15) / 16;
+  // One launch where the product's workgroups are sixteen waves by themselves; such a workgroup has a CU to itself, so all that attends has the
+  // CUs that the product leaves: at least eight chunks of them, and not behind a long context, where fewer chunks than asked for are longer walks
+  // (`pos`, also where pos_dev goes on from there).  us, two launches before / two now / this: 2560 x 10240, 32 heads of 80, one row behind 40 21.1 /
+  // 16.4 / 11.7, 200 21.9 / 20.5 / 15.5, 700 23.4 / 22.2 / 17.4, 1500 25.0 / 24.1 / 22.2, 2040 26.9 / 25.7 / 27.9; two rows (six chunks) behind 700
+  // 24.6 / 23.7 / 22.5, 1500 29.4 / 28.0 / 32.7.
+  const int chunks = strips < 256 ? (256 - (strips + 7) / 8 * 8) * 4 / std::max(batch * h, 1) : 0;
+  if (batch > 16 || k < 2048 || pos >= 1750 || !phi_eights(t) || chunks < std::min(n_split, 8)) {
+    const int ra = ohara_phi_attn_bf16(q, ldq, kcache, vcache, cos, sin, rot, batch, 1, h, dh, t_max, pos, pos_dev, n_split, workspace, out, stream);
+    return ra ? ra : ohara_linear_bias_bf16(x, ldx, wp, n, k, bias, batch, OHARA_LIN_BIAS, nullptr, 0, nullptr, 0, y, ldy, stream);
+  }
+  GemmArgs a{};
+  a.wp = reinterpret_cast<const uint4*>(wp);
+  a.x = x; a.ldx = ldx; a.B = batch; a.N = n; a.K = k;
+  a.out = y; a.ldo = ldy; a.bias = bias;
+  a.ny = 1; a.nstrips = strips;
+  t.ns = std::min(n_split, chunks);
+  const int fours = (batch * h * t.ns + 31) / 32 * 8;  // (whole eights: a strip's XCD is its workgroup's number)
+  hipLaunchKernelGGL(phi_attn_linear_kernel, dim3((unsigned)(fours + (strips + 7) / 8 * 8)), dim3(1024), 0, (hipStream_t)stream, t, a, fours);
   return ohara_launch_status();
 }
 

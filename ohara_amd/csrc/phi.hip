@@ -5,7 +5,7 @@
 //                                           phi.py:98-117, rotary.py:131-184
 // The projections with bias, new_gelu and the parallel-block sum are epilogues of the skinny
 // GEMM (gemm_epilogue.h).
-#include "common.h"
+#include "phi_attn.h"
 
 namespace {
 
@@ -69,277 +69,9 @@ __global__ void kv_append_kernel(const bf16_t* k, const bf16_t* v, int ld, int r
   *reinterpret_cast<uint4*>(vc + dst) = ldg16(v + (size_t)row * ld + c);
 }
 
-// ---- attention ---------------------------------------------------------------------------
-// One workgroup per (sequence, head, new token) and context chunk.  Sixteen lanes own one cached
-// position at a time (lane l the eight features 8l .. 8l+7) and fetch two positions per round before
-// using either (four measured slower: 178 registers halve the occupancy), so a workgroup walks 32
-// positions per round with an online softmax per 16-lane group;
-// the groups are merged through LDS at the end.  With several chunks (decode: few queries, long
-// context) every chunk leaves {weighted sum, max, sum} and the workgroup that finishes last combines
-// them in chunk order.
-//
-// The reference rotates every cached key again at each step (phi.py:104).  With the rotated query
-// qr and c, s the cosine / sine of key position t the score is
-//   sum_i (k1_i c_i - k2_i s_i) qr1_i + (k1_i s_i + k2_i c_i) qr2_i + sum_rest k_j q_j
-//     = sum_i k1_i (c_i qr1_i + s_i qr2_i) + k2_i (c_i qr2_i - s_i qr1_i) + sum_rest k_j q_j,
-// i.e. a dot product of the raw key row with a per-position weight vector built from two per-lane
-// constants A, B: w_j = c A_j + s B_j.  All of it in fp32, as the reference (phi.py:98-100).
-struct PhiAttnArgs {
-  const bf16_t* q;
-  int ldq;
-  const bf16_t* kc;
-  const bf16_t* vc;
-  const float* cos;  // (t_max, rot/2) fp32
-  const float* sin;
-  bf16_t* out;       // (rows, H*D)
-  int S, H, D, rot, t_max, pos;
-  const int32_t* pos_dev;
-  int ns;         // context chunks (decode): chunk c of a (sequence, head) is blockIdx.y
-  float* ws;      // ns > 1: per (row, head, chunk) D + 2 floats {weighted sum[D], max, sum}
-  int* counters;  // ns > 1: per (row, head) chunks finished; zero between calls
-};
-
-#ifndef PHI_ATTN_R
-#define PHI_ATTN_R 2
-#endif
-__global__ __launch_bounds__(256) void phi_attn_kernel(PhiAttnArgs a) {
-  __shared__ float qr[128];
-  __shared__ float gm[16], gl[16];
-  __shared__ float gacc[16][128];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int grp = wave * 4 + (lane >> 4), l = lane & 15;
-  const int D = a.D, half = a.rot >> 1;
-  // The cache is position-major: the heads of one position lie side by side, 2 * D bytes each, so the rows of
-  // neighbouring heads share 128-byte lines.  Workgroups are handed to the eight XCDs in turn, each with an L2 of
-  // its own: taken as launched, neighbouring heads would land on different XCDs and every L2 would fetch the
-  // shared lines again.  So the launch order is re-read: XCD x works through the x-th eighth of the (chunk,
-  // sequence, head) list, heads fastest.  (Any bijection is correct; this one needs a workgroup count that is a
-  // multiple of 8, otherwise the order stays as launched.)
-  int bx = blockIdx.x, by = blockIdx.y;
-  {
-    const int n = gridDim.x * gridDim.y;
-    if ((n & 7) == 0) {
-      const int id = by * gridDim.x + bx;
-      const int lid = (id & 7) * (n >> 3) + (id >> 3);
-      bx = lid % gridDim.x;
-      by = lid / gridDim.x;
-    }
-  }
-  int w = bx;
-  const int s = w % a.S; w /= a.S;
-  const int h = w % a.H;
-  const int seq = w / a.H;
-  const int row = seq * a.S + s;
-  const int pq = (a.pos_dev ? *a.pos_dev : a.pos) + s;  // position of this query; keys 0 .. pq are visible
-  if (pq < 0 || pq >= a.t_max) return;
-
-  if (tid < D) {
-    const bf16_t* qrow = a.q + (size_t)row * a.ldq + h * D;
-    float v = bf2f(qrow[tid]);
-    if (tid < half) {
-      const float c = a.cos[(size_t)pq * half + tid], sn = a.sin[(size_t)pq * half + tid];
-      v = v * c - bf2f(qrow[tid + half]) * sn;
-    } else if (tid < a.rot) {
-      const int i = tid - half;
-      const float c = a.cos[(size_t)pq * half + i], sn = a.sin[(size_t)pq * half + i];
-      v = bf2f(qrow[i]) * sn + v * c;
-    }
-    qr[tid] = v;
-  }
-  __syncthreads();
-
-  const int e0 = 8 * l;
-  const bool own = e0 < D;
-  float A[8], Bc[8];
-  int f[8];
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const int j = e0 + u;
-    A[u] = own ? qr[j] : 0.f;
-    Bc[u] = 0.f;
-    f[u] = -1;
-    if (own && j < half) {
-      Bc[u] = qr[j + half];
-      f[u] = j;
-    } else if (own && j < a.rot) {
-      Bc[u] = -qr[j - half];
-      f[u] = j - half;
-    }
-  }
-  const bool rotates = own && e0 < a.rot;
-  const bool vec8 = (half & 7) == 0;  // then rot % 16 == 0 and a lane's features are all rotated or all not
-  const uint4 one4 = make_uint4(0x3f800000u, 0x3f800000u, 0x3f800000u, 0x3f800000u), zero4 = make_uint4(0, 0, 0, 0);
-  const float scale = sqrtf(1.0f / (float)D);
-
-  float m = -INFINITY, lsum = 0.f, acc[8];
-#pragma unroll
-  for (int u = 0; u < 8; ++u) acc[u] = 0.f;
-  const size_t hd = (size_t)a.H * D;
-  // Lanes beyond the head (own == false) read the head's first features instead: their weights A / Bc are
-  // zero, so what they read only has to be mapped memory.
-  const int e0c = own ? e0 : 0;
-  const bf16_t* kb = a.kc + (size_t)seq * a.t_max * hd + (size_t)h * D + e0c;
-  const bf16_t* vb = a.vc + (size_t)seq * a.t_max * hd + (size_t)h * D + e0c;
-  // this workgroup's positions [t_lo, t_hi]
-  int t_lo = 0, t_hi = pq;
-  if (a.ns > 1) {
-    const int per = ((pq + a.ns) / a.ns + 15) & ~15;  // ceil((pq + 1) / ns) rounded up to whole rounds
-    t_lo = by * per;
-    t_hi = min(pq, t_lo + per - 1);
-  }
-  constexpr int R = PHI_ATTN_R;  // positions a lane group has in flight per round
-  const int fc = rotates ? f[0] : 0;
-  for (int t = t_lo + grp; t <= t_hi; t += 16 * R) {
-    // every load of the round is issued whatever its position (clamped to the chunk's last one): one run
-    // of loads without branches; a position past the end is skipped when the round is consumed
-    uint4 kv[R], vv[R];
-    float cs[R][8], sn[R][8];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int tt = min(t + 16 * r, t_hi);
-      kv[r] = ldg16(kb + (size_t)tt * hd);
-      vv[r] = ldg16(vb + (size_t)tt * hd);
-      if (vec8) {
-        // the lane's eight features lie in one half: their angles are eight adjacent table entries
-        const float* cp = a.cos + (size_t)tt * half + fc;
-        const float* sp = a.sin + (size_t)tt * half + fc;
-        const uint4 c0 = ldg16(cp), c1 = ldg16(cp + 4), s0 = ldg16(sp), s1 = ldg16(sp + 4);
-        const uint32_t cu[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-        const uint32_t su[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          cs[r][u] = __uint_as_float(cu[u]);
-          sn[r][u] = __uint_as_float(su[u]);
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const bool rot_u = rotates && f[u] >= 0;
-          cs[r][u] = rot_u ? a.cos[(size_t)tt * half + f[u]] : 1.0f;
-          sn[r][u] = rot_u ? a.sin[(size_t)tt * half + f[u]] : 0.0f;
-        }
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if (t + 16 * r > t_hi) break;  // uniform within the 16-lane group
-      const uint32_t ku[4] = {kv[r].x, kv[r].y, kv[r].z, kv[r].w};
-      float part = 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float c0 = (vec8 && !rotates) ? 1.0f : cs[r][2 * i], s0 = (vec8 && !rotates) ? 0.0f : sn[r][2 * i];
-        const float c1 = (vec8 && !rotates) ? 1.0f : cs[r][2 * i + 1], s1 = (vec8 && !rotates) ? 0.0f : sn[r][2 * i + 1];
-        part += lo_bf(ku[i]) * (c0 * A[2 * i] + s0 * Bc[2 * i]);
-        part += hi_bf(ku[i]) * (c1 * A[2 * i + 1] + s1 * Bc[2 * i + 1]);
-      }
-      part = lane_xor_sum<8>(lane_xor_sum<4>(lane_xor_sum<2>(lane_xor_sum<1>(part))));
-      const float sc = part * scale;
-      const float mn = fmaxf(m, sc);
-      // hardware exponential: its error (about 1e-6 relative) is far below the bf16 rounding of the output
-      const float corr = __expf(m - mn), p = __expf(sc - mn);  // m = -inf on the first round: corr = 0
-      lsum = lsum * corr + p;
-      const uint32_t vu[4] = {vv[r].x, vv[r].y, vv[r].z, vv[r].w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        acc[2 * i] = acc[2 * i] * corr + p * lo_bf(vu[i]);
-        acc[2 * i + 1] = acc[2 * i + 1] * corr + p * hi_bf(vu[i]);
-      }
-      m = mn;
-    }
-  }
-  if (l == 0) {
-    gm[grp] = m;
-    gl[grp] = lsum;
-  }
-  if (own) {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) gacc[grp][e0 + u] = acc[u];
-  }
-  __syncthreads();
-  if (tid < D) {
-    float M = -INFINITY, gv[16];
-#pragma unroll
-    for (int g = 0; g < 16; ++g) gv[g] = gacc[g][tid];
-#pragma unroll
-    for (int g = 0; g < 16; ++g) M = fmaxf(M, gm[g]);
-    float num = 0.f, den = 0.f;
-#pragma unroll
-    for (int g = 0; g < 16; ++g) {  // (no branch: every read would be waited for behind it; with the merge's below, whose values are asked for
-                                    // with the maxima: 32 heads of 80 behind 700 13.1 -> 11.2 us)
-      const bool in = gm[g] != -INFINITY;  // (not a group that saw no position, nor one whose scores are all -inf, which holds NaN)
-      const float wg = expf(gm[g] - M);
-      num += in ? wg * gv[g] : 0.f;
-      den += in ? wg * gl[g] : 0.f;
-    }
-    if (a.ns > 1) {
-      // write-through stores: the workgroup that merges may sit on another XCD
-      float* o = a.ws + (((size_t)row * a.H + h) * a.ns + by) * (D + 2);
-      st_coh4(o + tid, __float_as_uint(num));
-      if (tid == 0) {
-        st_coh4(o + D, __float_as_uint(M));  // -inf: this chunk lies beyond the query's position
-        st_coh4(o + D + 1, __float_as_uint(den));
-      }
-    } else {
-      a.out[(size_t)row * hd + (size_t)h * D + tid] = f2bf(num / den);
-    }
-  }
-  if (a.ns == 1) return;
-
-  // The workgroup that finishes last merges the chunks of its (row, head), in chunk order.  Every
-  // wave waits for its own write-through stores before the workgroup barrier; the counter is a
-  // relaxed device-scope atomic; the merge reads with cache-bypassing loads.
-  __shared__ int is_last;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  wait_own_stores();
-  __syncthreads();
-  int* counter = a.counters + (size_t)row * a.H + h;
-  if (tid == 0) {
-    const int old = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    is_last = old == a.ns - 1;
-    if (is_last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next call
-  }
-  __syncthreads();
-  if (!is_last) return;
-  const float* p = a.ws + ((size_t)row * a.H + h) * a.ns * (D + 2);
-  // ns <= 64: one round of loads for all (max, sum) pairs and the first sixteen chunks' values
-  float av[16];
-  if (tid < D) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) av[i] = __uint_as_float(ld_coh4(p + (size_t)min(i, a.ns - 1) * (D + 2) + tid));
-  }
-  if (tid < a.ns) {
-    // qr and gacc are free again: chunk maxima and sums go there
-    qr[tid] = __uint_as_float(ld_coh4(p + (size_t)tid * (D + 2) + D));
-    gacc[0][tid] = __uint_as_float(ld_coh4(p + (size_t)tid * (D + 2) + D + 1));
-  }
-  __syncthreads();
-  if (tid < D) {
-    float M = -INFINITY;
-    for (int c = 0; c < a.ns; ++c) M = fmaxf(M, qr[c]);
-    float num = 0.f, den = 0.f;
-    for (int c0 = 0; c0 < a.ns; c0 += 16) {  // sixteen chunks' values in flight, every load unconditional
-      if (c0) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) av[i] = __uint_as_float(ld_coh4(p + (size_t)min(c0 + i, a.ns - 1) * (D + 2) + tid));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      float mc[16], lc[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        mc[i] = qr[min(c0 + i, a.ns - 1)];
-        lc[i] = gacc[0][min(c0 + i, a.ns - 1)];
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const bool in = c0 + i < a.ns && mc[i] != -INFINITY;
-        const float wg = expf(mc[i] - M);
-        num += in ? wg * av[i] : 0.f;
-        den += in ? wg * lc[i] : 0.f;
-      }
-    }
-    a.out[(size_t)row * hd + (size_t)h * D + tid] = f2bf(num / den);
-  }
+template <bool EIGHTS>
+__global__ __launch_bounds__(256, 4) void phi_attn_kernel(PhiAttnArgs a) {
+  phi_attend<1, EIGHTS>(a, blockIdx.x);
 }
 
 // ---- attention over many new tokens (prefill) -----------------------------------------------
@@ -604,9 +336,7 @@ int launch_phi_prefill(const PhiAttnArgs& a, int batch, hipStream_t st) {
   constexpr int LDS = 2 * 2 * PF_T * (16 * DT + 4) * (int)sizeof(float);
   const int64_t nqb = (a.S + PF_Q - 1) / PF_Q, heads = (int64_t)a.H * batch, grid = nqb * ((heads + 7) / 8 * 8);
   if (grid > INT32_MAX) return OHARA_ESIZE;
-  // angles are read four floats at a time, on 16 bytes
-  const bool vec = ((a.rot >> 1) & 7) == 0 && (((uintptr_t)a.cos | (uintptr_t)a.sin) & 15) == 0;
-  auto kernel = vec ? phi_attn_prefill_kernel<DT, true> : phi_attn_prefill_kernel<DT, false>;
+  auto kernel = phi_eights(a) ? phi_attn_prefill_kernel<DT, true> : phi_attn_prefill_kernel<DT, false>;
   if (LDS > 64 * 1024) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), LDS, st, a, (int)nqb, (int)heads);
   return ohara_launch_status();
@@ -648,19 +378,9 @@ int64_t ohara_phi_attn_workspace_bytes(int batch, int h, int dh, int n_split) {
 int ohara_phi_attn_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, const uint16_t* vcache, const float* cos,
                         const float* sin, int rot, int batch, int seq_len, int h, int dh, int t_max, int pos,
                         const int32_t* pos_dev, int n_split, void* workspace, uint16_t* out, void* stream) {
-  if (!q || !kcache || !vcache || !cos || !sin || !out) return OHARA_EINVAL;
-  if (batch < 1 || seq_len < 1 || h < 1 || t_max < 1) return OHARA_EINVAL;
-  if (dh < 8 || dh > 128 || (dh & 7)) return OHARA_ESIZE;
-  if (rot < 2 || (rot & 1) || rot > dh) return OHARA_EINVAL;  // rotary.py:118-121
-  if (ldq < h * dh) return OHARA_EINVAL;
-  if (!pos_dev && (pos < 0 || pos + seq_len > t_max)) return OHARA_EINVAL;
-  if (pos_dev && seq_len != 1) return OHARA_EINVAL;
-  if (n_split < 1 || n_split > 64 || (n_split > 1 && (!workspace || seq_len != 1))) return OHARA_EINVAL;
-  const int64_t grid = (int64_t)batch * seq_len * h;
-  if (grid > INT32_MAX) return OHARA_ESIZE;
-  const size_t counters = (((size_t)batch * h * sizeof(int)) + 255) & ~(size_t)255;
-  PhiAttnArgs a{q, ldq, kcache, vcache, cos, sin, out, seq_len, h, dh, rot, t_max, pos, pos_dev, n_split,
-                reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + counters), reinterpret_cast<int*>(workspace)};
+  PhiAttnArgs a;
+  const int rc = phi_attn_args(a, q, ldq, kcache, vcache, cos, sin, rot, batch, seq_len, h, dh, t_max, pos, pos_dev, n_split, workspace, out);
+  if (rc) return rc;
   if (seq_len >= 16 && !pos_dev && (dh == 16 || dh == 32 || dh == 64 || dh == 80 || dh == 128) && h <= 65535 &&
       batch <= 65535) {
     // many new tokens: queries in tiles of 64 against key / value tiles in LDS, fp32 matrix products
@@ -672,7 +392,7 @@ int ohara_phi_attn_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, cons
       default: return launch_phi_prefill<8>(a, batch, (hipStream_t)stream);
     }
   }
-  hipLaunchKernelGGL(phi_attn_kernel, dim3((unsigned)grid, (unsigned)n_split), dim3(256), 0, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(phi_eights(a) ? phi_attn_kernel<true> : phi_attn_kernel<false>, dim3((unsigned)(batch * seq_len * h * n_split)), dim3(256), 0, (hipStream_t)stream, a);
   return ohara_launch_status();
 }
 

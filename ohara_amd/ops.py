@@ -696,6 +696,28 @@ def phi_attn(q, kcache, vcache, cos, sin, rot, batch, seq_len, h, dh, pos, pos_d
     return out
 
 
+def phi_attn_linear(q, kcache, vcache, cos, sin, rot, batch, h, dh, pos, x, w: PackedLinear, bias, pos_dev=None, out=None, y=None, n_split=1,
+                    workspace=None):
+    """``phi_attn`` of one token a sequence and, beside it in the same launch, ``linear_bias(x, w, bias)`` -> (out, y)."""
+    if q.stride(1) != 1:
+        raise ValueError("q must have unit column stride")
+    if cos.dtype != torch.float32 or sin.dtype != torch.float32:
+        raise ValueError("cos / sin must be fp32")
+    if x.dtype != BF16 or not x.is_cuda or x.stride(1) != 1:
+        raise ValueError("x must be a bf16 device matrix with unit column stride")
+    _need(bias, BF16, "bias")
+    if x.shape != (batch, w.k) or bias.numel() != w.n:
+        raise ValueError(f"x is {tuple(x.shape)} / bias {bias.numel()} entries, weight is {w.n} x {w.k}")
+    if out is None:
+        out = torch.empty(batch, h * dh, dtype=BF16, device=q.device)
+    if y is None:
+        y = torch.empty(batch, w.n, dtype=BF16, device=q.device)
+    check(lib().ohara_phi_attn_linear_bf16(_ptr(q), q.stride(0), _ptr(kcache), _ptr(vcache), _ptr(cos), _ptr(sin), rot, batch, h, dh, kcache.shape[1],
+                                           pos, _ptr(pos_dev), n_split, _ptr(workspace), _ptr(out), _ptr(x), x.stride(0), _ptr(w.data), w.n, w.k,
+                                           _ptr(bias), _ptr(y), y.stride(0), _stream()), "phi_attn_linear")
+    return out, y
+
+
 # ---- hybrid decoders: attention with a distance bias beside recurrent layers -------------------------
 # bf16 or fp32 activations: the entry point follows the dtype of the activations.
 

@@ -240,15 +240,22 @@ class Phi:
                 live = c.max_sequence_length if pos_dev is not None else start + S
                 kd = ops.kv_dequant(cache, "key", B, live)
                 vd = ops.kv_dequant(cache, "value", B, live)
-                ops.phi_attn(buf["q"], kd, vd, self.cos, self.sin, self.rot, B, S, H, D, start, pos_dev, out=buf["attn"],
-                             n_split=buf["ns"] if S == 1 else 1, workspace=buf["ws"])
+                keys, values = kd, vd
             else:
                 ops.phi_block_in(buf["h"], None, None, c.eps, L["w_in"], L["b_in"], d, self.ff, B, S, start, cache.key,
                                  cache.value, buf["q"], buf["act"], pos_dev)
-                ops.phi_attn(buf["q"], cache.key, cache.value, self.cos, self.sin, self.rot, B, S, H, D, start, pos_dev,
-                             out=buf["attn"], n_split=buf["ns"] if S == 1 else 1, workspace=buf["ws"])
-            ops.linear_bias(buf["attn"], L["dense"], L["dense_b"], out=buf["mixer"])
-            ops.linear_bias(buf["act"], L["fc2"], L["fc2_b"], "add2", add1=buf["mixer"], add2=cur, out=nxt)
+                keys, values = cache.key, cache.value
+            att = (buf["q"], keys, values, self.cos, self.sin, self.rot, B)
+            if S == 1:
+                # fc2 beside the attention, which it does not wait for; its rounded sums are the first addend of dense instead of the
+                # other way round, the same bits
+                ops.phi_attn_linear(*att, H, D, start, buf["act"], L["fc2"], L["fc2_b"], pos_dev, out=buf["attn"], y=buf["mixer"],
+                                    n_split=buf["ns"], workspace=buf["ws"])
+                ops.linear_bias(buf["attn"], L["dense"], L["dense_b"], "add2", add1=buf["mixer"], add2=cur, out=nxt)
+            else:
+                ops.phi_attn(*att, S, H, D, start, pos_dev, out=buf["attn"])
+                ops.linear_bias(buf["attn"], L["dense"], L["dense_b"], out=buf["mixer"])
+                ops.linear_bias(buf["act"], L["fc2"], L["fc2_b"], "add2", add1=buf["mixer"], add2=cur, out=nxt)
             cur, nxt = nxt, cur
         src = cur.view(B, S, d)[:, -1].contiguous() if (last_only and S > 1) else cur
         hn = ops.layernorm(src, self.ln_w, self.ln_b, c.eps)
