@@ -10,41 +10,62 @@
 namespace {
 
 // ---- LayerNorm: one workgroup per row ---------------------------------------------------
+// What bounds it: round trips, of few rows, one after the other.  So the row, the weight and the bias are asked for together and stay in
+// registers, C eighths a thread (C 0: any width, the row
+// read three times).  us, before / now: 1 x 2560 2.9 / 2.5, 700 x 2560 4.7 / 4.3, 4096 x 2560 15.1 / 12.0, 4096 x 4096 19.5 / 16.0.
+template <int C>
 __global__ __launch_bounds__(256) void layernorm_kernel(const bf16_t* x, int ldx, const bf16_t* w, const bf16_t* b,
                                                         bf16_t* out, int ldo, int d, float eps) {
   __shared__ float red[2][4];
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bf16_t* xr = x + (size_t)row * ldx;
+  uint4 xv[C ? C : 1], wv[C ? C : 1], bv[C ? C : 1];
+#pragma unroll
+  for (int c = 0; c < C; ++c) xv[c] = ldg16(xr + min((tid + 256 * c) * 8, d - 8));
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int k = min((tid + 256 * c) * 8, d - 8);
+    wv[c] = ldg16(w + k);
+    bv[c] = ldg16(b + k);
+  }
+  if (C) __builtin_amdgcn_sched_barrier(0);
+  auto each = [&](auto f) {  // f(column, the row's eight, weight, bias)
+    if (C) {
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+        if ((tid + 256 * c) * 8 < d) f((tid + 256 * c) * 8, xv[c], [&] { return wv[c]; }, [&] { return bv[c]; });
+    } else {
+      for (int k = tid * 8; k < d; k += 256 * 8) f(k, ldg16(xr + k), [&] { return ldg16(w + k); }, [&] { return ldg16(b + k); });
+    }
+  };
   // pass 1: mean
   float s = 0.f;
-  for (int k = tid * 8; k < d; k += 256 * 8) {
-    const uint4 v = ldg16(xr + k);
+  each([&](int, uint4 v, auto, auto) {
     const uint32_t u[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) s += lo_bf(u[i]) + hi_bf(u[i]);
-  }
+  });
   s = wave_sum(s);
   if (lane == 0) red[0][wave] = s;
   __syncthreads();
   const float mean = (((red[0][0] + red[0][1]) + red[0][2]) + red[0][3]) / (float)d;
-  // pass 2: biased variance around the mean (the row is re-read from cache)
+  // pass 2: biased variance around the mean
   float q = 0.f;
-  for (int k = tid * 8; k < d; k += 256 * 8) {
-    const uint4 v = ldg16(xr + k);
+  each([&](int, uint4 v, auto, auto) {
     const uint32_t u[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float a0 = lo_bf(u[i]) - mean, a1 = hi_bf(u[i]) - mean;
       q += a0 * a0 + a1 * a1;
     }
-  }
+  });
   q = wave_sum(q);
   if (lane == 0) red[1][wave] = q;
   __syncthreads();
   const float var = (((red[1][0] + red[1][1]) + red[1][2]) + red[1][3]) / (float)d;
   const float rstd = 1.0f / sqrtf(var + eps);
-  for (int k = tid * 8; k < d; k += 256 * 8) {
-    const uint4 v = ldg16(xr + k), g = ldg16(w + k), c = ldg16(b + k);
+  each([&](int k, uint4 v, auto weight, auto bias) {
+    const uint4 g = weight(), c = bias();
     const uint32_t u[4] = {v.x, v.y, v.z, v.w}, gu[4] = {g.x, g.y, g.z, g.w}, cu[4] = {c.x, c.y, c.z, c.w};
     uint32_t o[4];
 #pragma unroll
@@ -52,7 +73,7 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const bf16_t* x, int ldx
       o[i] = pack_bf((lo_bf(u[i]) - mean) * rstd * lo_bf(gu[i]) + lo_bf(cu[i]),
                      (hi_bf(u[i]) - mean) * rstd * hi_bf(gu[i]) + hi_bf(cu[i]));
     *reinterpret_cast<uint4*>(out + (size_t)row * ldo + k) = make_uint4(o[0], o[1], o[2], o[3]);
-  }
+  });
 }
 
 // ---- append: rows (seq, s) of k and v -> cache position pos + s ------------------------------
@@ -350,8 +371,8 @@ int ohara_layernorm_bf16(const uint16_t* x, int ldx, const uint16_t* weight, con
                          int rows, int d, float eps, void* stream) {
   if (!x || !weight || !bias || !out || rows < 1 || d < 8) return OHARA_EINVAL;
   if ((d & 7) || (ldx & 7) || (ldo & 7) || ldx < d || ldo < d) return OHARA_EINVAL;
-  hipLaunchKernelGGL(layernorm_kernel, dim3(rows), dim3(256), 0, (hipStream_t)stream, x, ldx, weight, bias, out, ldo, d,
-                     eps);
+  auto kernel = d <= 2048 ? layernorm_kernel<1> : d <= 4096 ? layernorm_kernel<2> : d <= 8192 ? layernorm_kernel<4> : layernorm_kernel<0>;
+  hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, (hipStream_t)stream, x, ldx, weight, bias, out, ldo, d, eps);
   return ohara_launch_status();
 }
 
