@@ -538,7 +538,7 @@ int ohara_depth_parts(int rows, int packed_rows, int k, float merge_us) {
   int best = 1;
   float low = 0.95f * least_time(rows, strips, k);
   for (int p = 2; p <= 8; p *= 2) {
-    if (k % (128 * p) || k / p < 512 || (int64_t)strips * p > INT32_MAX / 16) continue;
+    if (k % (128 * p) || k / p < (p == 2 ? 384 : 512) || (int64_t)strips * p > INT32_MAX / 16) continue;
     const float t = least_time(rows, strips * p, k / p) + (float)p * rows * strips * 16 * 8 * (1.f / 8e6f) + merge_us;
     if (t < low) {
       low = t;
