@@ -467,7 +467,7 @@ def gemv_ternary(q, s, sumq, w: PackedTernary, residual=None, out=None, want_acc
 
 # Rows up to which every workgroup of the fused BitLinear kernels quantises them in its own LDS; more are quantised once, then
 # multiplied in tiles.  us of a layer's four calls, fused / tiles, captured: width 2048 8 rows 69 / 56, 12 92 / 57, 16 114 / 57, 64 551 / 62;
-# 256 8 rows 26 / 27, 12 31 / 27, 64 118 / 32.  Launched one by one the tiles' eleven launches a layer take the host 119 us, so that a
+# 256 8 rows 26 / 27, 12 31 / 27, 64 118 / 32.  Launched one by one the tiles' ten launches a layer take the host 112 us, so that a
 # whole prompt of the 24-layer model takes 2.6 / 2.9 ms at 12 rows, 3.2 / 2.9 at 16, 14.7 / 2.8 at 64.
 BIT_ROWS = 12
 
