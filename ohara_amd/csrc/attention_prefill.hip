@@ -420,38 +420,24 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
 // heads, of 128: 93.2 us without, 91.5 with).  us, one after the other / this: 1024 x 16 25.8 / 21.9, 2048 x 6 45.7 / 36.0, 2048 x 16
 // 48.6 / 40.3, 3001 x 16 71.7 / 58.4, 4001 x 16 103.9 / 91.5, 32 x 300 x 6 behind 1500 115 / 92; heads of 64, 4001 x 16 68.8 / 55.7.
 // 238 VGPRs: 32 queries a wave do not fit (with fragments in parts of two they spill ten: 2048 x 6 55.6).
-template <int D>
-__global__ __launch_bounds__(256, 2) void attn_flow_kernel(PrefillArgs a) {
-  constexpr int NW = 4, QB = 16 * NW, NK = D / 32, ND = D / 16;
+template <int D, bool CHUNK>  // CHUNK: tiles first .. end - 1 of a walk; else from the start to the last that any query sees
+__device__ __forceinline__ void flow_walk(const KvTile<D>& tile, int first, int end, int wave, const uint4 (&qf)[D / 32], int qpos,
+                                          int q_first /* the wave's first query's position */, int wave_last, uint32_t lds0, float scale_log2e,
+                                          f32x4 (&o)[D / 16], float& m_run, float& l_run) {
+  constexpr int NW = 4, NK = D / 32, ND = D / 16;
   typedef KvTile<D> Tl;
   constexpr int BY = Tl::BYTES, LOADS = KT / Tl::RPL / NW;
-  extern __shared__ __align__(16) unsigned char smem[];
-  int head, qblk;
-  my_block(a, head, qblk);
-  const int b = head / a.H, h = head - b * a.H;
-  if (b >= a.B) return;
-  const Sequence sq = sequence(a, b);
-  if (qblk * QB >= sq.S) return;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int m = lane & 15, g = lane >> 4;
-  const int q0 = qblk * QB, wq0 = q0 + wave * 16;
-  const Tl tile(a, sq, h / (a.H / a.Hkv), lane);
+  const int m = tile.lane & 15, g = tile.lane >> 4;
   const typename Tl::template Offsets<NW> offs = tile.template offsets<NW>(KT, wave);
   const uint32_t koff = offs.k[0], voff = offs.v[0];
-  const int ntiles = (min(a.pos + q0 + QB, tile.len) + KT - 1) / KT;   // tiles any query of the workgroup sees
-  const int wave_last = min(a.pos + wq0 + 15, tile.len - 1);           // last position any query of the wave sees
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;  // keys of even and of odd tiles, then their values
-
-  uint4 qf[NK];
-  int qpos;
-  load_queries<D>(qf, qpos, a, sq, h, wq0 + m, g);
-  f32x4 o[ND];
 #pragma unroll
   for (int db = 0; db < ND; ++db) o[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
-  tile.template issue_half<NW, true>(0, lds0, wave, koff);
-  tile.template issue_half<NW, false>(0, lds0 + 2 * BY, wave, voff);
-  if (1 < ntiles) tile.template issue_half<NW, true>(1, lds0 + BY, wave, koff);
+  m_run = -INFINITY;
+  l_run = 0.f;
+  if (CHUNK && first >= end) return;
+  tile.template issue_half<NW, true>(first, lds0, wave, koff);
+  tile.template issue_half<NW, false>(first, lds0 + 2 * BY, wave, voff);
+  if (first + 1 < end) tile.template issue_half<NW, true>(first + 1, lds0 + BY, wave, koff);
 
   // where this lane's fragments lie (KvTile::keys and ::values): the permutations are an exclusive or
   const uint32_t kp = m * Tl::ROWB + (uint32_t)(g ^ (m & (Tl::PIECES - 1))) * 16;
@@ -482,6 +468,10 @@ __global__ __launch_bounds__(256, 2) void attn_flow_kernel(PrefillArgs a) {
   f32x4 s[NKB];  // tile t's scores, what they have to be multiplied with, and their maximum's shift
   float mul;
   Shift x;
+  if (CHUNK) {
+    mul = 1.0f;
+    x = {0.f, 1.f};
+  }
   auto shift = [&] {
     float top = -INFINITY;
 #pragma unroll
@@ -497,22 +487,22 @@ __global__ __launch_bounds__(256, 2) void attn_flow_kernel(PrefillArgs a) {
       for (int db = 0; db < ND; ++db) o[db] = mfma16(vf[w][db], pf[w], o[db]);
   };
 
-  if (1 < ntiles) tile_barrier<true, 2 * LOADS>();
+  if (first + 1 < end) tile_barrier<true, 2 * LOADS>();
   else tile_barrier<true, LOADS>();
-  {
+  if (!CHUNK || first * KT <= wave_last) {
     uint4 kf[NK][NKB];
     read_keys(kf, lds0);
     score(s, kf);
-    const bool masked = KT - 1 > a.pos + wq0;
-    if (masked) softmax_mask(s, 0, qpos, g, a.scale_log2e);
-    mul = masked ? 1.0f : a.scale_log2e;
+    const bool masked = first * KT + KT - 1 > q_first;
+    if (masked) softmax_mask(s, first * KT, qpos, g, scale_log2e);
+    mul = masked ? 1.0f : scale_log2e;
     shift();
   }
   auto round = [&](int t, auto parity) {
     constexpr int P = decltype(parity)::value;
     tile_barrier<true, 0>();  // the next keys and these values are there, and everyone is done with those before
-    if (t + 2 < ntiles) tile.template issue_half<NW, true>(t + 2, lds0 + P * BY, wave, koff);
-    if (t + 1 < ntiles) tile.template issue_half<NW, false>(t + 1, lds0 + (3 - P) * BY, wave, voff);
+    if (t + 2 < end) tile.template issue_half<NW, true>(t + 2, lds0 + P * BY, wave, koff);
+    if (t + 1 < end) tile.template issue_half<NW, false>(t + 1, lds0 + (3 - P) * BY, wave, voff);
     const int t1 = (t + 1) * KT;
     uint4 vf[NWIN][ND], pf[NWIN];
     auto flow = [&](auto masked) {  // masked: not every query of the wave sees the whole of tile t + 1
@@ -526,8 +516,8 @@ __global__ __launch_bounds__(256, 2) void attn_flow_kernel(PrefillArgs a) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int kk = 0; kk < NKB; ++kk) s[kk] = sn[kk];
-      mul = decltype(masked)::value ? 1.0f : a.scale_log2e;
-      if (decltype(masked)::value) softmax_mask(s, t1, qpos, g, a.scale_log2e);
+      mul = decltype(masked)::value ? 1.0f : scale_log2e;
+      if (decltype(masked)::value) softmax_mask(s, t1, qpos, g, scale_log2e);
       __builtin_amdgcn_s_setprio(1);
       __builtin_amdgcn_sched_barrier(0);
       add(vf, pf);
@@ -541,9 +531,10 @@ __global__ __launch_bounds__(256, 2) void attn_flow_kernel(PrefillArgs a) {
           for (int i = 0; i < 4; ++i) o[db][i] *= x.corr;
       }
     };
-    if (t1 + KT - 1 <= a.pos + wq0) {  // (wave-uniform)
+    const bool more = !CHUNK || t + 1 < end;  // (all of these are wave-uniform)
+    if (more && t1 + KT - 1 <= q_first) {
       flow(std::false_type());
-    } else if (t1 <= wave_last) {
+    } else if (more && t1 <= wave_last) {
       flow(std::true_type());
     } else if (t * KT <= wave_last) {  // the wave's last tile
       read_values(vf, lds0 + (2 + P) * BY);
@@ -551,10 +542,36 @@ __global__ __launch_bounds__(256, 2) void attn_flow_kernel(PrefillArgs a) {
       add(vf, pf);
     }
   };
-  for (int t = 0; t < ntiles; t += 2) {
+  for (int t = first; t < end; t += 2) {
     round(t, std::integral_constant<int, 0>());
-    if (t + 1 < ntiles) round(t + 1, std::integral_constant<int, 1>());
+    if (t + 1 < end) round(t + 1, std::integral_constant<int, 1>());
   }
+}
+template <int D>
+__global__ __launch_bounds__(256, 2) void attn_flow_kernel(PrefillArgs a) {
+  constexpr int NW = 4, QB = 16 * NW, NK = D / 32, ND = D / 16;
+  typedef KvTile<D> Tl;
+  extern __shared__ __align__(16) unsigned char smem[];
+  int head, qblk;
+  my_block(a, head, qblk);
+  const int b = head / a.H, h = head - b * a.H;
+  if (b >= a.B) return;
+  const Sequence sq = sequence(a, b);
+  if (qblk * QB >= sq.S) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  const int q0 = qblk * QB, wq0 = q0 + wave * 16;
+  const Tl tile(a, sq, h / (a.H / a.Hkv), lane);
+  const int ntiles = (min(a.pos + q0 + QB, tile.len) + KT - 1) / KT;   // tiles any query of the workgroup sees
+  const int wave_last = min(a.pos + wq0 + 15, tile.len - 1);           // last position any query of the wave sees
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;  // keys of even and of odd tiles, then their values
+
+  uint4 qf[NK];
+  int qpos;
+  load_queries<D>(qf, qpos, a, sq, h, wq0 + m, g);
+  f32x4 o[ND];
+  float m_run, l_run;
+  flow_walk<D, false>(tile, 0, ntiles, wave, qf, qpos, a.pos + wq0, wave_last, lds0, a.scale_log2e, o, m_run, l_run);
   store_rows<D>(o, l_run, a, sq, h, wq0 + m, g, 0);
 }
 
@@ -657,6 +674,8 @@ __global__ __launch_bounds__(TEAMS * 256, TEAMS) void attn_team_kernel(PrefillAr
 // partial sums for attn_chunks_merge_kernel.  us with both launches, the kernels above / these: 16 queries x 16 heads (4 KV heads) of
 // 128 behind 3000 34.5 / 10.8, 48 queries 35.1 / 13.0, 200 38.4 / 22.5; 4 x 48 behind 1900 25.1 / 17.3; 200 x 16 heads of 64 behind
 // 2000 21.6 / 13.5.
+// The walk over a chunk is attn_flow_kernel's; one after the other / so: 4 x 48 behind 1900 21.4 / 20.5, 4 x 200 behind 2000 42.4 / 39.5, 200 behind 3000
+// 27.6 / 25.9, 8 x 100 x 6 heads behind 3000 34.3 / 33.2 (on a slower card than the lines above).
 struct Cut {
   int tasks, ntb, chunks, tiles;  // tasks of a (sequence, KV head) and fours of them; chunks, and tiles of one
 };
@@ -684,7 +703,6 @@ __global__ __launch_bounds__(256, 2) void attn_chunk_kernel(ChunkArgs c) {
   const int wq0 = task / c.group * 16, h = kvh * c.group + task % c.group;
   const Sequence sq = sequence(a, b);
   const Tl tile(a, sq, kvh, lane);
-  const typename Tl::template Offsets<NW> offs = tile.template offsets<NW>(KT, wave);
   const int first = chunk * c.cut.tiles, seen = (min(a.pos + last_task / c.group * 16 + 16, tile.len) + KT - 1) / KT;
   const int end = min(first + c.cut.tiles, seen);                           // tiles any task of the workgroup sees
   const int wave_last = task < c.cut.tasks ? min(a.pos + wq0 + 15, tile.len - 1) : -1;  // last position any query of the wave sees
@@ -694,50 +712,8 @@ __global__ __launch_bounds__(256, 2) void attn_chunk_kernel(ChunkArgs c) {
   int qpos;
   load_queries<D>(qf, qpos, a, sq, h, task < c.cut.tasks ? wq0 + m : sq.S, g);
   f32x4 o[ND];
-#pragma unroll
-  for (int db = 0; db < ND; ++db) o[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
-  if (first < end) tile.template issue<NW, true>(first, lds0, wave, offs);
-  uint32_t cur = lds0;
-  for (int t = first; t < end; ++t) {
-    tile_barrier<true, 0>();
-    const uint32_t next = lds0 + Tl::SLOT - (cur - lds0);
-    if (t + 1 < end) tile.template issue<NW, true>(t + 1, next, wave, offs);
-    const int t0 = t * KT;
-    if (t0 <= wave_last) {
-      f32x4 s[NKB];
-      uint4 kf[NKB][NK];
-#pragma unroll
-      for (int kk = 0; kk < NKB; ++kk)
-#pragma unroll
-        for (int j = 0; j < NK; ++j) kf[kk][j] = tile.keys(cur, kk, j);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < NK; ++j)
-#pragma unroll
-        for (int kk = 0; kk < NKB; ++kk) s[kk] = mfma16(kf[kk][j], qf[j], j ? s[kk] : (f32x4){0.f, 0.f, 0.f, 0.f});
-      __builtin_amdgcn_sched_barrier(0);
-      uint4 pf[NWIN];
-      const float corr = softmax_tile(s, pf, m_run, l_run, t0, a.pos + wq0, qpos, g, a.scale_log2e);
-      if (__any(corr != 1.0f)) {
-#pragma unroll
-        for (int db = 0; db < ND; ++db)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o[db][i] *= corr;
-      }
-#pragma unroll
-      for (int w = 0; w < NWIN; ++w) {
-        uint4 vf[ND];
-#pragma unroll
-        for (int db = 0; db < ND; ++db) vf[db] = tile.values(cur, w, db);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int db = 0; db < ND; ++db) o[db] = mfma16(vf[db], pf[w], o[db]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    cur = next;
-  }
+  float m_run, l_run;
+  flow_walk<D, true>(tile, first, end, wave, qf, qpos, a.pos + wq0, wave_last, lds0, a.scale_log2e, o, m_run, l_run);
   if (task >= c.cut.tasks) return;
   l_run = lane_xor_sum<32>(lane_xor_sum<16>(l_run));
   float* part = c.part + ((size_t)(bh * c.cut.tasks + task) * c.cut.chunks + chunk) * PS;
