@@ -930,6 +930,23 @@ __global__ __launch_bounds__(256) void merge_add2_kernel(GemmArgs a, const float
 
 }  // namespace
 
+// One launch where the product's workgroups are sixteen waves by themselves; such a workgroup has a CU to itself, so all that attends has the
+// CUs that the product leaves: at least eight chunks of them, and not behind a long context, where fewer chunks than asked for are longer walks
+// (`pos`, also where pos_dev goes on from there).  us, two launches before / two now / this: 2560 x 10240, 32 heads of 80, one row behind 40 21.1 /
+// 16.4 / 11.7, 200 21.9 / 20.5 / 15.5, 700 23.4 / 22.2 / 17.4, 1500 25.0 / 24.1 / 22.2, 2040 26.9 / 25.7 / 27.9; two rows (six chunks) behind 700
+// 24.6 / 23.7 / 22.5, 1500 29.4 / 28.0 / 32.7.
+bool ohara_launch_phi_attn_linear(PhiAttnArgs t, GemmArgs a, hipStream_t st, int* rc) {
+  const int strips = (a.N + 15) / 16;
+  const int chunks = strips < 256 ? (256 - (strips + 7) / 8 * 8) * 4 / std::max(t.B * t.H, 1) : 0;
+  if (a.B > 16 || a.K < 2048 || t.pos >= 1750 || !phi_eights(t) || chunks < std::min(t.ns, 8)) return false;
+  a.ny = 1; a.nstrips = strips;
+  t.ns = std::min(t.ns, chunks);
+  const int fours = (t.B * t.H * t.ns + 31) / 32 * 8;  // (whole eights: a strip's XCD is its workgroup's number)
+  hipLaunchKernelGGL(phi_attn_linear_kernel, dim3((unsigned)(fours + (strips + 7) / 8 * 8)), dim3(1024), 0, st, t, a, fours);
+  *rc = ohara_launch_status();
+  return true;
+}
+
 extern "C" {
 
 int ohara_pack_rows_bf16(const uint16_t* w, int n, int k, int ldw, const int32_t* perm, int n_padded,
@@ -1056,35 +1073,6 @@ int ohara_linear_bias_add2_bf16(const uint16_t* x, int ldx, const uint16_t* wp, 
   else if (parts == 4) OHARA_MERGE(4);
   else OHARA_MERGE(8);
 #undef OHARA_MERGE
-  return ohara_launch_status();
-}
-
-int ohara_phi_attn_linear_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, const uint16_t* vcache, const float* cos, const float* sin, int rot,
-                               int batch, int h, int dh, int t_max, int pos, const int32_t* pos_dev, int n_split, void* workspace, uint16_t* out,
-                               const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, const uint16_t* bias, uint16_t* y, int ldy, void* stream) {
-  PhiAttnArgs t;
-  const int rc = phi_attn_args(t, q, ldq, kcache, vcache, cos, sin, rot, batch, 1, h, dh, t_max, pos, pos_dev, n_split, workspace, out);
-  if (rc) return rc;
-  if (!x || !wp || !bias || !y || n < 1 || k < 1 || (k & 7) || (ldx & 7) || ldx < k || (n & 3) || (ldy & 3) || ldy < n) return OHARA_EINVAL;
-  const int strips = (n + 15) / 16;
-  // One launch where the product's workgroups are sixteen waves by themselves; such a workgroup has a CU to itself, so all that attends has the
-  // CUs that the product leaves: at least eight chunks of them, and not behind a long context, where fewer chunks than asked for are longer walks
-  // (`pos`, also where pos_dev goes on from there).  us, two launches before / two now / this: 2560 x 10240, 32 heads of 80, one row behind 40 21.1 /
-  // 16.4 / 11.7, 200 21.9 / 20.5 / 15.5, 700 23.4 / 22.2 / 17.4, 1500 25.0 / 24.1 / 22.2, 2040 26.9 / 25.7 / 27.9; two rows (six chunks) behind 700
-  // 24.6 / 23.7 / 22.5, 1500 29.4 / 28.0 / 32.7.
-  const int chunks = strips < 256 ? (256 - (strips + 7) / 8 * 8) * 4 / std::max(batch * h, 1) : 0;
-  if (batch > 16 || k < 2048 || pos >= 1750 || !phi_eights(t) || chunks < std::min(n_split, 8)) {
-    const int ra = ohara_phi_attn_bf16(q, ldq, kcache, vcache, cos, sin, rot, batch, 1, h, dh, t_max, pos, pos_dev, n_split, workspace, out, stream);
-    return ra ? ra : ohara_linear_bias_bf16(x, ldx, wp, n, k, bias, batch, OHARA_LIN_BIAS, nullptr, 0, nullptr, 0, y, ldy, stream);
-  }
-  GemmArgs a{};
-  a.wp = reinterpret_cast<const uint4*>(wp);
-  a.x = x; a.ldx = ldx; a.B = batch; a.N = n; a.K = k;
-  a.out = y; a.ldo = ldy; a.bias = bias;
-  a.ny = 1; a.nstrips = strips;
-  t.ns = std::min(n_split, chunks);
-  const int fours = (batch * h * t.ns + 31) / 32 * 8;  // (whole eights: a strip's XCD is its workgroup's number)
-  hipLaunchKernelGGL(phi_attn_linear_kernel, dim3((unsigned)(fours + (strips + 7) / 8 * 8)), dim3(1024), 0, (hipStream_t)stream, t, a, fours);
   return ohara_launch_status();
 }
 

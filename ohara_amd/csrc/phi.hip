@@ -417,4 +417,20 @@ int ohara_phi_attn_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, cons
   return ohara_launch_status();
 }
 
+int ohara_phi_attn_linear_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, const uint16_t* vcache, const float* cos, const float* sin, int rot,
+                               int batch, int h, int dh, int t_max, int pos, const int32_t* pos_dev, int n_split, void* workspace, uint16_t* out,
+                               const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, const uint16_t* bias, uint16_t* y, int ldy, void* stream) {
+  PhiAttnArgs t;
+  int rc = phi_attn_args(t, q, ldq, kcache, vcache, cos, sin, rot, batch, 1, h, dh, t_max, pos, pos_dev, n_split, workspace, out);
+  if (rc) return rc;
+  if (!x || !wp || !bias || !y || n < 1 || k < 1 || (k & 7) || (ldx & 7) || ldx < k || (n & 3) || (ldy & 3) || ldy < n) return OHARA_EINVAL;
+  GemmArgs a{};
+  a.wp = reinterpret_cast<const uint4*>(wp);
+  a.x = x; a.ldx = ldx; a.B = batch; a.N = n; a.K = k;
+  a.out = y; a.ldo = ldy; a.bias = bias;
+  if (ohara_launch_phi_attn_linear(t, a, (hipStream_t)stream, &rc)) return rc;
+  rc = ohara_phi_attn_bf16(q, ldq, kcache, vcache, cos, sin, rot, batch, 1, h, dh, t_max, pos, pos_dev, n_split, workspace, out, stream);
+  return rc ? rc : ohara_linear_bias_bf16(x, ldx, wp, n, k, bias, batch, OHARA_LIN_BIAS, nullptr, 0, nullptr, 0, y, ldy, stream);
+}
+
 }  // extern "C"

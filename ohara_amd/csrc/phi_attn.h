@@ -1,9 +1,7 @@
 // Phi's attention of single tokens over the cache (ohara/models/phi.py:98-117, rotary.py:131-184), as a kernel of its own (phi.hip) and beside a product's
 // workgroups (gemm_skinny.hip).
 #pragma once
-#include "common.h"
-
-namespace {
+#include "gemm_epilogue.h"
 
 // ---- attention ---------------------------------------------------------------------------
 // Four waves - a team - per (sequence, head, new token) and context chunk; a workgroup is a team or several.  Sixteen lanes own one cached
@@ -61,6 +59,11 @@ inline int phi_attn_args(PhiAttnArgs& a, const uint16_t* q, int ldq, const uint1
 
 // A lane's eight features lie in one half of the rotated ones, or behind them, and their angles on 16 bytes.
 inline bool phi_eights(const PhiAttnArgs& a) { return ((a.rot >> 1) & 7) == 0 && (((uintptr_t)a.cos | (uintptr_t)a.sin) & 15) == 0; }
+
+// gemm_skinny.hip: the attention beside y = x W^T + bias in one launch, where that is the quicker way (else false, and nothing is launched).
+bool ohara_launch_phi_attn_linear(PhiAttnArgs t, GemmArgs a, hipStream_t st, int* rc);
+
+namespace {
 
 // `block`: the workgroup's place among those that do this.
 template <int TEAMS, bool EIGHTS>
