@@ -246,14 +246,16 @@ class Phi:
                                  cache.value, buf["q"], buf["act"], pos_dev)
                 keys, values = cache.key, cache.value
             att = (buf["q"], keys, values, self.cos, self.sin, self.rot, B)
-            if S == 1:
+            if S == 1 and B <= 16:
                 # fc2 beside the attention, which it does not wait for; its rounded sums are the first addend of dense instead of the
                 # other way round, the same bits
                 ops.phi_attn_linear(*att, H, D, start, buf["act"], L["fc2"], L["fc2_b"], pos_dev, out=buf["attn"], y=buf["mixer"],
                                     n_split=buf["ns"], workspace=buf["ws"])
                 ops.linear_bias(buf["attn"], L["dense"], L["dense_b"], "add2", add1=buf["mixer"], add2=cur, out=nxt)
             else:
-                ops.phi_attn(*att, S, H, D, start, pos_dev, out=buf["attn"])
+                # more sequences are two launches in any case, and the addends go to the deeper product: from 33 rows on that is multiplied in parts
+                # of its depth then (us a step of four layers, 2560 wide, 33, 40, 64, 128 sequences: 453 471 529 783 with them at dense, 404 421 492 730)
+                ops.phi_attn(*att, S, H, D, start, pos_dev, out=buf["attn"], n_split=buf["ns"] if S == 1 else 1, workspace=buf["ws"])
                 ops.linear_bias(buf["attn"], L["dense"], L["dense_b"], out=buf["mixer"])
                 ops.linear_bias(buf["act"], L["fc2"], L["fc2_b"], "add2", add1=buf["mixer"], add2=cur, out=nxt)
             cur, nxt = nxt, cur

@@ -93,3 +93,38 @@ def test_refused(cuda):
     assert all(s == -1 for s in (status(pos=8), status(ns=2), status(ldx=2040), status(ldx=2052), status(n=18), status(wp=None)))
     with pytest.raises(ValueError, match="weight is"):
         ops.phi_attn_linear(q, kv, kv, angles, angles, 32, 1, 1, 64, 0, x[:, :2040], packed, bias)
+
+
+def _phi(cuda, **kw):
+    from ohara_amd.phi import Phi, PhiConfig
+    from oracle import phi_ref as P
+
+    kw = dict(vocab_size=96, max_sequence_length=64, hidden_size=512, num_attention_heads=8, num_hidden_layers=2, rotary_dim=0.5, **kw)
+    return Phi(PhiConfig(**kw), P.init_weights(P.RefPhiConfig(**kw), seed=2, dtype=BF), device=cuda)
+
+
+@pytest.mark.parametrize("B", [1, 16, 17, 32, 33, 40])
+def test_deep_product_of_many_sequences(cuda, monkeypatch, B):
+    """One token each: the second product of the MLP goes beside the attention up to sixteen sequences; of more it takes the addends, as
+    the product that 33 rows and more multiply in parts of the depth, and as the prompt's."""
+    from ohara_amd import ops
+    from ohara_amd._lib import lib
+
+    m = _phi(cuda)
+    assert lib().ohara_linear_bias_add2_bytes(33, 512, 2048) > 0
+    g = torch.Generator(device=cuda).manual_seed(B)
+    ids = torch.randint(0, 96, (B, 5), generator=g, device=cuda)
+    cache = m.build_kv_cache(B)
+    m(ids[:, :4], cache, 0)
+    seen, linear_bias = [], ops.linear_bias
+
+    def spy(x, w, bias, epilogue="bias", **kw):
+        seen.append((w.k, epilogue))
+        return linear_bias(x, w, bias, epilogue, **kw)
+
+    monkeypatch.setattr(ops, "linear_bias", spy)
+    got = m(ids[:, 4:], cache, 4)
+    assert seen[:-1] == ([(512, "add2")] if B <= 16 else [(512, "bias"), (2048, "add2")]) * 2
+    monkeypatch.undo()
+    one = torch.cat([m(ids[b:b + 1], None)[:, -1:] for b in range(B)])  # the whole sequence at once: roundings at other places of the same layers
+    assert (got.float() - one.float()).abs().max() <= 2.0 ** -5 * one.float().abs().max()
