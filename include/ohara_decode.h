@@ -727,6 +727,10 @@ int ohara_phi_attn_linear_bf16(const uint16_t* q, int ldq, const uint16_t* kcach
                                int batch, int h, int dh, int t_max, int pos, const int32_t* pos_dev, int n_split, void* workspace, uint16_t* out,
                                const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, const uint16_t* bias, uint16_t* y, int ldy, void* stream);
 
+// Into how many chunks that cuts the context where one launch does both; 0 where it makes two launches (as it also does where an angle's eighths do
+// not lie on 16 bytes or inside one half of the rotated features).
+int ohara_phi_attn_linear_chunks(int batch, int h, int dh, int n_split, int pos, int n, int k);
+
 /* ---- hybrid decoders: attention with a distance bias beside recurrent layers -----------------------
  * (no counterpart in the reference.)  Entry points ending in _bf16 keep activations, caches and weights
  * in bfloat16, those ending in _f32 in 32-bit floats; the residual stream, every norm, score, softmax

@@ -930,19 +930,29 @@ __global__ __launch_bounds__(256) void merge_add2_kernel(GemmArgs a, const float
 
 }  // namespace
 
-// One launch where the product's workgroups are sixteen waves by themselves; such a workgroup has a CU to itself, so all that attends has the
-// CUs that the product leaves: at least eight chunks of them, and not behind a long context, where fewer chunks than asked for are longer walks
-// (`pos`, also where pos_dev goes on from there).  us, two launches before / two now / this: 2560 x 10240, 32 heads of 80, one row behind 40 21.1 /
-// 16.4 / 11.7, 200 21.9 / 20.5 / 15.5, 700 23.4 / 22.2 / 17.4, 1500 25.0 / 24.1 / 22.2, 2040 26.9 / 25.7 / 27.9; two rows (six chunks) behind 700
-// 24.6 / 23.7 / 22.5, 1500 29.4 / 28.0 / 32.7.
+// Chunks of the attention beside the product in one launch; 0: two launches.  One where the product's workgroups are sixteen waves by themselves.  Such
+// a workgroup has a CU to itself, and so has each four teams of the attention, on the CUs that are left: eight chunks of them at least, or all.
+// Launches of their own spread the teams over all CUs, and what bounds them is what a CU takes in; so one launch costs what a CU takes in more of the
+// keys and values, and gives the product's time.  The line is through 520 calls, of 512 x 2048 to 2560 x 10240 with 8 to 32 heads of 64, 80 and
+// 128, 1 to 16 rows, behind 0 to 2040: 0.07 us dearer on average than the quicker of the two, 2.9 at worst (`pos >= 1750` before: 1.3 and 45, and
+// in 126 of them dearer than this attention and product had been by themselves).  us, two launches / this: 2560 x 10240, 32 heads of 80, one row
+// behind 40 16.6 / 11.9, 700 22.3 / 17.5, 2040 25.1 / 24.8; 2048 x 8192, 32 of 64, four rows behind 200 20.6 / 16.6, 1500 33.3 / 41.4; sixteen
+// behind 1500 95 / 130; 1024 x 4096, 16 of 64, one row behind 40 10.7 / 9.9, 700 16.1 / 16.4; 512 x 2048, 8 of 64 behind 100 9.5 / 11.9.
+static int phi_beside(int batch, int h, int dh, int n_split, int pos, int n, int k) {
+  const int strips = (n + 15) / 16, heads = batch * h;
+  const int chunks = strips < 256 ? std::min(n_split, (256 - (strips + 7) / 8 * 8) * 4 / std::max(heads, 1)) : 0;
+  if (batch > 16 || k < 2048 || chunks < std::min(n_split, 8)) return 0;
+  auto walk = [&](int ns) { return ns > 1 ? std::min(phi_chunk(pos, ns), pos + 1) : pos + 1; };  // positions of a team
+  const int alone = walk(n_split), teams = heads * (pos / alone + 1);
+  const float more = (4.f * walk(chunks) - std::max(1.f, teams * (1.f / 256)) * alone) * dh * 4.f;  // bytes a CU takes in
+  return more <= 6e-3f * n * k + 20e3f ? chunks : 0;
+}
 bool ohara_launch_phi_attn_linear(PhiAttnArgs t, GemmArgs a, hipStream_t st, int* rc) {
-  const int strips = (a.N + 15) / 16;
-  const int chunks = strips < 256 ? (256 - (strips + 7) / 8 * 8) * 4 / std::max(t.B * t.H, 1) : 0;
-  if (a.B > 16 || a.K < 2048 || t.pos >= 1750 || !phi_eights(t) || chunks < std::min(t.ns, 8)) return false;
-  a.ny = 1; a.nstrips = strips;
-  t.ns = std::min(t.ns, chunks);
+  t.ns = phi_eights(t) ? phi_beside(a.B, t.H, t.D, t.ns, std::min(std::max(t.pos, 0), t.t_max - 1), a.N, a.K) : 0;
+  if (!t.ns) return false;
+  a.ny = 1; a.nstrips = (a.N + 15) / 16;
   const int fours = (t.B * t.H * t.ns + 31) / 32 * 8;  // (whole eights: a strip's XCD is its workgroup's number)
-  hipLaunchKernelGGL(phi_attn_linear_kernel, dim3((unsigned)(fours + (strips + 7) / 8 * 8)), dim3(1024), 0, st, t, a, fours);
+  hipLaunchKernelGGL(phi_attn_linear_kernel, dim3((unsigned)(fours + (a.nstrips + 7) / 8 * 8)), dim3(1024), 0, st, t, a, fours);
   *rc = ohara_launch_status();
   return true;
 }
@@ -966,6 +976,11 @@ int ohara_pack_rows_bf16(const uint16_t* w, int n, int k, int ldw, const int32_t
 }
 
 int ohara_projection_norm_ahead(int rows, int k, int packed_rows) { return rows > 0 && k > 0 && packed_rows > 0 && ohara_norm_ahead(rows, k, packed_rows); }
+
+int ohara_phi_attn_linear_chunks(int batch, int h, int dh, int n_split, int pos, int n, int k) {
+  if (batch < 1 || h < 1 || dh < 8 || dh > 128 || n_split < 1 || n_split > 64 || pos < 0 || n < 1 || k < 1 || (int64_t)batch * h > INT32_MAX) return OHARA_EINVAL;
+  return phi_beside(batch, h, dh, n_split, pos, n, k);
+}
 
 int ohara_swiglu_perm(int f, int32_t* perm_host) {
   if (f < 1 || !perm_host) return OHARA_EINVAL;

@@ -60,6 +60,12 @@ inline int phi_attn_args(PhiAttnArgs& a, const uint16_t* q, int ldq, const uint1
 // A lane's eight features lie in one half of the rotated ones, or behind them, and their angles on 16 bytes.
 inline bool phi_eights(const PhiAttnArgs& a) { return ((a.rot >> 1) & 7) == 0 && (((uintptr_t)a.cos | (uintptr_t)a.sin) & 15) == 0; }
 
+// Positions of a chunk where there are ns of them, the query at `pos`: whole rounds, of 64 at least.
+__host__ __device__ inline int phi_chunk(int pos, int ns) {
+  const int per = (pos + ns) / ns;
+  return ((per < 64 ? 64 : per) + 15) & ~15;
+}
+
 // gemm_skinny.hip: the attention beside y = x W^T + bias in one launch, where that is the quicker way (else false, and nothing is launched).
 bool ohara_launch_phi_attn_linear(PhiAttnArgs t, GemmArgs a, hipStream_t st, int* rc);
 
@@ -68,7 +74,7 @@ namespace {
 // `block`: the workgroup's place among those that do this.
 template <int TEAMS, bool EIGHTS>
 __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
-  constexpr int R = 2, LEAST = 64;  // positions a lane group has in flight; of a chunk
+  constexpr int R = 2;  // positions a lane group has in flight
   __shared__ float qr_[TEAMS][128];
   __shared__ float gm_[TEAMS][16], gl_[TEAMS][16];
   __shared__ float gacc_[TEAMS][16][128];
@@ -89,7 +95,7 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
   const int pos = a.pos_dev ? *a.pos_dev : a.pos;
   int per = 0, ns = 1;  // positions of a chunk; chunks (they belong to calls of one token a sequence)
   if (a.ns > 1) {
-    per = (max(LEAST, (max(pos, 0) + a.ns) / a.ns) + 15) & ~15;  // whole rounds
+    per = phi_chunk(max(pos, 0), a.ns);
     ns = max(pos, 0) / per + 1;
   }
   const int rows = a.B * a.S * a.H, n = rows * ns;

@@ -28,3 +28,19 @@ def test_norms_ahead_of_a_projection(rows, k, packed_rows, ahead):
     assert lib().ohara_projection_norm_ahead(rows, k, packed_rows) == ahead
     assert not ahead or rows > ops.norm_rows(k)
     assert lib().ohara_projection_norm_ahead(0, k, packed_rows) == lib().ohara_projection_norm_ahead(rows, k, 0) == 0
+
+
+# heads, their width, columns and depth of the product, sequences, chunks asked for, position -> chunks of the one launch (0: two)
+@pytest.mark.parametrize("h,dh,n,k,batch,ns,pos,chunks", [
+    *((32, 80, 2560, 10240, 1, 16, pos, 12) for pos in (0, 40, 700, 1500, 1750, 2047)),
+    (32, 80, 2560, 10240, 2, 8, 40, 0), (32, 80, 2560, 10240, 17, 1, 0, 0), (32, 80, 2560, 2040, 1, 16, 0, 0), (32, 64, 4096, 8192, 1, 16, 0, 0),
+    (32, 64, 2048, 8192, 4, 4, 200, 4), (32, 64, 2048, 8192, 4, 4, 1000, 0), (32, 64, 2048, 8192, 4, 4, 1740, 0),
+    (32, 64, 2048, 8192, 16, 1, 100, 1), (32, 64, 2048, 8192, 16, 1, 700, 0), (16, 64, 1024, 4096, 1, 16, 40, 16), (16, 64, 1024, 4096, 1, 16, 100, 0),
+    (8, 64, 512, 2048, 1, 16, 0, 16), (8, 64, 512, 2048, 1, 16, 100, 0), (8, 64, 512, 2048, 8, 8, 1500, 0), (24, 64, 1536, 6144, 1, 16, 1000, 16),
+])
+def test_phi_attention_beside_a_product(h, dh, n, k, batch, ns, pos, chunks):
+    from ohara_amd import _lib
+
+    of = _lib.lib().ohara_phi_attn_linear_chunks
+    assert of(batch, h, dh, ns, pos, n, k) == chunks
+    assert of(0, h, dh, ns, pos, n, k) == of(batch, h, dh, 65, pos, n, k) == of(batch, h, dh, ns, -1, n, k) == _lib.EINVAL
