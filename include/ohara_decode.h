@@ -722,7 +722,8 @@ int ohara_phi_attn_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, cons
                         const float* sin, int rot, int batch, int seq_len, int h, int dh, int t_max, int pos,
                         const int32_t* pos_dev, int n_split, void* workspace, uint16_t* out, void* stream);
 // The same for one token a sequence, and beside it a product that does not wait for it: y = x W^T + bias as ohara_linear_bias_bf16 gives it,
-// x (batch, k), y (batch, n).  Neither may read what the other writes.  Where pos_dev is given, `pos` is about where it starts.
+// x (batch, k), y (batch, n).  Neither may read what the other writes.  Where pos_dev is given, `pos` is about
+// where it will be: how far back the attention goes decides whether one launch or two are quicker.
 int ohara_phi_attn_linear_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, const uint16_t* vcache, const float* cos, const float* sin, int rot,
                                int batch, int h, int dh, int t_max, int pos, const int32_t* pos_dev, int n_split, void* workspace, uint16_t* out,
                                const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, const uint16_t* bias, uint16_t* y, int ldy, void* stream);

@@ -284,9 +284,10 @@ class Phi:
         history = torch.zeros(steps, B, dtype=torch.int64, device=self.device)
         history[0].copy_(ids)
         state = torch.tensor([P, 1, 0, 0], dtype=torch.int32, device=self.device)  # {pos, step, done, pad}
+        middle = P + (steps - 1) // 2  # of the positions these steps are at: which launches a recorded step makes depends on it
 
         def step():
-            lg = self._run(ids, B, 1, cache, 0, state, False)
+            lg = self._run(ids, B, 1, cache, middle, state, False)
             ops.argmax(lg, next_ids=ids, history=history, step_state=state)  # also advances pos and step
 
         todo = steps - 1

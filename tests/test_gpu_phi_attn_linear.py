@@ -133,3 +133,24 @@ def test_deep_product_of_many_sequences(cuda, monkeypatch, B):
     monkeypatch.undo()
     one = torch.cat([m(ids[b:b + 1], None)[:, -1:] for b in range(B)])  # the whole sequence at once: roundings at other places of the same layers
     assert (got.float() - one.float()).abs().max() <= 2.0 ** -5 * one.float().abs().max()
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("P,steps", [(1, 2), (9, 8), (30, 35)])
+def test_replies_say_where_they_are(cuda, monkeypatch, P, steps, int8):
+    """The steps of a reply read their position on the device; the launches are chosen by the middle of the positions they will be at."""
+    from ohara_amd import ops
+
+    m = _phi(cuda)
+    prompt = torch.randint(0, 96, (2, P), generator=torch.Generator().manual_seed(P)).to(cuda)
+    seen, call = [], ops.phi_attn_linear
+
+    def spy(*args, **kw):
+        seen.append((args[9], args[13] is not None))
+        return call(*args, **kw)
+
+    monkeypatch.setattr(ops, "phi_attn_linear", spy)
+    plain = m.generate_greedy(prompt, steps, use_graph=False, int8=int8)
+    if P > 1:  # (a prompt of one token goes through the same call)
+        assert set(seen) == {(P + (steps - 1) // 2, True)}
+    assert torch.equal(m.generate_greedy(prompt, steps, int8=int8), plain)
