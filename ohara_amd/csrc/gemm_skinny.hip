@@ -1024,11 +1024,14 @@ int ohara_linear_bias_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n
 // The merge of a residual is the norm behind it too: 1 us more than that norm's launch, and as long as that where the depth is under 2048 (two
 // parts: 128 x 768 3.0 / 3.2); the other one is a launch of its own, 3.  us with the norm, whole / in two parts of at least 384: 768 x 768, 64, 128,
 // 192 rows 5.4 6.8 7.2 / 5.0 5.5 6.3; 1024 x 1024, 96 and 128 rows 7.3 7.4 / 5.9 6.0; 1536 x 1536, 128, 192 rows 8.9 10 / 7.8 8.8, 384 rows 11.9 / 12.1.
-// Narrow and shallow products stay whole at any rows (512 x 1024, 128 rows 6.8 / 5.7): small models give a prompt the same bits alone and beside
-// others, which their users hold them to.  (Up to 32 rows a strip's workgroup over the whole depth is the faster one.)
+// Under 640 columns: the merge as beyond 2048, and parts of 512 at least (33 to 500 rows, 512 x 1280 8.4 / 6.5, 512 x 1792 9.4 / 7.4, 256 x 1536 9.0 /
+// 6.9 at 96 rows).  That leaves the products of a model of at most 512 columns whose MLP is 1024 wide whole at any rows, which is what gives its prompts the same
+// bits alone and side by side (there is no room for parts there); it costs them 1 us a product (512 x 1024, 128 rows 6.8 / 5.7).  Wider or
+// deeper models' prompts differ between the two by the order of fp32 sums, and by their number of rows.  (Up to 32 rows a strip's workgroup over the whole
+// depth is the faster one.)
 static int residual_parts(int rows, int n, int k) {
-  if (n < 640 && k < 2048) return 1;
-  return rows > 32 && (n & 15) == 0 && n <= 4096 ? ohara_depth_parts(rows, n, k, k < 2048 ? 0.1f : 1.f) : 1;
+  if (rows <= 32 || (n & 15) || n > 4096 || (n < 640 && k < 1024)) return 1;
+  return ohara_depth_parts(rows, n, k, n >= 640 && k < 2048 ? 0.1f : 1.f);
 }
 static int bias_parts(int rows, int n, int k) { return rows > 32 && (n & 15) == 0 ? ohara_depth_parts(rows, n, k, 3.f) : 1; }
 static int64_t parts_bytes(int parts, int rows, int n) { return parts > 1 ? (int64_t)parts * rows * n * (int64_t)sizeof(float) : 0; }

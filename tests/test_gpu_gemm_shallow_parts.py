@@ -10,6 +10,7 @@ BF = torch.bfloat16
 # columns, depth, rows, parts
 SHAPES = [
     (768, 768, 32, 1), (768, 768, 33, 2), (768, 768, 65, 2), (768, 768, 128, 2), (768, 768, 159, 2), (768, 768, 700, 1), (640, 768, 97, 2), (512, 1024, 97, 1), (768, 640, 100, 1),
+    (512, 768, 97, 1), (512, 1280, 33, 2), (512, 1280, 190, 2), (512, 1792, 250, 2), (384, 1280, 97, 2), (256, 1536, 500, 2), (16, 1024, 130, 1),
     (1024, 1024, 70, 2), (1536, 1536, 190, 2), (640, 1536, 300, 2), (768, 1792, 193, 2),
 ]
 

@@ -56,6 +56,31 @@ def test_prompts_side_by_side(cuda, heads, kv_heads, width, lens):
             assert (c.key[b] == 7.0).all() and (c.value[b] == 7.0).all()
 
 
+# a product of the layer is in parts of its depth alone (768 columns and 768 and 1536 deep; 1024 and 1024 and 2048; 512 and 2048) and whole
+# side by side, where there is no room for them
+@pytest.mark.parametrize("heads,width,inner", [(6, 768, 1536), (8, 1024, 2048), (4, 512, 2048)])
+def test_prompts_side_by_side_of_wider_models(cuda, heads, width, inner):
+    from ohara_amd._lib import lib
+
+    kw = dict(vocab_size=640, hidden_size=width, intermediate_size=inner, num_attention_heads=heads, num_key_value_heads=heads, num_hidden_layers=2,
+              max_sequence_length=512)
+    from ohara_amd.llama import Config, Llama
+
+    m = Llama(Config(**kw), R.init_weights(R.RefConfig(**kw), seed=5, dtype=BF, std=0.06, norm_jitter=0.1), device=cuda)
+    lens = [70, 100, 300, 129]
+    assert any(lib().ohara_gemm_residual_norm_bytes(n, width, k) for n in lens for k in (width, inner))
+    cache, alone, prompts = m.build_kv_cache(4), m.build_kv_cache(4), _ids(lens)
+    got = m.prompts(prompts, cache, [2, 0, 3, 1])
+    for i, (p, b) in enumerate(zip(prompts, [2, 0, 3, 1])):
+        want = m(p.view(1, -1).to(cuda), [c._row_view(b) for c in alone], 0, last_only=True)[0, 0]
+        # as for up to 64 rows above: fp32 sums in another order, rounded to 8 bits at the same places of two layers
+        tol = 2.0 ** -6
+        assert (got[i].float() - want.float()).abs().max() <= tol * want.float().abs().max()
+        for c, a in zip(cache, alone):
+            for x, y in ((c.key[b], a.key[b]), (c.value[b], a.value[b])):
+                assert (x[:lens[i]].float() - y[:lens[i]].float()).abs().max() <= tol * y.float().abs().max()
+
+
 def test_what_is_refused(cuda):
     m = _model(cuda, 4, 2, 512)
     cache = m.build_kv_cache(3)
