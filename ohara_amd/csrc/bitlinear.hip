@@ -217,32 +217,35 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const bf16_t* x, int ldx
 struct QuantSets {
   const bf16_t* nw[3];
 };
-// A workgroup a row, its 16-byte pieces in registers (PT a thread), for all sets at once: what they share - the row, its block norm, the sums of
+// T threads a row, its 16-byte pieces in registers (PT a thread), for all sets at once: what they share - the row, its block norm, the sums of
 // squares - is worked out once, and every load goes out before the first is used.  The sums of squares are added as the kernels above add a
 // row, lane l the pieces l, l + 64, ... in turn and then the lanes; the rest is exact in any order.  GATED: the row is silu(gate) * up, rounded
 // as silu_mul_kernel does.  us, a wave a row and a set that walked it four or five times through LDS, each walk behind the one before / this, in a
 // prompt of 300 rows: 2048 wide, one to three sets 9.2 / 5.6; 5632 wide, with the launch that multiplied gate and up 9.2 + 4.5 / 7.7.
-template <int PT, bool GATED>
+template <int T, int PT, bool GATED>
 __global__ __launch_bounds__(256) void row_quant_kernel(const bf16_t* x, int ldx, const bf16_t* up, const bf16_t* pre_w, QuantSets sets, int n_sets,
                                                         int rows, int K, float eps, int8_t* q, int ldq, float* s_out, int* sumq_out) {
-  __shared__ float sums[2][PT * 256], top[3][4];
+  static_assert(T == 64 || T == 256, "");
+  __shared__ float sums[2][T == 64 ? 1 : PT * 256], top[3][4];
   __shared__ int total[3][4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = blockIdx.x, pieces = K >> 3;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tid = T == 64 ? lane : threadIdx.x, pieces = K >> 3;
+  const int r = T == 64 ? blockIdx.x * 4 + wave : blockIdx.x;
+  if (T == 64 && r >= rows) return;
   uint4 v[PT], pw[PT], nw[3][PT];
 #pragma unroll
-  for (int i = 0; i < PT; ++i) v[i] = ldg16(x + (size_t)r * ldx + min(tid + 256 * i, pieces - 1) * 8);  // (past the end: the last piece, not counted)
+  for (int i = 0; i < PT; ++i) v[i] = ldg16(x + (size_t)r * ldx + min(tid + T * i, pieces - 1) * 8);  // (past the end: the last piece, not counted)
   if (GATED) {
 #pragma unroll
-    for (int i = 0; i < PT; ++i) pw[i] = ldg16(up + (size_t)r * ldx + min(tid + 256 * i, pieces - 1) * 8);
+    for (int i = 0; i < PT; ++i) pw[i] = ldg16(up + (size_t)r * ldx + min(tid + T * i, pieces - 1) * 8);
   } else if (pre_w) {
 #pragma unroll
-    for (int i = 0; i < PT; ++i) pw[i] = ldg16(pre_w + min(tid + 256 * i, pieces - 1) * 8);
+    for (int i = 0; i < PT; ++i) pw[i] = ldg16(pre_w + min(tid + T * i, pieces - 1) * 8);
   }
 #pragma unroll
   for (int k = 0; k < 3; ++k)
     if (k < n_sets) {
 #pragma unroll
-      for (int i = 0; i < PT; ++i) nw[k][i] = ldg16(sets.nw[k] + min(tid + 256 * i, pieces - 1) * 8);
+      for (int i = 0; i < PT; ++i) nw[k][i] = ldg16(sets.nw[k] + min(tid + T * i, pieces - 1) * 8);
     }
   __builtin_amdgcn_sched_barrier(0);
   if (GATED) {
@@ -256,11 +259,17 @@ __global__ __launch_bounds__(256) void row_quant_kernel(const bf16_t* x, int ldx
     }
   }
   auto inverse = [&](float* sum) {  // 1 / rms of the row in v
-#pragma unroll
-    for (int i = 0; i < PT; ++i) sum[tid + 256 * i] = sumsq8_bits(v[i]);
-    __syncthreads();
     float ss = 0.f;
-    for (int p = lane; p < pieces; p += 64) ss += sum[p];
+    if (T == 64) {
+#pragma unroll
+      for (int i = 0; i < PT; ++i)
+        if (tid + T * i < pieces) ss += sumsq8_bits(v[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < PT; ++i) sum[tid + T * i] = sumsq8_bits(v[i]);
+      __syncthreads();
+      for (int p = lane; p < pieces; p += 64) ss += sum[p];
+    }
     return 1.0f / sqrtf(wave_sum(ss) / (float)K + eps);
   };
   auto normed = [](uint4 u, uint4 w, float rinv) {
@@ -276,6 +285,7 @@ __global__ __launch_bounds__(256) void row_quant_kernel(const bf16_t* x, int ldx
     for (int i = 0; i < PT; ++i) v[i] = normed(v[i], pw[i], rinv0);
   }
   const float rinv = inverse(sums[1]);
+  float most[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k)
     if (k < n_sets) {
@@ -287,18 +297,18 @@ __global__ __launch_bounds__(256) void row_quant_kernel(const bf16_t* x, int ldx
 #pragma unroll
         for (int j = 0; j < 4; ++j) mx = fmaxf(mx, fmaxf(fabsf(lo_bf(w[j])), fabsf(hi_bf(w[j]))));
       }
-      const float wm = wave_max(mx);
-      if (lane == 0) top[k][wave] = wm;
+      most[k] = wave_max(mx);
+      if (T > 64 && lane == 0) top[k][wave] = most[k];
     }
-  __syncthreads();
+  if (T > 64) __syncthreads();
 #pragma unroll
   for (int k = 0; k < 3; ++k)
     if (k < n_sets) {
-      const float s = 127.0f / fmaxf(fmaxf(fmaxf(top[k][0], top[k][1]), fmaxf(top[k][2], top[k][3])), 1e-5f);
+      const float s = 127.0f / fmaxf(T == 64 ? most[k] : fmaxf(fmaxf(top[k][0], top[k][1]), fmaxf(top[k][2], top[k][3])), 1e-5f);
       int sq = 0;
 #pragma unroll
       for (int i = 0; i < PT; ++i) {
-        const int p = tid + 256 * i;
+        const int p = tid + T * i;
         const uint32_t uu[4] = {nw[k][i].x, nw[k][i].y, nw[k][i].z, nw[k][i].w};
         uint32_t pk[2] = {0u, 0u};
         int sum = 0;
@@ -315,9 +325,11 @@ __global__ __launch_bounds__(256) void row_quant_kernel(const bf16_t* x, int ldx
         }
       }
       sq = lanes_sum<32, 1>(sq);
-      if (lane == 0) total[k][wave] = sq;
+      if (T > 64 && lane == 0) total[k][wave] = sq;
+      if (T == 64 && lane == 0) sumq_out[(size_t)k * rows + r] = sq;
       if (tid == 0) s_out[(size_t)k * rows + r] = s;
     }
+  if (T == 64) return;
   __syncthreads();
   if (tid < n_sets) sumq_out[(size_t)tid * rows + r] = total[tid][0] + total[tid][1] + total[tid][2] + total[tid][3];
 }
@@ -325,11 +337,20 @@ __global__ __launch_bounds__(256) void row_quant_kernel(const bf16_t* x, int ldx
 template <bool GATED>
 int launch_row_quant(const bf16_t* x, int ldx, const bf16_t* up, const bf16_t* pre_w, const QuantSets& sets, int n_sets, int rows, int K, float eps,
                      int8_t* q, int ldq, float* s, int* sumq, hipStream_t st) {
-  const dim3 grid((unsigned)rows), block(256);
-  if (K <= 2048) hipLaunchKernelGGL((row_quant_kernel<1, GATED>), grid, block, 0, st, x, ldx, up, pre_w, sets, n_sets, rows, K, eps, q, ldq, s, sumq);
-  else if (K <= 4096) hipLaunchKernelGGL((row_quant_kernel<2, GATED>), grid, block, 0, st, x, ldx, up, pre_w, sets, n_sets, rows, K, eps, q, ldq, s, sumq);
-  else hipLaunchKernelGGL((row_quant_kernel<3, GATED>), grid, block, 0, st, x, ldx, up, pre_w, sets, n_sets, rows, K, eps, q, ldq, s, sumq);
-  return ohara_launch_status();
+  auto go = [&](auto kernel, int per) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + per - 1) / per)), dim3(256), 0, st, x, ldx, up, pre_w, sets, n_sets, rows, K, eps, q, ldq, s, sumq);
+    return ohara_launch_status();
+  };
+  // A wave a row has no barriers and a quarter of the workgroups, a workgroup a row a quarter of the chain.  us, a wave / a workgroup a row, one set and three:
+  // 256 wide, 1024, 4096 rows 4.8 5.5, 6.0 8.5 / 6.2 8.2, 12.3 18.7;  1024, 100, 1024, 4096 rows 5.0 5.9, 5.2 6.4, 7.7 13.4 / 5.0 5.5, 6.4 8.9, 13.0
+  // 20.9;  2816, 300, 1024, 4096 rows 6.5 10.2, 6.8 11.2, 15.1 28.6 / 6.1 8.7, 8.2 13.2, 19.9 35.3;  4096, 1024, 4096 rows 8.0 13.8, 20.5 37.0 / 8.7 14.0,
+  // 22.1 38.0;  5632, 4096 rows 36 65 / 27 48.
+  if (K <= 512) return go(row_quant_kernel<64, 1, GATED>, 4);
+  if (K <= 1024 && rows >= 300) return go(row_quant_kernel<64, 2, GATED>, 4);
+  if (K <= 2048 && rows >= 1024) return go(row_quant_kernel<64, 4, GATED>, 4);
+  if (K <= 3072 && rows >= 1024) return go(row_quant_kernel<64, 6, GATED>, 4);
+  if (K <= 2048) return go(row_quant_kernel<256, 1, GATED>, 1);
+  return K <= 4096 ? go(row_quant_kernel<256, 2, GATED>, 1) : go(row_quant_kernel<256, 3, GATED>, 1);
 }
 
 struct BitArgs {
