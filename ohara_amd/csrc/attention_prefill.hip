@@ -383,7 +383,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
       uint4 pf[QW][NWIN];
 #pragma unroll
       for (int qb = 0; qb < QW; ++qb) {
-        const float corr = softmax_tile(s[qb], pf[qb], m_run[qb], l_run[qb], t0, a.pos + wq0, qpos[qb], g, a.scale_log2e);
+        const float corr = softmax_tile(s[qb], pf[qb], m_run[qb], l_run[qb], t0, a.pos + wq0 + 16 * qb, qpos[qb], g, a.scale_log2e);
         if (__any(corr != 1.0f)) {  // most tiles leave the running maximum of every query of the wave alone
 #pragma unroll
           for (int db = 0; db < ND; ++db)
@@ -831,9 +831,7 @@ int launch_teams(PrefillArgs a, hipStream_t st) {
   return ohara_launch_status();
 }
 
-// All kernels of 16 queries a wave give the same bits, those of 32 where `pos` is a multiple of 32 (else a tile's scores are scaled before the
-// exponent for sixteen queries that need no mask); us with teams of 16 / 32 queries a workgroup and
-// attn_prefill_kernel's waves of 16 / 32 (64 / 128 a workgroup):
+// All kernels give the same bits; us with teams of 16 / 32 queries a workgroup and attn_prefill_kernel's waves of 16 / 32 (64 / 128 a workgroup):
 //   heads of 128                                                 heads of 64, 16 heads
 //     128 queries x 6 heads   4.5 /  5.5 /  5.5 /  7.1             160 queries      4.3 /  5.0 /  4.6 /  5.8
 //     48 behind 1900, 4 x 16 24.7 / 27.8 / 34   / 49               500              7.6 /  8.5 /  8.4 / 11.7
@@ -847,16 +845,19 @@ int launch_teams(PrefillArgs a, hipStream_t st) {
 // so: teams of 16 while every one has a CU to itself, and over more than two tiles while every two have one (with heads of 128
 // as teams of 32).  A shorter walk does not pay for the teams' barriers: us, teams / waves: heads of 64, 8 x 24 queries x 32 heads
 // 5.2 / 4.8; heads of 128, 8 x 33 x 16 6.2 / 5.4; over four tiles, 200 x 32 7.1 / 7.5.
-// 64 queries a workgroup: attn_flow_kernel, but one after the other where there are two tiles at most, which leaves little to overlap
-// (12 x 100 x 16 9.4 / 9.8, 16 x 64 x 32 11.3 / 11.6; three tiles, 8 x 192 x 32 17.3 / 16.5).
-// 128 queries a workgroup read each position once where 64 read it twice, and are slower by a quarter where there are few of
-// them or the second half of the last one is empty (heads of 128, 32 x 300 x 6 behind 1500: 92 / 126 us, 64 / 128 queries).  So
-// from three a CU on, if at least half of their second halves hold queries (2 x 4001 x 16 188 / 164, 16 x 500 x 12 39.5 / 35.5, 8 x 700
-// x 16 37.4 / 35.1, 16 x 1024 x 6 52.8 / 50.5; 8 x 2048 x 6 80.9 / 84.9; two a CU, 12 x 1024 x 6 41.8 / 44.7); with heads of 64 also from
-// the sixth workgroup of 64 queries a CU (28 x 112 x 24 behind 2000: 139 / 105; 4 x 2048 x 16 is both, 60.7 / 57.4; three, 3 x 2048 x 16 49.7 /
-// 54.0; 20 x 128 x 32 behind 250 27.6 / 27.7).
-// Before (one kernel, four waves, values through registers, the heads over all XCDs), for the table's lines: 5.8, 45, 16.5, 25,
-// 26, 167, 50, 46, 92; 5.2, 10.4, 12, 64.
+// The rest is drawn through 384 calls of 65 to 4096 tokens, 1 to 64 sequences, five combinations of heads of 64 and of 128, behind 0 to 2000: within
+// 1 % of the best of the three on average (29 % at worst), and 6 % quicker than attn_prefill_kernel alone.  us, its 16 / its 32 queries a wave /
+// attn_flow_kernel (16):
+// * 128 queries a workgroup read each position once where 64 read it twice, and are slower by a quarter where there are few of them or the second half of
+//   the last one is empty.  So from three a CU on, if at least half of their second halves hold queries (heads of 128: 16 x 468 x 16 behind 1000 160 / 122 /
+//   170, 8 x 512 x 16 26.7 / 26.7 / 25.8, 4 x 1073 x 16 behind 1500 156 / 131 / 117); with heads of 64 also from the sixth workgroup of 64 queries a
+//   CU (32 x 65 x 32 behind 1500 168 / 111 / 154; four, 8 x 512 x 16 14.8 / 18.1 / 16.9); with heads of 128 from the second of 128 if a sequence is one of
+//   them: all of one length (32 x 90 x 16 behind 1000 108 / 69 / 105, 16 x 100 x 32 18.5 / 15.8 / 18.3, 48 x 65 x 6 behind 1500 97 / 79 / 78).
+// * Else attn_flow_kernel (4001 x 6 heads of 128 behind 500 70 / 93 / 53, 8 x 65 x 16 behind 1000 35 / 44 / 26), but not over two tiles at most, which leaves
+//   little to overlap (12 x 100 x 16 9.4 / 9.8 of 16 queries), nor over a short walk where its workgroups, two a CU, need a second round: heads of 128, 8 x 300 x 16
+//   15.3 / 16.9 / 16.5, 4 x 383 x 32 19.6 / 21.1 / 20.6; heads of 64, of which the other has four a CU, 4 x 512 x 32 14.4 / 17.5 / 16.5, 16 x 128 x 32
+//   behind 37 11.4 / 12.5 / 13.5, and over walks of one length 16 x 94 x 32 behind 2000 78 / 82 / 89, 8 x 640 x 12 behind 1500 53 / 61 / 56 (of many
+//   lengths, 2 x 4045 x 8 from the start 66 / 85 / 54).
 template <int D>
 int launch_prefill_for(const PrefillArgs& a, const int32_t* lengths, hipStream_t st) {  // lengths: on the host, where they differ
   constexpr int CUS = 256;
@@ -876,8 +877,13 @@ int launch_prefill_for(const PrefillArgs& a, const int32_t* lengths, hipStream_t
   if constexpr (D == 128)
     if (long_walk && blocks(32) <= CUS) return launch_teams<D, 2>(a, st);
   const int64_t wide = blocks(128), halves = blocks(64);
-  if ((wide >= 3 * CUS || (D == 64 && halves > 5 * CUS)) && 2 * halves >= 3 * wide) return launch_waves<D, 2>(a, st);
-  return long_walk ? launch_flow<D>(a, st) : launch_waves<D, 1>(a, st);
+  const bool two_a_cu = D == 64 ? halves > 5 * CUS : wide > CUS && a.S <= 128;
+  if ((wide >= 3 * CUS || two_a_cu) && 2 * halves >= 3 * wide) return launch_waves<D, 2>(a, st);
+  const int far = a.pos + a.S;
+  const bool second_round = D == 128 ? halves > 2 * CUS && halves <= 3 * CUS && far <= 512
+                                     : (halves > 11 * CUS / 4 && halves <= 17 * CUS / 4 && far < 1000) ||
+                                           (halves > 13 * CUS / 4 && halves <= 4 * CUS && a.pos + 64 >= a.S);
+  return long_walk && !second_round ? launch_flow<D>(a, st) : launch_waves<D, 1>(a, st);
 }
 
 }  // namespace

@@ -37,3 +37,26 @@ def test_the_bits_of_calls_of_sixteen(cuda, B, S, H, Hkv, pos, D, odd):
             assert torch.allclose(got[b, s:s + n], want, rtol=0, atol=0, equal_nan=True)
     if not odd:
         assert torch.isfinite(got).all()
+
+
+# batch, queries, heads, key heads, head width, positions before them: 32 queries a wave, a tile that begins or ends between a wave's sixteens among them
+WIDE = [(32, 70, 24, 24, 64, 37), (28, 100, 24, 8, 64, 16), (22, 65, 24, 24, 128, 37), (17, 128, 32, 8, 128, 48), (24, 97, 16, 16, 128, 0), (9, 300, 32, 8, 128, 21),
+        (13, 200, 32, 32, 64, 5)]
+
+
+@pytest.mark.parametrize("B,S,H,Hkv,D,pos", WIDE)
+def test_the_bits_of_32_queries_a_wave(cuda, B, S, H, Hkv, D, pos):
+    """Wherever the queries stand: a sixteen whose tile needs no mask is scaled as where it has a wave to itself."""
+    from ohara_amd import ops
+
+    wide, halves = (-(-S // n) * H * B for n in (128, 64))
+    assert 2 * halves >= 3 * wide and (wide >= 768 or (halves > 1280 if D == 64 else wide > 256 and S <= 128))
+    g = torch.Generator(device=cuda).manual_seed(B + S)
+    q = (torch.randn(B, S, H, D, generator=g, device=cuda) * 2).to(BF)
+    k, v = (torch.randn(B, pos + S, Hkv, D, generator=g, device=cuda).to(BF) for _ in range(2))
+    got = ops.attn_prefill(q.view(B * S, H * D), k, v, H, Hkv, D, pos, S).view(B, S, H * D)
+    for b in (0, B - 1):
+        for s in range(0, S - 31, 16):
+            n = 16 if s + 32 <= S - 16 else S - s
+            want = ops.attn_prefill(q[b, s:s + n].reshape(n, H * D), k[b:b + 1], v[b:b + 1], H, Hkv, D, pos + s, n)
+            assert torch.equal(got[b, s:s + n], want)
