@@ -675,7 +675,8 @@ __global__ __launch_bounds__(TEAMS * 256, TEAMS) void attn_team_kernel(PrefillAr
 // 128 behind 3000 34.5 / 10.8, 48 queries 35.1 / 13.0, 200 38.4 / 22.5; 4 x 48 behind 1900 25.1 / 17.3; 200 x 16 heads of 64 behind
 // 2000 21.6 / 13.5.
 // The walk over a chunk is attn_flow_kernel's; one after the other / so: 4 x 48 behind 1900 21.4 / 20.5, 4 x 200 behind 2000 42.4 / 39.5, 200 behind 3000
-// 27.6 / 25.9, 8 x 100 x 6 heads behind 3000 34.3 / 33.2 (on a slower card than the lines above).
+// 27.6 / 25.9, 8 x 100 x 6 heads behind 3000 34.3 / 33.2 (on a slower card than the lines above).  Waves without a task (up to 16 queries of a KV head of
+// its own leave three) only load: 8 x 16 x 6 heads behind 3000 27.9 one after the other, 27.2 with them walking too, 26.9; 4 x 16 x 16 32.2, 31.1, 30.6.
 struct Cut {
   int tasks, ntb, chunks, tiles;  // tasks of a (sequence, KV head) and fours of them; chunks, and tiles of one
 };
@@ -705,16 +706,17 @@ __global__ __launch_bounds__(256, 2) void attn_chunk_kernel(ChunkArgs c) {
   const Tl tile(a, sq, kvh, lane);
   const int first = chunk * c.cut.tiles, seen = (min(a.pos + last_task / c.group * 16 + 16, tile.len) + KT - 1) / KT;
   const int end = min(first + c.cut.tiles, seen);                           // tiles any task of the workgroup sees
-  const int wave_last = task < c.cut.tasks ? min(a.pos + wq0 + 15, tile.len - 1) : -1;  // last position any query of the wave sees
+  const bool mine = task < c.cut.tasks;  // (a wave without a task only loads: it sees no position)
+  const int wave_first = mine ? a.pos + wq0 : -1, wave_last = mine ? min(a.pos + wq0 + 15, tile.len - 1) : -1;  // last position any query of the wave sees
   const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
 
   uint4 qf[NK];
   int qpos;
-  load_queries<D>(qf, qpos, a, sq, h, task < c.cut.tasks ? wq0 + m : sq.S, g);
+  load_queries<D>(qf, qpos, a, sq, h, mine ? wq0 + m : sq.S, g);
   f32x4 o[ND];
   float m_run, l_run;
-  flow_walk<D, true>(tile, first, end, wave, qf, qpos, a.pos + wq0, wave_last, lds0, a.scale_log2e, o, m_run, l_run);
-  if (task >= c.cut.tasks) return;
+  flow_walk<D, true>(tile, first, end, wave, qf, qpos, wave_first, wave_last, lds0, a.scale_log2e, o, m_run, l_run);
+  if (!mine) return;
   l_run = lane_xor_sum<32>(lane_xor_sum<16>(l_run));
   float* part = c.part + ((size_t)(bh * c.cut.tasks + task) * c.cut.chunks + chunk) * PS;
 #pragma unroll
