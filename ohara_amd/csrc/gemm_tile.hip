@@ -396,30 +396,63 @@ constexpr TileTime TIMES[6] = {
     {T64x128::TM, T64x128::TS, 2, 0.363f, 0.61f, 0.312f, 1.3f}, {T128::TM, T128::TS, 2, 0.60f, 0.56f, 0.453f, 1.45f},
     {T128x192::TM, T128x192::TS, 2, 0.747f, 0.64f, 0.6f, 3.15f}, {T256::TM, T256::TS, 1, 1.35f, 0.0f, 1.6f, 6.7f},
 };
-// From 1024 rows on, the tiles in halves among them: fitted to 117 products of 1024 to 16384 rows, 768 to 17920 packed rows, K 768 to 10240,
-// as they stand in a model (the activations just written, weights and caches of other layers before and after): the choice is within
-// 0.3 % of the best on average, 8 % at worst; the six with the times above take 9 % longer on average.  A tile alone on its CU pays its ends
-// once in every round.  Fewer rows are a round of small tiles or parts of the depth, to which those are fitted.
+// From 1024 rows on, the tiles in halves among them: drawn through 1117 products of 1024 to 16384 rows, 256 to 18000 packed rows, K 256 to 5632, with
+// the epilogues below, each as it stands in a model (128 MB of other work before it, then its activations written; weights, residual and output as that
+// leaves them): the choice is within 0.9 % of the best of the eight on average, 0.7 % on the products left out of the fit.  A tile alone on its CU
+// pays its ends once in every round.  Fewer rows are a round of small tiles or parts of the depth, to which the times above are fitted.
+// (Timed one behind the other, with residual and output in the L2s, the tiles of two a CU come out up to 15 % better than they are: 8192 rows 768 x 768 with
+// a residual 128 x 192 18.4 us there and 20.2 in the model, in halves 20.4 and 18.1.)
 constexpr TileTime MANY[10] = {
-    {T32::TM, T32::TS, 3, 0.14f, 0.376f, 0.079f, 2.2f},             {T64::TM, T64::TS, 2, 0.295f, 0.23f, 0.189f, 2.5f},
-    {T64x128::TM, T64x128::TS, 2, 0.405f, 0.529f, 0.346f, 2.13f},   {T128::TM, T128::TS, 2, 0.76f, 0.313f, 0.497f, 3.81f},
-    {T128x192::TM, T128x192::TS, 2, 0.94f, 0.575f, 0.633f, 4.81f},  {T256::TM, T256::TS, 1, 0.843f, 0.571f, 1.252f, 12.19f},
-    {H128x256::TM, H128x256::TS, 1, 0.561f, 0.53f, 0.762f, 7.48f},  {H128x192::TM, H128x192::TS, 1, 0.429f, 0.533f, 0.6f, 6.73f},
+    {T32::TM, T32::TS, 3, 0.114f, 0.157f, 0.113f, 0.706f}, {T64::TM, T64::TS, 2, 0.409f, 0.093f, 0.28f, 1.074f},
+    {T64x128::TM, T64x128::TS, 2, 0.533f, 0.f, 0.525f, 2.505f}, {T128::TM, T128::TS, 2, 0.884f, 0.527f, 0.456f, 4.059f},
+    {T128x192::TM, T128x192::TS, 2, 0.914f, 0.562f, 0.564f, 7.427f}, {T256::TM, T256::TS, 1, 0.842f, 0.814f, 1.527f, 15.093f},
+    {H128x256::TM, H128x256::TS, 1, 0.67f, 0.262f, 0.846f, 8.608f}, {H128x192::TM, H128x192::TS, 1, 0.37f, 1.327f, 0.861f, 5.699f},
     {T64x48::TM, T64x48::TS}, {T64x96::TM, T64x96::TS},  // (by the rule below)
 };
+constexpr int LARGEST = 5;  // 256 x 256
+// What an epilogue adds to a tile's ends there, us (beside the plain store's): nothing hides it where a CU has one tile.  Those of a residual, biases and gelu are
+// measured; the rotary one is by whole table rows where a wave's strips lie in one head, in pieces of 4 bytes where they do not, and so of heads of n.
+// us, one table for all epilogues / this: gelu, 2500 rows 4096 x 1024 50.4 / 40.5, 5500 rows 93.7 / 78.1, 2048 rows 17920 x 2560 246 / 213; rotary, heads
+// of 32, 16384 rows 768 x 256 28.4 / 18.6, of 96, 5500 rows 1920 x 1152 42.8 / 36.5, of 48, 8192 rows 2304 x 1536 80 / 70.
+enum Epilogue { PLAIN, GATED, RESIDUAL, BIAS, ADD2, HEAVY, ROTARY_64, ROTARY_32, ROTARY };  // ROTARY_n: heads of a multiple of n
+constexpr float EXTRA[9][8] = {
+    {},
+    {0.f, 0.01f, 0.02f, 0.04f, 0.06f, 0.92f, 0.46f, 0.35f},
+    {0.08f, 0.32f, 0.38f, 0.62f, 1.52f, 3.26f, 1.75f, 1.48f},
+    {0.03f, 0.43f, 0.59f, 1.1f, 1.44f, 6.1f, 3.8f, 2.4f},
+    {0.12f, 1.18f, 2.08f, 3.91f, 5.65f, 18.5f, 9.5f, 6.7f},
+    {0.22f, 1.69f, 2.42f, 5.63f, 8.6f, 24.3f, 12.4f, 8.96f},
+    {0.11f, 0.43f, 0.87f, 1.74f, 7.f, 2.4f, 1.2f, 7.f},
+    {0.f, 0.f, 0.f, 0.f, 11.67f, 16.28f, 8.14f, 11.67f},
+    {0.12f, 0.5f, 1.f, 2.f, 3.84f, 11.52f, 5.76f, 3.84f},
+};
+Epilogue epilogue_of(int epi, int dh, bool stage) {
+  switch (epi) {
+    case EPI_STORE: return PLAIN;
+    case EPI_SWIGLU: return GATED;
+    case EPI_RESIDUAL: return RESIDUAL;
+    case EPI_BIAS: return BIAS;
+    case EPI_BIAS_ADD2: return ADD2;
+    case EPI_ROPE: return stage ? ROTARY : dh % 64 == 0 ? ROTARY_64 : dh % 32 == 0 ? ROTARY_32 : ROTARY;
+    default: return HEAVY;
+  }
+}
 // Fewer than 1024 rows: 64 x 48 and 64 x 96 where such tiles fill the chip once and those of 32 or 64 would a third round or half of one more:
 // a CU takes in 50 to 90 GB/s, and one tile of 64 x 48 reads 112 rows of operands for the 3072 results of three of 32 x 32, which read 192.
 // us, the best of the six / 64 x 48: 128 rows 6144 x 768 with SwiGLU 6.8 / 5.9, 96 rows 6.0 / 5.7, 33 rows 11264 x 2048 14.2 / 11.8, 192 rows
 // 3072 x 2048 with rotary 13.7 / 11.7, 256 rows 14.8 / 12.1, 320 rows 2048 x 2048 12.6 / 11.5 (two rounds of 32 x 32: 160 rows 3072 x 2048
-// 10.8 / 11.4);  / 64 x 96: 65 to 128 rows 11264 x 2048 17.2 to 18.0 / 15.0 to 15.7, 512 rows 3072 x 2048 19.2 / 17.8 (192 rows 6144 x 768 7.6 / 7.4,
-// 160 rows 6.8 / 7.0).
-int one_round_tile(int rows, int strips, int K) {
+// 10.8 / 11.4), but not with an arithmetic epilogue, where its waves have twelve strips' rows each and the chain is short: with gelu 192 rows 3072 x 768 6.5 / 7.1,
+// 600 rows 1024 x 1024 7.9 / 8.8, 224 rows 2560 x 2560 12.6 / 13.1, 10240 deep 54 / 41.
+// 64 x 96 where what is read is the weights or a long depth, or 64 x 64 is a round and a half, and nothing but the sums is stored: 65 to 128 rows 11264 x 2048
+// 17.2 to 18.0 / 15.0 to 15.7, 320 rows 4096 x 4096 28.1 / 24.2 (192 rows 6144 x 768 7.6 / 7.4, 160 rows 6.8 / 7.0; with rotary 384 rows 3072 x 2048 13.8 /
+// 15.5, 1024 deep 8.5 / 10.2; with a residual 600 rows 2048 x 2048 13.8 / 14.8, 850 rows 1536 x 1536 10.7 / 11.6; 256 rows 5632 x 1024 with SwiGLU 8.2 / 8.7).
+int one_round_tile(int rows, int strips, int K, Epilogue epi) {
   auto tiles = [&](int r, int s) { return ((int64_t)rows + r - 1) / r * ((strips + s - 1) / s); };
   const int64_t narrow = tiles(T64x48::TM, T64x48::TS), wide = tiles(T64x96::TM, T64x96::TS);
-  if (K >= 512 && narrow >= 192 && narrow <= 256 && tiles(32, 2) > 512) return 8;
-  return rows > 64 && K >= 1024 && wide >= 192 && wide <= 256 ? 9 : -1;
+  if (K >= 512 && narrow >= 192 && narrow <= 256 && tiles(32, 2) > 512) return epi != HEAVY || K >= 4096 ? 8 : -1;
+  return epi <= GATED && rows > 64 && K >= 1024 && wide >= 192 && wide <= 256 && (rows <= 128 || K >= 4096 || tiles(64, 4) >= 384) ? 9 : -1;
 }
-float tile_time(const TileTime& t, int rows, int strips, int K) {
+float tile_time(const TileTime& t, int rows, int strips, int K, float extra = 0.f) {
   constexpr int CUS = 256;
   const int64_t tiles = ((int64_t)rows + t.rows - 1) / t.rows * ((strips + t.strips - 1) / t.strips);
   const int64_t waves = tiles / (CUS * t.slots), rest = tiles % (CUS * t.slots);
@@ -430,20 +463,16 @@ float tile_time(const TileTime& t, int rows, int strips, int K) {
     step += rest <= CUS || chain > chip ? chain : chip;
   }
   const float rounds = t.slots == 1 ? (float)((tiles + CUS - 1) / CUS) : tiles > CUS ? tiles * (1.f / CUS) : 1.f;
-  return step * K * (1.f / 64.f) + t.ends * rounds;
+  return step * K * (1.f / 64.f) + (t.ends + extra) * rounds;
 }
 
-// rotary: the epilogue of three strips a wave reads the tables in pieces of 4 bytes, and among many rows those tiles are not taken for it
-// (2048 rows 2304 x 768 128 x 192 20.7 us, 128 x 256 17.4; 8192 rows 53.1, 256 x 256 52.8)
-int fastest_tile(int rows, int strips, int K, bool rotary = false) {
+int fastest_tile(int rows, int strips, int K, Epilogue epi = PLAIN) {
   const bool many = rows >= 1024;
-  if (const int i = one_round_tile(rows, strips, K); !many && i >= 0) return i;
-  const TileTime* times = many ? MANY : TIMES;
+  if (const int i = one_round_tile(rows, strips, K, epi); !many && i >= 0) return i;
   int best = 0;
-  float low = tile_time(times[0], rows, strips, K);
-  for (int i = 1; i < (K < 64 ? 5 : many ? 8 : 6); ++i) {  // (halves walk whole steps)
-    if (many && rotary && times[i].strips == 12) continue;
-    const float t = tile_time(times[i], rows, strips, K);
+  float low = INFINITY;
+  for (int i = 0; i < (K < 64 ? 5 : many ? 8 : 6); ++i) {  // (halves walk whole steps)
+    const float t = many ? tile_time(MANY[i], rows, strips, K, EXTRA[epi][i]) : tile_time(TIMES[i], rows, strips, K);
     if (t < low) {
       low = t;
       best = i;
@@ -452,35 +481,23 @@ int fastest_tile(int rows, int strips, int K, bool rotary = false) {
   return best;
 }
 
-// A part of the rows in whole rounds of large tiles, one a CU, and the rest by itself, where the last round would be nearly empty: how many
-// rows and which tile (0 rows: all in one launch).  The times of two launches are those of MANY, added; taken from 8 % on.  us, one / two
-// launches: 2304 x 768 with rotary, 7600, 8192, 16384 rows 48.0 57.4 82.8 / 39.9 44.4 73.2; 6144 x 768 with SwiGLU, 5500, 11200 rows 66.2 117 /
-// 58.1 107; 3072 x 2048 with rotary, 5500, 11200 rows 87.8 144 / 65.1 125; 11264 x 2048 with SwiGLU, 3000 rows 142 / 125; 2048 x 5632, 11200
-// rows 226 / 204; 2560 x 10240, 8192 rows 375 / 326.  (At 7 % and less the model is not that good: 6144 x 768, 3000 rows 37.5 / 40.4.)
-struct Split {
-  int rows, tile;
-};
-Split split_rows(int rows, int strips, int K, bool rotary) {
-  Split best{0, 0};
-  if (rows < 1024 || K < 64) return best;
+// A part of the rows in whole rounds of 256 x 256, one a CU, and the rest by itself, where the last round would be nearly empty (0 rows: all in one launch).
+// The times of two launches are those above, added, and 5 us for the second one's start; taken from 3 % on.  us, one / two launches: 8192 rows 2304 x 768 with
+// rotary 43.9 / 41.7, heads of 64 43.4 / 39.1, 16384 rows 79.0 / 72.3, 5500 rows 6144 x 768 with SwiGLU 59.8 / 53.9, 5421 rows 2992 x 2560 99.4 / 81.8, 8192 rows
+// 2560 x 10240 375 / 326.  Of 456 products that the sum without those 5 us puts first 215 lose by it, those under 768 deep by 10 % on average and with a
+// bias by up to 40; of the 148 that this takes, 7 % quicker, 15 lose, one of them 33 % and the others 9 % at most.  (First rounds of 128 x 256 lose more often than not.)
+int split_rows(int rows, int strips, int K, Epilogue epi) {
+  if (rows < 1024 || K < 768) return 0;
+  auto time = [&](int i, int r) { return tile_time(MANY[i], r, strips, K, EXTRA[epi][i]); };
   auto least = [&](int r) {
-    float low = tile_time(MANY[0], r, strips, K);
-    for (int i = 1; i < 8; ++i)
-      if (!rotary || MANY[i].strips != 12) low = std::min(low, tile_time(MANY[i], r, strips, K));
+    float low = INFINITY;
+    for (int i = 0; i < 8; ++i) low = std::min(low, time(i, r));
     return low;
   };
-  float low = 0.92f * least(rows);
-  for (int i = 5; i < 7; ++i) {  // 256 x 256, 128 x 256
-    const int64_t across = (strips + MANY[i].strips - 1) / MANY[i].strips, down = ((int64_t)rows + MANY[i].rows - 1) / MANY[i].rows;
-    const int64_t first = across * down / 256 * 256 / across * MANY[i].rows;
-    if (first < 1 || first >= rows) continue;
-    const float t = tile_time(MANY[i], (int)first, strips, K) + least(rows - (int)first);
-    if (t < low) {
-      low = t;
-      best = {(int)first, i};
-    }
-  }
-  return best;
+  const int64_t across = (strips + T256::TS - 1) / T256::TS, down = ((int64_t)rows + T256::TM - 1) / T256::TM;
+  const int64_t first = across * down / 256 * 256 / across * T256::TM;
+  if (first < 1 || first >= rows) return 0;
+  return time(LARGEST, (int)first) + least(rows - (int)first) + 5.f < 0.97f * least(rows) ? (int)first : 0;
 }
 
 template <int EPI>
@@ -501,21 +518,22 @@ int launch_of(int tile, const GemmArgs& a, int nstrips, hipStream_t st) {
 template <int EPI>
 int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
   if (((uintptr_t)a.x & 15) != 0 || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return launch_tile<EPI, T64, false>(a, nstrips, st);
-  const Split split = split_rows(a.B, nstrips, a.K, EPI == EPI_ROPE);
-  if (!split.rows) return launch_of<EPI>(fastest_tile(a.B, nstrips, a.K, EPI == EPI_ROPE), a, nstrips, st);
+  const Epilogue epi = epilogue_of(EPI, a.Dh, a.stage);
+  const int split = split_rows(a.B, nstrips, a.K, epi);
+  if (!split) return launch_of<EPI>(fastest_tile(a.B, nstrips, a.K, epi), a, nstrips, st);
   GemmArgs first = a, rest = a;
-  first.B = split.rows;
-  rest.B = a.B - split.rows;
-  rest.x += (size_t)split.rows * a.ldx;
-  rest.row0 += split.rows;
+  first.B = split;
+  rest.B = a.B - split;
+  rest.x += (size_t)split * a.ldx;
+  rest.row0 += split;
   if (EPI != EPI_ROPE && EPI != EPI_PHI_IN) {  // (those find their rows from row0)
-    rest.out += (size_t)split.rows * a.ldo;
-    if (a.resid) rest.resid += (size_t)split.rows * a.ldr;
-    if (a.resid2) rest.resid2 += (size_t)split.rows * a.ldr2;
-    if (a.ids) rest.ids += split.rows;
+    rest.out += (size_t)split * a.ldo;
+    if (a.resid) rest.resid += (size_t)split * a.ldr;
+    if (a.resid2) rest.resid2 += (size_t)split * a.ldr2;
+    if (a.ids) rest.ids += split;
   }
-  const int rc = launch_of<EPI>(split.tile, first, nstrips, st);
-  return rc ? rc : launch_of<EPI>(fastest_tile(rest.B, nstrips, a.K, EPI == EPI_ROPE), rest, nstrips, st);
+  const int rc = launch_of<EPI>(LARGEST, first, nstrips, st);
+  return rc ? rc : launch_of<EPI>(fastest_tile(rest.B, nstrips, a.K, epi), rest, nstrips, st);
 }
 
 float least_time(int rows, int strips, int K) {
@@ -590,6 +608,11 @@ extern "C" int ohara_gemm_tile_of(int rows, int packed_rows, int k) {
   if (rows < 1 || packed_rows < 1 || k < 1) return OHARA_EINVAL;
   const TileTime& t = MANY[fastest_tile(rows, (packed_rows + 15) / 16, k)];  // (its sizes are those of both)
   return t.rows * 1000 + t.strips * 16;
+}
+
+extern "C" int ohara_gemm_first_rows(int rows, int packed_rows, int k, int epilogue, int dh) {
+  if (rows < 1 || packed_rows < 1 || k < 1 || epilogue < EPI_STORE || epilogue > EPI_BIAS_XIELU || (epilogue == EPI_ROPE && dh < 1)) return OHARA_EINVAL;
+  return split_rows(rows, (packed_rows + 15) / 16, k, epilogue_of(epilogue, dh, false));
 }
 
 extern "C" int ohara_gemm_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, int rows, int epilogue,

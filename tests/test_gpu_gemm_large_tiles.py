@@ -84,10 +84,18 @@ def _parts(rows, step=96):
     return [slice(a, a + step) for a in at] + [slice((at[-1] if at else -step) + step, rows)]
 
 
-@pytest.mark.parametrize("rows,n,k", [(4500, 4112, 200), (3000, 6160, 200), (4500, 11280, 136)])
-def test_rows_in_two_launches(cuda, rows, n, k):
-    """Whole rounds of large tiles and the rest by itself: every epilogue finds the rest's rows."""
+EPILOGUES = {"plain": 0, "residual": 1, "swiglu": 2, "bias": 4, "gelu": 5, "add2": 6, "softcap": 8, "lookup": 9, "xielu": 11}
+
+
+@pytest.mark.parametrize("rows,n,k,two", [(4500, 4048, 832, True), (1300, 11936, 1032, True), (4500, 4112, 200, False), (3000, 6160, 200, False), (4500, 11280, 136, False)])
+def test_rows_in_two_launches(cuda, rows, n, k, two):
+    """Whole rounds of large tiles and the rest by itself (short depths: all in one): every epilogue finds the rest's rows."""
     from ohara_amd import ops
+    from ohara_amd._lib import lib
+
+    for name, epilogue in EPILOGUES.items():
+        first = lib().ohara_gemm_first_rows(rows, n, k, epilogue, 0)
+        assert 0 < first < rows and first % 256 == 0 if two else first == 0, name
 
     g = torch.Generator(device=cuda).manual_seed(rows + n)
     r = lambda *s: torch.randn(*s, generator=g, device=cuda).to(BF)  # noqa: E731
@@ -104,10 +112,13 @@ def test_rows_in_two_launches(cuda, rows, n, k):
         assert torch.equal(call(slice(0, rows)), torch.cat([call(s) for s in _parts(rows)])), name
 
 
-@pytest.mark.parametrize("B,S,H,Hkv,D,k", [(2, 2250, 240, 8, 16, 136), (3, 1500, 48, 8, 64, 136), (3, 1000, 32, 8, 64, 520)])
-def test_rotary_rows_in_two_launches(cuda, B, S, H, Hkv, D, k):
+@pytest.mark.parametrize("B,S,H,Hkv,D,k,two", [(2, 1050, 58, 2, 128, 768, True), (2, 1050, 118, 2, 64, 768, True), (2, 1050, 162, 2, 48, 768, True),
+                                               (2, 2250, 240, 8, 16, 136, False), (3, 1500, 48, 8, 64, 136, False), (3, 1000, 32, 8, 64, 520, False)])
+def test_rotary_rows_in_two_launches(cuda, B, S, H, Hkv, D, k, two):
     from ohara_amd import ops
     from ohara_amd._lib import check, lib
+
+    assert (0 < lib().ohara_gemm_first_rows(B * S, (H + 2 * Hkv) * D, k, 3, D) < B * S) == two
 
     g = torch.Generator(device=cuda).manual_seed(S + D)
     rows, pos, T = B * S, 3, S + 5
@@ -135,10 +146,13 @@ def test_rotary_rows_in_two_launches(cuda, B, S, H, Hkv, D, k):
     assert all(torch.equal(keys2[B - b], keys[b]) and torch.equal(values2[B - b], values[b]) for b in range(B))
 
 
-def test_phi_rows_in_two_launches(cuda):
+@pytest.mark.parametrize("d,ff,two", [(768, 1792, True), (512, 2576, False)])
+def test_phi_rows_in_two_launches(cuda, d, ff, two):
     from ohara_amd import ops
+    from ohara_amd._lib import lib
 
-    B, S, d, ff, pos = 2, 2250, 512, 2576, 3  # 4112 packed rows
+    B, S, pos = 2, 2250, 3
+    assert (0 < lib().ohara_gemm_first_rows(B * S, 3 * d + ff, d, 7, 0) < B * S) == two
     g = torch.Generator(device=cuda).manual_seed(7)
     r = lambda *s: torch.randn(*s, generator=g, device=cuda).to(BF)  # noqa: E731
     x, bias, w = r(B * S, d), r(3 * d + ff), ops.pack_linear((r(3 * d + ff, d).float() * 0.1).to(BF))

@@ -44,3 +44,16 @@ def test_phi_attention_beside_a_product(h, dh, n, k, batch, ns, pos, chunks):
     of = _lib.lib().ohara_phi_attn_linear_chunks
     assert of(batch, h, dh, ns, pos, n, k) == chunks
     assert of(0, h, dh, ns, pos, n, k) == of(batch, h, dh, 65, pos, n, k) == of(batch, h, dh, ns, -1, n, k) == _lib.EINVAL
+
+
+# rows, packed rows, depth, epilogue, width of a rotary head -> rows of the first launch
+@pytest.mark.parametrize("rows,packed,k,epilogue,dh,first", [
+    (8192, 2304, 768, 3, 128, 7168), (16384, 2304, 768, 3, 64, 14336), (8192, 6144, 768, 2, 0, 0), (5421, 2992, 2560, 0, 0, 5376), (1023, 17920, 2560, 0, 0, 0),
+    (3615, 5776, 256, 0, 0, 0), (3615, 5776, 256, 4, 0, 0), (1870, 9008, 512, 4, 0, 0), (6209, 5600, 760, 0, 0, 0),
+])
+def test_rows_of_a_first_launch(rows, packed, k, epilogue, dh, first):
+    from ohara_amd import _lib
+
+    of = _lib.lib().ohara_gemm_first_rows
+    assert of(rows, packed, k, epilogue, dh) == first
+    assert of(0, packed, k, epilogue, dh) == of(rows, packed, k, 12, dh) == of(rows, packed, k, -1, dh) == of(rows, packed, k, 3, 0) == _lib.EINVAL
