@@ -60,7 +60,8 @@ class ContinuousBatcher:
 
     def _prefill(self, slots: list[int], prompts: list, last_only: bool = True) -> list[torch.Tensor]:
         """Run prompts (1-D ids, on the host) into free slots -> the logits (1 or len, V) of each: one call for all where the
-        model takes prompts of different lengths, else one call per prompt over its slot's rows of the cache."""
+        model takes prompts of different lengths, else one call per prompt over its slot's rows of the cache.  The caller
+        books the slots."""
         for b in slots:
             for c in self.cache:
                 c.lengths[b] = 0
@@ -84,7 +85,6 @@ class ContinuousBatcher:
             for b, ids in zip(slots, rows):
                 views = [c._row_view(b) for c in self.cache]
                 out.append(self.model.forward(ids.view(1, -1), views, 0, last_only=last_only)[0])
-        self._book(slots, [len(ids) for ids in prompts])
         return out
 
     GROUP_ROWS = 16384  # tokens of one call over several prompts
@@ -95,8 +95,8 @@ class ContinuousBatcher:
         return [self.model.forward(p.view(1, -1).to(self.model.device), [c._row_view(b) for c in self.cache], 0, last_only=True)[0]
                 for b, p in zip(slots, prompts)]
 
-    def _book(self, slots: list[int], lengths: list[int]) -> None:
-        """The slots hold so many tokens from now on."""
+    def _book(self, slots: list[int], lengths: list[int], toks: torch.Tensor | None = None) -> None:
+        """The slots hold so many tokens from now on, and are fed ``toks`` next (None: what they were to be fed)."""
         for b, length in zip(slots, lengths):
             for c in self.cache:
                 c.lengths[b] = length
@@ -104,7 +104,7 @@ class ContinuousBatcher:
             self.active[b] = True
         for c in self.cache:
             c.length = max(c.lengths)
-        self._mark(slots, lengths)
+        self._mark(slots, lengths, toks)
 
     def _mark(self, slots: list[int], lengths: list[int] | None, toks: torch.Tensor | None = None) -> None:
         """The slots on the model's device: taken with so many tokens and ``toks`` next, or left."""
@@ -142,7 +142,7 @@ class ContinuousBatcher:
         # one selection and one read-back for all of them (16 prompts of 100 to 800 tokens, d12, one behind the other:
         # 20.5 -> 19.2 ms with 15 steps)
         toks = self._select(torch.cat([logits.reshape(1, -1) for logits in self._prefill(slots, prompts)]))
-        self._mark(slots, [len(p) for p in prompts], toks)
+        self._book(slots, [len(p) for p in prompts], toks)
         return list(zip(slots, toks.tolist()))
 
     @torch.no_grad()
@@ -166,6 +166,7 @@ class ContinuousBatcher:
         tokens = [ids for _, ids in entries]
         if all(fresh):
             out = self._prefill(slots, tokens, last_only=False)
+            self._book(slots, [len(t) for t in tokens])
         elif not any(fresh) and all(len(t) == 1 for t in tokens) and sorted(slots) == [b for b in range(self.slots) if self.active[b]]:
             for b, t in zip(slots, tokens):
                 self.last[b] = int(t)

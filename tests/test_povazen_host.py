@@ -120,6 +120,22 @@ class _Model:
         return out[:, -1:] if last_only else out
 
 
+def test_prompts_that_join_mark_their_slots_once(monkeypatch):
+    """A launch on the device: positions, flags and the ids selected go in together, whatever the number of prompts."""
+    from ohara_amd.batching import ContinuousBatcher
+
+    batcher = ContinuousBatcher(_Model(), 4)
+    marks = []
+    mark = batcher._mark
+    monkeypatch.setattr(batcher, "_mark", lambda *a: (marks.append(a), mark(*a)))
+    monkeypatch.setattr(batcher, "_select", lambda logits: logits[:, 0].long() + 1)
+    assert batcher.add_many([[5, 6], [2, 8]]) == [(0, 7), (1, 9)] and len(marks) == 1
+    assert batcher.last.tolist() == [7, 9, 0, 0] and batcher.seq_pos.tolist() == [2, 2, 0, 0]
+    assert batcher.active_dev.tolist() == [1, 1, 0, 0] and batcher.lengths == batcher.cache[0].lengths == [2, 2, 0, 0]
+    batcher.feed([(None, [4, 2])])
+    assert len(marks) == 2 and batcher.seq_pos.tolist() == [2, 2, 2, 0] and batcher.active == [True, True, True, False]
+
+
 def test_replay_runs_the_batcher_and_gives_slots_back():
     from ohara_amd.trace import Replay
 
