@@ -27,12 +27,13 @@ def _attention(q, k, v, cos, sin, rot, pos):
     return want, want.abs() * 2.0 ** -8 + (p * vd.abs()).sum(1) * (near * (D + 4) * 2.0 ** -23 + 2.0 ** -18)[..., None] + 1e-30
 
 
-# batch, heads, head width, rotated, chunks, rows and depth of the product (the first four: one launch at all positions; the last four: two launches)
+# batch, heads, head width, rotated, chunks, rows and depth of the product (the first four: one launch at all positions; the last five: two launches)
 SHAPES = [
     (1, 3, 128, 16, 64, 2560, 10240), (2, 16, 64, 64, 16, 3000, 10240), (4, 24, 80, 32, 8, 1024, 10240),
     (1, 32, 80, 32, 16, 2560, 10240), (1, 32, 80, 32, 5, 2556, 2048), (2, 16, 64, 64, 16, 40, 2056), (1, 3, 128, 16, 64, 1000, 2304),
     (1, 32, 80, 32, 1, 2560, 2048), (4, 24, 80, 32, 8, 16, 2048),
     (2, 32, 80, 32, 8, 2560, 2304), (1, 8, 24, 12, 4, 64, 2048), (1, 8, 64, 32, 4, 64, 264), (17, 2, 64, 32, 4, 64, 2048),
+    (16, 32, 80, 40, 1, 16, 2048),
 ]
 
 
