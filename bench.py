@@ -334,7 +334,7 @@ def bench_prefill(model, cfg, dev):
     o = torch.empty_like(q)
     t = graph_time(lambda: ops.attn_prefill(q, kk, vv, H, H, D, 0, S, o))
     fl = 4.0 * B * H * D * S * (S + 1) / 2
-    kern.append({"kernel": "attn_prefill_kernel<128> causal", "rows": M, "us": round(t * 1e6, 1),
+    kern.append({"kernel": "attn_prefill, heads of 128, causal", "rows": M, "us": round(t * 1e6, 1),
                  "TFLOPs": round(fl / t / 1e12, 1), "mfma_util": round(fl / t / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4)})
     res["mfma_kernels"] = kern
     return res
@@ -856,7 +856,7 @@ def bench_povazen_kernels(cfg, dev):
         rows.append({"kernel": "prompt attention", "batch": B, "tokens": S,
                      "attn_bias_prefill_kernel": _flops(timed(lambda: ops.attn_bias(q, k, v, H, G, D, V, 0.1, slopes, gate, seq)),
                                                         fl, MFMA_BF16_PEAK_TFLOPS),
-                     "llama attn_prefill_kernel": _flops(timed(lambda: ops.attn_prefill(q, k, v, H, G, D, 0, S)), fl,
+                     "llama attn_prefill": _flops(timed(lambda: ops.attn_prefill(q, k, v, H, G, D, 0, S)), fl,
                                                          MFMA_BF16_PEAK_TFLOPS)})
     x = rnd(1, 2048)
     wn = torch.ones(2048, device=dev, dtype=bf)
@@ -1034,7 +1034,7 @@ def bench_vavelorn_kernels(name, dev):
                 MFMA_BF16_PEAK_TFLOPS),
             "povazen attn_bias_prefill_kernel": _flops(timed(lambda: ops.attn_bias(q, k, v, H, G, D, V, 0.1, slopes, gate, seq)), fl,
                                                        MFMA_BF16_PEAK_TFLOPS),
-            "llama attn_prefill_kernel": _flops(timed(lambda: ops.attn_prefill(q, k, v, H, G, D, 0, S)), fl, MFMA_BF16_PEAK_TFLOPS)})
+            "llama attn_prefill": _flops(timed(lambda: ops.attn_prefill(q, k, v, H, G, D, 0, S)), fl, MFMA_BF16_PEAK_TFLOPS)})
     side, norm, after = model.layers[0]["side"], model.layers[0]["norm2b"], model.layers[1]["norm1"]
     plain = ops.pack_linear(rnd(side.gate.n, d))
     for B in (1, 8, 32):

@@ -544,8 +544,10 @@ float least_time(int rows, int strips, int K) {
 
 }  // namespace
 
-// In how many parts the depth is multiplied: those of least time, the tiles' (as above) and the merge's, which is the sums written and
-// read at 8 TB/s (they stay in the caches) and merge_us.  us with what follows the product, whole / in parts:
+// In how many parts the depth is multiplied: those of least time, the tiles' and the merge's, which is the sums written and
+// read at 8 TB/s (they stay in the caches) and merge_us.  Priced with the six tiles of TIMES at any number of rows, also where another one is launched:
+// us, as chosen / best: 2048 x 5632, 1800 rows 63 whole / 55 in two parts, 768 x 3072, 1024 rows 23 whole / 18.6 in two; over 15 shapes and 29 numbers of
+// rows from 33 to 4096 4 % above the best choice on average.  us with what follows the product, whole / in parts:
 //   2048 x 5632, residual and norm, 33, 65, 192, 400, 700, 1500 rows  21.1 21.6 26.8 41.2 42.2 58.8 / 11.2 14.6 19.0 28.6 33.2 54.5
 //   768 x 3072                      65, 128, 256, 512, 700            11.9 11.9 12.0 13.7 17.6      /  7.5  8.0  9.9 12.3 14.2
 //   2560 x 10240, bias and addends  33, 128, 256, 700, 1000           31.7 43.0 59.4 72.3 116       / 20.1 28.3 32.7 52.8 71.1
