@@ -452,10 +452,13 @@ int one_round_tile(int rows, int strips, int K, Epilogue epi) {
   if (K >= 512 && narrow >= 192 && narrow <= 256 && tiles(32, 2) > 512) return epi != HEAVY || K >= 4096 ? 8 : -1;
   return epi <= GATED && rows > 64 && K >= 1024 && wide >= 192 && wide <= 256 && (rows <= 128 || K >= 4096 || tiles(64, 4) >= 384) ? 9 : -1;
 }
-float tile_time(const TileTime& t, int rows, int strips, int K, float extra = 0.f) {
+// `lone`: one full round and nothing behind it takes the chain's time, as a round that lacks a tile does; workgroups of several rounds drift apart.  us, where
+// that decides: 16384 rows 768 x 3072 with a residual 78.3 in 512 tiles of 128 x 192, 74.9 in 192 of 256 x 256; 768 x 768 23.1 / 22.1; 8192 rows 1024 x 1024
+// with a bias 22.5 of 128 x 128, 20.7 of 128 x 256 in halves.  (TIMES are fitted without.)
+float tile_time(const TileTime& t, int rows, int strips, int K, float extra = 0.f, bool lone = false) {
   constexpr int CUS = 256;
   const int64_t tiles = ((int64_t)rows + t.rows - 1) / t.rows * ((strips + t.strips - 1) / t.strips);
-  const int64_t waves = tiles / (CUS * t.slots), rest = tiles % (CUS * t.slots);
+  const int64_t waves = lone && tiles == CUS * t.slots ? 0 : tiles / (CUS * t.slots), rest = tiles - waves * CUS * t.slots;
   float step = waves * t.slots * t.full;
   if (rest) {
     const float others = t.slots == 1 ? rest * (1.f / CUS) : (float)((rest + CUS - 1) / CUS - 1);
@@ -472,7 +475,7 @@ int fastest_tile(int rows, int strips, int K, Epilogue epi = PLAIN) {
   int best = 0;
   float low = INFINITY;
   for (int i = 0; i < (K < 64 ? 5 : many ? 8 : 6); ++i) {  // (halves walk whole steps)
-    const float t = many ? tile_time(MANY[i], rows, strips, K, EXTRA[epi][i]) : tile_time(TIMES[i], rows, strips, K);
+    const float t = many ? tile_time(MANY[i], rows, strips, K, EXTRA[epi][i], true) : tile_time(TIMES[i], rows, strips, K);
     if (t < low) {
       low = t;
       best = i;
@@ -488,7 +491,7 @@ int fastest_tile(int rows, int strips, int K, Epilogue epi = PLAIN) {
 // bias by up to 40; of the 148 that this takes, 7 % quicker, 15 lose, one of them 33 % and the others 9 % at most.  (First rounds of 128 x 256 lose more often than not.)
 int split_rows(int rows, int strips, int K, Epilogue epi) {
   if (rows < 1024 || K < 768) return 0;
-  auto time = [&](int i, int r) { return tile_time(MANY[i], r, strips, K, EXTRA[epi][i]); };
+  auto time = [&](int i, int r) { return tile_time(MANY[i], r, strips, K, EXTRA[epi][i], true); };
   auto least = [&](int r) {
     float low = INFINITY;
     for (int i = 0; i < 8; ++i) low = std::min(low, time(i, r));

@@ -57,3 +57,11 @@ def test_rows_of_a_first_launch(rows, packed, k, epilogue, dh, first):
     of = _lib.lib().ohara_gemm_first_rows
     assert of(rows, packed, k, epilogue, dh) == first
     assert of(0, packed, k, epilogue, dh) == of(rows, packed, k, 12, dh) == of(rows, packed, k, -1, dh) == of(rows, packed, k, 3, 0) == _lib.EINVAL
+
+
+# rows of 512 tiles of 128 x 192, and of up to 32 fewer: the same tile for both
+@pytest.mark.parametrize("full,fewer,packed,k,tile", [(16384, 16256, 768, 768, 256256), (4096, 3900, 3072, 1024, 256256), (16384, 16256, 768, 3072, 256256)])
+def test_a_full_round_is_no_quicker_than_one_that_lacks_tiles(full, fewer, packed, k, tile):
+    from ohara_amd import _lib
+
+    assert _lib.lib().ohara_gemm_tile_of(full, packed, k) == _lib.lib().ohara_gemm_tile_of(fewer, packed, k) == tile
