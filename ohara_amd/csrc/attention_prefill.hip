@@ -47,12 +47,6 @@ __device__ __forceinline__ Sequence sequence(const PrefillArgs& a, int b) {
   return {(size_t)b * a.S, a.S, b};
 }
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uint2 lds_tr8(uint32_t addr) {
-  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((OHARA_LDS s16x4*)(uintptr_t)addr);
-  return __builtin_bit_cast(uint2, v);
-}
-
 // An XCD (ids go round-robin over the eight) gets whole heads, their late - longest - blocks first; where the heads do
 // not divide, an eighth of all blocks in the order of the heads, long and short ones in turn.  Where the sequences have lengths of
 // their own every eighth head, so that no XCD gets the long ones; the grid is rounded up to that (then head may be past the last).
@@ -253,11 +247,6 @@ __device__ __forceinline__ void store_rows(const f32x4 (&o)[N], float l, const P
 // and still give such kernels' results.  So a query whose sums are not finite walks its positions once more, by itself: the weights are
 // the same bits times a power of two (common.h: softmax bookkeeping).  That costs nothing where sums are finite; taking the masked values out of
 // the products, where a product with zeros says that it is needed, cost every call 0.3 to 0.6 us, or a tenth (8 x 15 behind 3000).
-__device__ __forceinline__ unsigned int not_finite(float sum) {  // of a lane's sums; bit m: query m of the wave
-  const unsigned long long l = __ballot(!(fabsf(sum) < INFINITY));
-  const unsigned int f = (unsigned int)l | (unsigned int)(l >> 32);
-  return (f | f >> 16) & 0xffffu;
-}
 // The queries q0 + m with a bit in `which` -> columns c0 .. c0 + cols - 1 of their rows.
 template <int D>
 __device__ __forceinline__ void walk_rows(const PrefillArgs& a, const Sequence& sq, int h, int q0, unsigned int which, int c0, int cols, int lane) {
@@ -311,7 +300,7 @@ __device__ __forceinline__ void store_few(const f32x4 (&o)[N], float l, const Pr
   float sum = 0.f;
 #pragma unroll
   for (int db = 0; db < N; ++db) sum += (o[db][0] + o[db][1]) + (o[db][2] + o[db][3]);
-  const unsigned int odd = not_finite(sum);
+  const unsigned int odd = columns_not_finite(sum);
   store_rows<D>(o, l, a, sq, h, odd >> (lane & 15) & 1 ? sq.S : q0 + (lane & 15), lane >> 4, d0);
   if (odd) walk_rows<D>(a, sq, h, q0, odd, 16 * d0, 16 * N, lane);
 }
@@ -764,7 +753,7 @@ __global__ __launch_bounds__(D * 4) void attn_chunks_merge_kernel(ChunkArgs c) {
     }
     M = mn;
   }
-  const unsigned int odd = FEW ? not_finite((sum[0] + sum[1]) + (sum[2] + sum[3])) : 0;
+  const unsigned int odd = FEW ? columns_not_finite((sum[0] + sum[1]) + (sum[2] + sum[3])) : 0;
   if (qi < a.S && !(odd >> m & 1)) {
     const float inv = 1.0f / l;
     *reinterpret_cast<uint2*>(a.out + ((size_t)b * a.S + qi) * a.H * D + (size_t)h * D + 16 * db + 4 * g) =

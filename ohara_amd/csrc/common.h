@@ -57,6 +57,18 @@ __device__ __forceinline__ uint4 lds16_at(uint32_t addr) {
   const u32x4 v = *(const OHARA_LDS u32x4*)(uintptr_t)addr;
   return make_uint4(v.x, v.y, v.z, v.w);
 }
+// ds_read_b64_tr_b16: within sixteen lanes, lane 4 r + c names columns 4 c .. 4 c + 3 of row r and lane n receives column n of the four rows.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 lds_tr8(uint32_t addr) {
+  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((OHARA_LDS s16x4*)(uintptr_t)addr);
+  return __builtin_bit_cast(uint2, v);
+}
+// Bit m: lane m, 16 + m, 32 + m or 48 + m has a sum that is not finite.
+__device__ __forceinline__ unsigned int columns_not_finite(float sum) {
+  const unsigned long long l = __ballot(!(fabsf(sum) < INFINITY));
+  const unsigned int f = (unsigned int)l | (unsigned int)(l >> 32);
+  return (f | f >> 16) & 0xffffu;
+}
 
 __device__ __forceinline__ float bf2f(bf16_t v) { return __uint_as_float(((uint32_t)v) << 16); }
 

@@ -5,7 +5,10 @@
 //                                           phi.py:98-117, rotary.py:131-184
 // The projections with bias, new_gelu and the parallel-block sum are epilogues of the skinny
 // GEMM (gemm_epilogue.h).
+#include "mfma_frag.h"
 #include "phi_attn.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -96,26 +99,349 @@ __global__ __launch_bounds__(256, 4) void phi_attn_kernel(PhiAttnArgs a) {
 }
 
 // ---- attention over many new tokens (prefill) -----------------------------------------------
-// One workgroup per (sequence, head, 64 queries); each of its four waves owns 16 queries.  Keys
-// and values go through LDS in tiles of 32 positions, as fp32, the keys rotated on the way; scores and the
-// weighted sum are fp32 matrix products (v_mfma_f32_16x16x4_f32), the same
-// arithmetic type the reference uses (phi.py:98-117).  Both products are formed transposed,
-//   S^T (position x query) = K . Q^T        O^T (feature x query) = V^T . P^T,
-// so that a lane's four score registers are rows 4g .. 4g+3 of one query column: the softmax
-// runs down registers plus two cross-group shuffles, and register r is already the B operand of
-// the second product's k-step r (the A operand then reads value row 4g + r).
-//
-// What bounds it: the fp32 products (a block of 16 positions is 40 of 32 cycles at head width 80: 330 of the 574 us of the largest call
-// below) and, where a workgroup has its CU to itself, the softmax and the widening of the next tile between them.  A tile's rows, and where
-// VEC (the rotated features come in eights) the partners of its keys and their cosines and sines, are asked for a tile ahead, rotated in
-// registers and put into the other half of LDS: one barrier a tile, where there were three with the table's round trip between two of
-// them; the queries likewise, in one round trip instead of twenty.  Operands are read together, two blocks' scores take turns, a
-// head's blocks run on one XCD.  32 heads of 80, us before / now: 100 tokens 18.8 / 13.8, 300 38 / 29, 700 94 / 67, 1500 219 / 157; 2 x 700
-// 114 / 78, 4 x 1500 775 / 574.  With 32 queries a workgroup 73 at 700 tokens and 735 at 4 x 1500, with 128 86 and 572.
-constexpr int PF_Q = 64, PF_T = 32;
+// phi.py:103-104: the pair (i, i + half) of a row, `up` the partner's place; which of a sum's two products is rounded first is fixed, for queries
+// and for keys.
+__device__ __forceinline__ float turned_first(float x, float up, float co, float sn) { return __builtin_fmaf(x, co, -__fmul_rn(up, sn)); }
+__device__ __forceinline__ float turned_query(float x, float down, float co, float sn) { return __builtin_fmaf(x, co, __fmul_rn(down, sn)); }
+__device__ __forceinline__ float turned_key(float x, float down, float co, float sn) { return __builtin_fmaf(down, sn, __fmul_rn(x, co)); }
 
-template <int DT, bool VEC>  // head width / 16
+// The queries q0 + m of a wave with a bit in `which`, one position at a time.  (Sums that are not finite: an infinite key's terms meet zeros in the
+// kernel below, a masked value's infinity a weight of zero.)
+template <int D>
+__device__ __forceinline__ void phi_walk_rows(const PhiAttnArgs& a, int seq, int h, int q0, unsigned int which, int lane) {
+  constexpr int N = (D + 63) / 64;  // features of a lane
+  const int half = a.rot >> 1;
+  const size_t hd = (size_t)a.H * D, at0 = (size_t)seq * a.t_max * hd + (size_t)h * D;
+  const float scale = sqrtf(1.0f / (float)D);
+  auto feature = [&](const bf16_t* row, int position, int j, bool query) {
+    if (j >= D) return 0.f;
+    const float x = bf2f(row[j]);
+    if (j >= a.rot) return x;
+    const float o = bf2f(row[j < half ? j + half : j - half]);
+    const size_t at = (size_t)position * half + (j < half ? j : j - half);
+    const float co = a.cos[at], sn = a.sin[at];
+    return j < half ? turned_first(x, o, co, sn) : query ? turned_query(x, o, co, sn) : turned_key(x, o, co, sn);
+  };
+#pragma unroll 1
+  for (int m = 0; m < 16 && q0 + m < a.S; ++m) {
+    if (!(which >> m & 1)) continue;
+    const size_t row = (size_t)seq * a.S + q0 + m;
+    const int pq = a.pos + q0 + m;
+    float x[N], o[N], top = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      x[i] = feature(a.q + row * a.ldq + h * D, pq, lane + 64 * i, true);
+      o[i] = 0.f;
+    }
+#pragma unroll 1
+    for (int t = 0; t <= pq; ++t) {
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < N; ++i) s = __builtin_fmaf(x[i], feature(a.kc + at0 + (size_t)t * hd, t, lane + 64 * i, false), s);
+      s = wave_sum(s) * scale;
+      const float higher = fmaxf(top, s), corr = top == higher ? 1.0f : __expf(top - higher), p = __expf(s - (higher == -INFINITY ? 0.f : higher));
+      top = higher;
+      l = l * corr + p;
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (lane + 64 * i < D) o[i] = o[i] * corr + p * bf2f(a.vc[at0 + (size_t)t * hd + lane + 64 * i]);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (lane + 64 * i < D) a.out[row * hd + (size_t)h * D + lane + 64 * i] = f2bf(o[i] * (1.0f / l));
+  }
+}
+
+// One workgroup per (sequence, head, 64 queries); each of its four waves owns 16 queries.  Keys and values go through LDS in tiles of 64 positions.
+// The reference computes in fp32 (phi.py:98-117): rotated features and weights are fp32 numbers, cached values and features that are not rotated
+// bf16 ones.  The first are taken apart into three bf16 terms (mfma_frag.h; keys as a tile is put into LDS), and both products are
+// v_mfma_f32_16x16x32_bf16 with fp32 sums: six of the nine products of terms for rotated features (what the other three add lies 2^-27 below), one for
+// the rest, three for weights times values - exact but for the sums.  At head width 80, 32 features rotated, a block of 16 queries x 16 positions is
+// 15.5 such products of 16 cycles, where the fp32 instruction (v_mfma_f32_16x16x4_f32) took 40 of 32.  Both products are formed transposed,
+//   S^T (position x query) = K . Q^T        O^T (feature x query) = V^T . P^T,
+// as in attention_prefill.hip: a lane's scores belong to one query, and are the B operand of the second product where they stand; its A operand is read
+// from rows of values by ds_read_b64_tr_b16.
+//
+// What bounds it: where workgroups have a CU to themselves the longest one's chain of tiles, 2.2 us each, in which products, softmax, the weights' terms and
+// the next tile's keys take turns (putting those among the products changed nothing); where two share it the vector unit, on which the last three
+// are twice the products' cycles.  32 heads of 80, us with fp32 products and tiles of 32 / so: 100 tokens 14.7 / 9.6, 300 30 / 15.5, 700 68 / 28, 1500
+// 157 / 60, 2040 281 / 98; 2 x 700 76 / 33, 4 x 1500 580 / 213; 64 behind 1000 93 / 37.  Results that differ from the rounded ones of 64 bits: 700 tokens
+// 0.030 / 0.019 %, 2040 0.044 / 0.029 %.
+template <int DT, int NR>  // head width / 16; chunks of 32 features with rotated ones among them
+struct PhiTile {
+  static constexpr int D = 16 * DT, NC = (D + 31) / 32;
+  // A key's row: the first terms of the first NR chunks, their second, their third ones, then the other chunks; an odd number of
+  // 16-byte pieces, as sixteen rows' reads want it.  A value's row: an odd number of 32 bytes.
+  static constexpr int PLANE = 64 * NR, KROW = 16 * ((4 * NC + 8 * NR) | 1), VROW = 32 * (DT | 1);
+  // positions: 64 where two workgroups with two tiles each share a CU's LDS (2 x 700 tokens, heads of 128, all rotated: 64 145 us, 32 60)
+  static constexpr int T = 4 * 64 * (KROW + VROW) <= 160 * 1024 ? 64 : 32, BUF = T * (KROW + VROW);
+  static __device__ __forceinline__ constexpr int byte_of(int feature) { return 2 * feature + (feature < 32 * NR ? 0 : 2 * PLANE); }
+};
+template <int DT, int NR>
 __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a, int nqb, int heads) {
+  typedef PhiTile<DT, NR> L;
+  constexpr int D = L::D, NC = L::NC, T = L::T, QB = 64;
+  // a thread's parts of a tile: fours of rotated pairs, eighths of the other features, of values
+  constexpr int NP = (NR * T + 63) / 64, CE = 2 * DT - 4 * NR + 2, NU = CE > 0 ? (CE * T + 255) / 256 : 1, NV = (2 * DT * T + 255) / 256;
+  extern __shared__ __align__(16) unsigned char smem[];  // two tiles
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int half = a.rot >> 1;
+  // an XCD (ids go round-robin over the eight) gets every eighth head; long contexts first
+  const int x8 = blockIdx.x & 7, q8 = blockIdx.x >> 3, nh = (heads + 7) >> 3;
+  const int head = (q8 % nh) * 8 + x8;
+  if (head >= heads) return;
+  const int seq = head / a.H, h = head - seq * a.H;
+  const int s0 = (nqb - 1 - q8 / nh) * QB;
+  const size_t hd = (size_t)a.H * D;
+  const int pos0 = a.pos, wq0 = s0 + 16 * wave;
+  const int t_end = pos0 + min(s0 + QB - 1, a.S - 1);
+  const bf16_t* kb = a.kc + (size_t)seq * a.t_max * hd + (size_t)h * D;
+  const bf16_t* vb = a.vc + (size_t)seq * a.t_max * hd + (size_t)h * D;
+
+  // This thread's part of a tile, asked for a tile ahead: four pairs of rotated features (NP times), eighths of rows of the others and of values.
+  const int quads = half >> 2, eighths = (D - a.rot) >> 3, first = a.rot >> 3;
+  int rp[NP], rf[NP], up[NU], uc[NU];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int idx = tid + 256 * i;
+    rp[i] = idx / quads;
+    rf[i] = 4 * (idx - rp[i] * quads);
+  }
+#pragma unroll
+  for (int i = 0; i < NU; ++i) {
+    const int idx = tid + 256 * i;
+    up[i] = eighths ? idx / eighths : T;
+    uc[i] = eighths ? 8 * (first + idx - up[i] * eighths) : 0;
+  }
+  uint2 k1[NP], k2[NP];
+  uint4 ca[NP], sa[NP], ku[NU], vv[NV];
+  auto fetch = [&](int t0) {  // (past the last position: that one's, masked)
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int t = min(t0 + min(rp[i], T - 1), t_end);
+      const bf16_t* row = kb + (size_t)t * hd + rf[i];
+      k1[i] = ldg8(row);
+      k2[i] = ldg8(row + half);
+      ca[i] = ldg16(a.cos + (size_t)t * half + rf[i]);
+      sa[i] = ldg16(a.sin + (size_t)t * half + rf[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NU; ++i) ku[i] = ldg16(kb + (size_t)min(t0 + min(up[i], T - 1), t_end) * hd + uc[i]);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = min(tid + 256 * i, T * 2 * DT - 1), p = idx / (2 * DT);
+      vv[i] = ldg16(vb + (size_t)min(t0 + p, t_end) * hd + 8 * (idx - p * 2 * DT));
+    }
+  };
+  auto put = [&](unsigned char* tile) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      if (rp[i] >= T) continue;
+      const float x[4] = {lo_bf(k1[i].x), hi_bf(k1[i].x), lo_bf(k1[i].y), hi_bf(k1[i].y)};
+      const float y[4] = {lo_bf(k2[i].x), hi_bf(k2[i].x), lo_bf(k2[i].y), hi_bf(k2[i].y)};
+      const uint32_t cw[4] = {ca[i].x, ca[i].y, ca[i].z, ca[i].w}, sw[4] = {sa[i].x, sa[i].y, sa[i].z, sa[i].w};
+      float lo[4], hi[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float co = __uint_as_float(cw[u]), sn = __uint_as_float(sw[u]);
+        lo[u] = turned_first(x[u], y[u], co, sn);
+        hi[u] = turned_key(y[u], x[u], co, sn);
+      }
+      bf16_t* at = reinterpret_cast<bf16_t*>(tile + rp[i] * L::KROW) + rf[i];
+      WideLds<bf16_t>::put4(at, L::PLANE / 2, lo);
+      WideLds<bf16_t>::put4(at + half, L::PLANE / 2, hi);
+    }
+#pragma unroll
+    for (int i = 0; i < NU; ++i)
+      if (up[i] < T) *reinterpret_cast<uint4*>(tile + up[i] * L::KROW + L::byte_of(uc[i])) = ku[i];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + 256 * i, p = idx / (2 * DT);
+      if (idx < T * 2 * DT) *reinterpret_cast<uint4*>(tile + T * L::KROW + p * L::VROW + 16 * (idx - p * 2 * DT)) = vv[i];
+    }
+  };
+
+  // This lane's query (those beyond the call's tokens repeat the last one and are not stored), eighths g of its chunks.
+  const int sq = min(wq0 + l16, a.S - 1), pq = pos0 + sq;
+  Wide<bf16_t> qw[NR];
+  uint4 qf[NC > NR ? NC - NR : 1];
+  {
+    const bf16_t* row = a.q + ((size_t)seq * a.S + sq) * a.ldq + h * D;
+    uint4 x[NC], o[NR], c0[NR], c1[NR], n0[NR], n1[NR];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int f = 32 * c + 8 * g;
+      x[c] = ldg16(row + min(f, D - 8));
+      if (c < NR) {
+        const bool rotated = f < a.rot, low = f < half;
+        const size_t at = (size_t)pq * half + (rotated ? (low ? f : f - half) : 0);
+        o[c] = ldg16(row + (rotated ? (low ? f + half : f - half) : 0));
+        c0[c] = ldg16(a.cos + at);
+        c1[c] = ldg16(a.cos + at + 4);
+        n0[c] = ldg16(a.sin + at);
+        n1[c] = ldg16(a.sin + at + 4);
+      }
+    }
+    fetch(0);
+    // what no tile's part is put on: features past the head, second and third terms of those that are not rotated
+    for (int i = tid; i < 2 * T * (L::KROW / 16); i += 256) {
+      const int r = i / (L::KROW / 16);
+      *reinterpret_cast<uint4*>(smem + (r / T) * L::BUF + (r % T) * L::KROW + 16 * (i - r * (L::KROW / 16))) = make_uint4(0, 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int f = 32 * c + 8 * g;
+      const uint32_t xw[4] = {x[c].x, x[c].y, x[c].z, x[c].w};
+      if (c < NR) {
+        const uint32_t ow[4] = {o[c].x, o[c].y, o[c].z, o[c].w};
+        const uint32_t cw[8] = {c0[c].x, c0[c].y, c0[c].z, c0[c].w, c1[c].x, c1[c].y, c1[c].z, c1[c].w};
+        const uint32_t sw[8] = {n0[c].x, n0[c].y, n0[c].z, n0[c].w, n1[c].x, n1[c].y, n1[c].z, n1[c].w};
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const float y = u & 1 ? hi_bf(xw[u / 2]) : lo_bf(xw[u / 2]), z = u & 1 ? hi_bf(ow[u / 2]) : lo_bf(ow[u / 2]);
+          const float co = __uint_as_float(cw[u]), sn = __uint_as_float(sw[u]);
+          v[u] = f < half ? turned_first(y, z, co, sn) : f < a.rot ? turned_query(y, z, co, sn) : f < D ? y : 0.f;
+        }
+        wide_from(qw[c], v);
+      } else {
+        qf[c - NR] = f < D ? x[c] : make_uint4(0, 0, 0, 0);
+      }
+    }
+  }
+  __syncthreads();
+  put(smem);
+  __syncthreads();
+
+  const int wave_hi = pos0 + min(wq0 + 15, a.S - 1);  // last position any query of the wave sees
+  const float mul = sqrtf(1.0f / (float)D) * OHARA_LOG2E;
+  f32x4 o[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t) o[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, lsum = 0.f;
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
+  const uint32_t kat = l16 * L::KROW + g * 16;                                      // keys of positions 16 b + l16
+  const uint32_t vat = T * L::KROW + (4 * g + (l16 >> 2)) * L::VROW + (l16 & 3) * 8;  // values, as ds_read_b64_tr_b16 takes them
+  auto window = [&](auto count, int t0, uint32_t kat, uint32_t vat) {  // 32 positions of a tile, or all of it
+    constexpr int NW = decltype(count)::value, NB = 2 * NW;
+    uint4 kf[NB][NC + 2 * NR];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int c = 0; c < NC + 2 * NR; ++c) kf[b][c] = lds16_at(kat + b * (16 * L::KROW) + c * 64);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 s[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) s[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    auto add = [&](int piece, uint4 q) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) s[b] = mma_bf(kf[b][piece], q, s[b]);
+    };
+#pragma unroll
+    for (int c = 0; c < NR; ++c) {
+      add(2 * NR + c, qw[c].t[0]);
+      add(NR + c, qw[c].t[1]);
+      add(c, qw[c].t[2]);
+      add(NR + c, qw[c].t[0]);
+      add(c, qw[c].t[1]);
+    }
+#pragma unroll
+    for (int c = 0; c < NR; ++c) add(c, qw[c].t[0]);
+#pragma unroll
+    for (int c = NR; c < NC; ++c) add(2 * NR + c, qf[c - NR]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (t0 + 16 * NB - 1 > pos0 + wq0) {  // (uniform) not every query of the wave sees all of it
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (t0 + 16 * b + 4 * g + r > pq) s[b][r] = -INFINITY;
+    }
+    float mx = s[0][0];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[b][r]);
+    mx = lane_xor_max<32>(lane_xor_max<16>(mx));
+    const float mn = fmaxf(m, ceilf(mx * mul));  // a whole number: what is rescaled is rescaled exactly, and seldom
+    const float corr = pow2_neg_int(m - mn), off = mn == -INFINITY ? 0.f : mn;
+    m = mn;
+    Wide<bf16_t> pf[NW];
+    float ps = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      float p[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * w + i / 4][i % 4], mul, -off));
+        ps += p[i];
+      }
+      wide_from(pf[w], p);
+    }
+    lsum = lsum * corr + ps;
+    if (__any(corr != 1.0f)) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[t][r] *= corr;
+    }
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      uint4 vf[DT];
+#pragma unroll
+      for (int t = 0; t < DT; ++t) {
+        const uint32_t at = vat + w * (32 * L::VROW) + t * 32;
+        const uint2 lo = lds_tr8(at), hi = lds_tr8(at + 16 * L::VROW);
+        vf[t] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 2; i >= 0; --i)
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[t] = mma_bf(vf[t], pf[w].t[i], o[t]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  constexpr bool BOTH = T == 64 && NC + 2 * NR <= 5;  // (more fragments than that do not fit)
+  uint32_t cur = 0;
+  for (int t0 = 0; t0 <= t_end; t0 += T) {
+    const bool more = t0 + T <= t_end;
+    if (more) fetch(t0 + T);  // in flight during this tile's products
+    const uint32_t kt = lds0 + cur + kat, vt = lds0 + cur + vat;
+    if (BOTH && t0 + 32 <= wave_hi) {
+      window(std::integral_constant<int, 2>(), t0, kt, vt);
+    } else {
+      if (t0 <= wave_hi) window(std::integral_constant<int, 1>(), t0, kt, vt);
+      if (!BOTH && T == 64 && t0 + 32 <= wave_hi) window(std::integral_constant<int, 1>(), t0 + 32, kt + 32 * L::KROW, vt + 32 * L::VROW);
+    }
+    cur = L::BUF - cur;
+    if (more) put(smem + cur);
+    __syncthreads();
+  }
+  lsum = lane_xor_sum<32>(lane_xor_sum<16>(lsum));
+  float sum = lsum;
+#pragma unroll
+  for (int t = 0; t < DT; ++t) sum += (o[t][0] + o[t][1]) + (o[t][2] + o[t][3]);
+  const unsigned int odd = columns_not_finite(sum);
+  if (wq0 + l16 < a.S && !(odd >> l16 & 1)) {
+    const float inv = 1.0f / lsum;
+    bf16_t* orow = a.out + ((size_t)seq * a.S + sq) * hd + (size_t)h * D + 4 * g;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+      *reinterpret_cast<uint2*>(orow + 16 * t) =
+          make_uint2(pack_bf(o[t][0] * inv, o[t][1] * inv), pack_bf(o[t][2] * inv, o[t][3] * inv));
+  }
+  if (odd) phi_walk_rows<D>(a, seq, h, wq0, odd, lane);
+}
+
+// Features rotated in other numbers than eights, or tables off 16 bytes: keys and values in LDS as fp32, the keys rotated there, in tiles of 32 positions;
+// both products fp32 ones.
+constexpr int PF_Q = 64, PF_T = 32;
+template <int DT>  // head width / 16
+__global__ __launch_bounds__(256, 2) void phi_attn_pairs_kernel(PhiAttnArgs a, int nqb, int heads) {
   constexpr int D = 16 * DT, LD = D + 4, C8 = D / 8, NV = (PF_T * C8 + 255) / 256;
   constexpr int BUF = 2 * PF_T * LD;  // floats: keys | values of a tile
   extern __shared__ __align__(16) float sm[];  // two of them; the rotated queries before the loop
@@ -131,26 +457,6 @@ __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a,
   const size_t hd = (size_t)a.H * D;
   const int pos0 = a.pos;
 
-  // An eighth of a row: features 8 c .. 8 c + 7; of a rotated one the partners start at feature `partner`, the angles at `angle`.
-  struct Eighth {
-    uint4 x, p, c0, c1, s0, s1;
-  };
-  auto load8 = [&](const bf16_t* row, int position, int c) {
-    Eighth e;
-    e.x = ldg16(row + 8 * c);
-    if (VEC) {
-      const bool lo = 8 * c < half, rotated = 8 * c < a.rot;
-      const int partner = rotated ? (lo ? 8 * c + half : 8 * c - half) : 8 * c, angle = rotated ? (lo ? 8 * c : 8 * c - half) : 0;
-      e.p = ldg16(row + partner);
-      const float* cp = a.cos + (size_t)position * half + angle;
-      const float* sp = a.sin + (size_t)position * half + angle;
-      e.c0 = ldg16(cp);
-      e.c1 = ldg16(cp + 4);
-      e.s0 = ldg16(sp);
-      e.s1 = ldg16(sp + 4);
-    }
-    return e;
-  };
   auto widen = [](uint4 v, float (&f)[8]) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -159,45 +465,12 @@ __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a,
       f[2 * i + 1] = hi_bf(w[i]);
     }
   };
-  // phi.py:103-104: the pair (i, i + half); which of a sum's two products is rounded first is fixed, for queries and for keys
-  auto turned = [&](const Eighth& e, int c, float (&f)[8], bool query) {
-    widen(e.x, f);
-    if (VEC && 8 * c < a.rot) {
-      float o8[8];
-      widen(e.p, o8);
-      const uint32_t cw[8] = {e.c0.x, e.c0.y, e.c0.z, e.c0.w, e.c1.x, e.c1.y, e.c1.z, e.c1.w};
-      const uint32_t sw[8] = {e.s0.x, e.s0.y, e.s0.z, e.s0.w, e.s1.x, e.s1.y, e.s1.z, e.s1.w};
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const float co = __uint_as_float(cw[u]), sn = __uint_as_float(sw[u]);
-        f[u] = 8 * c < half ? __builtin_fmaf(f[u], co, -__fmul_rn(o8[u], sn)) : (query ? __builtin_fmaf(f[u], co, __fmul_rn(o8[u], sn)) : __builtin_fmaf(o8[u], sn, __fmul_rn(f[u], co)));
-      }
-    }
-  };
   auto put8 = [](float* dst, const float (&f)[8], bool in) {
     *reinterpret_cast<float4*>(dst) = in ? make_float4(f[0], f[1], f[2], f[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
     *reinterpret_cast<float4*>(dst + 4) = in ? make_float4(f[4], f[5], f[6], f[7]) : make_float4(0.f, 0.f, 0.f, 0.f);
   };
 
   // rotated queries -> LDS -> registers (rows beyond the call's tokens are zero)
-  if (VEC) {
-    constexpr int NQ = PF_Q * C8 / 256 + (PF_Q * C8 % 256 ? 1 : 0);
-    Eighth e[NQ];
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      const int idx = min(tid + 256 * i, PF_Q * C8 - 1), qi = idx / C8, sq = min(s0 + qi, a.S - 1);
-      e[i] = load8(a.q + ((size_t)seq * a.S + sq) * a.ldq + h * D, pos0 + sq, idx - qi * C8);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      const int idx = tid + 256 * i, qi = idx / C8, c = idx - qi * C8;
-      if (qi >= PF_Q) continue;
-      float f[8];
-      turned(e[i], c, f, true);
-      put8(sm + qi * LD + 8 * c, f, s0 + qi < a.S);
-    }
-  } else
   for (int idx = tid; idx < PF_Q * D; idx += 256) {
     const int qi = idx / D, j = idx - qi * D;
     const int sq = s0 + qi;
@@ -232,8 +505,7 @@ __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a,
   float m = -INFINITY, lsum = 0.f;
 
   // this thread's eighths of a tile's rows
-  Eighth kr[NV];
-  uint4 vr[NV];
+  uint4 kr[NV], vr[NV];
   auto place = [&](int i, int& p, int& c) {
     const int idx = tid + 256 * i;
     p = idx / C8;
@@ -245,7 +517,7 @@ __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a,
       int p, c;
       place(i, p, c);
       const int t = min(t0 + min(p, PF_T - 1), t_end);
-      kr[i] = load8(kb + (size_t)t * hd, t, c);
+      kr[i] = ldg16(kb + (size_t)t * hd + 8 * c);
       vr[i] = ldg16(vb + (size_t)t * hd + 8 * c);
     }
   };
@@ -256,7 +528,7 @@ __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a,
       place(i, p, c);
       if (p >= PF_T) continue;
       float k[8], v[8];
-      turned(kr[i], c, k, false);
+      widen(kr[i], k);
       widen(vr[i], v);
       put8(ks + p * LD + 8 * c, k, t0 + p <= t_end);
       put8(ks + PF_T * LD + p * LD + 8 * c, v, t0 + p <= t_end);
@@ -270,19 +542,17 @@ __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a,
   for (int t0 = 0; t0 <= t_end; t0 += PF_T) {
     const bool more = t0 + PF_T <= t_end;
     if (more) fetch(t0 + PF_T);  // in flight during this tile's products
-    if (!VEC) {
-      // rotate the tile's keys in place: pair (i, i + half) of every position
-      for (int idx = tid; idx < PF_T * half; idx += 256) {
-        const int p = idx / half, i = idx - p * half;
-        if (t0 + p <= t_end) {
-          const float c = a.cos[(size_t)(t0 + p) * half + i], sn = a.sin[(size_t)(t0 + p) * half + i];
-          const float k1 = ks[p * LD + i], k2 = ks[p * LD + i + half];
-          ks[p * LD + i] = k1 * c - k2 * sn;
-          ks[p * LD + i + half] = k1 * sn + k2 * c;
-        }
+    // rotate the tile's keys in place: pair (i, i + half) of every position
+    for (int idx = tid; idx < PF_T * half; idx += 256) {
+      const int p = idx / half, i = idx - p * half;
+      if (t0 + p <= t_end) {
+        const float c = a.cos[(size_t)(t0 + p) * half + i], sn = a.sin[(size_t)(t0 + p) * half + i];
+        const float k1 = ks[p * LD + i], k2 = ks[p * LD + i + half];
+        ks[p * LD + i] = k1 * c - k2 * sn;
+        ks[p * LD + i + half] = k1 * sn + k2 * c;
       }
-      __syncthreads();
     }
+    __syncthreads();
     const float* vs = ks + PF_T * LD;
     if (t0 <= wave_hi) {  // (wave-uniform: else nothing of the tile is visible to the wave's queries)
       // operands are read together before the products (left to itself, the compiler waits for each), and the two blocks' chains of
@@ -354,13 +624,21 @@ __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a,
 
 template <int DT>
 int launch_phi_prefill(const PhiAttnArgs& a, int batch, hipStream_t st) {
-  constexpr int LDS = 2 * 2 * PF_T * (16 * DT + 4) * (int)sizeof(float);
   const int64_t nqb = (a.S + PF_Q - 1) / PF_Q, heads = (int64_t)a.H * batch, grid = nqb * ((heads + 7) / 8 * 8);
   if (grid > INT32_MAX) return OHARA_ESIZE;
-  auto kernel = phi_eights(a) ? phi_attn_prefill_kernel<DT, true> : phi_attn_prefill_kernel<DT, false>;
-  if (LDS > 64 * 1024) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), LDS, st, a, (int)nqb, (int)heads);
-  return ohara_launch_status();
+  auto launch = [&](auto kernel, int lds) {
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), lds, st, a, (int)nqb, (int)heads);
+    return ohara_launch_status();
+  };
+  if (!phi_eights(a)) return launch(phi_attn_pairs_kernel<DT>, 2 * 2 * PF_T * (16 * DT + 4) * (int)sizeof(float));
+  constexpr int NC = (DT + 1) / 2;  // a.rot is at most 16 DT
+  switch ((a.rot + 31) / 32) {
+    case 1: return launch(phi_attn_prefill_kernel<DT, 1>, 2 * PhiTile<DT, 1>::BUF);
+    case 2: return launch(phi_attn_prefill_kernel<DT, NC < 2 ? NC : 2>, 2 * PhiTile<DT, NC < 2 ? NC : 2>::BUF);
+    case 3: return launch(phi_attn_prefill_kernel<DT, NC < 3 ? NC : 3>, 2 * PhiTile<DT, NC < 3 ? NC : 3>::BUF);
+    default: return launch(phi_attn_prefill_kernel<DT, NC < 4 ? NC : 4>, 2 * PhiTile<DT, NC < 4 ? NC : 4>::BUF);
+  }
 }
 
 }  // namespace
@@ -404,7 +682,7 @@ int ohara_phi_attn_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, cons
   if (rc) return rc;
   if (seq_len >= 16 && !pos_dev && (dh == 16 || dh == 32 || dh == 64 || dh == 80 || dh == 128) && h <= 65535 &&
       batch <= 65535) {
-    // many new tokens: queries in tiles of 64 against key / value tiles in LDS, fp32 matrix products
+    // many new tokens: queries in tiles of 64 against key / value tiles in LDS
     switch (dh / 16) {
       case 1: return launch_phi_prefill<1>(a, batch, (hipStream_t)stream);
       case 2: return launch_phi_prefill<2>(a, batch, (hipStream_t)stream);
