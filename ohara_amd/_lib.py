@@ -136,6 +136,7 @@ _PROTOS = {
     "ohara_gemm_skinny_bf16": (_i, [_p, _i, _p, _i, _i, _p, _f, _i, _i, _p, _i, _p, _i, _p]),
     "ohara_projection_norm_ahead": (_i, [_i, _i, _i]),
     "ohara_gemm_tile_of": (_i, [_i, _i, _i]),
+    "ohara_gemm_tile_with": (_i, [_i, _i, _i, _i, _i]),
     "ohara_gemm_first_rows": (_i, [_i, _i, _i, _i, _i]),
     "ohara_gemm_bf16": (_i, [_p, _i, _p, _i, _i, _i, _i, _p, _i, _p, _i, _p]),
     "ohara_qkv_rope_append_bf16": (_i, [_p, _i, _p, _i, _p, _f, _i, _i, _i, _i, _i, _p, _p, _i, _p, _p, _p, _p, _i, _p]),

@@ -376,6 +376,16 @@ typedef Tile<2, 4, 4, 2, 2, 2, 0> T128;
 typedef Tile<2, 4, 4, 3, 2, 2, 0> T128x192;
 typedef Tile<4, 1, 1, 3, 4, 3, 1> T64x48;
 typedef Tile<2, 2, 2, 3, 4, 3, 0> T64x96;
+// For fewer than 1024 rows, mostly a CU to themselves (few_rows_tile)
+typedef Tile<1, 4, 3, 1, 4, 3, 0> T48x64;
+typedef Tile<1, 4, 5, 1, 4, 3, 0> T80x64;
+typedef Tile<2, 2, 3, 2, 2, 3, 0> T96x64;
+typedef Tile<2, 2, 3, 3, 4, 3, 0> T96;
+typedef Tile<2, 2, 4, 3, 2, 3, 0> T128x96;
+typedef Tile<2, 2, 2, 2, 4, 3, 0> W64;       // as T64, T128 and T128x192, a slot more
+typedef Tile<2, 4, 4, 2, 2, 3, 0> W128;
+typedef Tile<2, 4, 4, 3, 2, 3, 0> W128x192;
+typedef Tile<2, 4, 6, 2, 2, 3, 0> T192x128;
 typedef HalvesTile<2, 4, 8, 4, 1, 3, 4> T256;
 typedef HalvesTile<2, 4, 4, 4, 2, 3, 3> H128x256;
 typedef HalvesTile<2, 4, 4, 3, 2, 3, 3> H128x192;
@@ -484,6 +494,45 @@ int fastest_tile(int rows, int strips, int K, Epilogue epi = PLAIN) {
   return best;
 }
 
+// Fewer than 1024 rows are a round or two of tiles, and what decides is whether they are one: 192 rows 11264 x 2048 were 264 tiles of 64 x 128, eight CUs with
+// two, 22.1 us, and are 236 of 96 x 96, 18.2.  So there are tiles of more sizes, a ring of three slots each.  The times below are fitted to 1224 products
+// (17 of a model's widths and depths whole, 8 in parts; 33 to 1023 rows; each tile that makes 48 to 1600 workgroups; cold weights), those of a
+// tile alone on its CU within 3 to 5 %, of those that share one within 7 to 12 %.  Such a tile is taken where they promise 4 % (10 with an arithmetic
+// epilogue, whose waves hold more of it): of the 1201 products with a choice 340 change, 12 % quicker on average (as much as 30), 21 lose more than 3 %, the worst 9
+// (768 x 3072 in two parts, 860 rows: 10.7 / 11.7).  us, before / now: 224 rows 11264 x 2048 with SwiGLU 26.7 / 21.1, 320 rows 3072 x 2048 14.9 / 11.4, 1000 rows
+// 27.7 / 20.4, 400 rows 15.4 / 13.1.  A plain store keeps the tiles above: no model has one but for its vocabulary, whose rounds are many.
+constexpr int NEW_TILES = 10;  // the first of these tiles
+constexpr TileTime FEW[19] = {
+    {T32::TM, T32::TS, 3, 0.147f, 0.412f, 0.081f, 0.482f},          {T64::TM, T64::TS, 2, 0.302f, 0.252f, 0.208f, 0.779f},
+    {T64x128::TM, T64x128::TS, 2, 0.374f, 0.684f, 0.337f, 1.577f},  {T128::TM, T128::TS, 2, 0.637f, 0.476f, 0.563f, 1.948f},
+    {T128x192::TM, T128x192::TS, 2, 0.756f, 0.68f, 0.68f, 3.227f},  {T256::TM, T256::TS, 1, 1.35f, 0.f, 1.6f, 6.7f},
+    {H128x256::TM, H128x256::TS}, {H128x192::TM, H128x192::TS},     // (not among them)
+    {T64x48::TM, T64x48::TS, 1, 0.195f, 0.254f, 0.228f, 1.248f},    {T64x96::TM, T64x96::TS, 1, 0.287f, 0.234f, 0.336f, 1.634f},
+    {T48x64::TM, T48x64::TS, 1, 0.199f, 0.191f, 0.231f, 1.229f},    {T80x64::TM, T80x64::TS, 1, 0.261f, 0.193f, 0.302f, 1.51f},
+    {T96x64::TM, T96x64::TS, 2, 0.358f, 0.406f, 0.256f, 1.253f},    {T96::TM, T96::TS, 1, 0.355f, 0.242f, 0.426f, 1.968f},
+    {T128x96::TM, T128x96::TS, 1, 0.441f, 0.181f, 0.507f, 2.426f},  {W64::TM, W64::TS, 1, 0.23f, 0.19f, 0.264f, 1.314f},
+    {W128::TM, W128::TS, 1, 0.468f, 0.247f, 0.592f, 2.966f},        {W128x192::TM, W128x192::TS, 1, 0.599f, 0.262f, 0.758f, 4.159f},
+    {T192x128::TM, T192x128::TS, 1, 0.6f, 0.25f, 0.764f, 4.011f},
+};
+int few_rows_tile(int rows, int strips, int K, Epilogue epi) {
+  const int now = fastest_tile(rows, strips, K, epi);
+  if (rows >= 1024) return now;
+  int best = now;
+  float low = (epi == HEAVY ? 0.9f : 0.96f) * tile_time(FEW[now], rows, strips, K);
+  for (int i = NEW_TILES; i < 19; ++i) {
+    const float t = tile_time(FEW[i], rows, strips, K);
+    if (t < low) {
+      low = t;
+      best = i;
+    }
+  }
+  return best;
+}
+constexpr bool has_new_tiles(int epi) { return epi == EPI_RESIDUAL || epi == EPI_SWIGLU || epi == EPI_ROPE || epi == EPI_PHI_IN; }
+int tile_of(int rows, int strips, int K, int epi, Epilogue kind) {
+  return has_new_tiles(epi) ? few_rows_tile(rows, strips, K, kind) : fastest_tile(rows, strips, K, kind);
+}
+
 // A part of the rows in whole rounds of 256 x 256, one a CU, and the rest by itself, where the last round would be nearly empty (0 rows: all in one launch).
 // The times of two launches are those above, added, and 5 us for the second one's start; taken from 3 % on.  us, one / two launches: 8192 rows 2304 x 768 with
 // rotary 43.9 / 41.7, heads of 64 43.4 / 39.1, 16384 rows 79.0 / 72.3, 5500 rows 6144 x 768 with SwiGLU 59.8 / 53.9, 5421 rows 2992 x 2560 99.4 / 81.8, 8192 rows
@@ -505,6 +554,20 @@ int split_rows(int rows, int strips, int K, Epilogue epi) {
 
 template <int EPI>
 int launch_of(int tile, const GemmArgs& a, int nstrips, hipStream_t st) {
+  if constexpr (has_new_tiles(EPI)) {
+    switch (tile) {
+      case 10: return launch_tile<EPI, T48x64>(a, nstrips, st);
+      case 11: return launch_tile<EPI, T80x64>(a, nstrips, st);
+      case 12: return launch_tile<EPI, T96x64>(a, nstrips, st);
+      case 13: return launch_tile<EPI, T96>(a, nstrips, st);
+      case 14: return launch_tile<EPI, T128x96>(a, nstrips, st);
+      case 15: return launch_tile<EPI, W64>(a, nstrips, st);
+      case 16: return launch_tile<EPI, W128>(a, nstrips, st);
+      case 17: return launch_tile<EPI, W128x192>(a, nstrips, st);
+      case 18: return launch_tile<EPI, T192x128>(a, nstrips, st);
+      default: break;
+    }
+  }
   switch (tile) {
     case 0: return launch_tile<EPI, T32>(a, nstrips, st);
     case 1: return launch_tile<EPI, T64>(a, nstrips, st);
@@ -523,7 +586,7 @@ int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
   if (((uintptr_t)a.x & 15) != 0 || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return launch_tile<EPI, T64, false>(a, nstrips, st);
   const Epilogue epi = epilogue_of(EPI, a.Dh, a.stage);
   const int split = split_rows(a.B, nstrips, a.K, epi);
-  if (!split) return launch_of<EPI>(fastest_tile(a.B, nstrips, a.K, epi), a, nstrips, st);
+  if (!split) return launch_of<EPI>(tile_of(a.B, nstrips, a.K, EPI, epi), a, nstrips, st);
   GemmArgs first = a, rest = a;
   first.B = split;
   rest.B = a.B - split;
@@ -536,7 +599,7 @@ int launch_epi(const GemmArgs& a, int nstrips, hipStream_t st) {
     if (a.ids) rest.ids += split;
   }
   const int rc = launch_of<EPI>(LARGEST, first, nstrips, st);
-  return rc ? rc : launch_of<EPI>(fastest_tile(rest.B, nstrips, a.K, epi), rest, nstrips, st);
+  return rc ? rc : launch_of<EPI>(tile_of(rest.B, nstrips, a.K, EPI, epi), rest, nstrips, st);
 }
 
 float least_time(int rows, int strips, int K) {
@@ -575,7 +638,7 @@ int ohara_depth_parts(int rows, int packed_rows, int k, float merge_us) {
 int ohara_launch_gemm_parts(const GemmArgs& a, int packed_rows, int parts, float* sums, hipStream_t st) {
   const int nstrips = packed_rows / 16;
   if (parts < 2 || a.K % (128 * parts) || ((uintptr_t)a.x & 15) || (a.ldx & 7) || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return OHARA_EINVAL;
-  switch (fastest_tile(a.B, nstrips * parts, a.K / parts)) {
+  switch (few_rows_tile(a.B, nstrips * parts, a.K / parts, PLAIN)) {
     case 0: return launch_part<T32>(a, nstrips, parts, sums, st);
     case 1: return launch_part<T64>(a, nstrips, parts, sums, st);
     case 2: return launch_part<T64x128>(a, nstrips, parts, sums, st);
@@ -585,7 +648,16 @@ int ohara_launch_gemm_parts(const GemmArgs& a, int packed_rows, int parts, float
     case 6: return launch_part<H128x256>(a, nstrips, parts, sums, st);
     case 7: return launch_part<H128x192>(a, nstrips, parts, sums, st);
     case 8: return launch_part<T64x48>(a, nstrips, parts, sums, st);
-    default: return launch_part<T64x96>(a, nstrips, parts, sums, st);
+    case 9: return launch_part<T64x96>(a, nstrips, parts, sums, st);
+    case 10: return launch_part<T48x64>(a, nstrips, parts, sums, st);
+    case 11: return launch_part<T80x64>(a, nstrips, parts, sums, st);
+    case 12: return launch_part<T96x64>(a, nstrips, parts, sums, st);
+    case 13: return launch_part<T96>(a, nstrips, parts, sums, st);
+    case 14: return launch_part<T128x96>(a, nstrips, parts, sums, st);
+    case 15: return launch_part<W64>(a, nstrips, parts, sums, st);
+    case 16: return launch_part<W128>(a, nstrips, parts, sums, st);
+    case 17: return launch_part<W128x192>(a, nstrips, parts, sums, st);
+    default: return launch_part<T192x128>(a, nstrips, parts, sums, st);
   }
 }
 
@@ -613,6 +685,13 @@ extern "C" int ohara_gemm_tile_of(int rows, int packed_rows, int k) {
   if (rows < 1 || packed_rows < 1 || k < 1) return OHARA_EINVAL;
   const TileTime& t = MANY[fastest_tile(rows, (packed_rows + 15) / 16, k)];  // (its sizes are those of both)
   return t.rows * 1000 + t.strips * 16;
+}
+
+extern "C" int ohara_gemm_tile_with(int rows, int packed_rows, int k, int epilogue, int parts) {
+  if (rows < 1 || packed_rows < 1 || k < 1 || epilogue < EPI_STORE || epilogue > EPI_BIAS_XIELU || parts < 1 || k % parts) return OHARA_EINVAL;
+  const int strips = (packed_rows + 15) / 16;
+  const int i = parts > 1 ? few_rows_tile(rows, strips * parts, k / parts, PLAIN) : tile_of(rows, strips, k, epilogue, epilogue_of(epilogue, 64, false));
+  return FEW[i].rows * 1000 + FEW[i].strips * 16;
 }
 
 extern "C" int ohara_gemm_first_rows(int rows, int packed_rows, int k, int epilogue, int dh) {
