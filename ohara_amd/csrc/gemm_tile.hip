@@ -24,29 +24,24 @@
 
 namespace {
 
-// ALIGNED: activation rows start on 16 bytes and a tile of them spans less than 4 GiB (false: through registers, any)
-template <int EPI, class C, bool ALIGNED>
-__global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, int MT, int NT, int nstrips) {
-  constexpr int FM = C::FM, FN = C::FN, GM = 8;
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int T = MT * NT;
-  const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
-  const int base = T >> 3, rem = T & 7;
-  if (q >= base + (xcd < rem ? 1 : 0)) return;
-  const int pid = xcd * base + min(xcd, rem) + q;
-  const int grp = pid / (GM * NT), first = grp * GM, gsz = min(GM, MT - first), r = pid - grp * GM * NT;
-  const int row0 = (first + r % gsz) * C::TM, strip0 = (r / gsz) * C::TS;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / C::WN, wn = wave % C::WN;
-  const int m = lane & 15, g = lane >> 4;
-  XOffsets<C, ALIGNED> x;
-#pragma unroll
-  for (int i = 0; i < C::XPW; ++i) x.set(i, wave, lane, (typename XOffsets<C, ALIGNED>::type)(min(row0 + x.row(i, wave, lane), a.B - 1) - row0) * a.ldx);
-  f32x4 acc[FN][FM];
-  tile_product<C, ALIGNED>(acc, reinterpret_cast<const char*>(a.x + (size_t)row0 * a.ldx), x, a.wp, strip0, nstrips, a.K, wave, lane, smem);
-  const int rbase = row0 + wm * FM * 16, sbase = strip0 + wn * FN;
+constexpr int CUS = 256;
 
+// Tile `pid` of a run: eight activation tiles side by side.
+struct TilePlace {
+  int row0, strip0;
+};
+template <class C>
+__device__ __forceinline__ TilePlace tile_place(int pid, int MT, int NT) {
+  constexpr int GM = 8;
+  const int grp = pid / (GM * NT), first = grp * GM, gsz = min(GM, MT - first), r = pid - grp * GM * NT;
+  return {(first + r % gsz) * C::TM, (r / gsz) * C::TS};
+}
+
+// What a wave does with its sums: rows rbase + 16 t + (lane & 15), strips sbase + u.
+template <int EPI, class C>
+__device__ __forceinline__ void tile_epilogue(const GemmArgs& a, const f32x4 (&acc)[C::FN][C::FM], int rbase, int sbase, int nstrips, int lane) {
+  constexpr int FM = C::FM, FN = C::FN;
+  const int m = lane & 15, g = lane >> 4;
   // A thread finishes FM * FN fragments.  What their epilogues read (residual rows, biases, rotary
   // values) is fetched for a strip's before the first is used, instead of one dependent round trip
   // per fragment.
@@ -316,10 +311,81 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
   }
 }
 
+// ALIGNED: activation rows start on 16 bytes and a tile of them spans less than 4 GiB (false: through registers, any)
+template <int EPI, class C, bool ALIGNED>
+__global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, int MT, int NT, int nstrips) {
+  constexpr int FM = C::FM, FN = C::FN;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int T = MT * NT;
+  const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+  const int base = T >> 3, rem = T & 7;
+  if (q >= base + (xcd < rem ? 1 : 0)) return;
+  const auto [row0, strip0] = tile_place<C>(xcd * base + min(xcd, rem) + q, MT, NT);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  XOffsets<C, ALIGNED> x;
+#pragma unroll
+  for (int i = 0; i < C::XPW; ++i) x.set(i, wave, lane, (typename XOffsets<C, ALIGNED>::type)(min(row0 + x.row(i, wave, lane), a.B - 1) - row0) * a.ldx);
+  f32x4 acc[FN][FM];
+  tile_product<C, ALIGNED>(acc, reinterpret_cast<const char*>(a.x + (size_t)row0 * a.ldx), x, a.wp, strip0, nstrips, a.K, wave, lane, smem);
+  tile_epilogue<EPI, C>(a, acc, row0 + wave / C::WN * FM * 16, strip0 + wave % C::WN * FN, nstrips, lane);
+}
+
+// A workgroup a CU, which takes every 32nd tile of its XCD's run, where there are more tiles than CUs.  Its loads run from one tile into the next: what
+// halves_stream asks for in a tile's last steps are the first steps of the one behind it, which arrive under the epilogue.
+// us, a workgroup a tile / this: 8192 rows 6144 x 768 with SwiGLU 77.8 / 73.2, plain 77.2 / 73.3, 384 deep 55.8 / 48.6; 4001 rows 11264 x 2048 with SwiGLU 151 /
+// 144, 11200 rows 399 / 377; 8192 rows 7680 x 2560 237 / 233.  What is left of a boundary there, 8 of 24 us a tile: the epilogue's arithmetic (SwiGLU 4 us), or where
+// much is stored the memory (100 MB of a plain store 16.6 of 72.3 us); zeros instead of random numbers 53 us: the chip's clock under its load.
+template <int EPI, class C>
+__global__ __launch_bounds__(C::NW * 64, 2) void gemm_rounds_kernel(GemmArgs a, int MT, int NT, int nstrips) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int T = MT * NT, xcd = blockIdx.x & 7, base = T >> 3, rem = T & 7;
+  const int first = xcd * base + min(xcd, rem), run = base + (xcd < rem ? 1 : 0), step = gridDim.x >> 3;
+  int q = blockIdx.x >> 3;
+  if (q >= run) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  HalvesStream<C> stream(a.wp, a.K, nstrips, wave, lane, smem);
+  auto where = [&](TilePlace p) {  // the loads' place
+    XOffsets<C, true> x;
+#pragma unroll
+    for (int i = 0; i < C::XPW; ++i) {
+      x.set(i, wave, lane, (uint32_t)(min(p.row0 + x.row(i, wave, lane), a.B - 1) - p.row0) * a.ldx);
+      stream.xoff[i] = x.off[i];
+    }
+    stream.xb = reinterpret_cast<const char*>(a.x + (size_t)p.row0 * a.ldx);
+  };
+  // What a wave stores at least of a whole tile with these epilogues, which ask for nothing but their place inside the output.
+  constexpr int STORES = EPI == EPI_SWIGLU ? C::FM : EPI == EPI_STORE || EPI == EPI_RESIDUAL ? C::FM * (C::FN / 2) : 0;
+  auto whole = [&](TilePlace p) { return p.row0 + C::TM <= a.B && (p.strip0 + C::TS) * (EPI == EPI_SWIGLU ? 8 : 16) <= a.N; };
+  TilePlace here = tile_place<C>(first + q, MT, NT);
+  where(here);
+  stream.begin(here.strip0);
+  bool stored = false;
+  for (;;) {
+    f32x4 acc[C::FN][C::FM];
+    q += step;
+    const bool more = q < run;
+    const TilePlace next = more ? tile_place<C>(first + q, MT, NT) : here;  // (behind the last one: its own first steps, unused)
+    stream.template walk<STORES>(acc, next.strip0, stored, [&] { where(next); });
+    tile_epilogue<EPI, C>(a, acc, here.row0 + wave / C::WN * C::FM * 16, here.strip0 + wave % C::WN * C::FN, nstrips, lane);
+    if (!more) break;
+    stored = whole(here);
+    here = next;
+  }
+  wait_loads<0>();  // (into LDS that is no longer this workgroup's otherwise)
+}
+
 template <int EPI, class C, bool ALIGNED = true>
 int launch_tile(const GemmArgs& a, int nstrips, hipStream_t st) {
   const int64_t MT = (a.B + C::TM - 1) / C::TM, NT = (nstrips + C::TS - 1) / C::TS;
   if (MT * NT > INT32_MAX - 8) return OHARA_ESIZE;
+  if constexpr (C::HALVES) {
+    if (MT * NT > CUS && a.K % 64 == 0 && a.K >= 64 * C::XS) {
+      (void)hipFuncSetAttribute((const void*)gemm_rounds_kernel<EPI, C>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+      hipLaunchKernelGGL((gemm_rounds_kernel<EPI, C>), dim3(CUS), dim3(C::NW * 64), C::LDS, st, a, (int)MT, (int)NT, nstrips);
+      return ohara_launch_status();
+    }
+  }
   if (C::LDS > 64 * 1024)
     (void)hipFuncSetAttribute((const void*)gemm_tile_kernel<EPI, C, ALIGNED>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
   hipLaunchKernelGGL((gemm_tile_kernel<EPI, C, ALIGNED>), dim3((unsigned)(MT * NT + 7) / 8 * 8), dim3(C::NW * 64), C::LDS, st, a,
@@ -466,7 +532,6 @@ int one_round_tile(int rows, int strips, int K, Epilogue epi) {
 // that decides: 16384 rows 768 x 3072 with a residual 78.3 in 512 tiles of 128 x 192, 74.9 in 192 of 256 x 256; 768 x 768 23.1 / 22.1; 8192 rows 1024 x 1024
 // with a bias 22.5 of 128 x 128, 20.7 of 128 x 256 in halves.  (TIMES are fitted without.)
 float tile_time(const TileTime& t, int rows, int strips, int K, float extra = 0.f, bool lone = false) {
-  constexpr int CUS = 256;
   const int64_t tiles = ((int64_t)rows + t.rows - 1) / t.rows * ((strips + t.strips - 1) / t.strips);
   const int64_t waves = lone && tiles == CUS * t.slots ? 0 : tiles / (CUS * t.slots), rest = tiles - waves * CUS * t.slots;
   float step = waves * t.slots * t.full;

@@ -217,6 +217,122 @@ __device__ __forceinline__ void halves_product(f32x4 (&acc)[C::FN][C::FM], const
   }
 }
 
+// The same walk over tile after tile, for depths of whole steps: the loads run ahead of the products by the same number of phases throughout, out
+// of a tile into the one that follows, so that between two tiles there are only the barriers that bring the halves together.
+template <class C>
+struct HalvesStream {
+  static constexpr int FM = C::FM, FN = C::FN, NW = C::NW, PU = C::PU, PH = 2 / PU, XS = C::XS, WS = C::WS, WPW = C::WPW, XPP = C::XPP;
+  const char* xb;            // where the loads are: the tile's rows, this lane's offsets from there, strips
+  uint32_t xoff[C::XPW];
+  const char* wb[WPW];
+  const uint4* wp;
+  int nsteps, nstrips, wave;
+  uint32_t lds0, ldsw, lane16, xrd, wrd, xkey;
+  uint32_t xo, xi, wo, wi;   // slots: read from, asked for
+
+  __device__ __forceinline__ HalvesStream(const uint4* wp_, int K, int nstrips_, int wave_, int lane, unsigned char* smem)
+      : wp(wp_), nsteps(K >> 6), nstrips(nstrips_), wave(wave_) {
+    const int m = lane & 15, g = lane >> 4;
+    lds0 = (uint32_t)(uintptr_t)(OHARA_LDS unsigned char*)smem;
+    ldsw = lds0 + XS * C::XSLOT;
+    lane16 = lane * 16;
+    xrd = lds0 + (wave / C::WN * FM * 16 + m) * 128;
+    wrd = ldsw + wave % C::WN * FN * PU * 1024 + lane16;
+    xkey = g ^ (m & 7);
+    xo = wo = 0;
+    xi = (XS - 1) * C::XSLOT;
+    wi = (WS - 1) * C::WSLOT;
+  }
+  __device__ __forceinline__ void strips(int strip0) {
+#pragma unroll
+    for (int i = 0; i < WPW; ++i)
+      wb[i] = reinterpret_cast<const char*>(wp) + (size_t)min(strip0 + (wave + i * NW) / PU, nstrips - 1) * nsteps * 2048;
+  }
+  __device__ __forceinline__ void load_x(int s, uint32_t slot, int i) const { load_lds16(lds0 + slot + (wave + i * NW) * 1024, xb + (size_t)s * 128, xoff[i]); }
+  __device__ __forceinline__ void load_w(int p, uint32_t slot, int i) const {
+    const int t = wave + i * NW;
+    load_lds16(ldsw + slot + t * 1024, wb[i] + (size_t)(p * PU + t % PU) * 1024, lane16);
+  }
+  // The first tile's first phases, as many as the rings hold (its rows are set).
+  __device__ __forceinline__ void begin(int strip0) {
+    strips(strip0);
+#pragma unroll
+    for (int i = 0; i < C::XPW; ++i) load_x(0, 0, i);
+#pragma unroll
+    for (int p = 0; p < WS - 1; ++p) {
+      if (p > 0) {
+#pragma unroll
+        for (int i = 0; i < XPP; ++i) {
+          const int l = (p - 1) * XPP + i;
+          load_x(1 + l / C::XPW, (1 + l / C::XPW) * C::XSLOT, l % C::XPW);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < WPW; ++i) load_w(p, p * C::WSLOT, i);
+    }
+    wait_loads<(WS - 2) * (WPW + XPP)>();
+    __builtin_amdgcn_s_barrier();
+  }
+  // E < 0: a step whose loads are this tile's; else the E-th of the last XS - 1, whose activations (and, from phase 0 on, weights) are the next tile's.
+  // FIRST: a tile's first step, which nothing is added to; where `stored`, at least STORES stores of this wave lie between its loads and those before,
+  // so many more may be on their way (they finish in order).
+  template <int E, bool FIRST, int STORES>
+  __device__ __forceinline__ void step(f32x4 (&acc)[FN][FM], int s, int next_strip0, bool stored) {
+#pragma unroll
+    for (int h = 0; h < PH; ++h) {
+      uint4 xf[PU][FM], wf[PU][FN];
+#pragma unroll
+      for (int j = 0; j < PU; ++j) {
+#pragma unroll
+        for (int u = 0; u < FN; ++u) wf[j][u] = lds16_at(wrd + wo + (u * PU + j) * 1024);
+#pragma unroll
+        for (int t = 0; t < FM; ++t) xf[j][t] = lds16_at(xrd + xo + t * 2048 + (xkey ^ (4 * (h * PU + j))) * 16);
+      }
+      // Into the slots of the phase (the step) before: the other half has read them, a barrier ago.
+#pragma unroll
+      for (int i = 0; i < XPP; ++i) load_x(E < 0 ? s + XS - 1 : E, xi, h * XPP + i);
+      const int over = (E - (XS - 1)) * PH + h + WS - 1;  // phases past this tile's last one
+      if (E >= 0 && over == 0) strips(next_strip0);
+#pragma unroll
+      for (int i = 0; i < WPW; ++i) load_w(E < 0 || over < 0 ? s * PH + h + WS - 1 : over, wi, i);
+      // the next phase's have landed (WS - 2 phases, the first step, wait for loads in front of the stores)
+      static_assert(!FIRST || PH == WS - 2, "");
+      if (FIRST && STORES && stored) wait_loads<(WS - 2) * (WPW + XPP) + STORES>();
+      else wait_loads<(WS - 2) * (WPW + XPP)>();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < PU; ++j)
+#pragma unroll
+        for (int t = 0; t < FM; ++t)
+#pragma unroll
+          for (int u = 0; u < FN; ++u) acc[u][t] = mfma16(wf[j][u], xf[j][t], FIRST && h == 0 && j == 0 ? (f32x4){0.f, 0.f, 0.f, 0.f} : acc[u][t]);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      wo = wo + C::WSLOT == WS * C::WSLOT ? 0 : wo + C::WSLOT;
+      wi = wi + C::WSLOT == WS * C::WSLOT ? 0 : wi + C::WSLOT;
+    }
+    xo = xo + C::XSLOT == XS * C::XSLOT ? 0 : xo + C::XSLOT;
+    xi = xi + C::XSLOT == XS * C::XSLOT ? 0 : xi + C::XSLOT;
+  }
+  // One tile; rows_of_next() sets the next one's rows.  Its first phase has landed on entry, and the next one's on return.
+  template <int STORES, class F>
+  __device__ __forceinline__ void walk(f32x4 (&acc)[FN][FM], int next_strip0, bool stored, F rows_of_next) {
+    static_assert(XS == 3, "two steps at a tile's end");
+    const bool late = wave >= NW / 2;
+    if (late) __builtin_amdgcn_s_barrier();
+    step<-1, true, STORES>(acc, 0, 0, stored);
+    for (int s = 1; s < nsteps - 2; ++s) step<-1, false, 0>(acc, s, 0, false);
+    rows_of_next();
+    step<0, false, 0>(acc, nsteps - 2, next_strip0, false);
+    step<1, false, 0>(acc, nsteps - 1, next_strip0, false);
+    if (!late) __builtin_amdgcn_s_barrier();
+  }
+};
+
 template <class C, bool ALIGNED>
 __device__ __forceinline__ void tile_product(f32x4 (&acc)[C::FN][C::FM], const char* xb, const XOffsets<C, ALIGNED>& x, const uint4* wp,
                                              int strip0, int nstrips, int K, int wave, int lane, unsigned char* smem, int strip_steps = 0) {
