@@ -1262,9 +1262,9 @@ uint32_t* sampler_scratch_ptr() {
 //
 // A bf16 logit has one of 65536 bit patterns, dividing by the temperature and the softmax are
 // monotone, so every id with the same pattern has the same probability and the whole distribution is
-// the table (pattern -> count).  One pass counts the patterns into LDS (two 16-bit counts per dword,
-// 128 KB); everything the sampler has to find is then a walk over that table in descending key order,
-// 64 keys per thread with block-wide prefix sums in a fixed order:
+// the table (pattern -> count).  One pass counts the patterns into LDS (two 16-bit counts per dword, a magnitude's two signs,
+// 128 KB); everything the sampler has to find is then a walk over the patterns that occur in descending key order,
+// with block-wide prefix sums in a fixed order:
 //   * top-k: the key at which the cumulative count reaches k (ties at it survive, chat_engine.py:66-69);
 //   * softmax normaliser: sum of count * exp(x(key) - max) over the surviving keys;
 //   * nucleus: in descending order (ties lowest id first) a token is kept iff the mass before it is
@@ -1295,42 +1295,25 @@ __device__ __forceinline__ float key16_value(uint32_t key) {  // the bf16 value 
   return __uint_as_float(bits << 16);
 }
 
-// max of a and max of b over the workgroup in one exchange (two barriers instead of four)
-__device__ __forceinline__ void block_max_max_i(int& a, int& b, Smem& s) {
-  a = lanes_max<32, 1>(a);
-  b = lanes_max<32, 1>(b);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) {
-    s.wredi[w] = a;
-    s.hist[w] = b;
-  }
-  __syncthreads();
-  int ra = s.wredi[0], rb = s.hist[0];
-#pragma unroll
-  for (int i = 1; i < NW; ++i) {
-    ra = max(ra, s.wredi[i]);
-    rb = max(rb, s.hist[i]);
-  }
-  a = ra;
-  b = rb;
-}
-
 template <int EPT>
 __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
-  extern __shared__ uint32_t hist[];  // HB dwords: key k counted in half (k & 1) of dword k >> 1; then the list
+  extern __shared__ uint32_t hist[];  // HB dwords: patterns m and m | 0x8000 counted in the halves of dword m; then the list
   __shared__ Smem s;
   const int b = blockIdx.x, tid = threadIdx.x;
   const int V = a.V, nvalid = min(a.valid, V);
   const int base = tid * EPT;
   const float temp = a.temperature;
   const float u = a.u[(a.step_state && a.u_step_stride > 0 ? (size_t)a.step_state[1] * a.u_step_stride : 0) + b];
-  // One CU walks the whole row, so every instruction per id costs about half a microsecond: the two bf16 patterns of a
-  // register become order-preserving 16-bit keys with four integer instructions.  fn(id, key) is called for the valid ids among
-  // 8 id0 ..; key 0 cannot occur for a number (it is the pattern of one NaN) and is skipped.
+  // What bounds it: one CU walks the whole row, so every instruction per id costs about half a microsecond, and every step that one wave does for
+  // the others one or two.  Patterns are counted as they are, the largest is the list's first (order-preserving keys for every id, and
+  // their extremes, were 3 us of 18.7 over 65536 ids); a wave lists a block of patterns at a time, a pattern a lane (those threads whose
+  // 64 patterns occur, one after the other: 3.4 us); of the drawn pattern's ids the few threads that have one make a list (a count of every
+  // thread's: 3.3).  65536 ids, top-p 0.95 of a model's logits: 18.7 -> 14.1 us; 32000 ids 15.4 -> 11.9, 64 rows of 51200 19.5 -> 14.8.
+  // The two patterns of a register become order-preserving 16-bit keys with four integer instructions where the order matters.  fn(id, key) is called
+  // for the valid ids among 8 id0 ..; key 0 cannot occur for a number (it is the pattern of one NaN) and is skipped.
   // Where the order of a thread's ids does not matter - counting, and the search for a tie - it holds eighths NT chunks apart, `own`:
   // a wave's load is 1 KiB in one piece, and they stay in registers from one pass to the next.  (64 ids in a row a thread, read again for the
-  // second pass, were sixty-four lines a load: 25.6 us a row of 65536 ids, 22.2 so, 18.7 with the counting below without a question per id.)
+  // second pass, were sixty-four lines a load: 25.6 us a row of 65536 ids, 22.2 so.)
   // The draw in vocabulary order adds up 64 ids in a row a thread and reads them so.
   // All loads of a pass go out before the first is used (addresses past the valid ids fall back on the
   // chunk of the last valid id, whose values are not looked at): one round trip to the L2 per pass.
@@ -1368,80 +1351,120 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
     for (int i = tid; i < HB / 4; i += NT) h4[i] = make_uint4(0, 0, 0, 0);
     __syncthreads();
   }
-  // Counting and extremes, without a question per id: the key no number has is counted like the others (and left out of the list).
   typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-  u16x2 hi2 = {0, 0}, lo2 = {0xffff, 0xffff};
+  const int k = min(a.top_k, V);
+  int kmax = 0, n_live = nvalid, n_ent = 1;
+  bool one_value = false;
+  uint32_t* ent = hist + HB;  // entry = key << 16 | count (count < 65536: more than one value occurs)
+  if (!want_table) {
+    u16x2 hi2 = {0, 0};
 #pragma unroll
-  for (int c = 0; c < EPT / 8; ++c) {
-    const int id0 = 8 * (c * NT + tid);
-    const uint32_t w[4] = {own[c].x, own[c].y, own[c].z, own[c].w};
-    if (id0 + 8 <= nvalid) {
+    for (int c = 0; c < EPT / 8; ++c)
+      each_key(own[c], 8 * (c * NT + tid), [&](int, uint32_t key) { hi2[0] = max((int)hi2[0], (int)key); });
+    kmax = block_max_i((int)hi2[0], s);
+  } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t kk = w[j] ^ ((((w[j] >> 15) & 0x00010001u) * 0xffffu) | 0x80008000u);
-        hi2 = __builtin_elementwise_max(hi2, __builtin_bit_cast(u16x2, kk));
-        lo2 = __builtin_elementwise_min(lo2, __builtin_bit_cast(u16x2, kk));
-        if (want_table) {
-          atomicAdd(&hist[(kk & 0xffffu) >> 1], 1u << ((kk & 1u) << 4));
-          atomicAdd(&hist[kk >> 17], 1u << ((kk >> 12) & 16u));
+    for (int c = 0; c < EPT / 8; ++c) {
+      const int id0 = 8 * (c * NT + tid);
+      const uint32_t w[4] = {own[c].x, own[c].y, own[c].z, own[c].w};
+      if (id0 + 8 <= nvalid) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          atomicAdd(&hist[w[j] & 0x7fffu], (int)(w[j] << 16) < 0 ? 0x10000u : 1u);
+          atomicAdd(&hist[(w[j] >> 16) & 0x7fffu], (int)w[j] < 0 ? 0x10000u : 1u);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (id0 + i < nvalid) {
+            const uint32_t v = (w[i >> 1] >> (16 * (i & 1))) & 0xffffu;
+            atomicAdd(&hist[v & 0x7fffu], v & 0x8000u ? 0x10000u : 1u);
+          }
+      }
+    }
+    __syncthreads();
+    const int n_nan = (int)(hist[0x7fff] >> 16);  // ids with the pattern no number has: not listed
+    n_live = nvalid - n_nan;
+    // The patterns that occur, with their counts, compacted into a list in descending key order (a flat
+    // row of N(0,1)-like logits has about 1500 distinct patterns out of 65536): every later walk then
+    // touches one or two entries per thread instead of 64 table slots.  A thread counts those of 32 magnitudes, the largest
+    // first; positive ones descend as the threads do, negative ones the other way, behind them.
+    const int top = 32768 - 32 * (tid + 1);  // its smallest magnitude
+    const uint4* seg = reinterpret_cast<const uint4*>(hist + top);
+    int both = 0;  // positive ones | negative ones << 16
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {  // (neighbouring lanes at different eighths of their 128 bytes: in step they meet on two banks' worth)
+      const uint4 sv = seg[(q + tid) & 7];
+      const uint32_t w[4] = {sv.x, sv.y, sv.z, tid == 0 && ((q + tid) & 7) == 7 ? sv.w & 0xffffu : sv.w};  // (not that pattern)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) both += ((w[i] & 0xffffu) ? 1 : 0) + ((w[i] >> 16) ? 0x10000 : 0);
+    }
+    // prefix sums of both, and the number of blocks that hold any, in one exchange
+    const int lane = tid & 63, wave = tid >> 6;
+    const unsigned long long any = __ballot(both != 0);
+    const int incl = wave_incl_scan_i(both);
+    if (lane == 63) {
+      s.wredi[wave] = incl;
+      s.hist[wave] = __popcll(any);
+    }
+    __syncthreads();
+    uint32_t before = 0, total = 0;
+    int block = 0, blocks = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      const uint32_t t = (uint32_t)s.wredi[i];
+      const int n = s.hist[i];
+      if (i < wave) before += t, block += n;
+      total += t;
+      blocks += n;
+    }
+    const int n_pos = (int)(total & 0xffffu), n_neg = (int)(total >> 16);
+    n_ent = n_pos + n_neg;
+    const uint32_t excl = before + (uint32_t)(incl - both);
+    const int pos_at = (int)(excl & 0xffffu), neg_at = n_ent - (int)(excl >> 16) - (int)((uint32_t)both >> 16);  // this block's first of each
+    if (n_ent <= ENT_CAP) {
+      if (both) {
+        const int slot = block + __popcll(any & ((1ull << lane) - 1));
+        s.skey[slot] = (uint32_t)pos_at << 16 | (uint32_t)neg_at;
+        s.sid[slot] = top;
+      }
+      __syncthreads();
+      for (int j = wave; j < blocks; j += NW) {  // a pattern a lane: positive ones descending, then negative ones ascending in magnitude
+        const int mag = s.sid[j] + (lane < 32 ? 31 - lane : lane - 32);
+        const uint32_t at = s.skey[j], w = hist[mag];
+        const uint32_t c = lane < 32 ? w & 0xffffu : mag == 0x7fff ? 0u : w >> 16;
+        const unsigned long long there = __ballot(c != 0);
+        if (c) {
+          const unsigned long long mine = lane < 32 ? there : there >> 32 << 32;
+          const int slot = (int)(lane < 32 ? at >> 16 : at & 0xffffu) + __popcll(mine & ((1ull << lane) - 1));
+          ent[slot] = (lane < 32 ? (uint32_t)(mag | 0x8000) : (uint32_t)(0x7fff - mag)) << 16 | c;
         }
       }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (id0 + i < nvalid) {
-          const uint32_t v = (w[i >> 1] >> (16 * (i & 1))) & 0xffffu, key = v ^ ((v & 0x8000u) ? 0xffffu : 0x8000u);
-          hi2[0] = max((int)hi2[0], (int)key);
-          lo2[0] = min((int)lo2[0], (int)key);
-          if (want_table) atomicAdd(&hist[key >> 1], 1u << ((key & 1u) << 4));
+    } else if (both && pos_at == 0 && (n_pos || neg_at == 0)) {  // the first block with the larger sign: its largest key
+      for (int i = 0; i < 32; ++i) {
+        const int mag = n_pos ? top + 31 - i : top + i;
+        if (n_pos ? hist[mag] & 0xffffu : hist[mag] >> 16) {
+          if (!n_pos || (both & 0xffff)) s.misc[4] = n_pos ? mag | 0x8000 : 0x7fff - mag;
+          break;
         }
+      }
+    }
+    if (tid == 0) s.misc[0] = (int)(own[0].x & 0xffffu);
+    __syncthreads();
+    // a row of one single value is the only way a 16-bit count can overflow: its table is not looked at
+    if (nvalid == 65536 && n_ent <= 1 && (int)(n_ent ? ent[0] & 0xffffu : 0u) + n_nan != nvalid) {
+      one_value = true;
+      const uint32_t v = (uint32_t)s.misc[0];
+      kmax = (int)(v ^ ((v & 0x8000u) ? 0xffffu : 0x8000u));
+      n_live = kmax ? nvalid : 0;
+    } else if (n_ent) {
+      kmax = n_ent <= ENT_CAP ? (int)(ent[0] >> 16) : s.misc[4];
     }
   }
-  int kmax = max((int)hi2[0], (int)hi2[1]), nkmin = -min((int)lo2[0], (int)lo2[1]);
-  block_max_max_i(kmax, nkmin, s);  // (the barriers inside also complete the table)
-  const int kmin = -nkmin;
-  const int n_live = nvalid - (want_table ? (int)(hist[0] & 0xffffu) : 0);  // (asked for with the table only)
   int token = 0;
   if (kmax > 0) {
     const float m = xval((uint32_t)kmax);
-    const int k = min(a.top_k, V);
     const bool use_topk = a.top_k > 0 && k < n_live;  // k >= the number of valid ids: everything survives
-    // a row of one single value is the only way a 16-bit count can overflow: its table is not looked at
-    const bool one_value = kmax == kmin;
-    const bool need_table = (use_topk || nucleus) && !one_value;
-    // The keys that occur, with their counts, compacted into a list in descending key order (a flat
-    // row of N(0,1)-like logits has about 1500 distinct patterns out of 65536): every later walk then
-    // touches one or two entries per thread instead of 64 table slots.
-    uint32_t* ent = hist + HB;  // entry = key << 16 | count (count < 65536: more than one value occurs)
-    int n_ent = 1;
-    if (need_table) {
-      const uint4* seg = reinterpret_cast<const uint4*>(hist + HB - 32 * (tid + 1));  // my 64 keys, ascending
-      int nz = 0;  // counted with neighbouring lanes at different eighths of their 128 bytes (in step they meet on two banks' worth)
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const uint4 sv = seg[(q + tid) & 7];
-        const uint32_t w[4] = {tid == NT - 1 && ((q + tid) & 7) == 0 ? sv.x & 0xffff0000u : sv.x, sv.y, sv.z, sv.w};  // (not key 0)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) nz += ((w[i] >> 16) ? 1 : 0) + ((w[i] & 0xffffu) ? 1 : 0);
-      }
-      int off;
-      n_ent = block_excl_scan_i(nz, off, s);
-      if (n_ent <= ENT_CAP && nz) {  // few threads hold a key
-        const int kbase = 65536 - 64 * (tid + 1);  // key of the low half of seg[0].x
-#pragma unroll
-        for (int q = 7; q >= 0; --q) {
-          const uint4 sv = seg[q];
-          const uint32_t w[4] = {sv.x, sv.y, sv.z, sv.w};
-#pragma unroll
-          for (int i = 3; i >= 0; --i) {
-            const int key = kbase + 8 * q + 2 * i;
-            if (w[i] >> 16) ent[off++] = ((uint32_t)(key + 1) << 16) | (w[i] >> 16);
-            if (key && (w[i] & 0xffffu)) ent[off++] = ((uint32_t)key << 16) | (w[i] & 0xffffu);
-          }
-        }
-      }
-      __syncthreads();
-    }
     const bool listed = n_ent <= ENT_CAP;
     const int per = (n_ent + NT - 1) / NT;
     // fn(key, count) for this thread's share of the keys that occur, in descending key order (thread 0
@@ -1464,7 +1487,7 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
 #pragma unroll 1
       for (int j = 0; j < 64; ++j) {
         const int key = ktop - j;
-        const uint32_t c = key ? (hist[key >> 1] >> ((key & 1) << 4)) & 0xffffu : 0u;
+        const uint32_t c = !key ? 0u : key & 0x8000 ? hist[key & 0x7fff] & 0xffffu : hist[0x7fff - key] >> 16;
         if (c && fn((uint32_t)key, c)) return;
       }
     };
@@ -1501,15 +1524,16 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
         mass += (float)c * prob(key);
         return false;
       });
+      if (tid == 0) {  // (complete behind the scan's barriers)
+        s.misc[5] = 0;     // no boundary: everything kept
+        s.misc[7] = kmax;  // fallback of the draw: the first id of the largest key
+        s.misc[3] = 0;
+        s.misc[1] = 0;
+        s.misc[2] = -1;
+      }
       float lo, hi;
       const float Z = block_scan_f(mass, lo, hi, s);
       const float limit = a.top_p * Z;
-      if (tid == 0) {  // defaults: everything kept
-        s.misc[5] = (int)Tk;
-        s.misc[6] = -1;  // all ties of the boundary key
-        s.fmisc[0] = Z;
-      }
-      __syncthreads();
       if (lo <= limit && limit < hi) {
         // the last kept key, how many of its ties are kept, and the kept mass S
         float run = lo, S = hi;
@@ -1541,15 +1565,10 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
         }
       }
       __syncthreads();
-      const uint32_t Tn = (uint32_t)s.misc[5];
-      const int nk = s.misc[6];
-      const float target = u * s.fmisc[0];
-      __syncthreads();
-      if (tid == 0) {
-        s.misc[7] = kmax;  // fallback: the first id of the largest key
-        s.misc[3] = 0;
-      }
-      __syncthreads();
+      const bool bounded = s.misc[5] != 0;
+      const uint32_t Tn = bounded ? (uint32_t)s.misc[5] : Tk;
+      const int nk = bounded ? s.misc[6] : -1;  // -1: all ties of the boundary key
+      const float target = u * (bounded ? s.fmisc[0] : Z);
       if (lo <= target && target < hi) {
         float run = lo;
         uint32_t lastk = 0, lastc = 0;
@@ -1582,15 +1601,23 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
       __syncthreads();
       const uint32_t Td = (uint32_t)s.misc[7];
       const int r = s.misc[3];
-      // The r-th id, in id order, among the ids with key Td: the bf16 pattern behind the key is compared as loaded (two instructions an
-      // id), every thread notes where it occurs among its own, the totals of the NT-wide eighths say which of them holds the r-th, and a
-      // scan over that one which thread.
+      // The r-th id, in id order, among the ids with key Td: the bf16 pattern behind the key is compared as loaded (two instructions
+      // for two ids), the threads that have some list them, and of a short list each is compared with the others.  Of a long one every thread notes
+      // where they occur among its own, the totals of the NT-wide eighths say which of them holds the r-th, and a scan over that one which thread.
       constexpr int NC = EPT / 8;
       static_assert(NC <= 8, "one bit per id of the thread, one counter per eighth");
+      constexpr int FEW = 256;
       unsigned long long where = 0;
-      {
-        const uint32_t pat = (Td & 0x8000u) ? (Td & 0x7fffu) : (~Td & 0xffffu);  // key -> bf16 bits
-        const uint32_t pat2 = pat | (pat << 16);
+      const uint32_t pat = (Td & 0x8000u) ? (Td & 0x7fffu) : (~Td & 0xffffu);  // key -> bf16 bits
+      const uint32_t pat2 = pat | (pat << 16);
+      u16x2 least = {0xffff, 0xffff};
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const uint32_t w[4] = {own[c].x, own[c].y, own[c].z, own[c].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) least = __builtin_elementwise_min(least, __builtin_bit_cast(u16x2, w[j] ^ pat2));
+      }
+      if (least[0] == 0 || least[1] == 0) {
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
           const uint32_t w[4] = {own[c].x, own[c].y, own[c].z, own[c].w};
@@ -1606,9 +1633,25 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
           at = nv >= 8 ? at : nv <= 0 ? 0u : at & ((1u << nv) - 1u);
           where |= (unsigned long long)at << (8 * c);
         }
+        if (where) {
+          int slot = atomicAdd(&s.misc[1], __popcll(where));
+          for (unsigned long long left = where; left && slot < FEW; left &= left - 1, ++slot) {
+            const int bit = __ffsll((long long)left) - 1;
+            s.sid[slot] = 8 * ((bit >> 3) * NT + tid) + (bit & 7);
+          }
+        }
       }
+      __syncthreads();
+      const int found = s.misc[1];
+      if (found <= FEW) {
+        if (tid < found) {
+          const int mine = s.sid[tid];
+          int before = 0;
+          for (int i = 0; i < found; ++i) before += s.sid[i] < mine;
+          if (before == r) s.misc[2] = mine;
+        }
+      } else {
       if (tid < NC) s.hist[tid] = 0;
-      if (tid == 0) s.misc[2] = -1;
       __syncthreads();
 #pragma unroll
       for (int c = 0; c < NC; c += 2) {  // two eighths' counts in one word (a wave holds at most 512 of each)
@@ -1634,6 +1677,7 @@ __global__ __launch_bounds__(NT) void sample_hist_kernel(SampleArgs a) {
       if (c > 0 && off <= left && left < off + c) {
         for (int skip = left - off; skip > 0; --skip) mine &= mine - 1;  // drop the occurrences before it
         s.misc[2] = 8 * (eighth * NT + tid) + __ffs((int)mine) - 1;
+      }
       }
       __syncthreads();
       token = max(s.misc[2], 0);
@@ -1742,10 +1786,10 @@ int sample_dispatch(const void* logits, int logits_are_fp32, int ldl, int batch,
     hipLaunchKernelGGL(sample_parts_kernel, dim3(nparts, batch), dim3(NT), 0, st, a, scratch, nparts);
     return ohara_launch_status();
   }
-  // bf16 rows: selection on the histogram of the 16-bit patterns, except for a small top-k, where sorting
-  // the few survivors is as quick or quicker (top-k 50 + top-p 0.9: 32000 ids 12.8 us sorted, 15.4 by the table; 51200 18.7 and 18.6;
-  // 65536 20.1 and 19.0, where the two add up in different orders; top-p alone: 37 us (sharp row) to 139 us (flat row) with
-  // candidates / bisection, 19 us by the table whatever the row; plain multinomial 25 us)
+  // bf16 rows: selection on the histogram of the 16-bit patterns, except for a small top-k, where the few survivors are sorted (top-k 50 +
+  // top-p 0.95, us sorted / by the table: 8192 ids 12.5 / 9.8, 32000 13.2 / 12.9, 51200 19 / 14, 65536 20.4 / 14.8; but the two add up in different
+  // orders, and rows of many ties, or draws at the end of the kept mass, get other tokens; top-p alone: 37 us (sharp row) to 139 us (flat row) with
+  // candidates / bisection, 14 us by the table whatever the row; plain multinomial 25 us)
   const bool small_k = top_k > 0 && top_k <= CAP;
   if (!logits_are_fp32 && !small_k && vocab <= 65536 && (ldl & 7) == 0 &&
       (reinterpret_cast<uintptr_t>(logits) & 15) == 0) {
