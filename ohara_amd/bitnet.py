@@ -299,7 +299,7 @@ class BitDecodeSession:
     def _init_workspace(self) -> None:
         torch.cuda.current_stream().synchronize()
         check(lib().ohara_bitnet_decode_persistent(C.byref(self.model._c_model), C.byref(self._dst), self._pws.data_ptr(),
-                                                   self._nwg, 1, 1, 0, torch.cuda.current_stream().cuda_stream),
+                                                   self._nwg, 1, 1, 0, ops.current_stream()),
               "persistent init")
 
     def restart(self, u: torch.Tensor | None = None) -> None:
@@ -316,7 +316,7 @@ class BitDecodeSession:
             self.u[: u.shape[0]].copy_(u)
 
     def _launch_step(self) -> None:
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = ops.current_stream()
         greedy = 0 if self.sampling else 1
         check(lib().ohara_bitnet_decode_persistent(C.byref(self.model._c_model), C.byref(self._dst), self._pws.data_ptr(),
                                                    self._nwg, 0, greedy, int(self.spin_limit), stream),

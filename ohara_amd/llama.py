@@ -430,7 +430,7 @@ class Llama:
         st = self._state_struct(buf, kv_cache, logits, seq_pos=seq_pos)
         mode = _lib.OHARA_LOGITS_LAST if last_only else _lib.OHARA_LOGITS_ALL
         check(lib().ohara_llama_forward(C.byref(self._c_model), C.byref(st), S, 0 if ragged is not None else start_pos, 0,
-                                        mode, 0, torch.cuda.current_stream().cuda_stream), "llama_forward")
+                                        mode, 0, ops.current_stream()), "llama_forward")
         for cache, end in zip(kv_cache, ends):
             if ragged is not None:
                 cache._commit_ragged(B, end)
@@ -477,7 +477,7 @@ class Llama:
         logits = torch.empty(n, self.config.vocab_size, dtype=BF16, device=self.device)
         st = self._state_struct(buf, kv_cache, logits)
         check(lib().ohara_llama_prompts(C.byref(self._c_model), C.byref(st), n, length.data_ptr(), dev[2 * rows:].data_ptr(),
-                                        torch.cuda.current_stream().cuda_stream), "llama_prompts")
+                                        ops.current_stream()), "llama_prompts")
         return logits
 
     # -- device-resident greedy loop --------------------------------------------------
@@ -576,7 +576,7 @@ class DecodeSession:
         st = m._state_struct(pbuf, self.cache, self.logits, valid_vocab=self.valid_vocab)
         st.step_state = 0
         check(lib().ohara_llama_forward(C.byref(m._c_model), C.byref(st), P, 0, 0, _lib.OHARA_LOGITS_LAST,
-                                        0 if self.sampling else 1, torch.cuda.current_stream().cuda_stream), "prefill")
+                                        0 if self.sampling else 1, ops.current_stream()), "prefill")
         if self.sampling:
             ops.sample_topk_topp(self.logits, self.sampling.temperature, self.sampling.top_k, self.sampling.top_p,
                                  self.u[0], self.valid_vocab or None, out=pbuf.ids[:B])
@@ -611,7 +611,7 @@ class DecodeSession:
                                                                    self._nwg)
             torch.cuda.current_stream().synchronize()
             check(lib().ohara_llama_decode_persistent(C.byref(m._c_model), C.byref(self._dst), self._pws.data_ptr(),
-                                                      self._nwg, 1, 1, 0, torch.cuda.current_stream().cuda_stream),
+                                                      self._nwg, 1, 1, 0, ops.current_stream()),
                   "persistent init")
 
     def restart(self, u: torch.Tensor | None = None) -> None:
@@ -645,7 +645,7 @@ class DecodeSession:
 
     def _launch_step(self) -> None:
         m = self.model
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = ops.current_stream()
         greedy = 0 if self.sampling else 1
         if self.persistent:
             check(lib().ohara_llama_decode_persistent(C.byref(m._c_model), C.byref(self._dst), self._pws.data_ptr(),
@@ -681,7 +681,7 @@ class DecodeSession:
         if self.persistent and self._pws is not None:
             torch.cuda.current_stream().synchronize()
             check(lib().ohara_llama_decode_persistent(C.byref(self.model._c_model), C.byref(self._dst), self._pws.data_ptr(),
-                                                      self._nwg, 1, 1, 0, torch.cuda.current_stream().cuda_stream),
+                                                      self._nwg, 1, 1, 0, ops.current_stream()),
                   "persistent init")
 
     def phase_clocks(self, workgroup: int | None = 0) -> torch.Tensor:
@@ -705,7 +705,7 @@ class DecodeSession:
     def step(self, prof_kernel: int = -1, prof_start=None, prof_stop=None) -> None:
         """One eager decode step (enqueue only)."""
         self._room(1)
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = ops.current_stream()
         if self.persistent:
             # a single launch: bracket it directly
             if prof_start is not None:

@@ -16,8 +16,13 @@ from ._lib import check, lib
 BF16 = torch.bfloat16
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+def current_stream() -> int:
+    """The current device's current stream as its handle.  (``torch.cuda.current_stream().cuda_stream`` makes two objects for it: 2.7 us of the host's time
+    a call, where sampling a token is 13 in all and a launch's own 3; this is 0.2.)"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+_stream = current_stream
 
 
 def _ptr(t):
