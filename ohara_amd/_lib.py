@@ -206,6 +206,8 @@ _PROTOS = {
     "ohara_phi_attn_bf16": (_i, [_p, _i, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _i, _p, _p, _p]),
     "ohara_phi_attn_linear_bf16": (_i, [_p, _i, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _i, _p, _p, _p, _i, _p, _i, _i, _p, _p, _i, _p]),
     "ohara_phi_attn_linear_chunks": (_i, [_i, _i, _i, _i, _i, _i, _i]),
+    "ohara_phi_attn_out_bf16": (_i, [_p, _i, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _i, _p, _p, _i, _p, _i, _i, _p, _p, _i, _p, _p, _p, _i, _p, _i, _p]),
+    "ohara_phi_attn_out_chunks": (_i, [_i, _i, _i, _i, _i, _i, _i, _i]),
     "ohara_persistent_workspace_bytes": (_i64, [C.POINTER(OharaModel), _i, _i, _i]),
     "ohara_persistent_barrier_offset": (_i64, [C.POINTER(OharaModel), _i, _i, _i]),
     "ohara_persistent_polled": (_i, [C.POINTER(OharaModel), _i, _i]),

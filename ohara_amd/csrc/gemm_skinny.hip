@@ -301,6 +301,99 @@ __global__ __launch_bounds__(1024) void phi_attn_linear_kernel(PhiAttnArgs t, Ge
   else skinny<1, 0, EPI_BIAS, 16, 8>(a, blockIdx.x - fours);
 }
 
+// (chunks by fours of a head, merged by phi_dense_kernel)
+__global__ __launch_bounds__(1024) void phi_parts_linear_kernel(PhiAttnArgs t, GemmArgs a, int fours) {
+  if ((int)blockIdx.x < fours) phi_attend<4, true, true>(t, blockIdx.x);
+  else skinny<1, 0, EPI_BIAS, 16, 8>(a, blockIdx.x - fours);
+}
+// The attention's output projection, which merges its chunks: sixteen waves a strip, each over its share of K (at most SP k-steps, parts of four heads) of
+// up to ROWS rows.  Merged by the team that is last, a chunk's sums go to memory, a counter is asked, the sums come back and the row goes to memory and back:
+// trips that take 2 us each while the weights of the product beside them stream (one row of 32 heads of 80 behind 700, beside 2560 x 10240: 17.1 us, without
+// these trips 12.6).  The launch's end orders them for nothing; the sums come back with this product's weights, and a team's threads merge four features
+// each.  What that costs is a CU's reads of everyone's sums, 2.3 us with sixteen chunks a head (126 KB), so four teams of a workgroup take chunks
+// of one head and leave one sum: 0.6.  The order of the sums is the products' above.
+template <int ROWS, int SP>
+__global__ __launch_bounds__(1024) void phi_dense_kernel(PhiAttnArgs t, GemmArgs a) {
+  constexpr int NW = 16, NCH = 4;
+  __shared__ float red[NW - 1][64][4];
+  __shared__ __align__(16) bf16_t xs[NW][ROWS][SP * 32];
+  __shared__ __align__(16) float weight[NW][ROWS][4][NCH], part[NW][ROWS][4][NCH];
+  const int strip = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  const int KS = (a.K + 31) >> 5, per_wave = (KS + NW - 1) / NW;
+  const int j0 = wave * per_wave, j1 = min(KS, j0 + per_wave);
+  const int pos = t.pos_dev ? *t.pos_dev : t.pos;
+  EpiPre ep;
+  if (wave == 0) gemm_epilogue_fetch<EPI_BIAS_ADD2>(a, m, strip, g, ep);
+  // lane: a chunk's {max, sum} of a row and one of the heads that the share lies in; four features, of every row and chunk (past the last: the last)
+  const int D = t.D, last = (t.ns >> 2) - 1, h0 = min(32 * j0, a.K - 4) / D;
+  const int prow = lane / (4 * NCH), phead = lane / NCH & 3, pc = lane & (NCH - 1);
+  const float2 pair = *reinterpret_cast<const float2*>(phi_pairs(t, min(prow, a.B - 1), min(h0 + phead, t.H - 1)) + 2 * min(pc, last));
+  const int f = min(32 * j0 + 4 * lane, a.K - 4), h = f / D;
+  uint4 v[ROWS][NCH];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) v[r][c] = ldg16(phi_values(t, min(r, a.B - 1), h) + min(c, last) * D + (f - h * D));
+  const uint4* wrow = a.wp + (size_t)strip * KS * 64 + lane;
+  uint4 wv[SP];
+#pragma unroll
+  for (int c = 0; c < SP; ++c) wv[c] = ldg16_nt(wrow + (size_t)min(j0 + c, KS - 1) * 64);
+  __builtin_amdgcn_sched_barrier(0);
+  const int ns = (max(pos, 0) / phi_chunk(max(pos, 0), t.ns) >> 2) + 1;
+  {
+    const bool in = pc < ns && pair.x != -INFINITY;
+    float M = in ? pair.x : -INFINITY;
+#pragma unroll
+    for (int x = 1; x < NCH; x *= 2) M = fmaxf(M, __shfl_xor(M, x));
+    const float wg = expf(pair.x - M);
+    if (prow < ROWS) {
+      weight[wave][prow][phead][pc] = in ? wg : -1.f;  // (negative: not counted, whatever lies there)
+      part[wave][prow][phead][pc] = in ? wg * pair.y : 0.f;
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    float num[4] = {0.f, 0.f, 0.f, 0.f}, den = 0.f;
+    const float *wg = weight[wave][r][min(h - h0, 3)], *pt = part[wave][r][min(h - h0, 3)];
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      const float w = wg[c];
+      const bool in = !(w < 0.f);
+      const uint32_t u[4] = {v[r][c].x, v[r][c].y, v[r][c].z, v[r][c].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) num[i] += in ? w * __uint_as_float(u[i]) : 0.f;
+      den += pt[c];
+    }
+    if (lane < 8 * SP) *reinterpret_cast<uint2*>(&xs[wave][r][4 * lane]) = make_uint2(pack_bf(num[0] / den, num[1] / den), pack_bf(num[2] / den, num[3] / den));
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < SP; ++c) {
+    const bool live = m < a.B && 32 * (j0 + c) + 8 * g < a.K;
+    uint4 x = *reinterpret_cast<const uint4*>(&xs[wave][min(m, ROWS - 1)][32 * c + 8 * g]);
+    x = live ? x : make_uint4(0, 0, 0, 0);
+    if (j0 + c < j1) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[c]), __builtin_bit_cast(bf16x8, x), acc, 0, 0, 0);
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[wave - 1][lane][i] = acc[i];
+  }
+  __syncthreads();
+  if (wave) return;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int w = 0; w < NW - 1; ++w) acc[i] += red[w][lane][i];
+  }
+  if (m < a.B) gemm_epilogue<EPI_BIAS_ADD2, true>(a, m, strip, g, acc, ep);
+}
+
 // Rows without a norm, K up to 6144: a wave's share of K is at most CH k-steps, all of them requested before anything waits.  Above, rounds
 // of six cost a round trip each; and a request costs what it costs whether its data are used, so CH is the share, rounded up to even.
 // H = 2: a workgroup takes half a strip (eight columns, in both halves of the product's sixteen), where strips leave CUs idle.
@@ -957,7 +1050,43 @@ bool ohara_launch_phi_attn_linear(PhiAttnArgs t, GemmArgs a, hipStream_t st, int
   return true;
 }
 
+// Chunks of the attention whose fours the projection merges; 0: the calls above.  All teams and strips are on the chip at once, a workgroup to a CU, so
+// one or two rows, and no more fours than the strips leave CUs.  A context of one chunk is the calls' above where they are one launch (its sums need no
+// merge: the projection's costs 0.4 us), and of 256 where the product is the longer part anyway.  A team's positions bound the launch past the product's
+// time, two launches spread them over all CUs: the line is through 360 calls, 2048 to 3584 wide with heads of 64 to 128, products of twice and four times the
+// width, one and two rows behind 20 to 4000.  us with the projection, the calls above / this: 2560 x 10240, 32 heads of 80, one row behind 40 16.5 / 16.9, 200
+// 20.3 / 17.2, 700 22.5 / 18.0, 2040 29.5 / 25.0, two rows behind 40 21.7 / 17.8, 700 29.2 / 24.4, 1200 32.0 / 30.6, 2000 35 / 49; 2048 x 8192, 32 of 64, one behind
+// 700 22.2 / 16.9; 3584 x 14336, 28 of 128, one behind 400 34.5 / 26.2, 1400 37.3 / 37.1; 2048 x 4096, 16 of 128, two rows behind 3000 27.5 / 29.1.
+static int phi_merged(int batch, int h, int dh, int rot, int n_split, int pos, int n, int k) {
+  const int strips = (n + 15) / 16, heads = batch * h, depth = h * dh, share = ((depth + 31) / 32 + 15) / 16 * 32;
+  if (batch > 2 || depth < 2048 || share > 256 || k < 2048 || strips >= 256 || (rot >> 1 & 7)) return 0;
+  for (int first = 0; first < depth; first += share)  // a share's heads
+    if ((std::min(first + share, depth) - 1) / dh - first / dh > 3) return 0;
+  const int chunks = std::min(n_split, 16) / 4 * 4 < 4 ? 0 : 4 * std::min(std::min(n_split, 16) / 4, (256 - (strips + 7) / 8 * 8) / heads);
+  if (!chunks || std::min(phi_chunk(pos, chunks), pos + 1) > 128 + k / 64 || (int64_t)heads * dh * (pos + 1) > 10500000) return 0;
+  return pos >= ((int64_t)n * k <= 30000000 ? 64 : 256) || !phi_beside(batch, h, dh, n_split, pos, n, k) ? chunks : 0;
+}
+int ohara_launch_phi_attn_out(PhiAttnArgs t, GemmArgs a, GemmArgs out, hipStream_t st) {
+  t.ns = phi_eights(t) ? phi_merged(a.B, t.H, t.D, t.rot, t.ns, std::min(std::max(t.pos, 0), t.t_max - 1), a.N, a.K) : 0;
+  if (!t.ns) return OHARA_ESIZE;
+  const int strips = (a.N + 15) / 16, fours = (a.B * t.H * (t.ns >> 2) + 7) / 8 * 8;  // (whole eights: a strip's XCD is its workgroup's number)
+  a.ny = 1; a.nstrips = strips;
+  hipLaunchKernelGGL(phi_parts_linear_kernel, dim3((unsigned)(fours + (strips + 7) / 8 * 8)), dim3(1024), 0, st, t, a, fours);
+  const int rc = ohara_launch_status();
+  if (rc) return rc;
+  const bool five = (out.K + 31) / 32 <= 5 * 16;
+  auto kernel = a.B == 1 ? (five ? phi_dense_kernel<1, 5> : phi_dense_kernel<1, 8>) : five ? phi_dense_kernel<2, 5> : phi_dense_kernel<2, 8>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)strips), dim3(1024), 0, st, t, out);
+  return ohara_launch_status();
+}
+
 extern "C" {
+
+int ohara_phi_attn_out_chunks(int batch, int h, int dh, int rot, int n_split, int pos, int n, int k) {
+  if (batch < 1 || h < 1 || dh < 8 || dh > 128 || (dh & 7) || rot < 2 || (rot & 1) || rot > dh || n_split < 1 || n_split > 64 || pos < 0 || n < 1 || k < 1)
+    return OHARA_EINVAL;
+  return (int64_t)batch * h * dh > INT32_MAX ? 0 : phi_merged(batch, h, dh, rot, n_split, pos, n, k);
+}
 
 int ohara_pack_rows_bf16(const uint16_t* w, int n, int k, int ldw, const int32_t* perm, int n_padded,
                          uint16_t* dst, int64_t* bytes, void* stream) {

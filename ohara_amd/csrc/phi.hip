@@ -711,4 +711,25 @@ int ohara_phi_attn_linear_bf16(const uint16_t* q, int ldq, const uint16_t* kcach
   return rc ? rc : ohara_linear_bias_bf16(x, ldx, wp, n, k, bias, batch, OHARA_LIN_BIAS, nullptr, 0, nullptr, 0, y, ldy, stream);
 }
 
+int ohara_phi_attn_out_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, const uint16_t* vcache, const float* cos, const float* sin, int rot,
+                            int batch, int h, int dh, int t_max, int pos, const int32_t* pos_dev, int n_split, void* workspace, const uint16_t* x, int ldx,
+                            const uint16_t* wp, int n, int k, const uint16_t* bias, uint16_t* y, int ldy, const uint16_t* wp_out, const uint16_t* bias_out,
+                            const uint16_t* add, int ld_add, uint16_t* out, int ldo, void* stream) {
+  PhiAttnArgs t;
+  const int rc = phi_attn_args(t, q, ldq, kcache, vcache, cos, sin, rot, batch, 1, h, dh, t_max, pos, pos_dev, n_split, workspace, out);
+  if (rc) return rc;
+  if (!x || !wp || !bias || !y || n < 1 || k < 1 || (k & 7) || (ldx & 7) || ldx < k || (n & 3) || (ldy & 3) || ldy < n) return OHARA_EINVAL;
+  if (!wp_out || !bias_out || !add || (ld_add & 3) || ld_add < n || (ldo & 3) || ldo < n || !workspace || ((uintptr_t)workspace & 15)) return OHARA_EINVAL;
+  GemmArgs a{};
+  a.wp = reinterpret_cast<const uint4*>(wp);
+  a.x = x; a.ldx = ldx; a.B = batch; a.N = n; a.K = k;
+  a.out = y; a.ldo = ldy; a.bias = bias;
+  GemmArgs o{};
+  o.wp = reinterpret_cast<const uint4*>(wp_out);
+  o.B = batch; o.N = n; o.K = h * dh;
+  o.out = out; o.ldo = ldo; o.bias = bias_out;
+  o.resid = y; o.ldr = ldy; o.resid2 = add; o.ldr2 = ld_add;
+  return ohara_launch_phi_attn_out(t, a, o, (hipStream_t)stream);
+}
+
 }  // extern "C"

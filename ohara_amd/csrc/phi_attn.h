@@ -68,16 +68,26 @@ __host__ __device__ inline int phi_chunk(int pos, int ns) {
 
 // gemm_skinny.hip: the attention beside y = x W^T + bias in one launch, where that is the quicker way (else false, and nothing is launched).
 bool ohara_launch_phi_attn_linear(PhiAttnArgs t, GemmArgs a, hipStream_t st, int* rc);
+// The attention's chunks left in t.ws, beside the product or before it; then out = merged W^T + bias, added as EPI_BIAS_ADD2 adds.
+int ohara_launch_phi_attn_out(PhiAttnArgs t, GemmArgs a, GemmArgs out, hipStream_t st);
 
 namespace {
 
-// `block`: the workgroup's place among those that do this.
-template <int TEAMS, bool EIGHTS>
+// Where the sums of four chunks go that the next launch merges (phi_dense_kernel): values on 16 bytes, then {max, sum}.  a.ns is a multiple of four.
+__device__ __forceinline__ float* phi_values(const PhiAttnArgs& a, int row, int h) { return a.ws + ((size_t)row * a.H + h) * (a.ns >> 2) * a.D; }
+__device__ __forceinline__ float* phi_pairs(const PhiAttnArgs& a, int row, int h) {
+  return a.ws + (size_t)a.B * a.H * (a.ns >> 2) * a.D + ((size_t)row * a.H + h) * (a.ns >> 2) * 2;
+}
+
+// `block`: the workgroup's place among those that do this.  PARTS: one token a sequence; a workgroup's teams take four chunks
+// in turn of one head, and leave their sums together.
+template <int TEAMS, bool EIGHTS, bool PARTS = false>
 __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
   constexpr int R = 2;  // positions a lane group has in flight
   __shared__ float qr_[TEAMS][128];
   __shared__ float gm_[TEAMS][16], gl_[TEAMS][16];
   __shared__ float gacc_[TEAMS][16][128];
+  __shared__ float teams_m[TEAMS], teams_l[TEAMS];
   const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), tid = TEAMS == 1 ? threadIdx.x : threadIdx.x & 255;
   const int lane = tid & 63, wave = tid >> 6;
   float(&qr)[128] = qr_[team];
@@ -98,17 +108,24 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
     per = phi_chunk(max(pos, 0), a.ns);
     ns = max(pos, 0) / per + 1;
   }
-  const int rows = a.B * a.S * a.H, n = rows * ns;
-  int id = block * TEAMS + team;
+  static_assert(!PARTS || TEAMS == 4, "");
+  constexpr int APART = PARTS ? 1 : TEAMS;  // ids of a workgroup
+  const int rows = a.B * a.S * a.H, n = rows * (PARTS ? (ns + 3) >> 2 : ns);
+  int id = block * APART + (PARTS ? 0 : team);
   bool there = id < n;  // (the other teams of a workgroup come along to its barriers)
-  if ((n & (8 * TEAMS - 1)) == 0) {
-    const int share = n >> 3, mine = (block >> 3) * TEAMS + team;
+  if ((n & (8 * APART - 1)) == 0) {
+    const int share = n >> 3, mine = (block >> 3) * APART + (PARTS ? 0 : team);
     there = mine < share;
     id = (block & 7) * share + mine;
   }
   id = there ? id : 0;
-  const int by = id / rows;
+  int by = id / rows;
   int w = id - by * rows;
+  if (PARTS) {
+    if (!there) return;  // (the whole workgroup)
+    by = 4 * by + team;
+    there = by < ns;
+  }
   const int s = w % a.S; w /= a.S;
   const int h = w % a.H;
   const int seq = w / a.H;
@@ -236,7 +253,7 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
     for (int u = 0; u < 8; ++u) gacc[grp][e0 + u] = acc[u];
   }
   __syncthreads();
-  if (live && tid < D) {
+  if ((PARTS || live) && tid < D) {
     float M = -INFINITY, gv[16];
 #pragma unroll
     for (int g = 0; g < 16; ++g) gv[g] = gacc[g][tid];
@@ -251,7 +268,13 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
       num += in ? wg * gv[g] : 0.f;
       den += in ? wg * gl[g] : 0.f;
     }
-    if (ns > 1) {
+    if (PARTS) {
+      gacc[0][tid] = num;  // (this thread's column)
+      if (tid == 0) {
+        teams_m[team] = M;
+        teams_l[team] = den;
+      }
+    } else if (ns > 1) {
       // write-through stores: the workgroup that merges may sit on another XCD
       float* o = a.ws + (((size_t)row * a.H + h) * a.ns + by) * (D + 2);
       st_coh4(o + tid, __float_as_uint(num));
@@ -262,6 +285,23 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
     } else {
       a.out[(size_t)row * hd + (size_t)h * D + tid] = f2bf(num / den);
     }
+  }
+  if (PARTS) {
+    __syncthreads();
+    if (team || tid >= D) return;
+    float M = -INFINITY, num = 0.f, den = 0.f;
+#pragma unroll
+    for (int i = 0; i < TEAMS; ++i) M = fmaxf(M, teams_m[i]);
+#pragma unroll
+    for (int i = 0; i < TEAMS; ++i) {
+      const bool in = teams_m[i] != -INFINITY;
+      const float wg = expf(teams_m[i] - M);
+      num += in ? wg * gacc_[i][0][tid] : 0.f;
+      den += in ? wg * teams_l[i] : 0.f;
+    }
+    phi_values(a, row, h)[(by >> 2) * D + tid] = num;
+    if (tid == 0) *reinterpret_cast<float2*>(phi_pairs(a, row, h) + 2 * (by >> 2)) = make_float2(M, den);
+    return;
   }
   if (TEAMS == 1 ? ns == 1 : a.ns == 1) return;
 

@@ -723,6 +723,30 @@ def phi_attn_linear(q, kcache, vcache, cos, sin, rot, batch, h, dh, pos, x, w: P
     return out, y
 
 
+def phi_attn_out_chunks(batch, h, dh, rot, n_split, pos, n, k) -> int:
+    """Chunks of a context at most in ``phi_attn_out``; 0 where that call is refused."""
+    return lib().ohara_phi_attn_out_chunks(batch, h, dh, rot, n_split, pos, n, k)
+
+
+def phi_attn_out(q, kcache, vcache, cos, sin, rot, batch, h, dh, pos, x, w: PackedLinear, bias, pos_dev, y, n_split, workspace, w_out: PackedLinear,
+                 bias_out, add, out) -> torch.Tensor:
+    """``phi_attn_linear`` and then ``linear_bias(attention, w_out, bias_out, "add2", add1=y, add2=add)``, whose launch merges the attention's chunks."""
+    if q.stride(1) != 1:
+        raise ValueError("q must have unit column stride")
+    if cos.dtype != torch.float32 or sin.dtype != torch.float32:
+        raise ValueError("cos / sin must be fp32")
+    for t, name, width in ((x, "x", w.k), (y, "y", w.n), (add, "add", w.n), (out, "out", w.n)):
+        if t.dtype != BF16 or not t.is_cuda or t.stride(1) != 1 or t.shape != (batch, width):
+            raise ValueError(f"{name} must be a bf16 device matrix ({batch}, {width}) with unit column stride")
+    if w_out.n != w.n or w_out.k != h * dh or bias.numel() != w.n or bias_out.numel() != w.n:
+        raise ValueError(f"weights are {w.n} x {w.k} and {w_out.n} x {w_out.k} with {bias.numel()} and {bias_out.numel()} biases, heads {h} x {dh}")
+    check(lib().ohara_phi_attn_out_bf16(_ptr(q), q.stride(0), _ptr(kcache), _ptr(vcache), _ptr(cos), _ptr(sin), rot, batch, h, dh, kcache.shape[1], pos,
+                                        _ptr(pos_dev), n_split, _ptr(workspace), _ptr(x), x.stride(0), _ptr(w.data), w.n, w.k, _ptr(bias), _ptr(y),
+                                        y.stride(0), _ptr(w_out.data), _ptr(bias_out), _ptr(add), add.stride(0), _ptr(out), out.stride(0), _stream()),
+          "phi_attn_out")
+    return out
+
+
 # ---- hybrid decoders: attention with a distance bias beside recurrent layers -------------------------
 # bf16 or fp32 activations: the entry point follows the dtype of the activations.
 

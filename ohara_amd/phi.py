@@ -224,6 +224,8 @@ class Phi:
         cur, nxt = buf["x"]
         ops.embed(ids, self.wte, out=cur)
         int8 = kv_cache[0].int8
+        # one token of one or two sequences: the attention's chunks are merged by its output projection
+        merged = S == 1 and ops.phi_attn_out_chunks(B, H, D, self.rot, buf["ns"], start, d, self.ff)
         for L, cache in zip(self.layers, kv_cache):
             ops.layernorm(cur, L["ln_w"], L["ln_b"], c.eps, out=buf["h"])
             if int8:
@@ -246,7 +248,9 @@ class Phi:
                                  cache.value, buf["q"], buf["act"], pos_dev)
                 keys, values = cache.key, cache.value
             att = (buf["q"], keys, values, self.cos, self.sin, self.rot, B)
-            if S == 1 and B <= 16:
+            if merged:
+                ops.phi_attn_out(*att, H, D, start, buf["act"], L["fc2"], L["fc2_b"], pos_dev, buf["mixer"], buf["ns"], buf["ws"], L["dense"], L["dense_b"], cur, nxt)
+            elif S == 1 and B <= 16:
                 # fc2 beside the attention, which it does not wait for; its rounded sums are the first addend of dense instead of the
                 # other way round, the same bits
                 ops.phi_attn_linear(*att, H, D, start, buf["act"], L["fc2"], L["fc2_b"], pos_dev, out=buf["attn"], y=buf["mixer"],
