@@ -694,14 +694,16 @@ int ohara_gemm_residual_norm_bf16(const uint16_t* x, int ldx, const uint16_t* wp
  * (d rows each) and mlp.fc1 (ff rows): q rows -> q (leading dimension ldq), k / v rows -> the
  * caches at position pos + s as they are (un-rotated), fc1 rows -> new_gelu -> act.  Same rounding
  * points as ohara_layernorm_bf16 + ohara_linear_bias_bf16 + ohara_kv_append_bf16, except that the
- * variance comes from the sums of x and x^2.  ln_w == NULL: x already is the normalised input
- * (measured faster at Phi-2's sizes: a separate LayerNorm launch costs less than re-deriving the
- * statistics in each of the 1120 workgroups before their weight loads start).
+ * variance comes from the sums of x and x^2 where ohara_phi_block_norms is 0.  ln_w == NULL: x already is
+ * the normalised input (there a separate LayerNorm launch costs less than re-deriving the statistics
+ * in every workgroup before its weight loads start).
  * d % 16 == 0, ff % 4 == 0. */
 int ohara_phi_block_in_bf16(const uint16_t* x, int ldx, const uint16_t* ln_w, const uint16_t* ln_b, float eps,
                             const uint16_t* wp, const uint16_t* bias, int d, int ff, int batch, int seq_len, int pos,
                             const int32_t* pos_dev, uint16_t* q, int ldq, uint16_t* kcache, uint16_t* vcache, int t_max,
                             uint16_t* act, int ldact, void* stream);
+/* 1 where that call, given ln_w, is quicker than with a launch of ohara_layernorm_bf16 ahead of it (the same bits). */
+int ohara_phi_block_norms(int rows, int d, int ff);
 /* nn.LayerNorm over the last dimension (phi.py:132, :160): fp32 mean and biased variance,
  * out = bf16((x - mean) * rstd * weight + bias).  d % 8 == 0. */
 int ohara_layernorm_bf16(const uint16_t* x, int ldx, const uint16_t* weight, const uint16_t* bias, uint16_t* out, int ldo,

@@ -293,6 +293,114 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
   skinny<BT, NORM, EPI, NW, SP>(a, blockIdx.x);
 }
 
+// Phi's block head (EPI_PHI_IN) on rows before their LayerNorm, one or two, widths up to 256 SP: eight waves a strip, four a row's norm, which is
+// layernorm_kernel's to the bit.  A wave asks for the row, the norm's weight and bias and then for its whole share of the strip, so the statistics and
+// their barriers pass while the weights travel, and the norm's launch, a workgroup a row, is spared.  What it costs is every workgroup's reads of the row and
+// the norm's, 15 KB beside 80 of weights; so two workgroups to a CU, which keep the row and go from strip to strip with the next one's weights ahead of them.
+// us, norm and head / a workgroup a strip / this: 2560 x (7680 + 10240) one row 19.1 / 18.1 / 16.9 (16.4 without a norm), two 19.1 / 18.1 / 17.3; 2048 x (6144 +
+// 8192) 16.1 / 13.9 / 14.6, 15.9 / 13.9 / 14.4.
+template <int SP>
+__global__ __launch_bounds__(512, 4) void phi_in_kernel(GemmArgs a) {
+  constexpr int NW = 8;
+  __shared__ float red[2][NW - 1][64][4], sums[2][2][4];
+  __shared__ __align__(16) bf16_t xs[2][256 * SP];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  const int KS = (a.K + 31) >> 5, per_wave = (KS + NW - 1) / NW;
+  const int j0 = wave * per_wave, j1 = min(KS, j0 + per_wave);
+  const int r = wave >> 2, t = tid & 255, part = wave & 3;
+  const bf16_t* row = a.x + (size_t)min(r, a.B - 1) * a.ldx;
+  uint4 xv[2], nw[2], nb[2], wv[SP];
+  int at[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) at[c] = r < a.B ? (t + 256 * c) * 8 : a.K;  // (wave-uniform: four waves have no row of one)
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if (at[c] < a.K) xv[c] = ldg16(row + at[c]);
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if (at[c] < a.K) {
+      nw[c] = ldg16(a.norm_w + at[c]);
+      nb[c] = ldg16(a.norm_b + at[c]);
+    }
+  EpiPre ep;
+  auto ask = [&](int strip) {
+    const uint4* wrow = a.wp + (size_t)strip * KS * 64 + lane;
+#pragma unroll
+    for (int c = 0; c < SP; ++c) wv[c] = ldg16_nt(wrow + (size_t)min(j0 + c, KS - 1) * 64);
+    if (wave == 0) gemm_epilogue_fetch<EPI_PHI_IN>(a, m, strip, g, ep);
+  };
+  ask(blockIdx.x);
+  __builtin_amdgcn_sched_barrier(0);
+  float s = 0.f;
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if (at[c] < a.K) {
+      const uint32_t u[4] = {xv[c].x, xv[c].y, xv[c].z, xv[c].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s += lo_bf(u[i]) + hi_bf(u[i]);
+    }
+  s = wave_sum(s);
+  if (lane == 0) sums[0][r][part] = s;
+  __syncthreads();
+  const float mean = (((sums[0][r][0] + sums[0][r][1]) + sums[0][r][2]) + sums[0][r][3]) / (float)a.K;
+  float q = 0.f;
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if (at[c] < a.K) {
+      const uint32_t u[4] = {xv[c].x, xv[c].y, xv[c].z, xv[c].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float a0 = lo_bf(u[i]) - mean, a1 = hi_bf(u[i]) - mean;
+        q += a0 * a0 + a1 * a1;
+      }
+    }
+  q = wave_sum(q);
+  if (lane == 0) sums[1][r][part] = q;
+  __syncthreads();
+  const float var = (((sums[1][r][0] + sums[1][r][1]) + sums[1][r][2]) + sums[1][r][3]) / (float)a.K;
+  const float rstd = 1.0f / sqrtf(var + a.eps);
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if (at[c] < a.K) *reinterpret_cast<uint4*>(&xs[r][at[c]]) = lnorm8(xv[c], nw[c], nb[c], mean, rstd);
+  __syncthreads();
+  int into = 0;
+  for (int strip = blockIdx.x; strip < a.nstrips; strip += gridDim.x) {
+    uint4 w[SP];
+#pragma unroll
+    for (int c = 0; c < SP; ++c) w[c] = wv[c];
+    const EpiPre e = ep;
+    f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (strip + (int)gridDim.x < a.nstrips) ask(strip + gridDim.x);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < SP; ++c) {
+      const int k0 = 32 * (j0 + c) + 8 * g;
+      const uint4 x = *reinterpret_cast<const uint4*>(&xs[min(m, 1)][min(k0, a.K - 8)]);
+      const bool live = m < a.B && k0 < a.K;
+      if (j0 + c < j1)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[c]), __builtin_bit_cast(bf16x8, live ? x : make_uint4(0, 0, 0, 0)), acc,
+                                                      0, 0, 0);
+    }
+    if (wave > 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[into][wave - 1][lane][i] = acc[i];
+    }
+    __syncthreads();  // (the sums of the strip after this one go elsewhere; those behind it, past its barrier)
+    if (wave == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int w = 0; w < NW - 1; ++w) acc[i] += red[into][w][lane][i];
+      }
+      if (m < a.B) gemm_epilogue<EPI_PHI_IN, true>(a, m, strip, g, acc, e);
+    }
+    into ^= 1;
+  }
+}
+// (the widths of which a wave's share is eight to ten k-steps; fewer strips are a workgroup of sixteen waves each in skinny_kernel)
+static bool phi_in_norms(int rows, int d, int strips) { return rows <= 2 && d >= 2048 && d <= 2560 && strips >= 400; }
+
 // Phi's attention of single tokens beside the second product of its MLP, which does not wait for it: neither fills the chip - 352 teams of four waves,
 // whose chain of round trips bounds them, and 160 strips - and one after the other they took the sum of their times.  The attention's go first: its
 // chain is the longer one.  (Fewer of the product's loads in flight, 2 to 7 k-steps instead of 10, leave the times as they are.)
@@ -1240,9 +1348,16 @@ int ohara_phi_block_in_bf16(const uint16_t* x, int ldx, const uint16_t* ln_w, co
   a.out = q; a.ldo = ldq; a.out2 = act; a.ldo2 = ldact; a.split_n = 3 * d; a.bias = bias;
   a.S = seq_len; a.Tmax = t_max; a.pos = pos; a.pos_dev = pos_dev; a.kcache = kcache; a.vcache = vcache;
   const int packed_rows = (a.N + 15) / 16 * 16;
+  if (ln_w && phi_in_norms(a.B, d, packed_rows / 16) && !(((uintptr_t)ln_w | (uintptr_t)ln_b | (uintptr_t)x) & 15)) {
+    a.nstrips = packed_rows / 16;
+    hipLaunchKernelGGL(phi_in_kernel<10>, dim3((unsigned)std::min(a.nstrips, 512)), dim3(512), 0, (hipStream_t)stream, a);
+    return ohara_launch_status();
+  }
   if (!ln_w && ohara_tiles_win(a.B, a.K, packed_rows)) return ohara_launch_gemm_tile(a, EPI_PHI_IN, packed_rows, (hipStream_t)stream);  // prefill
   return launch_skinny(a, EPI_PHI_IN, packed_rows, (hipStream_t)stream);
 }
+
+int ohara_phi_block_norms(int rows, int d, int ff) { return rows > 0 && d > 0 && ff > 0 && ff < (1 << 28) && phi_in_norms(rows, d, (3 * d + ff + 15) / 16); }
 
 int ohara_gemm_softcap_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k, float cap, int rows,
                             uint16_t* out, int ldo, void* stream) {

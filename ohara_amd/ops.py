@@ -645,6 +645,11 @@ def linear_bias(x, w: PackedLinear, bias, epilogue: str = "bias", add1=None, add
     return out
 
 
+def phi_block_norms(rows, d, ff) -> bool:
+    """Whether ``phi_block_in`` on rows before their LayerNorm is quicker than ``layernorm`` ahead of it."""
+    return bool(lib().ohara_phi_block_norms(rows, d, ff))
+
+
 def phi_block_in(x, ln_w, ln_b, eps, w: PackedLinear, bias, d, ff, batch, seq_len, pos, kcache, vcache, q, act,
                  pos_dev=None) -> None:
     """LayerNorm + [q; k; v; fc1] projection with bias + cache append + new_gelu in one launch

@@ -226,15 +226,19 @@ class Phi:
         int8 = kv_cache[0].int8
         # one token of one or two sequences: the attention's chunks are merged by its output projection
         merged = S == 1 and ops.phi_attn_out_chunks(B, H, D, self.rot, buf["ns"], start, d, self.ff)
+        norms = ops.phi_block_norms(rows, d, self.ff)
         for L, cache in zip(self.layers, kv_cache):
-            ops.layernorm(cur, L["ln_w"], L["ln_b"], c.eps, out=buf["h"])
+            if norms:
+                h, ln_w, ln_b = cur, L["ln_w"], L["ln_b"]
+            else:
+                h, ln_w, ln_b = ops.layernorm(cur, L["ln_w"], L["ln_b"], c.eps, out=buf["h"]), None, None
             if int8:
                 # kv_cache.py:94-118 with quantisation: the new (un-rotated) rows are quantised into the cache and
                 # attention runs over what the reference's cache read returns - the dequantised prefix, the new rows
                 # included - as a bf16 working copy (the rotary attention kernel reads bf16 rows)
                 sk = torch.empty(B, S, H, D, dtype=BF16, device=self.device)
                 sv = torch.empty_like(sk)
-                ops.phi_block_in(buf["h"], None, None, c.eps, L["w_in"], L["b_in"], d, self.ff, B, S, 0, sk, sv, buf["q"],
+                ops.phi_block_in(h, ln_w, ln_b, c.eps, L["w_in"], L["b_in"], d, self.ff, B, S, 0, sk, sv, buf["q"],
                                  buf["act"])
                 ops.kv_quant_append(sk, sv, cache, start, pos_dev=pos_dev)
                 # (with the position on the device - a captured step - the copy covers the cache's whole capacity:
@@ -244,7 +248,7 @@ class Phi:
                 vd = ops.kv_dequant(cache, "value", B, live)
                 keys, values = kd, vd
             else:
-                ops.phi_block_in(buf["h"], None, None, c.eps, L["w_in"], L["b_in"], d, self.ff, B, S, start, cache.key,
+                ops.phi_block_in(h, ln_w, ln_b, c.eps, L["w_in"], L["b_in"], d, self.ff, B, S, start, cache.key,
                                  cache.value, buf["q"], buf["act"], pos_dev)
                 keys, values = cache.key, cache.value
             att = (buf["q"], keys, values, self.cos, self.sin, self.rot, B)
