@@ -98,7 +98,8 @@ int ohara_gemm_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k
 int ohara_projection_norm_ahead(int rows, int k, int packed_rows);
 /* The tile of such a product over rows that start on 16 bytes: 1000 * its rows + its packed rows (SwiGLU packs two a column). */
 int ohara_gemm_tile_of(int rows, int packed_rows, int k);
-/* The same of a product with an epilogue (as below), or of its sums in parts of the depth (parts > 1, which divide k; then the epilogue does not matter). */
+/* The same of a product with an epilogue (as below), or of its sums in parts of the depth (parts > 1, which divide k; then the epilogue does not matter);
+ * 1 more where it is one of the tiles in halves. */
 int ohara_gemm_tile_with(int rows, int packed_rows, int k, int epilogue, int parts);
 /* How many of the rows go first, where they take two launches (0: one).  epilogue: 0 store, 1 residual, 2 SwiGLU, 3 rotary with heads of dh, 4 bias, 6 bias and
  * two addends, 5 and 7 to 11 the arithmetic ones (bias and gelu, Phi's input, soft cap, gelu times an embedding, gated units, two-sided activation). */

@@ -572,13 +572,24 @@ constexpr TileTime FEW[19] = {
     {T32::TM, T32::TS, 3, 0.147f, 0.412f, 0.081f, 0.482f},          {T64::TM, T64::TS, 2, 0.302f, 0.252f, 0.208f, 0.779f},
     {T64x128::TM, T64x128::TS, 2, 0.374f, 0.684f, 0.337f, 1.577f},  {T128::TM, T128::TS, 2, 0.637f, 0.476f, 0.563f, 1.948f},
     {T128x192::TM, T128x192::TS, 2, 0.756f, 0.68f, 0.68f, 3.227f},  {T256::TM, T256::TS, 1, 1.35f, 0.f, 1.6f, 6.7f},
-    {H128x256::TM, H128x256::TS}, {H128x192::TM, H128x192::TS},     // (not among them)
+    {H128x256::TM, H128x256::TS}, {H128x192::TM, H128x192::TS},     // (below)
     {T64x48::TM, T64x48::TS, 1, 0.195f, 0.254f, 0.228f, 1.248f},    {T64x96::TM, T64x96::TS, 1, 0.287f, 0.234f, 0.336f, 1.634f},
     {T48x64::TM, T48x64::TS, 1, 0.199f, 0.191f, 0.231f, 1.229f},    {T80x64::TM, T80x64::TS, 1, 0.261f, 0.193f, 0.302f, 1.51f},
     {T96x64::TM, T96x64::TS, 2, 0.358f, 0.406f, 0.256f, 1.253f},    {T96::TM, T96::TS, 1, 0.355f, 0.242f, 0.426f, 1.968f},
     {T128x96::TM, T128x96::TS, 1, 0.441f, 0.181f, 0.507f, 2.426f},  {W64::TM, W64::TS, 1, 0.23f, 0.19f, 0.264f, 1.314f},
     {W128::TM, W128::TS, 1, 0.468f, 0.247f, 0.592f, 2.966f},        {W128x192::TM, W128x192::TS, 1, 0.599f, 0.262f, 0.758f, 4.159f},
     {T192x128::TM, T192x128::TS, 1, 0.6f, 0.25f, 0.764f, 4.011f},
+};
+// Tiles in halves among them: slower than the others until the operands of a large product come through them, and then by as much as a quarter
+// quicker.  Fitted to 9400 products of 200 to 1023 rows (1024 to 18000 packed rows, K 384 to 4096, weights of HBM), and compared with the times above and what those
+// lack on the same products, 2 us, with an arithmetic epilogue 4; no fewer tiles than leave most CUs idle, no less depth than the fit holds for.  Of those
+// products 3900 change, 9 % quicker on average, 180 lose more than 3 %; of 1760 with rotary 650 change (14 %, none loses), of 1820 heads of Phi blocks 600 (6 %), of 2390
+// products in parts 1600 (10 %, 70 lose).  us, before / in halves: 512 rows 11264 x 2048 with SwiGLU 32.7 / 28.0, 1000 rows 48.7 / 44.4; 700 rows 6144 x 768
+// 13.6 / 12.3; 700 rows 7680 x 2560 42.0 / 34.3; 700 rows 2560 x 10240 in four parts with their merge 51.7 / 47.4, 450 rows 48.3 / 39.4.
+constexpr TileTime HALVES[3] = {
+    {T256::TM, T256::TS, 1, 0.521f, 1.671f, 1.479f, 11.155f},
+    {H128x256::TM, H128x256::TS, 1, 0.507f, 0.766f, 0.768f, 6.323f},
+    {H128x192::TM, H128x192::TS, 1, 0.437f, 0.736f, 0.627f, 5.293f},
 };
 int few_rows_tile(int rows, int strips, int K, Epilogue epi) {
   const int now = fastest_tile(rows, strips, K, epi);
@@ -590,6 +601,18 @@ int few_rows_tile(int rows, int strips, int K, Epilogue epi) {
     if (t < low) {
       low = t;
       best = i;
+    }
+  }
+  if (K < 768) return best;
+  low = tile_time(FEW[best], rows, strips, K) + (epi == HEAVY ? 4.f : 2.f);
+  for (int i = 0; i < 3; ++i) {
+    const TileTime& h = HALVES[i];
+    if (((int64_t)rows + h.rows - 1) / h.rows * ((strips + h.strips - 1) / h.strips) < (i ? 96 : 136)) continue;
+    const float extra = epi == HEAVY ? (i ? 3.f : 6.f) : epi >= ROTARY_32 ? EXTRA[epi][LARGEST + i] : 0.f;
+    const float t = tile_time(h, rows, strips, K, extra);
+    if (t < low) {
+      low = t;
+      best = LARGEST + i;
     }
   }
   return best;
@@ -757,7 +780,7 @@ extern "C" int ohara_gemm_tile_with(int rows, int packed_rows, int k, int epilog
   if (rows < 1 || packed_rows < 1 || k < 1 || epilogue < EPI_STORE || epilogue > EPI_BIAS_XIELU || parts < 1 || k % parts) return OHARA_EINVAL;
   const int strips = (packed_rows + 15) / 16;
   const int i = parts > 1 ? few_rows_tile(rows, strips * parts, k / parts, PLAIN) : tile_of(rows, strips, k, epilogue, epilogue_of(epilogue, 64, false));
-  return FEW[i].rows * 1000 + FEW[i].strips * 16;
+  return FEW[i].rows * 1000 + FEW[i].strips * 16 + (i >= LARGEST && i < LARGEST + 3);
 }
 
 extern "C" int ohara_gemm_first_rows(int rows, int packed_rows, int k, int epilogue, int dh) {
