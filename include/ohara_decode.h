@@ -729,6 +729,8 @@ int64_t ohara_phi_attn_workspace_bytes(int batch, int h, int dh, int n_split);
 int ohara_phi_attn_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, const uint16_t* vcache, const float* cos,
                         const float* sin, int rot, int batch, int seq_len, int h, int dh, int t_max, int pos,
                         const int32_t* pos_dev, int n_split, void* workspace, uint16_t* out, void* stream);
+// In how many teams of waves a workgroup of such a prefill shares its queries' positions (rotated features in eights).
+int ohara_phi_prefill_teams(int batch, int seq_len, int h, int pos);
 // The same for one token a sequence, and beside it a product that does not wait for it: y = x W^T + bias as ohara_linear_bias_bf16 gives it,
 // x (batch, k), y (batch, n).  Neither may read what the other writes.  Where pos_dev is given, `pos` is about
 // where it will be: how far back the attention goes decides whether one launch or two are quicker.

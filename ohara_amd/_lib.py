@@ -206,6 +206,7 @@ _PROTOS = {
     "ohara_phi_attn_workspace_bytes": (_i64, [_i, _i, _i, _i]),
     "ohara_phi_attn_bf16": (_i, [_p, _i, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _i, _p, _p, _p]),
     "ohara_phi_attn_linear_bf16": (_i, [_p, _i, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _i, _p, _p, _p, _i, _p, _i, _i, _p, _p, _i, _p]),
+    "ohara_phi_prefill_teams": (_i, [_i, _i, _i, _i]),
     "ohara_phi_attn_linear_chunks": (_i, [_i, _i, _i, _i, _i, _i, _i]),
     "ohara_phi_attn_out_bf16": (_i, [_p, _i, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _i, _p, _p, _i, _p, _i, _i, _p, _p, _i, _p, _p, _p, _i, _p, _i, _p]),
     "ohara_phi_attn_out_chunks": (_i, [_i, _i, _i, _i, _i, _i, _i, _i]),

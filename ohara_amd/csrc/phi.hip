@@ -167,6 +167,7 @@ __device__ __forceinline__ void phi_walk_rows(const PhiAttnArgs& a, int seq, int
 // are twice the products' cycles.  32 heads of 80, us with fp32 products and tiles of 32 / so: 100 tokens 14.7 / 9.6, 300 30 / 15.5, 700 68 / 28, 1500
 // 157 / 60, 2040 281 / 98; 2 x 700 76 / 33, 4 x 1500 580 / 213; 64 behind 1000 93 / 37.  Results that differ from the rounded ones of 64 bits: 700 tokens
 // 0.030 / 0.019 %, 2040 0.044 / 0.029 %.
+// TEAMS = 2: two such fours of waves with tiles of their own take turns along the positions, and add up at the end (phi_teams).
 template <int DT, int NR>  // head width / 16; chunks of 32 features with rotated ones among them
 struct PhiTile {
   static constexpr int D = 16 * DT, NC = (D + 31) / 32;
@@ -177,14 +178,16 @@ struct PhiTile {
   static constexpr int T = 4 * 64 * (KROW + VROW) <= 160 * 1024 ? 64 : 32, BUF = T * (KROW + VROW);
   static __device__ __forceinline__ constexpr int byte_of(int feature) { return 2 * feature + (feature < 32 * NR ? 0 : 2 * PLANE); }
 };
-template <int DT, int NR>
-__global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a, int nqb, int heads) {
+template <int DT, int NR, int TEAMS>
+__global__ __launch_bounds__(256 * TEAMS, 2) void phi_attn_prefill_kernel(PhiAttnArgs a, int nqb, int heads) {
   typedef PhiTile<DT, NR> L;
   constexpr int D = L::D, NC = L::NC, T = L::T, QB = 64;
   // a thread's parts of a tile: fours of rotated pairs, eighths of the other features, of values
   constexpr int NP = (NR * T + 63) / 64, CE = 2 * DT - 4 * NR + 2, NU = CE > 0 ? (CE * T + 255) / 256 : 1, NV = (2 * DT * T + 255) / 256;
-  extern __shared__ __align__(16) unsigned char smem[];  // two tiles
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  extern __shared__ __align__(16) unsigned char all[];  // two tiles a team
+  const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), tid = TEAMS == 1 ? threadIdx.x : threadIdx.x & 255;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  unsigned char* const smem = all + team * 2 * L::BUF;
   const int l16 = lane & 15, g = lane >> 4;
   const int half = a.rot >> 1;
   // an XCD (ids go round-robin over the eight) gets every eighth head; long contexts first
@@ -283,7 +286,7 @@ __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a,
         n1[c] = ldg16(a.sin + at + 4);
       }
     }
-    fetch(0);
+    fetch(team * T);
     // what no tile's part is put on: features past the head, second and third terms of those that are not rotated
     for (int i = tid; i < 2 * T * (L::KROW / 16); i += 256) {
       const int r = i / (L::KROW / 16);
@@ -407,9 +410,10 @@ __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a,
   };
   constexpr bool BOTH = T == 64 && NC + 2 * NR <= 5;  // (more fragments than that do not fit)
   uint32_t cur = 0;
-  for (int t0 = 0; t0 <= t_end; t0 += T) {
-    const bool more = t0 + T <= t_end;
-    if (more) fetch(t0 + T);  // in flight during this tile's products
+  for (int round = 0; round <= t_end; round += TEAMS * T) {  // (the last round may have no tile for the second team)
+    const int t0 = round + team * T, next = t0 + TEAMS * T;
+    const bool more = next <= t_end;
+    if (more) fetch(next);  // in flight during this tile's products
     const uint32_t kt = lds0 + cur + kat, vt = lds0 + cur + vat;
     if (BOTH && t0 + 32 <= wave_hi) {
       window(std::integral_constant<int, 2>(), t0, kt, vt);
@@ -422,6 +426,28 @@ __global__ __launch_bounds__(256, 2) void phi_attn_prefill_kernel(PhiAttnArgs a,
     __syncthreads();
   }
   lsum = lane_xor_sum<32>(lane_xor_sum<16>(lsum));
+  if constexpr (TEAMS == 2) {  // the second team's sums, weighted to the larger of the two maxima (whole numbers: exactly)
+    constexpr int N = 4 * DT + 2;
+    static_assert(4 * N * 64 * 4 <= 2 * TEAMS * L::BUF, "");
+    float* there = reinterpret_cast<float*>(all) + (wave * N) * 64 + lane;
+    if (team) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) there[(4 * t + i) * 64] = o[t][i];
+      there[(N - 2) * 64] = m;
+      there[(N - 1) * 64] = lsum;
+    }
+    __syncthreads();
+    if (team) return;
+    const float m2 = there[(N - 2) * 64], M = fmaxf(m, m2);
+    const float w1 = pow2_neg_int(m - M), w2 = m2 == -INFINITY ? 0.f : pow2_neg_int(m2 - M);
+    lsum = lsum * w1 + there[(N - 1) * 64] * w2;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[t][i] = o[t][i] * w1 + there[(4 * t + i) * 64] * w2;
+  }
   float sum = lsum;
 #pragma unroll
   for (int t = 0; t < DT; ++t) sum += (o[t][0] + o[t][1]) + (o[t][2] + o[t][3]);
@@ -622,22 +648,44 @@ __global__ __launch_bounds__(256, 2) void phi_attn_pairs_kernel(PhiAttnArgs a, i
   }
 }
 
+// Teams of a workgroup: two where the longest chain of tiles is what the launch takes - workgroups to a CU each, or fewer tiles to a CU than
+// four fifths of that chain - and has some tiles to share.  us, one / two, 32 heads of 80: 128 tokens 10.0 / 10.0, 300 15.6 / 14.2, 500 21.7 / 18.8, 700 27.6 / 23.3,
+// 1500 59.8 / 71.4, 2 x 300 16.4 / 17.7, 4 x 200 14.8 / 19.8, 200 behind 500 27.7 / 23.1, 64 behind 1500 52.3 / 41.6; 24 of 128, 700 tokens 35.4 / 28.7; 16 of 64, all
+// rotated, 1000 39.1 / 31.0, 16 x 16 behind 300 17.3 / 15.6; 40 of 128, 64 rotated, 500 31.6 / 27.1, 800 44.6 / 50.8.
+int phi_teams(int64_t batch, int64_t S, int64_t h, int64_t pos) {
+  const int64_t blocks = (S + PF_Q - 1) / PF_Q, heads = batch * h, longest = (pos + S + 63) / 64;
+  const int64_t all = heads * blocks * (pos / 64) + heads * blocks * (blocks + 1) / 2;  // tiles, about
+  if (longest < 4) return 1;
+  return blocks * ((heads + 7) / 8 * 8) <= 256 || (longest >= 8 && 5 * all <= 4 * 256 * longest) ? 2 : 1;
+}
+
 template <int DT>
 int launch_phi_prefill(const PhiAttnArgs& a, int batch, hipStream_t st) {
   const int64_t nqb = (a.S + PF_Q - 1) / PF_Q, heads = (int64_t)a.H * batch, grid = nqb * ((heads + 7) / 8 * 8);
   if (grid > INT32_MAX) return OHARA_ESIZE;
-  auto launch = [&](auto kernel, int lds) {
-    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), lds, st, a, (int)nqb, (int)heads);
+  if (!phi_eights(a)) {
+    constexpr int LDS = 2 * 2 * PF_T * (16 * DT + 4) * (int)sizeof(float);
+    if (LDS > 64 * 1024) (void)hipFuncSetAttribute((const void*)phi_attn_pairs_kernel<DT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    hipLaunchKernelGGL(phi_attn_pairs_kernel<DT>, dim3((unsigned)grid), dim3(256), LDS, st, a, (int)nqb, (int)heads);
     return ohara_launch_status();
-  };
-  if (!phi_eights(a)) return launch(phi_attn_pairs_kernel<DT>, 2 * 2 * PF_T * (16 * DT + 4) * (int)sizeof(float));
+  }
   constexpr int NC = (DT + 1) / 2;  // a.rot is at most 16 DT
+  auto of = [&](auto chunks) {
+    constexpr int NR = decltype(chunks)::value < NC ? decltype(chunks)::value : NC, BUF = PhiTile<DT, NR>::BUF;
+    auto by = [&](auto teams) {
+      constexpr int TEAMS = decltype(teams)::value, LDS = TEAMS * 2 * BUF;
+      auto kernel = phi_attn_prefill_kernel<DT, NR, TEAMS>;
+      if (LDS > 64 * 1024) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256 * TEAMS), LDS, st, a, (int)nqb, (int)heads);
+      return ohara_launch_status();
+    };
+    return phi_teams(batch, a.S, a.H, a.pos) == 2 ? by(std::integral_constant<int, 2>()) : by(std::integral_constant<int, 1>());
+  };
   switch ((a.rot + 31) / 32) {
-    case 1: return launch(phi_attn_prefill_kernel<DT, 1>, 2 * PhiTile<DT, 1>::BUF);
-    case 2: return launch(phi_attn_prefill_kernel<DT, NC < 2 ? NC : 2>, 2 * PhiTile<DT, NC < 2 ? NC : 2>::BUF);
-    case 3: return launch(phi_attn_prefill_kernel<DT, NC < 3 ? NC : 3>, 2 * PhiTile<DT, NC < 3 ? NC : 3>::BUF);
-    default: return launch(phi_attn_prefill_kernel<DT, NC < 4 ? NC : 4>, 2 * PhiTile<DT, NC < 4 ? NC : 4>::BUF);
+    case 1: return of(std::integral_constant<int, 1>());
+    case 2: return of(std::integral_constant<int, 2>());
+    case 3: return of(std::integral_constant<int, 3>());
+    default: return of(std::integral_constant<int, 4>());
   }
 }
 
@@ -730,6 +778,10 @@ int ohara_phi_attn_out_bf16(const uint16_t* q, int ldq, const uint16_t* kcache, 
   o.out = out; o.ldo = ldo; o.bias = bias_out;
   o.resid = y; o.ldr = ldy; o.resid2 = add; o.ldr2 = ld_add;
   return ohara_launch_phi_attn_out(t, a, o, (hipStream_t)stream);
+}
+
+int ohara_phi_prefill_teams(int batch, int seq_len, int h, int pos) {
+  return batch < 1 || seq_len < 1 || h < 1 || pos < 0 ? OHARA_EINVAL : phi_teams(batch, seq_len, h, pos);
 }
 
 }  // extern "C"

@@ -48,13 +48,29 @@ def test_every_number_of_chunks(cuda, B, S, H, pos, D, rot):
         assert ((got[b].double() - want).abs() <= want.abs() * 2.0 ** -8 + mass * (D * 2.0 ** -18) + 1e-30).all()
 
 
-@pytest.mark.parametrize("at", [0, 20, 63, 64, 99])
-def test_infinities(cuda, at):
+@pytest.mark.parametrize("D,rot", [(32, 16), (64, 64), (80, 32), (128, 96), (128, 128)])
+@pytest.mark.parametrize("B,S,H,pos,teams", [(1, 193, 3, 0, 2), (1, 257, 2, 0, 2), (2, 16, 5, 240, 2), (1, 70, 3, 187, 2), (1, 130, 9, 380, 2), (1, 600, 32, 0, 2), (4, 200, 17, 0, 1),
+                                             (1, 192, 3, 0, 1)])
+def test_two_teams(cuda, B, S, H, pos, teams, D, rot):
+    """The last round with a tile for one team and for both, waves that see nothing of the second one's, on either side of the rule."""
+    from ohara_amd import ops
+    from ohara_amd._lib import lib
+
+    assert lib().ohara_phi_prefill_teams(B, S, H, pos) == teams
+    q, k, v, cos, sin = _case(cuda, B, S, H, D, rot, pos)
+    got = ops.phi_attn(q.view(B * S, H * D), k, v, cos, sin, rot, B, S, H, D, pos).view(B, S, H, D)
+    b = B - 1
+    want, mass = _plain(q[b], k[b], v[b], cos, sin, rot, pos)
+    assert ((got[b].double() - want).abs() <= want.abs() * 2.0 ** -8 + mass * (D * 2.0 ** -18) + 1e-30).all()
+
+
+@pytest.mark.parametrize("S,at", [(100, 0), (100, 20), (100, 63), (100, 64), (100, 99), (200, 63), (200, 64), (200, 130), (200, 199)])
+def test_infinities(cuda, S, at):
     """A key of minus infinity in a feature that is not rotated has no weight, one in a rotated feature may have none; an infinite value reaches the
     queries that see it."""
     from ohara_amd import ops
 
-    S, H, D, rot = 100, 3, 80, 32
+    H, D, rot = 3, 80, 32
     for what in ("plain key", "rotated key", "value"):
         q, k, v, cos, sin = _case(cuda, 1, S, H, D, rot, 0)
         q, k = q.abs() + 0.25, k.clone()
