@@ -334,7 +334,7 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
 
 // A workgroup a CU, which takes every 32nd tile of its XCD's run, where there are more tiles than CUs.  Its loads run from one tile into the next: what
 // halves_stream asks for in a tile's last steps are the first steps of the one behind it, which arrive under the epilogue.
-// us, a workgroup a tile / this: 8192 rows 6144 x 768 with SwiGLU 77.8 / 73.2, plain 77.2 / 73.3, 384 deep 55.8 / 48.6; 4001 rows 11264 x 2048 with SwiGLU 151 /
+// us, a workgroup a tile / this: 8192 rows 6144 x 768 with SwiGLU 77.8 / 73.2 (66 to 69 with the shorter silu), plain 77.2 / 73.3, 384 deep 55.8 / 48.6; 4001 rows 11264 x 2048 with SwiGLU 151 /
 // 144, 11200 rows 399 / 377; 8192 rows 7680 x 2560 237 / 233.  What is left of a boundary there, 8 of 24 us a tile: the epilogue's arithmetic (SwiGLU 4 us), or where
 // much is stored the memory (100 MB of a plain store 16.6 of 72.3 us); zeros instead of random numbers 53 us: the chip's clock under its load.
 template <int EPI, class C>
