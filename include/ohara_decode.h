@@ -96,7 +96,8 @@ int ohara_gemm_bf16(const uint16_t* x, int ldx, const uint16_t* wp, int n, int k
 /* 1 where rows are best normed ahead of their projection (norm_w then NULL) and not by it: more than 64, more than 32 where k > 1024 and the
  * packed rows are many, more than 16 where k > 2048.  What ohara_llama_forward does by itself. */
 int ohara_projection_norm_ahead(int rows, int k, int packed_rows);
-/* The tile of such a product over rows that start on 16 bytes: 1000 * its rows + its packed rows (SwiGLU packs two a column). */
+/* The tile of such a product over rows that start on 16 bytes: 1000 * its rows + its packed rows (SwiGLU packs two a column).  Under 1024 rows and from 20000
+ * packed rows on the call below says which one a plain store runs. */
 int ohara_gemm_tile_of(int rows, int packed_rows, int k);
 /* The same of a product with an epilogue (as below), or of its sums in parts of the depth (parts > 1, which divide k; then the epilogue does not matter);
  * 1 more where it is one of the tiles in halves. */

@@ -566,7 +566,7 @@ int fastest_tile(int rows, int strips, int K, Epilogue epi = PLAIN) {
 // tile alone on its CU within 3 to 5 %, of those that share one within 7 to 12 %.  Such a tile is taken where they promise 4 % (10 with an arithmetic
 // epilogue, whose waves hold more of it): of the 1201 products with a choice 340 change, 12 % quicker on average (as much as 30), 21 lose more than 3 %, the worst 9
 // (768 x 3072 in two parts, 860 rows: 10.7 / 11.7).  us, before / now: 224 rows 11264 x 2048 with SwiGLU 26.7 / 21.1, 320 rows 3072 x 2048 14.9 / 11.4, 1000 rows
-// 27.7 / 20.4, 400 rows 15.4 / 13.1.  A plain store keeps the tiles above: no model has one but for its vocabulary, whose rounds are many.
+// 27.7 / 20.4, 400 rows 15.4 / 13.1.
 constexpr int NEW_TILES = 10;  // the first of these tiles
 constexpr TileTime FEW[19] = {
     {T32::TM, T32::TS, 3, 0.147f, 0.412f, 0.081f, 0.482f},          {T64::TM, T64::TS, 2, 0.302f, 0.252f, 0.208f, 0.779f},
@@ -617,9 +617,12 @@ int few_rows_tile(int rows, int strips, int K, Epilogue epi) {
   }
   return best;
 }
-constexpr bool has_new_tiles(int epi) { return epi == EPI_RESIDUAL || epi == EPI_SWIGLU || epi == EPI_ROPE || epi == EPI_PHI_IN; }
+constexpr bool has_new_tiles(int epi) { return epi == EPI_RESIDUAL || epi == EPI_SWIGLU || epi == EPI_ROPE || epi == EPI_PHI_IN || epi == EPI_STORE; }
+// A plain store has them from 20000 packed rows on: a vocabulary, which no other plain store of a model comes near.  us, without / with: 32000 x 2048, 128, 192, 256, 384,
+// 700 rows 35.7 40.7 45.7 52.2 94.7 / 36.2 34.0 40.5 51.7 88.5; 65536 x 768, 128, 300, 384 rows 28.4 48.4 55.9 / 28.1 43.3 49.1; 51200 x 2560, 300, 700 rows 120.8
+// 194.8 / 107.1 164.6.
 int tile_of(int rows, int strips, int K, int epi, Epilogue kind) {
-  return has_new_tiles(epi) ? few_rows_tile(rows, strips, K, kind) : fastest_tile(rows, strips, K, kind);
+  return has_new_tiles(epi) && (epi != EPI_STORE || strips >= 1250) ? few_rows_tile(rows, strips, K, kind) : fastest_tile(rows, strips, K, kind);
 }
 
 // A part of the rows in whole rounds of 256 x 256, one a CU, and the rest by itself, where the last round would be nearly empty (0 rows: all in one launch).

@@ -38,6 +38,23 @@ def test_residual_and_gated(cuda, tile, rows, packed, k):
         assert torch.equal(ops.gemm(x, gates), torch.cat([ops.gemm(x[s], gates) for s in spans]))
 
 
+# ... of a vocabulary's plain store, whose other products run the tile of ohara_gemm_tile_of
+@pytest.mark.parametrize("tile,rows,packed,k", [(96064, 66, 32016, 2056), (96096, 66, 20016, 776), (128096, 97, 20016, 776), (192128, 192, 32016, 1032), (128193, 193, 20016, 776),
+                                                (128257, 193, 32016, 1032), (128192, 300, 32016, 1032), (256257, 385, 32016, 1032), (256257, 700, 20016, 768)])
+def test_vocabulary(cuda, tile, rows, packed, k):
+    from ohara_amd import ops
+    from ohara_amd._lib import lib
+
+    assert lib().ohara_gemm_tile_with(rows, packed, k, 0, 1) == tile
+    assert lib().ohara_gemm_tile_with(rows, 17936, k, 0, 1) == lib().ohara_gemm_tile_of(rows, 17936, k) + (lib().ohara_gemm_tile_of(rows, 17936, k) == 256256)
+    g = torch.Generator(device=cuda).manual_seed(rows + packed + k)
+    x = (torch.randn(rows, k, generator=g, device=cuda) * 3).to(BF)
+    w = (torch.randn(packed, k, generator=g, device=cuda) * 0.3).to(BF)
+    for n in (packed, packed - 5):
+        wp = ops.pack_linear(w[:n].contiguous())
+        assert torch.equal(ops.gemm(x, wp), torch.cat([ops.gemm(x[r:r + 32], wp) for r in range(0, rows, 32)]))
+
+
 # tile, head width, query heads, key heads, sequences, positions of each, K
 ROTARY = [
     (48064, 48, 10, 2, 3, 267, 1032), (80064, 128, 16, 4, 1, 341, 1032), (96064, 128, 16, 4, 2, 228, 2056), (96096, 80, 32, 32, 2, 136, 2056),
