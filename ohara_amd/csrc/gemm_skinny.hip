@@ -451,8 +451,8 @@ __global__ __launch_bounds__(1024) void phi_dense_kernel(PhiAttnArgs t, GemmArgs
   __builtin_amdgcn_sched_barrier(0);
   const int ns = (max(pos, 0) / phi_chunk(max(pos, 0), t.ns) >> 2) + 1;
   {
-    const bool in = pc < ns && pair.x != -INFINITY;
-    float M = in ? pair.x : -INFINITY;
+    const bool in = pc < ns;
+    float M = in ? pair.x : PHI_LOWEST;
 #pragma unroll
     for (int x = 1; x < NCH; x *= 2) M = fmaxf(M, __shfl_xor(M, x));
     const float wg = expf(pair.x - M);

@@ -73,6 +73,11 @@ int ohara_launch_phi_attn_out(PhiAttnArgs t, GemmArgs a, GemmArgs out, hipStream
 
 namespace {
 
+// Where a maximum of scores begins, the lowest finite number: a score of minus infinity then has the weight zero, as what came before a finite score has, and
+// nothing has to be left out where sums are merged - what saw no position adds zeros, a score that is not a number its NaN.  (From minus infinity on, a group
+// of lanes whose scores are all NaN, which a maximum ignores, looks like one that saw no position.)  The merges' products are rounded by themselves, in all kernels.
+constexpr float PHI_LOWEST = -__FLT_MAX__;
+
 // Where the sums of four chunks go that the next launch merges (phi_dense_kernel): values on 16 bytes, then {max, sum}.  a.ns is a multiple of four.
 __device__ __forceinline__ float* phi_values(const PhiAttnArgs& a, int row, int h) { return a.ws + ((size_t)row * a.H + h) * (a.ns >> 2) * a.D; }
 __device__ __forceinline__ float* phi_pairs(const PhiAttnArgs& a, int row, int h) {
@@ -208,7 +213,7 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
   }
   const float scale = sqrtf(1.0f / (float)D);
 
-  float m = -INFINITY, lsum = 0.f, acc[8];
+  float m = PHI_LOWEST, lsum = 0.f, acc[8];
 #pragma unroll
   for (int u = 0; u < 8; ++u) acc[u] = 0.f;
   for (int t = t_lo + grp; t <= t_hi;) {
@@ -230,7 +235,7 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
       const float sc = part * scale;
       const float mn = fmaxf(m, sc);
       // hardware exponential: its error (about 1e-6 relative) is far below the bf16 rounding of the output
-      const float corr = __expf(m - mn), p = __expf(sc - mn);  // m = -inf on the first round: corr = 0
+      const float corr = __expf(m - mn), p = __expf(sc - mn);
       lsum = lsum * corr + p;
       const uint32_t vu[4] = {vv[r].x, vv[r].y, vv[r].z, vv[r].w};
 #pragma unroll
@@ -254,7 +259,7 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
   }
   __syncthreads();
   if ((PARTS || live) && tid < D) {
-    float M = -INFINITY, gv[16];
+    float M = PHI_LOWEST, gv[16];
 #pragma unroll
     for (int g = 0; g < 16; ++g) gv[g] = gacc[g][tid];
 #pragma unroll
@@ -263,10 +268,10 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
 #pragma unroll
     for (int g = 0; g < 16; ++g) {  // (no branch: every read would be waited for behind it; with the merge's below, whose values are asked for
                                     // with the maxima: 32 heads of 80 behind 700 13.1 -> 11.2 us)
-      const bool in = gm[g] != -INFINITY;  // (not a group that saw no position, nor one whose scores are all -inf, which holds NaN)
+#pragma clang fp contract(off)
       const float wg = expf(gm[g] - M);
-      num += in ? wg * gv[g] : 0.f;
-      den += in ? wg * gl[g] : 0.f;
+      num += wg * gv[g];
+      den += wg * gl[g];
     }
     if (PARTS) {
       gacc[0][tid] = num;  // (this thread's column)
@@ -289,15 +294,15 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
   if (PARTS) {
     __syncthreads();
     if (team || tid >= D) return;
-    float M = -INFINITY, num = 0.f, den = 0.f;
+    float M = PHI_LOWEST, num = 0.f, den = 0.f;
 #pragma unroll
     for (int i = 0; i < TEAMS; ++i) M = fmaxf(M, teams_m[i]);
 #pragma unroll
     for (int i = 0; i < TEAMS; ++i) {
-      const bool in = teams_m[i] != -INFINITY;
+#pragma clang fp contract(off)
       const float wg = expf(teams_m[i] - M);
-      num += in ? wg * gacc_[i][0][tid] : 0.f;
-      den += in ? wg * teams_l[i] : 0.f;
+      num += wg * gacc_[i][0][tid];
+      den += wg * teams_l[i];
     }
     phi_values(a, row, h)[(by >> 2) * D + tid] = num;
     if (tid == 0) *reinterpret_cast<float2*>(phi_pairs(a, row, h) + 2 * (by >> 2)) = make_float2(M, den);
@@ -336,7 +341,7 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
   }
   __syncthreads();
   if (last && tid < D) {
-    float M = -INFINITY;
+    float M = PHI_LOWEST;
     for (int c = 0; c < ns; ++c) M = fmaxf(M, qr[c]);
     float num = 0.f, den = 0.f;
     for (int c0 = 0; c0 < ns; c0 += 16) {  // sixteen chunks' values in flight, every load unconditional
@@ -353,7 +358,8 @@ __device__ __forceinline__ void phi_attend(const PhiAttnArgs& a, int block) {
       }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const bool in = c0 + i < ns && mc[i] != -INFINITY;
+#pragma clang fp contract(off)
+        const bool in = c0 + i < ns;
         const float wg = expf(mc[i] - M);
         num += in ? wg * av[i] : 0.f;
         den += in ? wg * lc[i] : 0.f;
