@@ -105,51 +105,130 @@ __device__ __forceinline__ float turned_first(float x, float up, float co, float
 __device__ __forceinline__ float turned_query(float x, float down, float co, float sn) { return __builtin_fmaf(x, co, __fmul_rn(down, sn)); }
 __device__ __forceinline__ float turned_key(float x, float down, float co, float sn) { return __builtin_fmaf(down, sn, __fmul_rn(x, co)); }
 
-// The queries q0 + m of a wave with a bit in `which`, one position at a time.  (Sums that are not finite: an infinite key's terms meet zeros in the
-// kernel below, a masked value's infinity a weight of zero.)
-template <int D>
+// The queries q0 + m of a wave with a bit in `which`, whose sums are not finite: an infinite key's terms meet zeros in the kernel below, a masked value's
+// infinity a weight of zero.  So both products are fp32 ones here, of sixteen positions at a time, which the lanes that multiply them read themselves, and of
+// positions that some of the queries do not see a query takes its own only.  It is the launch's last part, a wave's chain of round trips and products.  us, finite
+// / a NaN key in all heads, where each such query walked by itself, a position at a time / so: 32 heads of 80, 100 tokens 10 / 856 / 28, 700 23 / 6600 / 104, 2000
+// 110 / 24800 / 469; 16 of 128, all rotated, 700 43 / 6730 / 173.
+template <int D, int NR>
 __device__ __forceinline__ void phi_walk_rows(const PhiAttnArgs& a, int seq, int h, int q0, unsigned int which, int lane) {
-  constexpr int N = (D + 63) / 64;  // features of a lane
-  const int half = a.rot >> 1;
+  constexpr int NC = (D + 31) / 32, DT = D / 16;
+  asm volatile("" : "+v"(lane));  // (computed anew: the caller's offsets would stay in registers through its loop)
+  const int l16 = lane & 15, g = lane >> 4, half = a.rot >> 1;
+  const int sq = min(q0 + l16, a.S - 1), pq = a.pos + sq, last = a.pos + min(q0 + 31 - __clz(which), a.S - 1);
   const size_t hd = (size_t)a.H * D, at0 = (size_t)seq * a.t_max * hd + (size_t)h * D;
-  const float scale = sqrtf(1.0f / (float)D);
-  auto feature = [&](const bf16_t* row, int position, int j, bool query) {
-    if (j >= D) return 0.f;
-    const float x = bf2f(row[j]);
-    if (j >= a.rot) return x;
-    const float o = bf2f(row[j < half ? j + half : j - half]);
-    const size_t at = (size_t)position * half + (j < half ? j : j - half);
-    const float co = a.cos[at], sn = a.sin[at];
-    return j < half ? turned_first(x, o, co, sn) : query ? turned_query(x, o, co, sn) : turned_key(x, o, co, sn);
+  // features 32 c + 8 g and on of a row; zeros past the head
+  struct Eighth {
+    uint4 x, o, c0, c1, s0, s1;
   };
-#pragma unroll 1
-  for (int m = 0; m < 16 && q0 + m < a.S; ++m) {
-    if (!(which >> m & 1)) continue;
-    const size_t row = (size_t)seq * a.S + q0 + m;
-    const int pq = a.pos + q0 + m;
-    float x[N], o[N], top = -INFINITY, l = 0.f;
+  auto ask = [&](const bf16_t* row, int position, int c) {
+    const int f = 32 * c + 8 * g;
+    Eighth e;
+    e.x = ldg16(row + min(f, D - 8));
+    if (c < NR) {
+      const int partner = f < half ? f + half : f < a.rot ? f - half : 0;
+      const size_t at = (size_t)position * half + (f < half ? f : f < a.rot ? f - half : 0);
+      e.o = ldg16(row + partner);
+      e.c0 = ldg16(a.cos + at);
+      e.c1 = ldg16(a.cos + at + 4);
+      e.s0 = ldg16(a.sin + at);
+      e.s1 = ldg16(a.sin + at + 4);
+    }
+    return e;
+  };
+  auto turn = [&](const Eighth& e, int c, bool query, float (&v)[8]) {
+    const int f = 32 * c + 8 * g;
+    const uint32_t xw[4] = {e.x.x, e.x.y, e.x.z, e.x.w};
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      x[i] = feature(a.q + row * a.ldq + h * D, pq, lane + 64 * i, true);
-      o[i] = 0.f;
+    for (int u = 0; u < 8; ++u) v[u] = f >= D ? 0.f : u & 1 ? hi_bf(xw[u / 2]) : lo_bf(xw[u / 2]);
+    if (c >= NR) return;
+    const uint32_t ow[4] = {e.o.x, e.o.y, e.o.z, e.o.w};
+    const uint32_t cw[8] = {e.c0.x, e.c0.y, e.c0.z, e.c0.w, e.c1.x, e.c1.y, e.c1.z, e.c1.w}, sw[8] = {e.s0.x, e.s0.y, e.s0.z, e.s0.w, e.s1.x, e.s1.y, e.s1.z, e.s1.w};
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float z = u & 1 ? hi_bf(ow[u / 2]) : lo_bf(ow[u / 2]), co = __uint_as_float(cw[u]), sn = __uint_as_float(sw[u]);
+      v[u] = f < half ? turned_first(v[u], z, co, sn) : f < a.rot ? (query ? turned_query(v[u], z, co, sn) : turned_key(v[u], z, co, sn)) : v[u];
+    }
+  };
+  float q[NC][8], m = PHI_LOWEST, l = 0.f;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) turn(ask(a.q + ((size_t)seq * a.S + sq) * a.ldq + h * D, pq, c), c, true, q[c]);
+  const float mul = sqrtf(1.0f / (float)D) * OHARA_LOG2E;
+  f32x4 o[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t) o[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int t0 = 0; t0 <= last; t0 += 16) {
+    f32x4 s = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int t = min(t0 + l16, last);
+    Eighth key[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) key[c] = ask(a.kc + at0 + (size_t)t * hd, t, c);
+    const bool whole = t0 + 15 <= a.pos + q0;  // (uniform) every query sees all of it
+    bf16_t v[4][DT];                           // of position t0 + 4 g + i, feature 16 t + l16
+    if (whole) {
+      const bf16_t* row = a.vc + at0 + (size_t)(t0 + 4 * g) * hd + l16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < DT; ++t) v[i][t] = row[i * hd + 16 * t];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      float k[8];
+      turn(key[c], c, false, k);
+      s = mma_f(k, q[c], s);
+    }
+    float p[4], mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (t0 + 4 * g + r > pq) s[r] = -INFINITY;
+      mx = fmaxf(mx, s[r]);
+    }
+    mx = lane_xor_max<32>(lane_xor_max<16>(mx));
+    const float mn = fmaxf(m, ceilf(mx * mul)), corr = pow2_neg_int(m - mn);
+    m = mn;
+    l *= corr;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      p[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], mul, -mn));
+      l += p[r];
+    }
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[t][r] *= corr;
+    if (whole) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf2f(v[i][t]), p[i], o[t], 0, 0, 0);
+      continue;
     }
 #pragma unroll 1
-    for (int t = 0; t <= pq; ++t) {
-      float s = 0.f;
+    for (int j0 = 0; j0 < 16; j0 += 4)
 #pragma unroll
-      for (int i = 0; i < N; ++i) s = __builtin_fmaf(x[i], feature(a.kc + at0 + (size_t)t * hd, t, lane + 64 * i, false), s);
-      s = wave_sum(s) * scale;
-      const float higher = fmaxf(top, s), corr = top == higher ? 1.0f : __expf(top - higher), p = __expf(s - (higher == -INFINITY ? 0.f : higher));
-      top = higher;
-      l = l * corr + p;
+      for (int r = 0; r < 4; ++r) {
+        const float w = __shfl(p[r], j0 * 4 + l16);
+        const bool in = t0 + j0 + r <= pq;
+        const bf16_t* row = a.vc + at0 + (size_t)min(t0 + j0 + r, last) * hd + 4 * g;
 #pragma unroll
-      for (int i = 0; i < N; ++i)
-        if (lane + 64 * i < D) o[i] = o[i] * corr + p * bf2f(a.vc[at0 + (size_t)t * hd + lane + 64 * i]);
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-      if (lane + 64 * i < D) a.out[row * hd + (size_t)h * D + lane + 64 * i] = f2bf(o[i] * (1.0f / l));
+        for (int t = 0; t < DT; ++t) {
+          const uint2 x = in ? ldg8(row + 16 * t) : make_uint2(0, 0);
+          o[t][0] = __builtin_fmaf(w, lo_bf(x.x), o[t][0]);
+          o[t][1] = __builtin_fmaf(w, hi_bf(x.x), o[t][1]);
+          o[t][2] = __builtin_fmaf(w, lo_bf(x.y), o[t][2]);
+          o[t][3] = __builtin_fmaf(w, hi_bf(x.y), o[t][3]);
+        }
+      }
   }
+  l = lane_xor_sum<32>(lane_xor_sum<16>(l));
+  if (q0 + l16 >= a.S || !(which >> l16 & 1)) return;
+  const float inv = 1.0f / l;
+  bf16_t* row = a.out + ((size_t)seq * a.S + sq) * hd + (size_t)h * D + 4 * g;
+#pragma unroll
+  for (int t = 0; t < DT; ++t) *reinterpret_cast<uint2*>(row + 16 * t) = make_uint2(pack_bf(o[t][0] * inv, o[t][1] * inv), pack_bf(o[t][2] * inv, o[t][3] * inv));
 }
 
 // One workgroup per (sequence, head, 64 queries); each of its four waves owns 16 queries.  Keys and values go through LDS in tiles of 64 positions.
@@ -460,7 +539,7 @@ __global__ __launch_bounds__(256 * TEAMS, 2) void phi_attn_prefill_kernel(PhiAtt
       *reinterpret_cast<uint2*>(orow + 16 * t) =
           make_uint2(pack_bf(o[t][0] * inv, o[t][1] * inv), pack_bf(o[t][2] * inv, o[t][3] * inv));
   }
-  if (odd) phi_walk_rows<D>(a, seq, h, wq0, odd, lane);
+  if (odd) phi_walk_rows<D, NR>(a, seq, h, wq0, odd, lane);
 }
 
 // Features rotated in other numbers than eights, or tables off 16 bytes: keys and values in LDS as fp32, the keys rotated there, in tiles of 32 positions;
