@@ -523,8 +523,8 @@ Epilogue epilogue_of(int epi, int dh, bool stage) {
 // 64 x 96 where what is read is the weights or a long depth, or 64 x 64 is a round and a half, and nothing but the sums is stored: 65 to 128 rows 11264 x 2048
 // 17.2 to 18.0 / 15.0 to 15.7, 320 rows 4096 x 4096 28.1 / 24.2 (192 rows 6144 x 768 7.6 / 7.4, 160 rows 6.8 / 7.0; with rotary 384 rows 3072 x 2048 13.8 /
 // 15.5, 1024 deep 8.5 / 10.2; with a residual 600 rows 2048 x 2048 13.8 / 14.8, 850 rows 1536 x 1536 10.7 / 11.6; 256 rows 5632 x 1024 with SwiGLU 8.2 / 8.7).
-int one_round_tile(int rows, int strips, int K, Epilogue epi) {
-  auto tiles = [&](int r, int s) { return ((int64_t)rows + r - 1) / r * ((strips + s - 1) / s); };
+int one_round_tile(int rows, int strips, int K, Epilogue epi, int parts) {
+  auto tiles = [&](int r, int s) { return ((int64_t)rows + r - 1) / r * ((strips + s - 1) / s) * parts; };
   const int64_t narrow = tiles(T64x48::TM, T64x48::TS), wide = tiles(T64x96::TM, T64x96::TS);
   if (K >= 512 && narrow >= 192 && narrow <= 256 && tiles(32, 2) > 512) return epi != HEAVY || K >= 4096 ? 8 : -1;
   return epi <= GATED && rows > 64 && K >= 1024 && wide >= 192 && wide <= 256 && (rows <= 128 || K >= 4096 || tiles(64, 4) >= 384) ? 9 : -1;
@@ -532,8 +532,11 @@ int one_round_tile(int rows, int strips, int K, Epilogue epi) {
 // `lone`: one full round and nothing behind it takes the chain's time, as a round that lacks a tile does; workgroups of several rounds drift apart.  us, where
 // that decides: 16384 rows 768 x 3072 with a residual 78.3 in 512 tiles of 128 x 192, 74.9 in 192 of 256 x 256; 768 x 768 23.1 / 22.1; 8192 rows 1024 x 1024
 // with a bias 22.5 of 128 x 128, 20.7 of 128 x 256 in halves.  (TIMES are fitted without.)
-float tile_time(const TileTime& t, int rows, int strips, int K, float extra = 0.f, bool lone = false) {
-  const int64_t tiles = ((int64_t)rows + t.rows - 1) / t.rows * ((strips + t.strips - 1) / t.strips);
+// In parts of the depth: K and the strips are a part's, which no tile reaches over.  us with the merge, counted as one product of all parts' strips / so: 375 rows
+// 2640 x 11264 in eight parts, 252 tiles of 128 x 256 that are 264, 49.3 / 39.5 (of 128 x 128); 375 rows 784 x 4096 in four 17.1 / 14.3; 612 rows 20.3 / 16.9;
+// 1702 rows 848 x 7168 45.8 / 35.6; of 1355 such calls 55 change, 9 % quicker on average, one of them 13 % slower (80 rows 784 x 4096 9.1 / 10.3).
+float tile_time(const TileTime& t, int rows, int strips, int K, float extra = 0.f, bool lone = false, int parts = 1) {
+  const int64_t tiles = ((int64_t)rows + t.rows - 1) / t.rows * ((strips + t.strips - 1) / t.strips) * parts;
   const int64_t waves = lone && tiles == CUS * t.slots ? 0 : tiles / (CUS * t.slots), rest = tiles - waves * CUS * t.slots;
   float step = waves * t.slots * t.full;
   if (rest) {
@@ -545,13 +548,13 @@ float tile_time(const TileTime& t, int rows, int strips, int K, float extra = 0.
   return step * K * (1.f / 64.f) + (t.ends + extra) * rounds;
 }
 
-int fastest_tile(int rows, int strips, int K, Epilogue epi = PLAIN) {
+int fastest_tile(int rows, int strips, int K, Epilogue epi = PLAIN, int parts = 1) {
   const bool many = rows >= 1024;
-  if (const int i = one_round_tile(rows, strips, K, epi); !many && i >= 0) return i;
+  if (const int i = one_round_tile(rows, strips, K, epi, parts); !many && i >= 0) return i;
   int best = 0;
   float low = INFINITY;
   for (int i = 0; i < (K < 64 ? 5 : many ? 8 : 6); ++i) {  // (halves walk whole steps)
-    const float t = many ? tile_time(MANY[i], rows, strips, K, EXTRA[epi][i], true) : tile_time(TIMES[i], rows, strips, K);
+    const float t = many ? tile_time(MANY[i], rows, strips, K, EXTRA[epi][i], true, parts) : tile_time(TIMES[i], rows, strips, K, 0.f, false, parts);
     if (t < low) {
       low = t;
       best = i;
@@ -582,7 +585,8 @@ constexpr TileTime FEW[19] = {
 };
 // Tiles in halves among them: slower than the others until the operands of a large product come through them, and then by as much as a quarter
 // quicker.  Fitted to 9400 products of 200 to 1023 rows (1024 to 18000 packed rows, K 384 to 4096, weights of HBM), and compared with the times above and what those
-// lack on the same products, 2 us, with an arithmetic epilogue 4; no fewer tiles than leave most CUs idle, no less depth than the fit holds for.  Of those
+// lack on the same products, 2 us, with an arithmetic epilogue or where it is 128 x 192 4 (845 rows 6848 x 1344 with SwiGLU 24.6 / 20.2, 804 rows 12288 x 1024 with rotary
+// 36.3 / 31.5, 474 rows 3008 x 5120 in four parts 32.3 / 28.9); no fewer tiles than leave most CUs idle, no less depth than the fit holds for.  Of those
 // products 3900 change, 9 % quicker on average, 180 lose more than 3 %; of 1760 with rotary 650 change (14 %, none loses), of 1820 heads of Phi blocks 600 (6 %), of 2390
 // products in parts 1600 (10 %, 70 lose).  us, before / in halves: 512 rows 11264 x 2048 with SwiGLU 32.7 / 28.0, 1000 rows 48.7 / 44.4; 700 rows 6144 x 768
 // 13.6 / 12.3; 700 rows 7680 x 2560 42.0 / 34.3; 700 rows 2560 x 10240 in four parts with their merge 51.7 / 47.4, 450 rows 48.3 / 39.4.
@@ -591,25 +595,26 @@ constexpr TileTime HALVES[3] = {
     {H128x256::TM, H128x256::TS, 1, 0.507f, 0.766f, 0.768f, 6.323f},
     {H128x192::TM, H128x192::TS, 1, 0.437f, 0.736f, 0.627f, 5.293f},
 };
-int few_rows_tile(int rows, int strips, int K, Epilogue epi) {
-  const int now = fastest_tile(rows, strips, K, epi);
+int few_rows_tile(int rows, int strips, int K, Epilogue epi, int parts = 1) {
+  const int now = fastest_tile(rows, strips, K, epi, parts);
   if (rows >= 1024) return now;
+  auto time = [&](const TileTime& t, float extra = 0.f) { return tile_time(t, rows, strips, K, extra, false, parts); };
   int best = now;
-  float low = (epi == HEAVY ? 0.9f : 0.96f) * tile_time(FEW[now], rows, strips, K);
+  float low = (epi == HEAVY ? 0.9f : 0.96f) * time(FEW[now]);
   for (int i = NEW_TILES; i < 19; ++i) {
-    const float t = tile_time(FEW[i], rows, strips, K);
+    const float t = time(FEW[i]);
     if (t < low) {
       low = t;
       best = i;
     }
   }
   if (K < 768) return best;
-  low = tile_time(FEW[best], rows, strips, K) + (epi == HEAVY ? 4.f : 2.f);
+  low = time(FEW[best]) + (epi == HEAVY || best == 4 ? 4.f : 2.f);
   for (int i = 0; i < 3; ++i) {
     const TileTime& h = HALVES[i];
-    if (((int64_t)rows + h.rows - 1) / h.rows * ((strips + h.strips - 1) / h.strips) < (i ? 96 : 136)) continue;
+    if (((int64_t)rows + h.rows - 1) / h.rows * ((strips + h.strips - 1) / h.strips) * parts < (i ? 96 : 136)) continue;
     const float extra = epi == HEAVY ? (i ? 3.f : 6.f) : epi >= ROTARY_32 ? EXTRA[epi][LARGEST + i] : 0.f;
-    const float t = tile_time(h, rows, strips, K, extra);
+    const float t = time(h, extra);
     if (t < low) {
       low = t;
       best = LARGEST + i;
@@ -703,7 +708,8 @@ float least_time(int rows, int strips, int K) {
 }  // namespace
 
 // In how many parts the depth is multiplied: those of least time, the tiles' and the merge's, which is the sums written and
-// read at 8 TB/s (they stay in the caches) and merge_us.  Priced with the six tiles of TIMES at any number of rows, also where another one is launched:
+// read at 8 TB/s (they stay in the caches) and merge_us.  Priced with the six tiles of TIMES at any number of rows, also where another one is launched, and as if
+// tiles reached from part to part:
 // us, as chosen / best: 2048 x 5632, 1800 rows 63 whole / 55 in two parts, 768 x 3072, 1024 rows 23 whole / 18.6 in two; over 15 shapes and 29 numbers of
 // rows from 33 to 4096 4 % above the best choice on average.  us with what follows the product, whole / in parts:
 //   2048 x 5632, residual and norm, 33, 65, 192, 400, 700, 1500 rows  21.1 21.6 26.8 41.2 42.2 58.8 / 11.2 14.6 19.0 28.6 33.2 54.5
@@ -730,7 +736,7 @@ int ohara_depth_parts(int rows, int packed_rows, int k, float merge_us) {
 int ohara_launch_gemm_parts(const GemmArgs& a, int packed_rows, int parts, float* sums, hipStream_t st) {
   const int nstrips = packed_rows / 16;
   if (parts < 2 || a.K % (128 * parts) || ((uintptr_t)a.x & 15) || (a.ldx & 7) || (uint64_t)T256::TM * a.ldx * 2 > UINT32_MAX) return OHARA_EINVAL;
-  switch (few_rows_tile(a.B, nstrips * parts, a.K / parts, PLAIN)) {
+  switch (few_rows_tile(a.B, nstrips, a.K / parts, PLAIN, parts)) {
     case 0: return launch_part<T32>(a, nstrips, parts, sums, st);
     case 1: return launch_part<T64>(a, nstrips, parts, sums, st);
     case 2: return launch_part<T64x128>(a, nstrips, parts, sums, st);
@@ -782,7 +788,7 @@ extern "C" int ohara_gemm_tile_of(int rows, int packed_rows, int k) {
 extern "C" int ohara_gemm_tile_with(int rows, int packed_rows, int k, int epilogue, int parts) {
   if (rows < 1 || packed_rows < 1 || k < 1 || epilogue < EPI_STORE || epilogue > EPI_BIAS_XIELU || parts < 1 || k % parts) return OHARA_EINVAL;
   const int strips = (packed_rows + 15) / 16;
-  const int i = parts > 1 ? few_rows_tile(rows, strips * parts, k / parts, PLAIN) : tile_of(rows, strips, k, epilogue, epilogue_of(epilogue, 64, false));
+  const int i = parts > 1 ? few_rows_tile(rows, strips, k / parts, PLAIN, parts) : tile_of(rows, strips, k, epilogue, epilogue_of(epilogue, 64, false));
   return FEW[i].rows * 1000 + FEW[i].strips * 16 + (i >= LARGEST && i < LARGEST + 3);
 }
 

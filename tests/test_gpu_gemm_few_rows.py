@@ -137,3 +137,15 @@ def test_parts_of_the_depth(cuda, tile, n, k, rows, parts):
                                               ws.data_ptr(), room, torch.cuda.current_stream().cuda_stream), "residual_norm")
     assert ((out.double() - (y + res.double())).abs() <= bound).all()
     assert (ws[room:] == 0xFF).all()
+
+
+# rows, columns, depth, parts, a tile that would make a round of workgroups if it reached from one part into the next
+@pytest.mark.parametrize("rows,n,k,parts,across", [(375, 2640, 11264, 8, 128256), (618, 3200, 9216, 4, 128256), (213, 672, 9216, 8, 80064), (375, 784, 4096, 4, 80064),
+                                                   (364, 1984, 6144, 8, 128192), (412, 656, 4096, 4, 80064)])
+def test_parts_are_counted_by_themselves(cuda, rows, n, k, parts, across):
+    from ohara_amd._lib import lib
+
+    strips, height, width = n // 16, across // 1000, across % 1000 // 16
+    down = -(-rows // height)
+    assert down * -(-strips * parts // width) <= 256 < down * -(-strips // width) * parts
+    assert lib().ohara_gemm_tile_with(rows, n, k, 1, parts) // 2 * 2 != across
