@@ -568,7 +568,8 @@ int fastest_tile(int rows, int strips, int K, Epilogue epi = PLAIN, int parts = 
 // (17 of a model's widths and depths whole, 8 in parts; 33 to 1023 rows; each tile that makes 48 to 1600 workgroups; cold weights), those of a
 // tile alone on its CU within 3 to 5 %, of those that share one within 7 to 12 %.  Such a tile is taken where they promise 4 % (10 with an arithmetic
 // epilogue, whose waves hold more of it): of the 1201 products with a choice 340 change, 12 % quicker on average (as much as 30), 21 lose more than 3 %, the worst 9
-// (768 x 3072 in two parts, 860 rows: 10.7 / 11.7).  us, before / now: 224 rows 11264 x 2048 with SwiGLU 26.7 / 21.1, 320 rows 3072 x 2048 14.9 / 11.4, 1000 rows
+// (768 x 3072 in two parts, 860 rows: 10.7 / 11.7).  Of 2401 others, drawn, with the rules below and their weights from memory, 974 are more than 2 % quicker than without
+// such tiles, 37 slower, the worst 7 (65 rows 12288 x 768 with rotary 10.3 / 11.0); from the cache, as 256 MB of weights stay, 80 x 64 loses up to 16.  us, before / now: 224 rows 11264 x 2048 with SwiGLU 26.7 / 21.1, 320 rows 3072 x 2048 14.9 / 11.4, 1000 rows
 // 27.7 / 20.4, 400 rows 15.4 / 13.1.
 constexpr int NEW_TILES = 10;  // the first of these tiles
 constexpr TileTime FEW[19] = {
@@ -595,13 +596,19 @@ constexpr TileTime HALVES[3] = {
     {H128x256::TM, H128x256::TS, 1, 0.507f, 0.766f, 0.768f, 6.323f},
     {H128x192::TM, H128x192::TS, 1, 0.437f, 0.736f, 0.627f, 5.293f},
 };
+// Where the times promise what is not so, us there / with the tile that stays: tiles of 64 x 48 that are a round against those of 48 x 64 (all 41 such products of
+// 3900 lose: 45 rows 10272 x 1920 with SwiGLU 14.8 / 13.6, 47 rows 9216 x 1536 with rotary 13.3 / 11.8), and tiles of 64 x 128 of which a few CUs have two against 96 x
+// 64 (217 rows of a Phi head 8272 x 2528, 260 of them: 32.6 / 30.1 with 128 x 96, 28.3 with 64 x 128; from 268 on those lose).
 int few_rows_tile(int rows, int strips, int K, Epilogue epi, int parts = 1) {
   const int now = fastest_tile(rows, strips, K, epi, parts);
   if (rows >= 1024) return now;
   auto time = [&](const TileTime& t, float extra = 0.f) { return tile_time(t, rows, strips, K, extra, false, parts); };
+  const int64_t wide = ((int64_t)rows + T64x128::TM - 1) / T64x128::TM * ((strips + T64x128::TS - 1) / T64x128::TS) * parts;
+  const bool just_over = now == 2 && wide > CUS && wide < CUS + CUS / 25;
   int best = now;
   float low = (epi == HEAVY ? 0.9f : 0.96f) * time(FEW[now]);
   for (int i = NEW_TILES; i < 19; ++i) {
+    if ((now == 8 && i == 10) || (just_over && i == 12)) continue;
     const float t = time(FEW[i]);
     if (t < low) {
       low = t;

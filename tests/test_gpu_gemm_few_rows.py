@@ -149,3 +149,12 @@ def test_parts_are_counted_by_themselves(cuda, rows, n, k, parts, across):
     down = -(-rows // height)
     assert down * -(-strips * parts // width) <= 256 < down * -(-strips // width) * parts
     assert lib().ohara_gemm_tile_with(rows, n, k, 1, parts) // 2 * 2 != across
+
+
+# rows, packed rows, depth, epilogue, parts, the tile: a round of 64 x 48, and 260, 264 and 268 of 64 x 128
+@pytest.mark.parametrize("rows,packed,k,epilogue,parts,tile", [(45, 10272, 1920, 2, 1, 64048), (136, 3872, 1600, 1, 1, 64048), (47, 9216, 1536, 3, 1, 64048), (44, 1408, 5120, 1, 8, 64048),
+                                                               (217, 8272, 2528, 7, 1, 128096), (217, 8384, 1280, 2, 1, 128096), (206, 8528, 816, 7, 1, 96064)])
+def test_tiles_that_stay(cuda, rows, packed, k, epilogue, parts, tile):
+    from ohara_amd._lib import lib
+
+    assert lib().ohara_gemm_tile_with(rows, packed, k, epilogue, parts) == tile
