@@ -30,7 +30,7 @@ def test_silu(cuda, rows, n):
     """Of weights times a one, the other factor one: the small tiles, the large ones, and numbers below -87 among the others and not."""
     from ohara_amd import ops
 
-    for x in (_every(cuda), _every(cuda).clamp(min=-80).nan_to_num(1.0)):
+    for x in (_every(cuda), _every(cuda).clamp(min=-87).nan_to_num(1.0)):
         x = x[torch.randperm(65536, device=cuda)[:n]] if n < 65536 else x
         gate, up = torch.zeros(n, 64, dtype=BF, device=cuda), torch.zeros(n, 64, dtype=BF, device=cuda)
         gate[:, 3], up[:, 3] = x, 1.0
@@ -39,7 +39,7 @@ def test_silu(cuda, rows, n):
         got = ops.gemm(row, ops.pack_gate_up(gate, up))
         d = x.double()
         want = (d / (1.0 + torch.exp(-d))).to(BF)
-        plain = d.isfinite() & (d >= -86)  # (below: a reciprocal beyond fp32's normal numbers; infinities times the other columns' zeros are NaN)
+        plain = d.isfinite() & (d >= -87)  # (below: a reciprocal beyond fp32's normal numbers; infinities times the other columns' zeros are NaN)
         assert torch.equal(got[:, plain], want[plain].expand(rows, -1))
-        small = d.isfinite() & (d < -86)
+        small = d.isfinite() & (d < -87)
         assert (got[:, small].abs() <= 1e-35).all()

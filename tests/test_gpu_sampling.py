@@ -182,6 +182,55 @@ def test_rows_of_one_single_value(cuda):
             assert abs(int(got[b]) - int(float(u[b]) * V)) <= 2, (V, b, int(got[b]))
 
 
+@pytest.mark.parametrize("T,k,p", [(1.0, 0, 0.9), (0.8, 0, 0.3), (1.3, 1500, 0.95), (1.0, 3000, 1.0)])
+@pytest.mark.parametrize("lowest,highest,signs", [(2.0 ** -24, 8.0, (1, -1)), (2.0 ** -6, 2.0 ** 30, (-1,))])
+def test_rows_of_many_patterns(cuda, lowest, highest, signs, T, k, p):
+    """More different numbers than the count table's list holds, of both signs and none above zero: the largest of them and the walk without the list.  (Those
+    that a draw may land on differ in their probabilities too: among equal ones the oracle knows no order of the logits.)"""
+    from ohara_amd import ops
+
+    g = torch.Generator().manual_seed(k + len(signs))
+    every = torch.arange(32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    every = every[(every >= lowest) & (every <= highest)]
+    every = torch.cat([every * s for s in signs])
+    V, B, tol = 20000, 4, 5e-5
+    assert 4096 < every.numel() < 8192
+    rows = torch.stack([torch.cat([every, every[torch.randint(0, every.numel(), (V - every.numel(),), generator=g)]])[torch.randperm(V, generator=g)] for _ in range(B)])
+    for trial in range(4):
+        u = torch.rand(B, generator=g)
+        if trial == 0:
+            u[0], u[-1] = 0.0, 0.999999
+        want, margin = sample_next_token_ref(rows.unsqueeze(1), T, p, k, u=u, return_margin=True)
+        ids, cdf = candidate_cdf_ref(rows.unsqueeze(1), T, p, k)
+        got = ops.sample_topk_topp(rows.to(cuda), T, k, p, u.to(cuda)).cpu()
+        for b in range(B):
+            j = int((ids[b] == int(got[b])).nonzero()[0])
+            assert (float(cdf[b, j - 1]) if j else 0.0) - tol <= float(u[b]) <= float(cdf[b, j]) + tol, (b, int(got[b]))
+            if float(margin[b]) > tol:
+                assert int(got[b]) == int(want[b, 0]), (b, int(got[b]), int(want[b, 0]), float(margin[b]))
+
+
+@pytest.mark.parametrize("value", [-1.5, -0.0, 0.0, 3.0])
+@pytest.mark.parametrize("others", [0, 1, 7])
+def test_counts_that_fill_their_sixteen_bits(cuda, value, others):
+    """65536 ids of one value, whose count carries into the other sign's or out of the word; all but a few, which does not; and as many with a padded tail."""
+    from ohara_amd import ops
+
+    V = 65536
+    row = torch.full((2, V), value, dtype=torch.bfloat16, device=cuda)
+    if others:
+        row[:, V // 3: V // 3 + others] = value - 20.0
+    u = torch.tensor([0.25, 0.9], device=cuda)
+    for valid in (None, V - 5):
+        n = (valid or V) - others
+        for k, p, kept in ((0, 0.5, int(0.5 * n) + 1), (2000, 1.0, n), (2000, 0.5, int(0.5 * n) + 1)):
+            got = ops.sample_topk_topp(row, 1.0, k, p, u, valid).cpu()
+            for b in range(2):
+                at = int(float(u[b]) * kept)
+                at += others if at >= V // 3 else 0
+                assert abs(int(got[b]) - at) <= 2, (valid, k, p, b, int(got[b]), at)
+
+
 @pytest.mark.parametrize("V,B,T,k,p,std", [(65536, 8, 0.8, 50, 0.9, 0.55), (65536, 3, 1.0, 1, 1.0, 1.0),
                                            (32000, 5, 0.7, 64, 0.0, 2.0), (50000, 2, 1.2, 40, 0.95, 6.0)])
 def test_small_top_k_over_several_workgroups(cuda, V, B, T, k, p, std):
