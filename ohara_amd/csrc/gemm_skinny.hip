@@ -297,8 +297,9 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
 // layernorm_kernel's to the bit.  A wave asks for the row, the norm's weight and bias and then for its whole share of the strip, so the statistics and
 // their barriers pass while the weights travel, and the norm's launch, a workgroup a row, is spared.  What it costs is every workgroup's reads of the row and
 // the norm's, 15 KB beside 80 of weights; so two workgroups to a CU, which keep the row and go from strip to strip with the next one's weights ahead of them.
-// us, norm and head / a workgroup a strip / this: 2560 x (7680 + 10240) one row 19.1 / 18.1 / 16.9 (16.4 without a norm), two 19.1 / 18.1 / 17.3; 2048 x (6144 +
-// 8192) 16.1 / 13.9 / 14.6, 15.9 / 13.9 / 14.4.
+// us, norm and head / this in a workgroup a strip / 512 of them: 2560 x (7680 + 10240) one row 18.8 / 18.6 / 17.0 (16.4 without a norm), two 18.9 / 19.3 / 16.7; 2304 x
+// (6912 + 9216) 16.7 / 15.8 / 14.7, 17.0 / 16.5 / 15.0; 2048 x (6144 + 8192) 14.7 / 14.4 / 13.5, 15.4 / 14.8 / 13.8; 640 strips of 2048 12.4 / 11.2 / 10.7.  (256: 18.1, 15.4,
+// 13.4, 10.5; 400 18.8, 15.4, 13.7, 10.7.)
 template <int SP>
 __global__ __launch_bounds__(512, 4) void phi_in_kernel(GemmArgs a) {
   constexpr int NW = 8;
@@ -398,8 +399,10 @@ __global__ __launch_bounds__(512, 4) void phi_in_kernel(GemmArgs a) {
     into ^= 1;
   }
 }
-// (the widths of which a wave's share is eight to ten k-steps; fewer strips are a workgroup of sixteen waves each in skinny_kernel)
-static bool phi_in_norms(int rows, int d, int strips) { return rows <= 2 && d >= 2048 && d <= 2560 && strips >= 400; }
+// A wave's share is eight k-steps at least, and as many as it holds at most: wider rows and narrower ones are normed by a launch of their own, the strips by
+// skinny_kernel, fewer of them a workgroup of sixteen waves each.
+constexpr int PHI_IN_STEPS = 10;
+static bool phi_in_norms(int rows, int d, int strips) { return rows <= 2 && d >= 2048 && d <= 256 * PHI_IN_STEPS && strips >= 400; }
 
 // Phi's attention of single tokens beside the second product of its MLP, which does not wait for it: neither fills the chip - 352 teams of four waves,
 // whose chain of round trips bounds them, and 160 strips - and one after the other they took the sum of their times.  The attention's go first: its
@@ -1350,7 +1353,7 @@ int ohara_phi_block_in_bf16(const uint16_t* x, int ldx, const uint16_t* ln_w, co
   const int packed_rows = (a.N + 15) / 16 * 16;
   if (ln_w && phi_in_norms(a.B, d, packed_rows / 16) && !(((uintptr_t)ln_w | (uintptr_t)ln_b | (uintptr_t)x) & 15)) {
     a.nstrips = packed_rows / 16;
-    hipLaunchKernelGGL(phi_in_kernel<10>, dim3((unsigned)std::min(a.nstrips, 512)), dim3(512), 0, (hipStream_t)stream, a);
+    hipLaunchKernelGGL(phi_in_kernel<PHI_IN_STEPS>, dim3((unsigned)std::min(a.nstrips, 512)), dim3(512), 0, (hipStream_t)stream, a);
     return ohara_launch_status();
   }
   if (!ln_w && ohara_tiles_win(a.B, a.K, packed_rows)) return ohara_launch_gemm_tile(a, EPI_PHI_IN, packed_rows, (hipStream_t)stream);  // prefill

@@ -333,7 +333,7 @@ __global__ __launch_bounds__(C::NW * 64, 2) void gemm_tile_kernel(GemmArgs a, in
 }
 
 // A workgroup a CU, which takes every 32nd tile of its XCD's run, where there are more tiles than CUs.  Its loads run from one tile into the next: what
-// halves_stream asks for in a tile's last steps are the first steps of the one behind it, which arrive under the epilogue.
+// HalvesStream asks for in a tile's last steps are the first steps of the one behind it, which arrive under the epilogue.
 // us, a workgroup a tile / this: 8192 rows 6144 x 768 with SwiGLU 77.8 / 73.2 (66 to 69 with the shorter silu), plain 77.2 / 73.3, 384 deep 55.8 / 48.6; 4001 rows 11264 x 2048 with SwiGLU 151 /
 // 144, 11200 rows 399 / 377; 8192 rows 7680 x 2560 237 / 233.  What is left of a boundary there, 8 of 24 us a tile: the epilogue's arithmetic (SwiGLU 4 us), or where
 // much is stored the memory (100 MB of a plain store 16.6 of 72.3 us); zeros instead of random numbers 53 us: the chip's clock under its load.
@@ -476,7 +476,8 @@ constexpr TileTime TIMES[6] = {
 // From 1024 rows on, the tiles in halves among them: drawn through 1117 products of 1024 to 16384 rows, 256 to 18000 packed rows, K 256 to 5632, with
 // the epilogues below, each as it stands in a model (128 MB of other work before it, then its activations written; weights, residual and output as that
 // leaves them): the choice is within 0.9 % of the best of the eight on average, 0.7 % on the products left out of the fit.  A tile alone on its CU
-// pays its ends once in every round.  Fewer rows are a round of small tiles or parts of the depth, to which the times above are fitted.
+// pays its ends once in every round.  (All with a workgroup a tile; since gemm_rounds_kernel the halves of more tiles than CUs take 5 to 13 % less than these
+// times, and the choice is 0.5 to 2 % above the best of seven tiles on the widths of a model.)  Fewer rows are a round of small tiles or parts of the depth, to which the times above are fitted.
 // (Timed one behind the other, with residual and output in the L2s, the tiles of two a CU come out up to 15 % better than they are: 8192 rows 768 x 768 with
 // a residual 128 x 192 18.4 us there and 20.2 in the model, in halves 20.4 and 18.1.)
 constexpr TileTime MANY[10] = {
@@ -568,9 +569,9 @@ int fastest_tile(int rows, int strips, int K, Epilogue epi = PLAIN, int parts = 
 // (17 of a model's widths and depths whole, 8 in parts; 33 to 1023 rows; each tile that makes 48 to 1600 workgroups; cold weights), those of a
 // tile alone on its CU within 3 to 5 %, of those that share one within 7 to 12 %.  Such a tile is taken where they promise 4 % (10 with an arithmetic
 // epilogue, whose waves hold more of it): of the 1201 products with a choice 340 change, 12 % quicker on average (as much as 30), 21 lose more than 3 %, the worst 9
-// (768 x 3072 in two parts, 860 rows: 10.7 / 11.7).  Of 2401 others, drawn, with the rules below and their weights from memory, 974 are more than 2 % quicker than without
-// such tiles, 37 slower, the worst 7 (65 rows 12288 x 768 with rotary 10.3 / 11.0); from the cache, as 256 MB of weights stay, 80 x 64 loses up to 16.  us, before / now: 224 rows 11264 x 2048 with SwiGLU 26.7 / 21.1, 320 rows 3072 x 2048 14.9 / 11.4, 1000 rows
-// 27.7 / 20.4, 400 rows 15.4 / 13.1.
+// (768 x 3072 in two parts, 860 rows: 10.7 / 11.7).  Of 2401 others, drawn, with the rules below and their weights from memory, 974 are more than 2 % quicker than
+// without such tiles, 37 slower, the worst 7 (65 rows 12288 x 768 with rotary 10.3 / 11.0); with weights that stay in the 256 MB of cache 80 x 64 loses up to 16.
+// us, before / now: 224 rows 11264 x 2048 with SwiGLU 26.7 / 21.1, 320 rows 3072 x 2048 14.9 / 11.4, 1000 rows 27.7 / 20.4, 400 rows 15.4 / 13.1.
 constexpr int NEW_TILES = 10;  // the first of these tiles
 constexpr TileTime FEW[19] = {
     {T32::TM, T32::TS, 3, 0.147f, 0.412f, 0.081f, 0.482f},          {T64::TM, T64::TS, 2, 0.302f, 0.252f, 0.208f, 0.779f},
@@ -587,10 +588,11 @@ constexpr TileTime FEW[19] = {
 // Tiles in halves among them: slower than the others until the operands of a large product come through them, and then by as much as a quarter
 // quicker.  Fitted to 9400 products of 200 to 1023 rows (1024 to 18000 packed rows, K 384 to 4096, weights of HBM), and compared with the times above and what those
 // lack on the same products, 2 us, with an arithmetic epilogue or where it is 128 x 192 4 (845 rows 6848 x 1344 with SwiGLU 24.6 / 20.2, 804 rows 12288 x 1024 with rotary
-// 36.3 / 31.5, 474 rows 3008 x 5120 in four parts 32.3 / 28.9); no fewer tiles than leave most CUs idle, no less depth than the fit holds for.  Of those
-// products 3900 change, 9 % quicker on average, 180 lose more than 3 %; of 1760 with rotary 650 change (14 %, none loses), of 1820 heads of Phi blocks 600 (6 %), of 2390
-// products in parts 1600 (10 %, 70 lose).  us, before / in halves: 512 rows 11264 x 2048 with SwiGLU 32.7 / 28.0, 1000 rows 48.7 / 44.4; 700 rows 6144 x 768
-// 13.6 / 12.3; 700 rows 7680 x 2560 42.0 / 34.3; 700 rows 2560 x 10240 in four parts with their merge 51.7 / 47.4, 450 rows 48.3 / 39.4.
+// 36.3 / 31.5, 474 rows 3008 x 5120 in four parts 32.3 / 28.9); no fewer tiles than leave most CUs idle, no depth under 768, where 515 more of those products
+// would change, 0.4 % quicker on average, and 152 of them lose more than 3 %.  (39 whole products with a residual, 4096 to 10240 deep, beyond the fit, take 24 % less.)
+// Of those of 768 and more 3900 change, 9 % quicker on average, 180 lose more than 3 %; of 1760 with rotary 650 change (14 %, none loses), of 1820 heads of Phi
+// blocks 600 (6 %), of 2390 products in parts 1600 (10 %, 70 lose).  us, before / in halves: 512 rows 11264 x 2048 with SwiGLU 32.7 / 28.0, 1000 rows 48.7 / 44.4;
+// 700 rows 6144 x 768 13.6 / 12.3; 700 rows 7680 x 2560 42.0 / 34.3; 700 rows 2560 x 10240 in four parts with their merge 51.7 / 47.4, 450 rows 48.3 / 39.4.
 constexpr TileTime HALVES[3] = {
     {T256::TM, T256::TS, 1, 0.521f, 1.671f, 1.479f, 11.155f},
     {H128x256::TM, H128x256::TS, 1, 0.507f, 0.766f, 0.768f, 6.323f},
@@ -630,9 +632,9 @@ int few_rows_tile(int rows, int strips, int K, Epilogue epi, int parts = 1) {
   return best;
 }
 constexpr bool has_new_tiles(int epi) { return epi == EPI_RESIDUAL || epi == EPI_SWIGLU || epi == EPI_ROPE || epi == EPI_PHI_IN || epi == EPI_STORE; }
-// A plain store has them from 20000 packed rows on: a vocabulary, which no other plain store of a model comes near.  us, without / with: 32000 x 2048, 128, 192, 256, 384,
-// 700 rows 35.7 40.7 45.7 52.2 94.7 / 36.2 34.0 40.5 51.7 88.5; 65536 x 768, 128, 300, 384 rows 28.4 48.4 55.9 / 28.1 43.3 49.1; 51200 x 2560, 300, 700 rows 120.8
-// 194.8 / 107.1 164.6.
+// A plain store has them from 20000 packed rows on, a vocabulary: under that ohara_gemm_tile_of says what it runs, whatever the number of rows.  us, without / with: 32000 x
+// 2048, 128, 192, 256, 384, 700 rows 35.7 40.7 45.7 52.2 94.7 / 36.2 34.0 40.5 51.7 88.5; 65536 x 768, 128, 300, 384 rows 28.4 48.4 55.9 / 28.1 43.3 49.1.  (With a
+// bias, as Phi's is stored, there are none of them: that epilogue's tiles are the six and the two of a round.)
 int tile_of(int rows, int strips, int K, int epi, Epilogue kind) {
   return has_new_tiles(epi) && (epi != EPI_STORE || strips >= 1250) ? few_rows_tile(rows, strips, K, kind) : fastest_tile(rows, strips, K, kind);
 }
